@@ -178,6 +178,22 @@ int samfast_gemm_i8_scale_bias(
     int64_t M, int N, int K, int dtype, void* stream);
 
 /*
+ * The whole quantised nn.Linear.forward: samfast_quant_rowwise_i8 followed by
+ * samfast_gemm_i8_scale_bias, same codes, accumulators and result.  `layout` is the layout of wq
+ * (and of the activation codes between the two steps).  `workspace`: at least
+ * samfast_linear_i8_workspace(M, N, K, layout) bytes of device memory, 16-byte aligned, contents
+ * irrelevant before and after; may be NULL where that is 0.  The size function returns
+ * SAMFAST_E_INVALID for a negative or zero dimension or an unknown layout; with
+ * SAMFAST_LAYOUT_SPARSE24 it answers for samfast_linear_i8_sparse24.
+ */
+#define SAMFAST_LAYOUT_SPARSE24 2  /* samfast_linear_i8_workspace only */
+int samfast_linear_i8(
+    const void* x, int64_t ldx, const int8_t* wq, const float* sw, const float* bias,
+    void* y, int64_t ldy, void* workspace,
+    int64_t M, int N, int K, int dtype, int layout, void* stream);
+int64_t samfast_linear_i8_workspace(int64_t M, int N, int K, int layout);
+
+/*
  * LayerNorm over each row followed by the per-row int8 quantiser, with an optional
  * row gather: output row r is computed from source row src_row[r] of x (src_row NULL =
  * identity); src_row[r] < 0 yields an all-zero row with scale 1e-5/127.
@@ -294,6 +310,12 @@ int samfast_gemm_i8_sparse24_fused(
     const float* sw, const float* bias, void* y, int64_t ldy,
     int64_t M, int N, int K, int dtype, int epilogue,
     const void* residual, int64_t ld_res, int layout, void* stream);
+
+/* samfast_linear_i8 with the weight in the packed 2:4 form. */
+int samfast_linear_i8_sparse24(
+    const void* x, int64_t ldx, const int8_t* wc, const int32_t* widx, const float* sw,
+    const float* bias, void* y, int64_t ldy, void* workspace,
+    int64_t M, int N, int K, int dtype, void* stream);
 
 #ifdef __cplusplus
 }

@@ -1157,6 +1157,39 @@ extern "C" int samfast_gemm_i8_fused_quant(const int8_t* xq, const float* sx, co
   return samfast_quant_rowwise_i8(y, ldy, yq, sy, M, N, dtype, yq_layout, stream);
 }
 
+// ---- a whole quantised Linear ---------------------------------------------------------------
+extern "C" int64_t samfast_linear_i8_workspace(int64_t M, int N, int K, int layout) {
+  using namespace samfast;
+  SF_REQUIRE(M > 0 && N > 0 && K > 0 && layout >= SAMFAST_LAYOUT_ROWMAJOR && layout <= SAMFAST_LAYOUT_SPARSE24,
+             "linear_i8_workspace: bad shape M=%lld N=%d K=%d or layout %d", (long long)M, N, K, layout);
+  // codes, then the row scales
+  return ((M * K + 15) & ~(int64_t)15) + M * 4;
+}
+
+extern "C" int samfast_linear_i8(const void* x, int64_t ldx, const int8_t* wq, const float* sw, const float* bias,
+                                 void* y, int64_t ldy, void* workspace, int64_t M, int N, int K, int dtype,
+                                 int layout, void* stream) {
+  using namespace samfast;
+  SF_REQUIRE(M == 0 || (workspace && aligned16(workspace)), "linear_i8: the workspace must be non-null and 16-byte aligned");
+  int8_t* xq = reinterpret_cast<int8_t*>(workspace);
+  float* sx = reinterpret_cast<float*>(xq + ((M * K + 15) & ~(int64_t)15));
+  const int rc = samfast_quant_rowwise_i8(x, ldx, xq, sx, M, K, dtype, layout, stream);
+  if (rc != SAMFAST_OK) return rc;
+  return samfast_gemm_i8_fused(xq, sx, wq, sw, bias, y, ldy, M, N, K, dtype, SAMFAST_EPILOGUE_NONE, nullptr, 0, nullptr, layout, stream);
+}
+
+extern "C" int samfast_linear_i8_sparse24(const void* x, int64_t ldx, const int8_t* wc, const int32_t* widx,
+                                          const float* sw, const float* bias, void* y, int64_t ldy, void* workspace,
+                                          int64_t M, int N, int K, int dtype, void* stream) {
+  using namespace samfast;
+  SF_REQUIRE(M == 0 || (workspace && aligned16(workspace)), "linear_i8_sparse24: the workspace must be non-null and 16-byte aligned");
+  int8_t* xq = reinterpret_cast<int8_t*>(workspace);
+  float* sx = reinterpret_cast<float*>(xq + ((M * K + 15) & ~(int64_t)15));
+  const int rc = samfast_quant_rowwise_i8(x, ldx, xq, sx, M, K, dtype, SAMFAST_LAYOUT_KB64, stream);
+  if (rc != SAMFAST_OK) return rc;
+  return samfast_gemm_i8_sparse24_fused(xq, sx, wc, widx, sw, bias, y, ldy, M, N, K, dtype, SAMFAST_EPILOGUE_NONE, nullptr, 0, SAMFAST_LAYOUT_KB64, stream);
+}
+
 // ---- the same call for callers that cannot allocate ---------------------------------------
 // The counter workspace of samfast_gemm_i8_fused_quant lives in a file-scope device array, one
 // copy per GPU, held until the process ends.  Its address on a device is looked up once per

@@ -1,0 +1,197 @@
+// The per-call host work of the hot entry points as native code: reading shapes, strides and
+// pointers out of torch tensors, allocating outputs and workspaces and calling the C ABI.  Done in
+// Python (ops.py) this costs 20-30 us per call, several times what a small call runs on the GPU
+// (a Linear over 7 tokens: 7 us of kernels); here it is 2-3 us plus the launches.
+//
+// Every function returns None for a call it does not cover - a CPU tensor, another type, a strided
+// view, a shape the C ABI refuses - and the caller then takes the Python route in ops.py, whose
+// checks and error texts stay the one definition of what is accepted.
+//
+// The C ABI is reached through pointers that bind() receives from the ctypes handle, so that one
+// copy of libsamfast.so serves both (also when SAMFAST_LIB names another file).
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/GradMode.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "samfast.h"
+
+namespace {
+
+decltype(&samfast_linear_i8) p_linear_i8;
+decltype(&samfast_linear_i8_workspace) p_linear_i8_workspace;
+decltype(&samfast_linear_i8_sparse24) p_linear_i8_sparse24;
+decltype(&samfast_attn_relpos_bias_fwd) p_attn_bias;
+
+struct Bound { const char* name; void** slot; };
+const Bound kBound[] = {
+    {"samfast_linear_i8", reinterpret_cast<void**>(&p_linear_i8)},
+    {"samfast_linear_i8_workspace", reinterpret_cast<void**>(&p_linear_i8_workspace)},
+    {"samfast_linear_i8_sparse24", reinterpret_cast<void**>(&p_linear_i8_sparse24)},
+    {"samfast_attn_relpos_bias_fwd", reinterpret_cast<void**>(&p_attn_bias)},
+};
+
+// a plain strided GPU tensor on the current device (the launches go to its current stream)
+bool on_current_gpu(const at::Tensor& t, c10::DeviceIndex dev) {
+  return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.device().index() == dev && !t.key_set().has(c10::DispatchKey::Python);
+}
+
+const at::Tensor* tensor_arg(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+void* stream_of(c10::DeviceIndex dev) { return c10::hip::getCurrentHIPStream(dev).stream(); }
+
+const void* ptr(const at::Tensor& t) { return t.const_data_ptr(); }
+
+// What the dense and the sparse Linear share: x is (..., K) contiguous bf16, sw_bits / bias_bits are
+// the fp32 scales and bias as the modules hold them (int32 bit patterns).  Fills y and the workspace.
+struct LinearCall {
+  const at::Tensor *x, *sw, *bias;
+  int64_t M, N, K;
+  at::Tensor y, work;
+  const float* sw_ptr() const { return static_cast<const float*>(ptr(*sw)); }
+  const float* bias_ptr() const { return bias ? static_cast<const float*>(ptr(*bias)) : nullptr; }
+  void* work_ptr() const { return work.defined() ? work.data_ptr() : nullptr; }
+
+  bool accept(c10::DeviceIndex dev) const {
+    return on_current_gpu(*x, dev) && on_current_gpu(*sw, dev) && (!bias || on_current_gpu(*bias, dev)) &&
+           x->scalar_type() == at::kBFloat16 && x->dim() >= 1 && x->is_contiguous() && x->numel() > 0 &&
+           K > 0 && x->size(-1) == K && N <= INT32_MAX && K <= INT32_MAX &&
+           sw->scalar_type() == at::kInt && sw->is_contiguous() && sw->numel() == N &&
+           (!bias || (bias->scalar_type() == at::kInt && bias->is_contiguous() && bias->numel() == N));
+  }
+  void allocate(int64_t need) {
+    c10::SmallVector<int64_t, 5> shape(x->sizes().begin(), x->sizes().end());
+    shape.back() = N;
+    y = at::empty(shape, x->options().requires_grad(false));
+    if (need > 0) work = at::empty({need}, x->options().dtype(at::kByte).requires_grad(false));
+  }
+};
+
+// linear(x, wq, layout, sw_bits, bias_bits or None): the whole int8 Linear on bf16 rows.
+// wq is (N, K), or (K/64, N, 64) for layout 1.
+PyObject* host_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 5) Py_RETURN_NONE;
+  const at::Tensor* wq = tensor_arg(args[1]);
+  const int layout = static_cast<int>(PyLong_AsLong(args[2]));
+  const bool kb = layout == SAMFAST_LAYOUT_KB64;
+  LinearCall c = {tensor_arg(args[0]), tensor_arg(args[3]), tensor_arg(args[4])};
+  if (!c.x || !wq || !c.sw || (args[4] != Py_None && !c.bias)) Py_RETURN_NONE;
+  const c10::DeviceIndex dev = c10::hip::current_device();
+  if (!on_current_gpu(*wq, dev) || wq->scalar_type() != at::kChar || wq->dim() != (kb ? 3 : 2) || !wq->is_contiguous()) Py_RETURN_NONE;
+  c.N = wq->size(kb ? 1 : 0);
+  c.K = kb ? wq->size(0) * 64 : wq->size(1);
+  if (!c.accept(dev)) Py_RETURN_NONE;
+  c.M = c.x->numel() / c.K;
+  const int64_t need = p_linear_i8_workspace(c.M, static_cast<int>(c.N), static_cast<int>(c.K), layout);
+  if (need < 0) Py_RETURN_NONE;
+  c.allocate(need);
+  const int rc = p_linear_i8(ptr(*c.x), c.K, static_cast<const int8_t*>(ptr(*wq)), c.sw_ptr(), c.bias_ptr(), c.y.data_ptr(), c.N,
+                             c.work_ptr(), c.M, static_cast<int>(c.N), static_cast<int>(c.K), SAMFAST_BF16, layout, stream_of(dev));
+  if (rc != SAMFAST_OK) Py_RETURN_NONE;
+  return THPVariable_Wrap(std::move(c.y));
+  END_HANDLE_TH_ERRORS
+}
+
+// sparse_linear(x, wc, widx, sw_bits, bias_bits or None): the same with the packed 2:4 weight
+PyObject* host_sparse_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 5) Py_RETURN_NONE;
+  const at::Tensor *wc = tensor_arg(args[1]), *widx = tensor_arg(args[2]);
+  LinearCall c = {tensor_arg(args[0]), tensor_arg(args[3]), tensor_arg(args[4])};
+  if (!c.x || !wc || !widx || !c.sw || (args[4] != Py_None && !c.bias)) Py_RETURN_NONE;
+  const c10::DeviceIndex dev = c10::hip::current_device();
+  if (!on_current_gpu(*wc, dev) || !on_current_gpu(*widx, dev) || wc->scalar_type() != at::kChar || widx->scalar_type() != at::kInt ||
+      wc->dim() != 3 || widx->dim() != 3 || !wc->is_contiguous() || !widx->is_contiguous() || wc->size(2) != 32 ||
+      widx->size(0) != wc->size(0) || widx->size(1) != wc->size(1) || widx->size(2) != 2)
+    Py_RETURN_NONE;
+  c.N = wc->size(1);
+  c.K = wc->size(0) * 64;
+  if (!c.accept(dev)) Py_RETURN_NONE;
+  c.M = c.x->numel() / c.K;
+  const int64_t need = p_linear_i8_workspace(c.M, static_cast<int>(c.N), static_cast<int>(c.K), SAMFAST_LAYOUT_SPARSE24);
+  if (need < 0) Py_RETURN_NONE;
+  c.allocate(need);
+  const int rc = p_linear_i8_sparse24(ptr(*c.x), c.K, static_cast<const int8_t*>(ptr(*wc)), static_cast<const int32_t*>(ptr(*widx)),
+                                      c.sw_ptr(), c.bias_ptr(), c.y.data_ptr(), c.N, c.work_ptr(), c.M, static_cast<int>(c.N),
+                                      static_cast<int>(c.K), SAMFAST_BF16, stream_of(dev));
+  if (rc != SAMFAST_OK) Py_RETURN_NONE;
+  return THPVariable_Wrap(std::move(c.y));
+  END_HANDLE_TH_ERRORS
+}
+
+// attention(q, k, v, rel_h (B, nH, N, gh, 1), rel_w (B, nH, N, 1, gw), scale): attention with the
+// caller's bias factors, read through their strides; returns a contiguous (B, nH, N, hd) tensor
+PyObject* host_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 6) Py_RETURN_NONE;
+  const at::Tensor* t[5];
+  const c10::DeviceIndex dev = c10::hip::current_device();
+  for (int i = 0; i < 5; ++i) {
+    t[i] = tensor_arg(args[i]);
+    if (!t[i] || !on_current_gpu(*t[i], dev) || t[i]->dim() != (i < 3 ? 4 : 5) || t[i]->scalar_type() != t[0]->scalar_type()) Py_RETURN_NONE;
+    if (t[i]->requires_grad() && c10::GradMode::is_enabled()) Py_RETURN_NONE;
+  }
+  const at::Tensor &q = *t[0], &k = *t[1], &v = *t[2], &rh = *t[3], &rw = *t[4];
+  const int64_t B = q.size(0), nH = q.size(1), N = q.size(2), hd = q.size(3), gh = rh.size(3), gw = rw.size(4);
+  const bool half = q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf;
+  if (!half || k.sizes() != q.sizes() || v.sizes() != q.sizes() || B == 0 || B > INT32_MAX || nH > INT32_MAX || hd > 128 || gh > 64 || gw > 64 || gh * gw != N)
+    Py_RETURN_NONE;
+  for (const at::Tensor* b : {&rh, &rw})
+    if (b->size(0) != B || b->size(1) != nH || b->size(2) != N) Py_RETURN_NONE;
+  if (rh.size(4) != 1 || rw.size(3) != 1 || q.stride(3) != 1 || k.stride(3) != 1 || v.stride(3) != 1 || rh.stride(3) != 1 || rw.stride(4) != 1)
+    Py_RETURN_NONE;
+  const double scale = PyFloat_AsDouble(args[5]);
+  at::Tensor out = at::empty({B, nH, N, hd}, q.options().requires_grad(false));
+  const int rc = p_attn_bias(ptr(q), ptr(k), ptr(v), ptr(rh), ptr(rw), out.data_ptr(), static_cast<int>(B), static_cast<int>(nH),
+                             static_cast<int>(gh), static_cast<int>(gw), static_cast<int>(hd), q.stride(0), q.stride(1), q.stride(2),
+                             k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2), nH * N * hd, N * hd, hd,
+                             rh.stride(0), rh.stride(1), rh.stride(2), rw.stride(0), rw.stride(1), rw.stride(2),
+                             q.scalar_type() == at::kHalf ? SAMFAST_F16 : SAMFAST_BF16, static_cast<float>(scale), stream_of(dev));
+  if (rc != SAMFAST_OK) Py_RETURN_NONE;
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+// bind({name: address}): the C ABI functions used above
+PyObject* host_bind(PyObject*, PyObject* table) {
+  for (const Bound& b : kBound) {
+    PyObject* v = PyDict_GetItemString(table, b.name);  // borrowed
+    if (!v) return PyErr_Format(PyExc_KeyError, "samfast: %s is not in the table", b.name);
+    void* p = PyLong_AsVoidPtr(v);
+    if (!p) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_ValueError, "samfast: %s has no address", b.name);
+    *b.slot = p;
+  }
+  Py_RETURN_NONE;
+}
+
+PyObject* host_bound_names(PyObject*, PyObject*) {
+  PyObject* out = PyList_New(0);
+  for (const Bound& b : kBound) {
+    PyObject* s = PyUnicode_FromString(b.name);
+    PyList_Append(out, s);
+    Py_DECREF(s);
+  }
+  return out;
+}
+
+PyCFunction fastcall(PyObject* (*f)(PyObject*, PyObject* const*, Py_ssize_t)) {
+  return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f));
+}
+PyMethodDef kMethods[] = {
+    {"bind", host_bind, METH_O, nullptr},
+    {"bound_names", host_bound_names, METH_NOARGS, nullptr},
+    {"linear", fastcall(host_linear), METH_FASTCALL, nullptr},
+    {"sparse_linear", fastcall(host_sparse_linear), METH_FASTCALL, nullptr},
+    {"attention", fastcall(host_attention), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_samfast_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__samfast_host() { return PyModule_Create(&kModule); }

@@ -7,11 +7,14 @@ or a call fails, a RuntimeError carrying samfast_last_error() is raised.
 """
 
 import ctypes
+import importlib.util
 import os
 from pathlib import Path
 
 _LIB_PATH = Path(__file__).resolve().parent / "lib" / "libsamfast.so"
+_HOST_PATH = Path(__file__).resolve().parent / "lib" / "_samfast_host.so"
 _lib = None
+_host = None
 
 SAMFAST_BF16 = 0
 SAMFAST_F16 = 1  # attention entry points only
@@ -29,6 +32,9 @@ _SIGNATURES = {
     "samfast_attn_relpos_bias_fwd": (
         _i32, [_ptr] * 6 + [_i32] * 5 + [_i64] * 18 + [_i32, _f32, _ptr]),
     "samfast_quant_rowwise_i8": (_i32, [_ptr, _i64, _ptr, _ptr, _i64, _i32, _i32, _i32, _ptr]),
+    "samfast_linear_i8": (_i32, [_ptr, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _i32, _i32, _i32, _i32, _ptr]),
+    "samfast_linear_i8_sparse24": (_i32, [_ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _i32, _i32, _i32, _ptr]),
+    "samfast_linear_i8_workspace": (_i64, [_i64, _i32, _i32, _i32]),
     "samfast_gemm_i8_i32": (_i32, [_ptr, _ptr, _ptr, _i64, _i32, _i32, _ptr]),
     "samfast_gemm_i8_scale_bias": (
         _i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i32, _i32, _i32, _ptr]),
@@ -84,6 +90,23 @@ def load() -> ctypes.CDLL:
             fn.argtypes = argtypes
         _lib = lib
     return _lib
+
+
+def host():
+    """The native host module (csrc/host_torch.cpp), loaded once and pointed at the library."""
+    global _host
+    if _host is None:
+        if not _HOST_PATH.exists():
+            raise RuntimeError(
+                f"samfast: {_HOST_PATH} not found - build it with "
+                "`python segment-anything-fast_amd/build.py` (there is no fallback path)")
+        lib = load()
+        spec = importlib.util.spec_from_file_location("_samfast_host", str(_HOST_PATH))
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in mod.bound_names()})
+        _host = mod
+    return _host
 
 
 def check(code: int, what: str) -> None:

@@ -27,7 +27,7 @@ import os
 import torch
 import torch.nn.functional as F
 
-from . import ops
+from . import _lib, ops
 
 USE_CUSTOM_KERNEL = bool(int(os.environ.get("SEGMENT_ANYTHING_FAST_USE_FLASH_4", 1)))
 
@@ -86,6 +86,12 @@ def _attention_rel_h_rel_w(q_, k_, v_, rel_h_, rel_w_):
     """q_, k_, v_: (B, nH, N, hd); rel_h_: (B, nH, N, k_h, 1); rel_w_: (B, nH, N, 1, k_w).
     Returns (B, nH, N, hd) = softmax(q k^T / sqrt(hd) + rel_h + rel_w) v."""
     hd = q_.size(-1)
+    if USE_CUSTOM_KERNEL and q_.is_cuda and ops._launch_log is None:
+        # one native call on the factors as they are: the operator below wants them packed side by
+        # side (flash_4.py:352), a copy that costs an eighth of the attention itself
+        out = _lib.host().attention(q_, k_, v_, rel_h_, rel_w_, 1.0 / math.sqrt(hd))
+        if out is not None:
+            return out
     k_h, k_w = rel_h_.size(3), rel_w_.size(4)
     if _kernel_guards(q_, k_, v_) and ops.attn_supported(q_.size(-2), (k_h, k_w), hd, q_.dtype):
         sm_scale = 1.0 / math.sqrt(hd)

@@ -23,7 +23,7 @@ from typing import Callable, Optional
 import torch
 import torch.nn as nn
 
-from . import ops
+from . import _lib, ops
 from ._lib import EPILOGUE_NONE, LAYOUT_KB64, LAYOUT_ROWMAJOR
 from .tools import replace_with_custom_fn_if_matches_filter
 
@@ -135,9 +135,17 @@ class Int8LinearBase(nn.Module):
             yq, sy = ops.quant_rowwise(y, layout=out_layout)
         return y, yq, sy
 
+    def _forward_native(self, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """The whole Linear through the native host module; None for a call it does not cover."""
+        return None
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """The kernels compute on bf16 rows; any other floating input is cast on the way in and
         the result cast back, so the module keeps its input's dtype as nn.Linear does."""
+        if ops._launch_log is None and x.is_cuda:
+            y = self._forward_native(x)
+            if y is not None:
+                return y
         lead = x.shape[:-1]
         x2 = x.reshape(-1, self.in_features)
         if x2.dtype != torch.bfloat16:
@@ -171,12 +179,18 @@ class Int8DynamicLinear(Int8LinearBase):
                                  residual=residual, dst_row=dst_row, out=out, layout=layout)
 
     def _weight_for(self, layout: int) -> torch.Tensor:
+        wq = self._buffers["wq"]
         if layout != LAYOUT_KB64:
-            return self.wq
-        key = (self.wq.data_ptr(), self.wq._version, str(self.wq.device))
-        if self._wq_kb64 is None or self._wq_kb64_key != key:  # rebuilt after load_state_dict / .to()
-            self._wq_kb64, self._wq_kb64_key = ops.to_kb64(self.wq), key
+            return wq
+        key = self._wq_kb64_key  # rebuilt after load_state_dict / .to()
+        if key is None or key[0] is not wq or key[1] != wq.data_ptr() or key[2] != wq._version:
+            self._wq_kb64, self._wq_kb64_key = ops.to_kb64(wq), (wq, wq.data_ptr(), wq._version)
         return self._wq_kb64
+
+    def _forward_native(self, x: torch.Tensor) -> Optional[torch.Tensor]:
+        buffers = self._buffers
+        layout = LAYOUT_KB64 if self.in_features % 64 == 0 else LAYOUT_ROWMAJOR
+        return _lib.host().linear(x, self._weight_for(layout), layout, buffers["sw_bits"], buffers.get("bias_bits"))
 
     def linear_fused_quant(self, xq, sx, epilogue, residual=None, out=None, layout=LAYOUT_ROWMAJOR,
                            ln=None, out_layout=LAYOUT_ROWMAJOR):
