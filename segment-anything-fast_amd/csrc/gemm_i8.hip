@@ -50,6 +50,7 @@
 // counter back to zero for the next launch.  The other workgroup resident on the CU keeps the
 // matrix pipe busy meanwhile.
 #include "gemm_i8_shared.hpp"
+#include "linear_i8_small.hpp"
 #include "quant_row.hpp"
 #include <pthread.h>
 #include <stdlib.h>
@@ -995,6 +996,8 @@ static int gemm_common(int epi, const int8_t* xq, const float* sx, const int8_t*
   }
   const int64_t total = (int64_t)a.tiles_m * a.tiles_n;
   SF_REQUIRE(total < (1ll << 30), "gemm_i8: too many tiles");
+  // few rows: the K loop dealt out inside small tiles
+  if (!tail && epi == EPI_SCALE_BIAS_BF16 && gemm_i8_skinny_covers(a)) return gemm_i8_skinny_launch(a, stream);
   // resident workgroups that walk a list of tiles each (SAMFAST_GEMM_PERSIST=1), where built
   if (!tail && !generic_k && tm == 2 && gemm_i8_persist_covers(epi, a)) return gemm_i8_persist_launch(epi, a, stream);
   const unsigned int grid = (unsigned int)(((total + 7) / 8) * 8);
@@ -1162,6 +1165,7 @@ extern "C" int64_t samfast_linear_i8_workspace(int64_t M, int N, int K, int layo
   using namespace samfast;
   SF_REQUIRE(M > 0 && N > 0 && K > 0 && layout >= SAMFAST_LAYOUT_ROWMAJOR && layout <= SAMFAST_LAYOUT_SPARSE24,
              "linear_i8_workspace: bad shape M=%lld N=%d K=%d or layout %d", (long long)M, N, K, layout);
+  if (layout != SAMFAST_LAYOUT_SPARSE24 && linear_i8_small_covers(M, N, K)) return 0;
   // codes, then the row scales
   return ((M * K + 15) & ~(int64_t)15) + M * 4;
 }
@@ -1170,6 +1174,14 @@ extern "C" int samfast_linear_i8(const void* x, int64_t ldx, const int8_t* wq, c
                                  void* y, int64_t ldy, void* workspace, int64_t M, int N, int K, int dtype,
                                  int layout, void* stream) {
   using namespace samfast;
+  if (M > 0 && linear_i8_small_covers(M, N, K)) {
+    SF_REQUIRE(dtype == SAMFAST_BF16 && (layout == SAMFAST_LAYOUT_ROWMAJOR || layout == SAMFAST_LAYOUT_KB64),
+               "linear_i8: only bf16, weights row-major or K-block major");
+    SF_REQUIRE(x && wq && sw && y && aligned16(x) && aligned16(wq) && aligned16(y), "linear_i8: null or unaligned pointer");
+    SF_REQUIRE(ldx >= K && ldx % 8 == 0 && ldy >= N && ldy % 8 == 0, "linear_i8: row strides must be multiples of 8, >= K and >= N");
+    return linear_i8_small_launch(reinterpret_cast<const unsigned short*>(x), ldx, wq, sw, bias, reinterpret_cast<unsigned short*>(y), ldy,
+                                  (int)M, N, K, layout, reinterpret_cast<hipStream_t>(stream));
+  }
   SF_REQUIRE(M == 0 || (workspace && aligned16(workspace)), "linear_i8: the workspace must be non-null and 16-byte aligned");
   int8_t* xq = reinterpret_cast<int8_t*>(workspace);
   float* sx = reinterpret_cast<float*>(xq + ((M * K + 15) & ~(int64_t)15));

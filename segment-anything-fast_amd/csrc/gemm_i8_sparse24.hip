@@ -498,6 +498,7 @@ static int sparse_common(int epi, const int8_t* xq, const float* sx, const int8_
   a.group_x = a.tiles_w <= 6 ? 1 : 8;
   const int64_t total = (int64_t)a.tiles_x * a.tiles_w;
   SF_REQUIRE(total < (1ll << 30), "gemm_i8_sparse24: too many tiles");
+  if (gemm_i8_sp24_skinny_covers(epi, a)) return gemm_i8_sp24_skinny_launch(a, stream);
   if (gemm_i8_sp24_persist_covers(epi, a)) return gemm_i8_sp24_persist_launch(epi, a, stream);
   const unsigned int grid = (unsigned int)(((total + 7) / 8) * 8);
   switch (epi) {

@@ -52,4 +52,9 @@ SF_DEVICE int sp_slot_to_row(int slot) {
 bool gemm_i8_sp24_persist_covers(int epi, const SparseArgs& a);
 int gemm_i8_sp24_persist_launch(int epi, const SparseArgs& a, hipStream_t stream);
 
+// Small tiles with the K range dealt out over eight wavefronts (gemm_i8_sp24_skinny.hip): scale + bias
+// epilogue, few rows.  tiles_x / tiles_w are recomputed.
+bool gemm_i8_sp24_skinny_covers(int epi, const SparseArgs& a);
+int gemm_i8_sp24_skinny_launch(const SparseArgs& a, hipStream_t stream);
+
 }  // namespace samfast

@@ -1,0 +1,325 @@
+// A whole quantised Linear over a handful of rows in one launch: row quantiser, int8 product and
+// the scale + bias epilogue (what quant_rowwise.hip + gemm_i8.hip do in two).
+//
+// Such a call is latency: the two launches and their gap, a row's way through memory twice, and a
+// K loop that a 64 x 128 tile walks serially on a GPU it leaves empty.  Here a 512-thread workgroup
+// owns 16 * NT output columns and ALL rows (MT tiles of 16):
+//   * every wavefront first requests its share of the weight columns straight into registers (the K
+//     range is dealt out to the eight wavefronts in steps of 64, at most NCH each), so that the
+//     weights travel while the rows are quantised;
+//   * the workgroup quantises the rows itself - each workgroup repeats that for its own columns, which
+//     is why the form ends at a few dozen rows - and leaves the codes in LDS;
+//   * v_mfma_i32_16x16x64_i8, codes as A and weights as B (both take 16 consecutive k bytes of one
+//     row per lane), then the eight partial sums meet in LDS: integer sums, so the order is free
+//     and the results have the bits of the two-launch form.
+#include "gemm_i8_shared.hpp"
+#include "linear_i8_small.hpp"
+#include "quant_row.hpp"
+
+// every fp32 step below is rounded on its own (no fused multiply-add), as in the other forms
+#pragma clang fp contract(off)
+
+namespace samfast {
+
+struct SmallArgs {
+  const unsigned short* x;  // one launch: bf16 rows
+  int64_t ldx;
+  const int8_t* xq;         // product alone: codes, and their row scales
+  const float* sx;
+  const int8_t* w;
+  const float* sw;
+  const float* bias;
+  unsigned short* y;
+  int64_t ldy;
+  int M, N, K;
+  int row_pitch;     // bytes between consecutive weight rows: K, or 64 (K-block major)
+  int64_t w_kstep;   // bytes between consecutive 64-byte k steps: 64, or N * 64
+  int64_t x_kstep;
+  int tiles_m, tiles;  // product alone: row tiles, tiles
+};
+
+constexpr int kSmallWaves = 8;
+
+// The eight wavefronts' partial sums of a 16 MT x 16 NT tile meet in LDS ([wave][m][t][register][lane]; a
+// lane holds column lane % 16, rows 4 (lane / 16) + register of its 16 x 16 tiles) and leave through the
+// scale + bias epilogue, two adjacent columns of one row per thread.
+template <int MT, int NT, typename RowScale>
+SF_DEVICE void finish_tile(const SmallArgs& a, const i32x4 (&acc)[MT][NT], unsigned char* lds, int m0, int n0, int tid, RowScale row_scale) {
+  const int lane = tid & 63, wave = tid >> 6;
+  int* red = reinterpret_cast<int*>(lds);
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[((wave * MT + m) * NT + t) * 256 + r * 64 + lane] = acc[m][t][r];
+  __syncthreads();
+  for (int p = tid; p < MT * NT * 128; p += 64 * kSmallWaves) {
+    // consecutive threads: the column pairs of one row, then the next row
+    const int pair = p % (8 * NT), r = p / (8 * NT);
+    const int t = pair / 8, c = 2 * (pair % 8), m = r / 16, row16 = r % 16;
+    const int row = m0 + r, n = n0 + 16 * t + c;
+    if (row >= a.M || n >= a.N) continue;  // N % 8 == 0: a pair is in or out together
+    const int at = (m * NT + t) * 256 + (row16 & 3) * 64 + (row16 >> 2) * 16 + c;
+    int s0 = 0, s1 = 0;
+#pragma unroll
+    for (int w = 0; w < kSmallWaves; ++w) {
+      const u32x2 v = *reinterpret_cast<const u32x2*>(red + w * (MT * NT * 256) + at);
+      s0 += (int)v[0];
+      s1 += (int)v[1];
+    }
+    const float s = row_scale(row);
+    float b0 = 0.f, b1 = 0.f;
+    if (a.bias) { b0 = a.bias[n]; b1 = a.bias[n + 1]; }
+    float t0 = (float)s0 * s, t1 = (float)s1 * s;
+    t0 = t0 * a.sw[n];
+    t1 = t1 * a.sw[n + 1];
+    *reinterpret_cast<unsigned int*>(a.y + (int64_t)row * a.ldy + n) = pack_bf16x2(t0 + b0, t1 + b1);
+  }
+}
+
+template <int NCH, int RPW, int NT>  // RPW: rows per wavefront, so 8, 16 or 32 rows in all
+__global__ __launch_bounds__(64 * kSmallWaves, 2) void linear_i8_small_kernel(SmallArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  constexpr int MT = (RPW + 1) / 2, ROWS = 16 * MT;
+  float* sx = reinterpret_cast<float*>(lds);          // ROWS scales
+  unsigned char* codes = lds + ROWS * 4;              // ROWS x (K + 16) bytes; later the partial sums
+  const int pitch = a.K + 16;                         // an odd number of 16-byte pieces: operand reads spread over the banks
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = blockIdx.x * 16 * NT;
+  const int nk = a.K / 64;
+  const int lr = lane & 15, lq = lane >> 4;
+
+  // weights first: step wave + 8 i, columns n0 + 16 t + lr, k bytes 16 lq .. +15
+  i32x4 wf[NCH][NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int8_t* wrow = a.w + (int64_t)min(n0 + 16 * t + lr, a.N - 1) * a.row_pitch + 16 * lq;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int step = wave + kSmallWaves * i;
+      if (step < nk) wf[i][t] = *reinterpret_cast<const i32x4*>(wrow + step * a.w_kstep);  // uniform
+    }
+  }
+
+  // rows wave, wave + 8, ...: the arithmetic of RowQuantizer::finish_row, codes into LDS
+  const int nchunk = a.K / 8;
+  u32x4 xw[RPW][NCH];
+#pragma unroll
+  for (int j = 0; j < RPW; ++j) {
+    const int row = wave + kSmallWaves * j;
+    const u32x4* src = reinterpret_cast<const u32x4*>(a.x + row * a.ldx);
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const u32x4 z = {0u, 0u, 0u, 0u};
+      xw[j][i] = z;
+      if (row < a.M && lane + 64 * i < nchunk) xw[j][i] = src[lane + 64 * i];
+    }
+  }
+  // (rows at or past M hold zeros: they are quantised along, which keeps the rows' serial chains -
+  // maximum, lane reduction, two divisions - independent and in flight together)
+  float amax[RPW], scale[RPW], inv_scale[RPW];
+#pragma unroll
+  for (int j = 0; j < RPW; ++j) {
+    amax[j] = 0.f;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        amax[j] = fmaxf(amax[j], fmaxf(fabsf(bf16_lo_to_f32(xw[j][i][e])), fabsf(bf16_hi_to_f32(xw[j][i][e]))));
+  }
+#pragma unroll
+  for (int j = 0; j < RPW; ++j) amax[j] = wave_max_nonneg(amax[j]);
+#pragma unroll
+  for (int j = 0; j < RPW; ++j) {
+    scale[j] = fmaxf(amax[j], 1e-5f) / 127.0f;
+    inv_scale[j] = 1.0f / scale[j];
+  }
+#pragma unroll
+  for (int j = 0; j < RPW; ++j) {
+    const int row = wave + kSmallWaves * j;
+    bool saw_nan = false;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i)
+      if (lane + 64 * i < nchunk) {
+        float f[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          f[2 * e] = bf16_lo_to_f32(xw[j][i][e]);
+          f[2 * e + 1] = bf16_hi_to_f32(xw[j][i][e]);
+        }
+        unsigned int c[2];
+        saw_nan |= quantize_chunk<8>(f, scale[j], inv_scale[j], c);
+        const u32x2 o = {c[0], c[1]};
+        *reinterpret_cast<u32x2*>(codes + row * pitch + (lane + 64 * i) * 8) = o;
+      }
+    const bool row_nan = __any(saw_nan);
+    if (lane == 0) sx[row] = row_nan ? __uint_as_float(0x7fc00000u) : scale[j];
+  }
+  __syncthreads();
+
+  i32x4 acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[m][t] = i32x4{0, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int step = wave + kSmallWaves * i;
+    if (step < nk) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const i32x4 xf = *reinterpret_cast<const i32x4*>(codes + (16 * m + lr) * pitch + step * 64 + 16 * lq);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[m][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xf, wf[i][t], acc[m][t], 0, 0, 0);
+      }
+    }
+  }
+
+  __syncthreads();  // nobody reads the codes any more
+  finish_tile<MT, NT>(a, acc, codes, 0, n0, tid, [&](int row) { return sx[row]; });
+}
+
+// The product alone, on codes that a quantiser launch has written: the same dealing of the K range over
+// eight wavefronts for launches whose 64 x 128 tiles would leave most CUs empty and walk K serially.
+// A workgroup owns 16 MT rows x 16 NT columns; both operands go from memory into registers (K-block major:
+// 1 KB of whole lines per load), DEPTH steps ahead.
+template <int MT, int NT>
+__global__ __launch_bounds__(64 * kSmallWaves, 2) void gemm_i8_skinny_kernel(SmallArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  constexpr int DEPTH = MT + NT <= 4 ? 4 : MT + NT <= 6 ? 3 : 2;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lq = lane >> 4;
+  // row tiles of one column panel next to each other on an XCD: the weights are the larger operand
+  const unsigned int pid = xcd_contiguous_id(blockIdx.x, a.tiles);
+  if (pid >= (unsigned int)a.tiles) return;  // uniform
+  const int m0 = (int)(pid % a.tiles_m) * 16 * MT, n0 = (int)(pid / a.tiles_m) * 16 * NT;
+  const int8_t* xrow[MT];
+  const int8_t* wrow[NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) xrow[m] = a.xq + (int64_t)min(m0 + 16 * m + lr, a.M - 1) * a.row_pitch + 16 * lq;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) wrow[t] = a.w + (int64_t)min(n0 + 16 * t + lr, a.N - 1) * a.row_pitch + 16 * lq;
+  const int nk = a.K / 64;
+  const int steps = (nk - wave + kSmallWaves - 1) / kSmallWaves;  // 0 for the last wavefronts of a short K
+
+  i32x4 xf[DEPTH][MT], wf[DEPTH][NT];
+  auto request = [&](int i, int d) {
+    const int64_t step = wave + kSmallWaves * i;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) wf[d][t] = *reinterpret_cast<const i32x4*>(wrow[t] + step * a.w_kstep);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) xf[d][m] = *reinterpret_cast<const i32x4*>(xrow[m] + step * a.x_kstep);
+  };
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d)
+    if (d < steps) request(d, d);
+  i32x4 acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[m][t] = i32x4{0, 0, 0, 0};
+  for (int i = 0; i < steps; i += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+      if (i + d < steps) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) acc[m][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xf[d][m], wf[d][t], acc[m][t], 0, 0, 0);
+        if (i + d + DEPTH < steps) request(i + d + DEPTH, d);
+      }
+  }
+  finish_tile<MT, NT>(a, acc, lds, m0, n0, tid, [&](int row) { return a.sx[row]; });
+}
+
+bool linear_i8_small_covers(int64_t M, int N, int K) {
+  if (knob_or(KNOB_LINEAR_SMALL, 1) <= 0 || K % 64 != 0 || N % 8 != 0 || K > 5120) return false;
+  // every workgroup quantises every row, 0.3 us per 8 rows of 1280: past these lines the separate quantiser
+  // and the small-tile product take less GPU time than the repetition (16 x 3072: 9.1 us against 8.6), below
+  // them one launch also saves the host the second one (7 x 256 -> 2048: 5.5 us a call against 8.7)
+  return M <= 8 || (M <= 16 && K <= 2048) || (M <= 32 && K <= 768);
+}
+
+template <int NCH, int RPW, int NT>
+static int launch_small(const SmallArgs& a, hipStream_t stream) {
+  constexpr int MT = (RPW + 1) / 2;
+  const int codes = 16 * MT * (a.K + 16), red = kSmallWaves * MT * NT * 1024;
+  const size_t lds = 16 * MT * 4 + (codes > red ? codes : red);
+  hipLaunchKernelGGL((linear_i8_small_kernel<NCH, RPW, NT>), dim3((a.N + 16 * NT - 1) / (16 * NT)), dim3(64 * kSmallWaves), lds, stream, a);
+  return check_launch("linear_i8_small_kernel");
+}
+
+int linear_i8_small_launch(const unsigned short* x, int64_t ldx, const int8_t* wq, const float* sw, const float* bias, unsigned short* y,
+                           int64_t ldy, int M, int N, int K, int layout, hipStream_t stream) {
+  SmallArgs a = {};
+  a.x = x; a.ldx = ldx; a.w = wq; a.sw = sw; a.bias = bias; a.y = y; a.ldy = ldy; a.M = M; a.N = N; a.K = K;
+  const bool kb = layout == SAMFAST_LAYOUT_KB64;
+  a.row_pitch = kb ? 64 : K;
+  a.w_kstep = kb ? (int64_t)N * 64 : 64;
+  // two column tiles per workgroup once single ones are more than the GPU has CUs: half the repeated
+  // row work for the same number of rounds
+  const bool wide = N > 16 * 256;
+  auto by_rows = [&](auto nch) {
+    constexpr int NCH = decltype(nch)::value;
+    if (M <= 8) return wide ? launch_small<NCH, 1, 2>(a, stream) : launch_small<NCH, 1, 1>(a, stream);
+    if (M <= 16) return wide ? launch_small<NCH, 2, 2>(a, stream) : launch_small<NCH, 2, 1>(a, stream);
+    if constexpr (NCH <= 2) return wide ? launch_small<NCH, 4, 2>(a, stream) : launch_small<NCH, 4, 1>(a, stream);
+    set_error("linear_i8_small: %d rows of %d values are not covered", M, K);
+    return (int)SAMFAST_E_UNSUPPORTED;
+  };
+  if (K <= 512) return by_rows(std::integral_constant<int, 1>{});
+  if (K <= 1024) return by_rows(std::integral_constant<int, 2>{});
+  if (K <= 1536) return by_rows(std::integral_constant<int, 3>{});
+  if (K <= 2048) return by_rows(std::integral_constant<int, 4>{});
+  if (K <= 3072) return by_rows(std::integral_constant<int, 6>{});
+  if (K <= 4096) return by_rows(std::integral_constant<int, 8>{});
+  return by_rows(std::integral_constant<int, 10>{});
+}
+
+// The smallest tile whose tiles still fit the GPU's CUs once: a smaller tile means a shorter chain, a second
+// round costs more than that gains.  Measured on K-block major codes, us, against the tiled kernels:
+// 128 x 3840 x 1280 in 64 x 32 tiles 4.7 (6.3), 64 x 1280 x 5120 in 16 x 32 5.6 (14.6), 512 x 1280 x 5120 in
+// 64 x 64 12.8 (21.9); the largest tile only pays on a long K loop (512 x 1280 x 1280: 6.3 against 6.4).
+// Returns 16-row tiles * 8 + 16-column tiles, 0 = none.
+static int skinny_shape(int M, int N, int K) {
+  auto fits = [&](int mt, int nt) { return (int64_t)((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * nt - 1) / (16 * nt)) <= 256; };
+  if (fits(1, 1)) return 1 * 8 + 1;
+  if (fits(1, 2)) return 1 * 8 + 2;
+  if (fits(2, 2)) return 2 * 8 + 2;
+  if (fits(4, 2)) return 4 * 8 + 2;
+  if (K >= 2048 && fits(4, 4)) return 4 * 8 + 4;
+  return 0;
+}
+
+bool gemm_i8_skinny_covers(const GemmArgs& a) {
+  return knob_or(KNOB_GEMM_SKINNY, 1) > 0 && skinny_shape(a.M, a.N, a.K) != 0;
+}
+
+template <int MT, int NT>
+static int launch_skinny(SmallArgs a, hipStream_t stream) {
+  a.tiles_m = (a.M + 16 * MT - 1) / (16 * MT);
+  a.tiles = a.tiles_m * ((a.N + 16 * NT - 1) / (16 * NT));
+  const unsigned int grid = (unsigned int)((a.tiles + 7) / 8 * 8);
+  hipLaunchKernelGGL((gemm_i8_skinny_kernel<MT, NT>), dim3(grid), dim3(64 * kSmallWaves), kSmallWaves * MT * NT * 1024, stream, a);
+  return check_launch("gemm_i8_skinny_kernel");
+}
+
+int gemm_i8_skinny_launch(const GemmArgs& g, hipStream_t stream) {
+  SmallArgs a = {};
+  a.xq = g.x; a.sx = g.sx; a.w = g.w; a.sw = g.sw; a.bias = g.bias;
+  a.y = reinterpret_cast<unsigned short*>(g.out);
+  a.ldy = g.ldo; a.M = g.M; a.N = g.N; a.K = g.K;
+  a.row_pitch = g.row_pitch; a.x_kstep = g.x_kstep; a.w_kstep = g.w_kstep;
+  switch (skinny_shape(a.M, a.N, a.K)) {
+    case 1 * 8 + 1: return launch_skinny<1, 1>(a, stream);
+    case 1 * 8 + 2: return launch_skinny<1, 2>(a, stream);
+    case 2 * 8 + 2: return launch_skinny<2, 2>(a, stream);
+    case 4 * 8 + 2: return launch_skinny<4, 2>(a, stream);
+    default: return launch_skinny<4, 4>(a, stream);
+  }
+}
+
+}  // namespace samfast

@@ -33,6 +33,8 @@ enum Knob {
   KNOB_GEMM_PERSIST_SKEW, // SAMFAST_GEMM_PERSIST_SKEW: start delay of every second resident workgroup, 64 cycles per k tile
   KNOB_GEMM_PERSIST_PRIO, // SAMFAST_GEMM_PERSIST_PRIO: 0 = no wave priority changes in the persistent kernel
   KNOB_GEMM_SPLITK,       // SAMFAST_GEMM_SPLITK: 0 off, 1 where it pays (launches that leave the GPU half empty)
+  KNOB_LINEAR_SMALL,      // SAMFAST_GEMM_LINEAR_SMALL: 0 = whole Linears over few rows as two launches as well
+  KNOB_GEMM_SKINNY,       // SAMFAST_GEMM_SKINNY: 0 = products over few rows through the tiled kernels
   KNOB_ATTN_WAVES,        // SAMFAST_ATTN_WAVES: 4 / 8 wavefronts per global-attention workgroup
   KNOB_ATTN_WINDOW_ROWS,  // SAMFAST_ATTN_WINDOW_ROWS: 1 = window keys as grid rows padded to 16 (attn_window_rows_kernel) where built
   KNOB_SPARSE_PERSIST,    // SAMFAST_SPARSE_PERSIST: 2:4 GEMM, 0 = one workgroup per tile (default), 1 = resident workgroups from two tiles each on, 2 wherever built
