@@ -311,6 +311,19 @@ int samfast_gemm_i8_sparse24_fused(
     int64_t M, int N, int K, int dtype, int epilogue,
     const void* residual, int64_t ld_res, int layout, void* stream);
 
+/*
+ * Row-wise glue of a block with half-type Linears (modeling/image_encoder.py:167-183):
+ *   samfast_layernorm  out = LayerNorm(x) over rows of K values; with r / sum given, sum = x + r (rounded
+ *                      to the element type; may alias x or r) and out = LayerNorm(sum): `shortcut + x`
+ *                      with the norm that follows.  fp32 statistics, biased variance.  Contiguous rows,
+ *                      K % 8 == 0, K <= 4096.
+ *   samfast_gelu       y = gelu_erf(x), n values (a multiple of 8); y may be x.
+ */
+int samfast_layernorm(
+    const void* x, const void* r, const void* gamma, const void* beta, float eps,
+    void* sum, void* out, int64_t M, int K, int dtype, void* stream);
+int samfast_gelu(const void* x, void* y, int64_t n, int dtype, void* stream);
+
 /* samfast_linear_i8 with the weight in the packed 2:4 form. */
 int samfast_linear_i8_sparse24(
     const void* x, int64_t ldx, const int8_t* wc, const int32_t* widx, const float* sw,

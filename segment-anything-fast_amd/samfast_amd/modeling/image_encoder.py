@@ -111,7 +111,12 @@ class ImageEncoderViT(nn.Module):
         carry = None
         for i, blk in enumerate(self.blocks):
             if not blk._int8_fused_ok(x):
-                x, carry = blk(x), None
+                if not blk._half_fused_ok(x):
+                    x, carry = blk(x), None
+                    continue
+                nxt = self.blocks[i + 1] if i + 1 < len(self.blocks) else None
+                chained = nxt is not None and not nxt._int8_fused_ok(x) and nxt._half_fused_ok(x)
+                x, carry = blk._forward_half_fused(x, carry, nxt.norm1 if chained else None)
                 continue
             nxt = self.blocks[i + 1] if i + 1 < len(self.blocks) else None
             next_norm = None
@@ -257,9 +262,68 @@ class Block(nn.Module):
         tokens = mlp.lin2.linear_fused(gq, sg, _lib.EPILOGUE_RESIDUAL, residual=tokens, out=tokens, layout=L)
         return tokens.view(B, H, W, C), None
 
+    def _half_fused_ok(self, x: torch.Tensor) -> bool:
+        """Whether this block, its Linears left in the half type, can run through _forward_half_fused:
+        inference on a GPU in bf16 / fp16 at a shape the attention kernels cover, the modules the
+        ones the constructor built (nobody has put a hook or another class in their place)."""
+        attn, mlp = self.attn, self.mlp
+        if not (FUSED_BLOCK and flash_4.USE_CUSTOM_KERNEL and x.is_cuda and x.dim() == 4
+                and x.dtype in (torch.bfloat16, torch.float16) and attn.use_rel_pos and not torch.is_grad_enabled()):
+            return False
+        if not (type(self.norm1) is nn.LayerNorm and type(self.norm2) is nn.LayerNorm and type(attn) is Attention
+                and type(mlp) is MLPBlock and type(mlp.act) is nn.GELU and mlp.act.approximate == "none"
+                and all(type(m) is nn.Linear for m in (attn.qkv, attn.proj, mlp.lin1, mlp.lin2))):
+            return False
+        B, H, W, C = x.shape
+        for n in (self.norm1, self.norm2):
+            if n.weight is None or n.bias is None or n.weight.dtype != x.dtype or n.normalized_shape != (C,):
+                return False
+        if any(m._forward_hooks or m._forward_pre_hooks for m in (self.norm1, attn, attn.qkv, attn.proj, self.norm2,
+                                                                  mlp, mlp.lin1, mlp.act, mlp.lin2)):
+            return False
+        ws = self.window_size
+        gh, gw = (ws, ws) if ws > 0 else (H, W)
+        return (attn.qkv.weight.dtype == x.dtype and C % 8 == 0 and C <= 4096 and mlp.lin1.out_features % 8 == 0
+                and attn.rel_pos_h.dtype == x.dtype and attn.rel_pos_w.dtype == x.dtype
+                and attn.rel_pos_h.shape[0] == 2 * gh - 1 and attn.rel_pos_w.shape[0] == 2 * gw - 1
+                and ops.attn_supported(gh * gw, (gh, gw), C // attn.num_heads, x.dtype)
+                and (ws == 0 or ws * ws <= 208))
+
+    def _forward_half_fused(self, x: torch.Tensor, carry=None, next_norm=None):
+        """image_encoder.py:167-183 with half-type Linears: the four library products plus four
+        launches.  The attention kernel cuts the windows out of the image-ordered tokens, so the
+        products run on the image's tokens only (the zero-padded windows have a fifth more) and nothing
+        is partitioned, padded or copied; each residual add runs with the norm that follows it.
+        `carry`: norm1's output, where the previous block has made it; `next_norm`: the next block's norm1.
+        Returns (tokens, carry for the next block)."""
+        B, H, W, C = x.shape
+        attn, mlp, ws = self.attn, self.mlp, self.window_size
+        nH = attn.num_heads
+        hd = C // nH
+        tokens = x.contiguous().view(B * H * W, C)
+        h = carry if carry is not None else ops.layernorm(tokens, self.norm1.weight, self.norm1.bias, self.norm1.eps)
+        qkv = attn.qkv(h).view(B, H * W, 3, nH, hd)
+        q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
+        if ws > 0:
+            # a zero-padded token's k and v rows: the qkv bias
+            pads = (torch.zeros((2, nH, hd), dtype=x.dtype, device=x.device) if attn.qkv.bias is None
+                    else attn.qkv.bias[C:].view(2, nH, hd))
+            o = ops.attn_relpos_windowed(q, k, v, attn.rel_pos_h, attn.rel_pos_w, pads[0], pads[1], (H, W), ws, attn.scale)
+        else:
+            o = ops.attn_relpos(q, k, v, attn.rel_pos_h, attn.rel_pos_w, (H, W), attn.scale).permute(0, 2, 1, 3)
+        o = attn.proj(o.reshape(B * H * W, C))
+        tokens, h = ops.layernorm(tokens, self.norm2.weight, self.norm2.bias, self.norm2.eps, add=o)
+        m = mlp.lin2(ops.gelu_(mlp.lin1(h)))
+        if next_norm is None:
+            return tokens.add_(m).view(B, H, W, C), None
+        tokens, h = ops.layernorm(tokens, next_norm.weight, next_norm.bias, next_norm.eps, add=m)
+        return tokens.view(B, H, W, C), h
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self._int8_fused_ok(x):
             return self._forward_int8_fused(x)[0]
+        if self._half_fused_ok(x):
+            return self._forward_half_fused(x)[0]
         shortcut = x
         x = self.norm1(x)
         if self.window_size > 0:

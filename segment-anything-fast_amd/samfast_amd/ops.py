@@ -549,6 +549,42 @@ def gemm_i8_sparse24_fused(xq: torch.Tensor, sx: torch.Tensor, wc: torch.Tensor,
     return out
 
 
+def layernorm(x: torch.Tensor, gamma: torch.Tensor, beta: torch.Tensor, eps: float,
+              add: Optional[torch.Tensor] = None):
+    """LayerNorm over the last axis of contiguous half-type rows.  With `add`: (x + add, its LayerNorm)
+    in one launch."""
+    _require_gpu(x, gamma, beta, add)
+    K = x.shape[-1]
+    for t in (gamma, beta):
+        if t.dtype != x.dtype or t.numel() != K or not t.is_contiguous():
+            raise RuntimeError("samfast: gamma / beta must match x in dtype and length K")
+    if not x.is_contiguous() or (add is not None and (add.shape != x.shape or add.dtype != x.dtype or not add.is_contiguous())):
+        raise RuntimeError("samfast: layernorm needs contiguous rows, and `add` of the same shape and dtype")
+    out = torch.empty_like(x)
+    total = torch.empty_like(x) if add is not None else None
+    M = x.numel() // K if K else 0
+    lib = _lib.load()
+    code = _timed(
+        "layernorm", (8.0 if add is not None else 4.0) * M * K, "byte",
+        lambda: lib.samfast_layernorm(
+            x.data_ptr(), add.data_ptr() if add is not None else None, gamma.data_ptr(), beta.data_ptr(), float(eps),
+            total.data_ptr() if add is not None else None, out.data_ptr(), M, K, _dtype_code(x), _stream()))
+    _lib.check(code, "layernorm")
+    return out if add is None else (total, out)
+
+
+def gelu_(x: torch.Tensor) -> torch.Tensor:
+    """Exact-erf GELU of a contiguous half-type tensor, in place."""
+    _require_gpu(x)
+    if not x.is_contiguous():
+        raise RuntimeError("samfast: gelu_ needs a contiguous tensor")
+    lib = _lib.load()
+    code = _timed("gelu", 4.0 * x.numel(), "byte",
+                  lambda: lib.samfast_gelu(x.data_ptr(), x.data_ptr(), x.numel(), _dtype_code(x), _stream()))
+    _lib.check(code, "gelu")
+    return x
+
+
 _window_maps = {}
 
 
