@@ -1,0 +1,689 @@
+// Global attention (64-wide key grid) with caller-computed bias factors.
+//
+// The mathematics of attn_global_kernel (attn_relpos.hip) - S^T = K Q^T by 32x32x16 MFMAs with rel_w as the initial
+// accumulator, rel_h one scalar per (query, key row), base-2 softmax, O^T = V^T P^T on transposing LDS reads -
+// on a loop that is pipelined inside a wavefront: between the exponentials of one half row of keys stand the
+// matrix instructions of the next half row's scores and of the previous one's P V, and the LDS reads that feed
+// them.  No running maximum is taken in the common case, LDS reads meet no bank twice (GridRow), and the
+// workgroups of a head touch its K and V ahead, so that the rows come out of their XCD's L2.
+//   Bound: at 8 x 16 x 4096 x 80 (745 us, 920 TFLOP/s; 805 us with attn_global_kernel) the power limit: the same
+//   loop with its MFMAs alone, on the same values, takes 666 us - 429 on zeros.  At one image of 12 heads
+//   (65 us against 83) the last, half-empty round and the prologue.
+//   (The encoder, which hands over tables, keeps attn_global_kernel: its int8 Linears turn any other order of these
+//   roundings into other codes.)
+//
+// Two kernels.  attn_global_bias_kernel: a wavefront owns 32 queries and walks whole key rows; workgroups of 8 (one
+// per CU: every row staged once for 256 queries) or 4 wavefronts (two per CU).  attn_global_split_kernel: the keys
+// of every row are split between two wavefronts, whose results (maximum reference, denominator, output) meet in
+// LDS once, at the end; workgroups of two query tiles x two key halves (64 queries, under 54 KB of LDS), three per CU
+// at hd 64, so that one image's 12 heads are 768 workgroups: three on each of the 256 CUs, where 128-query
+// workgroups leave half of the CUs with one and half with two.  bias_form picks.
+#include "attn_relpos_shared.hpp"
+
+namespace samfast {
+
+template <int HD, int WAVES>
+struct BiasCfg : GridRow<HD> {
+  using R = GridRow<HD>;
+  static constexpr int BM = 32 * WAVES;       // queries per workgroup
+  static constexpr int KDPW = (R::KP + WAVES - 1) / WAVES, VDPW = (R::VP + WAVES - 1) / WAVES;  // wave instructions per tile a wave issues at most
+  // LDS: two K tiles, three V tiles (a row's V is still read while the next row's has to be there), rel_h
+  static constexpr int V_OFF = 2 * R::KTILE;
+  static constexpr int RH = 32;               // key rows whose rel_h is at hand
+  static constexpr int RELH_OFF = V_OFF + 3 * R::VTILE;
+  static constexpr int LDS_BYTES = RELH_OFF + RH * BM * 4;
+  static_assert(LDS_BYTES <= (WAVES == 4 ? 80 : 160) * 1024, "workgroups per CU");
+};
+
+template <typename T, int HD, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArgs a) {
+  using C = BiasCfg<HD, WAVES>;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS_BYTES];
+  float* relhT = reinterpret_cast<float*>(lds + C::RELH_OFF);  // [kh % RH][BM], * log2(e); a wave reads only its own columns
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 31, lh = lane >> 5;
+
+  const unsigned int nqb = a.N / C::BM;
+  const unsigned int total = (unsigned int)(a.B * a.nH) * nqb;
+  const unsigned int pid = xcd_contiguous_id(blockIdx.x, total);
+  if (pid >= total) return;
+  const int bh = pid / nqb, qb = pid % nqb;
+  const int b = bh / a.nH, h = bh % a.nH;
+  const int q0 = qb * C::BM + 32 * wave;  // the wavefront's first query: half of one grid row
+
+  const unsigned short* kbase = a.k + b * a.k_sb + h * a.k_sh;
+  const unsigned short* vbase = a.v + b * a.v_sb + h * a.v_sh;
+
+  // ---- K / V rows: global memory -> LDS directly, wave instruction i of a tile fills pieces 64 i .. 64 i + 63 ----
+  unsigned int koff[C::KDPW];  // bytes, from the tile's first key row; unsigned: scalar-base load form
+  int voff[C::VDPW];           // negative: a spare piece, the lane loads nothing
+#pragma unroll
+  for (int m = 0; m < C::KDPW; ++m) {
+    int row;
+    const int at = C::k_source(64 * (wave + WAVES * m) + lane, row);
+    koff[m] = (unsigned int)(row * (int)a.k_sn) * 2u + at;
+  }
+#pragma unroll
+  for (int m = 0; m < C::VDPW; ++m) {
+    int row;
+    const int at = C::v_source(64 * (wave + WAVES * m) + lane, row);
+    voff[m] = at < 0 ? -1 : row * (int)a.v_sn * 2 + at;
+  }
+  const unsigned int lds_base = (unsigned int)(uintptr_t)((__attribute__((address_space(3))) unsigned char*)lds);
+  auto k_dma = [&](int kt, int buf) __attribute__((always_inline)) {
+    const unsigned char* src = reinterpret_cast<const unsigned char*>(kbase + (int64_t)kt * 64 * a.k_sn);
+#pragma unroll
+    for (int m = 0; m < C::KDPW; ++m)
+      if (wave + WAVES * m < C::KP) lds_dma16(src, koff[m], lds_base + buf * C::KTILE + (wave + WAVES * m) * 1024);
+  };
+  auto v_dma = [&](int kt, unsigned int buf_off) __attribute__((always_inline)) {
+    const unsigned char* src = reinterpret_cast<const unsigned char*>(vbase + (int64_t)kt * 64 * a.v_sn);
+#pragma unroll
+    for (int m = 0; m < C::VDPW; ++m)
+      if (wave + WAVES * m < C::VP && (!C::ONES_ROW || voff[m] >= 0))
+        lds_dma16(src, (unsigned int)voff[m], lds_base + C::V_OFF + buf_off + (wave + WAVES * m) * 1024);
+  };
+  k_dma(0, 0);
+  v_dma(0, 0);
+  k_dma(1, 1);  // N % 128 == 0: at least two key rows
+  v_dma(1, C::VTILE);
+
+  // ---- Q^T operand: query lr, channels 16s + 8lh .. +7 ----
+  u32x4 qf[C::KS];
+  {
+    const unsigned short* qp = a.q + b * a.q_sb + h * a.q_sh + (int64_t)(q0 + lr) * a.q_sn + 8 * lh;
+#pragma unroll
+    for (int s = 0; s < C::KS; ++s) qf[s] = load_x8_global(qp + 16 * s);
+  }
+  // The workgroups of a head walk its key rows in step, so every row would be waited for at the latency of
+  // the Infinity Cache or HBM.  Each of them touches its own share of the head's K and V first: together
+  // they have the head in their XCD's L2 by the time they get to it.
+  constexpr int NTOUCH = 2 * C::BM * (HD / 8) / (64 * WAVES);
+  unsigned int touched[NTOUCH];
+#pragma unroll
+  for (int i = 0; i < NTOUCH; ++i) {
+    const int P = (tid + 64 * WAVES * i) % (C::BM * (HD / 8)), row = P / (HD / 8), col = P % (HD / 8);
+    const bool is_v = 2 * i >= NTOUCH;
+    touched[i] = *reinterpret_cast<const unsigned int*>((is_v ? vbase : kbase) + (int64_t)(qb * C::BM + row) * (is_v ? a.v_sn : a.k_sn) + col * 8);
+  }
+
+  // V^T operand of the P V product through transposing LDS reads (ds_read_b64_tr_b16): in
+  // each group of 16 lanes, lane l receives as element j the l%4-th 16-bit value of the 8
+  // bytes addressed by lane 4j + l/4 of the group.  Source lane 4j + i therefore points at
+  // key j of the lane half's four keys, channels 4i .. 4i+3 of the group's 16 channels, and
+  // lane l ends up with channel l of four consecutive keys: the MFMA A operand.
+  int vrd[C::DT], krd[C::KS];
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt) vrd[dt] = C::V_OFF + C::v_read(lane, dt);
+#pragma unroll
+  for (int ks = 0; ks < C::KS; ++ks) krd[ks] = C::k_read(lr, lh, ks);
+  // the spare pieces of the three V tiles: (1, 0, ..) and zeros
+  auto ones = [&]() __attribute__((always_inline)) {
+    if (C::ONES_ROW)
+      for (int r = tid; r < 192; r += 64 * WAVES) {
+        u32x4* p = reinterpret_cast<u32x4*>(lds + C::V_OFF + r * (C::VP * 16) + HD * 2);
+        p[0] = u32x4{T::kOne, 0u, 0u, 0u};
+        p[1] = u32x4{0u, 0u, 0u, 0u};
+      }
+  };
+  ones();
+
+  // ---- bias: rel_w / sm_scale of the lane's query is the initial accumulator of the score tiles of the two
+  //      half rows; rel_h * log2(e) stands in LDS, 32 key rows at a time ----
+  auto fill_relh = [&](int kh0) __attribute__((always_inline)) {
+    // lane: query lr, key rows kh0 + 16 lh .. +15
+    const unsigned short* src = a.rh + b * a.rh_sb + h * a.rh_sh + (int64_t)(q0 + lr) * a.rh_sn + kh0 + 16 * lh;
+    unsigned short v[16];
+    if (a.relh_x8) {
+      *reinterpret_cast<u32x4*>(v) = load_x8_global(src);
+      *reinterpret_cast<u32x4*>(v + 8) = load_x8_global(src + 8);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) v[e] = kh0 + 16 * lh + e < a.gh ? src[e] : (unsigned short)0;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) relhT[(16 * lh + e) * C::BM + 32 * wave + lr] = T::from_bits(v[e]) * kLog2e;
+  };
+  f32x16 b1[2];
+  fill_relh(0);
+  {
+    const unsigned short* rwp = a.rw + b * a.rw_sb + h * a.rw_sh + (int64_t)(q0 + lr) * a.rw_sn + 4 * lh;
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const u32x2 w = *reinterpret_cast<const u32x2*>(rwp + 32 * half + 8 * j);
+        b1[half][4 * j + 0] = T::lo(w[0]) * a.inv_scale;
+        b1[half][4 * j + 1] = T::hi(w[0]) * a.inv_scale;
+        b1[half][4 * j + 2] = T::lo(w[1]) * a.inv_scale;
+        b1[half][4 * j + 3] = T::hi(w[1]) * a.inv_scale;
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < NTOUCH; ++i) asm volatile("" : : "v"(touched[i]));
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of the first two rows has landed
+  __syncthreads();
+
+  // ---- main loop over half rows of 32 keys ----
+  f32x16 oacc[C::DT];
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
+  float m_i = -INFINITY, l_i = 0.f;
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4* trptr_t;
+
+  // The loop is pipelined inside a wavefront, instruction by instruction: between the exponentials of half row
+  // i stand the matrix instructions of the scores of half row i + 1 and of P V of half row i - 1, and the
+  // LDS reads that feed them, so that none of the three pipes waits for another's burst.
+  u32x4 kf[C::KS], vf[2][C::DT], pkA[2], pkB[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    pkA[j] = pkB[j] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int dt = 0; dt < C::DT; ++dt) vf[j][dt] = u32x4{0u, 0u, 0u, 0u};
+  }
+  auto read_v = [&](int j, int dt, unsigned int v_off) __attribute__((always_inline)) {
+    const unsigned char* p = lds + v_off + vrd[dt] + 16 * j * (C::VP * 16);
+    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((trptr_t)p));
+    const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((trptr_t)(p + 8 * C::VP * 16)));
+    vf[j][dt] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+  };
+  // s, pk: scores and probabilities of this half row, its V at v_off, rel_h of its row b0; s_next: scores of the
+  // next one, from K at k_off with the initial accumulator b_next; pk_prev, v_prev: the one before
+  auto half_row = [&](f32x16& s, f32x16& s_next, u32x4 (&pk)[2], u32x4 (&pk_prev)[2], const f32x16& b_next, int k_off, unsigned int v_off,
+                      unsigned int v_prev, float b0, bool has_prev) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < C::KS; ++ks) kf[ks] = *reinterpret_cast<const u32x4*>(lds + krd[ks] + k_off);
+    if (has_prev) {  // (before the first half row: the zeros above, with probabilities of zero)
+#pragma unroll
+      for (int dt = 0; dt < C::DT; ++dt) read_v(1, dt, v_prev);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // online softmax, one query per lane.  The exponent offset m_i is a reference, not the running
+    // maximum: probabilities may sit anywhere below 2 (the final division by the denominator,
+    // accumulated with the same offsets, makes the result independent of it), so no maximum is taken in
+    // the common case.  Whether one has reached 2 shows in the top exponent bit of the packed pairs,
+    // or-ed together.  Then - always in the first half row, where m_i is -inf, and again when the maximum has
+    // grown by T::kMargin powers of two - the maximum is found, the accumulators are rescaled and the
+    // probabilities formed once more.
+    unsigned int seen = 0u;
+    auto pair = [&](int w, float neg_mrow) __attribute__((always_inline)) {  // packed pair w of 8
+      pk[w >> 2][w & 3] = T::pack2(fast_exp2(fmaf(s[2 * w], a.c, neg_mrow)), fast_exp2(fmaf(s[2 * w + 1], a.c, neg_mrow)));
+    };
+    auto score = [&](int ks) __attribute__((always_inline)) { s_next = T::mfma(kf[ks], qf[ks], ks == 0 ? b_next : s_next); };
+    auto pv = [&](int j, int dt) __attribute__((always_inline)) { oacc[dt] = T::mfma(vf[j][dt], pk_prev[j], oacc[dt]); };
+    const float neg_mrow = b0 - m_i;
+    float l1 = 0.f;
+    float e0, e1;  // a pair is packed one step after its exponentials were issued
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      const float x0 = fmaf(s[2 * g], a.c, neg_mrow), x1 = fmaf(s[2 * g + 1], a.c, neg_mrow);
+      if (g > 0) pk[(g - 1) >> 2][(g - 1) & 3] = T::pack2(e0, e1);
+      e0 = fast_exp2(x0);
+      e1 = fast_exp2(x1);
+      if (g > 0 && !(g & 1)) seen |= pk[(g - 1) >> 2][(g - 2) & 3] | pk[(g - 1) >> 2][(g - 1) & 3];
+      // the denominator sums what the product multiplies: the rounded probabilities
+      if (!C::ONES_ROW) (g & 1 ? l1 : l_i) = T::add2(pk_prev[g >> 2][g & 3], g & 1 ? l1 : l_i);
+      __builtin_amdgcn_sched_barrier(0);
+      if (g == 0) pv(0, 0);
+      if (g == 1) {
+#pragma unroll
+        for (int dt = 1; dt < C::DT; ++dt) pv(0, dt);
+      }
+      if (g >= 2 && g < 2 + C::KS) score(g - 2);
+      if (g >= 2 && g < 2 + C::DT) read_v(0, g - 2, v_off);
+      if (g == 6) pv(1, 0);
+      if (g == 7) {
+#pragma unroll
+        for (int dt = 1; dt < C::DT; ++dt) pv(1, dt);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    pk[1][3] = T::pack2(e0, e1);
+    seen |= pk[1][2] | pk[1][3];
+    if (!C::ONES_ROW) l_i += l1;
+    if (__any((seen & 0x40004000u) != 0u)) {  // uniform; an infinity and a NaN included
+      float mx = s[0];
+#pragma unroll
+      for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+      mx = max_with_lane_xor32(mx);
+      const float m_new = fmaxf(m_i, fmaf(mx, a.c, b0) + T::kMargin);
+      const float alpha = fast_exp2(m_i - m_new);  // first half row: 0
+      m_i = m_new;
+      l_i *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
+#pragma unroll
+      for (int w = 0; w < 8; ++w) pair(w, b0 - m_i);
+    }
+  };
+
+  const int nkt = a.N / 64;
+  // V tiles rotate: row kt's, and the one row kt + 2 goes to (row kt - 1's)
+  unsigned int v_cur = 0, v_free = 2 * C::VTILE;
+  constexpr unsigned int VHALF = 32 * C::VP * 16;
+  f32x16 sA, sB;
+#pragma unroll
+  for (int ks = 0; ks < C::KS; ++ks) sA = T::mfma(*reinterpret_cast<const u32x4*>(lds + krd[ks]), qf[ks], ks == 0 ? b1[0] : sA);
+  auto key_row = [&](int kt, auto buf_c) __attribute__((always_inline)) {
+    constexpr int BUF = decltype(buf_c)::value;  // kt & 1, for constant LDS offsets
+    if (kt == C::RH) {  // the wavefront's own columns: no barrier
+      fill_relh(kt);
+    }
+    const float b0 = relhT[(kt % C::RH) * C::BM + 32 * wave + lr];
+    half_row(sA, sB, pkA, pkB, b1[1], BUF * C::KTILE + 32 * (C::KP * 16), v_cur, v_free + VHALF, b0, kt > 0);
+    // row kt + 1 has landed (own share) and everybody has left K row kt and V row kt - 1: refill them
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (kt + 2 < nkt) {
+      k_dma(kt + 2, BUF);
+      v_dma(kt + 2, v_free);
+    }
+    // (after the last row kf is whatever the buffer holds: that product is not used)
+    half_row(sB, sA, pkB, pkA, b1[0], (BUF ^ 1) * C::KTILE, v_cur + VHALF, v_cur, b0, true);
+    v_free = v_cur;
+    v_cur = v_cur == 2 * C::VTILE ? 0 : v_cur + C::VTILE;
+  };
+  for (int kt = 0; kt < nkt; kt += 2) {  // nkt is even
+    key_row(kt, std::integral_constant<int, 0>{});
+    key_row(kt + 1, std::integral_constant<int, 1>{});
+  }
+  // P V of the last half row
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt) read_v(1, dt, v_free + VHALF);
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int dt = 0; dt < C::DT; ++dt) oacc[dt] = T::mfma(vf[j][dt], pkB[j], oacc[dt]);
+  if (!C::ONES_ROW) {
+#pragma unroll
+    for (int g = 0; g < 8; ++g) l_i = T::add2(pkB[g >> 2][g & 3], l_i);
+  }
+
+  // ---- epilogue: O = acc / l, 4 adjacent channels per store ----
+  float l;
+  if (C::ONES_ROW) {
+    // output row HD (the ones row) = tile DT-1, row HD % 32, held by the lh = (HD % 32) / 4 % 2 lanes
+    constexpr int orow = HD % 32;
+    constexpr int oreg = 4 * (orow / 8) + orow % 4, olh = (orow / 4) % 2;
+    const float own = oacc[C::DT - 1][oreg];
+    const float other = xor32(own);
+    l = (lh == olh) ? own : other;
+  } else {
+    l = l_i + xor32(l_i);
+  }
+  const float inv = 1.0f / l;
+  unsigned short* op = a.out + b * a.o_sb + h * a.o_sh + (int64_t)(q0 + lr) * a.o_sn;
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int d = 32 * dt + 8 * j + 4 * lh;
+      if (d < HD) {
+        const u32x2 o = {T::pack2(oacc[dt][4 * j] * inv, oacc[dt][4 * j + 1] * inv),
+                         T::pack2(oacc[dt][4 * j + 2] * inv, oacc[dt][4 * j + 3] * inv)};
+        *reinterpret_cast<u32x2*>(op + d) = o;
+      }
+    }
+}
+
+template <int HD>
+struct SplitCfg : GridRow<HD> {
+  using R = GridRow<HD>;
+  static constexpr int QW = 2;                  // query tiles of 32 per workgroup
+  static constexpr int WAVES = 2 * QW;
+  static constexpr int BM = 32 * QW;
+  static constexpr int KDPW = (R::KP + WAVES - 1) / WAVES, VDPW = (R::VP + WAVES - 1) / WAVES;
+  static constexpr int V_OFF = 2 * R::KTILE;    // LDS: K tiles of both stages, V tiles of both stages, rel_h
+  static constexpr int RELH_OFF = V_OFF + 2 * R::VTILE;
+  static constexpr int RH = 32;                 // key rows whose rel_h is at hand
+  static constexpr int LDS_BYTES = RELH_OFF + RH * BM * 4;
+  static_assert(3 * LDS_BYTES <= 160 * 1024, "three workgroups per CU");
+  static_assert(QW * 64 * (16 * R::DT + 2) * 4 <= RELH_OFF, "the second halves' results");
+};
+
+template <typename T, int HD>
+__global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void attn_global_split_kernel(AttnArgs a) {
+  using C = SplitCfg<HD>;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS_BYTES];
+  float* relhT = reinterpret_cast<float*>(lds + C::RELH_OFF);  // [kh % RH][BM], * log2(e)
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 31, lh = lane >> 5;
+  const int qt = wave & (C::QW - 1), kg = wave / C::QW;  // query tile, key half
+
+  const unsigned int nqb = a.N / C::BM;
+  const unsigned int total = (unsigned int)(a.B * a.nH) * nqb;
+  const unsigned int pid = xcd_contiguous_id(blockIdx.x, total);
+  if (pid >= total) return;
+  const int bh = pid / nqb, qb = pid % nqb;
+  const int b = bh / a.nH, h = bh % a.nH;
+  const int q0 = qb * C::BM + 32 * qt;  // the wavefront's first query: half of one grid row
+
+  const unsigned short* kbase = a.k + b * a.k_sb + h * a.k_sh;
+  const unsigned short* vbase = a.v + b * a.v_sb + h * a.v_sh;
+
+  // ---- K / V rows: global memory -> LDS directly, wave instruction i of a tile fills pieces 64 i .. 64 i + 63 ----
+  unsigned int koff[C::KDPW];  // bytes, from the tile's first key row; unsigned: scalar-base load form
+  int voff[C::VDPW];           // negative: a spare piece, the lane loads nothing
+#pragma unroll
+  for (int m = 0; m < C::KDPW; ++m) {
+    int row;
+    const int at = C::k_source(64 * (wave + C::WAVES * m) + lane, row);
+    koff[m] = (unsigned int)(row * (int)a.k_sn) * 2u + at;
+  }
+#pragma unroll
+  for (int m = 0; m < C::VDPW; ++m) {
+    int row;
+    const int at = C::v_source(64 * (wave + C::WAVES * m) + lane, row);
+    voff[m] = at < 0 ? -1 : row * (int)a.v_sn * 2 + at;
+  }
+  const unsigned int lds_base = (unsigned int)(uintptr_t)((__attribute__((address_space(3))) unsigned char*)lds);
+  auto k_dma = [&](int kt, int buf) __attribute__((always_inline)) {
+    const unsigned char* src = reinterpret_cast<const unsigned char*>(kbase + (int64_t)kt * 64 * a.k_sn);
+#pragma unroll
+    for (int m = 0; m < C::KDPW; ++m)
+      if (wave + C::WAVES * m < C::KP) lds_dma16(src, koff[m], lds_base + buf * C::KTILE + (wave + C::WAVES * m) * 1024);
+  };
+  auto v_dma = [&](int kt, int buf) __attribute__((always_inline)) {
+    const unsigned char* src = reinterpret_cast<const unsigned char*>(vbase + (int64_t)kt * 64 * a.v_sn);
+#pragma unroll
+    for (int m = 0; m < C::VDPW; ++m)
+      if (wave + C::WAVES * m < C::VP && (!C::ONES_ROW || voff[m] >= 0))
+        lds_dma16(src, (unsigned int)voff[m], lds_base + C::V_OFF + buf * C::VTILE + (wave + C::WAVES * m) * 1024);
+  };
+  k_dma(0, 0);
+  v_dma(0, 0);
+  k_dma(1, 1);  // N % 128 == 0: at least two key rows
+  v_dma(1, 1);
+  // operand reads of this wavefront's key half
+  int vrd[C::DT], krd[C::KS];
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt) vrd[dt] = C::V_OFF + 32 * kg * (C::VP * 16) + C::v_read(lane, dt);
+#pragma unroll
+  for (int ks = 0; ks < C::KS; ++ks) krd[ks] = 32 * kg * (C::KP * 16) + C::k_read(lr, lh, ks);
+
+  // The workgroups of a head walk its key rows in step, so every row would be waited for at the latency of the
+  // Infinity Cache or HBM.  Each of them touches its own share of the head's K and V first: together they
+  // have the head in their XCD's L2 by the time they get to it.
+  constexpr int NTOUCH = 2 * C::BM * (HD / 8) / (64 * C::WAVES);
+  unsigned int touched[NTOUCH];
+#pragma unroll
+  for (int i = 0; i < NTOUCH; ++i) {
+    const int P = (tid + 64 * C::WAVES * i) % (C::BM * (HD / 8)), row = P / (HD / 8), col = P % (HD / 8);
+    const bool is_v = 2 * i >= NTOUCH;
+    touched[i] = *reinterpret_cast<const unsigned int*>((is_v ? vbase : kbase) + (int64_t)(qb * C::BM + row) * (is_v ? a.v_sn : a.k_sn) + col * 8);
+  }
+
+  // ---- Q^T operand: query lr, channels 16s + 8lh .. +7 ----
+  u32x4 qf[C::KS];
+  {
+    const unsigned short* qp = a.q + b * a.q_sb + h * a.q_sh + (int64_t)(q0 + lr) * a.q_sn + 8 * lh;
+#pragma unroll
+    for (int s = 0; s < C::KS; ++s) qf[s] = load_x8_global(qp + 16 * s);
+  }
+
+  // the spare pieces of V tile `buf`: (1, 0, ..) and zeros
+  auto ones = [&](int buf) __attribute__((always_inline)) {
+    if (C::ONES_ROW && tid < 64) {
+      u32x4* p = reinterpret_cast<u32x4*>(lds + C::V_OFF + buf * C::VTILE + tid * (C::VP * 16) + HD * 2);
+      p[0] = u32x4{T::kOne, 0u, 0u, 0u};
+      p[1] = u32x4{0u, 0u, 0u, 0u};
+    }
+  };
+  ones(0);
+  ones(1);
+  // rel_h of key rows kh0 .. kh0 + 31, shared by the two key halves
+  auto fill_relh = [&](int kh0) __attribute__((always_inline)) {
+    const unsigned short* rhb = a.rh + b * a.rh_sb + h * a.rh_sh + (int64_t)(qb * C::BM) * a.rh_sn;
+    const int ql = tid / 4, part = tid % 4;  // 64 queries x 4 pieces of 8 key rows
+    static_assert(C::BM * 4 == 64 * C::WAVES, "one piece per thread");
+    unsigned short v8[8];
+    const unsigned short* src = rhb + (int64_t)ql * a.rh_sn + kh0 + 8 * part;
+    if (a.relh_x8) {
+      *reinterpret_cast<u32x4*>(v8) = load_x8_global(src);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v8[e] = kh0 + 8 * part + e < a.gh ? src[e] : (unsigned short)0;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) relhT[(8 * part + e) * C::BM + ql] = T::from_bits(v8[e]) * kLog2e;
+  };
+
+  // ---- rel_w / sm_scale of this wavefront's keys, the initial accumulator of every score tile ----
+  f32x16 b1;
+  {
+    const unsigned short* rwp = a.rw + b * a.rw_sb + h * a.rw_sh + (int64_t)(q0 + lr) * a.rw_sn + 32 * kg + 4 * lh;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const u32x2 w = *reinterpret_cast<const u32x2*>(rwp + 8 * j);
+      b1[4 * j + 0] = T::lo(w[0]) * a.inv_scale;
+      b1[4 * j + 1] = T::hi(w[0]) * a.inv_scale;
+      b1[4 * j + 2] = T::lo(w[1]) * a.inv_scale;
+      b1[4 * j + 3] = T::hi(w[1]) * a.inv_scale;
+    }
+  }
+  fill_relh(0);
+#pragma unroll
+  for (int i = 0; i < NTOUCH; ++i) asm volatile("" : : "v"(touched[i]));
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of tile 0 has landed
+  __syncthreads();
+
+  // ---- main loop over key grid rows ----
+  f32x16 oacc[C::DT];
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
+  float m_i = -INFINITY, l_i = 0.f;
+
+  const int nkt = a.N / 64;
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4* trptr_t;
+  // The loop is pipelined inside a wavefront as attn_global_kernel's is: between the exponentials of row kt stand
+  // the matrix instructions of the scores of row kt + 1 and of P V of row kt - 1.
+  u32x4 kf[C::KS], vf[2][C::DT], pkA[2], pkB[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    pkA[j] = pkB[j] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int dt = 0; dt < C::DT; ++dt) vf[j][dt] = u32x4{0u, 0u, 0u, 0u};
+  }
+  auto read_v = [&](int j, int dt, int buf) __attribute__((always_inline)) {
+    const unsigned char* p = lds + vrd[dt] + buf * C::VTILE + 16 * j * (C::VP * 16);
+    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((trptr_t)p));
+    const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((trptr_t)(p + 8 * C::VP * 16)));
+    vf[j][dt] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+  };
+  auto row = [&](int kt, auto buf_c, f32x16& s, f32x16& s_next, u32x4 (&pk)[2], u32x4 (&pk_prev)[2]) __attribute__((always_inline)) {
+    constexpr int BUF = decltype(buf_c)::value;  // kt & 1, for constant LDS offsets
+    if (kt == C::RH) {  // uniform; everybody has left row kt - 1 (the barrier at its end)
+      fill_relh(kt);
+      __syncthreads();
+    }
+    const float b0 = relhT[(kt % C::RH) * C::BM + 32 * qt + lr];
+#pragma unroll
+    for (int ks = 0; ks < C::KS; ++ks) kf[ks] = *reinterpret_cast<const u32x4*>(lds + krd[ks] + (BUF ^ 1) * C::KTILE);
+    __builtin_amdgcn_sched_barrier(0);
+    if (kt + 2 < nkt) k_dma(kt + 2, BUF);  // row kt's scores are made: its K buffer is free
+    __builtin_amdgcn_sched_barrier(0);
+
+    unsigned int seen = 0u;
+    auto pair = [&](int w, float neg_mrow) __attribute__((always_inline)) {  // packed pair w of 8
+      pk[w >> 2][w & 3] = T::pack2(fast_exp2(fmaf(s[2 * w], a.c, neg_mrow)), fast_exp2(fmaf(s[2 * w + 1], a.c, neg_mrow)));
+    };
+    auto score = [&](int ks) __attribute__((always_inline)) { s_next = T::mfma(kf[ks], qf[ks], ks == 0 ? b1 : s_next); };
+    auto pv = [&](int j, int dt) __attribute__((always_inline)) { oacc[dt] = T::mfma(vf[j][dt], pk_prev[j], oacc[dt]); };
+    const float neg_mrow = b0 - m_i;
+    float l1 = 0.f;
+    // (the last row's kf is whatever the buffer holds: its product is not used)
+    float e0, e1;  // a pair is packed one step after its exponentials were issued
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      const float x0 = fmaf(s[2 * g], a.c, neg_mrow), x1 = fmaf(s[2 * g + 1], a.c, neg_mrow);
+      if (g > 0) pk[(g - 1) >> 2][(g - 1) & 3] = T::pack2(e0, e1);
+      e0 = fast_exp2(x0);
+      e1 = fast_exp2(x1);
+      if (g > 0 && !(g & 1)) seen |= pk[(g - 1) >> 2][(g - 2) & 3] | pk[(g - 1) >> 2][(g - 1) & 3];
+      if (!C::ONES_ROW) (g & 1 ? l1 : l_i) = T::add2(pk_prev[g >> 2][g & 3], g & 1 ? l1 : l_i);
+      __builtin_amdgcn_sched_barrier(0);
+      if (g == 0) pv(0, 0);
+      if (g == 1) {
+#pragma unroll
+        for (int dt = 1; dt < C::DT; ++dt) pv(0, dt);
+      }
+      if (g >= 2 && g < 2 + C::KS) score(g - 2);
+      if (g == 6) pv(1, 0);
+      if (g == 7) {
+#pragma unroll
+        for (int dt = 1; dt < C::DT; ++dt) pv(1, dt);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // this row's V for the next round
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int dt = 0; dt < C::DT; ++dt) read_v(j, dt, BUF);
+    pk[1][3] = T::pack2(e0, e1);
+    seen |= pk[1][2] | pk[1][3];
+    if (!C::ONES_ROW) l_i += l1;
+    if (__any((seen & 0x40004000u) != 0u)) {  // a probability has reached 2: move the reference (attn_relpos.hip)
+      float mx = s[0];
+#pragma unroll
+      for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+      mx = max_with_lane_xor32(mx);
+      const float m_new = fmaxf(m_i, fmaf(mx, a.c, b0) + T::kMargin);
+      const float alpha = fast_exp2(m_i - m_new);
+      m_i = m_new;
+      l_i *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
+#pragma unroll
+      for (int w = 0; w < 8; ++w) pair(w, b0 - m_i);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of K row kt + 2 and V row kt + 1 has landed
+    __syncthreads();
+    if (kt + 2 < nkt) v_dma(kt + 2, BUF);  // row kt's V is in registers
+  };
+  f32x16 sA, sB;
+#pragma unroll
+  for (int ks = 0; ks < C::KS; ++ks)
+    sA = T::mfma(*reinterpret_cast<const u32x4*>(lds + krd[ks]), qf[ks], ks == 0 ? b1 : sA);
+  __syncthreads();  // K row 0 has been read by everyone: its buffer may be refilled
+  for (int kt = 0; kt < nkt; kt += 2) {  // nkt is even
+    row(kt, std::integral_constant<int, 0>{}, sA, sB, pkA, pkB);
+    row(kt + 1, std::integral_constant<int, 1>{}, sB, sA, pkB, pkA);
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int dt = 0; dt < C::DT; ++dt) oacc[dt] = T::mfma(vf[j][dt], pkB[j], oacc[dt]);  // P V of the last row
+  if (!C::ONES_ROW) {
+#pragma unroll
+    for (int g = 0; g < 8; ++g) l_i = T::add2(pkB[g >> 2][g & 3], l_i);
+  }
+
+  // ---- the two key halves meet: reference, denominator and accumulators of half 1 through LDS ----
+  float* other = reinterpret_cast<float*>(lds) + qt * 64 * (16 * C::DT + 2) + lane;  // word w of lane: 64 w + lane
+  if (kg == 1) {
+#pragma unroll
+    for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) other[64 * (16 * dt + r)] = oacc[dt][r];
+    other[64 * 16 * C::DT] = m_i;
+    other[64 * (16 * C::DT + 1)] = l_i;
+  }
+  __syncthreads();
+  if (kg == 1) return;
+  {
+    const float m1 = other[64 * 16 * C::DT], l1 = other[64 * (16 * C::DT + 1)];
+    const float m = fmaxf(m_i, m1);
+    const float f0 = fast_exp2(m_i - m), f1 = fast_exp2(m1 - m);
+    l_i = l_i * f0 + l1 * f1;
+#pragma unroll
+    for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) oacc[dt][r] = oacc[dt][r] * f0 + other[64 * (16 * dt + r)] * f1;
+  }
+  float l;
+  if (C::ONES_ROW) {
+    constexpr int orow = HD % 32;
+    constexpr int oreg = 4 * (orow / 8) + orow % 4, olh = (orow / 4) % 2;
+    const float own = oacc[C::DT - 1][oreg], partner = xor32(own);
+    l = (lh == olh) ? own : partner;
+  } else {
+    l = l_i + xor32(l_i);
+  }
+  const float inv = 1.0f / l;
+  unsigned short* op = a.out + b * a.o_sb + h * a.o_sh + (int64_t)(q0 + lr) * a.o_sn;
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int d = 32 * dt + 8 * j + 4 * lh;
+      if (d < HD) {
+        const u32x2 o = {T::pack2(oacc[dt][4 * j] * inv, oacc[dt][4 * j + 1] * inv),
+                         T::pack2(oacc[dt][4 * j + 2] * inv, oacc[dt][4 * j + 3] * inv)};
+        *reinterpret_cast<u32x2*>(op + d) = o;
+      }
+    }
+}
+
+// Which form of the global kernel: 8 or 4 wavefronts of attn_global_kernel, or 2 for the key-split one.  What
+// decides is how the workgroups divide among the 256 CUs: the forms hold 256 queries (one workgroup per CU),
+// 128 (two) and 64 (hd 64: three, hd 80: two).  The prices are microseconds of one full round over 64 key rows
+// and of a last, partial one with one / two workgroups per CU, measured over 1 to 8 images of 8 to 16 heads; 1 x 12 heads
+// x 4096, hd 64: 72 us key-split, 75 with 8 wavefronts, 78 with 4; 2 x 9: 107, 149, 123; 1 x 16, hd 80: 116, 96, 102.
+static int bias_form(const AttnArgs& a, int hd) {
+  const int force = knob(KNOB_ATTN_WAVES);
+  const bool by8 = a.N % 256 == 0;
+  if (force == 4 || force == 8) return force == 8 && by8 ? 8 : 4;
+  const int split = knob_or(KNOB_ATTN_SPLIT, 1);
+  if (split == 2) return 2;
+  auto price = [](int64_t wgs, int per_cu, int full, int one, int two) {
+    const int64_t slots = 256 * per_cu, rest = wgs % slots;
+    const int last = rest == 0 ? 0 : rest <= 256 ? one : rest <= 512 ? two : full;
+    return wgs / slots * full + last;
+  };
+  const int64_t slices = (int64_t)a.B * a.nH;
+  const int64_t p2 = hd == 64 ? price(slices * (a.N / 64), 3, 66, 30, 50) : price(slices * (a.N / 64), 2, 58, 42, 58);
+  const int64_t p4 = hd == 64 ? price(slices * (a.N / 128), 2, 79, 50, 79) : price(slices * (a.N / 128), 2, 97, 59, 97);
+  const int64_t p8 = price(slices * (a.N / 256), 1, hd == 64 ? 76 : 90, hd == 64 ? 76 : 90, 0);
+  if (split != 0 && p2 <= p4 && p2 <= p8 && !(p2 == p4 && hd == 80)) return 2;
+  return by8 && p8 <= p4 ? 8 : 4;
+}
+template <typename T, int HD>
+static void launch_bias(const AttnArgs& a, int form, hipStream_t stream) {
+  auto grid = [&](int queries) { return dim3((unsigned int)(((int64_t)a.B * a.nH * (a.N / queries) + 7) / 8 * 8)); };
+  if (form == 8) hipLaunchKernelGGL((attn_global_bias_kernel<T, HD, 8>), grid(256), dim3(512), 0, stream, a);
+  else if (form == 4) hipLaunchKernelGGL((attn_global_bias_kernel<T, HD, 4>), grid(128), dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL((attn_global_split_kernel<T, HD>), grid(64), dim3(256), 0, stream, a);
+}
+
+int attn_global_bias_launch(const AttnArgs& a0, int hd, int dtype, hipStream_t stream) {
+  AttnArgs a = a0;
+  // rel_h rows can be read 16 bytes at a time, and the last piece read lies inside them
+  a.relh_x8 = a.gh % 32 == 0 && a.rh_sn % 8 == 0 && a.rh_sh % 8 == 0 && a.rh_sb % 8 == 0 && aligned16(a.rh);
+  const int form = bias_form(a, hd);
+  if (dtype == SAMFAST_F16) {
+    if (hd == 64) launch_bias<ElemF16, 64>(a, form, stream); else launch_bias<ElemF16, 80>(a, form, stream);
+  } else {
+    if (hd == 64) launch_bias<ElemBf16, 64>(a, form, stream); else launch_bias<ElemBf16, 80>(a, form, stream);
+  }
+  return check_launch("attn_global_bias_kernel");
+}
+
+}  // namespace samfast

@@ -24,8 +24,8 @@
 //   rel_w is identical for every key tile -> kept in registers as the INITIAL
 //   accumulator of the score MFMA (pre-divided by sm_scale), and rel_h is one
 //   scalar per (query, key tile) -> folded into the running-max bookkeeping.
-//   With FUSED the two factors are produced in the prologue by MFMA from the
-//   (2S-1, hd) tables: rel_h^T = Rh[qh+gh-1-kh] Q^T directly, rel_w through the
+//   The two factors are produced in the prologue by MFMA from the (2S-1, hd) tables
+//   (caller-computed factors: attn_global_bias.hip): rel_h^T = Rh[qh+gh-1-kh] Q^T directly, rel_w through the
 //   full product T = Rw Q^T followed by the per-query diagonal gather
 //   rel_w[q, kw] = T[qw - kw + 63, q] staged through LDS.
 //
@@ -76,7 +76,7 @@ struct GlobalCfg {
   static_assert(X_BYTES <= LDS_BYTES, "gather scratch must fit in the workgroup's LDS");
 };
 
-template <typename T, int HD, int QT, bool FUSED, int WAVES>
+template <typename T, int HD, int QT, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void attn_global_kernel(AttnArgs a) {
   using C = GlobalCfg<HD, QT, WAVES>;
   __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS_BYTES];
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void attn_global_ke
       }
     }
   };
-  if (FUSED) {
+  {
     const unsigned short* tw = a.rw;
     // rel_w: T[rel][q] for rel in [0,128) in two passes of 64 through LDS scratch
     float* X = reinterpret_cast<float*>(lds) + wave * 32 * C::XSTR;
@@ -262,28 +262,6 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void attn_global_ke
     __syncthreads();  // every wave is done with the scratch: the stages may be filled
     first_tile();     // in flight while rel_h is formed
     relh_from_table();
-  } else {
-    first_tile();
-    const unsigned short* rhb = a.rh + b * a.rh_sb + h * a.rh_sh + (int64_t)q_wg * a.rh_sn;
-    for (int idx = tid; idx < C::BM * a.gh; idx += 64 * WAVES) {
-      const int ql = idx % C::BM, kh = idx / C::BM;
-      relhT[kh * C::BM + ql] = T::from_bits(rhb[(int64_t)ql * a.rh_sn + kh]) * kLog2e;
-    }
-#pragma unroll
-    for (int t = 0; t < QT; ++t) {
-      const unsigned short* rwp =
-          a.rw + b * a.rw_sb + h * a.rw_sh + (int64_t)(q_wg + q_wave + 32 * t + lr) * a.rw_sn;
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const u32x2 w = *reinterpret_cast<const u32x2*>(rwp + 32 * nt + 8 * j + 4 * lh);
-          b1[t][nt][4 * j + 0] = T::lo(w[0]) * a.inv_scale;
-          b1[t][nt][4 * j + 1] = T::hi(w[0]) * a.inv_scale;
-          b1[t][nt][4 * j + 2] = T::lo(w[1]) * a.inv_scale;
-          b1[t][nt][4 * j + 3] = T::hi(w[1]) * a.inv_scale;
-        }
-    }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of tile 0 has landed
   __syncthreads();                                   // tile 0 and relhT complete
@@ -835,14 +813,14 @@ __global__ __launch_bounds__(WindowCfg<HD>::THREADS, 2) void attn_window_kernel(
 // =============================================================================
 template <typename T, int HD, bool FUSED>
 static int launch_hd(const AttnArgs& a, bool global_path, hipStream_t stream) {
-  if (global_path) {
+  if constexpr (FUSED) if (global_path) {
     constexpr int QT = 1;
     auto launch = [&](auto wc) {
       constexpr int WAVES = decltype(wc)::value;
       using C = GlobalCfg<HD, QT, WAVES>;
       const int64_t total = (int64_t)a.B * a.nH * (a.N / C::BM);
       const unsigned int grid = (unsigned int)(((total + 7) / 8) * 8);
-      hipLaunchKernelGGL((attn_global_kernel<T, HD, QT, FUSED, WAVES>), dim3(grid), dim3(64 * WAVES), 0, stream, a);
+      hipLaunchKernelGGL((attn_global_kernel<T, HD, QT, WAVES>), dim3(grid), dim3(64 * WAVES), 0, stream, a);
     };
     // 256 queries per workgroup when that still gives every CU several workgroups
     // (SAMFAST_ATTN_WAVES=4 / 8 overrides the choice where the shape allows it)
@@ -914,6 +892,7 @@ static int attn_dispatch(bool fused, AttnArgs& a, int hd, int dtype, float sm_sc
   a.inv_scale = 1.0f / sm_scale;
   // windows whose rows fit the padded-row key layout take that kernel (attn_window_rows.hip)
   if (!global_path && attn_window_rows_covers(a)) return attn_window_rows_launch(a, hd, dtype, fused, stream);
+  if (global_path && !fused) return attn_global_bias_launch(a, hd, dtype, stream);
   auto by_type = [&](auto elem) {
     using T = decltype(elem);
     if (hd == 64)

@@ -28,6 +28,7 @@ struct AttnArgs {
   int img_h, img_w, ws, wins_x, wins_y;
   const unsigned short* pad_k;
   const unsigned short* pad_v;
+  int relh_x8;  // attn_global_bias.hip: rel_h rows can be read 16 bytes at a time
 };
 
 constexpr float kLog2e = 1.4426950408889634f;
@@ -38,11 +39,18 @@ constexpr float kLazyLog2 = 8.0f;  // softmax reference lags the running maximum
 // as four 32-bit words (u32x4) everywhere outside these functions.
 struct ElemBf16 {
   static constexpr unsigned int kOne = 0x3F80u;   // 1.0
+  // global kernel: how far (log2) above the running maximum the exponent reference is put; bf16
+  // probabilities keep their eight bits at any size
+  static constexpr float kMargin = 16.0f;
   static constexpr unsigned int kMask = 0xF149u;  // -1e30: added to a score (before the scale), it removes the key
   static SF_DEVICE f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
   }
   static SF_DEVICE unsigned int pack2(float lo, float hi) { return pack_bf16x2(lo, hi); }
+  // c + the two values of a packed pair, one instruction
+  static SF_DEVICE float add2(unsigned int w, float c) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w), __builtin_bit_cast(bf16x2, kOne << 16 | kOne), c, false);
+  }
   static SF_DEVICE float lo(unsigned int w) { return bf16_lo_to_f32(w); }
   static SF_DEVICE float hi(unsigned int w) { return bf16_hi_to_f32(w); }
   static SF_DEVICE float from_bits(unsigned short h) { return bf16_bits_to_f32(h); }
@@ -51,6 +59,7 @@ struct ElemF16 {
   typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
   typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
   static constexpr unsigned int kOne = 0x3C00u;   // 1.0
+  static constexpr float kMargin = 4.0f;  // fp16 ends at 2^-24: 2^-20 of the maximum, against 2^-11 of a rounding
   static constexpr unsigned int kMask = 0xFB53u;  // -60000 (fp16 ends at 65504): times scale*log2(e) still below -2^12
   static SF_DEVICE f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
@@ -58,6 +67,9 @@ struct ElemF16 {
   static SF_DEVICE unsigned int pack2(float lo, float hi) {  // round to nearest even
     const f32x2 v = {lo, hi};
     return __builtin_bit_cast(unsigned int, __builtin_convertvector(v, f16x2));
+  }
+  static SF_DEVICE float add2(unsigned int w, float c) {
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, w), __builtin_bit_cast(f16x2, kOne << 16 | kOne), c, false);
   }
   static SF_DEVICE float from_bits(unsigned short h) { return (float)__builtin_bit_cast(_Float16, h); }
   static SF_DEVICE float lo(unsigned int w) { return from_bits((unsigned short)(w & 0xffffu)); }
@@ -84,6 +96,51 @@ SF_DEVICE float max_with_lane_xor32(float v) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
+// One wave instruction: 64 pieces of 16 bytes from base + off to LDS at `dst` (piece of lane l: dst + 16 l).
+// Written out because the compiler would make every LDS read that follows wait for the builtin's loads;
+// whoever calls it waits for the arrival by hand (vmcnt) before the barrier in front of the readers.
+SF_DEVICE void lds_dma16(const unsigned char* base, unsigned int off, unsigned int dst) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(dst) : "memory");
+}
+
+// How the global kernels keep one key grid row (64 keys) of K and of V in LDS: rows of 16-byte pieces, placed so
+// that no read of a wavefront meets a bank twice.
+//   K is read 16 bytes per lane, 32 keys at a time.  HD = 64: 128-byte rows, piece c of row r at position
+//   c ^ (r / 2 % 8); HD = 80: 160-byte rows, position c ^ (r / 8 % 2).
+//   V is read by ds_read_b64_tr_b16, four keys x 64 bytes per half wavefront.  HD = 64: the row's two 64-byte
+//   halves change places in rows 2, 3 of every four; HD = 80: 192-byte rows (16 words past a multiple of
+//   the banks), the two spare pieces hold (1, 0, ...) and zeros: channel 80 of every key is one, and
+//   the P V product delivers the softmax denominator in its otherwise unused output rows.
+template <int HD>
+struct GridRow {
+  static constexpr int KS = HD / 16;           // score k-steps
+  static constexpr int DT = (HD + 31) / 32;    // output channel tiles
+  static constexpr bool ONES_ROW = HD % 32 != 0;
+  static constexpr int KP = HD / 8, VP = ONES_ROW ? 12 : HD / 8;  // pieces per row = wave instructions per tile
+  static constexpr int KTILE = 64 * KP * 16, VTILE = 64 * VP * 16;
+  static SF_DEVICE int k_swizzle(int row) { return HD == 64 ? (row >> 1) & 7 : (row >> 3) & 1; }
+  // byte offset inside the source row of the piece at LDS position P of a tile (or -1: a spare piece)
+  static SF_DEVICE int k_source(int P, int& row) {
+    row = P / KP;
+    return ((P % KP) ^ k_swizzle(row)) * 16;
+  }
+  static SF_DEVICE int v_source(int P, int& row) {
+    row = P / VP;
+    const int pos = P % VP;
+    if (ONES_ROW) return pos < HD / 8 ? pos * 16 : -1;
+    return (pos ^ (4 * ((row >> 1) & 1))) * 16;
+  }
+  // LDS offset inside a K tile of the lane's operand piece (key lr, channels 16 ks + 8 lh)
+  static SF_DEVICE int k_read(int lr, int lh, int ks) { return lr * (KP * 16) + (((2 * ks + lh) ^ k_swizzle(lr)) * 16); }
+  // LDS offset inside a V tile of the lane's transposing read, output tile dt (key and channel of a source lane:
+  // see attn_global_kernel)
+  static SF_DEVICE int v_read(int lane, int dt) {
+    const int g = lane >> 4, sl = lane & 15, key = 4 * (g >> 1) + (sl >> 2);
+    const int half = ONES_ROW ? dt : dt ^ ((key >> 1) & 1);
+    return key * (VP * 16) + half * 64 + 32 * (g & 1) + 8 * (sl & 3);
+  }
+};
+
 // all LDS operations this wavefront has issued are complete and ordered
 SF_DEVICE void wave_lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
@@ -100,6 +157,9 @@ SF_DEVICE u32x4 onehot_x8(int slot, int lh) {
   }
   return w;
 }
+
+// Global attention with caller-computed bias factors (attn_global_bias.hip)
+int attn_global_bias_launch(const AttnArgs& a, int hd, int dtype, hipStream_t stream);
 
 // Window kernel with the keys laid out as grid rows padded to 16 (attn_window_rows.hip): whether it
 // covers the call (gw <= 16, gh <= 14) and its launch.

@@ -1,0 +1,52 @@
+"""Global attention with caller-computed factors: every form of the kernel against the oracle."""
+
+import math
+
+import pytest
+import torch
+
+from helpers import bias_inputs
+from oracle import relpos_attention as ora
+
+pytestmark = pytest.mark.gpu
+
+FORMS = {"eight wavefronts": dict(SAMFAST_ATTN_WAVES=8), "four": dict(SAMFAST_ATTN_WAVES=4), "key split": dict(SAMFAST_ATTN_SPLIT=2)}
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("B,nH,gh,hd,ramp,dtype", [
+    (1, 3, 64, 64, 0.0, torch.bfloat16),
+    (2, 1, 64, 80, 0.0, torch.float16),
+    (1, 1, 2, 80, 0.0, torch.bfloat16),     # the shortest grid: two key rows
+    (2, 2, 34, 64, 0.0, torch.float16),     # rel_h renewed for two rows only, its rows not 16-byte aligned
+    (1, 2, 36, 80, 30.0, torch.bfloat16),   # logits that rise along the keys: the reference moves again and again
+    (1, 2, 64, 64, 30.0, torch.float16),
+])
+def test_bias_kernels_vs_oracle(form, B, nH, gh, hd, ramp, dtype):
+    from samfast_amd import _lib, ops
+    print(f"case {form} B={B} nH={nH} gh={gh} hd={hd} {dtype}", flush=True)
+    q, k, v, rel_h, rel_w = bias_inputs(B, nH, gh, 64, hd, seed=gh + hd, dtype=dtype)
+    if ramp:
+        u = torch.full((hd,), 1 / math.sqrt(hd))
+        steps = torch.arange(gh * 64) / (gh * 64)
+        q = (q.float() + 4.0 * u).to(dtype)
+        k = (k.float() + ramp * steps[None, None, :, None] * u).to(dtype)
+    ref = ora.attention_rel_h_rel_w(q, k, v, rel_h, rel_w, compute_dtype=torch.float32)
+    with _lib.knobs(**FORMS[form]):
+        out = ops.attn_relpos_bias(q.cuda(), k.cuda(), v.cuda(), rel_h.squeeze(-1).cuda(), rel_w.squeeze(-2).cuda())
+    diff = (out.float().cpu() - ref.float()).abs()
+    print(f"max-abs {diff.max().item():.2e} mean-abs {diff.mean().item():.2e}", flush=True)
+    assert diff.max().item() <= 2e-2 and diff.mean().item() <= 1e-3
+
+
+def test_bias_kernels_read_strided_factors():
+    """The factors as slices of one (B, nH, N, 128) tensor, q / k / v of a token-major buffer: same bits as contiguous."""
+    from samfast_amd import ops
+    B, nH, N, hd = 1, 2, 4096, 64
+    g = torch.Generator(device="cuda").manual_seed(1)
+    qkv = torch.randn((B, N, 3, nH, hd), generator=g, device="cuda").to(torch.bfloat16)
+    both = (torch.randn((B, nH, N, 128), generator=g, device="cuda") * 0.5).to(torch.bfloat16)
+    q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
+    a = ops.attn_relpos_bias(q, k, v, both[..., :64], both[..., 64:])
+    b = ops.attn_relpos_bias(q.contiguous(), k.contiguous(), v.contiguous(), both[..., :64].contiguous(), both[..., 64:].contiguous())
+    assert torch.equal(a, b)
