@@ -47,6 +47,77 @@ __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowwise_bf16_k
   RQ::finish_row(a, row, nchunk, lane, xw, gw, bw);
 }
 
+// WPR wavefronts share a row: fewer registers per lane for long rows (one wavefront with 4096 values needs 238: two
+// per SIMD and 2.2 TB/s at 65536 rows, 5.1 TB/s with four sharing), and for few rows more wavefronts with
+// fewer loads each to wait for.  The shares' maxima meet in LDS.  Bound: HBM, at the rate of a copy, from 8192 rows on.
+template <int NCH, int EPC, int WPR>
+__global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowshare_bf16_kernel(QuantArgs a) {
+  constexpr int RPB = kQuantWavesPerBlock / WPR;  // rows per workgroup
+  using RQ = RowQuantizer<NCH, EPC, false>;
+  typedef typename RQ::in_t in_t;
+  __shared__ float part[kQuantWavesPerBlock];
+  __shared__ int nan_seen[kQuantWavesPerBlock];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sub = wave % WPR;
+  const int64_t row = (int64_t)blockIdx.x * RPB + wave / WPR;
+  const bool live = row < a.M;  // uniform over the wavefront
+  const int nchunk = a.K / EPC;
+  // chunk i of the lane: (i * WPR + sub) * 64 + lane, so that the wavefronts of a row read it side by side
+  in_t xw[NCH];
+  float amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int c = (i * WPR + sub) * 64 + lane;
+    const in_t z = {};
+    xw[i] = z;
+    if (live && c < nchunk) xw[i] = __builtin_nontemporal_load(reinterpret_cast<const in_t*>(a.x + row * a.ldx) + c);
+  }
+#pragma unroll
+  for (int i = 0; i < NCH; ++i)
+#pragma unroll
+    for (int e = 0; e < RQ::W; ++e) amax = fmaxf(amax, fmaxf(fabsf(bf16_lo_to_f32(xw[i][e])), fabsf(bf16_hi_to_f32(xw[i][e]))));
+  amax = wave_max_nonneg(amax);
+  if (lane == 0) part[wave] = amax;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < WPR; ++w) amax = fmaxf(amax, part[wave / WPR * WPR + w]);
+  const float scale = fmaxf(amax, 1e-5f) / 127.0f;
+  const float inv_scale = 1.0f / scale;
+  bool saw_nan = false;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int c = (i * WPR + sub) * 64 + lane;
+    if (live && c < nchunk) {
+      float f[EPC];
+#pragma unroll
+      for (int e = 0; e < RQ::W; ++e) {
+        f[2 * e] = bf16_lo_to_f32(xw[i][e]);
+        f[2 * e + 1] = bf16_hi_to_f32(xw[i][e]);
+      }
+      unsigned int codes[EPC / 4];
+      saw_nan |= quantize_chunk<EPC>(f, scale, inv_scale, codes);
+      RQ::store_chunk(a, row, c, codes);
+    }
+  }
+  const bool any_nan = __any(saw_nan);  // (the maximum drops NaNs: see RowQuantizer::finish_row)
+  if (lane == 0) nan_seen[wave] = any_nan;
+  __syncthreads();
+  if (live && sub == 0 && lane == 0) {
+    int n = 0;
+#pragma unroll
+    for (int w = 0; w < WPR; ++w) n |= nan_seen[wave + w];
+    a.sx[row] = n ? __uint_as_float(0x7fc00000u) : scale;
+  }
+}
+
+template <int NCH, int EPC, int WPR>
+static int launch_rowshare(const QuantArgs& a, hipStream_t stream) {
+  constexpr int RPB = kQuantWavesPerBlock / WPR;
+  hipLaunchKernelGGL((quant_rowshare_bf16_kernel<NCH, EPC, WPR>), dim3((unsigned int)((a.M + RPB - 1) / RPB)), dim3(64 * kQuantWavesPerBlock), 0, stream, a);
+  return check_launch("quant_rowshare_bf16_kernel");
+}
+
 template <int NCH, int EPC, bool LN>
 static int launch_quant(const QuantArgs& a, hipStream_t stream) {
   const int64_t blocks = (a.M + kQuantWavesPerBlock - 1) / kQuantWavesPerBlock;
@@ -55,17 +126,42 @@ static int launch_quant(const QuantArgs& a, hipStream_t stream) {
   return check_launch("quant_rowwise_bf16_kernel");
 }
 
+template <int WPR>
+static int launch_shares(const QuantArgs& a, hipStream_t s) {
+  // shares that 4-element chunks divide among the 64 lanes exactly and 8-element chunks do not
+  if (a.K == 3 * 256 * WPR) return launch_rowshare<3, 4, WPR>(a, s);
+  if (a.K == 5 * 256 * WPR) return launch_rowshare<5, 4, WPR>(a, s);
+  const int need = (a.K / 8 + 64 * WPR - 1) / (64 * WPR);
+  if (need <= 1) return launch_rowshare<1, 8, WPR>(a, s);
+  if (need <= 2) return launch_rowshare<2, 8, WPR>(a, s);
+  if (WPR == 2 || need <= 3) return launch_rowshare<3, 8, WPR>(a, s);
+  return launch_rowshare<4, 8, WPR>(a, s);
+}
+
 template <bool LN>
 static int dispatch_quant(const QuantArgs& a, hipStream_t s) {
   // rows that 4-element chunks divide among the 64 lanes exactly and 8-element chunks do not
   if (a.K == 768) return launch_quant<3, 4, LN>(a, s);
   if (a.K == 1280) return launch_quant<5, 4, LN>(a, s);
   const int need = (a.K / 8 + 63) / 64;
+  if constexpr (!LN) {
+    // Rows of more than 1024: wavefronts that share a row (us, one wavefront a row / two / four).
+    //   Where one wavefront would need 128 registers and more, at any M: 65536 x 4096: 308 / 166 / 159, 16384 x 3072:
+    //   38 / 32 / 30, 65536 x 2560: 115 / 102 / 105, 4096 x 2048: 9.2 / 8.0 / 9.0.
+    //   Else while the rows are too few to fill the GPU with one wavefront each: 512 x 5120: 6.5 / 5.4 / 4.1, 5003 x 5120:
+    //   19.1 / 21.8 / 17.1, 16384 x 5120: 46 / 55 / 48; 1000 x 1536: 3.9 / 3.6 / 3.2, 8192 x 1536: 12.1 / 11.3 / 12.9.
+    if (need == 3 && a.M <= 8192) return a.M <= 1024 ? launch_shares<4>(a, s) : launch_shares<2>(a, s);
+    if (need == 4 || need == 5) return a.M <= 1024 ? launch_shares<4>(a, s) : launch_shares<2>(a, s);
+    if (need >= 6 && need <= 8) return launch_shares<4>(a, s);
+    // (below 11 chunks, quarters that do not fill their lanes lose from 2048 rows on)
+    if (need > 8 && a.M <= (need > 10 || a.K % 1024 == 0 ? 6144 : 2048)) return launch_shares<4>(a, s);
+  } else {
+    if (need == 4) return launch_quant<4, 8, LN>(a, s);
+    if (need > 4 && need <= 6) return launch_quant<6, 8, LN>(a, s);
+    if (need > 6 && need <= 8) return launch_quant<8, 8, LN>(a, s);
+  }
   if (need <= 2) return launch_quant<2, 8, LN>(a, s);
   if (need <= 3) return launch_quant<3, 8, LN>(a, s);
-  if (need <= 4) return launch_quant<4, 8, LN>(a, s);
-  if (need <= 6) return launch_quant<6, 8, LN>(a, s);
-  if (need <= 8) return launch_quant<8, 8, LN>(a, s);
   if (need <= 10) return launch_quant<10, 8, LN>(a, s);
   if (need <= 12) return launch_quant<12, 8, LN>(a, s);
   return launch_quant<16, 8, LN>(a, s);

@@ -56,3 +56,23 @@ def test_nan_and_shapes_through_the_native_route():
     x[1, 2, 7] = float("nan")
     nan = torch.isnan(m(x)).all(-1)
     assert nan[1, 2] and nan.sum() == 1
+
+
+@pytest.mark.parametrize("M,K", [(3, 1032), (1025, 1536), (8193, 1032), (1000, 2048), (1030, 2040), (7, 2560), (9, 3072), (5, 2176), (4097, 2184),
+                                 (6, 4096), (11, 3080), (5, 5120), (6145, 5120), (13, 4608), (3, 5128), (2, 8192)])
+def test_quantiser_with_shared_rows_bit_exact(M, K):
+    """Rows that two or four wavefronts share, in both layouts, with a NaN row and a zero row."""
+    import numpy as np
+    from samfast_amd import _lib, ops
+    print(f"case shared rows M={M} K={K}", flush=True)
+    x, _, _ = linear_inputs(M, K, 8, seed=M + K)
+    x[M - 1] = 0
+    q_ref, s_ref = orq.quantize_rows_absmax(x)
+    xq, sx = ops.quant_rowwise(x.cuda())
+    assert np.array_equal(xq.cpu().numpy(), q_ref) and np.array_equal(sx.cpu().numpy(), s_ref)
+    if K % 64 == 0:
+        xk, sk = ops.quant_rowwise(x.cuda(), _lib.LAYOUT_KB64)
+        assert torch.equal(ops.from_kb64(xk), xq) and torch.equal(sk, sx)
+    x[0, K - 1] = float("nan")
+    sn = ops.quant_rowwise(x.cuda())[1]
+    assert torch.isnan(sn[0]) and torch.equal(sn[1:], sx[1:])
