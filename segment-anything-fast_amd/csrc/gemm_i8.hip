@@ -623,10 +623,13 @@ __global__ __launch_bounds__(256, (TM == 4 ? 1 : 2)) void gemm_i8_kernel(GemmArg
 //     iteration to land;
 //   * the epilogue is staged through LDS 64 rows at a time (the full bf16 tile does not fit
 //     next to nothing in 48 KB), residual values are fetched after the conversion work.
-// The tile is BM x BN = 128 x 256 (waves 2 x 2, each 64 x 128: 2 x 4 MFMA tiles), or 64 x 128
-// (each wave 32 x 64: 1 x 2 tiles, 32 accumulators, 27 KB of LDS) for launches whose large tiles
-// would leave most of the GPU's workgroup slots empty (4096 rows of a single image): four times
-// the workgroups, each a quarter of the work.
+// The tile is BM x BN = 128 x 256 (waves 2 x 2, each 64 x 128: 2 x 4 MFMA tiles), 128 x 128 (each wave
+// 64 x 64: 2 x 2 tiles, 64 accumulators, 35 or 51 KB of LDS), or 64 x 128 (each wave 32 x 64: 1 x 2
+// tiles, 32 accumulators, 27 KB of LDS) for launches whose larger tiles would leave most of the GPU's
+// workgroup slots empty (the images of a small batch): two or four times the workgroups.
+// The loop is bound by LDS (fragment reads and tile writes: 288 / 384 / 576 cycles per k tile of a
+// 64 x 128 / 128 x 128 / 128 x 256 workgroup, against 128 / 256 / 512 of matrix instructions) and, on
+// operands that are not mostly zero, by the power limit.  STAGES = 3 keeps a tile more in flight.
 // KSPLIT = 2 (64 x 128 tiles only) puts eight wavefronts on a tile: wavefronts 0-3 take the even k
 // tiles, wavefronts 4-7 the odd ones, each half with operand stages of its own, so the chain of
 // dependent iterations a single small launch has to sit through is half as long (a 4096-row lin2 at
@@ -634,10 +637,10 @@ __global__ __launch_bounds__(256, (TM == 4 ? 1 : 2)) void gemm_i8_kernel(GemmArg
 // int32 and meet in LDS after the loop - integer addition is order-free, so the result has the
 // same bits - and wavefronts 0-3 run the epilogue.
 // =============================================================================================
-template <int BM, int BN, int KSPLIT = 1>
+template <int BM, int BN, int KSPLIT = 1, int STAGES = 2>
 struct Gemm3Cfg {
   static constexpr int TMW = BM / 64, TNW = BN / 64;  // MFMA tiles per wavefront: rows, columns
-  static constexpr int NST = 2;
+  static constexpr int NST = STAGES;
   static constexpr int GSTAGE = (BM + BN) * GLD;
   static constexpr int NLD = (BM + BN) / 64;          // global->LDS wave instructions per tile and wavefront
   static constexpr int EP_PITCH = BN * 2 + 32;        // staged output tile: row pitch in bytes
@@ -650,15 +653,15 @@ struct Gemm3Cfg {
   static constexpr int PASSES = 64 / ROWS_PER_PASS;   // passes over a staged 64-row tile
   static constexpr int MIN_WG = BM == 128 ? 3 : (KSPLIT == 2 ? 2 : 4);
   static_assert(64 * EP_PITCH <= NST * GSTAGE, "a 64-row output tile must fit in the operand stages");
-  static_assert((BM == 128 && BN == 256) || (BM == 64 && BN == 128), "tile shapes built");
+  static_assert((BM == 128 && (BN == 256 || BN == 128)) || (BM == 64 && BN == 128), "tile shapes built");
   static_assert(KSPLIT == 1 || (KSPLIT == 2 && BM == 64), "the K split is built for the small tile");
   static_assert(KSPLIT == 1 || BM * BN * 4 <= KSPLIT * NST * GSTAGE, "the partial sums must fit in the operand stages");
 };
 
-template <int EPI, int BM, int BN, int KSPLIT = 1>
-__global__ __launch_bounds__((Gemm3Cfg<BM, BN, KSPLIT>::THREADS), (Gemm3Cfg<BM, BN, KSPLIT>::MIN_WG)) void gemm_i8_kernel3(GemmArgs a) {
+template <int EPI, int BM, int BN, int KSPLIT = 1, int STAGES = 2>
+__global__ __launch_bounds__((Gemm3Cfg<BM, BN, KSPLIT, STAGES>::THREADS), (Gemm3Cfg<BM, BN, KSPLIT, STAGES>::MIN_WG)) void gemm_i8_kernel3(GemmArgs a) {
   static_assert(EPI != EPI_I32, "bf16 epilogues only");
-  using C = Gemm3Cfg<BM, BN, KSPLIT>;
+  using C = Gemm3Cfg<BM, BN, KSPLIT, STAGES>;
   constexpr int TMW = C::TMW, TNW = C::TNW, NLD = C::NLD, GSTAGE = C::GSTAGE;
   __shared__ __attribute__((aligned(16))) unsigned char lds_all[C::LDS_BYTES];
   unsigned char* sc = lds_all + KSPLIT * C::NST * GSTAGE;
@@ -743,15 +746,21 @@ __global__ __launch_bounds__((Gemm3Cfg<BM, BN, KSPLIT>::THREADS), (Gemm3Cfg<BM, 
   const int b_off = BM * GLD + (wn * (BN / 2) + lr) * GLD + frag_chunk;
 
   const int nk = a.K / GBK;
-  dma_issue(grp, 0);
-  for (int kt = grp, it = 0; kt < nk; kt += KSPLIT, ++it) {  // (K split: nk % KSPLIT == 0, both groups iterate alike)
-    const int stage_off = (it & 1) * GSTAGE;
-    // own share of tile kt has landed; after the barrier the whole tile is visible and every
-    // wavefront has left tile kt-1, whose stage may be refilled
-    __builtin_amdgcn_s_waitcnt(0x0070);
+#pragma unroll
+  for (int p = 0; p < C::NST - 1; ++p)
+    if (grp + p * KSPLIT < nk) dma_issue(grp + p * KSPLIT, p * GSTAGE);
+  int stage_off = 0, fill_off = (C::NST - 1) * GSTAGE;
+  for (int kt = grp; kt < nk; kt += KSPLIT) {  // (K split: nk % KSPLIT == 0, both groups iterate alike)
+    // own share of tile kt has landed (with three stages, tile kt+1 may still be on its way); after the
+    // barrier the whole tile is visible and every wavefront has left tile kt-1, whose stage may be refilled
+    constexpr int FLY = (C::NST - 2) * NLD;
+    static_assert(FLY < 16, "vmcnt threshold");
+    if (C::NST > 2 && kt + (C::NST - 2) * KSPLIT < nk) __builtin_amdgcn_s_waitcnt(0x0070 | FLY);
+    else __builtin_amdgcn_s_waitcnt(0x0070);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    if (kt + KSPLIT < nk) dma_issue(kt + KSPLIT, stage_off ^ GSTAGE);
+    if (kt + (C::NST - 1) * KSPLIT < nk) dma_issue(kt + (C::NST - 1) * KSPLIT, fill_off);
+    fill_off = fill_off == (C::NST - 1) * GSTAGE ? 0 : fill_off + GSTAGE;
     const unsigned char* src = lds + stage_off;
 #pragma unroll
     for (int step = 0; step < 2; ++step) {
@@ -767,6 +776,7 @@ __global__ __launch_bounds__((Gemm3Cfg<BM, BN, KSPLIT>::THREADS), (Gemm3Cfg<BM, 
         for (int i = 0; i < TMW; ++i)
           acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[i], bv[j], acc[i][j], 0, 0, 0);
     }
+    stage_off = stage_off == (C::NST - 1) * GSTAGE ? 0 : stage_off + GSTAGE;
   }
 
   bool active = true;  // whether this wavefront takes part in the epilogue's data movement
@@ -1004,24 +1014,41 @@ static int gemm_common(int epi, const int8_t* xq, const float* sx, const int8_t*
   const bool generic = generic_k;
   // the three-workgroups-per-CU form of the main kernel (SAMFAST_GEMM_WG3=0: two per CU)
   if (!tail && !generic && tm == 2 && epi != EPI_I32 && knob(KNOB_GEMM_WG3) != 0) {
-    // 64 x 128 tiles when 128 x 256 ones would leave more than half of the 768 workgroup slots of
-    // the GPU empty (SAMFAST_GEMM_TILE=64 / 128 forces either)
-    const int ft = knob(KNOB_GEMM_TILE);
-    const bool small = ft != kKnobUnset ? ft == 64 : total < knob_or(KNOB_GEMM_SMALL_BELOW, 385);
-    if (small) {
-      a.tiles_m = (int)((M + 63) / 64);
+    // The tile by the number of 128 x 128 ones the output has (us, random operands, 64 x 128 / 128 x 128 /
+    // 128 x 256; SAMFAST_GEMM_TILE forces one).  LDS bytes per matrix instruction fall by a third from
+    // each tile to the next; what stands against the larger tile is a GPU it does not fill.
+    //   up to 319: 64 x 128.       160 (2048 x 5120 -> 1280): 24.8 / 27.2 / 43.9, 240 (5000 x 3072 -> 768): 19.1 / 19.2 / 28.0
+    //   320 to 1024: 128 x 128.    640 (8192 x 5120 -> 1280): 66 / 59 / 65, 768 (12288 x 4096 -> 1024): 66 / 54 / 57,
+    //                              720 (5000 x 768 -> 2304): 17.8 / 15.6 / 17.6
+    //     but beyond 768 only on short K loops, without a residual.  960 (4096 x 1280 -> 3840): 32.5 / 25.9 / 25.8, with
+    //                              GELU 33.2 / 29.5 / 30.8, residual 32.9 / 28.5 / 28.0; 1024 (4096 x 4096 -> 4096): 87.5 / 69.0 / 67.0
+    //     and not for GELU after a loop of less than 16 k tiles: 1280 workgroup slots that are not all in
+    //                              the epilogue at once.  768 (4096 x 768 -> 3072) inside an encoder: 20.5 / 21.2
+    //   else 128 x 256.            1280 (4096 x 1280 -> 5120): 40 / 35 / 33
+    const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128);
+    const bool to_1024 = K <= 1280 && epi != EPI_RESIDUAL_BF16, gelu_short = epi == EPI_GELU_BF16 && K < 1024;
+    const int ft = knob_or(KNOB_GEMM_TILE, t128 < 320 || (gelu_short && t128 <= 768) ? 64 : t128 <= (to_1024 ? 1024 : 768) ? 96 : 128);
+    const bool small = ft == 64, middle = ft == 96;
+    if (small || middle) {
+      const int rows = small ? 64 : 128;
+      a.tiles_m = (int)((M + rows - 1) / rows);
       a.tiles_n = (N + 127) / 128;
-      a.group_m = a.tiles_n <= 6 ? 1 : 1024 / 64;
+      a.group_m = a.tiles_n <= 6 ? 1 : 1024 / rows;
     }
     const int64_t total3 = (int64_t)a.tiles_m * a.tiles_n;
     // small tiles that do not even fill the GPU's slots once, on a long K loop: two wavefront groups
     // per tile, each on every second k tile (SAMFAST_GEMM_SPLITK=0 off, 2 wherever it is built)
     const int sk = knob_or(KNOB_GEMM_SPLITK, 1);
     const bool ksplit = small && (K / GBK) % 2 == 0 && (sk >= 2 || (sk == 1 && total3 <= 768 && K / GBK >= 12));
+    // a third operand stage pays where the loop is long (320 tiles, 4096 x 5120 -> 1280: 39.7 -> 36.7;
+    // 960 tiles, K = 1280: 25.9 -> 27.7)
+    const bool deep = middle && K >= 1536;
     const unsigned int grid3 = (unsigned int)(((total3 + 7) / 8) * 8);
 #define SF_GEMM3(E)                                                                                          \
   do {                                                                                                       \
-    if (small && ksplit) hipLaunchKernelGGL((gemm_i8_kernel3<E, 64, 128, 2>), dim3(grid3), dim3(512), 0, stream, a); \
+    if (deep) hipLaunchKernelGGL((gemm_i8_kernel3<E, 128, 128, 1, 3>), dim3(grid3), dim3(256), 0, stream, a); \
+    else if (middle) hipLaunchKernelGGL((gemm_i8_kernel3<E, 128, 128>), dim3(grid3), dim3(256), 0, stream, a); \
+    else if (small && ksplit) hipLaunchKernelGGL((gemm_i8_kernel3<E, 64, 128, 2>), dim3(grid3), dim3(512), 0, stream, a); \
     else if (small) hipLaunchKernelGGL((gemm_i8_kernel3<E, 64, 128>), dim3(grid3), dim3(256), 0, stream, a); \
     else hipLaunchKernelGGL((gemm_i8_kernel3<E, 128, 256>), dim3(grid3), dim3(256), 0, stream, a);           \
   } while (0)

@@ -27,8 +27,7 @@ int check_launch(const char* what);
 enum Knob {
   KNOB_GEMM_TM,           // SAMFAST_GEMM_TM: 4 = 256 x 256 tiles in the two-per-CU kernel
   KNOB_GEMM_WG3,          // SAMFAST_GEMM_WG3: 0 = two workgroups per CU instead of three
-  KNOB_GEMM_TILE,         // SAMFAST_GEMM_TILE: 64 / 128 forces the small / large tile of the three-per-CU kernel
-  KNOB_GEMM_SMALL_BELOW,  // SAMFAST_GEMM_SMALL_BELOW: tile count below which the small tile is taken
+  KNOB_GEMM_TILE,         // SAMFAST_GEMM_TILE: 64 / 96 / 128 forces 64 x 128 / 128 x 128 / 128 x 256 tiles in the three-per-CU kernel
   KNOB_GEMM_PERSIST,      // SAMFAST_GEMM_PERSIST: 0 off, 1 where it pays, 2 wherever it is built
   KNOB_GEMM_PERSIST_SKEW, // SAMFAST_GEMM_PERSIST_SKEW: start delay of every second resident workgroup, 64 cycles per k tile
   KNOB_GEMM_PERSIST_PRIO, // SAMFAST_GEMM_PERSIST_PRIO: 0 = no wave priority changes in the persistent kernel

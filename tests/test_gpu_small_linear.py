@@ -76,3 +76,25 @@ def test_quantiser_with_shared_rows_bit_exact(M, K):
     x[0, K - 1] = float("nan")
     sn = ops.quant_rowwise(x.cuda())[1]
     assert torch.isnan(sn[0]) and torch.equal(sn[1:], sx[1:])
+
+
+@pytest.mark.parametrize("M,N,K,epi", [(2433, 2056, 256, 0), (2440, 2056, 1536, 0), (4000, 1288, 1344, 1), (1025, 4616, 1600, 2), (5000, 1288, 3072, 2)])
+def test_middle_tile_agrees_with_the_small_one(M, N, K, epi):
+    """128 x 128 tiles with two and three operand stages, ragged rows and columns: chosen by themselves,
+    the bits of the 64 x 128 tiles and of integer arithmetic."""
+    from samfast_amd import _lib, ops
+    print(f"case middle tile M={M} N={N} K={K} epi={epi}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    xq = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8)
+    wq = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8)
+    sx, sw, bias = torch.rand(M, generator=g) * 1e-3, torch.rand(N, generator=g) * 1e-2, torch.randn(N, generator=g)
+    res = torch.randn((M, N), generator=g).to(torch.bfloat16).cuda() if epi == _lib.EPILOGUE_RESIDUAL else None
+    xk, wk = ops.to_kb64(xq.cuda()), ops.to_kb64(wq.cuda())
+    run = lambda: ops.gemm_i8_fused(xk, sx.cuda(), wk, sw.cuda(), bias.cuda(), epi, residual=res, layout=_lib.LAYOUT_KB64)
+    y = run()
+    with _lib.knobs(SAMFAST_GEMM_TILE=64):
+        assert torch.equal(run(), y)
+    if epi == _lib.EPILOGUE_NONE:
+        rows = torch.tensor([0, 1, 63, 64, 127, 128, M - 130, M - 1])
+        acc = (xq[rows].double() @ wq.double().t()).float()
+        assert torch.equal(y[rows.cuda()].cpu(), (acc * sx[rows, None] * sw + bias).to(torch.bfloat16))
