@@ -100,7 +100,10 @@ static int launch_layernorm(const RowsArgs& a, hipStream_t stream) {
   using E8 = integral_constant<int, 8>;
   if (a.K == 768) return go(integral_constant<int, 3>{}, E4{});
   if (a.K == 1280) return go(integral_constant<int, 5>{}, E4{});
+  // the neck's 256 channels: every lane holds four of them (with 8 per lane half of the wavefront idles)
+  if (a.K <= 256) return go(integral_constant<int, 1>{}, E4{});
   const int need = (a.K / 8 + 63) / 64;
+  if (need <= 1) return go(integral_constant<int, 1>{}, E8{});
   if (need <= 2) return go(integral_constant<int, 2>{}, E8{});
   if (need <= 4) return go(integral_constant<int, 4>{}, E8{});
   return go(integral_constant<int, 8>{}, E8{});

@@ -48,3 +48,31 @@ def test_half_blocks_equal_module_composition(B, C, heads, window, bias, dtype, 
         assert not enc.blocks[0]._half_fused_ok(x)
         ref = enc.blocks[1](enc.blocks[0](x))
     assert ((y.float() - ref.float()).norm() / ref.float().norm()).item() < 8 * torch.finfo(dtype).eps
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,C,H,W", [(1, 256, 64, 64), (3, 256, 5, 7), (2, 8, 3, 3), (1, 264, 2, 3), (1, 512, 1, 5), (1, 520, 2, 2), (0, 256, 4, 4)])
+def test_layernorm2d_over_channels_last(B, C, H, W, dtype):
+    """One launch on a channels-last map; a contiguous one, and one under autograd, stay composed."""
+    from samfast_amd.modeling.common import LayerNorm2d
+    print(f"case layernorm2d {B}x{C}x{H}x{W} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(C + H)
+    norm = LayerNorm2d(C)
+    with torch.no_grad():
+        norm.weight.copy_(1 + 0.1 * torch.randn(C, generator=g))
+        norm.bias.copy_(0.1 * torch.randn(C, generator=g))
+    norm = norm.to(dtype)
+    x = (torch.randn((B, C, H, W), generator=g) * 2 + 0.5).to(dtype)
+    ref = F.layer_norm(x.permute(0, 2, 3, 1).double(), (C,), norm.weight.double(), norm.bias.double(), norm.eps).permute(0, 3, 1, 2)
+    gpu = norm.cuda()
+    xl = x.cuda().contiguous(memory_format=torch.channels_last)
+    eps = torch.finfo(dtype).eps
+    with torch.no_grad():
+        y = gpu(xl)
+        assert y.shape == x.shape and (B == 0 or gpu._rows_ok(xl))
+        # one rounding of the result, fp32 statistics
+        assert ((y.cpu().double() - ref).abs() <= eps * ref.abs() + 2e-5).all()
+        if B and H * W > 1:
+            # the composition rounds five intermediates to the type
+            assert ((gpu(x.cuda()).cpu().double() - ref).abs() <= 8 * eps * (ref.abs() + 1)).all()
+    assert not gpu._rows_ok(xl)  # gradients wanted
