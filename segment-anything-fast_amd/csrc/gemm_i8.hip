@@ -1008,12 +1008,17 @@ static int gemm_common(int epi, const int8_t* xq, const float* sx, const int8_t*
   SF_REQUIRE(total < (1ll << 30), "gemm_i8: too many tiles");
   // few rows: the K loop dealt out inside small tiles
   if (!tail && epi == EPI_SCALE_BIAS_BF16 && gemm_i8_skinny_covers(a)) return gemm_i8_skinny_launch(a, stream);
+  // outputs the GPU holds once, K >= 1280: one tile per CU (not where one of the other members is asked for)
+  if (!tail && tm == 2 && knob(KNOB_GEMM_TILE) == kKnobUnset && knob(KNOB_GEMM_WG3) != 0 && knob_or(KNOB_GEMM_PERSIST, 1) < 2 &&
+      knob_or(KNOB_GEMM_SPLITK, 1) < 2 && gemm_i8_once_covers(epi, a))
+    return gemm_i8_once_launch(epi, a, stream);
   // resident workgroups that walk a list of tiles each (SAMFAST_GEMM_PERSIST=1), where built
   if (!tail && !generic_k && tm == 2 && gemm_i8_persist_covers(epi, a)) return gemm_i8_persist_launch(epi, a, stream);
   const unsigned int grid = (unsigned int)(((total + 7) / 8) * 8);
   const bool generic = generic_k;
   // the three-workgroups-per-CU form of the main kernel (SAMFAST_GEMM_WG3=0: two per CU)
   if (!tail && !generic && tm == 2 && epi != EPI_I32 && knob(KNOB_GEMM_WG3) != 0) {
+    // (Most outputs of up to 256 tiles on a loop of K >= 1280 have left for gemm_i8_once.hip.)
     // The tile by the number of 128 x 128 ones the output has (us, random operands, 64 x 128 / 128 x 128 /
     // 128 x 256; SAMFAST_GEMM_TILE forces one).  LDS bytes per matrix instruction fall by a third from
     // each tile to the next; what stands against the larger tile is a GPU it does not fill.

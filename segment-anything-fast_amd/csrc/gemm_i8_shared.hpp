@@ -50,4 +50,8 @@ SF_DEVICE int lds_swizzle(int row) { return ((row >> 1) & 3) ^ ((row >> 3) & 1);
 bool gemm_i8_persist_covers(int epi, const GemmArgs& a);
 int gemm_i8_persist_launch(int epi, const GemmArgs& a, hipStream_t stream);
 
+// One tile per CU (gemm_i8_once.hip), the same way.
+bool gemm_i8_once_covers(int epi, const GemmArgs& a);
+int gemm_i8_once_launch(int epi, const GemmArgs& a, hipStream_t stream);
+
 }  // namespace samfast

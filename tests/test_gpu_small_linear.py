@@ -98,3 +98,31 @@ def test_middle_tile_agrees_with_the_small_one(M, N, K, epi):
         rows = torch.tensor([0, 1, 63, 64, 127, 128, M - 130, M - 1])
         acc = (xq[rows].double() @ wq.double().t()).float()
         assert torch.equal(y[rows.cuda()].cpu(), (acc * sx[rows, None] * sw + bias).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("bm,tn,M,N,K,epi", [
+    # (rows of the tile, columns / 32): whole tiles, ragged rows and columns, one tile, the shortest K loop and odd counts of k tiles
+    (128, 3, 4096, 768, 768, 2), (128, 3, 130, 200, 896, 0), (128, 4, 128, 128, 1024, 1), (128, 4, 2433, 1000, 3072, 2),
+    (128, 5, 4000, 1288, 1280, 2), (128, 5, 1, 8, 1408, 0), (256, 6, 257, 2304, 448, 0), (256, 6, 4096, 3072, 768, 1),
+    (256, 8, 1000, 776, 384, 1), (256, 8, 255, 4096, 1024, 0), (256, 10, 3900, 5120, 1280, 1), (256, 10, 513, 328, 576, 0),
+])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_one_tile_per_cu_agrees_with_the_small_tiles(bm, tn, M, N, K, epi, layout):
+    from samfast_amd import _lib, ops
+    print(f"case once {bm}x{32 * tn} M={M} N={N} K={K} epi={epi} layout={layout}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    xq = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8)
+    wq = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8)
+    sx, sw, bias = torch.rand(M, generator=g) * 1e-3, torch.rand(N, generator=g) * 1e-2, torch.randn(N, generator=g)
+    res = torch.randn((M, N), generator=g).to(torch.bfloat16).cuda() if epi == _lib.EPILOGUE_RESIDUAL else None
+    xk, wk = xq.cuda(), wq.cuda()
+    if layout == _lib.LAYOUT_KB64:
+        xk, wk = ops.to_kb64(xk), ops.to_kb64(wk)
+    run = lambda **kw: ops.gemm_i8_fused(xk, sx.cuda(), wk, sw.cuda(), bias.cuda() if M % 2 == 0 else None, epi, layout=layout, **kw)
+    with _lib.knobs(SAMFAST_GEMM_ONCE=bm * 16 + tn, SAMFAST_GEMM_SKINNY=0):
+        y = run(residual=res)
+        if res is not None:  # in place, as the encoder's residual stream
+            inplace = res.clone()
+            assert run(residual=inplace, out=inplace) is not None and torch.equal(inplace, y)
+    with _lib.knobs(SAMFAST_GEMM_TILE=64, SAMFAST_GEMM_SKINNY=0):
+        assert torch.equal(run(residual=res), y)
