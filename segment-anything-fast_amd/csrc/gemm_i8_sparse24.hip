@@ -131,10 +131,12 @@ SF_DEVICE void sp24_epilogue(const SparseArgs& a, i32x16 (&acc)[4][2], int x0, i
 // residual load instruction covers two whole 512-byte row segments.
 constexpr int SEP_STRIDE = 544;                     // tile row pitch in bytes
 
-template <int EPI>
-SF_DEVICE void sp24_epilogue_staged(const SparseArgs& a, i32x16 (&acc)[4][2], unsigned char* lds,
+// KS groups of 256 threads share it: with two, a wavefront holds X tile tb0 of its 64 X rows only.
+template <int EPI, int KS>
+SF_DEVICE void sp24_epilogue_staged(const SparseArgs& a, i32x16 (&acc)[4][2 / KS], unsigned char* lds,
                                     const unsigned char* sc, int x0, int w0, int wa, int wb,
-                                    int lr, int lh, int tid) {
+                                    int lr, int lh, int tid, int tb0) {
+  constexpr int NTB = 2 / KS, PASSES = 16 / KS, RPP = 8 * KS;  // output rows per pass
   __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt 0, lgkmcnt 0
   __builtin_amdgcn_s_barrier();        // nobody reads operand stages any more
   __builtin_amdgcn_sched_barrier(0);
@@ -143,13 +145,13 @@ SF_DEVICE void sp24_epilogue_staged(const SparseArgs& a, i32x16 (&acc)[4][2], un
   const int n = w0 + chunk * 8;
   const bool col_ok = n < a.N;  // N % 8 == 0
   auto out_row = [&](int p) {
-    const int m = x0 + 8 * p + rsub;
+    const int m = x0 + RPP * p + rsub;
     return (m < a.M && col_ok) ? m : -1;
   };
-  u32x4 res[16];
+  u32x4 res[PASSES];
   if (EPI == SEPI_RESIDUAL) {  // requested before the conversion work, waited for once
 #pragma unroll
-    for (int p = 0; p < 16; ++p) {
+    for (int p = 0; p < PASSES; ++p) {
       const u32x4 z = {0u, 0u, 0u, 0u};
       res[p] = z;
       const int dr = out_row(p);
@@ -157,9 +159,9 @@ SF_DEVICE void sp24_epilogue_staged(const SparseArgs& a, i32x16 (&acc)[4][2], un
     }
   }
   {
-    float sxs[2];
+    float sxs[NTB];
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb) sxs[tb] = *reinterpret_cast<const float*>(sc + (wb * 64 + tb * 32 + lr) * 4);
+    for (int tb = 0; tb < NTB; ++tb) sxs[tb] = *reinterpret_cast<const float*>(sc + (wb * 64 + (tb0 + tb) * 32 + lr) * 4);
 #pragma unroll
     for (int g = 0; g < 4; ++g)
 #pragma unroll
@@ -174,7 +176,7 @@ SF_DEVICE void sp24_epilogue_staged(const SparseArgs& a, i32x16 (&acc)[4][2], un
           bv[t] = a.bias ? *reinterpret_cast<const f32x4*>(sc + 1536 + (nl + 4 * t) * 4) : z;
         }
 #pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
+        for (int tb = 0; tb < NTB; ++tb) {
           u32x4 o;
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
@@ -194,7 +196,7 @@ SF_DEVICE void sp24_epilogue_staged(const SparseArgs& a, i32x16 (&acc)[4][2], un
             for (int c = 0; c < 4; ++c)
               o[c] = pack_bf16x2(gelu_erf(bf16_lo_to_f32(o[c])), gelu_erf(bf16_hi_to_f32(o[c])));
           }
-          *reinterpret_cast<u32x4*>(lds + (wb * 64 + tb * 32 + lr) * SEP_STRIDE + nl * 2) = o;
+          *reinterpret_cast<u32x4*>(lds + (wb * 64 + (tb0 + tb) * 32 + lr) * SEP_STRIDE + nl * 2) = o;
         }
       }
   }
@@ -204,9 +206,9 @@ SF_DEVICE void sp24_epilogue_staged(const SparseArgs& a, i32x16 (&acc)[4][2], un
 
   unsigned short* outp = reinterpret_cast<unsigned short*>(a.out);
 #pragma unroll
-  for (int p = 0; p < 16; ++p) {
+  for (int p = 0; p < PASSES; ++p) {
     const int dr = out_row(p);
-    u32x4 val = *reinterpret_cast<const u32x4*>(lds + (8 * p + rsub) * SEP_STRIDE + chunk * 16);
+    u32x4 val = *reinterpret_cast<const u32x4*>(lds + (RPP * p + rsub) * SEP_STRIDE + chunk * 16);
     if (EPI == SEPI_RESIDUAL) {
 #pragma unroll
       for (int c = 0; c < 4; ++c)
@@ -217,14 +219,20 @@ SF_DEVICE void sp24_epilogue_staged(const SparseArgs& a, i32x16 (&acc)[4][2], un
   }
 }
 
-template <int EPI>
-__global__ __launch_bounds__(256, 2) void gemm_i8_sp24_kernel(SparseArgs a) {
+// KS = 2: two groups of four wavefronts per tile, each on every second k tile with stages of its own; the
+// integer sums meet in LDS and each group finishes one of a wavefront's two X tiles.  For outputs of so
+// few tiles that a CU has one: its SIMDs would hold one wavefront, whose every barrier and fragment read is waited for.
+template <int EPI, int KS = 1>
+__global__ __launch_bounds__(256 * KS, 2) void gemm_i8_sp24_kernel(SparseArgs a) {
   constexpr int NST = S_NST;
   constexpr bool STAGED = EPI != SEPI_I32;  // epilogue through LDS
   static_assert(128 * SEP_STRIDE <= NST * S_STAGE, "output tile must fit in the operand stages");
-  __shared__ __attribute__((aligned(16))) unsigned char lds[NST * S_STAGE + (STAGED ? SEP_SCALE_BYTES : 0)];
+  static_assert(KS == 1 || (KS == 2 && STAGED), "the K split is built for the staged epilogues");
+  __shared__ __attribute__((aligned(16))) unsigned char lds_all[KS * NST * S_STAGE + (STAGED ? SEP_SCALE_BYTES : 0)];
 
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x & 255;  // inside the group
+  const int grp = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  unsigned char* lds = lds_all + grp * (NST * S_STAGE);  // the group's operand stages
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wa = wave >> 1, wb = wave & 1;  // position along W rows / X rows
@@ -258,9 +266,10 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_sp24_kernel(SparseArgs a) {
   typedef __attribute__((address_space(1))) const void* gptr_t;
   typedef __attribute__((address_space(3))) void* lptr_t;
   auto dma_issue = [&](int kt, int stage_off) {
-    const int8_t* xb = a.x + kt * a.x_kstep;
-    const int8_t* wb_ = a.wc + (int64_t)kt * a.N * 32;
-    const int8_t* ib = reinterpret_cast<const int8_t*>(a.widx) + (int64_t)kt * a.N * 8;
+    const int k = kt * KS + grp;
+    const int8_t* xb = a.x + k * a.x_kstep;
+    const int8_t* wb_ = a.wc + (int64_t)k * a.N * 32;
+    const int8_t* ib = reinterpret_cast<const int8_t*>(a.widx) + (int64_t)k * a.N * 8;
     // tile bases stay in scalar registers and the lane offsets 32-bit at the point of use, so the
     // loads take the scalar-base form (the 64-bit per-lane address form costs the MFMA stream
     // several times more per load)
@@ -325,7 +334,7 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_sp24_kernel(SparseArgs a) {
   if constexpr (STAGED) {
     // row scales, column scales and bias of this tile, 4 bytes per lane, straight into LDS; they
     // are the oldest loads in flight, so every later vmcnt wait covers them
-    unsigned char* sc = lds + NST * S_STAGE;
+    unsigned char* sc = lds_all + KS * NST * S_STAGE;  // (both groups fetch the same)
     const int mm = min(x0 + (wave_u & 1) * 64 + lane, a.M - 1);
     const int nn = min(w0 + wave_u * 64 + lane, a.N - 1);
     __builtin_amdgcn_global_load_lds((gptr_t)(a.sx + mm), (lptr_t)(sc + (wave_u & 1) * 256), 4, 0, 0);
@@ -333,7 +342,7 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_sp24_kernel(SparseArgs a) {
     __builtin_amdgcn_global_load_lds((gptr_t)((a.bias ? a.bias : a.sw) + nn),
                                      (lptr_t)(sc + 1536 + wave_u * 256), 4, 0, 0);
   }
-  const int nk = a.K / SBK;  // even and >= NST (checked by the host)
+  const int nk = a.K / SBK / KS;  // even and >= NST (checked by the host)
   int st[NST];  // st[j] = LDS offset of the stage holding tile kt + j (uniform, rotated)
 #pragma unroll
   for (int j = 0; j < NST; ++j) {
@@ -399,8 +408,37 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_sp24_kernel(SparseArgs a) {
   iteration(kt + 2, C0{}, C0{}, C1{}, C0{});
   iteration(kt + 3, C1{}, C0{}, C0{}, C0{});
 
-  if constexpr (STAGED)
-    sp24_epilogue_staged<EPI>(a, acc, lds, lds + NST * S_STAGE, x0, w0, wa, wb, lr, lh, tid);
+  if constexpr (KS == 2) {
+    // group g finishes X tile g: the other group's share of it comes through LDS
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();  // nobody reads operand stages any more
+    __builtin_amdgcn_sched_barrier(0);
+    i32x4* red = reinterpret_cast<i32x4*>(lds_all);
+    static_assert(2 * 256 * 16 * 16 <= KS * NST * S_STAGE, "the partial sums must fit in the operand stages");
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        i32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = grp == 0 ? acc[i][1][4 * r + e] : acc[i][0][4 * r + e];
+        red[((1 - grp) * 16 + 4 * i + r) * 256 + tid] = v;
+      }
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    i32x16 sum[4][1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const i32x4 v = red[(grp * 16 + 4 * i + r) * 256 + tid];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[i][0][4 * r + e] = v[e] + (grp == 0 ? acc[i][0][4 * r + e] : acc[i][1][4 * r + e]);
+      }
+    sp24_epilogue_staged<EPI, KS>(a, sum, lds_all, lds_all + KS * NST * S_STAGE, x0, w0, wa, wb, lr, lh, threadIdx.x, grp);
+  } else if constexpr (STAGED)
+    sp24_epilogue_staged<EPI, KS>(a, acc, lds_all, lds_all + NST * S_STAGE, x0, w0, wa, wb, lr, lh, tid, 0);
   else
     sp24_epilogue<EPI>(a, acc, x0, w0, wa, wb, lr, lh);
 }
@@ -501,16 +539,25 @@ static int sparse_common(int epi, const int8_t* xq, const float* sx, const int8_
   if (gemm_i8_sp24_skinny_covers(epi, a)) return gemm_i8_sp24_skinny_launch(a, stream);
   if (gemm_i8_sp24_persist_covers(epi, a)) return gemm_i8_sp24_persist_launch(epi, a, stream);
   const unsigned int grid = (unsigned int)(((total + 7) / 8) * 8);
+  // The K split where a CU has one tile and the loop is long (us, one group / two; SAMFAST_GEMM_SPLITK=0 off, 2
+  // wherever it is built): 5003 x 5120 -> 1280 (200 tiles) 27.9 / 26.5, 4096 x 5120 -> 1280 (160) 27.9 / 25.8, 1500 x 5120
+  // -> 1280 (60) 24.9 / 22.0, 4096 x 3072 -> 768 (96) 19.3 / 17.9, 8192 x 3072 -> 768 (192) 20.6 / 20.6.  Shorter loops do not pay
+  // for the meeting in LDS (6500 x 1280 -> 1280: 13.5 / 14.2), and two tiles to a CU are better apart (8192 x 5120 ->
+  // 1280, 320 tiles: 43.3 / 51.3).  What bounds both is operand delivery, 12 TB/s over the CUs in use.
+  const int sk = knob_or(KNOB_GEMM_SPLITK, 1);
+  const bool ksplit = epi != SEPI_I32 && K % (4 * SBK) == 0 && K / SBK >= 2 * S_NST && (sk >= 2 || (sk == 1 && total <= 208 && K >= 3072));
+#define SF_SP24(E)                                                                                              \
+  do {                                                                                                          \
+    if (ksplit) hipLaunchKernelGGL((gemm_i8_sp24_kernel<E, 2>), dim3(grid), dim3(512), 0, stream, a);           \
+    else hipLaunchKernelGGL((gemm_i8_sp24_kernel<E>), dim3(grid), dim3(256), 0, stream, a);                     \
+  } while (0)
   switch (epi) {
-    case SEPI_I32:
-      hipLaunchKernelGGL((gemm_i8_sp24_kernel<SEPI_I32>), dim3(grid), dim3(256), 0, stream, a); break;
-    case SEPI_SCALE_BIAS:
-      hipLaunchKernelGGL((gemm_i8_sp24_kernel<SEPI_SCALE_BIAS>), dim3(grid), dim3(256), 0, stream, a); break;
-    case SEPI_GELU:
-      hipLaunchKernelGGL((gemm_i8_sp24_kernel<SEPI_GELU>), dim3(grid), dim3(256), 0, stream, a); break;
-    default:
-      hipLaunchKernelGGL((gemm_i8_sp24_kernel<SEPI_RESIDUAL>), dim3(grid), dim3(256), 0, stream, a); break;
+    case SEPI_I32: hipLaunchKernelGGL((gemm_i8_sp24_kernel<SEPI_I32>), dim3(grid), dim3(256), 0, stream, a); break;
+    case SEPI_SCALE_BIAS: SF_SP24(SEPI_SCALE_BIAS); break;
+    case SEPI_GELU: SF_SP24(SEPI_GELU); break;
+    default: SF_SP24(SEPI_RESIDUAL); break;
   }
+#undef SF_SP24
   return check_launch("gemm_i8_sp24_kernel");
 }
 

@@ -31,7 +31,7 @@ enum Knob {
   KNOB_GEMM_PERSIST,      // SAMFAST_GEMM_PERSIST: 0 off, 1 where it pays, 2 wherever it is built
   KNOB_GEMM_PERSIST_SKEW, // SAMFAST_GEMM_PERSIST_SKEW: start delay of every second resident workgroup, 64 cycles per k tile
   KNOB_GEMM_PERSIST_PRIO, // SAMFAST_GEMM_PERSIST_PRIO: 0 = no wave priority changes in the persistent kernel
-  KNOB_GEMM_SPLITK,       // SAMFAST_GEMM_SPLITK: 0 off, 1 where it pays (launches that leave the GPU half empty)
+  KNOB_GEMM_SPLITK,       // SAMFAST_GEMM_SPLITK: 0 off, 1 where it pays (launches that leave the GPU half empty; 2:4: one tile per CU), 2 wherever built
   KNOB_GEMM_ONCE,         // SAMFAST_GEMM_ONCE: 0 = off, 1 where it pays, rows * 16 + columns / 32 = that tile of the one-tile-per-CU kernel
   KNOB_LINEAR_SMALL,      // SAMFAST_GEMM_LINEAR_SMALL: 0 = whole Linears over few rows as two launches as well
   KNOB_GEMM_SKINNY,       // SAMFAST_GEMM_SKINNY: 0 = products over few rows through the tiled kernels

@@ -265,3 +265,27 @@ def test_seeded_sweep_of_ragged_shapes_sparse_bit_exact():
         ref = orq.int8_gemm_i64(xq.numpy(), dense)
         acc = ops.gemm_i8_sparse24_i32(xq.cuda(), wc, widx)
         assert np.array_equal(acc.cpu().numpy().astype(np.int64), ref)
+
+
+@pytest.mark.parametrize("M,N,K,epi", [(1, 8, 512, 0), (5003, 1280, 5120, 0), (130, 264, 768, 1), (4096, 768, 3072, 2), (129, 1288, 512, 2), (257, 520, 1280, 1)])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_sparse24_split_k_loop_agrees(M, N, K, epi, layout):
+    """Two wavefront groups on alternate k tiles: the bits of one group walking them all."""
+    from samfast_amd import _lib, ops
+    print(f"case sparse split M={M} N={N} K={K} epi={epi} layout={layout}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    xq = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8).cuda()
+    wc, widx = ops.prune24_pack(torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8).cuda())
+    sx, sw = (torch.rand(M, generator=g) * 1e-3).cuda(), (torch.rand(N, generator=g) * 1e-2).cuda()
+    bias = torch.randn(N, generator=g).cuda() if M % 2 else None
+    res = torch.randn((M, N), generator=g).to(torch.bfloat16).cuda() if epi == _lib.EPILOGUE_RESIDUAL else None
+    x = ops.to_kb64(xq) if layout == _lib.LAYOUT_KB64 else xq
+    run = lambda **kw: ops.gemm_i8_sparse24_fused(x, sx, wc, widx, sw, bias, epi, layout=layout, **kw)
+    with _lib.knobs(SAMFAST_GEMM_SKINNY=0, SAMFAST_GEMM_SPLITK=0):
+        want = run(residual=res)
+    with _lib.knobs(SAMFAST_GEMM_SKINNY=0, SAMFAST_GEMM_SPLITK=2):
+        assert torch.equal(run(residual=res), want)
+        if res is not None:
+            buf = res.clone()
+            run(residual=buf, out=buf)
+            assert torch.equal(buf, want)
