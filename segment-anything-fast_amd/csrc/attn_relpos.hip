@@ -558,6 +558,26 @@ __global__ __launch_bounds__(WindowCfg<HD>::THREADS, 2) void attn_window_kernel(
     }
   };
   window_dma(kbase, a.k_sn, kpad, kl);
+  // V rows past the last key, up to the 16-key step boundary, are multiplied by P = 0: zeros; and the ones
+  // channel (P = 0 beyond the last key anyway)
+  auto v_rest = [&]() {
+    for (int idx = tid; idx < (16 * nsteps - N) * (HD / 8); idx += C::THREADS) {
+      const int row = N + idx / (HD / 8), col = idx % (HD / 8);
+      const u32x4 z = {0u, 0u, 0u, 0u};
+      *reinterpret_cast<u32x4*>(vl + (row * C::VSTR + col * 8) * 2) = z;
+    }
+    if (C::ONES_ROW && tid < 16 * nsteps) {
+      const u32x4 one = {T::kOne, 0u, 0u, 0u};
+      *reinterpret_cast<u32x4*>(vl + (tid * C::VSTR + HD) * 2) = one;
+    }
+  };
+  // With the caller's factors nothing else lives in V's area: V travels with K, one memory latency and one
+  // barrier less (with the factors' pairs below: 25 x 12 windows of 14 x 14 x 64 16.3 -> 15.7 us, 10 x 12 x 80 10.6 ->
+  // 10.0, 400 x 16 x 80 193 -> 187)
+  if constexpr (!FUSED) {
+    window_dma(vbase, a.v_sn, vpad, vl);
+    v_rest();
+  }
 
   // ---- bias operands while the staging loads are in flight: lane (query, lh) element e <->
   //      slot 8*lh + e.  The gather scratch lives where K will be stored afterwards ----------
@@ -609,19 +629,35 @@ __global__ __launch_bounds__(WindowCfg<HD>::THREADS, 2) void attn_window_kernel(
     } else {
       const unsigned short* rhp = a.rh + b * a.rh_sb + h * a.rh_sh + (int64_t)qc * a.rh_sn;
       const unsigned short* rwp = a.rw + b * a.rw_sb + h * a.rw_sh + (int64_t)qc * a.rw_sn;
+      if (a.rel_x2) {
+        // rows of an even number of factors that start on 4 bytes: the lane's eight slots as four pairs
+        u32x4 ph, pw;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float fh[2] = {0.f, 0.f}, fw[2] = {0.f, 0.f};
-#pragma unroll
-        for (int v = 0; v < 2; ++v) {
-          const int slot = 8 * lh + 2 * i + v;
-          const float rh_raw = T::from_bits(rhp[min(slot, a.gh - 1)]) * a.inv_scale;
-          const float rw_raw = T::from_bits(rwp[min(slot, a.gw - 1)]) * a.inv_scale;
-          fh[v] = (slot < a.gh) ? rh_raw : 0.f;
-          fw[v] = (slot < a.gw) ? rw_raw : 0.f;
+        for (int i = 0; i < 4; ++i) {
+          ph[i] = reinterpret_cast<const unsigned int*>(rhp)[min(4 * lh + i, a.gh / 2 - 1)];
+          pw[i] = reinterpret_cast<const unsigned int*>(rwp)[min(4 * lh + i, a.gw / 2 - 1)];
         }
-        bhw[i] = T::pack2(fh[0], fh[1]);
-        bww[i] = T::pack2(fw[0], fw[1]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int slot = 8 * lh + 2 * i;
+          bhw[i] = slot < a.gh ? T::pack2(T::lo(ph[i]) * a.inv_scale, T::hi(ph[i]) * a.inv_scale) : 0u;
+          bww[i] = slot < a.gw ? T::pack2(T::lo(pw[i]) * a.inv_scale, T::hi(pw[i]) * a.inv_scale) : 0u;
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float fh[2] = {0.f, 0.f}, fw[2] = {0.f, 0.f};
+#pragma unroll
+          for (int v = 0; v < 2; ++v) {
+            const int slot = 8 * lh + 2 * i + v;
+            const float rh_raw = T::from_bits(rhp[min(slot, a.gh - 1)]) * a.inv_scale;
+            const float rw_raw = T::from_bits(rwp[min(slot, a.gw - 1)]) * a.inv_scale;
+            fh[v] = (slot < a.gh) ? rh_raw : 0.f;
+            fw[v] = (slot < a.gw) ? rw_raw : 0.f;
+          }
+          bhw[i] = T::pack2(fh[0], fh[1]);
+          bww[i] = T::pack2(fw[0], fw[1]);
+        }
       }
     }
     if (lh == 1) bhw[3] = (bhw[3] & 0xffffu) | (T::kMask << 16);  // slot 15: the masking value
@@ -632,18 +668,11 @@ __global__ __launch_bounds__(WindowCfg<HD>::THREADS, 2) void attn_window_kernel(
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's share of K has landed
   __syncthreads();  // K complete; every wavefront is done with the scratch: V may overwrite it
-  window_dma(vbase, a.v_sn, vpad, vl);
-  // V rows past the last key, up to the 16-key step boundary, are multiplied by P = 0: zeros
-  for (int idx = tid; idx < (16 * nsteps - N) * (HD / 8); idx += C::THREADS) {
-    const int row = N + idx / (HD / 8), col = idx % (HD / 8);
-    const u32x4 z = {0u, 0u, 0u, 0u};
-    *reinterpret_cast<u32x4*>(vl + (row * C::VSTR + col * 8) * 2) = z;
+  if constexpr (FUSED) {
+    window_dma(vbase, a.v_sn, vpad, vl);
+    v_rest();
   }
-  if (C::ONES_ROW && tid < 16 * nsteps) {  // the ones channel (P = 0 beyond the last key anyway)
-    const u32x4 one = {T::kOne, 0u, 0u, 0u};
-    *reinterpret_cast<u32x4*>(vl + (tid * C::VSTR + HD) * 2) = one;
-  }
-  if (!has_tile) {  // a wavefront without a query tile only helps with the staging and with the output
+  if (FUSED && !has_tile) {  // a wavefront without a query tile only helps with the staging and with the output
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();  // V complete (the barrier the others reach after their first score tile)
   }
@@ -735,10 +764,10 @@ __global__ __launch_bounds__(WindowCfg<HD>::THREADS, 2) void attn_window_kernel(
           if (!C::ONES_ROW) lsum += p;
         }
         if (!C::ONES_ROW) l_run = l_run * alpha + lsum;
-        if (nt == 0) {  // V travelled under the first score tile; every wavefront's share has landed
+        if (FUSED && nt == 0) {  // V travelled under the first score tile; every wavefront's share has landed
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
           __syncthreads();
-        } else if (move) {
+        } else if (nt > 0 && move) {
 #pragma unroll
           for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
@@ -890,6 +919,9 @@ static int attn_dispatch(bool fused, AttnArgs& a, int hd, int dtype, float sm_sc
   if (a.B == 0) return SAMFAST_OK;
   a.c = sm_scale * kLog2e;
   a.inv_scale = 1.0f / sm_scale;
+  // both factors' rows can be read in pairs: no pair reaches past a row's end or straddles a word
+  a.rel_x2 = !fused && a.gh % 2 == 0 && a.gw % 2 == 0 && ((reinterpret_cast<uintptr_t>(a.rh) | reinterpret_cast<uintptr_t>(a.rw)) & 3u) == 0 &&
+             ((a.rh_sb | a.rh_sh | a.rh_sn | a.rw_sb | a.rw_sh | a.rw_sn) & 1) == 0;
   // windows whose rows fit the padded-row key layout take that kernel (attn_window_rows.hip)
   if (!global_path && attn_window_rows_covers(a)) return attn_window_rows_launch(a, hd, dtype, fused, stream);
   if (global_path && !fused) return attn_global_bias_launch(a, hd, dtype, stream);

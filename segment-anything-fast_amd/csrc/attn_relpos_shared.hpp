@@ -29,6 +29,7 @@ struct AttnArgs {
   const unsigned short* pad_k;
   const unsigned short* pad_v;
   int relh_x8;  // attn_global_bias.hip: rel_h rows can be read 16 bytes at a time
+  int rel_x2;   // window kernel: rows of the caller's factors can be read 4 bytes at a time
 };
 
 constexpr float kLog2e = 1.4426950408889634f;

@@ -50,3 +50,28 @@ def test_bias_kernels_read_strided_factors():
     a = ops.attn_relpos_bias(q, k, v, both[..., :64], both[..., 64:])
     b = ops.attn_relpos_bias(q.contiguous(), k.contiguous(), v.contiguous(), both[..., :64].contiguous(), both[..., 64:].contiguous())
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("gh,gw", [(14, 14), (2, 2), (13, 14), (14, 5), (6, 8), (1, 16), (15, 13)])
+@pytest.mark.parametrize("hd,dtype", [(64, torch.bfloat16), (80, torch.float16)])
+def test_window_factors_read_in_pairs_or_one_by_one(gh, gw, hd, dtype):
+    """Factor rows of even length are read as pairs where they start on 4 bytes; a view that starts on
+    2 takes single reads, with the same bits, and both follow the softmax in 64 bits."""
+    from samfast_amd.flash_4 import _attention_rel_h_rel_w
+    print(f"case window factors {gh}x{gw} hd={hd} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(gh * 100 + gw + hd)
+    N = gh * gw
+    q, k, v = (torch.randn((3, 2, N, hd), generator=g).mul(0.5).to(dtype) for _ in range(3))
+    rh, rw = torch.randn((3, 2, N, gh, 1), generator=g).mul(0.5).to(dtype), torch.randn((3, 2, N, 1, gw), generator=g).mul(0.5).to(dtype)
+
+    def shifted(t):  # the same values one element into a longer buffer
+        return torch.cat([torch.zeros(1, dtype=dtype), t.flatten()]).cuda()[1:].view(t.shape)
+
+    args = [t.cuda() for t in (q, k, v)]
+    y = _attention_rel_h_rel_w(*args, rh.cuda(), rw.cuda())
+    assert torch.equal(y, _attention_rel_h_rel_w(*args, shifted(rh), shifted(rw)))
+    s = q.double() @ k.double().transpose(-1, -2) * hd ** -0.5 + (rh.double() + rw.double()).flatten(-2)
+    ref = s.softmax(-1) @ v.double()
+    # probabilities and result in the half type, as the operator's other tests
+    eps = torch.finfo(dtype).eps
+    assert (y.cpu().double() - ref).abs().max() <= 4 * eps * v.abs().max().item()
