@@ -76,3 +76,17 @@ def test_layernorm2d_over_channels_last(B, C, H, W, dtype):
             # the composition rounds five intermediates to the type
             assert ((gpu(x.cuda()).cpu().double() - ref).abs() <= 8 * eps * (ref.abs() + 1)).all()
     assert not gpu._rows_ok(xl)  # gradients wanted
+
+
+def test_layernorm2d_stays_composed_under_transforms():
+    from samfast_amd.modeling.common import LayerNorm2d
+    norm = LayerNorm2d(16).to(torch.bfloat16).cuda()
+    x = torch.randn((2, 3, 16, 4, 4), device="cuda").to(torch.bfloat16).flatten(0, 1).contiguous(memory_format=torch.channels_last).view(2, 3, 16, 4, 4)
+    with torch.no_grad():
+        want = torch.stack([norm(t) for t in x])
+        assert norm._rows_ok(x[0])
+        got = torch.vmap(norm)(x)
+        assert (got.float() - want.float()).abs().max() <= 8 * torch.finfo(torch.bfloat16).eps * (want.float().abs().max() + 1)
+        with torch.autograd.forward_ad.dual_level():
+            dual = torch.autograd.forward_ad.make_dual(x[0], torch.ones_like(x[0]))
+            assert torch.autograd.forward_ad.unpack_dual(norm(dual)).tangent is not None
