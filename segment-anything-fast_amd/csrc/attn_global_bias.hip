@@ -173,7 +173,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
   for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
-  float m_i = -INFINITY, l_i = 0.f;
+  float m_i = T::kLowest, l_i = 0.f;
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) s16x4* trptr_t;
 
@@ -209,9 +209,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
     // maximum: probabilities may sit anywhere below 2 (the final division by the denominator,
     // accumulated with the same offsets, makes the result independent of it), so no maximum is taken in
     // the common case.  Whether one has reached 2 shows in the top exponent bit of the packed pairs,
-    // or-ed together.  Then - always in the first half row, where m_i is -inf, and again when the maximum has
-    // grown by T::kMargin powers of two - the maximum is found, the accumulators are rescaled and the
-    // probabilities formed once more.
+    // or-ed together.  Then - always where the first keys are met, m_i being T::kLowest, and again when the maximum
+    // has grown by T::kMargin powers of two - the maximum is found, the accumulators are rescaled and the
+    // probabilities formed once more.  m_i is finite throughout: keys that a factor of -inf, or of the type's lowest
+    // value, has taken away have probabilities of zero whatever stands before or behind them.
     unsigned int seen = 0u;
     auto pair = [&](int w, float neg_mrow) __attribute__((always_inline)) {  // packed pair w of 8
       pk[w >> 2][w & 3] = T::pack2(fast_exp2(fmaf(s[2 * w], a.c, neg_mrow)), fast_exp2(fmaf(s[2 * w + 1], a.c, neg_mrow)));
@@ -253,8 +254,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
       mx = max_with_lane_xor32(mx);
-      const float m_new = fmaxf(m_i, fmaf(mx, a.c, b0) + T::kMargin);
-      const float alpha = fast_exp2(m_i - m_new);  // first half row: 0
+      const float m_new = fmaxf(m_i, fmaf(mx, a.c, b0 + T::kMargin));
+      const float alpha = fast_exp2(m_i - m_new);  // first keys: 0; none yet: 1, on accumulators of zero
       m_i = m_new;
       l_i *= alpha;
 #pragma unroll
@@ -485,7 +486,7 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
   for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
-  float m_i = -INFINITY, l_i = 0.f;
+  float m_i = T::kLowest, l_i = 0.f;
 
   const int nkt = a.N / 64;
   typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -563,7 +564,7 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
       mx = max_with_lane_xor32(mx);
-      const float m_new = fmaxf(m_i, fmaf(mx, a.c, b0) + T::kMargin);
+      const float m_new = fmaxf(m_i, fmaf(mx, a.c, b0 + T::kMargin));
       const float alpha = fast_exp2(m_i - m_new);
       m_i = m_new;
       l_i *= alpha;
@@ -609,6 +610,7 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
   __syncthreads();
   if (kg == 1) return;
   {
+    // (a half all of whose keys are taken away: its reference is T::kLowest, its sums are zero)
     const float m1 = other[64 * 16 * C::DT], l1 = other[64 * (16 * C::DT + 1)];
     const float m = fmaxf(m_i, m1);
     const float f0 = fast_exp2(m_i - m), f1 = fast_exp2(m1 - m);

@@ -43,6 +43,10 @@ struct ElemBf16 {
   // global kernel: how far (log2) above the running maximum the exponent reference is put; bf16
   // probabilities keep their eight bits at any size
   static constexpr float kMargin = 16.0f;
+  // global kernel with the caller's factors: the exponent reference (log2) before any key has been met.  Keys below it
+  // are as good as masked.  Down to it every probability is finite: at 2^31 a reference and a difference from it
+  // are each rounded by at most 64, so that a probability stays below 2^(128 - kMargin).
+  static constexpr float kLowest = -2147483648.0f;
   static constexpr unsigned int kMask = 0xF149u;  // -1e30: added to a score (before the scale), it removes the key
   static SF_DEVICE f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
@@ -61,6 +65,7 @@ struct ElemF16 {
   typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
   static constexpr unsigned int kOne = 0x3C00u;   // 1.0
   static constexpr float kMargin = 4.0f;  // fp16 ends at 2^-24: 2^-20 of the maximum, against 2^-11 of a rounding
+  static constexpr float kLowest = -134217728.0f;  // as above, with 2^27, roundings of 4 and 65504 as the end
   static constexpr unsigned int kMask = 0xFB53u;  // -60000 (fp16 ends at 65504): times scale*log2(e) still below -2^12
   static SF_DEVICE f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);

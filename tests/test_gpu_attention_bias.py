@@ -52,6 +52,46 @@ def test_bias_kernels_read_strided_factors():
     assert torch.equal(a, b)
 
 
+MASKS = {
+    "first half of every row": lambda gh: (None, slice(0, 32)),
+    "second half of every row": lambda gh: (None, slice(32, 64)),
+    "all columns but one": lambda gh: (None, slice(0, 63)),
+    "first rows": lambda gh: (slice(0, 3), None),
+    "all rows but the last": lambda gh: (slice(0, gh - 1), None),
+    "first rows and first half": lambda gh: (slice(0, 2), slice(0, 32)),
+}
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("mask", MASKS)
+@pytest.mark.parametrize("hd,dtype,values", [
+    (64, torch.bfloat16, (-math.inf, torch.finfo(torch.bfloat16).min, -1e30, -1e9, -1e4)),
+    (80, torch.bfloat16, (-math.inf, torch.finfo(torch.bfloat16).min, -1e30, -1e9, -1e4)),
+    (64, torch.float16, (-math.inf, torch.finfo(torch.float16).min, -1e3)),
+    (80, torch.float16, (-math.inf, torch.finfo(torch.float16).min, -1e3)),
+])
+def test_bias_kernels_with_masked_keys(form, mask, hd, dtype, values):
+    """Factors that take keys away - for every query, and for every second one - against the softmax in 64 bits."""
+    from samfast_amd import _lib, ops
+    B, nH, gh = 1, 2, 4
+    q, k, v, rel_h, rel_w = bias_inputs(B, nH, gh, 64, hd, seed=gh + hd, dtype=dtype)
+    rows, cols = MASKS[mask](gh)
+    for value in values:
+        for step in (1, 2):
+            print(f"case masked {form}, {mask}, hd={hd} {dtype} {value} every {step}", flush=True)
+            rh, rw = rel_h.squeeze(-1).clone(), rel_w.squeeze(-2).clone()
+            if rows is not None:
+                rh[:, :, ::step, rows] = value
+            if cols is not None:
+                rw[:, :, ::step, cols] = value
+            s = q.double() @ k.double().transpose(-1, -2) * hd ** -0.5 + (rh.double()[..., None] + rw.double()[..., None, :]).flatten(-2)
+            ref = s.softmax(-1) @ v.double()
+            with _lib.knobs(**FORMS[form]):
+                out = ops.attn_relpos_bias(q.cuda(), k.cuda(), v.cuda(), rh.cuda(), rw.cuda())
+            # probabilities and result in the half type: half an ulp each, and one for the sums between
+            assert (out.cpu().double() - ref).abs().max() <= 4 * torch.finfo(dtype).eps * v.abs().max().item()
+
+
 @pytest.mark.parametrize("gh,gw", [(14, 14), (2, 2), (13, 14), (14, 5), (6, 8), (1, 16), (15, 13)])
 @pytest.mark.parametrize("hd,dtype", [(64, torch.bfloat16), (80, torch.float16)])
 def test_window_factors_read_in_pairs_or_one_by_one(gh, gw, hd, dtype):
