@@ -22,6 +22,8 @@
 
 namespace samfast {
 
+constexpr float kCeiling = 256.0f;  // of a half row's sum of probabilities: each stays far inside both types
+
 template <int HD, int WAVES>
 struct BiasCfg : GridRow<HD> {
   using R = GridRow<HD>;
@@ -206,31 +208,34 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
     __builtin_amdgcn_sched_barrier(0);
 
     // online softmax, one query per lane.  The exponent offset m_i is a reference, not the running
-    // maximum: probabilities may sit anywhere below 2 (the final division by the denominator,
-    // accumulated with the same offsets, makes the result independent of it), so no maximum is taken in
-    // the common case.  Whether one has reached 2 shows in the top exponent bit of the packed pairs,
-    // or-ed together.  Then - always where the first keys are met, m_i being T::kLowest, and again when the maximum
-    // has grown by T::kMargin powers of two - the maximum is found, the accumulators are rescaled and the
-    // probabilities formed once more.  m_i is finite throughout: keys that a factor of -inf, or of the type's lowest
-    // value, has taken away have probabilities of zero whatever stands before or behind them.
+    // maximum (the final division by the denominator, accumulated with the same offsets, makes the
+    // result independent of it): probabilities may sit anywhere below a ceiling, so no maximum of the scores is
+    // taken in the common case.  Whether one has grown too large shows where the denominator is summed here in the
+    // half row's sum, else (ONES_ROW) in the top exponent bit of the packed pairs, or-ed together: 2.  Then -
+    // always where the first keys are met, m_i being T::kLowest - the maximum is found, the accumulators are
+    // rescaled and the probabilities formed once more.  m_i is finite throughout: keys that a factor of -inf, or of
+    // the type's lowest value, has taken away have probabilities of zero whatever stands before or behind them.
     unsigned int seen = 0u;
+    float l0 = 0.f, l1 = 0.f;  // this half row's share of the denominator, unrounded (two chains)
     auto pair = [&](int w, float neg_mrow) __attribute__((always_inline)) {  // packed pair w of 8
-      pk[w >> 2][w & 3] = T::pack2(fast_exp2(fmaf(s[2 * w], a.c, neg_mrow)), fast_exp2(fmaf(s[2 * w + 1], a.c, neg_mrow)));
+      const float p0 = fast_exp2(fmaf(s[2 * w], a.c, neg_mrow)), p1 = fast_exp2(fmaf(s[2 * w + 1], a.c, neg_mrow));
+      pk[w >> 2][w & 3] = T::pack2(p0, p1);
+      if (!C::ONES_ROW) l0 += p0 + p1;
     };
     auto score = [&](int ks) __attribute__((always_inline)) { s_next = T::mfma(kf[ks], qf[ks], ks == 0 ? b_next : s_next); };
     auto pv = [&](int j, int dt) __attribute__((always_inline)) { oacc[dt] = T::mfma(vf[j][dt], pk_prev[j], oacc[dt]); };
     const float neg_mrow = b0 - m_i;
-    float l1 = 0.f;
     float e0, e1;  // a pair is packed one step after its exponentials were issued
 #pragma unroll
     for (int g = 0; g < 8; ++g) {
       const float x0 = fmaf(s[2 * g], a.c, neg_mrow), x1 = fmaf(s[2 * g + 1], a.c, neg_mrow);
-      if (g > 0) pk[(g - 1) >> 2][(g - 1) & 3] = T::pack2(e0, e1);
+      if (g > 0) {
+        pk[(g - 1) >> 2][(g - 1) & 3] = T::pack2(e0, e1);
+        if (!C::ONES_ROW) l0 += e0, l1 += e1;
+      }
       e0 = fast_exp2(x0);
       e1 = fast_exp2(x1);
-      if (g > 0 && !(g & 1)) seen |= pk[(g - 1) >> 2][(g - 2) & 3] | pk[(g - 1) >> 2][(g - 1) & 3];
-      // the denominator sums what the product multiplies: the rounded probabilities
-      if (!C::ONES_ROW) (g & 1 ? l1 : l_i) = T::add2(pk_prev[g >> 2][g & 3], g & 1 ? l1 : l_i);
+      if (C::ONES_ROW && g > 0 && !(g & 1)) seen |= pk[(g - 1) >> 2][(g - 2) & 3] | pk[(g - 1) >> 2][(g - 1) & 3];
       __builtin_amdgcn_sched_barrier(0);
       if (g == 0) pv(0, 0);
       if (g == 1) {
@@ -247,9 +252,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
       __builtin_amdgcn_sched_barrier(0);
     }
     pk[1][3] = T::pack2(e0, e1);
-    seen |= pk[1][2] | pk[1][3];
-    if (!C::ONES_ROW) l_i += l1;
-    if (__any((seen & 0x40004000u) != 0u)) {  // uniform; an infinity and a NaN included
+    if (C::ONES_ROW) seen |= pk[1][2] | pk[1][3];
+    else l0 = (l0 + e0) + (l1 + e1);
+    if (__any(C::ONES_ROW ? (seen & 0x40004000u) != 0u : l0 > kCeiling)) {  // uniform; an infinity included
       float mx = s[0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
@@ -258,6 +263,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
       const float alpha = fast_exp2(m_i - m_new);  // first keys: 0; none yet: 1, on accumulators of zero
       m_i = m_new;
       l_i *= alpha;
+      l0 = 0.f;
 #pragma unroll
       for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
@@ -265,6 +271,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
 #pragma unroll
       for (int w = 0; w < 8; ++w) pair(w, b0 - m_i);
     }
+    if (!C::ONES_ROW) l_i += l0;
   };
 
   const int nkt = a.N / 64;
@@ -304,10 +311,6 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int dt = 0; dt < C::DT; ++dt) oacc[dt] = T::mfma(vf[j][dt], pkB[j], oacc[dt]);
-  if (!C::ONES_ROW) {
-#pragma unroll
-    for (int g = 0; g < 8; ++g) l_i = T::add2(pkB[g >> 2][g & 3], l_i);
-  }
 
   // ---- epilogue: O = acc / l, 4 adjacent channels per store ----
   float l;
@@ -520,23 +523,27 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
     __builtin_amdgcn_sched_barrier(0);
 
     unsigned int seen = 0u;
+    float l0 = 0.f, l1 = 0.f;  // this row's share of the denominator, unrounded (two chains)
     auto pair = [&](int w, float neg_mrow) __attribute__((always_inline)) {  // packed pair w of 8
-      pk[w >> 2][w & 3] = T::pack2(fast_exp2(fmaf(s[2 * w], a.c, neg_mrow)), fast_exp2(fmaf(s[2 * w + 1], a.c, neg_mrow)));
+      const float p0 = fast_exp2(fmaf(s[2 * w], a.c, neg_mrow)), p1 = fast_exp2(fmaf(s[2 * w + 1], a.c, neg_mrow));
+      pk[w >> 2][w & 3] = T::pack2(p0, p1);
+      if (!C::ONES_ROW) l0 += p0 + p1;
     };
     auto score = [&](int ks) __attribute__((always_inline)) { s_next = T::mfma(kf[ks], qf[ks], ks == 0 ? b1 : s_next); };
     auto pv = [&](int j, int dt) __attribute__((always_inline)) { oacc[dt] = T::mfma(vf[j][dt], pk_prev[j], oacc[dt]); };
     const float neg_mrow = b0 - m_i;
-    float l1 = 0.f;
     // (the last row's kf is whatever the buffer holds: its product is not used)
     float e0, e1;  // a pair is packed one step after its exponentials were issued
 #pragma unroll
     for (int g = 0; g < 8; ++g) {
       const float x0 = fmaf(s[2 * g], a.c, neg_mrow), x1 = fmaf(s[2 * g + 1], a.c, neg_mrow);
-      if (g > 0) pk[(g - 1) >> 2][(g - 1) & 3] = T::pack2(e0, e1);
+      if (g > 0) {
+        pk[(g - 1) >> 2][(g - 1) & 3] = T::pack2(e0, e1);
+        if (!C::ONES_ROW) l0 += e0, l1 += e1;
+      }
       e0 = fast_exp2(x0);
       e1 = fast_exp2(x1);
-      if (g > 0 && !(g & 1)) seen |= pk[(g - 1) >> 2][(g - 2) & 3] | pk[(g - 1) >> 2][(g - 1) & 3];
-      if (!C::ONES_ROW) (g & 1 ? l1 : l_i) = T::add2(pk_prev[g >> 2][g & 3], g & 1 ? l1 : l_i);
+      if (C::ONES_ROW && g > 0 && !(g & 1)) seen |= pk[(g - 1) >> 2][(g - 2) & 3] | pk[(g - 1) >> 2][(g - 1) & 3];
       __builtin_amdgcn_sched_barrier(0);
       if (g == 0) pv(0, 0);
       if (g == 1) {
@@ -557,9 +564,9 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
 #pragma unroll
       for (int dt = 0; dt < C::DT; ++dt) read_v(j, dt, BUF);
     pk[1][3] = T::pack2(e0, e1);
-    seen |= pk[1][2] | pk[1][3];
-    if (!C::ONES_ROW) l_i += l1;
-    if (__any((seen & 0x40004000u) != 0u)) {  // a probability has reached 2: move the reference (attn_relpos.hip)
+    if (C::ONES_ROW) seen |= pk[1][2] | pk[1][3];
+    else l0 = (l0 + e0) + (l1 + e1);
+    if (__any(C::ONES_ROW ? (seen & 0x40004000u) != 0u : l0 > kCeiling)) {  // move the reference, as above
       float mx = s[0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
@@ -568,6 +575,7 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
       const float alpha = fast_exp2(m_i - m_new);
       m_i = m_new;
       l_i *= alpha;
+      l0 = 0.f;
 #pragma unroll
       for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
@@ -575,6 +583,7 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
 #pragma unroll
       for (int w = 0; w < 8; ++w) pair(w, b0 - m_i);
     }
+    if (!C::ONES_ROW) l_i += l0;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of K row kt + 2 and V row kt + 1 has landed
     __syncthreads();
     if (kt + 2 < nkt) v_dma(kt + 2, BUF);  // row kt's V is in registers
@@ -592,10 +601,6 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int dt = 0; dt < C::DT; ++dt) oacc[dt] = T::mfma(vf[j][dt], pkB[j], oacc[dt]);  // P V of the last row
-  if (!C::ONES_ROW) {
-#pragma unroll
-    for (int g = 0; g < 8; ++g) l_i = T::add2(pkB[g >> 2][g & 3], l_i);
-  }
 
   // ---- the two key halves meet: reference, denominator and accumulators of half 1 through LDS ----
   float* other = reinterpret_cast<float*>(lds) + qt * 64 * (16 * C::DT + 2) + lane;  // word w of lane: 64 w + lane

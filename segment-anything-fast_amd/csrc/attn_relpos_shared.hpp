@@ -52,10 +52,6 @@ struct ElemBf16 {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
   }
   static SF_DEVICE unsigned int pack2(float lo, float hi) { return pack_bf16x2(lo, hi); }
-  // c + the two values of a packed pair, one instruction
-  static SF_DEVICE float add2(unsigned int w, float c) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w), __builtin_bit_cast(bf16x2, kOne << 16 | kOne), c, false);
-  }
   static SF_DEVICE float lo(unsigned int w) { return bf16_lo_to_f32(w); }
   static SF_DEVICE float hi(unsigned int w) { return bf16_hi_to_f32(w); }
   static SF_DEVICE float from_bits(unsigned short h) { return bf16_bits_to_f32(h); }
@@ -73,9 +69,6 @@ struct ElemF16 {
   static SF_DEVICE unsigned int pack2(float lo, float hi) {  // round to nearest even
     const f32x2 v = {lo, hi};
     return __builtin_bit_cast(unsigned int, __builtin_convertvector(v, f16x2));
-  }
-  static SF_DEVICE float add2(unsigned int w, float c) {
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, w), __builtin_bit_cast(f16x2, kOne << 16 | kOne), c, false);
   }
   static SF_DEVICE float from_bits(unsigned short h) { return (float)__builtin_bit_cast(_Float16, h); }
   static SF_DEVICE float lo(unsigned int w) { return from_bits((unsigned short)(w & 0xffffu)); }

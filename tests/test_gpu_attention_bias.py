@@ -39,6 +39,26 @@ def test_bias_kernels_vs_oracle(form, B, nH, gh, hd, ramp, dtype):
     assert diff.max().item() <= 2e-2 and diff.mean().item() <= 1e-3
 
 
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_denominator_sums_unrounded_probabilities(form, dtype):
+    """One key of probability one (a power of two) against 4095 of one smaller probability, whose rounding - the same for all
+    of them - stays out of the denominator at head_dim 64."""
+    from samfast_amd import _lib, ops
+    print(f"case denominator {form} {dtype}", flush=True)
+    N, hd = 4096, 64
+    q, k, v = torch.zeros((1, 1, N, hd)), torch.zeros((1, 1, N, hd)), torch.zeros((1, 1, N, hd))
+    q[..., 0] = torch.linspace(2.0, 7.0, N)
+    k[0, 0, 0, 0], v[0, 0, 0] = 8.0, 1.0
+    q, k, v = (t.to(dtype) for t in (q, k, v))
+    zeros = torch.zeros((1, 1, N, 64), dtype=dtype)
+    ref = (q.double() @ k.double().transpose(-1, -2) * hd ** -0.5).softmax(-1) @ v.double()
+    with _lib.knobs(**FORMS[form]):
+        out = ops.attn_relpos_bias(q.cuda(), k.cuda(), v.cuda(), zeros.cuda(), zeros.cuda())
+    # the result's own rounding, half an eps, and a sixteenth for exponentials and sums in fp32
+    assert ((out.cpu().double() - ref).abs() / ref).max() <= (0.5 + 0.0625) * torch.finfo(dtype).eps
+
+
 def test_bias_kernels_read_strided_factors():
     """The factors as slices of one (B, nH, N, 128) tensor, q / k / v of a token-major buffer: same bits as contiguous."""
     from samfast_amd import ops
