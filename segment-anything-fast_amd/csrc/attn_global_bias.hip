@@ -211,7 +211,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
     // maximum (the final division by the denominator, accumulated with the same offsets, makes the
     // result independent of it): probabilities may sit anywhere below a ceiling, so no maximum of the scores is
     // taken in the common case.  Whether one has grown too large shows where the denominator is summed here in the
-    // half row's sum, else (ONES_ROW) in the top exponent bit of the packed pairs, or-ed together: 2.  Then -
+    // half row's sum, else (ONES_ROW) in the packed pairs (T::note, T::outgrown).  Then -
     // always where the first keys are met, m_i being T::kLowest - the maximum is found, the accumulators are
     // rescaled and the probabilities formed once more.  m_i is finite throughout: keys that a factor of -inf, or of
     // the type's lowest value, has taken away have probabilities of zero whatever stands before or behind them.
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
       }
       e0 = fast_exp2(x0);
       e1 = fast_exp2(x1);
-      if (C::ONES_ROW && g > 0 && !(g & 1)) seen |= pk[(g - 1) >> 2][(g - 2) & 3] | pk[(g - 1) >> 2][(g - 1) & 3];
+      if (C::ONES_ROW && g > 0 && !(g & 1)) seen = T::note(seen, pk[(g - 1) >> 2][(g - 2) & 3], pk[(g - 1) >> 2][(g - 1) & 3]);
       __builtin_amdgcn_sched_barrier(0);
       if (g == 0) pv(0, 0);
       if (g == 1) {
@@ -252,9 +252,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
       __builtin_amdgcn_sched_barrier(0);
     }
     pk[1][3] = T::pack2(e0, e1);
-    if (C::ONES_ROW) seen |= pk[1][2] | pk[1][3];
+    if (C::ONES_ROW) seen = T::note(seen, pk[1][2], pk[1][3]);
     else l0 = (l0 + e0) + (l1 + e1);
-    if (__any(C::ONES_ROW ? (seen & 0x40004000u) != 0u : l0 > kCeiling)) {  // uniform; an infinity included
+    if (__any(C::ONES_ROW ? T::outgrown(seen) : l0 > kCeiling)) {  // uniform; an infinity included
       float mx = s[0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
@@ -543,7 +543,7 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
       }
       e0 = fast_exp2(x0);
       e1 = fast_exp2(x1);
-      if (C::ONES_ROW && g > 0 && !(g & 1)) seen |= pk[(g - 1) >> 2][(g - 2) & 3] | pk[(g - 1) >> 2][(g - 1) & 3];
+      if (C::ONES_ROW && g > 0 && !(g & 1)) seen = T::note(seen, pk[(g - 1) >> 2][(g - 2) & 3], pk[(g - 1) >> 2][(g - 1) & 3]);
       __builtin_amdgcn_sched_barrier(0);
       if (g == 0) pv(0, 0);
       if (g == 1) {
@@ -564,9 +564,9 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
 #pragma unroll
       for (int dt = 0; dt < C::DT; ++dt) read_v(j, dt, BUF);
     pk[1][3] = T::pack2(e0, e1);
-    if (C::ONES_ROW) seen |= pk[1][2] | pk[1][3];
+    if (C::ONES_ROW) seen = T::note(seen, pk[1][2], pk[1][3]);
     else l0 = (l0 + e0) + (l1 + e1);
-    if (__any(C::ONES_ROW ? (seen & 0x40004000u) != 0u : l0 > kCeiling)) {  // move the reference, as above
+    if (__any(C::ONES_ROW ? T::outgrown(seen) : l0 > kCeiling)) {  // move the reference, as above
       float mx = s[0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);

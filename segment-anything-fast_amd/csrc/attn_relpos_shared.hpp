@@ -40,9 +40,12 @@ constexpr float kLazyLog2 = 8.0f;  // softmax reference lags the running maximum
 // as four 32-bit words (u32x4) everywhere outside these functions.
 struct ElemBf16 {
   static constexpr unsigned int kOne = 0x3F80u;   // 1.0
-  // global kernel: how far (log2) above the running maximum the exponent reference is put; bf16
-  // probabilities keep their eight bits at any size
+  // global kernel with the caller's factors: how far (log2) above the maximum the exponent reference is put when it is
+  // moved; bf16 probabilities keep their eight bits at any size.  note() gathers packed pairs, outgrown() says whether
+  // one of them has reached 2: the top exponent bit, so that or-ing them is enough.
   static constexpr float kMargin = 16.0f;
+  static SF_DEVICE unsigned int note(unsigned int seen, unsigned int w0, unsigned int w1) { return seen | w0 | w1; }
+  static SF_DEVICE bool outgrown(unsigned int seen) { return (seen & 0x40004000u) != 0u; }
   // global kernel with the caller's factors: the exponent reference (log2) before any key has been met.  Keys below it
   // are as good as masked.  Down to it every probability is finite: at 2^31 a reference and a difference from it
   // are each rounded by at most 64, so that a probability stays below 2^(128 - kMargin).
@@ -60,8 +63,19 @@ struct ElemF16 {
   typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
   typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
   static constexpr unsigned int kOne = 0x3C00u;   // 1.0
-  static constexpr float kMargin = 4.0f;  // fp16 ends at 2^-24: 2^-20 of the maximum, against 2^-11 of a rounding
-  static constexpr float kLowest = -134217728.0f;  // as above, with 2^27, roundings of 4 and 65504 as the end
+  // as above, but a probability below 2^-14 is short of bits: the reference never stands above the maximum, and it
+  // moves when a probability exceeds 2^kLazyLog2 (one v_pk_maximum3_f16 for two pairs; with bf16's
+  // or, and therefore a ceiling of 2, 8 x 16 x 4096 x 80 took 820 us for 769, so often did the reference move)
+  static constexpr float kMargin = 0.0f;
+  static SF_DEVICE unsigned int note(unsigned int seen, unsigned int w0, unsigned int w1) {
+    const f16x2 a = __builtin_bit_cast(f16x2, seen), b = __builtin_bit_cast(f16x2, w0), c = __builtin_bit_cast(f16x2, w1);
+    return __builtin_bit_cast(unsigned int, __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c));
+  }
+  static SF_DEVICE bool outgrown(unsigned int seen) {
+    const f16x2 m = __builtin_bit_cast(f16x2, seen);
+    return m[0] > (_Float16)256.0f || m[1] > (_Float16)256.0f;
+  }
+  static constexpr float kLowest = -134217728.0f;  // as above, with 2^27, roundings of 4 and the end of the type at 2^16
   static constexpr unsigned int kMask = 0xFB53u;  // -60000 (fp16 ends at 65504): times scale*log2(e) still below -2^12
   static SF_DEVICE f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);

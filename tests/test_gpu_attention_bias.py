@@ -59,6 +59,26 @@ def test_denominator_sums_unrounded_probabilities(form, dtype):
     assert ((out.cpu().double() - ref).abs() / ref).max() <= (0.5 + 0.0625) * torch.finfo(dtype).eps
 
 
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("hd", [64, 80])
+@pytest.mark.parametrize("where", [0, 31, 40, 2000, 4095])
+def test_fp16_probabilities_far_below_the_maximum(form, hd, where):
+    """One key 2^12 to 2^14 above 4095 equal ones, which carry half of the sum: their probabilities keep the type's bits."""
+    from samfast_amd import _lib, ops
+    print(f"case tail {form} hd={hd} key {where}", flush=True)
+    N = 4096
+    q, k, v = torch.zeros((1, 1, N, hd)), torch.zeros((1, 1, N, hd)), torch.ones((1, 1, N, hd))
+    q[..., 0] = torch.linspace(12.0, 13.9, N) * math.log(2) * math.sqrt(hd)
+    k[0, 0, where, 0], v[0, 0, where] = 1.0, 0.0
+    q, k, v = (t.to(torch.float16) for t in (q, k, v))
+    zeros = torch.zeros((1, 1, N, 64), dtype=torch.float16)
+    ref = (q.double() @ k.double().transpose(-1, -2) * hd ** -0.5).softmax(-1) @ v.double()
+    with _lib.knobs(**FORMS[form]):
+        out = ops.attn_relpos_bias(q.cuda(), k.cuda(), v.cuda(), zeros.cuda(), zeros.cuda())
+    # a normal fp16 probability and the result, rounded once each (2^-11); 2^-13 for exponentials and sums in fp32
+    assert ((out.cpu().double() - ref).abs() / ref).max() <= 2.0 ** -10 + 2.0 ** -13
+
+
 def test_bias_kernels_read_strided_factors():
     """The factors as slices of one (B, nH, N, 128) tensor, q / k / v of a token-major buffer: same bits as contiguous."""
     from samfast_amd import ops
