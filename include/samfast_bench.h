@@ -19,8 +19,10 @@ extern "C" {
  * SAMFAST_GEMM_PERSIST, SAMFAST_GEMM_PERSIST_SKEW, SAMFAST_GEMM_PERSIST_PRIO,
  * SAMFAST_GEMM_SPLITK, SAMFAST_GEMM_ONCE, SAMFAST_GEMM_LINEAR_SMALL, SAMFAST_GEMM_SKINNY,
  * SAMFAST_ATTN_WAVES, SAMFAST_ATTN_SPLIT, SAMFAST_ATTN_WINDOW_ROWS, SAMFAST_SPARSE_PERSIST.  This
- * call sets one (`unset` != 0: back to "not given", `value` ignored).  Every variant of a kernel
- * returns the same bits; the knobs only move time.  Returns SAMFAST_E_INVALID for an unknown name.
+ * call sets one (`unset` != 0: back to "not given", `value` ignored).  The knobs move time; every
+ * variant of a kernel returns the same bits, with two exceptions that sum in another order:
+ * SAMFAST_ATTN_SPLIT and SAMFAST_ATTN_WINDOW_ROWS.  (Neither default looks at the number of slices:
+ * a slice's result does not depend on its batch.)  Returns SAMFAST_E_INVALID for an unknown name.
  */
 int samfast_bench_set_knob(const char* name, int value, int unset);
 

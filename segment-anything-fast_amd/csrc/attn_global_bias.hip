@@ -17,7 +17,8 @@
 // of every row are split between two wavefronts, whose results (maximum reference, denominator, output) meet in
 // LDS once, at the end; workgroups of two query tiles x two key halves (64 queries, under 54 KB of LDS), three per CU
 // at hd 64, so that one image's 12 heads are 768 workgroups: three on each of the 256 CUs, where 128-query
-// workgroups leave half of the CUs with one and half with two.  bias_form picks.
+// workgroups leave half of the CUs with one and half with two.  bias_form picks, by head_dim: the two kernels round
+// differently, and a slice's bits are not to depend on the batch.
 #include "attn_relpos_shared.hpp"
 
 namespace samfast {
@@ -649,28 +650,24 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
     }
 }
 
-// Which form of the global kernel: 8 or 4 wavefronts of attn_global_kernel, or 2 for the key-split one.  What
-// decides is how the workgroups divide among the 256 CUs: the forms hold 256 queries (one workgroup per CU),
-// 128 (two) and 64 (hd 64: three, hd 80: two).  The prices are microseconds of one full round over 64 key rows
-// and of a last, partial one with one / two workgroups per CU, measured over 1 to 8 images of 8 to 16 heads; 1 x 12 heads
-// x 4096, hd 64: 72 us key-split, 75 with 8 wavefronts, 78 with 4; 2 x 9: 107, 149, 123; 1 x 16, hd 80: 116, 96, 102.
+// Which form of the global kernel.  Split keys round differently from unsplit ones, so that choice looks at head_dim
+// alone: a slice has the same bits whatever batch it travels in.  hd 64 is split (us, split / unsplit with 8 / with 4
+// wavefronts, 4096 tokens: 1 x 8 heads 48 / 73 / 53, 1 x 12: 66 / 71 / 76, 2 x 9: 102 / 142 / 116, 1 x 16: 87 / 79 / 82,
+// 8 x 16: 655 / 628 / 634), hd 80, where only two such workgroups fit a CU, is not (55 / 74 / 59, 84 / 78 / 83, 130 / 159 / 136,
+// 105 / 91 / 95, 851 / 714 / 730).  8 wavefronts or 4, which agree bit for bit: by how the workgroups of 256
+// queries (one per CU) and of 128 (two) divide among the 256 CUs.  The prices are microseconds of one full round over
+// 64 key rows and, of 128 queries, of a last one with one workgroup per CU.
+// Returns 8, 4, or 2 for the key-split form.
 static int bias_form(const AttnArgs& a, int hd) {
   const int force = knob(KNOB_ATTN_WAVES);
   const bool by8 = a.N % 256 == 0;
   if (force == 4 || force == 8) return force == 8 && by8 ? 8 : 4;
   const int split = knob_or(KNOB_ATTN_SPLIT, 1);
-  if (split == 2) return 2;
-  auto price = [](int64_t wgs, int per_cu, int full, int one, int two) {
-    const int64_t slots = 256 * per_cu, rest = wgs % slots;
-    const int last = rest == 0 ? 0 : rest <= 256 ? one : rest <= 512 ? two : full;
-    return wgs / slots * full + last;
-  };
-  const int64_t slices = (int64_t)a.B * a.nH;
-  const int64_t p2 = hd == 64 ? price(slices * (a.N / 64), 3, 66, 30, 50) : price(slices * (a.N / 64), 2, 58, 42, 58);
-  const int64_t p4 = hd == 64 ? price(slices * (a.N / 128), 2, 79, 50, 79) : price(slices * (a.N / 128), 2, 97, 59, 97);
-  const int64_t p8 = price(slices * (a.N / 256), 1, hd == 64 ? 76 : 90, hd == 64 ? 76 : 90, 0);
-  if (split != 0 && p2 <= p4 && p2 <= p8 && !(p2 == p4 && hd == 80)) return 2;
-  return by8 && p8 <= p4 ? 8 : 4;
+  if (split == 2 || (split != 0 && hd == 64)) return 2;
+  const int64_t slices = (int64_t)a.B * a.nH, wgs4 = slices * (a.N / 128), wgs8 = slices * (a.N / 256), rest4 = wgs4 % 512;
+  const int full4 = hd == 64 ? 80 : 95, one4 = hd == 64 ? 53 : 59, full8 = hd == 64 ? 79 : 91;
+  const int64_t p4 = wgs4 / 512 * full4 + (rest4 == 0 ? 0 : rest4 <= 256 ? one4 : full4);
+  return by8 && (wgs8 + 255) / 256 * full8 <= p4 ? 8 : 4;
 }
 template <typename T, int HD>
 static void launch_bias(const AttnArgs& a, int form, hipStream_t stream) {

@@ -36,7 +36,7 @@ enum Knob {
   KNOB_LINEAR_SMALL,      // SAMFAST_GEMM_LINEAR_SMALL: 0 = whole Linears over few rows as two launches as well
   KNOB_GEMM_SKINNY,       // SAMFAST_GEMM_SKINNY: 0 = products over few rows through the tiled kernels
   KNOB_ATTN_WAVES,        // SAMFAST_ATTN_WAVES: 4 / 8 wavefronts per global-attention workgroup
-  KNOB_ATTN_SPLIT,        // SAMFAST_ATTN_SPLIT: global attention with the keys split between two wavefronts, 0 = never, 1 = where it pays, 2 = always
+  KNOB_ATTN_SPLIT,        // SAMFAST_ATTN_SPLIT: global attention with the keys split between two wavefronts (other bits), 0 = never, 1 = head_dim 64, 2 = always
   KNOB_ATTN_WINDOW_ROWS,  // SAMFAST_ATTN_WINDOW_ROWS: 1 = window keys as grid rows padded to 16 (attn_window_rows_kernel) where built
   KNOB_SPARSE_PERSIST,    // SAMFAST_SPARSE_PERSIST: 2:4 GEMM, 0 = one workgroup per tile (default), 1 = resident workgroups from two tiles each on, 2 wherever built
   KNOB_COUNT

@@ -79,6 +79,21 @@ def test_fp16_probabilities_far_below_the_maximum(form, hd, where):
     assert ((out.cpu().double() - ref).abs() / ref).max() <= 2.0 ** -10 + 2.0 ** -13
 
 
+@pytest.mark.parametrize("hd,dtype", [(64, torch.bfloat16), (80, torch.float16)])
+@pytest.mark.parametrize("gh", [64, 16, 6])
+def test_a_slice_has_the_same_bits_in_any_batch(hd, dtype, gh):
+    from samfast_amd import ops
+    print(f"case batch hd={hd} {dtype} gh={gh}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(hd + gh)
+    N = gh * 64
+    q, k, v = ((torch.randn((4, 16, N, hd), generator=g, device="cuda") * 0.5).to(dtype) for _ in range(3))
+    rh = (torch.randn((4, 16, N, gh), generator=g, device="cuda") * 0.5).to(dtype)
+    rw = (torch.randn((4, 16, N, 64), generator=g, device="cuda") * 0.5).to(dtype)
+    whole = ops.attn_relpos_bias(q, k, v, rh, rw)
+    for b, h in ((1, 8), (1, 12), (2, 9), (3, 12)):
+        assert torch.equal(ops.attn_relpos_bias(*(t[:b, :h] for t in (q, k, v, rh, rw))), whole[:b, :h]), (b, h)
+
+
 def test_bias_kernels_read_strided_factors():
     """The factors as slices of one (B, nH, N, 128) tensor, q / k / v of a token-major buffer: same bits as contiguous."""
     from samfast_amd import ops
