@@ -262,25 +262,31 @@ class Block(nn.Module):
         tokens = mlp.lin2.linear_fused(gq, sg, _lib.EPILOGUE_RESIDUAL, residual=tokens, out=tokens, layout=L)
         return tokens.view(B, H, W, C), None
 
+    def _as_built(self) -> bool:
+        """Whether calling this block is what its constructor wrote and nothing else: no subclass, hook or
+        forward of an instance's own on it or on the modules inside, and no hook on every module."""
+        attn, mlp = self.attn, self.mlp
+        built = ((self, Block), (self.norm1, nn.LayerNorm), (attn, Attention), (self.norm2, nn.LayerNorm),
+                 (mlp, MLPBlock), (mlp.act, nn.GELU),
+                 *((m, nn.Linear) for m in (attn.qkv, attn.proj, mlp.lin1, mlp.lin2)))
+        return (all(type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__
+                    for m, cls in built)
+                and not nn.modules.module._global_forward_hooks and not nn.modules.module._global_forward_pre_hooks)
+
     def _half_fused_ok(self, x: torch.Tensor) -> bool:
         """Whether this block, its Linears left in the half type, can run through _forward_half_fused:
-        inference on a GPU in bf16 / fp16 at a shape the attention kernels cover, the modules the
-        ones the constructor built (nobody has put a hook or another class in their place)."""
+        inference on a GPU in bf16 / fp16 at a shape the attention kernels cover, with nobody's hook or
+        class in the way."""
         attn, mlp = self.attn, self.mlp
         if not (FUSED_BLOCK and flash_4.USE_CUSTOM_KERNEL and x.is_cuda and x.dim() == 4
                 and x.dtype in (torch.bfloat16, torch.float16) and attn.use_rel_pos and not torch.is_grad_enabled()):
             return False
-        if not (type(self.norm1) is nn.LayerNorm and type(self.norm2) is nn.LayerNorm and type(attn) is Attention
-                and type(mlp) is MLPBlock and type(mlp.act) is nn.GELU and mlp.act.approximate == "none"
-                and all(type(m) is nn.Linear for m in (attn.qkv, attn.proj, mlp.lin1, mlp.lin2))):
+        if not self._as_built() or mlp.act.approximate != "none":
             return False
         B, H, W, C = x.shape
         for n in (self.norm1, self.norm2):
             if n.weight is None or n.bias is None or n.weight.dtype != x.dtype or n.normalized_shape != (C,):
                 return False
-        if any(m._forward_hooks or m._forward_pre_hooks for m in (self.norm1, attn, attn.qkv, attn.proj, self.norm2,
-                                                                  mlp, mlp.lin1, mlp.act, mlp.lin2)):
-            return False
         ws = self.window_size
         gh, gw = (ws, ws) if ws > 0 else (H, W)
         return (attn.qkv.weight.dtype == x.dtype and C % 8 == 0 and C <= 4096 and mlp.lin1.out_features % 8 == 0

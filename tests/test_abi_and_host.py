@@ -350,3 +350,33 @@ def test_int8_linear_keeps_one_bias():
     q = q.to(torch.bfloat16)
     assert q.bias.dtype == torch.float32
     assert Int8DynamicLinear.from_float(nn.Linear(64, 16, bias=False)).bias is None
+
+
+def test_a_block_counts_as_built_only_without_hooks_and_overrides():
+    """Only such a block may leave its modules uncalled (the fused half-type route)."""
+    from samfast_amd.modeling import Block
+    blk = Block(64, 2, use_rel_pos=True, window_size=3, input_size=(8, 8))
+    assert blk._as_built()
+    nothing = lambda *args: None
+    inside = (blk, blk.norm1, blk.attn, blk.attn.qkv, blk.attn.proj, blk.norm2, blk.mlp, blk.mlp.lin1, blk.mlp.act, blk.mlp.lin2)
+    for m in inside:
+        for register in (m.register_forward_hook, m.register_forward_pre_hook):
+            handle = register(nothing)
+            assert not blk._as_built()
+            handle.remove()
+        m.forward = nothing
+        assert not blk._as_built()
+        del m.forward
+    for register in (nn.modules.module.register_module_forward_hook, nn.modules.module.register_module_forward_pre_hook):
+        handle = register(nothing)
+        assert not blk._as_built()
+        handle.remove()
+    assert blk._as_built()
+    blk.mlp.act = nn.ReLU()
+    assert not blk._as_built()
+
+    class Other(Block):
+        def forward(self, x):
+            return x
+
+    assert not Other(64, 2, use_rel_pos=True, window_size=3, input_size=(8, 8))._as_built()

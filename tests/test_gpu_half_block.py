@@ -50,6 +50,37 @@ def test_half_blocks_equal_module_composition(B, C, heads, window, bias, dtype, 
     assert ((y.float() - ref.float()).norm() / ref.float().norm()).item() < 8 * torch.finfo(dtype).eps
 
 
+def test_hooks_and_subclasses_of_a_block_are_honoured():
+    """Inside an encoder, where consecutive blocks are chained, a block with a hook is called as a module."""
+    from samfast_amd.modeling import ImageEncoderViT, image_encoder as ie
+    torch.manual_seed(3)
+    enc = ImageEncoderViT(img_size=1024, embed_dim=128, depth=3, num_heads=2, use_rel_pos=True, window_size=14, global_attn_indexes=(1,))
+    enc = enc.cuda().to(torch.bfloat16).eval()
+    x = torch.randn((1, 64, 64, 128), device="cuda").to(torch.bfloat16)
+    seen = []
+    with torch.no_grad():
+        plain = enc.forward_blocks(x)
+        handles = [b.register_forward_hook(lambda m, a, out, i=i: seen.append((i, out))) for i, b in enumerate(enc.blocks)]
+        watched = enc.forward_blocks(x)
+        assert [i for i, _ in seen] == [0, 1, 2] and torch.equal(seen[2][1], watched)
+        assert ((watched.float() - plain.float()).norm() / plain.float().norm()).item() < 8 * torch.finfo(torch.bfloat16).eps
+        for h in handles:
+            h.remove()
+        handle = enc.blocks[2].register_forward_hook(lambda m, a, out: torch.zeros_like(out))
+        assert not enc.forward_blocks(x).any()
+        handle.remove()
+
+        class Skipped(ie.Block):
+            def forward(self, x):
+                return x
+
+        before = enc.blocks[:2]
+        enc.blocks[2].__class__ = Skipped
+        whole = enc.forward_blocks(x)
+        enc.blocks = before
+        assert torch.equal(whole, enc.forward_blocks(x))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,C,H,W", [(1, 256, 64, 64), (3, 256, 5, 7), (2, 8, 3, 3), (1, 264, 2, 3), (1, 512, 1, 5), (1, 520, 2, 2), (0, 256, 4, 4)])
 def test_layernorm2d_over_channels_last(B, C, H, W, dtype):
