@@ -139,7 +139,7 @@ extern "C" int samfast_layernorm(const void* x, const void* r, const void* gamma
   SF_REQUIRE((M + 3) / 4 < (1ll << 31), "layernorm: M too large");
   SF_REQUIRE((r == nullptr) == (sum == nullptr), "layernorm: the added rows and the sum go together");
   SF_REQUIRE(M == 0 || (x && gamma && beta && out), "layernorm: null pointer");
-  SF_REQUIRE(eps > 0.f, "layernorm: eps must be positive");
+  SF_REQUIRE(eps >= 0.f, "layernorm: eps must not be negative");
   SF_REQUIRE(aligned16(x) && aligned16(r) && aligned16(gamma) && aligned16(beta) && aligned16(sum) && aligned16(out),
              "layernorm: operands must be 16-byte aligned");
   if (M == 0) return SAMFAST_OK;

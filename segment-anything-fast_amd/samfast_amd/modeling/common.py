@@ -38,9 +38,9 @@ class LayerNorm2d(nn.Module):
                 or torch._C._functorch.is_functorch_wrapped_tensor(x) or torch.autograd.forward_ad._current_level >= 0):
             return False
         return (x.is_cuda and x.dim() == 4 and x.dtype in (torch.bfloat16, torch.float16) and not torch.is_grad_enabled()
-                and self.weight.dtype == x.dtype and self.bias.dtype == x.dtype and self.weight.device == x.device
+                and self.weight.dtype == x.dtype and self.bias.dtype == x.dtype and self.eps >= 0
                 and x.shape[1] == self.weight.numel() and x.shape[1] % 8 == 0 and x.shape[1] <= 4096
-                and x.data_ptr() % 16 == 0 and x.permute(0, 2, 3, 1).is_contiguous())
+                and ops.rows_launchable(x.permute(0, 2, 3, 1), self.weight, self.bias))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self._rows_ok(x):

@@ -285,8 +285,14 @@ class Block(nn.Module):
             return False
         B, H, W, C = x.shape
         for n in (self.norm1, self.norm2):
-            if n.weight is None or n.bias is None or n.weight.dtype != x.dtype or n.normalized_shape != (C,):
+            if n.weight is None or n.bias is None or n.weight.dtype != x.dtype or n.normalized_shape != (C,) or not n.eps >= 0:
                 return False
+        # what the row kernels read as it is (the qkv bias: the window kernel's padding rows)
+        rows = [self.norm1.weight, self.norm1.bias, self.norm2.weight, self.norm2.bias]
+        if attn.qkv.bias is not None:
+            rows.append(attn.qkv.bias)
+        if not ops.rows_launchable(*rows) or x.device != rows[0].device or x.data_ptr() % 16 != 0:
+            return False
         ws = self.window_size
         gh, gw = (ws, ws) if ws > 0 else (H, W)
         return (attn.qkv.weight.dtype == x.dtype and C % 8 == 0 and C <= 4096 and mlp.lin1.out_features % 8 == 0

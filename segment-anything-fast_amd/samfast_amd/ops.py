@@ -549,6 +549,13 @@ def gemm_i8_sparse24_fused(xq: torch.Tensor, sx: torch.Tensor, wc: torch.Tensor,
     return out
 
 
+def rows_launchable(*tensors: torch.Tensor) -> bool:
+    """Whether the row kernels can take these tensors as they are: on the current device, whose stream
+    the launches go to, contiguous from a 16-byte boundary on."""
+    device = torch.cuda.current_device()
+    return all(t.device.index == device and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
+
+
 def layernorm(x: torch.Tensor, gamma: torch.Tensor, beta: torch.Tensor, eps: float,
               add: Optional[torch.Tensor] = None):
     """LayerNorm over the last axis of contiguous half-type rows.  With `add`: (x + add, its LayerNorm)

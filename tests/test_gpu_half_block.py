@@ -50,6 +50,47 @@ def test_half_blocks_equal_module_composition(B, C, heads, window, bias, dtype, 
     assert ((y.float() - ref.float()).norm() / ref.float().norm()).item() < 8 * torch.finfo(dtype).eps
 
 
+def _shifted(t):
+    """The same values, one element past a 16-byte boundary."""
+    return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("what", ["eps", "norm parameters", "qkv bias", "input", "another current device"])
+def test_half_block_and_layernorm2d_where_a_launch_does_not_serve(what, monkeypatch):
+    """eps = 0 runs like any other; tensors off a 16-byte boundary, and a device that is not the current one, go
+    through the composition."""
+    from samfast_amd.modeling import image_encoder as ie
+    from samfast_amd.modeling.common import LayerNorm2d
+    print(f"case no launch: {what}", flush=True)
+    torch.manual_seed(5)
+    blk = ie.Block(128, 2, use_rel_pos=True, window_size=14, input_size=(64, 64)).cuda().to(torch.bfloat16).eval()
+    norm = LayerNorm2d(128).cuda().to(torch.bfloat16)
+    x = torch.randn((1, 20, 20, 128), device="cuda").to(torch.bfloat16)
+    composed = what != "eps"
+    with torch.no_grad():
+        if what == "eps":
+            blk.norm1.eps = blk.norm2.eps = norm.eps = 0.0
+        elif what == "norm parameters":
+            for m in (blk.norm2, norm):
+                m.weight.data = _shifted(m.weight.data)
+        elif what == "qkv bias":
+            blk.attn.qkv.bias.data = _shifted(blk.attn.qkv.bias.data)
+        elif what == "input":
+            x = _shifted(x)
+            assert x.data_ptr() % 16 != 0 and x.is_contiguous()
+        maps = x.permute(0, 3, 1, 2)
+        with monkeypatch.context() as m:
+            if what == "another current device":
+                m.setattr(torch.cuda, "current_device", lambda: 1)
+            assert blk._half_fused_ok(x) is not composed
+            assert norm._rows_ok(maps) is not (composed and what != "qkv bias")
+        y, z = blk(x), norm(maps)
+        monkeypatch.setattr(ie, "FUSED_BLOCK", False)
+        assert ((y.float() - blk(x).float()).norm() / y.float().norm()).item() < 8 * torch.finfo(torch.bfloat16).eps
+        ref = F.layer_norm(x.double(), (128,), norm.weight.double(), norm.bias.double(), norm.eps).permute(0, 3, 1, 2)
+        assert ((z.double() - ref).abs() <= 8 * torch.finfo(torch.bfloat16).eps * (ref.abs() + 1)).all()
+
+
 def test_hooks_and_subclasses_of_a_block_are_honoured():
     """Inside an encoder, where consecutive blocks are chained, a block with a hook is called as a module."""
     from samfast_amd.modeling import ImageEncoderViT, image_encoder as ie
