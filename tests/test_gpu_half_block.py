@@ -50,6 +50,26 @@ def test_half_blocks_equal_module_composition(B, C, heads, window, bias, dtype, 
     assert ((y.float() - ref.float()).norm() / ref.float().norm()).item() < 8 * torch.finfo(dtype).eps
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gelu_of_every_value(dtype):
+    """No value further from x * Phi(x) than with the module it stands for, nor more of them; infinities and NaN alike."""
+    from samfast_amd import ops
+    print(f"case gelu {dtype}", flush=True)
+    x = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(dtype)
+    exact = x.double() * 0.5 * torch.special.erfc(-x.double() * 0.5 ** 0.5)
+    got, module = ops.gelu_(x.cuda().clone()).cpu(), F.gelu(x.cuda()).cpu()
+    finite = torch.isfinite(x.float())
+    assert torch.equal(got[~finite].float().nan_to_num(nan=-1.0), module[~finite].float().nan_to_num(nan=-1.0))
+    assert torch.isfinite(got[finite].float()).all()
+    missed = lambda y: (y[finite] != exact[finite].to(dtype)).sum().item()
+    print(f"not correctly rounded: {missed(got)}, module {missed(module)}", flush=True)
+    assert missed(got) <= missed(module)
+    # half a unit of the type with fp32 steps in front of it, or half of fp16's smallest step; beyond |x| = 5, where Phi(-|x|)
+    # is below 3e-7, the fit runs on with an error of at most 3e-12
+    bound = 0.51 * torch.finfo(dtype).eps * exact[finite].abs() + (2.0 ** -25 if dtype == torch.float16 else 3e-12)
+    assert ((got[finite].double() - exact[finite]).abs() <= bound).all()
+
+
 def _shifted(t):
     """The same values, one element past a 16-byte boundary."""
     return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
