@@ -4,8 +4,8 @@
 // (a Linear over 7 tokens: 7 us of kernels); here it is 2-3 us plus the launches.
 //
 // Every function returns None for a call it does not cover - a CPU tensor, another type, a strided
-// view, a shape the C ABI refuses - and the caller then takes the Python route in ops.py, whose
-// checks and error texts stay the one definition of what is accepted.
+// view, a shape the C ABI refuses, a call that somebody watches (plain_call) - and the caller then takes
+// the Python route, whose checks and error texts stay the one definition of what is accepted.
 //
 // The C ABI is reached through pointers that bind() receives from the ctypes handle, so that one
 // copy of libsamfast.so serves both (also when SAMFAST_LIB names another file).
@@ -13,7 +13,9 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -35,12 +37,31 @@ const Bound kBound[] = {
     {"samfast_attn_relpos_bias_fwd", reinterpret_cast<void**>(&p_attn_bias)},
 };
 
-// a plain strided GPU tensor on the current device (the launches go to its current stream)
-bool on_current_gpu(const at::Tensor& t, c10::DeviceIndex dev) {
-  return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.device().index() == dev && !t.key_set().has(c10::DispatchKey::Python);
+// Whether nobody but the kernels has to see this thread's calls: a launch on raw pointers passes by tracers,
+// functional transforms (vmap, grad, functionalization) and dispatch and function modes.  All but the last stand as
+// dispatch keys that the thread has included beyond the default ones.
+bool plain_call() {
+  return (c10::impl::tls_local_dispatch_key_set().included_ | c10::default_included_set) == c10::default_included_set &&
+         !at::impl::torch_function_mode_enabled();
 }
 
-const at::Tensor* tensor_arg(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+// A tensor that is its memory and nothing more: no wrapper of a transform, subclass, conjugate or negative view, sparse or
+// nested layout, no forward-mode tangent.
+bool plain_tensor(const at::Tensor& t) {
+  constexpr c10::DispatchKeySet expected = c10::DispatchKeySet(
+      {c10::DispatchKey::Dense, c10::DispatchKey::ADInplaceOrView, c10::DispatchKey::AutogradFunctionality,
+       c10::DispatchKey::AutocastCUDA, c10::DispatchKey::AutocastCPU});
+  const c10::DispatchKeySet keys(c10::DispatchKeySet::RAW, t.key_set().raw_repr() & ~static_cast<uint64_t>(c10::full_backend_mask));
+  return (keys | expected) == expected && !t._fw_grad(/*level=*/0).defined();
+}
+
+// a plain strided GPU tensor on the current device (the launches go to its current stream)
+bool on_current_gpu(const at::Tensor& t, c10::DeviceIndex dev) {
+  return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.device().index() == dev && plain_tensor(t);
+}
+
+// (exactly a Tensor or Parameter: a subclass may override what happens to it)
+const at::Tensor* tensor_arg(PyObject* o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
 
 void* stream_of(c10::DeviceIndex dev) { return c10::hip::getCurrentHIPStream(dev).stream(); }
 
@@ -75,7 +96,7 @@ struct LinearCall {
 // wq is (N, K), or (K/64, N, 64) for layout 1.
 PyObject* host_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 5) Py_RETURN_NONE;
+  if (n != 5 || !plain_call()) Py_RETURN_NONE;
   const at::Tensor* wq = tensor_arg(args[1]);
   const int layout = static_cast<int>(PyLong_AsLong(args[2]));
   const bool kb = layout == SAMFAST_LAYOUT_KB64;
@@ -100,7 +121,7 @@ PyObject* host_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // sparse_linear(x, wc, widx, sw_bits, bias_bits or None): the same with the packed 2:4 weight
 PyObject* host_sparse_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 5) Py_RETURN_NONE;
+  if (n != 5 || !plain_call()) Py_RETURN_NONE;
   const at::Tensor *wc = tensor_arg(args[1]), *widx = tensor_arg(args[2]);
   LinearCall c = {tensor_arg(args[0]), tensor_arg(args[3]), tensor_arg(args[4])};
   if (!c.x || !wc || !widx || !c.sw || (args[4] != Py_None && !c.bias)) Py_RETURN_NONE;
@@ -128,7 +149,7 @@ PyObject* host_sparse_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // caller's bias factors, read through their strides; returns a contiguous (B, nH, N, hd) tensor
 PyObject* host_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 6) Py_RETURN_NONE;
+  if (n != 6 || !plain_call()) Py_RETURN_NONE;
   const at::Tensor* t[5];
   const c10::DeviceIndex dev = c10::hip::current_device();
   for (int i = 0; i < 5; ++i) {
@@ -155,6 +176,12 @@ PyObject* host_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (rc != SAMFAST_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
+}
+
+// plain(tensor): whether a launch that only the kernels see may stand for operations on this tensor
+PyObject* host_plain(PyObject*, PyObject* arg) {
+  const at::Tensor* t = tensor_arg(arg);
+  return PyBool_FromLong(t && plain_call() && plain_tensor(*t));
 }
 
 // bind({name: address}): the C ABI functions used above
@@ -185,6 +212,7 @@ PyCFunction fastcall(PyObject* (*f)(PyObject*, PyObject* const*, Py_ssize_t)) {
 PyMethodDef kMethods[] = {
     {"bind", host_bind, METH_O, nullptr},
     {"bound_names", host_bound_names, METH_NOARGS, nullptr},
+    {"plain", host_plain, METH_O, nullptr},
     {"linear", fastcall(host_linear), METH_FASTCALL, nullptr},
     {"sparse_linear", fastcall(host_sparse_linear), METH_FASTCALL, nullptr},
     {"attention", fastcall(host_attention), METH_FASTCALL, nullptr},

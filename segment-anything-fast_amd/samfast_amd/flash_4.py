@@ -86,9 +86,10 @@ def _attention_rel_h_rel_w(q_, k_, v_, rel_h_, rel_w_):
     """q_, k_, v_: (B, nH, N, hd); rel_h_: (B, nH, N, k_h, 1); rel_w_: (B, nH, N, 1, k_w).
     Returns (B, nH, N, hd) = softmax(q k^T / sqrt(hd) + rel_h + rel_w) v."""
     hd = q_.size(-1)
-    if USE_CUSTOM_KERNEL and q_.is_cuda and ops._launch_log is None:
+    if USE_CUSTOM_KERNEL and q_.is_cuda and ops._launch_log is None and not torch.compiler.is_compiling():
         # one native call on the factors as they are: the operator below wants them packed side by
-        # side (flash_4.py:352), a copy that costs an eighth of the attention itself
+        # side (flash_4.py:352), a copy that costs an eighth of the attention itself.  Where a tracer,
+        # a transform or a mode is to see the operator, the call declines.
         out = _lib.host().attention(q_, k_, v_, rel_h_, rel_w_, 1.0 / math.sqrt(hd))
         if out is not None:
             return out

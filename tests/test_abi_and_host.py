@@ -380,3 +380,50 @@ def test_a_block_counts_as_built_only_without_hooks_and_overrides():
             return x
 
     assert not Other(64, 2, use_rel_pos=True, window_size=3, input_size=(8, 8))._as_built()
+
+
+def test_native_calls_decline_where_somebody_watches():
+    """The host module launches on raw pointers; under a tracer, a functional transform, a dispatch or function mode,
+    and for tensors that are more than their memory, the call has to go through torch's dispatcher."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from samfast_amd import _lib
+    plain = _lib.host().plain
+    x = torch.randn(2, 3)
+    assert plain(x) and plain(nn.Parameter(x)) and plain(x.t()) and plain(x[:0])
+    with torch.no_grad():
+        assert plain(x)
+    with torch.inference_mode():
+        assert plain(x) and plain(torch.zeros(2))
+    assert plain(torch.ones(2, requires_grad=True) * 2)
+    answers = []
+
+    def watched(t):
+        answers.append((plain(t), plain(x)))
+        return t * 2
+
+    torch.jit.trace(watched, x, check_trace=False)
+    torch.vmap(watched)(x)
+    torch.func.grad(lambda t: watched(t).sum())(x)
+    torch.func.functionalize(watched)(x)
+
+    class Through(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Pass(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    for mode in (Through, Pass):
+        with mode():
+            watched(x)
+    assert len(answers) == 6 and not any(any(a) for a in answers), answers
+    with torch.autograd.forward_ad.dual_level():
+        assert not plain(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)))
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert not plain(x.as_subclass(Sub)) and not plain(torch._neg_view(x)) and not plain(x.to_sparse())
+    assert plain(x)

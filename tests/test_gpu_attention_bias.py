@@ -107,6 +107,31 @@ def test_bias_kernels_read_strided_factors():
     assert torch.equal(a, b)
 
 
+def test_the_operator_is_there_for_those_who_watch():
+    """A trace records it, vmap loops over it, a dispatch mode sees it - and nobody gets another result."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from samfast_amd.flash_4 import _attention_rel_h_rel_w as attention
+    args = [t.cuda() for t in bias_inputs(1, 2, 64, 64, 64, seed=1)]
+    other = [t.cuda() for t in bias_inputs(1, 2, 64, 64, 64, seed=2)]
+    want, want_other = attention(*args), attention(*other)
+    traced = torch.jit.trace(attention, args, check_trace=False)
+    assert "customflash::custom_flash_aligned" in str(traced.graph)
+    assert torch.equal(traced(*other), want_other)
+    both = torch.vmap(attention)(*(torch.stack(pair) for pair in zip(args, other)))
+    assert torch.equal(both[0], want) and torch.equal(both[1], want_other)
+
+    class Names(TorchDispatchMode):
+        names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Names():
+        got = attention(*args)
+    assert torch.equal(got, want) and any("custom_flash_aligned" in n for n in Names.names)
+
+
 MASKS = {
     "first half of every row": lambda gh: (None, slice(0, 32)),
     "second half of every row": lambda gh: (None, slice(32, 64)),
