@@ -33,14 +33,10 @@ class LayerNorm2d(nn.Module):
         self.eps = eps
 
     def _rows_ok(self, x: torch.Tensor) -> bool:
-        # a launch is invisible to tracers, functional transforms and forward-mode tangents
-        if (torch.compiler.is_compiling() or torch.jit.is_tracing() or type(x) not in (torch.Tensor, nn.Parameter)
-                or torch._C._functorch.is_functorch_wrapped_tensor(x) or torch.autograd.forward_ad._current_level >= 0):
-            return False
         return (x.is_cuda and x.dim() == 4 and x.dtype in (torch.bfloat16, torch.float16) and not torch.is_grad_enabled()
                 and self.weight.dtype == x.dtype and self.bias.dtype == x.dtype and self.eps >= 0
                 and x.shape[1] == self.weight.numel() and x.shape[1] % 8 == 0 and x.shape[1] <= 4096
-                and ops.rows_launchable(x.permute(0, 2, 3, 1), self.weight, self.bias))
+                and ops.unwatched(x) and ops.rows_launchable(x.permute(0, 2, 3, 1), self.weight, self.bias))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self._rows_ok(x):

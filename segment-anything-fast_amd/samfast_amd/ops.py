@@ -549,6 +549,14 @@ def gemm_i8_sparse24_fused(xq: torch.Tensor, sx: torch.Tensor, wc: torch.Tensor,
     return out
 
 
+def unwatched(x: torch.Tensor) -> bool:
+    """Whether launches that only the kernels see may stand for a module's tensor operations on x: no
+    compiler, tracer, transform, mode or forward-mode tangent has to see them, and autocast, which would
+    give some of them another type, is off."""
+    return (not torch.compiler.is_compiling() and torch.autograd.forward_ad._current_level < 0
+            and not torch.is_autocast_enabled("cuda") and _lib.host().plain(x))
+
+
 def rows_launchable(*tensors: torch.Tensor) -> bool:
     """Whether the row kernels can take these tensors as they are: on the current device, whose stream
     the launches go to, contiguous from a 16-byte boundary on."""

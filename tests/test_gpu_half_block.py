@@ -182,3 +182,39 @@ def test_layernorm2d_stays_composed_under_transforms():
         with torch.autograd.forward_ad.dual_level():
             dual = torch.autograd.forward_ad.make_dual(x[0], torch.ones_like(x[0]))
             assert torch.autograd.forward_ad.unpack_dual(norm(dual)).tangent is not None
+
+
+def test_half_block_and_layernorm2d_are_composed_where_somebody_watches(monkeypatch):
+    """Autocast gives the types it gives the composition, and a dispatch mode sees its operations."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from samfast_amd.modeling import image_encoder as ie
+    from samfast_amd.modeling.common import LayerNorm2d
+    torch.manual_seed(6)
+    blk = ie.Block(128, 2, use_rel_pos=True, window_size=14, input_size=(64, 64)).cuda().to(torch.bfloat16).eval()
+    norm = LayerNorm2d(128).cuda().to(torch.bfloat16)
+    x = torch.randn((1, 20, 20, 128), device="cuda").to(torch.bfloat16)
+    maps = x.permute(0, 3, 1, 2)
+
+    class Names(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            names.append(func.overloadpacket.__name__)
+            return func(*args, **(kwargs or {}))
+
+    def calls():
+        with torch.autocast("cuda", dtype=torch.float16):
+            cast = blk(x), norm(maps)
+        names.clear()
+        with Names():
+            seen = blk(x), norm(maps)
+        return cast + seen, list(names)
+
+    names = []
+    with torch.no_grad():
+        assert blk._half_fused_ok(x) and norm._rows_ok(maps)
+        got, got_names = calls()
+        monkeypatch.setattr(ie, "FUSED_BLOCK", False)
+        monkeypatch.setattr(LayerNorm2d, "_rows_ok", lambda self, x: False)
+        want, want_names = calls()
+    assert got_names == want_names and "gelu" in got_names
+    for g, w in zip(got, want):
+        assert g.dtype == w.dtype and torch.equal(g, w)
