@@ -179,8 +179,8 @@ int samfast_gemm_i8_scale_bias(
 
 /*
  * The whole quantised nn.Linear.forward: samfast_quant_rowwise_i8 followed by
- * samfast_gemm_i8_scale_bias, same codes, accumulators and result.  `layout` is the layout of wq
- * (and of the activation codes between the two steps).  `workspace`: at least
+ * samfast_gemm_i8_scale_bias, same codes, accumulators and result.  `layout` is the layout of wq;
+ * nothing of the weights is kept from one call for the next.  `workspace`: at least
  * samfast_linear_i8_workspace(M, N, K, layout) bytes of device memory, 16-byte aligned, contents
  * irrelevant before and after; may be NULL where that is 0.  The size function returns
  * SAMFAST_E_INVALID for a negative or zero dimension or an unknown layout; with

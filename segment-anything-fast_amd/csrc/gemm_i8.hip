@@ -374,7 +374,7 @@ __global__ __launch_bounds__(256, (TM == 4 ? 1 : 2)) void gemm_i8_kernel(GemmArg
     const int row = c >> 2, kc = c & 3;
     if (i < TM) {
       const int gm = min(m0 + row, a.M - 1);
-      ox[i] = gm * a.row_pitch + kc * 16;
+      ox[i] = gm * a.x_pitch + kc * 16;
       lx[i] = row * GLD + ((kc ^ lds_swizzle(row)) * 16);
     }
     // W: consecutive chunk groups go to consecutive LDS slots (no write bank conflicts);
@@ -382,7 +382,7 @@ __global__ __launch_bounds__(256, (TM == 4 ? 1 : 2)) void gemm_i8_kernel(GemmArg
     const int slot = row & 127;
     const int wrow = (row & 128) + (slot & 31) * 4 + (slot >> 5);
     const int gn = min(n0 + wrow, a.N - 1);
-    ow[i] = gn * a.row_pitch + kc * 16;
+    ow[i] = gn * a.w_pitch + kc * 16;
     lw[i] = GBM * GLD + row * GLD + ((kc ^ lds_swizzle(row)) * 16);
   }
 
@@ -494,11 +494,11 @@ __global__ __launch_bounds__(256, (TM == 4 ? 1 : 2)) void gemm_i8_kernel(GemmArg
       const int rho = 16 * (wave_u + 4 * i) + (lane >> 2);  // LDS row of this lane's chunk
       const int chunk = (lane & 3) ^ lds_swizzle(rho);
       if (i < GBM / 64) {  // X rows
-        dma_off[i] = (unsigned int)(min(m0 + rho, a.M - 1) * a.row_pitch + chunk * 16);
+        dma_off[i] = (unsigned int)(min(m0 + rho, a.M - 1) * a.x_pitch + chunk * 16);
       } else {             // W slots (slot s of a 128-column half holds W row (s%32)*4 + s/32)
         const int sl = rho - GBM;
         const int wrow = (sl & 128) + (sl & 31) * 4 + ((sl & 127) >> 5);
-        dma_off[i] = (unsigned int)(min(n0 + wrow, a.N - 1) * a.row_pitch + chunk * 16);
+        dma_off[i] = (unsigned int)(min(n0 + wrow, a.N - 1) * a.w_pitch + chunk * 16);
       }
     }
     typedef __attribute__((address_space(1))) const void* gptr_t;
@@ -697,12 +697,12 @@ __global__ __launch_bounds__((Gemm3Cfg<BM, BN, KSPLIT, STAGES>::THREADS), (Gemm3
     const int rho = 16 * (wave_u + 4 * i) + (lane >> 2);
     const int chunk = (lane & 3) ^ lds_swizzle(rho);
     if (i < BM / 64) {
-      dma_off[i] = (unsigned int)(min(m0 + rho, a.M - 1) * a.row_pitch + chunk * 16);
+      dma_off[i] = (unsigned int)(min(m0 + rho, a.M - 1) * a.x_pitch + chunk * 16);
     } else {
       const int sl = rho - BM;                      // slot inside the W part of the stage
       const int half = sl / (BN / 2), sh = sl % (BN / 2);
       const int wrow = half * (BN / 2) + (sh & 31) * TNW + (sh >> 5);
-      dma_off[i] = (unsigned int)(min(n0 + wrow, a.N - 1) * a.row_pitch + chunk * 16);
+      dma_off[i] = (unsigned int)(min(n0 + wrow, a.N - 1) * a.w_pitch + chunk * 16);
     }
   }
   auto dma_issue = [&](int kt, int stage_off) {
@@ -947,10 +947,11 @@ static int gemm_common(int epi, const int8_t* xq, const float* sx, const int8_t*
                        const float* sw, const float* bias, void* out, int64_t ldo, int64_t M,
                        int N, int K, hipStream_t stream, const void* residual = nullptr,
                        int64_t ld_res = 0, const int32_t* dst_row = nullptr,
-                       int layout = SAMFAST_LAYOUT_ROWMAJOR, const GemmTail* tail = nullptr) {
+                       int layout = SAMFAST_LAYOUT_ROWMAJOR, const GemmTail* tail = nullptr, int w_layout = -1) {
+  if (w_layout < 0) w_layout = layout;  // `layout` is X's; W's follows unless it is given
   // no rows: nothing to do, and the row operands of an empty call may be null
   SF_REQUIRE(wq && (M == 0 || (xq && out)), "gemm_i8: null pointer");
-  SF_REQUIRE(layout == SAMFAST_LAYOUT_ROWMAJOR || layout == SAMFAST_LAYOUT_KB64, "gemm_i8: unknown layout %d", layout);
+  for (int l : {layout, w_layout}) SF_REQUIRE(l == SAMFAST_LAYOUT_ROWMAJOR || l == SAMFAST_LAYOUT_KB64, "gemm_i8: unknown layout %d", l);
   SF_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_i8: bad shape M=%lld N=%d K=%d", (long long)M, N, K);
   SF_REQUIRE(M < (1ll << 31) - 256, "gemm_i8: M=%lld too large", (long long)M);
   SF_REQUIRE(M * K < (1ll << 31) && (int64_t)N * K < (1ll << 31),
@@ -976,11 +977,9 @@ static int gemm_common(int epi, const int8_t* xq, const float* sx, const int8_t*
   GemmArgs a;
   a.x = xq; a.w = wq; a.out = out; a.sx = sx; a.sw = sw; a.bias = bias;
   a.ldo = ldo; a.M = (int)M; a.N = N; a.K = K;
-  if (layout == SAMFAST_LAYOUT_KB64) {
-    a.row_pitch = GBK; a.x_kstep = M * GBK; a.w_kstep = (int64_t)N * GBK;
-  } else {
-    a.row_pitch = K; a.x_kstep = GBK; a.w_kstep = GBK;
-  }
+  const bool x_kb = layout == SAMFAST_LAYOUT_KB64, w_kb = w_layout == SAMFAST_LAYOUT_KB64;
+  a.x_pitch = x_kb ? GBK : K; a.x_kstep = x_kb ? M * GBK : GBK;
+  a.w_pitch = w_kb ? GBK : K; a.w_kstep = w_kb ? (int64_t)N * GBK : GBK;
   a.residual = reinterpret_cast<const unsigned short*>(residual);
   a.ld_res = ld_res; a.dst_row = dst_row;
   const bool generic_k = K / GBK < 4;  // fewer k tiles than LDS stages
@@ -1193,33 +1192,67 @@ extern "C" int samfast_gemm_i8_fused_quant(const int8_t* xq, const float* sx, co
 }
 
 // ---- a whole quantised Linear ---------------------------------------------------------------
+namespace samfast {
+
+// (N, K) row-major -> (K/64, N, 64): 16 bytes per thread, written in whole lines.  4.9 MB: 3 us.
+__global__ __launch_bounds__(256) void kblock_major_kernel(const int8_t* w, int8_t* out, int N, int K) {
+  const int i = blockIdx.x * 256 + threadIdx.x;  // piece of `out`; N * K < 2^31
+  const int kb = i / (4 * N), row = (i >> 2) - kb * N, c = i & 3;
+  if (kb < K / 64) reinterpret_cast<u32x4*>(out)[i] = *reinterpret_cast<const u32x4*>(w + (int64_t)row * K + kb * 64 + c * 16);
+}
+
+// Whether a Linear with row-major weights puts them into K-block major order first, in the workspace of the call (a
+// copy that outlived it would have to follow every write to the weights, on every stream).  The codes are always K-block
+// major, and the products read row-major weights beside them; whole lines of both pay from many rows on.  us, read as
+// they are / reordered / K-block major already: 4096 x 1280 -> 3840: 32.8 / 37 / 32.6, 8192 x 1024 -> 4096: 53.9 / 54.7 / 52.1,
+// 16384 x 1280 -> 3840: 105 / 102 / 98, 16384 x 5120 -> 1280: 136 / 137 / 133, 65536 x 1280 -> 3840: 380 / 352 / 348,
+// 65536 x 5120 -> 1280: 657 / 575 / 571.  (Row-major codes as well: 35, 65, 120, 140, 408, 640.)
+static bool linear_reorders_weights(int64_t M) { return M >= 16384; }
+
+// bytes of the codes in a Linear's workspace; their row scales follow, then reordered weights
+static int64_t linear_codes_bytes(int64_t M, int K) { return (M * K + 15) & ~(int64_t)15; }
+static int64_t linear_scales_bytes(int64_t M) { return (M * 4 + 15) & ~(int64_t)15; }
+
+}  // namespace samfast
+
 extern "C" int64_t samfast_linear_i8_workspace(int64_t M, int N, int K, int layout) {
   using namespace samfast;
   SF_REQUIRE(M > 0 && N > 0 && K > 0 && layout >= SAMFAST_LAYOUT_ROWMAJOR && layout <= SAMFAST_LAYOUT_SPARSE24,
              "linear_i8_workspace: bad shape M=%lld N=%d K=%d or layout %d", (long long)M, N, K, layout);
   if (layout != SAMFAST_LAYOUT_SPARSE24 && linear_i8_small_covers(M, N, K)) return 0;
-  // codes, then the row scales
-  return ((M * K + 15) & ~(int64_t)15) + M * 4;
+  const int64_t weights = layout == SAMFAST_LAYOUT_ROWMAJOR && linear_reorders_weights(M) ? (int64_t)N * K : 0;
+  return linear_codes_bytes(M, K) + linear_scales_bytes(M) + weights;
 }
 
 extern "C" int samfast_linear_i8(const void* x, int64_t ldx, const int8_t* wq, const float* sw, const float* bias,
                                  void* y, int64_t ldy, void* workspace, int64_t M, int N, int K, int dtype,
                                  int layout, void* stream) {
   using namespace samfast;
+  SF_REQUIRE(layout == SAMFAST_LAYOUT_ROWMAJOR || layout == SAMFAST_LAYOUT_KB64, "linear_i8: unknown layout %d", layout);
   if (M > 0 && linear_i8_small_covers(M, N, K)) {
-    SF_REQUIRE(dtype == SAMFAST_BF16 && (layout == SAMFAST_LAYOUT_ROWMAJOR || layout == SAMFAST_LAYOUT_KB64),
-               "linear_i8: only bf16, weights row-major or K-block major");
+    SF_REQUIRE(dtype == SAMFAST_BF16, "linear_i8: only bf16");
     SF_REQUIRE(x && wq && sw && y && aligned16(x) && aligned16(wq) && aligned16(y), "linear_i8: null or unaligned pointer");
     SF_REQUIRE(ldx >= K && ldx % 8 == 0 && ldy >= N && ldy % 8 == 0, "linear_i8: row strides must be multiples of 8, >= K and >= N");
     return linear_i8_small_launch(reinterpret_cast<const unsigned short*>(x), ldx, wq, sw, bias, reinterpret_cast<unsigned short*>(y), ldy,
                                   (int)M, N, K, layout, reinterpret_cast<hipStream_t>(stream));
   }
   SF_REQUIRE(M == 0 || (workspace && aligned16(workspace)), "linear_i8: the workspace must be non-null and 16-byte aligned");
+  SF_REQUIRE(N > 0 && K > 0 && K % GBK == 0 && (int64_t)N * K < (1ll << 31) && wq && aligned16(wq),
+             "linear_i8: K=%d must be a multiple of %d, the weights (N=%d) 16-byte aligned and under 2 GiB", K, GBK, N);
   int8_t* xq = reinterpret_cast<int8_t*>(workspace);
-  float* sx = reinterpret_cast<float*>(xq + ((M * K + 15) & ~(int64_t)15));
-  const int rc = samfast_quant_rowwise_i8(x, ldx, xq, sx, M, K, dtype, layout, stream);
+  float* sx = reinterpret_cast<float*>(xq + linear_codes_bytes(M, K));
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const int rc = samfast_quant_rowwise_i8(x, ldx, xq, sx, M, K, dtype, SAMFAST_LAYOUT_KB64, stream);
   if (rc != SAMFAST_OK) return rc;
-  return samfast_gemm_i8_fused(xq, sx, wq, sw, bias, y, ldy, M, N, K, dtype, SAMFAST_EPILOGUE_NONE, nullptr, 0, nullptr, layout, stream);
+  if (layout == SAMFAST_LAYOUT_ROWMAJOR && linear_reorders_weights(M)) {
+    int8_t* wk = xq + linear_codes_bytes(M, K) + linear_scales_bytes(M);
+    hipLaunchKernelGGL(kblock_major_kernel, dim3((unsigned int)(((int64_t)N * K / 16 + 255) / 256)), dim3(256), 0, s, wq, wk, N, K);
+    const int rl = check_launch("kblock_major_kernel");
+    if (rl != SAMFAST_OK) return rl;
+    wq = wk;
+    layout = SAMFAST_LAYOUT_KB64;
+  }
+  return gemm_common(EPI_SCALE_BIAS_BF16, xq, sx, wq, sw, bias, y, ldy, M, N, K, s, nullptr, 0, nullptr, SAMFAST_LAYOUT_KB64, nullptr, layout);
 }
 
 extern "C" int samfast_linear_i8_sparse24(const void* x, int64_t ldx, const int8_t* wc, const int32_t* widx,
@@ -1228,7 +1261,7 @@ extern "C" int samfast_linear_i8_sparse24(const void* x, int64_t ldx, const int8
   using namespace samfast;
   SF_REQUIRE(M == 0 || (workspace && aligned16(workspace)), "linear_i8_sparse24: the workspace must be non-null and 16-byte aligned");
   int8_t* xq = reinterpret_cast<int8_t*>(workspace);
-  float* sx = reinterpret_cast<float*>(xq + ((M * K + 15) & ~(int64_t)15));
+  float* sx = reinterpret_cast<float*>(xq + linear_codes_bytes(M, K));
   const int rc = samfast_quant_rowwise_i8(x, ldx, xq, sx, M, K, dtype, SAMFAST_LAYOUT_KB64, stream);
   if (rc != SAMFAST_OK) return rc;
   return samfast_gemm_i8_sparse24_fused(xq, sx, wc, widx, sw, bias, y, ldy, M, N, K, dtype, SAMFAST_EPILOGUE_NONE, nullptr, 0, SAMFAST_LAYOUT_KB64, stream);

@@ -108,7 +108,7 @@ __global__ __launch_bounds__(512, 2) void gemm_i8_once_kernel(GemmArgs a) {
   for (int i = 0; i < NLD; ++i) {
     const int row = (i < 2 ? 32 * lw + 16 * i : C::WROWS * lw + 16 * (i - 2)) + (lane >> 2);
     const int chunk = (lane & 3) ^ once_swizzle(row);
-    off[i] = (unsigned int)((i < 2 ? min(m0 + row, a.M - 1) : min(n0 + row, a.N - 1)) * a.row_pitch + chunk * 16);
+    off[i] = (unsigned int)((i < 2 ? min(m0 + row, a.M - 1) * a.x_pitch : min(n0 + row, a.N - 1) * a.w_pitch) + chunk * 16);
   }
   auto fill = [&](int t, int stage) {
     const int kt = t * KG + grp;

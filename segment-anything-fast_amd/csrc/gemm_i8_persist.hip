@@ -104,11 +104,11 @@ __global__ __launch_bounds__(256, PERSIST_MIN_WG) void gemm_i8_persist_kernel(Ge
       const int rho = 16 * (wave_u + 4 * i) + (lane >> 2);
       const int chunk16 = ((lane & 3) ^ lds_swizzle(rho)) * 16;
       if (i < PBM / 64) {
-        dma_off[i] = (unsigned int)((m0 + rho) * a.row_pitch + chunk16);
+        dma_off[i] = (unsigned int)((m0 + rho) * a.x_pitch + chunk16);
       } else {
         const int sl = rho - PBM;
         const int wrow = (sl & 128) + (sl & 31) * 4 + ((sl & 127) >> 5);
-        dma_off[i] = (unsigned int)((n0 + wrow) * a.row_pitch + chunk16);
+        dma_off[i] = (unsigned int)((n0 + wrow) * a.w_pitch + chunk16);
       }
       asm volatile("" : "+v"(dma_off[i]));  // a 32-bit value from here on (not a widened 64-bit product)
     }

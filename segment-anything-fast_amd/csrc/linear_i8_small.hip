@@ -32,9 +32,8 @@ struct SmallArgs {
   unsigned short* y;
   int64_t ldy;
   int M, N, K;
-  int row_pitch;     // bytes between consecutive weight rows: K, or 64 (K-block major)
-  int64_t w_kstep;   // bytes between consecutive 64-byte k steps: 64, or N * 64
-  int64_t x_kstep;
+  int x_pitch, w_pitch;      // bytes between consecutive code / weight rows: K, or 64 (K-block major)
+  int64_t x_kstep, w_kstep;  // bytes between consecutive 64-byte k steps: 64, or rows * 64
   int tiles_m, tiles;  // product alone: row tiles, tiles
 };
 
@@ -95,7 +94,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 2) void linear_i8_small_kernel(Sm
   i32x4 wf[NCH][NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const int8_t* wrow = a.w + (int64_t)min(n0 + 16 * t + lr, a.N - 1) * a.row_pitch + 16 * lq;
+    const int8_t* wrow = a.w + (int64_t)min(n0 + 16 * t + lr, a.N - 1) * a.w_pitch + 16 * lq;
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const int step = wave + kSmallWaves * i;
@@ -199,9 +198,9 @@ __global__ __launch_bounds__(64 * kSmallWaves, 2) void gemm_i8_skinny_kernel(Sma
   const int8_t* xrow[MT];
   const int8_t* wrow[NT];
 #pragma unroll
-  for (int m = 0; m < MT; ++m) xrow[m] = a.xq + (int64_t)min(m0 + 16 * m + lr, a.M - 1) * a.row_pitch + 16 * lq;
+  for (int m = 0; m < MT; ++m) xrow[m] = a.xq + (int64_t)min(m0 + 16 * m + lr, a.M - 1) * a.x_pitch + 16 * lq;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) wrow[t] = a.w + (int64_t)min(n0 + 16 * t + lr, a.N - 1) * a.row_pitch + 16 * lq;
+  for (int t = 0; t < NT; ++t) wrow[t] = a.w + (int64_t)min(n0 + 16 * t + lr, a.N - 1) * a.w_pitch + 16 * lq;
   const int nk = a.K / 64;
   const int steps = (nk - wave + kSmallWaves - 1) / kSmallWaves;  // 0 for the last wavefronts of a short K
 
@@ -257,7 +256,7 @@ int linear_i8_small_launch(const unsigned short* x, int64_t ldx, const int8_t* w
   SmallArgs a = {};
   a.x = x; a.ldx = ldx; a.w = wq; a.sw = sw; a.bias = bias; a.y = y; a.ldy = ldy; a.M = M; a.N = N; a.K = K;
   const bool kb = layout == SAMFAST_LAYOUT_KB64;
-  a.row_pitch = kb ? 64 : K;
+  a.w_pitch = kb ? 64 : K;
   a.w_kstep = kb ? (int64_t)N * 64 : 64;
   // two column tiles per workgroup once single ones are more than the GPU has CUs: half the repeated
   // row work for the same number of rounds
@@ -312,7 +311,7 @@ int gemm_i8_skinny_launch(const GemmArgs& g, hipStream_t stream) {
   a.xq = g.x; a.sx = g.sx; a.w = g.w; a.sw = g.sw; a.bias = g.bias;
   a.y = reinterpret_cast<unsigned short*>(g.out);
   a.ldy = g.ldo; a.M = g.M; a.N = g.N; a.K = g.K;
-  a.row_pitch = g.row_pitch; a.x_kstep = g.x_kstep; a.w_kstep = g.w_kstep;
+  a.x_pitch = g.x_pitch; a.w_pitch = g.w_pitch; a.x_kstep = g.x_kstep; a.w_kstep = g.w_kstep;
   switch (skinny_shape(a.M, a.N, a.K)) {
     case 1 * 8 + 1: return launch_skinny<1, 1>(a, stream);
     case 1 * 8 + 2: return launch_skinny<1, 2>(a, stream);

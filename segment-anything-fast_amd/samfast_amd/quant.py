@@ -188,9 +188,8 @@ class Int8DynamicLinear(Int8LinearBase):
         return self._wq_kb64
 
     def _forward_native(self, x: torch.Tensor) -> Optional[torch.Tensor]:
-        buffers = self._buffers
-        layout = LAYOUT_KB64 if self.in_features % 64 == 0 else LAYOUT_ROWMAJOR
-        return _lib.host().linear(x, self._weight_for(layout), layout, buffers["sw_bits"], buffers.get("bias_bits"))
+        buffers = self._buffers  # the weights as they stand: no copy that could be behind them
+        return _lib.host().linear(x, buffers["wq"], LAYOUT_ROWMAJOR, buffers["sw_bits"], buffers.get("bias_bits"))
 
     def linear_fused_quant(self, xq, sx, epilogue, residual=None, out=None, layout=LAYOUT_ROWMAJOR,
                            ln=None, out_layout=LAYOUT_ROWMAJOR):

@@ -31,6 +31,67 @@ def test_dense_linear_over_few_rows_bit_exact(M, N, K):
     assert torch.equal(y.cpu().view(torch.int16), ref.view(torch.int16))
 
 
+def _linear(N, K, seed):
+    from samfast_amd import Int8DynamicLinear
+    g = torch.Generator().manual_seed(seed)
+    lin = torch.nn.Linear(K, N, dtype=torch.bfloat16)
+    with torch.no_grad():
+        lin.weight.copy_(torch.randn((N, K), generator=g) * 0.02)
+        lin.bias.copy_(torch.randn(N, generator=g))
+    return Int8DynamicLinear.from_float(lin.cuda())
+
+
+def _unfused(lin, x):
+    """The same Linear as two calls on row-major codes and weights."""
+    from samfast_amd import _lib, ops
+    xq, sx = ops.quant_rowwise(x)
+    return ops.gemm_i8_fused(xq, sx, lin.wq, lin.sw, lin.bias_f32, _lib.EPILOGUE_NONE)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (7, 2048, 256), (100, 3840, 1280), (33, 8, 64), (700, 520, 192),        # one launch, small tiles, fewer k tiles than stages
+    (4096, 768, 768), (4000, 1288, 5120), (5000, 2304, 768), (16383, 1280, 1280),  # one tile per CU, 128 x 128 tiles, resident
+    (16384, 1288, 320), (20001, 776, 1280),                                 # weights reordered on the way
+])
+def test_a_linear_reads_its_weights_as_they_stand(M, N, K):
+    """Row-major weights beside K-block major codes: the bits of row-major both, and of weights written a moment ago."""
+    print(f"case weights M={M} N={N} K={K}", flush=True)
+    lin, other = _linear(N, K, 1), _linear(N, K, 2)
+    x = torch.randn((M, K), device="cuda").to(torch.bfloat16)
+    assert torch.equal(lin(x), _unfused(lin, x))
+    lin.wq.data.copy_(other.wq)
+    lin.sw_bits.data.copy_(other.sw_bits)
+    lin.bias_bits.data.copy_(other.bias_bits)
+    assert torch.equal(lin(x), _unfused(other, x))
+
+
+@pytest.mark.parametrize("M", [7, 4096, 16384])
+def test_a_linears_first_call_anywhere(M):
+    """Built in inference mode; first called while a graph is recorded; then called from another stream."""
+    print(f"case first call M={M}", flush=True)
+    x = torch.randn((M, 256), device="cuda").to(torch.bfloat16)
+    with torch.inference_mode():
+        lin = _linear(264, 256, 3)
+        assert torch.equal(lin(x), _unfused(lin, x))
+    lin = _linear(264, 256, 4)
+    want = _unfused(lin, x)
+    graph = torch.cuda.CUDAGraph()
+    with torch.no_grad(), torch.cuda.graph(graph):
+        recorded = lin(x)
+    assert torch.equal(lin(x), want)  # before any replay
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        there = lin(x)
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(there, want)
+    for _ in range(3):
+        recorded.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(recorded, want)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 8, 256), (31, 40, 384), (33, 264, 256), (65, 1280, 5120), (500, 1288, 2048), (130, 4096, 1280)])
 def test_sparse_linear_over_few_rows_bit_exact(M, N, K):
     from samfast_amd import Int8Sparse24Linear
