@@ -111,9 +111,10 @@ SF_DEVICE float max_with_lane_xor32(float v) {
 
 // One wave instruction: 64 pieces of 16 bytes from base + off to LDS at `dst` (piece of lane l: dst + 16 l).
 // Written out because the compiler would make every LDS read that follows wait for the builtin's loads;
-// whoever calls it waits for the arrival by hand (vmcnt) before the barrier in front of the readers.
+// whoever calls it waits for the arrival by hand (vmcnt) before the barrier in front of the readers.  The destination is
+// an operand in m0, so that the compiler knows the register is taken and moves it there itself.
 SF_DEVICE void lds_dma16(const unsigned char* base, unsigned int off, unsigned int dst) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(dst) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "{m0}"(dst) : "memory");
 }
 
 // How the global kernels keep one key grid row (64 keys) of K and of V in LDS: rows of 16-byte pieces, placed so

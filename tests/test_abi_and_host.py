@@ -427,3 +427,10 @@ def test_native_calls_decline_where_somebody_watches():
 
     assert not plain(x.as_subclass(Sub)) and not plain(torch._neg_view(x)) and not plain(x.to_sparse())
     assert plain(x)
+
+
+def test_no_inline_assembly_writes_m0_itself():
+    """m0 cannot be listed as clobbered; a statement that needs a value in it takes it as an operand there."""
+    for src in sorted((ROOT / "segment-anything-fast_amd" / "csrc").glob("*.h*")):
+        for statement in re.findall(r"\basm\b[^;]*;", re.sub(r"//[^\n]*", "", src.read_text())):
+            assert not re.search(r'[a-z_0-9]+ m0\s*,', statement), (src.name, statement)
