@@ -148,13 +148,19 @@ static int dispatch_quant(const QuantArgs& a, hipStream_t s) {
     // Rows of more than 1024: wavefronts that share a row (us, one wavefront a row / two / four).
     //   Where one wavefront would need 128 registers and more, at any M: 65536 x 4096: 308 / 166 / 159, 16384 x 3072:
     //   38 / 32 / 30, 65536 x 2560: 115 / 102 / 105, 4096 x 2048: 9.2 / 8.0 / 9.0.
-    //   Else while the rows are too few to fill the GPU with one wavefront each: 512 x 5120: 6.5 / 5.4 / 4.1, 5003 x 5120:
-    //   19.1 / 21.8 / 17.1, 16384 x 5120: 46 / 55 / 48; 1000 x 1536: 3.9 / 3.6 / 3.2, 8192 x 1536: 12.1 / 11.3 / 12.9.
+    //   Else while the rows are too few to fill the GPU with one wavefront each: 512 x 5120: 6.5 / 5.4 / 4.1, 1000 x 1536: 3.9 / 3.6 /
+    //   3.2, 8192 x 1536: 12.1 / 11.3 / 12.9.
+    //   K > 4096 beyond that (one / four): where quarters fill their lanes (K % 1024 == 0) the sharing form is the faster one as
+    //   long as its stores spread: 4096 x 5120 row-major 15.4 / 12.8, 16384 x 5120 43.7 / 40.6, K-block major 5003 x 5120 18.5 / 16.9,
+    //   8001 x 5120 26.5 / 23.4, 6001 x 6144 26.0 / 25.3.  K-block major codes of M % 16 == 0 rows have their K blocks a multiple of
+    //   1 KB apart, and the four stores meet: 4096 x 5120 15.2 / 16.6, 8192 x 5120 27.4 / 27.9.  Quarters that do not fill: 4001 x 4608
+    //   14.1 / 16.2.  From 11 chunks per lane on one wavefront is short of registers: 8192 x 8192 46.3 / 43.5.  At 32768 rows one
+    //   wavefront is ahead in either layout (K-block major 85.6 / 104.7 at K = 5120).
     if (need == 3 && a.M <= 8192) return a.M <= 1024 ? launch_shares<4>(a, s) : launch_shares<2>(a, s);
     if (need == 4 || need == 5) return a.M <= 1024 ? launch_shares<4>(a, s) : launch_shares<2>(a, s);
     if (need >= 6 && need <= 8) return launch_shares<4>(a, s);
-    // (below 11 chunks, quarters that do not fill their lanes lose from 2048 rows on)
-    if (need > 8 && a.M <= (need > 10 || a.K % 1024 == 0 ? 6144 : 2048)) return launch_shares<4>(a, s);
+    const bool spread = !a.kb64 || a.M % 16 != 0;
+    if (need > 8 && (a.M <= 2048 || (a.M <= 16384 && (need > 12 || (a.K % 1024 == 0 && spread))))) return launch_shares<4>(a, s);
   } else {
     if (need == 4) return launch_quant<4, 8, LN>(a, s);
     if (need > 4 && need <= 6) return launch_quant<6, 8, LN>(a, s);

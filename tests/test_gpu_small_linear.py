@@ -120,7 +120,8 @@ def test_nan_and_shapes_through_the_native_route():
 
 
 @pytest.mark.parametrize("M,K", [(3, 1032), (1025, 1536), (8193, 1032), (1000, 2048), (1030, 2040), (7, 2560), (9, 3072), (5, 2176), (4097, 2184),
-                                 (6, 4096), (11, 3080), (5, 5120), (6145, 5120), (13, 4608), (3, 5128), (2, 8192)])
+                                 (6, 4096), (11, 3080), (5, 5120), (6145, 5120), (13, 4608), (3, 5128), (2, 8192),
+                                 (2049, 4608), (4097, 5120), (4112, 5120), (2050, 6144), (2064, 6656), (2049, 7168)])
 def test_quantiser_with_shared_rows_bit_exact(M, K):
     """Rows that two or four wavefronts share, in both layouts, with a NaN row and a zero row."""
     import numpy as np
