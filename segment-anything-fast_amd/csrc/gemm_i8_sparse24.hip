@@ -540,12 +540,13 @@ static int sparse_common(int epi, const int8_t* xq, const float* sx, const int8_
   if (gemm_i8_sp24_persist_covers(epi, a)) return gemm_i8_sp24_persist_launch(epi, a, stream);
   const unsigned int grid = (unsigned int)(((total + 7) / 8) * 8);
   // The K split where a CU has one tile and the loop is long (us, one group / two; SAMFAST_GEMM_SPLITK=0 off, 2
-  // wherever it is built): 5003 x 5120 -> 1280 (200 tiles) 27.9 / 26.5, 4096 x 5120 -> 1280 (160) 27.9 / 25.8, 1500 x 5120
-  // -> 1280 (60) 24.9 / 22.0, 4096 x 3072 -> 768 (96) 19.3 / 17.9, 8192 x 3072 -> 768 (192) 20.6 / 20.6.  Shorter loops do not pay
-  // for the meeting in LDS (6500 x 1280 -> 1280: 13.5 / 14.2), and two tiles to a CU are better apart (8192 x 5120 ->
-  // 1280, 320 tiles: 43.3 / 51.3).  What bounds both is operand delivery, 12 TB/s over the CUs in use.
+  // wherever it is built).  K = 5120, while every tile has a CU: 60 tiles (1500 x 5120 -> 1280) 24.9 / 22.0, 160 (4096) 29.5 /
+  // 25.5, 200 (5003) 28.4 / 26.8, 220 28.9 / 28.0, 255 (6528) 31.7 / 30.8; 265 40.1 / 47.2, 320 42.8 / 48.6.  K = 3072 and 4096 pay
+  // less for the meeting in LDS the more CUs there are to feed, and nothing from 192 tiles on: 96 (4096 x 3072 -> 768) 17.8 /
+  // 16.4, 144 18.4 / 17.1, 192 19.1 / 19.0 and (2048 x 3072 -> 3072) 19.0 / 19.6, 225 20.8 / 21.1; 128 (4096 x 4096 -> 1024) 22.0 / 20.3, 192
+  // 23.0 / 22.9.  Shorter loops do not pay (6500 x 1280 -> 1280: 13.5 / 14.2).  What bounds both is operand delivery.
   const int sk = knob_or(KNOB_GEMM_SPLITK, 1);
-  const bool ksplit = epi != SEPI_I32 && K % (4 * SBK) == 0 && K / SBK >= 2 * S_NST && (sk >= 2 || (sk == 1 && total <= 208 && K >= 3072));
+  const bool ksplit = epi != SEPI_I32 && K % (4 * SBK) == 0 && K / SBK >= 2 * S_NST && (sk >= 2 || (sk == 1 && K >= 3072 && total <= (K >= 5120 ? 256 : 160)));
 #define SF_SP24(E)                                                                                              \
   do {                                                                                                          \
     if (ksplit) hipLaunchKernelGGL((gemm_i8_sp24_kernel<E, 2>), dim3(grid), dim3(512), 0, stream, a);           \

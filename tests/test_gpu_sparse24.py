@@ -267,7 +267,7 @@ def test_seeded_sweep_of_ragged_shapes_sparse_bit_exact():
         assert np.array_equal(acc.cpu().numpy().astype(np.int64), ref)
 
 
-@pytest.mark.parametrize("M,N,K,epi", [(1, 8, 512, 0), (5003, 1280, 5120, 0), (130, 264, 768, 1), (4096, 768, 3072, 2), (129, 1288, 512, 2), (257, 520, 1280, 1)])
+@pytest.mark.parametrize("M,N,K,epi", [(1, 8, 512, 0), (5003, 1280, 5120, 0), (130, 264, 768, 1), (4096, 768, 3072, 2), (129, 1288, 512, 2), (257, 520, 1280, 1), (6528, 1280, 5120, 2)])
 @pytest.mark.parametrize("layout", [0, 1])
 def test_sparse24_split_k_loop_agrees(M, N, K, epi, layout):
     """Two wavefront groups on alternate k tiles: the bits of one group walking them all."""
