@@ -316,8 +316,8 @@ int samfast_gemm_i8_sparse24_fused(
  *   samfast_layernorm  out = LayerNorm(x) over rows of K values; with r / sum given, sum = x + r (rounded
  *                      to the element type; may alias x or r) and out = LayerNorm(sum): `shortcut + x`
  *                      with the norm that follows.  fp32 statistics, biased variance.  Contiguous rows,
- *                      K % 8 == 0, K <= 4096.
- *   samfast_gelu       y = gelu_erf(x), n values (a multiple of 8); y may be x.
+ *                      K % 8 == 0, K <= 4096, eps >= 0.
+ *   samfast_gelu       y = x * Phi(x), n values (a multiple of 8); +inf gives +inf, -inf NaN; y may be x.
  */
 int samfast_layernorm(
     const void* x, const void* r, const void* gamma, const void* beta, float eps,

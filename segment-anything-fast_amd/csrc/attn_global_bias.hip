@@ -6,8 +6,8 @@
 // matrix instructions of the next half row's scores and of the previous one's P V, and the LDS reads that feed
 // them.  No running maximum is taken in the common case, LDS reads meet no bank twice (GridRow), and the
 // workgroups of a head touch its K and V ahead, so that the rows come out of their XCD's L2.
-//   Bound: at 8 x 16 x 4096 x 80 (745 us, 920 TFLOP/s; 805 us with attn_global_kernel) the power limit: the same
-//   loop with its MFMAs alone, on the same values, takes 666 us - 429 on zeros.  At one image of 12 heads
+//   Bound: at 8 x 16 x 4096 x 80 (fp16 760 us, 900 TFLOP/s, bf16 710; fp16 805 with attn_global_kernel) the power limit:
+//   the same loop with its MFMAs alone, on the same values, takes 666 us - 429 on zeros.  At one image of 12 heads
 //   (65 us against 83) the last, half-empty round and the prologue.
 //   (The encoder, which hands over tables, keeps attn_global_kernel: its int8 Linears turn any other order of these
 //   roundings into other codes.)

@@ -238,7 +238,7 @@ bool linear_i8_small_covers(int64_t M, int N, int K) {
   if (knob_or(KNOB_LINEAR_SMALL, 1) <= 0 || K % 64 != 0 || N % 8 != 0 || K > 5120) return false;
   // every workgroup quantises every row, 0.3 us per 8 rows of 1280: past these lines the separate quantiser
   // and the small-tile product take less GPU time than the repetition (16 x 3072: 9.1 us against 8.6), below
-  // them one launch also saves the host the second one (7 x 256 -> 2048: 5.5 us a call against 8.7)
+  // them one launch also saves the host the second one (7 x 256 -> 2048: 6.7 us a call against 8.7)
   return M <= 8 || (M <= 16 && K <= 2048) || (M <= 32 && K <= 768);
 }
 
