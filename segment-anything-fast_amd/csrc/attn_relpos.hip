@@ -640,8 +640,8 @@ __global__ __launch_bounds__(WindowCfg<HD>::THREADS, 2) void attn_window_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int slot = 8 * lh + 2 * i;
-          bhw[i] = slot < a.gh ? T::pack2(T::lo(ph[i]) * a.inv_scale, T::hi(ph[i]) * a.inv_scale) : 0u;
-          bww[i] = slot < a.gw ? T::pack2(T::lo(pw[i]) * a.inv_scale, T::hi(pw[i]) * a.inv_scale) : 0u;
+          bhw[i] = slot < a.gh ? T::pack2(bias_slot<T>(T::lo(ph[i]), a), bias_slot<T>(T::hi(ph[i]), a)) : 0u;
+          bww[i] = slot < a.gw ? T::pack2(bias_slot<T>(T::lo(pw[i]), a), bias_slot<T>(T::hi(pw[i]), a)) : 0u;
         }
       } else {
 #pragma unroll
@@ -650,8 +650,8 @@ __global__ __launch_bounds__(WindowCfg<HD>::THREADS, 2) void attn_window_kernel(
 #pragma unroll
           for (int v = 0; v < 2; ++v) {
             const int slot = 8 * lh + 2 * i + v;
-            const float rh_raw = T::from_bits(rhp[min(slot, a.gh - 1)]) * a.inv_scale;
-            const float rw_raw = T::from_bits(rwp[min(slot, a.gw - 1)]) * a.inv_scale;
+            const float rh_raw = bias_slot<T>(T::from_bits(rhp[min(slot, a.gh - 1)]), a);
+            const float rw_raw = bias_slot<T>(T::from_bits(rwp[min(slot, a.gw - 1)]), a);
             fh[v] = (slot < a.gh) ? rh_raw : 0.f;
             fw[v] = (slot < a.gw) ? rw_raw : 0.f;
           }
@@ -712,7 +712,8 @@ __global__ __launch_bounds__(WindowCfg<HD>::THREADS, 2) void attn_window_kernel(
     for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
-    float m_run = -3.0e38f, l_run = 0.f;
+    // (in units of the scores: kLowest is one of exponents)  Finite, and above what a masked tile holds: that contributes zero
+    float m_run = T::kLowest * (a.inv_scale / kLog2e), l_run = 0.f;
 #pragma unroll
     for (int nt = 0; nt < C::NT; ++nt) {
       if (32 * nt < N) {  // uniform

@@ -46,7 +46,7 @@ struct ElemBf16 {
   static constexpr float kMargin = 16.0f;
   static SF_DEVICE unsigned int note(unsigned int seen, unsigned int w0, unsigned int w1) { return seen | w0 | w1; }
   static SF_DEVICE bool outgrown(unsigned int seen) { return (seen & 0x40004000u) != 0u; }
-  // global kernel with the caller's factors: the exponent reference (log2) before any key has been met.  Keys below it
+  // kernels with the caller's factors: the exponent reference (log2) before any key has been met.  Keys below it
   // are as good as masked.  Down to it every probability is finite: at 2^31 a reference and a difference from it
   // are each rounded by at most 64, so that a probability stays below 2^(128 - kMargin).
   static constexpr float kLowest = -2147483648.0f;
@@ -154,6 +154,13 @@ struct GridRow {
     return key * (VP * 16) + half * 64 + 32 * (g & 1) + 8 * (sl & 3);
   }
 };
+
+// A factor of the caller's as an operand of the window kernels' bias products, whose other operand is zeros and ones: divided
+// by the scale and not below T::kMask, the value that takes a key away (0 * -inf would be a NaN for every key; a NaN stays one).
+template <typename T>
+SF_DEVICE float bias_slot(float factor, const AttnArgs& a) {
+  return __builtin_elementwise_maximum(factor * a.inv_scale, T::from_bits(T::kMask));
+}
 
 // all LDS operations this wavefront has issued are complete and ordered
 SF_DEVICE void wave_lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }

@@ -238,7 +238,7 @@ __global__ __launch_bounds__(RowsCfg<HD>::THREADS, 2) void attn_window_rows_kern
 #pragma unroll
         for (int v = 0; v < 2; ++v) {
           const int slot = 8 * lh + 2 * i + v;
-          const float raw = T::from_bits(rwp[min(slot, a.gw - 1)]) * a.inv_scale;
+          const float raw = bias_slot<T>(T::from_bits(rwp[min(slot, a.gw - 1)]), a);
           pr[v] = slot < a.gw ? (T::pack2(raw, 0.f) & 0xffffu) : T::kMask;
         }
         bww[i] = pr[0] | (pr[1] << 16);
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(RowsCfg<HD>::THREADS, 2) void attn_window_rows_kern
     for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
-    float m_run = -3.0e38f, l_run = 0.f;  // m_run in exponent (log2) units
+    float m_run = T::kLowest, l_run = 0.f;  // m_run in exponent (log2) units, above what a masked tile holds
     const unsigned char* krow = kl + (lr * C::KSTR + 8 * lh) * 2;
 #pragma unroll
     for (int nt = 0; nt < C::NT; ++nt) {

@@ -281,7 +281,7 @@ class Block(nn.Module):
         if not (FUSED_BLOCK and flash_4.USE_CUSTOM_KERNEL and x.is_cuda and x.dim() == 4
                 and x.dtype in (torch.bfloat16, torch.float16) and attn.use_rel_pos and not torch.is_grad_enabled()):
             return False
-        if not self._as_built() or mlp.act.approximate != "none" or not ops.unwatched(x):
+        if not ops.unwatched(x) or not self._as_built() or mlp.act.approximate != "none":
             return False
         B, H, W, C = x.shape
         for n in (self.norm1, self.norm2):

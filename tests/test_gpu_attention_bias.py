@@ -172,6 +172,34 @@ def test_bias_kernels_with_masked_keys(form, mask, hd, dtype, values):
             assert (out.cpu().double() - ref).abs().max() <= 4 * torch.finfo(dtype).eps * v.abs().max().item()
 
 
+@pytest.mark.parametrize("layout", ["tokens", "rows"])
+@pytest.mark.parametrize("gh,gw", [(14, 14), (13, 14), (14, 5), (6, 8), (7, 13)])
+@pytest.mark.parametrize("hd,dtype,values", [
+    (64, torch.bfloat16, (-math.inf, torch.finfo(torch.bfloat16).min, -1e30, -1e9, -1e4)),
+    (80, torch.bfloat16, (-math.inf, -1e9)),
+    (64, torch.float16, (-math.inf, torch.finfo(torch.float16).min, -1e3)),
+    (80, torch.float16, (-math.inf, -1e3)),
+])
+def test_window_kernels_with_masked_keys(layout, gh, gw, hd, dtype, values):
+    """As on the grid: rows and columns taken away, the first key tiles of 32 whole among them, for every and every second query."""
+    from samfast_amd import _lib, ops
+    q, k, v, rel_h, rel_w = bias_inputs(3, 2, gh, gw, hd, seed=gh + gw, dtype=dtype)
+    for rows, cols in ((slice(0, gh - 1), None), (None, slice(0, gw - 1)), (slice(0, 3), slice(0, 2)), (slice(1, gh), None), (slice(3, 5), slice(2, 4))):
+        for value in values:
+            for step in (1, 2):
+                print(f"case masked window {layout} {gh}x{gw} hd={hd} {dtype} {rows} {cols} {value} every {step}", flush=True)
+                rh, rw = rel_h.squeeze(-1).clone(), rel_w.squeeze(-2).clone()
+                if rows is not None:
+                    rh[:, :, ::step, rows] = value
+                if cols is not None:
+                    rw[:, :, ::step, cols] = value
+                s = q.double() @ k.double().transpose(-1, -2) * hd ** -0.5 + (rh.double()[..., None] + rw.double()[..., None, :]).flatten(-2)
+                ref = s.softmax(-1) @ v.double()
+                with _lib.knobs(SAMFAST_ATTN_WINDOW_ROWS=int(layout == "rows")):
+                    out = ops.attn_relpos_bias(q.cuda(), k.cuda(), v.cuda(), rh.cuda(), rw.cuda())
+                assert (out.cpu().double() - ref).abs().max() <= 4 * torch.finfo(dtype).eps * v.abs().max().item()
+
+
 @pytest.mark.parametrize("gh,gw", [(14, 14), (2, 2), (13, 14), (14, 5), (6, 8), (1, 16), (15, 13)])
 @pytest.mark.parametrize("hd,dtype", [(64, torch.bfloat16), (80, torch.float16)])
 def test_window_factors_read_in_pairs_or_one_by_one(gh, gw, hd, dtype):
