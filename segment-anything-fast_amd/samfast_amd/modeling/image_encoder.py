@@ -186,17 +186,16 @@ class Block(nn.Module):
     def _pad_rows(self, nH: int, hd: int, device):
         """(nH, hd) bf16 k and v rows of a zero-padded token: the qkv bias, rounded as the
         Linear's epilogue rounds it."""
-        bias = self.attn.qkv.bias_f32
-        key = None if bias is None else (bias.data_ptr(), self.attn.qkv.bias_bits._version, str(device))
-        if getattr(self, "_pad_key", "unset") != key:
-            C = nH * hd
+        from ..quant import kept_copy
+        qkv, C = self.attn.qkv, nH * hd
+
+        def rows():
+            bias = qkv.bias_f32
             if bias is None:
-                pk = pv = torch.zeros((nH, hd), dtype=torch.bfloat16, device=device)
-            else:
-                pk = bias[C:2 * C].to(torch.bfloat16).view(nH, hd).contiguous()
-                pv = bias[2 * C:3 * C].to(torch.bfloat16).view(nH, hd).contiguous()
-            self._pad_key, self._pad_kv = key, (pk, pv)
-        return self._pad_kv
+                return (torch.zeros((nH, hd), dtype=torch.bfloat16, device=device),) * 2
+            return tuple(bias[i * C:(i + 1) * C].to(torch.bfloat16).view(nH, hd).contiguous() for i in (1, 2))
+
+        return kept_copy(self, "_pad_kv", qkv.sw_bits if qkv.bias_bits is None else qkv.bias_bits, rows)
 
     def _chains_from_previous(self) -> bool:
         """Whether this block's norm1 + quantiser can run in the previous block's lin2 launch:

@@ -71,6 +71,24 @@ def quantize_weight_per_channel(weight: torch.Tensor, convention: str = "absmax1
     return q.contiguous(), scale.to(torch.float32).contiguous()
 
 
+def kept_copy(holder: nn.Module, name: str, source: torch.Tensor, make: Callable[[], object]):
+    """What make() derives from `source`, a buffer of the module: kept on `holder` and made anew when the
+    buffer is another one, elsewhere or written to (load_state_dict, .to()).  It is complete before
+    it is kept, so that any stream and thread may read it.  Made while a graph is recorded, it exists
+    at the replays only, and writes to inference tensors leave no trace: neither is kept."""
+    counted = not source.is_inference()
+    hit = holder.__dict__.get(name)
+    if hit is not None and counted and hit[0] is source and hit[1] == source.data_ptr() and hit[2] == source._version:
+        return hit[3]
+    made = make()
+    if not counted or (source.is_cuda and torch.cuda.is_current_stream_capturing()):
+        return made
+    if source.is_cuda:
+        torch.cuda.current_stream(source.device).synchronize()
+    holder.__dict__[name] = (source, source.data_ptr(), source._version, made)
+    return made
+
+
 class Int8LinearBase(nn.Module):
     """What every int8 Linear here shares: shapes, per-channel weight scales and bias.
 
@@ -162,8 +180,6 @@ class Int8DynamicLinear(Int8LinearBase):
                  bias: Optional[torch.Tensor]) -> None:
         super().__init__(in_features, out_features, sw, bias)
         self.register_buffer("wq", wq)
-        self._wq_kb64 = None  # derived K-block major copy, not part of the state dict
-        self._wq_kb64_key = None
 
     @classmethod
     def from_float(cls, linear: nn.Linear, weight_convention: str = "absmax127") -> "Int8DynamicLinear":
@@ -180,12 +196,7 @@ class Int8DynamicLinear(Int8LinearBase):
 
     def _weight_for(self, layout: int) -> torch.Tensor:
         wq = self._buffers["wq"]
-        if layout != LAYOUT_KB64:
-            return wq
-        key = self._wq_kb64_key  # rebuilt after load_state_dict / .to()
-        if key is None or key[0] is not wq or key[1] != wq.data_ptr() or key[2] != wq._version:
-            self._wq_kb64, self._wq_kb64_key = ops.to_kb64(wq), (wq, wq.data_ptr(), wq._version)
-        return self._wq_kb64
+        return wq if layout != LAYOUT_KB64 else kept_copy(self, "_kb64", wq, lambda: ops.to_kb64(wq))
 
     def _forward_native(self, x: torch.Tensor) -> Optional[torch.Tensor]:
         buffers = self._buffers  # the weights as they stand: no copy that could be behind them

@@ -108,7 +108,7 @@ def test_bias_kernels_read_strided_factors():
 
 
 def test_the_operator_is_there_for_those_who_watch():
-    """A trace records it, vmap loops over it, a dispatch mode sees it - and nobody gets another result."""
+    """A trace and a compiled graph record it, vmap loops over it, a dispatch mode sees it - and nobody gets another result."""
     from torch.utils._python_dispatch import TorchDispatchMode
     from samfast_amd.flash_4 import _attention_rel_h_rel_w as attention
     args = [t.cuda() for t in bias_inputs(1, 2, 64, 64, 64, seed=1)]
@@ -119,6 +119,15 @@ def test_the_operator_is_there_for_those_who_watch():
     assert torch.equal(traced(*other), want_other)
     both = torch.vmap(attention)(*(torch.stack(pair) for pair in zip(args, other)))
     assert torch.equal(both[0], want) and torch.equal(both[1], want_other)
+
+    graphs = []
+
+    def keep(graph_module, example_inputs):
+        graphs.append(graph_module.code)
+        return graph_module.forward
+
+    assert torch.equal(torch.compile(attention, backend=keep, fullgraph=True)(*args), want)
+    assert "custom_flash_aligned" in graphs[0]
 
     class Names(TorchDispatchMode):
         names = []

@@ -92,6 +92,35 @@ def test_a_linears_first_call_anywhere(M):
         assert torch.equal(recorded, want)
 
 
+def test_the_blocks_copy_of_a_weight_is_complete_wherever_it_is_made():
+    """The K-block major copy that linear_fused keeps: first needed while a graph is recorded, then on two streams, and in
+    inference mode."""
+    from samfast_amd import _lib, ops
+    lin = _linear(264, 256, 5)
+    x = torch.randn((300, 256), device="cuda").to(torch.bfloat16)
+    want = _unfused(lin, x)
+    xk, sx = ops.quant_rowwise(x, _lib.LAYOUT_KB64)
+    run = lambda m: m.linear_fused(xk, sx, _lib.EPILOGUE_NONE, layout=_lib.LAYOUT_KB64)
+    graph = torch.cuda.CUDAGraph()
+    with torch.no_grad(), torch.cuda.graph(graph):
+        recorded = run(lin)
+    assert torch.equal(run(lin), want)  # before any replay
+    for _ in range(3):
+        recorded.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(recorded, want)
+    fresh, side = _linear(264, 256, 5), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        there = run(fresh)
+    here = run(fresh)
+    torch.cuda.synchronize()
+    assert torch.equal(there, want) and torch.equal(here, want)
+    with torch.inference_mode():
+        assert torch.equal(run(_linear(264, 256, 5)), want)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 8, 256), (31, 40, 384), (33, 264, 256), (65, 1280, 5120), (500, 1288, 2048), (130, 4096, 1280)])
 def test_sparse_linear_over_few_rows_bit_exact(M, N, K):
     from samfast_amd import Int8Sparse24Linear
