@@ -18,6 +18,7 @@
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/PyInterpreter.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "samfast.h"
@@ -37,12 +38,25 @@ const Bound kBound[] = {
     {"samfast_attn_relpos_bias_fwd", reinterpret_cast<void**>(&p_attn_bias)},
 };
 
+PyObject* device_context = nullptr;  // the mode of `with torch.device(..)` and torch.set_default_device, set by bind()
+
+// Function modes see calls in Python; the one that only gives factory functions their device need not see these.
+bool function_mode_watches() {
+  using at::impl::PythonTorchFunctionTLS;
+  if (!at::impl::torch_function_mode_enabled()) return false;
+  for (int64_t i = 0; i < PythonTorchFunctionTLS::stack_len(); ++i) {
+    PyObject* mode = PythonTorchFunctionTLS::get_stack_at(i)->ptr(getPyInterpreter());
+    if (reinterpret_cast<PyObject*>(Py_TYPE(mode)) != device_context) return true;
+  }
+  return false;
+}
+
 // Whether nobody but the kernels has to see this thread's calls: a launch on raw pointers passes by tracers,
 // functional transforms (vmap, grad, functionalization) and dispatch and function modes.  All but the last stand as
 // dispatch keys that the thread has included beyond the default ones.
 bool plain_call() {
   return (c10::impl::tls_local_dispatch_key_set().included_ | c10::default_included_set) == c10::default_included_set &&
-         !at::impl::torch_function_mode_enabled();
+         !function_mode_watches();
 }
 
 // A tensor that is its memory and nothing more: no wrapper of a transform, subclass, conjugate or negative view, sparse or
@@ -192,6 +206,13 @@ PyObject* host_bind(PyObject*, PyObject* table) {
     void* p = PyLong_AsVoidPtr(v);
     if (!p) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_ValueError, "samfast: %s has no address", b.name);
     *b.slot = p;
+  }
+  if (!device_context) {
+    PyObject* module = PyImport_ImportModule("torch.utils._device");
+    if (!module) return nullptr;
+    device_context = PyObject_GetAttrString(module, "DeviceContext");  // kept
+    Py_DECREF(module);
+    if (!device_context) return nullptr;
   }
   Py_RETURN_NONE;
 }

@@ -396,6 +396,8 @@ def test_native_calls_decline_where_somebody_watches():
     with torch.inference_mode():
         assert plain(x) and plain(torch.zeros(2))
     assert plain(torch.ones(2, requires_grad=True) * 2)
+    with torch.device("cpu"):  # a function mode, but one for factory functions
+        assert plain(x)
     answers = []
 
     def watched(t):
@@ -418,7 +420,9 @@ def test_native_calls_decline_where_somebody_watches():
     for mode in (Through, Pass):
         with mode():
             watched(x)
-    assert len(answers) == 6 and not any(any(a) for a in answers), answers
+    with torch.device("cpu"), Pass():
+        watched(x)
+    assert len(answers) == 7 and not any(any(a) for a in answers), answers
     with torch.autograd.forward_ad.dual_level():
         assert not plain(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)))
 
