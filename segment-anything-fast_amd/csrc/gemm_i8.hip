@@ -1007,10 +1007,13 @@ static int gemm_common(int epi, const int8_t* xq, const float* sx, const int8_t*
   SF_REQUIRE(total < (1ll << 30), "gemm_i8: too many tiles");
   // few rows: the K loop dealt out inside small tiles
   if (!tail && epi == EPI_SCALE_BIAS_BF16 && gemm_i8_skinny_covers(a)) return gemm_i8_skinny_launch(a, stream);
-  // outputs the GPU holds once, K >= 1280: one tile per CU (not where one of the other members is asked for)
-  if (!tail && tm == 2 && knob(KNOB_GEMM_TILE) == kKnobUnset && knob(KNOB_GEMM_WG3) != 0 && knob_or(KNOB_GEMM_PERSIST, 1) < 2 &&
-      knob_or(KNOB_GEMM_SPLITK, 1) < 2 && gemm_i8_once_covers(epi, a))
-    return gemm_i8_once_launch(epi, a, stream);
+  // (not where one of the other members is asked for)
+  const bool unasked = !tail && tm == 2 && knob(KNOB_GEMM_TILE) == kKnobUnset && knob(KNOB_GEMM_WG3) != 0 &&
+                       knob_or(KNOB_GEMM_PERSIST, 1) < 2 && knob_or(KNOB_GEMM_SPLITK, 1) < 2;
+  // whole rounds of 256 x 256 or 256 x 320 tiles: the halves of a workgroup by turns
+  if (unasked && knob_or(KNOB_GEMM_ONCE, 1) <= 1 && gemm_i8_pingpong_covers(epi, a)) return gemm_i8_pingpong_launch(epi, a, stream);
+  // outputs the GPU holds once, K >= 1280: one tile per CU
+  if (unasked && gemm_i8_once_covers(epi, a)) return gemm_i8_once_launch(epi, a, stream);
   // resident workgroups that walk a list of tiles each (SAMFAST_GEMM_PERSIST=1), where built
   if (!tail && !generic_k && tm == 2 && gemm_i8_persist_covers(epi, a)) return gemm_i8_persist_launch(epi, a, stream);
   const unsigned int grid = (unsigned int)(((total + 7) / 8) * 8);
@@ -1207,7 +1210,9 @@ __global__ __launch_bounds__(256) void kblock_major_kernel(const int8_t* w, int8
 // they are / reordered / K-block major already: 4096 x 1280 -> 3840: 32.8 / 37 / 32.6, 8192 x 1024 -> 4096: 53.9 / 54.7 / 52.1,
 // 16384 x 1280 -> 3840: 105 / 102 / 98, 16384 x 5120 -> 1280: 136 / 137 / 133, 65536 x 1280 -> 3840: 380 / 352 / 348,
 // 65536 x 5120 -> 1280: 657 / 575 / 571.  (Row-major codes as well: 35, 65, 120, 140, 408, 640.)
-static bool linear_reorders_weights(int64_t M) { return M >= 16384; }
+// The products by turns (gemm_pingpong.hpp) read 128 bytes of a row at a time: nothing to reorder there (the Linear 65536 x
+// 1280 -> 3840: 335 as they are, 339 reordered).
+static bool linear_reorders_weights(int64_t M, int N, int K) { return M >= 16384 && !gemm_i8_pingpong_reads_rows(M, N, K); }
 
 // bytes of the codes in a Linear's workspace; their row scales follow, then reordered weights
 static int64_t linear_codes_bytes(int64_t M, int K) { return (M * K + 15) & ~(int64_t)15; }
@@ -1220,7 +1225,7 @@ extern "C" int64_t samfast_linear_i8_workspace(int64_t M, int N, int K, int layo
   SF_REQUIRE(M > 0 && N > 0 && K > 0 && layout >= SAMFAST_LAYOUT_ROWMAJOR && layout <= SAMFAST_LAYOUT_SPARSE24,
              "linear_i8_workspace: bad shape M=%lld N=%d K=%d or layout %d", (long long)M, N, K, layout);
   if (layout != SAMFAST_LAYOUT_SPARSE24 && linear_i8_small_covers(M, N, K)) return 0;
-  const int64_t weights = layout == SAMFAST_LAYOUT_ROWMAJOR && linear_reorders_weights(M) ? (int64_t)N * K : 0;
+  const int64_t weights = layout == SAMFAST_LAYOUT_ROWMAJOR && linear_reorders_weights(M, N, K) ? (int64_t)N * K : 0;
   return linear_codes_bytes(M, K) + linear_scales_bytes(M) + weights;
 }
 
@@ -1244,7 +1249,7 @@ extern "C" int samfast_linear_i8(const void* x, int64_t ldx, const int8_t* wq, c
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int rc = samfast_quant_rowwise_i8(x, ldx, xq, sx, M, K, dtype, SAMFAST_LAYOUT_KB64, stream);
   if (rc != SAMFAST_OK) return rc;
-  if (layout == SAMFAST_LAYOUT_ROWMAJOR && linear_reorders_weights(M)) {
+  if (layout == SAMFAST_LAYOUT_ROWMAJOR && linear_reorders_weights(M, N, K)) {
     int8_t* wk = xq + linear_codes_bytes(M, K) + linear_scales_bytes(M);
     hipLaunchKernelGGL(kblock_major_kernel, dim3((unsigned int)(((int64_t)N * K / 16 + 255) / 256)), dim3(256), 0, s, wq, wk, N, K);
     const int rl = check_launch("kblock_major_kernel");

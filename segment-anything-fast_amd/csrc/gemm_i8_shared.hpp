@@ -50,6 +50,12 @@ SF_DEVICE int lds_swizzle(int row) { return ((row >> 1) & 3) ^ ((row >> 3) & 1);
 bool gemm_i8_persist_covers(int epi, const GemmArgs& a);
 int gemm_i8_persist_launch(int epi, const GemmArgs& a, hipStream_t stream);
 
+// 256 x 256 tiles by turns (gemm_i8_pingpong.hip), the same way.
+bool gemm_i8_pingpong_covers(int epi, const GemmArgs& a);
+int gemm_i8_pingpong_launch(int epi, const GemmArgs& a, hipStream_t stream);
+// Whether a plain product of this shape goes there, where row-major operands are read in whole lines as well.
+bool gemm_i8_pingpong_reads_rows(int64_t M, int N, int K);
+
 // One tile per CU (gemm_i8_once.hip), the same way.
 bool gemm_i8_once_covers(int epi, const GemmArgs& a);
 int gemm_i8_once_launch(int epi, const GemmArgs& a, hipStream_t stream);

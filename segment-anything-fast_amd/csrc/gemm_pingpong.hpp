@@ -1,0 +1,478 @@
+// One matrix product y = x . w^T for the element types of this library (int8, bf16, fp16): output tiles of 256 rows and 256 or 320
+// columns, one resident workgroup of eight wavefronts per CU, two per SIMD that take turns at the matrix pipe.
+//
+// What bounds it is power, not the matrix pipe.  The pipe is busy 0.93-0.96 of the loop's cycles, and on operands
+// like an encoder's the clock settles at 1.5-1.7 GHz of 2.4, so every choice here is about energy per product or
+// about cycles in which nothing is multiplied:
+//   * v_mfma_*_16x16x(64 bytes): bare loops of them sustain 3.9 POP/s on Gaussian codes (bf16: 1.93 PFLOP/s) where the
+//     32x32 forms sustain 3.5 (1.8): half the accumulator bytes per product cross the register file;
+//   * 256 x 256 tiles: a third fewer operand bytes from the L2s than 128 x 256 (the loads are 17 % of the energy, the
+//     LDS reads 7 %: loops without them run that much faster at the same pipe occupancy);
+//   * turns: the wavefronts 0-3 multiply while 4-7 (their SIMD partners) read fragments and request tiles, and
+//     the other way round, a barrier between turns of 32 matrix instructions.  The same code with both halves in
+//     step keeps the pipe busy 0.59 of the time.
+// A k tile is 128 bytes of every row, so row-major operands are read in whole lines as well as K-block-major ones.  Two
+// of them fit the LDS; a wavefront multiplies its 64 rows by the lower 64 of its 128 columns in the first turn and
+// by the upper 64 in the second.  After the first the X rows and the lower columns are free again, after the
+// second the upper ones, and each part is requested anew as soon as it is free: every load has one and a half k tiles
+// (2500 cycles) to arrive although only two are held.
+//
+// Epilogues: int8 (float(acc) * sx[m]) * sw[n] + bias[n] in three separately rounded fp32 operations, the half
+// types acc + bias[n]; rounded to the output type; then nothing, GELU of the rounded value, or + residual (one more
+// rounding).  A wavefront's columns are dealt to the LDS rows so that a lane ends with four adjacent ones and stores
+// 128-byte segments straight from the accumulators, between the turns.  (Held in registers and sent out a few per turn of
+// the next tile, as gemm_i8_persist_kernel does, the stores lengthened every turn: 65536 x 1280 -> 3840 took 363 us for 310.)
+//
+// Inside the ViT-H encoder at 65536 rows, us per launch, before / with this kernel: 1280 -> 3840 309 / 263 (2.45 POP/s), 5120 -> 1280 with
+// the residual 404 / 337 (2.55), 1280 -> 1280 with it 136 / 135 (0.4 GB of rows through HBM).
+#pragma once
+
+#include "gemm_i8_shared.hpp"
+#include "attn_relpos_shared.hpp"
+
+#include <type_traits>
+
+#pragma clang fp contract(off)
+
+namespace samfast {
+
+struct PPArgs {
+  const unsigned char* x;  // byte addresses; x_pitch / w_pitch bytes between rows, *_kstep between the 64-byte pieces of a row
+  const unsigned char* w;
+  unsigned short* out;
+  const float* sx;         // int8: row scales, column scales
+  const float* sw;
+  const void* bias;        // int8: fp32, else the element type; may be null
+  const unsigned short* residual;
+  int64_t ldo, ld_res;     // elements
+  int64_t x_kstep, w_kstep;
+  unsigned int x_pitch, w_pitch;
+  int M, N, nk;            // nk: 128-byte k tiles
+  int tiles_m, tiles_n, group_m;
+};
+
+struct PPInt8 {
+  typedef i32x4 acc_t;
+  typedef ElemBf16 Out;
+  static constexpr bool SCALED = true;
+  static SF_DEVICE acc_t mma(i32x4 a, i32x4 b, acc_t c) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0); }
+};
+struct PPBf16 {
+  typedef f32x4 acc_t;
+  typedef ElemBf16 Out;
+  static constexpr bool SCALED = false;
+  static SF_DEVICE acc_t mma(i32x4 a, i32x4 b, acc_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+};
+struct PPF16 {
+  typedef f32x4 acc_t;
+  typedef ElemF16 Out;
+  static constexpr bool SCALED = false;
+  typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+  static SF_DEVICE acc_t mma(i32x4 a, i32x4 b, acc_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  }
+};
+
+enum { PP_PLAIN = 0, PP_GELU = 1, PP_RESIDUAL = 2 };
+
+// vmcnt <= N and every LDS read of this wavefront done
+template <int N>
+SF_DEVICE void pp_wait() {
+  __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | ((N >> 4) << 14));
+}
+
+// TN: 16-column fragments of a wavefront's half of the tile (the tile has 256 rows and 32 TN columns).  A turn multiplies H
+// of them.  The fragments' columns are dealt so that a lane ends with quads and at most one pair of adjacent columns:
+// element e of a quad q is column 64 q + 4 lr + e of the half, of the pair 64 NQ + 2 lr + e.
+template <int TN>
+struct PPTile {
+  static_assert(TN == 8 || TN == 10, "widths built: 256, 320");
+  static constexpr int BM = 256, BN = 32 * TN, H = TN / 2;
+  static constexpr int NQ = TN / 4;
+  static constexpr bool PAIR = TN % 4 != 0;
+  static constexpr int STAGE = (BM + BN) * 128;        // one k tile of X and W
+  static constexpr int SCALES = BM * 4 + 2 * BN * 4;   // int8: sx, sw, bias; half types: bias in the first bytes
+  static constexpr int NLOADS = 4 + H;                 // of a wavefront per k tile
+  static constexpr int NSTORES = 16 * (NQ + PAIR);
+  static_assert(2 * STAGE + SCALES <= 160 * 1024, "LDS of a CU");
+  static_assert(NLOADS + NSTORES < 64, "vmcnt threshold");
+  // column of the half that fragment j of a turn holds in its row r
+  static SF_DEVICE int column(int turn, int j, int r) { return j < 4 ? 64 * turn + 4 * r + j : 64 * NQ + 2 * r + turn; }
+  // fragment (of both turns) of element e of quad q / of the pair
+  static constexpr int quad(int q, int e) { return q * H + e; }
+  static constexpr int pair(int e) { return e * H + H - 1; }
+};
+
+// NT: non-temporal stores
+template <class E, int EPI, int TN, bool NT>
+__global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
+  typedef typename E::Out Out;
+  using P = PPTile<TN>;
+  constexpr bool RES = EPI == PP_RESIDUAL;
+  constexpr int H = P::H;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * P::STAGE + P::SCALES];
+  unsigned char* sc = lds + 2 * P::STAGE;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave & 3, wn = wave >> 2;  // 64 rows, half of the columns; wn is also the side that takes turns
+  const int lr = lane & 15, lq = lane >> 4;
+
+  // ---- the tiles of this workgroup: XCD x owns a contiguous range, its workgroups walk it side by side -----------
+  const unsigned int total = (unsigned int)a.tiles_m * (unsigned int)a.tiles_n;
+  const unsigned int xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3, per_x = gridDim.x >> 3;
+  const unsigned int chunk = (total + 7u) >> 3;
+  const unsigned int first = xcd * chunk + slot;
+  const unsigned int last = min(total, (xcd + 1u) * chunk);
+  if (slot >= chunk || first >= last) return;  // uniform over the workgroup
+  const int nt = (int)((last - first + per_x - 1u) / per_x);
+  // Origin of tile ti.  Tiles at the lower and right edge are moved back inside (M >= 256, N >= BN), so that every load is in
+  // bounds; the rows and columns that belong to the tile before (skip_m, skip_n) are not stored.
+  auto tile_origin = [&](int ti, int& m0, int& n0, int& skip_m, int& skip_n) __attribute__((always_inline)) {
+    const unsigned int pid = first + (unsigned int)ti * per_x;
+    const unsigned int per_group = (unsigned int)a.group_m * a.tiles_n;
+    const unsigned int first_m = (pid / per_group) * a.group_m;
+    const unsigned int gsz = min((unsigned int)a.tiles_m - first_m, (unsigned int)a.group_m);
+    const unsigned int in_group = pid % per_group;
+    m0 = (int)(first_m + in_group % gsz) * P::BM;
+    n0 = (int)(in_group / gsz) * P::BN;
+    skip_m = max(m0 + P::BM - a.M, 0);
+    skip_n = max(n0 + P::BN - a.N, 0);
+    m0 -= skip_m;
+    n0 -= skip_n;
+  };
+
+  typedef __attribute__((address_space(1))) const void* gptr_t;
+  typedef __attribute__((address_space(3))) void* lptr_t;
+  // ---- tile loads.  A wave instruction fills eight LDS rows of 128 bytes.  16-byte chunk c of LDS row r lives at
+  // position c ^ ((r >> 1) & 7): a fragment read (16 rows, four chunks, served in the groups of once_swizzle's note)
+  // then touches every bank once.  W rows lie half by half, in it turn by turn, in it fragment by fragment.
+  // Of the 4 H eights of W rows that a turn reads, wavefronts 0-3 request LO of the first turn and H - LO of the second each,
+  // wavefronts 4-7 the others.
+  unsigned int off_x, off_w[H];
+  int at_w[H];  // their LDS rows
+  constexpr int LO = (H + 1) / 2;
+  const int lo = wn == 0 ? LO : H - LO;  // this wavefront's loads for the first turn
+#pragma unroll
+  for (int i = 0; i < H; ++i) {
+    const int turn = i >= lo, v = turn ? (wn == 0 ? wm * (H - LO) : 4 * (H - LO) + wm * LO) + i - lo
+                                       : (wn == 0 ? wm * LO : 4 * LO + wm * (H - LO)) + i;
+    at_w[i] = (v / (2 * H)) * 16 * TN + turn * 16 * H + (v % (2 * H)) * 8;
+  }
+  {
+    auto chunk_of = [&](int row) __attribute__((always_inline)) { return (lane & 7) ^ ((row >> 1) & 7); };
+    const int cx = chunk_of(wave * 8 + (lane >> 3));
+    off_x = (unsigned int)(wave * 8 + (lane >> 3)) * a.x_pitch + (unsigned int)((cx >> 2) * a.x_kstep) + (cx & 3) * 16;
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      const int half = at_w[i] / (16 * TN), in = at_w[i] % (16 * TN), turn = in / (16 * H), j = in % (16 * H) / 16;
+      const int r = in % 16 + (lane >> 3), cw = chunk_of(r);
+      const int col = half * 16 * TN + P::column(turn, j, r);
+      off_w[i] = (unsigned int)col * a.w_pitch + (unsigned int)((cw >> 2) * a.w_kstep) + (cw & 3) * 16;
+    }
+  }
+  const unsigned char *xk, *wk;  // tile row 0 / column 0 in the k tile that is requested next
+  auto load = [&](const unsigned char* base, unsigned int o, int row, int stage) __attribute__((always_inline)) {
+    asm volatile("" : "+s"(base));  // uniform base, 32-bit lane offset
+    asm volatile("" : "+v"(o));
+    __builtin_amdgcn_global_load_lds((gptr_t)(base + o), (lptr_t)(lds + stage + row * 128), 16, 0, 0);
+  };
+  auto load_x = [&](int stage) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) load(xk + (int64_t)(64 * i) * a.x_pitch, off_x, (wave + 8 * i) * 8, stage);
+  };
+  auto load_w = [&](int turn, int stage) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      const bool mine = H % 2 == 0 ? (i >= LO) == (turn == 1) : i < H - LO ? turn == 0 : i >= LO ? turn == 1 : (i >= lo) == (turn == 1);
+      if (mine) load(wk, off_w[i], P::BM + at_w[i], stage);
+    }
+  };
+  int m0, n0, skip_m, skip_n, lt = 0, lk = 0;
+  auto first_ktile = [&]() __attribute__((always_inline)) {
+    int m, n, sm, sn;
+    tile_origin(lt, m, n, sm, sn);
+    xk = a.x + (int64_t)m * a.x_pitch;
+    wk = a.w + (int64_t)n * a.w_pitch;
+  };
+  first_ktile();
+  tile_origin(0, m0, n0, skip_m, skip_n);
+  auto next_ktile = [&]() __attribute__((always_inline)) {
+    xk += 2 * a.x_kstep;
+    wk += 2 * a.w_kstep;
+    if (++lk == a.nk) {
+      // the first k tiles of the next tile (behind the last one: its own again, read by nobody)
+      lk = 0;
+      if (lt + 1 < nt) ++lt;
+      first_ktile();
+    }
+  };
+  // scales and bias of the tile, 64 lanes of 4 bytes an instruction, the same number for every wavefront (some repeated)
+  auto load_scales = [&]() __attribute__((always_inline)) {
+    if constexpr (E::SCALED) {
+      constexpr int XS = P::BM / 64, WS = P::BN / 64, SLICES = XS + 2 * WS;
+#pragma unroll
+      for (int e = 0; e < (SLICES + 7) / 8; ++e) {
+        const int s = (wave + 8 * e) % SLICES;
+        const int part = s < XS ? 0 : s < XS + WS ? 1 : 2, q = (part == 0 ? s : (s - XS) % WS) * 64;
+        const float* src = part == 0 ? a.sx + m0 : (part == 1 || !a.bias ? a.sw : reinterpret_cast<const float*>(a.bias)) + n0;
+        const int dst = (part == 0 ? 0 : part == 1 ? P::BM * 4 : P::BM * 4 + P::BN * 4) + q * 4;
+        __builtin_amdgcn_global_load_lds((gptr_t)(src + q + lane), (lptr_t)(sc + dst), 4, 0, 0);
+      }
+    } else {
+      // columns in pairs (N is even); 320 columns are two and a half slices: they overlap
+      const int q = P::BN == 320 ? (wave % 3) * 96 : (wave & 1) * 128;
+      if (a.bias) __builtin_amdgcn_global_load_lds((gptr_t)(reinterpret_cast<const unsigned short*>(a.bias) + n0 + q + 2 * lane), (lptr_t)(sc + q * 2), 4, 0, 0);
+    }
+  };
+
+  // ---- fragments and products: rows 16 i + lr of the wavefront's 64, columns through j --------------------------
+  const int frag = (lq ^ ((lr >> 1) & 7)) * 16;
+  const int x_off[2] = {(wm * 64 + lr) * 128 + frag, (wm * 64 + lr) * 128 + (frag ^ 64)};
+  const int w_off[2] = {(P::BM + wn * 16 * TN + lr) * 128 + frag, (P::BM + wn * 16 * TN + lr) * 128 + (frag ^ 64)};
+  i32x4 fx[2][4], fw[2][H];
+  typename E::acc_t acc[4][TN];
+  auto read = [&](int turn, int stage) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (turn == 0)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fx[k][i] = *reinterpret_cast<const i32x4*>(lds + stage + x_off[k] + i * 2048);
+#pragma unroll
+      for (int j = 0; j < H; ++j) fw[k][j] = *reinterpret_cast<const i32x4*>(lds + stage + w_off[k] + (turn * H + j) * 2048);
+    }
+  };
+  auto multiply = [&](auto turn, auto zero) __attribute__((always_inline)) {
+    constexpr int T = decltype(turn)::value;
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int jj = 0; jj < H; ++jj) {
+          const int j = i & 1 ? H - 1 - jj : jj;  // one operand stays from each instruction to the next
+          const typename E::acc_t z = {};
+          acc[i][T * H + j] = E::mma(fx[k][i], fw[k][j], decltype(zero)::value && k == 0 ? z : acc[i][T * H + j]);
+        }
+    // (the products are pure values to the compiler; this pins them to their turn)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < H; ++j) asm volatile("" : "+v"(acc[i][T * H + j]));
+    __builtin_amdgcn_s_setprio(0);
+  };
+  auto meet = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // ---- output: rows wm * 64 + 16 i + 4 lq + r, quads and pair of columns from col0 on ------------------------------
+  typedef __attribute__((address_space(1))) unsigned char* gbyte_t;
+  const int col0 = wn * 16 * TN;
+  // address of row 16 i + r, group g of this lane in the tile at `tile` (uniform base, 32-bit lane offset; the pitch is
+  // made opaque at every use: as loop invariants the 16 row offsets would be kept in registers)
+  auto lane_again = [&]() __attribute__((always_inline)) {  // (made again at every use: kept, it would be spilled)
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    return l;
+  };
+  auto at = [&](const unsigned short* tile, int64_t ld, int i, int r, int g) __attribute__((always_inline)) {
+    const int l = lane_again();
+    unsigned int pitch = (unsigned int)ld * 2u;
+    asm volatile("" : "+s"(pitch));
+    const unsigned char* p = reinterpret_cast<const unsigned char*>(tile) + (unsigned int)(wm * 64 + 16 * i + r) * pitch + (col0 + 64 * g) * 2;
+    asm volatile("" : "+s"(p));
+    unsigned int lane_off = (unsigned int)(4 * (l >> 4)) * pitch + (g < P::NQ ? 8 : 4) * (l & 15);
+    asm volatile("" : "+v"(lane_off));
+    return (gbyte_t)(uintptr_t)p + lane_off;
+  };
+  typedef __attribute__((address_space(1))) u32x2* gquad_t;
+  typedef __attribute__((address_space(1))) unsigned int* gpair_t;
+  constexpr int EARLY = P::NQ * 4 + (P::PAIR ? 4 : 0);  // residual values of the first row group: requested in the last k tile
+  u32x2 res[RES ? 4 : 1][4][P::NQ];
+  unsigned int res_pair[RES && P::PAIR ? 4 : 1][4];
+  auto load_residual = [&](int i) __attribute__((always_inline)) {
+    const unsigned short* tile = a.residual + (int64_t)m0 * a.ld_res + n0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+      for (int g = 0; g < P::NQ; ++g) res[i][r][g] = *(gquad_t)at(tile, a.ld_res, i, r, g);
+      if constexpr (P::PAIR) res_pair[i][r] = *(gpair_t)at(tile, a.ld_res, i, r, P::NQ);
+    }
+  };
+  auto finish = [&](auto whole) __attribute__((always_inline)) {
+    constexpr bool FULL = decltype(whole)::value;
+    const int l = lane_again(), lr = l & 15, lq = l >> 4;
+    if constexpr (RES) {
+      load_residual(1);
+      load_residual(2);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // column scales and bias of the quads and the pair
+    float sw[P::NQ + 1][4], bias[P::NQ + 1][4];
+#pragma unroll
+    for (int g = 0; g < P::NQ + P::PAIR; ++g) {
+      const int n = g < P::NQ ? 4 : 2, col = col0 + 64 * g + n * lr;
+#pragma unroll
+      for (int e = 0; e < n; ++e) {
+        if constexpr (E::SCALED) {
+          sw[g][e] = reinterpret_cast<const float*>(sc + P::BM * 4 + col * 4)[e];
+          bias[g][e] = a.bias ? reinterpret_cast<const float*>(sc + P::BM * 4 + P::BN * 4 + col * 4)[e] : 0.f;
+        } else {
+          const unsigned int b = a.bias ? reinterpret_cast<const unsigned int*>(sc + col * 2)[e >> 1] : 0u;
+          bias[g][e] = e & 1 ? Out::hi(b) : Out::lo(b);
+        }
+      }
+    }
+    unsigned short* const tile = a.out + (int64_t)m0 * a.ldo + n0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (RES)
+        if (i == 1) load_residual(3);  // (three of the four row groups at a time: registers)
+      f32x4 sx;
+      if constexpr (E::SCALED) sx = *reinterpret_cast<const f32x4*>(sc + (wm * 64 + 16 * i + 4 * lq) * 4);
+      // two adjacent columns of row r, rounded; group g, elements e and e + 1, plus the residual pair v
+      auto two = [&](int r, int g, int e, unsigned int v) __attribute__((always_inline)) {
+        float y[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const auto s = acc[i][g < P::NQ ? P::quad(g, e + c) : P::pair(e + c)][r];
+          if constexpr (E::SCALED) {
+            // three separately rounded fp32 operations (no fused multiply-add)
+            float t = (float)s * sx[r];
+            t = t * sw[g][e + c];
+            y[c] = t + bias[g][e + c];
+          } else {
+            y[c] = s + bias[g][e + c];
+          }
+        }
+        unsigned int o = Out::pack2(y[0], y[1]);
+        if constexpr (EPI == PP_GELU) {
+          // activation of the rounded Linear output, as a separate GELU would see it
+          if constexpr (E::SCALED) o = Out::pack2(gelu_erf(Out::lo(o)), gelu_erf(Out::hi(o)));
+          else o = Out::pack2(gelu_value(Out::lo(o)), gelu_value(Out::hi(o)));
+        }
+        if constexpr (RES) o = Out::pack2(Out::lo(o) + Out::lo(v), Out::hi(o) + Out::hi(v));
+        return o;
+      };
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = wm * 64 + 16 * i + 4 * lq + r;
+#pragma unroll
+        for (int g = 0; g < P::NQ; ++g) {
+          const u32x2 v = RES ? res[RES ? i : 0][r][g] : u32x2{0u, 0u};
+          const u32x2 o = {two(r, g, 0, v[0]), two(r, g, 2, v[1])};
+          const gquad_t dst = (gquad_t)at(tile, a.ldo, i, r, g);
+          if (FULL || (row >= skip_m && col0 + 64 * g + 4 * lr >= skip_n)) {
+            if (NT) __builtin_nontemporal_store(o, dst);
+            else *dst = o;
+          }
+        }
+        if constexpr (P::PAIR) {
+          const unsigned int o = two(r, P::NQ, 0, RES ? res_pair[RES ? i : 0][r] : 0u);
+          const gpair_t dst = (gpair_t)at(tile, a.ldo, i, r, P::NQ);
+          if (FULL || (row >= skip_m && col0 + 64 * P::NQ + 2 * lr >= skip_n)) {
+            if (NT) __builtin_nontemporal_store(o, dst);
+            else *dst = o;
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // keep the conversion narrow
+      }
+    }
+  };
+
+  // ---- prologue: k tile 0, and of k tile 1 what the first turn of a k tile needs ---------------------------------
+  load_x(0);
+  load_w(0, 0);
+  load_w(1, 0);
+  next_ktile();
+  load_x(P::STAGE);
+  load_w(0, P::STAGE);
+  pp_wait<P::NLOADS>();  // the X rows and first columns of k tile 0
+  meet();
+  if (wn == 1) meet();  // from here on the upper half is one turn behind
+
+  int stage = 0;
+  // One k tile.  First turn: X rows and its columns are read; the second turn's columns of the k tile behind this one are
+  // requested (their place was read in the turn before this).  Second turn: its columns read; X rows and the first
+  // turn's columns of the k tile two behind requested.  Either wait leaves a k tile's worth of the youngest loads in flight: what
+  // the next turn of either half reads was requested before those.  EXTRA other operations (a whole tile's stores in front of
+  // its first k tile, residual values ahead of the last) are younger than what is waited for, if `extra` says that they were issued.
+  auto ktile = [&](auto zero, auto extra_n, bool extra) __attribute__((always_inline)) {
+    using T0 = std::integral_constant<int, 0>;
+    using T1 = std::integral_constant<int, 1>;
+    constexpr int EXTRA = decltype(extra_n)::value;
+    constexpr bool LAST = RES && !decltype(zero)::value && EXTRA > 0;
+    const int other = stage ^ P::STAGE;
+    read(0, stage);
+    load_w(1, other);
+    next_ktile();
+    if constexpr (LAST) load_residual(0);
+    if (EXTRA > 0 && extra) pp_wait<P::NLOADS + EXTRA>();
+    else pp_wait<P::NLOADS>();
+    meet();
+    multiply(T0{}, zero);
+    meet();
+    read(1, stage);
+    load_x(stage);
+    load_w(0, stage);
+    if constexpr (decltype(zero)::value) load_scales();
+    if (EXTRA > 0 && extra) pp_wait<P::NLOADS + EXTRA>();
+    else pp_wait<P::NLOADS>();
+    meet();
+    multiply(T1{}, zero);
+    meet();
+    stage = other;
+  };
+  using Yes = std::true_type;
+  using No = std::false_type;
+  bool stored = false;  // a whole tile's stores are on their way
+  for (int ti = 0; ti < nt; ++ti) {
+    ktile(Yes{}, std::integral_constant<int, P::NSTORES>{}, stored);
+    for (int k = 1; k < a.nk - (RES ? 1 : 0); ++k) ktile(No{}, std::integral_constant<int, 0>{}, false);
+    if constexpr (RES) ktile(No{}, std::integral_constant<int, EARLY>{}, true);
+    stored = skip_m == 0 && skip_n == 0;
+    if (stored) finish(Yes{});
+    else finish(No{});
+    if (ti + 1 < nt) tile_origin(ti + 1, m0, n0, skip_m, skip_n);
+  }
+  if (wn == 0) meet();
+  __builtin_amdgcn_s_waitcnt(0x0070);  // the last loads land before the LDS is given back
+}
+
+// ---- host side ---------------------------------------------------------------------------------------------------------
+// Time of a launch in units of one 16-column fragment for one k tile: rounds of the CUs, each as long as its k tiles and a start
+// and an end worth eight more of them, a tile two fragments more expensive than its columns (X rows, turns).  The width with the
+// least; `used`: the share of those CU-cycles that makes output.
+// us, 256 / 320 columns: int8 65536 x 1280 -> 5120 372 / 360, 4096 x 1280 -> 5120 (320 / 256 tiles) 33.0 / 28.1.  (192 columns, at an
+// equal number of columns per CU, lost: 65536 x 1280 -> 3840 284 / 305, 4096 x 1024 -> 3072 17.5 / 18.3.)
+struct PPChoice {
+  int tn;
+  int64_t rounds;
+  double used;
+};
+static inline PPChoice pp_choose(int64_t M, int N, int nk, bool wide) {
+  PPChoice best = {0, 0, 0.0};
+  double least = 0.0;
+  for (int tn = 8; tn <= (wide ? 10 : 8); tn += 2) {
+    if (N < 32 * tn || M < 256) continue;
+    const int64_t rounds = (((M + 255) / 256) * ((N + 32 * tn - 1) / (32 * tn)) + 255) / 256;
+    const double cost = (double)rounds * (tn + 2) * (nk + 8);
+    if (best.tn == 0 || cost < least) {
+      best = PPChoice{tn, rounds, (double)M * N / (256.0 * rounds * 256 * 32 * tn)};
+      least = cost;
+    }
+  }
+  return best;
+}
+
+// what the kernels take beside the shape rules of their callers: 32-bit offsets inside a tile
+static inline bool pp_addressable(const PPArgs& a) { return a.ldo < (1ll << 22) && a.ld_res < (1ll << 22) && a.nk >= 5; }
+
+static inline unsigned int pp_grid(const PPArgs& a) { return (unsigned int)min((int64_t)256, ((int64_t)a.tiles_m * a.tiles_n + 7) / 8 * 8); }
+
+}  // namespace samfast

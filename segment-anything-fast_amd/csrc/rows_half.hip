@@ -109,26 +109,6 @@ static int launch_layernorm(const RowsArgs& a, hipStream_t stream) {
   return go(integral_constant<int, 8>{}, E8{});
 }
 
-// GELU(x) = x * Phi(x) for values that arrive and leave in the half types.  h = Phi(-|x|) = 2^P(|x|), so that the negative
-// side keeps its relative accuracy; P is a degree-7 least-squares fit (Chebyshev nodes, reweighted towards the least
-// maximum) of log2 Phi(-z) on [0, 5.5] with P(0) = -1 exactly, within 5.4e-6 there.  Odd, with a negative leading coefficient,
-// it falls beyond that without a clamp, and h runs into zero as Phi does.  Of all fp16 values 45 are not rounded correctly (577
-// with erf in fp32, where 1 + erf cancels), of all bf16 values 89 (340).  The infinities are x * Phi's: +inf for the positive
-// one, NaN for the negative one, as x * 0.5 * (1 + erf) gives them.
-SF_DEVICE float gelu_value(float x) {
-  const float z = fabsf(x);
-  float p = -1.73511671e-06f;
-  p = fmaf(p, z, 5.9744074e-05f);
-  p = fmaf(p, z, -0.000916868041f);
-  p = fmaf(p, z, 0.00845726952f);
-  p = fmaf(p, z, -0.0538610406f);
-  p = fmaf(p, z, -0.458561927f);
-  p = fmaf(p, z, -1.15120995f);
-  p = fmaf(p, z, -1.f);
-  const float h = fast_exp2(p);
-  return x * (x > 0.f ? 1.f - h : h);
-}
-
 // 16 bytes per lane and step; a workgroup covers 8 KB with both its steps in flight, and there are as many as that takes
 // (4096 that loop: 303 us for 335 M values, this way 229).  4096 x 5120: 14.2 us, 5 x 4096 x 4096: 48.
 template <typename T>

@@ -31,6 +31,7 @@ enum Knob {
   KNOB_GEMM_PERSIST,      // SAMFAST_GEMM_PERSIST: 0 off, 1 where it pays, 2 wherever it is built
   KNOB_GEMM_PERSIST_SKEW, // SAMFAST_GEMM_PERSIST_SKEW: start delay of every second resident workgroup, 64 cycles per k tile
   KNOB_GEMM_PERSIST_PRIO, // SAMFAST_GEMM_PERSIST_PRIO: 0 = no wave priority changes in the persistent kernel
+  KNOB_GEMM_PINGPONG,     // SAMFAST_GEMM_PINGPONG: 256-row tiles by turns (gemm_pingpong.hpp), 0 off, 1 where it pays, 2 wherever built
   KNOB_GEMM_SPLITK,       // SAMFAST_GEMM_SPLITK: 0 off, 1 where it pays (launches that leave the GPU half empty; 2:4: one tile per CU), 2 wherever built
   KNOB_GEMM_ONCE,         // SAMFAST_GEMM_ONCE: 0 = off, 1 where it pays, rows * 16 + columns / 32 = that tile of the one-tile-per-CU kernel
   KNOB_LINEAR_SMALL,      // SAMFAST_GEMM_LINEAR_SMALL: 0 = whole Linears over few rows as two launches as well
@@ -110,6 +111,26 @@ SF_DEVICE float gelu_erf(float x) {
   p = fmaf(p, z, -9.99994340e-01f);
   const float h = __builtin_amdgcn_exp2f(p);
   return fmaf(-ax, h, __builtin_amdgcn_fmed3f(x, 0.0f, 3.4028234664e38f));
+}
+
+// GELU(x) = x * Phi(x) for values that arrive and leave in the half types.  h = Phi(-|x|) = 2^P(|x|), so that the negative
+// side keeps its relative accuracy; P is a degree-7 least-squares fit (Chebyshev nodes, reweighted towards the least
+// maximum) of log2 Phi(-z) on [0, 5.5] with P(0) = -1 exactly, within 5.4e-6 there.  Odd, with a negative leading coefficient,
+// it falls beyond that without a clamp, and h runs into zero as Phi does.  Of all fp16 values 45 are not rounded correctly (577
+// with erf in fp32, where 1 + erf cancels), of all bf16 values 89 (340).  The infinities are x * Phi's: +inf for the positive
+// one, NaN for the negative one, as x * 0.5 * (1 + erf) gives them.
+SF_DEVICE float gelu_value(float x) {
+  const float z = fabsf(x);
+  float p = -1.73511671e-06f;
+  p = fmaf(p, z, 5.9744074e-05f);
+  p = fmaf(p, z, -0.000916868041f);
+  p = fmaf(p, z, 0.00845726952f);
+  p = fmaf(p, z, -0.0538610406f);
+  p = fmaf(p, z, -0.458561927f);
+  p = fmaf(p, z, -1.15120995f);
+  p = fmaf(p, z, -1.f);
+  const float h = fast_exp2(p);
+  return x * (x > 0.f ? 1.f - h : h);
 }
 
 // Consecutive workgroup ids are dealt round-robin to the 8 XCDs, each with its

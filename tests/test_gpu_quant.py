@@ -637,6 +637,37 @@ def test_gemm_persistent_form_agrees(M, N, K, epi):
         assert torch.allclose(sample.float(), act, rtol=2 ** -7, atol=1e-6)  # one bf16 step
 
 
+@pytest.mark.parametrize("M,N,K,epi", [
+    # (chosen width) one tile and the shortest loop; ragged rows and columns, moved back tiles; lists of two tiles, whole and not
+    (256, 256, 640, 0), (256, 320, 768, 0), (300, 264, 1280, 2), (1000, 1288, 896, 0), (2433, 2056, 1536, 2),
+    (4096, 5120, 768, 0), (20480, 1024, 640, 2), (17000, 1288, 768, 2), (33000, 648, 768, 0),
+])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_gemm_by_turns_agrees(M, N, K, epi, layout):
+    """256 x {256, 320} tiles whose two halves take turns: the bits of the 64 x 128 tiles; residual also in place."""
+    from samfast_amd import _lib, ops
+    print(f"case gemm by turns M={M} N={N} K={K} epi={epi} layout={layout}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    xk = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8, device="cuda")
+    wk = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device="cuda")
+    sx, sw = (torch.rand(n, generator=g, device="cuda") * 1e-2 for n in (M, N))
+    bias = torch.randn(N, generator=g, device="cuda") if M % 2 == 0 else None
+    res = torch.randn((M, N), generator=g, device="cuda").to(torch.bfloat16) if epi == _lib.EPILOGUE_RESIDUAL else None
+    if layout == _lib.LAYOUT_KB64:
+        xk, wk = ops.to_kb64(xk), ops.to_kb64(wk)
+    run = lambda **kw: ops.gemm_i8_fused(xk, sx, wk, sw, bias, epi, layout=layout, **kw)
+    with _lib.knobs(SAMFAST_GEMM_TILE=64, SAMFAST_GEMM_SKINNY=0):
+        want = run(residual=res)
+    with _lib.knobs(SAMFAST_GEMM_PINGPONG=2, SAMFAST_GEMM_SKINNY=0):
+        for _ in range(3):
+            if res is None:
+                got = run()
+            else:
+                got = res.clone()
+                run(residual=got, out=got)
+            assert torch.equal(got, want)
+
+
 def test_gelu_epilogue_all_bf16_inputs():
     """Every bf16 bit pattern through the GELU epilogue.  Zero weights and bias[n] = the bf16
     value with bits n make column n of the Linear output that value, so one launch evaluates the
