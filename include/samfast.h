@@ -156,6 +156,14 @@ int samfast_quant_rowwise_i8(
     int64_t M, int K, int dtype, int layout, void* stream);
 
 /*
+ * The same of GELU(x), rounded to `dtype` as SAMFAST_EPILOGUE_GELU rounds it: the activation between an
+ * MLP's two Linears (modeling/common.py:26) and the second one's quantiser.
+ */
+int samfast_gelu_quant_rowwise_i8(
+    const void* x, int64_t ldx, int8_t* xq, float* sx,
+    int64_t M, int K, int dtype, int layout, void* stream);
+
+/*
  * acc[m, n] = sum_k xq[m, k] * wq[n, k], int32, exact.  xq (M, K) and wq (N, K)
  * int8 contiguous; acc (M, N) int32 contiguous.  The torch._int_mm step of the
  * quantised Linear (same call site), exposed so accumulators can be compared

@@ -446,9 +446,10 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
 
 // ---- host side ---------------------------------------------------------------------------------------------------------
 // Time of a launch in units of one 16-column fragment for one k tile: rounds of the CUs, each as long as its k tiles and a start
-// and an end worth eight more of them, a tile two fragments more expensive than its columns (X rows, turns).  The width with the
+// and an end worth eight more of them, a tile two or three and a half fragments more expensive than its columns.  The width with the
 // least; `used`: the share of those CU-cycles that makes output.
-// us, 256 / 320 columns: int8 65536 x 1280 -> 5120 372 / 360, 4096 x 1280 -> 5120 (320 / 256 tiles) 33.0 / 28.1.  (192 columns, at an
+// us, 256 / 320 columns: int8 inside the encoder 65536 x 1280 -> 3840 263 / 301; 4096 x 1280 -> 5120 (320 / 256 tiles) 33.0 / 28.1, 8192 x 1280 ->
+// 5120 (three / two rounds) 57.7 / 52.6, 20480 x 1280 -> 5120 (seven / five) 129.5 / 124.1.  (192 columns, at an
 // equal number of columns per CU, lost: 65536 x 1280 -> 3840 284 / 305, 4096 x 1024 -> 3072 17.5 / 18.3.)
 struct PPChoice {
   int tn;
@@ -461,7 +462,7 @@ static inline PPChoice pp_choose(int64_t M, int N, int nk, bool wide) {
   for (int tn = 8; tn <= (wide ? 10 : 8); tn += 2) {
     if (N < 32 * tn || M < 256) continue;
     const int64_t rounds = (((M + 255) / 256) * ((N + 32 * tn - 1) / (32 * tn)) + 255) / 256;
-    const double cost = (double)rounds * (tn + 2) * (nk + 8);
+    const double cost = (double)rounds * (tn == 8 ? 10.0 : 13.5) * (nk + 8);
     if (best.tn == 0 || cost < least) {
       best = PPChoice{tn, rounds, (double)M * N / (256.0 * rounds * 256 * 32 * tn)};
       least = cost;

@@ -20,7 +20,19 @@ namespace samfast {
 
 constexpr int kQuantWavesPerBlock = 4;
 
-template <int NCH, int EPC, bool LN>
+// GELU of values that lie in bf16, back in bf16, as the GEMM's epilogue makes it
+template <int NCH, typename in_t>
+SF_DEVICE void gelu_chunks(in_t (&xw)[NCH]) {
+#pragma unroll
+  for (int i = 0; i < NCH; ++i)
+#pragma unroll
+    for (int j = 0; j < (int)(sizeof(in_t) / 4); ++j) xw[i][j] = pack_bf16x2(gelu_erf(bf16_lo_to_f32(xw[i][j])), gelu_erf(bf16_hi_to_f32(xw[i][j])));
+}
+
+// ACT: the values are GELU's of what lies in memory.  Between an MLP's two Linears the activation runs here rather than in
+// the first one's epilogue: this kernel waits for memory and the vector ALU is free (65536 x 5120: 175 us without, 215 with it),
+// while a GEMM's wavefronts multiply nothing in the meantime (65536 x 1280 -> 5120: 465 us with GELU, 375 without).
+template <int NCH, int EPC, bool LN, bool ACT>
 __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowwise_bf16_kernel(QuantArgs a) {
   using RQ = RowQuantizer<NCH, EPC, LN>;
   const int lane = threadIdx.x & 63;
@@ -44,13 +56,14 @@ __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowwise_bf16_k
   // long rows (the 671 MB lin1 output at ViT-H batch 16) are read once and never again: streamed
   RQ::template load_row<(!LN && NCH >= 8)>(a.x + srow * a.ldx, nchunk, lane, xw);
   if (LN) RQ::load_affine(a.gamma, a.beta, nchunk, lane, gw, bw);
+  if (ACT) gelu_chunks(xw);
   RQ::finish_row(a, row, nchunk, lane, xw, gw, bw);
 }
 
 // WPR wavefronts share a row: fewer registers per lane for long rows (one wavefront with 4096 values needs 238: two
 // per SIMD and 2.2 TB/s at 65536 rows, 5.1 TB/s with four sharing), and for few rows more wavefronts with
 // fewer loads each to wait for.  The shares' maxima meet in LDS.  Bound: HBM, at the rate of a copy, from 8192 rows on.
-template <int NCH, int EPC, int WPR>
+template <int NCH, int EPC, int WPR, bool ACT>
 __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowshare_bf16_kernel(QuantArgs a) {
   constexpr int RPB = kQuantWavesPerBlock / WPR;  // rows per workgroup
   using RQ = RowQuantizer<NCH, EPC, false>;
@@ -73,6 +86,7 @@ __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowshare_bf16_
     xw[i] = z;
     if (live && c < nchunk) xw[i] = __builtin_nontemporal_load(reinterpret_cast<const in_t*>(a.x + row * a.ldx) + c);
   }
+  if (ACT) gelu_chunks(xw);
 #pragma unroll
   for (int i = 0; i < NCH; ++i)
 #pragma unroll
@@ -111,38 +125,38 @@ __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowshare_bf16_
   }
 }
 
-template <int NCH, int EPC, int WPR>
+template <int NCH, int EPC, int WPR, bool ACT>
 static int launch_rowshare(const QuantArgs& a, hipStream_t stream) {
   constexpr int RPB = kQuantWavesPerBlock / WPR;
-  hipLaunchKernelGGL((quant_rowshare_bf16_kernel<NCH, EPC, WPR>), dim3((unsigned int)((a.M + RPB - 1) / RPB)), dim3(64 * kQuantWavesPerBlock), 0, stream, a);
+  hipLaunchKernelGGL((quant_rowshare_bf16_kernel<NCH, EPC, WPR, ACT>), dim3((unsigned int)((a.M + RPB - 1) / RPB)), dim3(64 * kQuantWavesPerBlock), 0, stream, a);
   return check_launch("quant_rowshare_bf16_kernel");
 }
 
-template <int NCH, int EPC, bool LN>
+template <int NCH, int EPC, bool LN, bool ACT>
 static int launch_quant(const QuantArgs& a, hipStream_t stream) {
   const int64_t blocks = (a.M + kQuantWavesPerBlock - 1) / kQuantWavesPerBlock;
-  hipLaunchKernelGGL((quant_rowwise_bf16_kernel<NCH, EPC, LN>), dim3((unsigned int)blocks),
+  hipLaunchKernelGGL((quant_rowwise_bf16_kernel<NCH, EPC, LN, ACT>), dim3((unsigned int)blocks),
                      dim3(64 * kQuantWavesPerBlock), 0, stream, a);
   return check_launch("quant_rowwise_bf16_kernel");
 }
 
-template <int WPR>
+template <int WPR, bool ACT>
 static int launch_shares(const QuantArgs& a, hipStream_t s) {
   // shares that 4-element chunks divide among the 64 lanes exactly and 8-element chunks do not
-  if (a.K == 3 * 256 * WPR) return launch_rowshare<3, 4, WPR>(a, s);
-  if (a.K == 5 * 256 * WPR) return launch_rowshare<5, 4, WPR>(a, s);
+  if (a.K == 3 * 256 * WPR) return launch_rowshare<3, 4, WPR, ACT>(a, s);
+  if (a.K == 5 * 256 * WPR) return launch_rowshare<5, 4, WPR, ACT>(a, s);
   const int need = (a.K / 8 + 64 * WPR - 1) / (64 * WPR);
-  if (need <= 1) return launch_rowshare<1, 8, WPR>(a, s);
-  if (need <= 2) return launch_rowshare<2, 8, WPR>(a, s);
-  if (WPR == 2 || need <= 3) return launch_rowshare<3, 8, WPR>(a, s);
-  return launch_rowshare<4, 8, WPR>(a, s);
+  if (need <= 1) return launch_rowshare<1, 8, WPR, ACT>(a, s);
+  if (need <= 2) return launch_rowshare<2, 8, WPR, ACT>(a, s);
+  if (WPR == 2 || need <= 3) return launch_rowshare<3, 8, WPR, ACT>(a, s);
+  return launch_rowshare<4, 8, WPR, ACT>(a, s);
 }
 
-template <bool LN>
+template <bool LN, bool ACT>
 static int dispatch_quant(const QuantArgs& a, hipStream_t s) {
   // rows that 4-element chunks divide among the 64 lanes exactly and 8-element chunks do not
-  if (a.K == 768) return launch_quant<3, 4, LN>(a, s);
-  if (a.K == 1280) return launch_quant<5, 4, LN>(a, s);
+  if (a.K == 768) return launch_quant<3, 4, LN, ACT>(a, s);
+  if (a.K == 1280) return launch_quant<5, 4, LN, ACT>(a, s);
   const int need = (a.K / 8 + 63) / 64;
   if constexpr (!LN) {
     // Rows of more than 1024: wavefronts that share a row (us, one wavefront a row / two / four).
@@ -156,21 +170,21 @@ static int dispatch_quant(const QuantArgs& a, hipStream_t s) {
     //   1 KB apart, and the four stores meet: 4096 x 5120 15.2 / 16.6, 8192 x 5120 27.4 / 27.9.  Quarters that do not fill: 4001 x 4608
     //   14.1 / 16.2.  From 11 chunks per lane on one wavefront is short of registers: 8192 x 8192 46.3 / 43.5.  At 32768 rows one
     //   wavefront is ahead in either layout (K-block major 85.6 / 104.7 at K = 5120).
-    if (need == 3 && a.M <= 8192) return a.M <= 1024 ? launch_shares<4>(a, s) : launch_shares<2>(a, s);
-    if (need == 4 || need == 5) return a.M <= 1024 ? launch_shares<4>(a, s) : launch_shares<2>(a, s);
-    if (need >= 6 && need <= 8) return launch_shares<4>(a, s);
+    if (need == 3 && a.M <= 8192) return a.M <= 1024 ? launch_shares<4, ACT>(a, s) : launch_shares<2, ACT>(a, s);
+    if (need == 4 || need == 5) return a.M <= 1024 ? launch_shares<4, ACT>(a, s) : launch_shares<2, ACT>(a, s);
+    if (need >= 6 && need <= 8) return launch_shares<4, ACT>(a, s);
     const bool spread = !a.kb64 || a.M % 16 != 0;
-    if (need > 8 && (a.M <= 2048 || (a.M <= 16384 && (need > 12 || (a.K % 1024 == 0 && spread))))) return launch_shares<4>(a, s);
+    if (need > 8 && (a.M <= 2048 || (a.M <= 16384 && (need > 12 || (a.K % 1024 == 0 && spread))))) return launch_shares<4, ACT>(a, s);
   } else {
-    if (need == 4) return launch_quant<4, 8, LN>(a, s);
-    if (need > 4 && need <= 6) return launch_quant<6, 8, LN>(a, s);
-    if (need > 6 && need <= 8) return launch_quant<8, 8, LN>(a, s);
+    if (need == 4) return launch_quant<4, 8, LN, ACT>(a, s);
+    if (need > 4 && need <= 6) return launch_quant<6, 8, LN, ACT>(a, s);
+    if (need > 6 && need <= 8) return launch_quant<8, 8, LN, ACT>(a, s);
   }
-  if (need <= 2) return launch_quant<2, 8, LN>(a, s);
-  if (need <= 3) return launch_quant<3, 8, LN>(a, s);
-  if (need <= 10) return launch_quant<10, 8, LN>(a, s);
-  if (need <= 12) return launch_quant<12, 8, LN>(a, s);
-  return launch_quant<16, 8, LN>(a, s);
+  if (need <= 2) return launch_quant<2, 8, LN, ACT>(a, s);
+  if (need <= 3) return launch_quant<3, 8, LN, ACT>(a, s);
+  if (need <= 10) return launch_quant<10, 8, LN, ACT>(a, s);
+  if (need <= 12) return launch_quant<12, 8, LN, ACT>(a, s);
+  return launch_quant<16, 8, LN, ACT>(a, s);
 }
 
 static int check_common(const char* who, const void* x, int64_t ldx, const int8_t* xq, const float* sx,
@@ -192,17 +206,30 @@ static int check_common(const char* who, const void* x, int64_t ldx, const int8_
 
 }  // namespace samfast
 
-extern "C" int samfast_quant_rowwise_i8(const void* x, int64_t ldx, int8_t* xq, float* sx,
-                                        int64_t M, int K, int dtype, int layout, void* stream) {
-  using namespace samfast;
-  const int rc = check_common("quant_rowwise", x, ldx, xq, sx, M, K, dtype, layout);
+namespace samfast {
+
+template <bool ACT>
+static int quant_rowwise(const char* who, const void* x, int64_t ldx, int8_t* xq, float* sx, int64_t M, int K, int dtype, int layout, void* stream) {
+  const int rc = check_common(who, x, ldx, xq, sx, M, K, dtype, layout);
   if (rc != SAMFAST_OK) return rc;
   if (M == 0) return SAMFAST_OK;
   QuantArgs a = {};
   a.x = reinterpret_cast<const unsigned short*>(x);
   a.ldx = ldx; a.xq = xq; a.sx = sx; a.M = M; a.K = K;
   a.kb64 = layout == SAMFAST_LAYOUT_KB64;
-  return dispatch_quant<false>(a, reinterpret_cast<hipStream_t>(stream));
+  return dispatch_quant<false, ACT>(a, reinterpret_cast<hipStream_t>(stream));
+}
+
+}  // namespace samfast
+
+extern "C" int samfast_quant_rowwise_i8(const void* x, int64_t ldx, int8_t* xq, float* sx,
+                                        int64_t M, int K, int dtype, int layout, void* stream) {
+  return samfast::quant_rowwise<false>("quant_rowwise", x, ldx, xq, sx, M, K, dtype, layout, stream);
+}
+
+extern "C" int samfast_gelu_quant_rowwise_i8(const void* x, int64_t ldx, int8_t* xq, float* sx,
+                                             int64_t M, int K, int dtype, int layout, void* stream) {
+  return samfast::quant_rowwise<true>("gelu_quant_rowwise", x, ldx, xq, sx, M, K, dtype, layout, stream);
 }
 
 extern "C" int samfast_layernorm_quant_i8(const void* x, int64_t ldx, const void* gamma,
@@ -223,5 +250,5 @@ extern "C" int samfast_layernorm_quant_i8(const void* x, int64_t ldx, const void
   a.beta = reinterpret_cast<const unsigned short*>(beta);
   a.src_row = src_row; a.eps = eps; a.inv_K = 1.0f / (float)K;
   a.kb64 = layout == SAMFAST_LAYOUT_KB64;
-  return dispatch_quant<true>(a, reinterpret_cast<hipStream_t>(stream));
+  return dispatch_quant<true, false>(a, reinterpret_cast<hipStream_t>(stream));
 }

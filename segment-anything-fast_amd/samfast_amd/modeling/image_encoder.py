@@ -17,7 +17,7 @@ reference's own composition through flash_4._attention_rel_h_rel_w.
 When, in addition, the four Linears of a Block have been swapped for
 quant.Int8DynamicLinear, Block.forward (:167-183) runs with no eager glue as nine kernel
 launches: LayerNorm + quantise, qkv GEMM, attention, quantise, proj GEMM + residual, LayerNorm
-+ quantise, lin1 GEMM + GELU, quantise, lin2 GEMM + residual.  With SAMFAST_FUSED_QUANT=1 the
++ quantise, lin1 GEMM, GELU + quantise, lin2 GEMM + residual.  With SAMFAST_FUSED_QUANT=1 the
 three quantisers that follow a GEMM run inside that GEMM (proj + norm2 + quantise, lin1 +
 quantise, lin2 + the NEXT block's norm1 + quantise: five launches per block, same bits; slower
 at the measured shapes, hence not the default).  SAMFAST_FUSED_BLOCK=0 keeps the
@@ -208,6 +208,7 @@ class Block(nn.Module):
         `carry` = (xq, sx): this block's norm1 output, already quantised by the previous block's
         lin2 launch.  `next_norm` = (gamma, beta, eps) of the next block's norm1: lin2 then
         also returns that block's carry.  Returns (tokens (B, H, W, C), carry for the next block)."""
+        from .. import quant
         B, H, W, C = x.shape
         attn, mlp = self.attn, self.mlp
         nH = attn.num_heads
@@ -252,8 +253,14 @@ class Block(nn.Module):
             # proj + `shortcut + x`, then norm2 + lin1's quantiser on the rows just written
             tokens, hq, sh = attn.proj.linear_fused_quant(oq, so, _lib.EPILOGUE_RESIDUAL, residual=tokens,
                                                           layout=L, ln=norm2, out_layout=L)
-        # lin1 + GELU + lin2's quantiser, lin2 + `x + mlp(...)` (+ the next block's norm1 and quantiser)
-        _, gq, sg = mlp.lin1.linear_fused_quant(hq, sh, _lib.EPILOGUE_GELU, layout=L, out_layout=L)
+        # lin1, GELU, lin2's quantiser, lin2 + `x + mlp(...)` (+ the next block's norm1 and quantiser).  GELU runs in the
+        # quantiser, except where lin1 is short: there the product hides some of it and the quantiser nothing
+        # (lin1 + quantiser, us, GELU in lin1 / in the quantiser: 4096 x 1280 51.7 / 47.4, 65536 x 1280 661 / 601, 65536 x 768 335 /
+        # 313; but 20480 x 768 105 / 107, and a ViT-B image 1693 / 1746 for all twelve blocks)
+        if quant.FUSED_QUANT or (C < 1024 and tokens.shape[0] < 32768):
+            _, gq, sg = mlp.lin1.linear_fused_quant(hq, sh, _lib.EPILOGUE_GELU, layout=L, out_layout=L)
+        else:
+            gq, sg = ops.quant_rowwise(mlp.lin1.linear_fused(hq, sh, _lib.EPILOGUE_NONE, layout=L), layout=L, gelu=True)
         if next_norm is not None:
             tokens, nq, sn = mlp.lin2.linear_fused_quant(gq, sg, _lib.EPILOGUE_RESIDUAL, residual=tokens,
                                                          out=tokens, layout=L, ln=next_norm, out_layout=L)

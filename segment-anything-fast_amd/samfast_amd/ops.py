@@ -248,8 +248,9 @@ def _operand_shape(q: torch.Tensor, layout: int) -> Tuple[int, int]:
     return q.shape[0], q.shape[1]
 
 
-def quant_rowwise(x: torch.Tensor, layout: int = _lib.LAYOUT_ROWMAJOR) -> Tuple[torch.Tensor, torch.Tensor]:
-    """(M, K) bf16 (row stride free, K contiguous) -> (int8 codes in `layout`, fp32 scales (M,))."""
+def quant_rowwise(x: torch.Tensor, layout: int = _lib.LAYOUT_ROWMAJOR, gelu: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(M, K) bf16 (row stride free, K contiguous) -> (int8 codes in `layout`, fp32 scales (M,)); with `gelu`, of
+    GELU(x) as _lib.EPILOGUE_GELU rounds it."""
     _require_gpu(x)
     if x.dim() != 2 or x.stride(1) != 1:
         raise RuntimeError("samfast: quant_rowwise needs a 2-D tensor with contiguous rows")
@@ -257,12 +258,13 @@ def quant_rowwise(x: torch.Tensor, layout: int = _lib.LAYOUT_ROWMAJOR) -> Tuple[
     xq = _xq_empty(M, K, layout, x.device)
     sx = torch.empty((M,), dtype=torch.float32, device=x.device)
     lib = _lib.load()
+    call = lib.samfast_gelu_quant_rowwise_i8 if gelu else lib.samfast_quant_rowwise_i8
     code = _timed(
-        "quant_rowwise", 3.0 * M * K + 4.0 * M, "byte",
-        lambda: lib.samfast_quant_rowwise_i8(
+        "gelu_quant_rowwise" if gelu else "quant_rowwise", 3.0 * M * K + 4.0 * M, "byte",
+        lambda: call(
             x.data_ptr(), x.stride(0), xq.data_ptr(), sx.data_ptr(), M, K, _dtype_code(x),
             int(layout), _stream()))
-    _lib.check(code, "quant_rowwise_i8")
+    _lib.check(code, "gelu_quant_rowwise_i8" if gelu else "quant_rowwise_i8")
     return xq, sx
 
 

@@ -637,6 +637,27 @@ def test_gemm_persistent_form_agrees(M, N, K, epi):
         assert torch.allclose(sample.float(), act, rtol=2 ** -7, atol=1e-6)  # one bf16 step
 
 
+@pytest.mark.parametrize("M,K", [(1, 8), (5, 768), (7, 1280), (3, 1536), (1030, 2048), (9, 3072), (5, 4096), (2050, 5120), (16400, 4352), (2, 8192)])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_gelu_quantiser_is_the_epilogue_and_the_quantiser(M, K, layout):
+    """GELU inside the row quantiser: the codes and scales of the GEMM's GELU epilogue and the plain quantiser."""
+    from samfast_amd import _lib, ops
+    print(f"case gelu quantiser M={M} K={K} layout={layout}", flush=True)
+    if layout == _lib.LAYOUT_KB64 and K % 64 != 0:
+        pytest.skip("K-block major needs K % 64 == 0")
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    xq, wq = (torch.randint(-127, 128, (n, 64), generator=g, dtype=torch.int8, device="cuda") for n in (M, K))
+    sx, sw = (torch.rand(n, generator=g, device="cuda") * 1e-2 for n in (M, K))
+    pre, act = (ops.gemm_i8_fused(xq, sx, wq, sw, None, e) for e in (_lib.EPILOGUE_NONE, _lib.EPILOGUE_GELU))
+    pre[0, 1], act[0, 1] = float("nan"), float("nan")
+    codes, scales = ops.quant_rowwise(pre, layout, gelu=True)
+    want_codes, want_scales = ops.quant_rowwise(act, layout)
+    assert torch.isnan(scales[0]) and torch.equal(scales[1:], want_scales[1:])
+    rows = (ops.from_kb64(c) if layout == _lib.LAYOUT_KB64 else c for c in (codes, want_codes))
+    a, b = rows
+    assert torch.equal(a[1:], b[1:])
+
+
 @pytest.mark.parametrize("M,N,K,epi", [
     # (chosen width) one tile and the shortest loop; ragged rows and columns, moved back tiles; lists of two tiles, whole and not
     (256, 256, 640, 0), (256, 320, 768, 0), (300, 264, 1280, 2), (1000, 1288, 896, 0), (2433, 2056, 1536, 2),
