@@ -202,6 +202,19 @@ int samfast_linear_i8(
 int64_t samfast_linear_i8_workspace(int64_t M, int N, int K, int layout);
 
 /*
+ * A block's Linear in the half types: y = x w^T + bias (summed in fp32, rounded to `dtype`), then by `epilogue`
+ * (SAMFAST_EPILOGUE_*) nothing, exact-erf GELU of that, or + residual (rounded once more; residual and y may be the
+ * same buffer).  x (M, K) with row stride ldx elements, w (N, K) contiguous, bias (N) or NULL, y / residual row
+ * strides ldy / ld_res.  Row strides multiples of 8, pointers 16-byte aligned (the bias 4).  Only for shapes for which
+ * samfast_linear_half_pays returns 1; SAMFAST_E_UNSUPPORTED otherwise.  Stands for nn.Linear with
+ * the step behind it (modeling/image_encoder.py:228,251,180-181, modeling/common.py:26).
+ */
+int samfast_linear_half_pays(int64_t M, int N, int K, int epilogue);
+int samfast_linear_half(
+    const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t ldy,
+    int64_t M, int N, int K, int dtype, int epilogue, const void* residual, int64_t ld_res, void* stream);
+
+/*
  * LayerNorm over each row followed by the per-row int8 quantiser, with an optional
  * row gather: output row r is computed from source row src_row[r] of x (src_row NULL =
  * identity); src_row[r] < 0 yields an all-zero row with scale 1e-5/127.

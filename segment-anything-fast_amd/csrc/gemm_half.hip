@@ -1,0 +1,106 @@
+// bf16 / fp16 Linears of an encoder block: the turn-taking kernels of gemm_pingpong.hpp with the block's own epilogues, so that GELU and
+// the residual add cost no pass over memory of their own.
+#include "gemm_pingpong.hpp"
+
+namespace samfast {
+
+// The kernel for a product: columns / 32 of a tile; 8 and 10 the resident kernel, 3 to 5 the split one, 0 none (the library's product and
+// a pass of its own for GELU or residual are ahead).  The lines, by the rounds of the CUs and the share of their time that makes output
+// (us, library with its pass / here, residuals with the LayerNorm behind them):
+//   GELU: from half of the CUs on.  4096 x 768 -> 3072 33.8 / 28.7, 4096 x 1280 -> 5120 75.3 / 51.8, 20480 x 1024 -> 4096 188 / 165,
+//     65536 x 1280 -> 5120 863 / 768.
+//   plain: up to 8 rounds, 0.7.  4096 x 1024 -> 3072 27.7 / 26.2, 8192 x 768 -> 2304 35.8 / 30.7, 20480 x 1024 -> 3072 107 / 102, 32768 x 768 ->
+//     2304 119 / 104; but 4096 x 768 -> 2304 (0.56) 19.8 / 20.2, 65536 x 768 -> 2304 (9 rounds) 201 / 221.
+//   residual: 128-row tiles where the CUs hold them all at once.  4096 x 1280 -> 1280 31.1 / 23.6, 4096 x 5120 -> 1280 61.3 / 55.9.
+//     Else 256 x 256, on long loops within one round from 0.7 on (12288 x 5120 -> 1280 134 / 125; 0.5: 8192 x 4096 -> 1024 70 / 83, two
+//     rounds: 32768 x 4096 -> 1024 227 / 243), on short ones up to four rounds from 0.55 on (8192 x 1280 -> 1280 44.4 / 40.4, 32768 x
+//     1280 -> 1280 175 / 145; 0.5: 8192 x 1024 -> 1024 31.9 / 33.9, five rounds: 65536 x 1280 -> 1280 277 / 292).
+static int half_choose(int64_t M, int N, int K, int epi) {
+  const int force = knob_or(KNOB_GEMM_HALF, 1);
+  if (force <= 0 || K % 64 != 0 || K < 320 || M < 256 || N < 96) return 0;
+  if (force >= 3) return N >= 32 * force && (force != 10 || epi != PP_RESIDUAL) ? force : 0;
+  if (epi == PP_RESIDUAL)
+    for (int tn = 3; tn <= 5; ++tn) {
+      const int64_t tiles = ((M + 127) / 128) * ((N + 32 * tn - 1) / (32 * tn));
+      if (tiles <= 256 && tiles >= 128 && N >= 32 * tn) return tn;
+    }
+  const PPChoice c = pp_choose(M, N, K / 64, epi != PP_RESIDUAL);
+  if (c.tn == 0) return 0;
+  bool pays = c.used >= 0.5;
+  if (epi == PP_PLAIN) pays = c.rounds <= 8 && c.used >= 0.7;
+  if (epi == PP_RESIDUAL) pays = K >= 2048 ? c.rounds == 1 && c.used >= 0.7 : c.rounds <= 4 && c.used >= 0.75;
+  return pays ? c.tn : 0;
+}
+
+template <class E>
+static int half_launch(PPArgs a, int tn, int epi, hipStream_t stream) {
+  a.group_m = 4;
+  a.tiles_n = (a.N + 32 * tn - 1) / (32 * tn);
+  if (tn >= 8) {
+    a.tiles_m = (a.M + 255) / 256;
+    const dim3 grid(pp_grid(a));
+#define SF_PP(EPI, TN) hipLaunchKernelGGL((gemm_pingpong_kernel<E, EPI, TN, false>), grid, dim3(512), 0, stream, a)
+    if (epi == PP_GELU) { if (tn == 8) SF_PP(PP_GELU, 8); else SF_PP(PP_GELU, 10); }
+    else if (epi == PP_RESIDUAL) SF_PP(PP_RESIDUAL, 8);
+    else { if (tn == 8) SF_PP(PP_PLAIN, 8); else SF_PP(PP_PLAIN, 10); }
+#undef SF_PP
+    return check_launch("gemm_pingpong_kernel");
+  }
+  a.tiles_m = (a.M + 127) / 128;
+  const dim3 grid((unsigned int)(((int64_t)a.tiles_m * a.tiles_n + 7) / 8 * 8));
+#define SF_PP(EPI, TN) hipLaunchKernelGGL((gemm_pingpong_split_kernel<E, EPI, TN>), grid, dim3(512), 0, stream, a)
+#define SF_PP_ALL(TN) do { if (epi == PP_RESIDUAL) SF_PP(PP_RESIDUAL, TN); else if (epi == PP_GELU) SF_PP(PP_GELU, TN); else SF_PP(PP_PLAIN, TN); } while (0)
+  if (tn == 3) SF_PP_ALL(3);
+  else if (tn == 4) SF_PP_ALL(4);
+  else SF_PP_ALL(5);
+#undef SF_PP_ALL
+#undef SF_PP
+  return check_launch("gemm_pingpong_split_kernel");
+}
+
+}  // namespace samfast
+
+extern "C" int samfast_linear_half_pays(int64_t M, int N, int K, int epilogue) {
+  using namespace samfast;
+  const int epi = epilogue == SAMFAST_EPILOGUE_GELU ? PP_GELU : epilogue == SAMFAST_EPILOGUE_RESIDUAL ? PP_RESIDUAL : PP_PLAIN;
+  return N > 0 && N % 8 == 0 && half_choose(M, N, K, epi) != 0;
+}
+
+extern "C" int samfast_linear_half(const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t ldy,
+                                   int64_t M, int N, int K, int dtype, int epilogue, const void* residual, int64_t ld_res, void* stream) {
+  using namespace samfast;
+  if (dtype != SAMFAST_BF16 && dtype != SAMFAST_F16) SF_FAIL(SAMFAST_E_UNSUPPORTED, "linear_half: element type %d is neither SAMFAST_BF16 nor SAMFAST_F16", dtype);
+  int epi;
+  switch (epilogue) {
+    case SAMFAST_EPILOGUE_NONE: epi = PP_PLAIN; break;
+    case SAMFAST_EPILOGUE_GELU: epi = PP_GELU; break;
+    case SAMFAST_EPILOGUE_RESIDUAL: epi = PP_RESIDUAL; break;
+    default: SF_FAIL(SAMFAST_E_INVALID, "linear_half: unknown epilogue %d", epilogue);
+  }
+  SF_REQUIRE(M > 0 && N > 0 && K > 0 && N % 8 == 0, "linear_half: bad shape M=%lld N=%d K=%d (N must be a multiple of 8)", (long long)M, N, K);
+  SF_REQUIRE(x && w && y && (epi != PP_RESIDUAL || residual), "linear_half: null pointer");
+  SF_REQUIRE(aligned16(x) && aligned16(w) && aligned16(y) && aligned16(residual) && (reinterpret_cast<uintptr_t>(bias) & 3u) == 0,
+             "linear_half: operands must be 16-byte aligned, the bias 4-byte");
+  SF_REQUIRE(ldx >= K && ldx % 8 == 0 && ldy >= N && ldy % 8 == 0 && (epi != PP_RESIDUAL || (ld_res >= N && ld_res % 8 == 0)),
+             "linear_half: row strides must be multiples of 8 and hold a row");
+  SF_REQUIRE(M < (1ll << 31) - 512 && ldx < (1ll << 22) && K < (1 << 22), "linear_half: too large");
+  const int tn = half_choose(M, N, K, epi);
+  PPArgs a = {};
+  a.x = reinterpret_cast<const unsigned char*>(x);
+  a.w = reinterpret_cast<const unsigned char*>(w);
+  a.out = reinterpret_cast<unsigned short*>(y);
+  a.bias = bias;
+  a.residual = reinterpret_cast<const unsigned short*>(residual);
+  a.ldo = ldy;
+  a.ld_res = epi == PP_RESIDUAL ? ld_res : 0;
+  a.x_kstep = a.w_kstep = 64;
+  a.x_pitch = (unsigned int)(ldx * 2);
+  a.w_pitch = (unsigned int)(K * 2);
+  a.M = (int)M;
+  a.N = N;
+  a.nk = K / 64;
+  if (tn == 0 || !pp_addressable(a))
+    SF_FAIL(SAMFAST_E_UNSUPPORTED, "linear_half: no kernel for M=%lld N=%d K=%d (samfast_linear_half_pays)", (long long)M, N, K);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  return dtype == SAMFAST_F16 ? half_launch<PPF16>(a, tn, epi, s) : half_launch<PPBf16>(a, tn, epi, s);
+}

@@ -444,6 +444,276 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
   __builtin_amdgcn_s_waitcnt(0x0070);  // the last loads land before the LDS is given back
 }
 
+// ---- outputs the GPU holds once: 128-row tiles, K shared between the sides ------------------------------------------
+// An image's products onto few columns: 4096 rows and 768, 1024 or 1280 columns are exactly 256 tiles of 128 x {96, 128, 160}.  The
+// wavefronts 0-3 multiply the lower 64 bytes of every k tile, 4-7 the upper ones, by turns as above; each holds 64 rows and half
+// of the columns, and the two sides' sums meet in LDS at the end, where each side finishes half of the rows.  What bounds it is
+// the load path: 288 rows of 128 bytes for 640 cycles of products are 58 of the 64 bytes per clock that a CU takes in (bf16 4096 x 5120
+// -> 1280: 61 us, 41 without the products, 37 without the loads).  With the residual, us, library's product + residual in the
+// next LayerNorm / this + LayerNorm: 4096 x 5120 -> 1280 61.3 / 55.9, 4096 x 1280 -> 1280 31.1 / 23.6, 4096 x 768 -> 768 31.6 / 18.6.
+// (int8 keeps gemm_i8_once.hip: 4096 x 5120 -> 1280 30.0 there, 32.7 here.)
+template <int TN>
+struct PPSplitTile {
+  static_assert(TN >= 3 && TN <= 5, "widths built: 96, 128, 160");
+  static constexpr int BM = 128, BN = 32 * TN;
+  static constexpr int STAGE = (BM + BN) * 128;
+  static constexpr int NST = TN == 3 ? 5 : 4;
+  static constexpr int SCALES = BM * 4 + 2 * ((BN + 63) / 64 * 64) * 4;
+  static constexpr int LO = (TN + 1) / 2;             // loads of W per k tile for wavefronts 0-3 (two of X); 4-7: TN - LO
+  static constexpr int N0 = TN == 3 ? 2 : 4;          // adjacent columns of a lane; the others (TN - N0: none or one) follow 16 N0 further on
+  static_assert(NST * STAGE + SCALES <= 160 * 1024 && 16 * TN * 1024 <= NST * STAGE, "LDS of a CU");
+};
+
+template <class E, int EPI, int TN>
+__global__ __launch_bounds__(512, 2) void gemm_pingpong_split_kernel(PPArgs a) {
+  typedef typename E::Out Out;
+  using P = PPSplitTile<TN>;
+  constexpr bool RES = EPI == PP_RESIDUAL, ONE = TN > P::N0;
+  constexpr int NST = P::NST, N0 = P::N0, NP = N0 / 2;  // NP: pairs of a lane's adjacent columns
+  __shared__ __attribute__((aligned(16))) unsigned char lds[NST * P::STAGE + P::SCALES];
+  unsigned char* sc = lds + NST * P::STAGE;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int side = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+  const int lr = lane & 15, lq = lane >> 4;
+  const unsigned int total = (unsigned int)a.tiles_m * (unsigned int)a.tiles_n;
+  const unsigned int pid = xcd_contiguous_id(blockIdx.x, total);
+  if (pid >= total) return;  // uniform over the workgroup
+  const unsigned int per_group = (unsigned int)a.group_m * a.tiles_n;
+  const unsigned int first_m = (pid / per_group) * a.group_m;
+  const unsigned int gsz = min((unsigned int)a.tiles_m - first_m, (unsigned int)a.group_m);
+  const unsigned int in_group = pid % per_group;
+  int m0 = (int)(first_m + in_group % gsz) * P::BM, n0 = (int)(in_group / gsz) * P::BN;
+  // tiles at the edges are moved back inside (M >= 128, N >= BN), see above
+  const int skip_m = max(m0 + P::BM - a.M, 0), skip_n = max(n0 + P::BN - a.N, 0);
+  m0 -= skip_m;
+  n0 -= skip_n;
+
+  typedef __attribute__((address_space(1))) const void* gptr_t;
+  typedef __attribute__((address_space(3))) void* lptr_t;
+  typedef __attribute__((address_space(1))) unsigned char* gbyte_t;
+  typedef __attribute__((address_space(1))) unsigned int* gword_t;
+
+  // ---- output geometry: rows wm * 64 + 32 side + 16 i + 4 lq + r; the lane's adjacent columns, and of the column behind them
+  // the pair (even, odd) of row r that even lanes store, of row r + 1 that odd ones do
+  const int col0 = wn * 16 * TN + N0 * lr, col1 = wn * 16 * TN + 16 * N0 + (lr & ~1), row0 = wm * 64 + 32 * side + 4 * lq;
+  auto at = [&](const unsigned short* p, int64_t ld, int i, int r, bool one) __attribute__((always_inline)) {
+    const int row = row0 + 16 * i + r + (one ? lr & 1 : 0);
+    return (gbyte_t)(uintptr_t)(p + (int64_t)m0 * ld + n0) + (unsigned int)((row * (int)ld + (one ? col1 : col0)) * 2);
+  };
+  unsigned int res[RES ? 2 : 1][4][NP], res_one[RES && ONE ? 2 : 1][2];
+  if constexpr (RES) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if constexpr (NP == 2) {
+          const u32x2 v = *(__attribute__((address_space(1))) u32x2*)at(a.residual, a.ld_res, i, r, false);
+          res[i][r][0] = v[0];
+          res[i][r][NP - 1] = v[1];
+        } else {
+          res[i][r][0] = *(gword_t)at(a.residual, a.ld_res, i, r, false);
+        }
+      }
+      if constexpr (ONE) {
+        res_one[i][0] = *(gword_t)at(a.residual, a.ld_res, i, 0, true);
+        res_one[i][1] = *(gword_t)at(a.residual, a.ld_res, i, 2, true);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // the oldest operations in flight: no threshold below counts them
+  }
+
+  // ---- scales and bias, 64 lanes of 4 bytes an instruction -----------------------------------------------------------
+  if constexpr (E::SCALED) {
+    constexpr int XS = P::BM / 64, WS = (P::BN + 63) / 64, SLICES = XS + 2 * WS;
+    static_assert(SLICES <= 8, "one slice per wavefront");
+    const int s = wave % SLICES, part = s < XS ? 0 : s < XS + WS ? 1 : 2, q = (part == 0 ? s : (s - XS) % WS) * 64;
+    const float* src = part == 0 ? a.sx + m0 : (part == 1 || !a.bias ? a.sw : reinterpret_cast<const float*>(a.bias)) + n0;
+    const int limit = part == 0 ? P::BM - 1 : P::BN - 1;
+    const int dst = (part == 0 ? 0 : P::BM * 4 + (part - 1) * WS * 256) + q * 4;
+    __builtin_amdgcn_global_load_lds((gptr_t)(src + min(q + lane, limit)), (lptr_t)(sc + dst), 4, 0, 0);
+  } else if (a.bias) {
+    // columns in pairs (N is even)
+    const int q = (wave & 1) * 128;
+    __builtin_amdgcn_global_load_lds((gptr_t)(reinterpret_cast<const unsigned short*>(a.bias) + n0 + min(q + 2 * lane, P::BN - 2)), (lptr_t)(sc + q * 2), 4, 0, 0);
+  }
+
+  // ---- tile loads: eights of rows as above.  Every wavefront two of X; of W 0-3 take LO each, 4-7 the others ----------
+  unsigned int off_x, off_w[P::LO];
+  int at_w[P::LO];
+  const int nw = side == 0 ? P::LO : TN - P::LO;
+  {
+    const int r = wave * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+    off_x = (unsigned int)r * a.x_pitch + (unsigned int)((c >> 2) * a.x_kstep) + (c & 3) * 16;
+#pragma unroll
+    for (int i = 0; i < P::LO; ++i) {
+      // LDS row at_w: half by half, fragment by fragment; fragment j of a lane row is column N0 lr + j, or 16 N0 + lr
+      at_w[i] = min(side == 0 ? (wave & 3) * P::LO + i : 4 * P::LO + (wave & 3) * (TN - P::LO) + i, 4 * TN - 1) * 8;
+      const int in = at_w[i] % (16 * TN), j = in / 16, rr = in % 16 + (lane >> 3), cw = (lane & 7) ^ ((rr >> 1) & 7);
+      const int col = at_w[i] / (16 * TN) * 16 * TN + (j < N0 ? N0 * rr + j : 16 * N0 + rr);
+      off_w[i] = (unsigned int)col * a.w_pitch + (unsigned int)((cw >> 2) * a.w_kstep) + (cw & 3) * 16;
+    }
+  }
+  const unsigned char* xk = a.x + (int64_t)m0 * a.x_pitch;
+  const unsigned char* wk = a.w + (int64_t)n0 * a.w_pitch;
+  auto load = [&](const unsigned char* base, unsigned int o, int row, int stage) __attribute__((always_inline)) {
+    asm volatile("" : "+s"(base));
+    asm volatile("" : "+v"(o));
+    __builtin_amdgcn_global_load_lds((gptr_t)(base + o), (lptr_t)(lds + stage + row * 128), 16, 0, 0);
+  };
+  auto fill = [&](int stage) __attribute__((always_inline)) {
+    load(xk, off_x, wave * 8, stage);
+    load(xk + (int64_t)64 * a.x_pitch, off_x, (wave + 8) * 8, stage);
+#pragma unroll
+    for (int i = 0; i < P::LO; ++i)
+      if (i < nw) load(wk, off_w[i], P::BM + at_w[i], stage);
+    xk += 2 * a.x_kstep;
+    wk += 2 * a.w_kstep;
+  };
+  // at most `tiles` k tiles of this wavefront's loads still in flight; LDS reads done
+  auto arrive = [&](auto tiles) __attribute__((always_inline)) {
+    constexpr int T = decltype(tiles)::value;
+    if (P::LO == TN - P::LO || side == 0) pp_wait<T * (2 + P::LO)>();
+    else pp_wait<T * (2 + TN - P::LO)>();
+  };
+  auto meet = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  const int frag = ((lq + 4 * side) ^ ((lr >> 1) & 7)) * 16;
+  const int x_off = (wm * 64 + lr) * 128 + frag, w_off = (P::BM + wn * 16 * TN + lr) * 128 + frag;
+  typename E::acc_t acc[4][TN];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = typename E::acc_t{};
+  const int nk = a.nk;  // >= NST
+#pragma unroll
+  for (int p = 0; p < NST - 1; ++p) fill(p * P::STAGE);
+  arrive(std::integral_constant<int, NST - 2>{});
+  meet();
+  if (side == 1) meet();  // one turn behind
+  // k tile t: fragments read, k tile t + NST - 1 requested into the stage that both sides have left, t + 1 awaited; then the products
+  auto ktile = [&](int t, int rd, int wr, bool steady) __attribute__((always_inline)) {
+    i32x4 fx[4], fw[TN];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) fx[i] = *reinterpret_cast<const i32x4*>(lds + rd + x_off + i * 2048);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) fw[j] = *reinterpret_cast<const i32x4*>(lds + rd + w_off + j * 2048);
+    if (steady) {
+      fill(wr);
+      arrive(std::integral_constant<int, NST - 2>{});
+    } else {
+      pp_wait<0>();
+    }
+    meet();
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int jj = 0; jj < TN; ++jj) {
+        const int j = i & 1 ? TN - 1 - jj : jj;
+        acc[i][j] = E::mma(fx[i], fw[j], acc[i][j]);
+      }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(acc[i][j]));
+    __builtin_amdgcn_s_setprio(0);
+    meet();
+  };
+  auto up = [&](int s) __attribute__((always_inline)) { return s == (NST - 1) * P::STAGE ? 0 : s + P::STAGE; };
+  int rd = 0, wr = (NST - 1) * P::STAGE;
+  for (int t = 0; t < nk; ++t) {
+    ktile(t, rd, wr, t + NST - 1 < nk);
+    rd = up(rd);
+    wr = up(wr);
+  }
+  if (side == 0) meet();
+  meet();  // nobody reads operand stages any more
+
+  // ---- the sides' sums meet: side 0 finishes row groups 0 and 1, side 1 the other two -----------------------------------
+  typedef typename E::acc_t acc_t;
+  acc_t* red = reinterpret_cast<acc_t*>(lds) + (wave & 3) * 2 * TN * 64 + lane;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const acc_t upper = acc[2 + i][j], lower = acc[i][j];  // (values: a choice between places would put the sums into memory)
+      acc[i][j] = side == 0 ? lower : upper;
+      red[side * 8 * TN * 64 + (i * TN + j) * 64] = side == 0 ? upper : lower;
+    }
+  pp_wait<0>();
+  meet();
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] += red[(1 - side) * 8 * TN * 64 + (i * TN + j) * 64];
+
+  // ---- output ----------------------------------------------------------------------------------------------------------
+  const bool full = skip_m == 0 && skip_n == 0;
+  constexpr int WPAD = (P::BN + 63) / 64 * 64;
+  float sw[TN], bias[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int col = j < N0 ? col0 + j : wn * 16 * TN + 16 * N0 + lr;
+    if constexpr (E::SCALED) {
+      sw[j] = reinterpret_cast<const float*>(sc + P::BM * 4)[col];
+      bias[j] = a.bias ? reinterpret_cast<const float*>(sc + P::BM * 4)[WPAD + col] : 0.f;
+    } else {
+      bias[j] = a.bias ? Out::lo((unsigned int)reinterpret_cast<const unsigned short*>(sc)[col]) : 0.f;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    f32x4 sx;
+    if constexpr (E::SCALED) sx = *reinterpret_cast<const f32x4*>(sc + (row0 + 16 * i) * 4);
+    auto value = [&](int j, int r) __attribute__((always_inline)) {
+      if constexpr (E::SCALED) {
+        // three separately rounded fp32 operations (no fused multiply-add)
+        float t = (float)acc[i][j][r] * sx[r];
+        t = t * sw[j];
+        return t + bias[j];
+      } else {
+        return acc[i][j][r] + bias[j];
+      }
+    };
+    auto last_step = [&](unsigned int o, unsigned int v) __attribute__((always_inline)) {
+      if constexpr (EPI == PP_GELU) {
+        if constexpr (E::SCALED) o = Out::pack2(gelu_erf(Out::lo(o)), gelu_erf(Out::hi(o)));
+        else o = Out::pack2(gelu_value(Out::lo(o)), gelu_value(Out::hi(o)));
+      }
+      if constexpr (RES) o = Out::pack2(Out::lo(o) + Out::lo(v), Out::hi(o) + Out::hi(v));
+      return o;
+    };
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      unsigned int o[NP];
+#pragma unroll
+      for (int p = 0; p < NP; ++p) o[p] = last_step(Out::pack2(value(2 * p, r), value(2 * p + 1, r)), RES ? res[RES ? i : 0][r][p] : 0u);
+      const gbyte_t dst = at(a.out, a.ldo, i, r, false);
+      if (full || (row0 + 16 * i + r >= skip_m && col0 >= skip_n)) {
+        if constexpr (NP == 2) *(__attribute__((address_space(1))) u32x2*)dst = u32x2{o[0], o[NP - 1]};
+        else *(gword_t)dst = o[0];
+      }
+    }
+    if constexpr (ONE) {
+#pragma unroll
+      for (int r = 0; r < 4; r += 2) {
+        // lanes 2 n and 2 n + 1 hold columns 2 n, 2 n + 1 of both rows: the even one collects row r, the odd one row r + 1
+        const float a0 = value(TN - 1, r), a1 = value(TN - 1, r + 1);
+        const float other = __shfl_xor(lr & 1 ? a0 : a1, 1, 64);
+        const unsigned int o = last_step(lr & 1 ? Out::pack2(other, a1) : Out::pack2(a0, other), RES ? res_one[RES ? i : 0][r >> 1] : 0u);
+        const int row = row0 + 16 * i + r + (lr & 1);
+        if (full || (row >= skip_m && col1 >= skip_n)) *(gword_t)at(a.out, a.ldo, i, r, true) = o;
+      }
+    }
+  }
+}
+
 // ---- host side ---------------------------------------------------------------------------------------------------------
 // Time of a launch in units of one 16-column fragment for one k tile: rounds of the CUs, each as long as its k tiles and a start
 // and an end worth eight more of them, a tile two or three and a half fragments more expensive than its columns.  The width with the

@@ -308,10 +308,11 @@ class Block(nn.Module):
                 and (ws == 0 or ws * ws <= 208))
 
     def _forward_half_fused(self, x: torch.Tensor, carry=None, next_norm=None):
-        """image_encoder.py:167-183 with half-type Linears: the four library products plus four
-        launches.  The attention kernel cuts the windows out of the image-ordered tokens, so the
-        products run on the image's tokens only (the zero-padded windows have a fifth more) and nothing
-        is partitioned, padded or copied; each residual add runs with the norm that follows it.
+        """image_encoder.py:167-183 with half-type Linears: four products, those that pay on this library's kernels with
+        GELU or the residual add in them (ops.linear_half), and two or three launches around them.  The
+        attention kernel cuts the windows out of the image-ordered tokens, so the products run on the image's tokens only
+        (the zero-padded windows have a fifth more) and nothing is partitioned, padded or copied; a residual
+        add that is in no product runs with the norm that follows it.
         `carry`: norm1's output, where the previous block has made it; `next_norm`: the next block's norm1.
         Returns (tokens, carry for the next block)."""
         B, H, W, C = x.shape
@@ -320,7 +321,8 @@ class Block(nn.Module):
         hd = C // nH
         tokens = x.contiguous().view(B * H * W, C)
         h = carry if carry is not None else ops.layernorm(tokens, self.norm1.weight, self.norm1.bias, self.norm1.eps)
-        qkv = attn.qkv(h).view(B, H * W, 3, nH, hd)
+        qkv = ops.linear_half(h, attn.qkv)
+        qkv = (attn.qkv(h) if qkv is None else qkv).view(B, H * W, 3, nH, hd)
         q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
         if ws > 0:
             # a zero-padded token's k and v rows: the qkv bias
@@ -329,12 +331,20 @@ class Block(nn.Module):
             o = ops.attn_relpos_windowed(q, k, v, attn.rel_pos_h, attn.rel_pos_w, pads[0], pads[1], (H, W), ws, attn.scale)
         else:
             o = ops.attn_relpos(q, k, v, attn.rel_pos_h, attn.rel_pos_w, (H, W), attn.scale).permute(0, 2, 1, 3)
-        o = attn.proj(o.reshape(B * H * W, C))
-        tokens, h = ops.layernorm(tokens, self.norm2.weight, self.norm2.bias, self.norm2.eps, add=o)
-        m = mlp.lin2(ops.gelu_(mlp.lin1(h)))
-        if next_norm is None:
-            return tokens.add_(m).view(B, H, W, C), None
-        tokens, h = ops.layernorm(tokens, next_norm.weight, next_norm.bias, next_norm.eps, add=m)
+        o = o.reshape(B * H * W, C)
+
+        def add(rows, linear, total, norm):
+            """(total + linear(rows), norm of that)"""
+            summed = ops.linear_half(rows, linear, _lib.EPILOGUE_RESIDUAL, residual=total)
+            if summed is None and norm is not None:
+                return ops.layernorm(total, norm.weight, norm.bias, norm.eps, add=linear(rows))
+            if summed is None:
+                return total + linear(rows), None
+            return summed, None if norm is None else ops.layernorm(summed, norm.weight, norm.bias, norm.eps)
+
+        tokens, h = add(o, attn.proj, tokens, self.norm2)
+        m = ops.linear_half(h, mlp.lin1, _lib.EPILOGUE_GELU)
+        tokens, h = add(ops.gelu_(mlp.lin1(h)) if m is None else m, mlp.lin2, tokens, next_norm)
         return tokens.view(B, H, W, C), h
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:

@@ -590,6 +590,34 @@ def layernorm(x: torch.Tensor, gamma: torch.Tensor, beta: torch.Tensor, eps: flo
     return out if add is None else (total, out)
 
 
+def linear_half(x: torch.Tensor, linear: torch.nn.Linear, epilogue: int = _lib.EPILOGUE_NONE,
+                residual: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """linear(x) on contiguous half-type rows with `epilogue` behind it (GELU, or + residual into `out`, which may be the
+    residual), on this library's kernel; None, and nothing done, where the shape or the weights as they lie
+    are left to the framework's product."""
+    w, b = linear.weight, linear.bias
+    M, K = x.shape
+    N = w.shape[0]
+    lib = _lib.load()
+    if not lib.samfast_linear_half_pays(M, N, K, int(epilogue)):
+        return None
+    for t in (w, b):
+        if t is not None and (type(t) not in (torch.nn.Parameter, torch.Tensor) or t.dtype != x.dtype or t.device != x.device
+                              or not t.is_contiguous() or t.data_ptr() % 16 != 0):
+            return None
+    if not x.is_contiguous() or x.data_ptr() % 16 != 0 or x.device.index != torch.cuda.current_device():
+        return None
+    if out is None:
+        out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    code = _timed(
+        "linear_half", 2.0 * M * N * K, "flop",
+        lambda: lib.samfast_linear_half(
+            x.data_ptr(), K, w.data_ptr(), b.data_ptr() if b is not None else None, out.data_ptr(), N, M, N, K,
+            _dtype_code(x), int(epilogue), residual.data_ptr() if residual is not None else None, N, _stream()))
+    _lib.check(code, "linear_half")
+    return out
+
+
 def gelu_(x: torch.Tensor) -> torch.Tensor:
     """Exact-erf GELU of a contiguous half-type tensor, in place."""
     _require_gpu(x)

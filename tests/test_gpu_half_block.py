@@ -26,6 +26,54 @@ def test_add_layernorm_and_gelu_rows(M, K, dtype):
     assert ((got - ref).abs() <= eps * ref.abs() + 1e-6).all()
 
 
+@pytest.mark.parametrize("M,N,K,epi,tile", [
+    # columns / 32 of the tile (8, 10: resident, 3-5: K shared by the sides); whole and ragged edges, the shortest loop, several rounds
+    (256, 256, 320, 0, 8), (700, 520, 384, 1, 8), (4096, 3840, 320, 2, 8), (20000, 1032, 320, 0, 8),
+    (256, 320, 320, 1, 10), (900, 648, 448, 0, 10), (9000, 1288, 320, 1, 10),
+    (256, 96, 320, 2, 3), (700, 200, 832, 0, 3), (300, 128, 320, 1, 4), (4096, 1024, 1024, 2, 4), (256, 160, 320, 0, 5), (4000, 1288, 1280, 2, 5),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_half_linear_with_its_epilogues(M, N, K, epi, tile, dtype):
+    from samfast_amd import _lib, ops
+    print(f"case half linear M={M} N={N} K={K} epi={epi} tile={tile} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    linear = torch.nn.Linear(K, N, bias=M % 2 == 0, device="cuda", dtype=dtype).requires_grad_(False)
+    for p in linear.parameters():
+        p.normal_(0.0, 0.05, generator=g)
+    x = torch.randn((M, K), generator=g, device="cuda").to(dtype)
+    total = torch.randn((M, N), generator=g, device="cuda").to(dtype) if epi == _lib.EPILOGUE_RESIDUAL else None
+    with _lib.knobs(SAMFAST_GEMM_HALF=tile):
+        outs = [ops.linear_half(x, linear, epi, residual=total, out=None) for _ in range(3)]
+        if total is not None:
+            inplace = total.clone()
+            outs.append(ops.linear_half(x, linear, epi, residual=inplace, out=inplace))
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+    xd, wd, b = x.double(), linear.weight.double(), 0.0 if linear.bias is None else linear.bias.double()
+    ref = xd @ wd.t() + b
+    eps = torch.finfo(dtype).eps
+    # one rounding to the type, and fp32 sums: at most K rounded additions of partial sums below sum |x||w|
+    bound = 0.5 * eps * ref.abs() + K * 2.0 ** -24 * (xd.abs() @ wd.abs().t() + 1.0) + 2.0 ** -25
+    if epi == _lib.EPILOGUE_GELU:  # slope at most 1.13, its own rounding, the fit
+        ref = ref * 0.5 * torch.special.erfc(-ref * 0.5 ** 0.5)
+        bound = 1.13 * bound + 0.51 * eps * ref.abs() + 2.0 ** -24
+    elif total is not None:
+        ref = ref + total.double()
+        bound = bound * (1 + eps) + 0.5 * eps * ref.abs()
+    assert ((outs[0].double() - ref).abs() <= bound * 1.0001).all()
+
+
+def test_half_linear_leaves_what_it_does_not_take():
+    from samfast_amd import ops
+    linear = torch.nn.Linear(1024, 4096, device="cuda", dtype=torch.bfloat16).requires_grad_(False)
+    x = torch.zeros((4096, 1024), device="cuda", dtype=torch.bfloat16)
+    assert ops.linear_half(x, linear, 1) is not None
+    assert ops.linear_half(x[:100], linear, 1) is None                       # too few rows
+    assert ops.linear_half(_shifted(x), linear, 1) is None                   # off a 16-byte boundary
+    assert ops.linear_half(torch.zeros((4096, 2048), device="cuda", dtype=torch.bfloat16)[:, ::2], linear, 1) is None
+    linear.weight.data = linear.weight.data.t().contiguous().t()
+    assert ops.linear_half(x, linear, 1) is None
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,C,heads,window,bias", [(1, 768, 12, 14, True), (2, 320, 4, 0, True), (1, 320, 4, 11, False)])
 def test_half_blocks_equal_module_composition(B, C, heads, window, bias, dtype, monkeypatch):
