@@ -37,6 +37,9 @@ from .common import LayerNorm2d, MLPBlock
 
 KB64_OPERANDS = os.environ.get("SAMFAST_KB64", "1") != "0"
 WINDOWS_IN_PLACE = os.environ.get("SAMFAST_WINDOWS_IN_PLACE", "1") != "0"
+# The neck on the kernels here up to this many tokens; beyond, the library's larger convolution tiles are ahead (us, library / here,
+# width 1280: one image 107 / 45, four 198 / 102, eight 284 / 187, sixteen 261 / 365)
+NECK_TOKENS = 40960
 FUSED_BLOCK = bool(int(os.environ.get("SAMFAST_FUSED_BLOCK", 1)))
 
 
@@ -130,7 +133,36 @@ class ImageEncoderViT(nn.Module):
         if self.pos_embed is not None:
             x = x + self.pos_embed
         x = self.forward_blocks(x)
+        if self._neck_launchable(x):
+            conv1, norm1, conv3, norm2 = self.neck
+            rows = lambda norm: lambda y: ops.layernorm(y, norm.weight, norm.bias, norm.eps)
+            return rows(norm2)(ops.neck_convs(x, conv1.weight, rows(norm1), conv3.weight)).permute(0, 3, 1, 2)
         return self.neck(x.permute(0, 3, 1, 2))
+
+    def _neck_launchable(self, x: torch.Tensor) -> bool:
+        """Whether the neck is what the constructor builds and nothing else (no hook, subclass or other convolution), over few
+        enough tokens for the kernels here, with nobody watching."""
+        if not (FUSED_BLOCK and x.is_cuda and x.dim() == 4 and x.dtype in (torch.bfloat16, torch.float16) and not torch.is_grad_enabled()
+                and x.shape[0] * x.shape[1] * x.shape[2] <= NECK_TOKENS and ops.unwatched(x)):
+            return False
+        kinds = (nn.Conv2d, LayerNorm2d, nn.Conv2d, LayerNorm2d)
+        if type(self.neck) is not nn.Sequential or len(self.neck) != 4 or tuple(type(m) for m in self.neck) != kinds:
+            return False
+        if any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in (self.neck, *self.neck)):
+            return False
+        if nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks:
+            return False
+        conv1, norm1, conv3, norm2 = self.neck
+        for m, size in ((conv1, 1), (conv3, 3)):
+            if not (m.kernel_size == (size, size) and m.padding == (size // 2, size // 2) and m.stride == m.dilation == (1, 1)
+                    and m.groups == 1 and m.bias is None and m.padding_mode == "zeros"
+                    and m.in_channels % 64 == 0 and m.out_channels % 64 == 0 and m.in_channels <= 4096 and m.out_channels <= 4096):
+                return False
+        tensors = (x, conv1.weight, norm1.weight, norm1.bias, conv3.weight, norm2.weight, norm2.bias)
+        return (all(type(t) in (torch.Tensor, nn.Parameter) and t.dtype == x.dtype for t in tensors) and ops.rows_launchable(*tensors)
+                and conv1.in_channels == x.shape[3] and norm1.weight.numel() == conv1.out_channels == conv3.in_channels
+                and conv3.in_channels * 18 <= 96 * 1024 and norm2.weight.numel() == conv3.out_channels
+                and norm1.eps >= 0 and norm2.eps >= 0)
 
 
 class Block(nn.Module):

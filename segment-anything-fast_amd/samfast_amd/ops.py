@@ -618,6 +618,26 @@ def linear_half(x: torch.Tensor, linear: torch.nn.Linear, epilogue: int = _lib.E
     return out
 
 
+def neck_convs(x: torch.Tensor, w1: torch.Tensor, norm, w3: torch.Tensor) -> torch.Tensor:
+    """3x3 conv (w3, zero padding) of norm(1x1 conv (w1)) over contiguous channels-last half-type images (B, H, W, C);
+    `norm` maps the (B, H, W, C1) rows in between.  Returns (B, H, W, C2)."""
+    _require_gpu(x, w1, w3)
+    B, H, W, C = x.shape
+    mid, out = w1.shape[0], w3.shape[0]
+    lib = _lib.load()
+    y = torch.empty((B, H, W, mid), dtype=x.dtype, device=x.device)
+    taps = torch.empty((out, 9, mid), dtype=x.dtype, device=x.device)
+    code = _timed("neck_conv", 2.0 * B * H * W * mid * C, "flop", lambda: lib.samfast_neck_conv(
+        x.data_ptr(), w1.data_ptr(), y.data_ptr(), B, H, W, C, mid, 1, _dtype_code(x), w3.data_ptr(), taps.data_ptr(), out, mid, _stream()))
+    _lib.check(code, "neck_conv")
+    y = norm(y)
+    z = torch.empty((B, H, W, out), dtype=x.dtype, device=x.device)
+    code = _timed("neck_conv", 2.0 * B * H * W * out * 9 * mid, "flop", lambda: lib.samfast_neck_conv(
+        y.data_ptr(), taps.data_ptr(), z.data_ptr(), B, H, W, mid, out, 9, _dtype_code(x), None, None, 0, 0, _stream()))
+    _lib.check(code, "neck_conv")
+    return z
+
+
 def gelu_(x: torch.Tensor) -> torch.Tensor:
     """Exact-erf GELU of a contiguous half-type tensor, in place."""
     _require_gpu(x)

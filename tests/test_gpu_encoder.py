@@ -465,3 +465,50 @@ def test_chained_blocks_equal_separate_quantiser_launches(monkeypatch):
     assert torch.isfinite(chained.float()).all()
     assert torch.equal(chained.view(torch.int16), separate.view(torch.int16))
     assert torch.equal(chained.view(torch.int16), one_by_one.view(torch.int16))
+
+
+@pytest.mark.parametrize("B,H,W,C,mid,out", [(1, 64, 64, 128, 256, 256), (1, 5, 7, 64, 64, 128), (2, 9, 64, 320, 128, 64), (3, 1, 1, 64, 64, 64), (1, 66, 3, 192, 256, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_neck_convolutions_on_rows(B, H, W, C, mid, out, dtype):
+    """1 x 1 and 3 x 3 over channels-last images, ragged sizes, against the convolutions in 64 bits."""
+    from samfast_amd import ops
+    print(f"case neck B={B} {H}x{W} {C}->{mid}->{out} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(H * W + C)
+    x = torch.randn((B, H, W, C), generator=g).to(dtype)
+    w1 = (torch.randn((mid, C, 1, 1), generator=g) * 0.1).to(dtype)
+    w3 = (torch.randn((out, mid, 3, 3), generator=g) * 0.1).to(dtype)
+    between = []
+    def keep(y):
+        between.append(y.clone())
+        return y
+    got = [ops.neck_convs(x.cuda(), w1.cuda(), keep, w3.cuda()).cpu() for _ in range(2)]
+    assert torch.equal(got[0], got[1])
+    eps = torch.finfo(dtype).eps
+    y = between[0].cpu()
+    for val, src, w, pad in ((y, x, w1, 0), (got[0], y, w3, 1)):
+        conv = lambda a, b: torch.nn.functional.conv2d(a.double().permute(0, 3, 1, 2), b.double(), padding=pad).permute(0, 2, 3, 1)
+        ref = conv(src, w)
+        # one rounding to the type behind fp32 sums of K products
+        bound = 0.5 * eps * ref.abs() + w[0].numel() * 2.0 ** -24 * (conv(src.abs(), w.abs()) + 1e-3) + 2.0 ** -25
+        assert ((val.double() - ref).abs() <= bound * 1.0001).all()
+
+
+def test_neck_with_a_hook_or_another_convolution_is_called_as_modules():
+    from samfast_amd.modeling import ImageEncoderViT
+    torch.manual_seed(1)
+    enc = ImageEncoderViT(img_size=1024, embed_dim=128, depth=0, num_heads=2, use_rel_pos=True, window_size=14).cuda().to(torch.bfloat16).eval()
+    x = torch.randn((1, 64, 64, 128), device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        assert enc._neck_launchable(x)
+        calls = []
+        handle = enc.neck[2].register_forward_hook(lambda *a: calls.append(1))
+        assert not enc._neck_launchable(x)
+        enc.neck(x.permute(0, 3, 1, 2))
+        handle.remove()
+        assert calls and enc._neck_launchable(x)
+        enc.neck[2].padding_mode = "reflect"
+        assert not enc._neck_launchable(x)
+        enc.neck[2].padding_mode = "zeros"
+        enc.neck[2].weight.data = enc.neck[2].weight.data.to(memory_format=torch.channels_last)
+        assert not enc._neck_launchable(x)
+    assert not enc._neck_launchable(x)  # gradients are recorded
