@@ -225,6 +225,14 @@ int samfast_neck_conv(
     int dtype, const void* relay_src, void* relay_dst, int relay_rows, int relay_cin, void* stream);
 
 /*
+ * Sam.preprocess (modeling/sam.py:164-174) and the cast to the encoder's type: y (B, 3, S, S) of x (B, 3, h, w), uint8 or fp32,
+ * (x - mean) / std in fp32 with three means and deviations, zeros below and to the right.  S a multiple of 8.
+ */
+int samfast_preprocess(
+    const void* x, int x_is_u8, const float* mean, const float* std, void* y, int64_t B, int h, int w, int S,
+    int dtype, void* stream);
+
+/*
  * LayerNorm over each row followed by the per-row int8 quantiser, with an optional
  * row gather: output row r is computed from source row src_row[r] of x (src_row NULL =
  * identity); src_row[r] < 0 yields an all-zero row with scale 1e-5/127.

@@ -20,7 +20,7 @@ import torch.nn as nn
 
 class GraphedEncoder(nn.Module):
     """Wraps `encoder` (ImageEncoderViT or any module with a static forward) for inputs of one
-    fixed shape / dtype.  `forward(x)` copies x into the recorded input buffer, replays the
+    fixed shape / dtype.  `forward(x)` copies x into the recorded input buffer (unless x is that buffer), replays the
     graph and returns the recorded output buffer (valid until the next call)."""
 
     def __init__(self, encoder: nn.Module, example: torch.Tensor, warmup: int = 3) -> None:
@@ -46,7 +46,8 @@ class GraphedEncoder(nn.Module):
         if x.shape != self._in.shape or x.dtype != self._in.dtype:
             raise RuntimeError(f"samfast: GraphedEncoder was recorded for {tuple(self._in.shape)} "
                                f"{self._in.dtype}, got {tuple(x.shape)} {x.dtype}")
-        self._in.copy_(x)
+        if x is not self._in:
+            self._in.copy_(x)
         self._graph.replay()
         return self._out
 
@@ -112,6 +113,12 @@ class ReplayedEncoder(nn.Module):
         stride = patch.stride if patch is not None else (16, 16)
         rows = x.shape[0] * (x.shape[2] // stride[0]) * (x.shape[3] // stride[1])
         return 0 < rows <= self.max_rows and not torch.cuda.is_current_stream_capturing()
+
+    def input_buffer(self, shape, dtype, device) -> Optional[torch.Tensor]:
+        """The buffer that the recording for such an input reads, if there is one: an input written there on the current stream,
+        and then passed to forward, is not copied."""
+        graph = self._graphs.get((tuple(shape), dtype, device))
+        return None if graph is None else graph._in
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not self.replays(x):

@@ -638,6 +638,28 @@ def neck_convs(x: torch.Tensor, w1: torch.Tensor, norm, w3: torch.Tensor) -> tor
     return z
 
 
+def preprocess(x: torch.Tensor, mean: torch.Tensor, std: torch.Tensor, size: int, dtype: torch.dtype,
+               out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """(x - mean) / std, zero-padded to (B, 3, size, size), in the half type `dtype`, into `out` where given; None, and
+    nothing done, for what the kernel does not read."""
+    if not (x.is_cuda and x.dim() == 4 and x.shape[1] == 3 and x.dtype in (torch.uint8, torch.float32) and dtype in (torch.bfloat16, torch.float16)
+            and x.numel() > 0 and size % 8 == 0 and max(x.shape[2:]) <= size <= 65536 and x.is_contiguous()
+            and x.device.index == torch.cuda.current_device() and not torch.is_grad_enabled() and unwatched(x)):
+        return None
+    for t in (mean, std):
+        if t.dtype != torch.float32 or t.numel() != 3 or not t.is_contiguous() or t.device != x.device:
+            return None
+    shape = (x.shape[0], 3, size, size)
+    if out is None or out.shape != shape or out.dtype != dtype or out.device != x.device or not out.is_contiguous():
+        out = torch.empty(shape, dtype=dtype, device=x.device)
+    lib = _lib.load()
+    code = _timed("preprocess", x.numel() * x.element_size() + 2.0 * out.numel(), "byte", lambda: lib.samfast_preprocess(
+        x.data_ptr(), int(x.dtype == torch.uint8), mean.data_ptr(), std.data_ptr(), out.data_ptr(), x.shape[0], x.shape[2], x.shape[3], size,
+        _dtype_code(out), _stream()))
+    _lib.check(code, "preprocess")
+    return out
+
+
 def gelu_(x: torch.Tensor) -> torch.Tensor:
     """Exact-erf GELU of a contiguous half-type tensor, in place."""
     _require_gpu(x)

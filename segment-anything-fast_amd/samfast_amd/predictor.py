@@ -7,10 +7,12 @@ predictor runs unchanged.  Prompt decoding (`predict`, `predict_torch`) belongs
 to the mask decoder, which this package does not contain.
 """
 
-from typing import Tuple
+from typing import Optional, Tuple
 
 import torch
 
+from . import ops
+from .graphs import ReplayedEncoder
 from .modeling import Sam
 
 
@@ -41,10 +43,23 @@ class SamPredictor:
         self.reset_image()
         self.original_size = original_image_size
         self.input_size = tuple(transformed_image.shape[-2:])
-        x = self.model.preprocess(transformed_image)
-        dtype = next(self.model.image_encoder.parameters()).dtype
-        self.features = self.model.image_encoder(x.to(dtype))
+        encoder = self.model.image_encoder
+        dtype = next(encoder.parameters()).dtype
+        x = self._preprocessed(transformed_image, size, dtype)
+        self.features = encoder(self.model.preprocess(transformed_image).to(dtype) if x is None else x)
         self.is_image_set = True
+
+    def _preprocessed(self, image: torch.Tensor, size: int, dtype: torch.dtype) -> Optional[torch.Tensor]:
+        """The encoder's input in one launch, in the buffer that a recorded encoder reads where there is one; None where
+        the model's own preprocess has to run (a class of its own, a method put in its place, an input the kernel
+        does not read)."""
+        model = self.model
+        if type(model).preprocess is not Sam.preprocess or "preprocess" in model.__dict__:
+            return None
+        buffer, encoder = None, model.image_encoder
+        if type(encoder) is ReplayedEncoder and not encoder._forward_hooks and not encoder._forward_pre_hooks:
+            buffer = encoder.input_buffer((image.shape[0], 3, size, size), dtype, image.device)
+        return ops.preprocess(image, model.pixel_mean, model.pixel_std, size, dtype, buffer)
 
     def get_image_embedding(self) -> torch.Tensor:
         if not self.is_image_set:

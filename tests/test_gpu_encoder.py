@@ -512,3 +512,56 @@ def test_neck_with_a_hook_or_another_convolution_is_called_as_modules():
         enc.neck[2].weight.data = enc.neck[2].weight.data.to(memory_format=torch.channels_last)
         assert not enc._neck_launchable(x)
     assert not enc._neck_launchable(x)  # gradients are recorded
+
+
+@pytest.mark.parametrize("B,h,w,size", [(1, 64, 64, 64), (2, 64, 37, 64), (1, 5, 64, 64), (3, 1, 24, 24), (1, 767, 1024, 1024)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("raw", [torch.uint8, torch.float32])
+def test_preprocess_in_one_launch(B, h, w, size, dtype, raw):
+    """The bits of Sam.preprocess and the cast; strided and foreign inputs are left to it."""
+    from samfast_amd import ops
+    from samfast_amd.modeling import Sam
+    print(f"case preprocess B={B} {h}x{w} in {size} {dtype} {raw}", flush=True)
+    sam = Sam(torch.nn.Identity()).cuda()
+    sam.image_encoder.img_size = size
+    g = torch.Generator().manual_seed(h + w)
+    x = torch.randint(0, 256, (B, 3, h, w), generator=g).to(raw)
+    if raw is torch.float32:
+        x = x + torch.rand(x.shape, generator=g) * 300 - 150
+        x[0, 0, 0, 0], x[0, 1, 0, 0] = float("inf"), float("nan")
+    x = x.cuda()
+    with torch.no_grad():
+        want = sam.preprocess(x).to(dtype)
+        got = ops.preprocess(x, sam.pixel_mean, sam.pixel_std, size, dtype)
+        into = torch.full_like(want, 7.0)
+        assert ops.preprocess(x, sam.pixel_mean, sam.pixel_std, size, dtype, into) is into
+        for y in (got, into):
+            assert torch.equal(y.nan_to_num(nan=1.5), want.nan_to_num(nan=1.5)) and torch.equal(y.isnan(), want.isnan())
+        assert ops.preprocess(x.double(), sam.pixel_mean, sam.pixel_std, size, dtype) is None
+        assert ops.preprocess(x[..., :1], sam.pixel_mean, sam.pixel_std, size, dtype) is None or w == 1
+        assert ops.preprocess(x, sam.pixel_mean.to(dtype), sam.pixel_std, size, dtype) is None
+    assert ops.preprocess(x, sam.pixel_mean, sam.pixel_std, size, dtype) is None
+
+
+def test_predictor_keeps_a_model_s_own_preprocess_and_writes_where_the_recording_reads():
+    import samfast_amd
+    from samfast_amd.modeling import ImageEncoderViT, Sam
+    from samfast_amd.graphs import ReplayedEncoder
+    torch.manual_seed(2)
+    enc = ImageEncoderViT(img_size=1024, embed_dim=128, depth=2, num_heads=2, use_rel_pos=True, window_size=14, global_attn_indexes=(1,))
+    sam = Sam(ReplayedEncoder(enc.to(torch.bfloat16).eval())).cuda().eval()
+    pred = samfast_amd.SamPredictor(sam)
+    images = [torch.randint(0, 256, (1, 3, 700, 1024), device="cuda", dtype=torch.uint8) for _ in range(2)]
+    with torch.no_grad():
+        want = [sam.image_encoder._orig_mod(sam.preprocess(i).to(torch.bfloat16)) for i in images]
+    for turn in (0, 1, 0, 1):
+        pred.set_torch_image(images[turn], (700, 1024))
+        kept = pred.get_image_embedding()
+        pred.set_torch_image(images[1 - turn], (700, 1024))
+        assert torch.equal(kept, want[turn]) and torch.equal(pred.get_image_embedding(), want[1 - turn])
+    class Other(Sam):
+        def preprocess(self, x):
+            return super().preprocess(x * 0)
+    sam.__class__ = Other
+    pred.set_torch_image(images[0], (700, 1024))
+    assert not torch.equal(pred.get_image_embedding(), want[0])
