@@ -233,6 +233,19 @@ int samfast_preprocess(
     int dtype, void* stream);
 
 /*
+ * An int8 block's middle in one launch: tokens = proj(quantise(x)) + residual and xq, sx = quantise(norm2(tokens)), with the
+ * bits of samfast_quant_rowwise_i8, samfast_gemm_i8_fused (RESIDUAL) and samfast_layernorm_quant_i8
+ * (modeling/image_encoder.py:178-181, 251).  x (M, C) with row stride ldx, wq (C/64, C, 64) K-block major, residual and tokens
+ * (M, C) contiguous, possibly the same buffer, xq K-block major.  C is 768; samfast_proj_block_pays says at how many rows it is
+ * ahead of the three launches.
+ */
+int samfast_proj_block_pays(int64_t M, int C);
+int samfast_proj_block_i8(
+    const void* x, int64_t ldx, const int8_t* wq, const float* sw, const float* bias,
+    const void* residual, void* tokens, const void* gamma, const void* beta, float eps,
+    int8_t* xq, float* sx, int64_t M, int C, int dtype, void* stream);
+
+/*
  * LayerNorm over each row followed by the per-row int8 quantiser, with an optional
  * row gather: output row r is computed from source row src_row[r] of x (src_row NULL =
  * identity); src_row[r] < 0 yields an all-zero row with scale 1e-5/127.

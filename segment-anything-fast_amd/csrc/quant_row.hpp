@@ -176,6 +176,14 @@ struct RowQuantizer {
   // Everything after the loads: (LayerNorm,) absmax, scale, codes of output row `row`.
   static SF_DEVICE void finish_row(const QuantArgs& a, int64_t row, int nchunk, int lane,
                                    const in_t (&xw)[NCH], const in_t (&gw)[NCH], const in_t (&bw)[NCH]) {
+    const float scale = finish(a, nchunk, lane, xw, gw, bw, [&](int c, const unsigned int (&codes)[EPC / 4]) { store_chunk(a, row, c, codes); });
+    if (lane == 0) a.sx[row] = scale;
+  }
+
+  // The same with the chunks' codes handed to store(chunk, codes); returns the row's scale (in every lane).
+  template <typename Store>
+  static SF_DEVICE float finish(const QuantArgs& a, int nchunk, int lane, const in_t (&xw)[NCH], const in_t (&gw)[NCH], const in_t (&bw)[NCH],
+                                Store store) {
     // the row as floats, unpacked once
     float f[NCH][EPC];
 #pragma unroll
@@ -245,13 +253,13 @@ struct RowQuantizer {
       if (c < nchunk) {
         unsigned int codes[EPC / 4];
         saw_nan |= quantize_chunk<EPC>(f[i], scale, inv_scale, codes);
-        store_chunk(a, row, c, codes);
+        store(c, codes);
       }
     }
     // the maximum above drops NaNs (fmaxf returns its other operand); a row that holds one gets a
     // NaN scale, so that the Linear reading it returns NaN for this row as a float Linear would
     const bool row_nan = __any(saw_nan);
-    if (lane == 0) a.sx[row] = row_nan ? __uint_as_float(0x7fc00000u) : scale;
+    return row_nan ? __uint_as_float(0x7fc00000u) : scale;
   }
 };
 

@@ -33,6 +33,8 @@ _SIGNATURES = {
         _i32, [_ptr] * 6 + [_i32] * 5 + [_i64] * 18 + [_i32, _f32, _ptr]),
     "samfast_quant_rowwise_i8": (_i32, [_ptr, _i64, _ptr, _ptr, _i64, _i32, _i32, _i32, _ptr]),
     "samfast_neck_conv": (_i32, [_ptr, _ptr, _ptr, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _ptr, _ptr, _i32, _i32, _ptr]),
+    "samfast_proj_block_pays": (_i32, [_i64, _i32]),
+    "samfast_proj_block_i8": (_i32, [_ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _f32, _ptr, _ptr, _i64, _i32, _i32, _ptr]),
     "samfast_preprocess": (_i32, [_ptr, _i32, _ptr, _ptr, _ptr, _i64, _i32, _i32, _i32, _i32, _ptr]),
     "samfast_linear_half_pays": (_i32, [_i64, _i32, _i32, _i32]),
     "samfast_linear_half": (_i32, [_ptr, _i64, _ptr, _ptr, _ptr, _i64, _i64, _i32, _i32, _i32, _i32, _ptr, _i64, _ptr]),

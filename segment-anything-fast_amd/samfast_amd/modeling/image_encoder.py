@@ -281,10 +281,16 @@ class Block(nn.Module):
             else:
                 o = ops.attn_relpos(q, k, v, attn.rel_pos_h, attn.rel_pos_w, (H, W), attn.scale)
                 o = o.permute(0, 2, 1, 3).reshape(B * H * W, C)
-            oq, so = ops.quant_rowwise(o, layout=L)
-            # proj + `shortcut + x`, then norm2 + lin1's quantiser on the rows just written
-            tokens, hq, sh = attn.proj.linear_fused_quant(oq, so, _lib.EPILOGUE_RESIDUAL, residual=tokens,
-                                                          layout=L, ln=norm2, out_layout=L)
+            # proj's quantiser, proj + `shortcut + x`, norm2 + lin1's quantiser: one launch for few tokens
+            one = None
+            if type(attn.proj) is quant.Int8DynamicLinear and L == _lib.LAYOUT_KB64 and not quant.FUSED_QUANT:
+                one = ops.proj_block(o, attn.proj._weight_for(L), attn.proj.sw, attn.proj.bias_f32, tokens, norm2)
+            if one is not None:
+                tokens, hq, sh = one
+            else:
+                oq, so = ops.quant_rowwise(o, layout=L)
+                tokens, hq, sh = attn.proj.linear_fused_quant(oq, so, _lib.EPILOGUE_RESIDUAL, residual=tokens,
+                                                              layout=L, ln=norm2, out_layout=L)
         # lin1, GELU, lin2's quantiser, lin2 + `x + mlp(...)` (+ the next block's norm1 and quantiser).  GELU runs in the
         # quantiser, except where lin1 is short: there the product hides some of it and the quantiser nothing
         # (lin1 + quantiser, us, GELU in lin1 / in the quantiser: 4096 x 1280 51.7 / 47.4, 65536 x 1280 661 / 601, 65536 x 768 335 /

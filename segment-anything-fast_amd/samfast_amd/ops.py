@@ -551,6 +551,36 @@ def gemm_i8_sparse24_fused(xq: torch.Tensor, sx: torch.Tensor, wc: torch.Tensor,
     return out
 
 
+def proj_block(x: torch.Tensor, wq: torch.Tensor, sw: torch.Tensor, bias: Optional[torch.Tensor], residual: torch.Tensor,
+               ln: Tuple[torch.Tensor, torch.Tensor, float]) -> Optional[Tuple[torch.Tensor, torch.Tensor, torch.Tensor]]:
+    """(tokens, xq, sx): tokens = int8 Linear of x's rows + residual, and norm = ln's quantised rows of them, all K-block
+    major, in one launch with the bits of quant_rowwise, gemm_i8_fused and layernorm_quant; None, and nothing done,
+    where the three are ahead or the operands do not lie as the kernel reads them."""
+    M, C = x.shape
+    gamma, beta, eps = ln
+    lib = _lib.load()
+    if not lib.samfast_proj_block_pays(M, C) or not eps > 0 or x.dtype != torch.bfloat16:
+        return None
+    if residual.dtype != x.dtype or residual.shape != x.shape or wq.shape != (C // 64, C, 64):
+        return None
+    if x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0 or not rows_launchable(wq, sw, residual, gamma, beta):
+        return None
+    if gamma.dtype != x.dtype or beta.dtype != x.dtype or (bias is not None and not rows_launchable(bias)):
+        return None
+    _require_gpu(x, wq, sw, bias, residual, gamma, beta)
+    tokens = torch.empty_like(residual)
+    xq = _xq_empty(M, C, _lib.LAYOUT_KB64, x.device)
+    sx = torch.empty((M,), dtype=torch.float32, device=x.device)
+    code = _timed(
+        "proj_block", 2.0 * M * C * C, "op",
+        lambda: lib.samfast_proj_block_i8(
+            x.data_ptr(), x.stride(0), wq.data_ptr(), sw.data_ptr(), bias.data_ptr() if bias is not None else None,
+            residual.data_ptr(), tokens.data_ptr(), gamma.data_ptr(), beta.data_ptr(), float(eps), xq.data_ptr(), sx.data_ptr(),
+            M, C, _dtype_code(x), _stream()))
+    _lib.check(code, "proj_block_i8")
+    return tokens, xq, sx
+
+
 def unwatched(x: torch.Tensor) -> bool:
     """Whether launches that only the kernels see may stand for a module's tensor operations on x: no
     compiler, tracer, transform, mode or forward-mode tangent has to see them, and autocast, which would

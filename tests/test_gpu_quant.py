@@ -689,6 +689,44 @@ def test_gemm_by_turns_agrees(M, N, K, epi, layout):
             assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("M,bias,pitch", [(1, True, 768), (15, False, 776), (17, True, 2304), (2305, True, 768), (4096, False, 768), (4097, True, 1536),
+                                          (5121, True, 768), (8191, False, 768)])
+def test_proj_block_is_its_three_launches(M, bias, pitch):
+    """Quantiser, proj + residual, norm2 and the next quantiser in one launch (16 rows a workgroup, 32 from 4097 on): the bits of
+    the separate launches, also for rows with NaN, zeros and infinities and with the tokens written in place."""
+    from samfast_amd import _lib, ops
+    print(f"case proj block M={M} bias={bias} pitch={pitch}", flush=True)
+    C, L = 768, _lib.LAYOUT_KB64
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn((M, pitch), generator=g, device="cuda").to(torch.bfloat16)[:, :C]
+    x[M // 2], x[0, 5] = 0.0, float("nan")
+    res = torch.randn((M, C), generator=g, device="cuda").to(torch.bfloat16)
+    res[M - 1, C - 1] = float("inf")
+    w = ops.to_kb64(torch.randint(-127, 128, (C, C), generator=g, dtype=torch.int8, device="cuda"))
+    sw = torch.rand(C, generator=g, device="cuda") * 1e-3
+    b = torch.randn(C, generator=g, device="cuda") if bias else None
+    gamma, beta = (torch.randn(C, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    xq, sx = ops.quant_rowwise(x, layout=L)
+    want = ops.gemm_i8_fused(xq, sx, w, sw, b, _lib.EPILOGUE_RESIDUAL, residual=res, layout=L)
+    want_q, want_s = ops.layernorm_quant(want, gamma, beta, 1e-6, layout=L)
+    lib = _lib.load()
+    if lib.samfast_proj_block_pays(M, C):
+        tokens, hq, hs = ops.proj_block(x, w, sw, b, res, (gamma, beta, 1e-6))
+    else:
+        assert ops.proj_block(x, w, sw, b, res, (gamma, beta, 1e-6)) is None
+        tokens, hq, hs = res.clone(), torch.empty_like(want_q), torch.empty_like(want_s)
+        code = lib.samfast_proj_block_i8(
+            x.data_ptr(), pitch, w.data_ptr(), sw.data_ptr(), b.data_ptr() if bias else None, tokens.data_ptr(), tokens.data_ptr(),
+            gamma.data_ptr(), beta.data_ptr(), 1e-6, hq.data_ptr(), hs.data_ptr(), M, C, _lib.SAMFAST_BF16, torch.cuda.current_stream().cuda_stream)
+        _lib.check(code, "proj_block_i8")
+    finite = torch.ones(M, dtype=torch.bool, device="cuda")
+    finite[0] = finite[M - 1] = False  # (a NaN's payload and the codes beside a NaN scale are nobody's contract)
+    assert torch.isnan(tokens[0]).all() and torch.isnan(hs[0])
+    assert torch.equal(tokens[finite], want[finite]) and torch.equal(hs[finite], want_s[finite])
+    assert torch.equal(torch.isnan(hs), torch.isnan(want_s))
+    assert torch.equal(ops.from_kb64(hq)[finite], ops.from_kb64(want_q)[finite])
+
+
 def test_gelu_epilogue_all_bf16_inputs():
     """Every bf16 bit pattern through the GELU epilogue.  Zero weights and bias[n] = the bf16
     value with bits n make column n of the Linear output that value, so one launch evaluates the
