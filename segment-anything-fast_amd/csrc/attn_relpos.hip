@@ -406,7 +406,8 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void attn_global_ke
 }
 
 // =============================================================================
-// window kernel: gh <= 15, gw <= 16, N = gh*gw <= 208; one workgroup per (window, head)
+// window kernel: gh <= 15, gw <= 16, N = gh*gw <= 208; one workgroup per (window, head), or two
+// or three for those that are left over beside whole rounds of 256
 // =============================================================================
 // Eight wavefronts: all of them stage K / V, wavefront w then owns query tile w (32 queries;
 // 7 tiles for 196 tokens).  Registers are kept under 128 per lane (online softmax over the
@@ -460,8 +461,20 @@ __global__ __launch_bounds__(WindowCfg<HD>::THREADS, 2) void attn_window_kernel(
   if (tid < 2 * C::HOT_ENTRIES) *reinterpret_cast<u32x4*>(hot + tid * 16) = onehot_x8<T>(tid >> 1, tid & 1);
   // all heads of a window run on one XCD: their 2*HD-byte slices of a token share cache lines
   const unsigned int total = (unsigned int)((a.ws > 0 ? a.B * a.wins_x * a.wins_y : a.B) * a.nH);
-  const int bh = (int)xcd_contiguous_id(blockIdx.x, total);
-  if ((unsigned int)bh >= total) return;  // uniform over the workgroup
+  // every XCD has a contiguous range of the items with one workgroup (a.whole, a multiple of 8) and one of the others' parts
+  const unsigned int xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
+  const unsigned int whole_x = (unsigned int)a.whole >> 3;
+  unsigned int item = xcd * whole_x + slot;
+  int tile0 = 0, tiles = C::NT;
+  if (slot >= whole_x) {
+    const unsigned int per = ((total - (unsigned int)a.whole) * (unsigned int)a.parts + 7u) >> 3;
+    const unsigned int part = xcd * per + (slot - whole_x);
+    item = (unsigned int)a.whole + part / (unsigned int)a.parts;
+    if (slot - whole_x >= per || item >= total) return;  // uniform over the workgroup
+    tiles = a.part_tiles;
+    tile0 = (int)(part % (unsigned int)a.parts) * tiles;
+  }
+  const int bh = (int)item;
   const int bwin = bh / a.nH, h = bh % a.nH;
   // image-ordered mode: bwin = (image, window row, window column)
   int b = bwin, win_y0 = 0, win_x0 = 0;
@@ -493,8 +506,10 @@ __global__ __launch_bounds__(WindowCfg<HD>::THREADS, 2) void attn_window_kernel(
 
   const int ntq = (N + 31) / 32;
   const int nsteps = (N + 15) / 16;
-  const bool has_tile = wave < ntq;  // uniform per wavefront
-  const int qi = 32 * wave + lr;
+  // uniform per wavefront; tiles of padding tokens alone (a window over the image's lower edge) are left out
+  const int tile = tile0 + wave;
+  const bool has_tile = wave < tiles && tile < ntq && (a.ws <= 0 || win_y0 + div_gw(32 * tile) < a.img_h);
+  const int qi = 32 * tile + lr;
   const int qc = min(qi, N - 1);
 
   // ---- requests first: this wavefront's query rows, then the K / V staging loads ----------
@@ -826,9 +841,10 @@ __global__ __launch_bounds__(WindowCfg<HD>::THREADS, 2) void attn_window_kernel(
   {
     constexpr int PPT = HD / 8;  // 16-byte pieces per token
     unsigned short* obase = a.out + b * a.o_sb + h * a.o_sh;
-    for (int p = tid; p < N * PPT; p += C::THREADS) {
-      const int n = (p * (65536 / PPT + 1)) >> 16;  // p / PPT, exact for p < 4096
-      const int col = p - n * PPT;
+    const int n0 = 32 * tile0, rows = min(N - n0, 32 * tiles);
+    for (int p = tid; p < rows * PPT; p += C::THREADS) {
+      const int row = (p * (65536 / PPT + 1)) >> 16;  // p / PPT, exact for p < 4096
+      const int n = n0 + row, col = p - row * PPT;
       const int otok = tok_of(n);  // padding tokens produce no output
       if (otok >= 0) {
         const u32x4 o = *reinterpret_cast<const u32x4*>(kl + n * (C::KSTR * 2) + col * 16);
@@ -862,8 +878,21 @@ static int launch_hd(const AttnArgs& a, bool global_path, hipStream_t stream) {
     return check_launch("attn_global_kernel");
   }
   const int64_t wins = a.ws > 0 ? (int64_t)a.B * a.wins_x * a.wins_y : a.B;
-  const unsigned int grid = (unsigned int)(((wins * a.nH + 7) / 8) * 8);
-  hipLaunchKernelGGL((attn_window_kernel<T, HD, FUSED>), dim3(grid), dim3(WindowCfg<HD>::THREADS), 0, stream, a);
+  const int64_t total = wins * a.nH;
+  AttnArgs b = a;
+  // Whole rounds of 256 items get a workgroup each; what is left over is cut into halves or thirds, by query tiles, while that makes at most
+  // a workgroup more per CU: otherwise a few CUs run two workgroups side by side and the others wait for them (the
+  // staging is done again, by CUs that would idle).  us, before / whole / halves / thirds, windows of 14 x 14: 25 x 12 x 64 15.9 / 15.9 / 13.4 /
+  // 13.3, in an image 18.1 / 15.2 / 15.0 / 14.6, 5 x 12 x 64 9.4 / 9.4 / 8.0 / 7.9, 30 x 12 x 64 (104 left) 16.2 / 15.8 / 13.8 / 17.7, 2 images x 12 x
+  // 64 (88 left) 24.6 / 24.0 / 22.5 / 24.5, 2 images x 16 x 80 (32 left) 32.6 / 29.8 / 29.4 / 29.5; 25 x 16 x 80 (144 left) 19.0 / 18.7 / 21.5 / 20.8.
+  // (Before: contiguous eighths of all items, padding tiles computed as well.)
+  const int ntq = (a.N + 31) / 32, left = (int)(total % 256);
+  const int parts = left * 3 <= 256 ? 3 : left * 2 <= 256 ? 2 : 1;
+  b.whole = (int)(total - left);
+  b.part_tiles = (ntq + parts - 1) / parts;
+  b.parts = (ntq + b.part_tiles - 1) / b.part_tiles;
+  const unsigned int grid = (unsigned int)((b.whole + ((total - b.whole) * b.parts + 7) / 8 * 8));
+  hipLaunchKernelGGL((attn_window_kernel<T, HD, FUSED>), dim3(grid), dim3(WindowCfg<HD>::THREADS), 0, stream, b);
   return check_launch("attn_window_kernel");
 }
 

@@ -30,6 +30,7 @@ struct AttnArgs {
   const unsigned short* pad_v;
   int relh_x8;  // attn_global_bias.hip: rel_h rows can be read 16 bytes at a time
   int rel_x2;   // window kernel: rows of the caller's factors can be read 4 bytes at a time
+  int whole, parts, part_tiles;  // window kernel: items with a workgroup each; the others are `parts` workgroups of part_tiles query tiles
 };
 
 constexpr float kLog2e = 1.4426950408889634f;

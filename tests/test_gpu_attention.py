@@ -266,6 +266,35 @@ def test_global_kernel_wave_count_variants_agree(hd, gh):
     _check(outs["8"], ref, "8 wavefronts per workgroup")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("few,many,nH,gh,gw,hd", [(1, 42, 12, 14, 14, 64), (25, 42, 12, 14, 14, 64), (30, 42, 12, 14, 14, 64), (5, 12, 16, 13, 14, 80),
+                                                  (32, 31, 8, 14, 14, 64), (40, 63, 4, 5, 7, 80), (3, 63, 4, 4, 8, 64)])
+def test_windows_cut_into_parts_keep_their_bits(few, many, nH, gh, gw, hd, dtype):
+    """Windows beyond whole rounds of 256 workgroups are cut into halves or thirds by query tiles: the bits that they have in a batch
+    whose windows stay whole (42 x 12, 12 x 16, 31 x 8 and 63 x 4 leave more than 128 over, 32 x 8 none)."""
+    from samfast_amd import ops
+    print(f"case window parts few={few} many={many} nH={nH} grid={gh}x{gw} hd={hd} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(few * 100 + many)
+    B = max(few, many)
+    q, k, v = ((0.5 * torch.randn((B, nH, gh * gw, hd), generator=g, device="cuda")).to(dtype) for _ in range(3))
+    rh, rw = ((0.5 * torch.randn((B, nH, gh * gw, n), generator=g, device="cuda")).to(dtype) for n in (gh, gw))
+    a, b = (ops.attn_relpos_bias(q[:n], k[:n], v[:n], rh[:n], rw[:n]) for n in (few, many))
+    n = min(few, many)
+    assert torch.isfinite(a.float()).all() and torch.equal(a[:n], b[:n])
+
+
+@pytest.mark.parametrize("few,many,nH,H,W,hd", [(1, 4, 12, 64, 64, 64), (2, 4, 12, 64, 64, 64), (2, 5, 16, 64, 64, 80), (1, 9, 4, 30, 17, 64), (3, 7, 3, 15, 64, 80)])
+def test_image_windows_cut_into_parts_keep_their_bits(few, many, nH, H, W, hd):
+    """The same for windows cut out of images, whose tiles of padding tokens alone are left out."""
+    from samfast_amd import ops
+    print(f"case image window parts few={few} many={many} nH={nH} {H}x{W} hd={hd}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(few * 100 + many)
+    rnd = lambda *shape: (0.5 * torch.randn(shape, generator=g, device="cuda")).to(torch.bfloat16)
+    qkv, pk, pv, th, tw = rnd(many, H * W, 3, nH, hd).permute(2, 0, 3, 1, 4), rnd(nH, hd), rnd(nH, hd), rnd(27, hd), rnd(27, hd)
+    a, b = (ops.attn_relpos_windowed(*(t[:n] for t in qkv), th, tw, pk, pv, (H, W), 14, hd ** -0.5) for n in (few, many))
+    assert torch.isfinite(a.float()).all() and torch.equal(a, b[:few])
+
+
 @pytest.mark.parametrize("batch", [1, 8])
 @pytest.mark.parametrize("head,hidden_dim", [(16, 80), (12, 64)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
