@@ -4,37 +4,48 @@
 
 namespace samfast {
 
-// The kernel for a product: columns / 32 of a tile; 8 and 10 the resident kernel, 3 to 5 the split one, 0 none (the library's product and
-// a pass of its own for GELU or residual are ahead).  The lines, by the rounds of the CUs and the share of their time that makes output
-// (us, library with its pass / here, residuals with the LayerNorm behind them):
+// The kernel for a product: columns / 32 of a tile; 8 and 10 the resident kernel (kHalfTall: with 320 rows and 256 columns), 3 to 5 the
+// split one, 0 none (the library's product and a pass of its own for GELU or residual are ahead).  The lines, by the rounds of the
+// CUs and the share of their time that makes output (us, library with its pass / here, residuals with the LayerNorm behind them):
 //   GELU: from half of the CUs on.  4096 x 768 -> 3072 33.8 / 28.7, 4096 x 1280 -> 5120 75.3 / 51.8, 20480 x 1024 -> 4096 188 / 165,
 //     65536 x 1280 -> 5120 863 / 768.
 //   plain: up to 8 rounds, 0.7.  4096 x 1024 -> 3072 27.7 / 26.2, 8192 x 768 -> 2304 35.8 / 30.7, 20480 x 1024 -> 3072 107 / 102, 32768 x 768 ->
 //     2304 119 / 104; but 4096 x 768 -> 2304 (0.56) 19.8 / 20.2, 65536 x 768 -> 2304 (9 rounds) 201 / 221.
 //   residual: 128-row tiles where the CUs hold them all at once.  4096 x 1280 -> 1280 31.1 / 23.6, 4096 x 5120 -> 1280 61.3 / 55.9.
-//     Else 256 x 256, on long loops within one round from 0.7 on (12288 x 5120 -> 1280 134 / 125; 0.5: 8192 x 4096 -> 1024 70 / 83, two
-//     rounds: 32768 x 4096 -> 1024 227 / 243), on short ones up to four rounds from 0.55 on (8192 x 1280 -> 1280 44.4 / 40.4, 32768 x
-//     1280 -> 1280 175 / 145; 0.5: 8192 x 1024 -> 1024 31.9 / 33.9, five rounds: 65536 x 1280 -> 1280 277 / 292).
+//     Else 320 x 256 where that fills its rounds from 0.8 on: 20480 x 4096 -> 1024 (1.0) 171 / 142, 20480 x 1024 -> 1024 76.6 / 56.3, 24576 x 3072
+//     -> 768 (0.9) 148 / 109, 40960 x 5120 -> 1280 (three rounds, 0.83) 553 / 472, 57344 x 5120 -> 1280 (four, 0.88) 702 / 628, 36864 x
+//     4096 -> 1024 (two, 0.9) 290 / 259.
+//     Else 256 x 256, on long loops within one round from 0.7 on (12288 x 5120 -> 1280 138 / 132; 0.5: 8192 x 4096 -> 1024 69 / 83, two
+//     rounds: 32768 x 4096 -> 1024 236 / 248), on short ones up to four rounds from 0.75 on (12288 x 1024 -> 1024 42.6 / 40.4, 32768 x
+//     1280 -> 1280 181 / 147; 0.5: 8192 x 1024 -> 1024 31.1 / 33.9, five rounds: 65536 x 1280 -> 1280 276 / 284).
+constexpr int kHalfTall = 58;  // 320 rows, 256 columns
 static int half_choose(int64_t M, int N, int K, int epi) {
   const int force = knob_or(KNOB_GEMM_HALF, 1);
   if (force <= 0 || K % 64 != 0 || K < 320 || M < 256 || N < 96) return 0;
+  if (force == kHalfTall) return epi == PP_RESIDUAL && N >= 256 && M >= 320 ? force : 0;
   if (force >= 3) return N >= 32 * force && (force != 10 || epi != PP_RESIDUAL) ? force : 0;
   if (epi == PP_RESIDUAL)
     for (int tn = 3; tn <= 5; ++tn) {
       const int64_t tiles = ((M + 127) / 128) * ((N + 32 * tn - 1) / (32 * tn));
       if (tiles <= 256 && tiles >= 128 && N >= 32 * tn) return tn;
     }
-  const PPChoice c = pp_choose(M, N, K / 64, epi != PP_RESIDUAL);
+  const PPChoice c = pp_choose(M, N, K / 64, epi == PP_RESIDUAL);
   if (c.tn == 0) return 0;
   bool pays = c.used >= 0.5;
   if (epi == PP_PLAIN) pays = c.rounds <= 8 && c.used >= 0.7;
-  if (epi == PP_RESIDUAL) pays = K >= 2048 ? c.rounds == 1 && c.used >= 0.7 : c.rounds <= 4 && c.used >= 0.75;
-  return pays ? c.tn : 0;
+  if (epi == PP_RESIDUAL) pays = c.tm == 5 ? c.used >= 0.8 : K >= 2048 ? c.rounds == 1 && c.used >= 0.7 : c.rounds <= 4 && c.used >= 0.75;
+  return pays ? (c.tm == 5 ? kHalfTall : c.tn) : 0;
 }
 
 template <class E>
 static int half_launch(PPArgs a, int tn, int epi, hipStream_t stream) {
   a.group_m = 4;
+  if (tn == kHalfTall) {
+    a.tiles_m = (a.M + 319) / 320;
+    a.tiles_n = (a.N + 255) / 256;
+    hipLaunchKernelGGL((gemm_pingpong_kernel<E, PP_RESIDUAL, 8, false, 5>), dim3(pp_grid(a)), dim3(512), 0, stream, a);
+    return check_launch("gemm_pingpong_kernel");
+  }
   a.tiles_n = (a.N + 32 * tn - 1) / (32 * tn);
   if (tn >= 8) {
     a.tiles_m = (a.M + 255) / 256;

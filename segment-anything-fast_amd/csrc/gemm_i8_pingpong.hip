@@ -30,17 +30,18 @@ static bool pays(int epi, int K, const PPChoice& c) {
   //     K = 5120, 1.0 (65536 -> 3840) 1126 / 994; but 0.59 (5000 -> 3840) 30.0 / 37.6
   //   shorter loops, 0.85, and at K = 768 not within one round: 0.94 (20480 x 768 -> 3072) 58.7 / 56.4, 1.0 (4096 x 1024 -> 4096) 23.4 /
   //     20.3; but 0.75 (12288 x 768 -> 3072) 38.0 / 40.5, 0.94 (5000 x 768 -> 3072, one round) 19.1 / 18.9
-  //   residual, K >= 2048, 0.7: 0.73 (28672 x 5120 -> 1280) 191 / 177, 0.94 (12288 x 5120 -> 1280) 81.6 / 65.6, 1.0 (65536) 406 / 345;
-  //     but 0.66 (28672 x 3072 -> 768) 71.1 / 76.1
-  //   residual, K from 1280, 0.9: 0.94 (12288 x 1280 -> 1280) 28.7 / 27.7, 1.0 (65536) 137 / 135; but 0.73 (28672) 58 / 70, and K = 1024
-  //     (65536 x 1024 -> 1024) 97 / 101
-  if (epi == EPI_RESIDUAL_BF16) return K >= 2048 ? c.used >= 0.7 : K >= 1280 && c.used >= 0.9;
+  //   residual, K >= 2048, 0.7: 0.75 (12288 x 4096 -> 1024) 58.4 / 51.9, 0.94 (12288 x 5120 -> 1280) 85.0 / 68.6, 1.0 (20480 x 4096 -> 1024, 320
+  //     rows) 93.9 / 72.6, (65536 x 5120 -> 1280) 401 / 337, 0.88 (28672 x 5120 -> 1280, 320 rows) 200 / 161; but 0.66 (28672 x 3072 -> 768) 75.5 / 80.1
+  //   residual, K from 1280 on, 0.9, from 1024 on within one round: 0.94 (24576 x 1280 -> 1280) 53.7 / 53.6, 1.0 (65536) 138 / 135, 1.0 (20480 x
+  //     1024 -> 1024, 320 rows) 35.6 / 31.7; but 0.88 (57344 x 1280 -> 1280) 123.9 / 126.6, K = 1024 in two rounds (40960 -> 1024) 57.2 / 61.9, and
+  //     inside an encoder 0.75 (12288 x 1024 -> 1024) and K = 768 (24576 -> 768) cost 1 % of it (alone 32.0 / 24.0 and 30.4 / 28.0)
+  if (epi == EPI_RESIDUAL_BF16) return K >= 2048 ? c.used >= 0.7 : c.used >= 0.9 && (K >= 1280 || (K >= 1024 && c.rounds == 1));
   return K >= 1280 ? c.used >= 0.75 : c.used >= 0.85 && (K >= 1024 || c.rounds > 1);
 }
 
 bool gemm_i8_pingpong_reads_rows(int64_t M, int N, int K) {
   if (K % 128 != 0 || K < 640) return false;  // (no knob: a workspace sized by this answer must fit the call that follows)
-  const PPChoice c = pp_choose(M, N, K / 128, true);
+  const PPChoice c = pp_choose(M, N, K / 128, false);
   return c.tn != 0 && pays(EPI_SCALE_BIAS_BF16, K, c);
 }
 
@@ -48,7 +49,7 @@ bool gemm_i8_pingpong_covers(int epi, const GemmArgs& g) {
   const int mode = knob_or(KNOB_GEMM_PINGPONG, 1);
   if (mode <= 0 || (epi != EPI_SCALE_BIAS_BF16 && epi != EPI_RESIDUAL_BF16) || g.dst_row || g.tile_counters) return false;
   if (g.K % 128 != 0 || !pp_addressable(pp_args(g))) return false;
-  const PPChoice c = pp_choose(g.M, g.N, g.K / 128, epi != EPI_RESIDUAL_BF16);
+  const PPChoice c = pp_choose(g.M, g.N, g.K / 128, epi == EPI_RESIDUAL_BF16);
   if (c.tn == 0) return false;
   if (mode >= 2) return true;
   return pays(epi, g.K, c);
@@ -56,15 +57,18 @@ bool gemm_i8_pingpong_covers(int epi, const GemmArgs& g) {
 
 int gemm_i8_pingpong_launch(int epi, const GemmArgs& g, hipStream_t stream) {
   PPArgs a = pp_args(g);
-  const int tn = pp_choose(g.M, g.N, a.nk, epi != EPI_RESIDUAL_BF16).tn;
+  const PPChoice c = pp_choose(g.M, g.N, a.nk, epi == EPI_RESIDUAL_BF16);
+  const int tn = c.tn;
   a.group_m = 4;
-  a.tiles_m = (a.M + 255) / 256;
+  a.tiles_m = (a.M + 64 * c.tm - 1) / (64 * c.tm);
   a.tiles_n = (a.N + 32 * tn - 1) / (32 * tn);
   // an output larger than the last-level cache that is read once (qkv, lin1) is streamed out
   const bool nt = g.stream_out != 0;
 #define SF_PP(E, TN, NT) hipLaunchKernelGGL((gemm_pingpong_kernel<PPInt8, E, TN, NT>), dim3(pp_grid(a)), dim3(512), 0, stream, a)
 #define SF_PP_PLAIN(TN) do { if (nt) SF_PP(PP_PLAIN, TN, true); else SF_PP(PP_PLAIN, TN, false); } while (0)
-  if (epi == EPI_RESIDUAL_BF16) SF_PP(PP_RESIDUAL, 8, false);
+  if (epi == EPI_RESIDUAL_BF16 && c.tm == 5)
+    hipLaunchKernelGGL((gemm_pingpong_kernel<PPInt8, PP_RESIDUAL, 8, false, 5>), dim3(pp_grid(a)), dim3(512), 0, stream, a);
+  else if (epi == EPI_RESIDUAL_BF16) SF_PP(PP_RESIDUAL, 8, false);
   else if (tn == 8) SF_PP_PLAIN(8);
   else SF_PP_PLAIN(10);
 #undef SF_PP_PLAIN

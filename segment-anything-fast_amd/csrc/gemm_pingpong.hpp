@@ -1,5 +1,5 @@
 // One matrix product y = x . w^T for the element types of this library (int8, bf16, fp16): output tiles of 256 rows and 256 or 320
-// columns, one resident workgroup of eight wavefronts per CU, two per SIMD that take turns at the matrix pipe.
+// columns, or 320 rows and 256 columns, one resident workgroup of eight wavefronts per CU, two per SIMD that take turns at the matrix pipe.
 //
 // What bounds it is power, not the matrix pipe.  The pipe is busy 0.93-0.96 of the loop's cycles, and on operands
 // like an encoder's the clock settles at 1.5-1.7 GHz of 2.4, so every choice here is about energy per product or
@@ -83,19 +83,19 @@ SF_DEVICE void pp_wait() {
   __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | ((N >> 4) << 14));
 }
 
-// TN: 16-column fragments of a wavefront's half of the tile (the tile has 256 rows and 32 TN columns).  A turn multiplies H
-// of them.  The fragments' columns are dealt so that a lane ends with quads and at most one pair of adjacent columns:
+// TM: 16-row fragments of a wavefront (the tile has 64 TM rows).  TN: 16-column fragments of a wavefront's half of the tile (the
+// tile has 32 TN columns).  A turn multiplies H of them.  The fragments' columns are dealt so that a lane ends with quads and at most one pair of adjacent columns:
 // element e of a quad q is column 64 q + 4 lr + e of the half, of the pair 64 NQ + 2 lr + e.
-template <int TN>
+template <int TN, int TM>
 struct PPTile {
-  static_assert(TN == 8 || TN == 10, "widths built: 256, 320");
-  static constexpr int BM = 256, BN = 32 * TN, H = TN / 2;
+  static_assert((TN == 8 || TN == 10) && TM + TN / 2 <= 9 && TM >= 4, "tiles built: 256 x {256, 320}, 320 x 256");
+  static constexpr int BM = 64 * TM, BN = 32 * TN, H = TN / 2;
   static constexpr int NQ = TN / 4;
   static constexpr bool PAIR = TN % 4 != 0;
   static constexpr int STAGE = (BM + BN) * 128;        // one k tile of X and W
   static constexpr int SCALES = BM * 4 + 2 * BN * 4;   // int8: sx, sw, bias; half types: bias in the first bytes
-  static constexpr int NLOADS = 4 + H;                 // of a wavefront per k tile
-  static constexpr int NSTORES = 16 * (NQ + PAIR);
+  static constexpr int NLOADS = TM + H;                // of a wavefront per k tile
+  static constexpr int NSTORES = 4 * TM * (NQ + PAIR);
   static_assert(2 * STAGE + SCALES <= 160 * 1024, "LDS of a CU");
   static_assert(NLOADS + NSTORES < 64, "vmcnt threshold");
   // column of the half that fragment j of a turn holds in its row r
@@ -106,10 +106,10 @@ struct PPTile {
 };
 
 // NT: non-temporal stores
-template <class E, int EPI, int TN, bool NT>
+template <class E, int EPI, int TN, bool NT, int TM = 4>
 __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
   typedef typename E::Out Out;
-  using P = PPTile<TN>;
+  using P = PPTile<TN, TM>;
   constexpr bool RES = EPI == PP_RESIDUAL;
   constexpr int H = P::H;
   __shared__ __attribute__((aligned(16))) unsigned char lds[2 * P::STAGE + P::SCALES];
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 3, wn = wave >> 2;  // 64 rows, half of the columns; wn is also the side that takes turns
+  const int wm = wave & 3, wn = wave >> 2;  // 16 TM rows, half of the columns; wn is also the side that takes turns
   const int lr = lane & 15, lq = lane >> 4;
 
   // ---- the tiles of this workgroup: XCD x owns a contiguous range, its workgroups walk it side by side -----------
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
   const unsigned int last = min(total, (xcd + 1u) * chunk);
   if (slot >= chunk || first >= last) return;  // uniform over the workgroup
   const int nt = (int)((last - first + per_x - 1u) / per_x);
-  // Origin of tile ti.  Tiles at the lower and right edge are moved back inside (M >= 256, N >= BN), so that every load is in
+  // Origin of tile ti.  Tiles at the lower and right edge are moved back inside (M >= BM, N >= BN), so that every load is in
   // bounds; the rows and columns that belong to the tile before (skip_m, skip_n) are not stored.
   auto tile_origin = [&](int ti, int& m0, int& n0, int& skip_m, int& skip_n) __attribute__((always_inline)) {
     const unsigned int pid = first + (unsigned int)ti * per_x;
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
   };
   auto load_x = [&](int stage) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) load(xk + (int64_t)(64 * i) * a.x_pitch, off_x, (wave + 8 * i) * 8, stage);
+    for (int i = 0; i < TM; ++i) load(xk + (int64_t)(64 * i) * a.x_pitch, off_x, (wave + 8 * i) * 8, stage);
   };
   auto load_w = [&](int turn, int stage) __attribute__((always_inline)) {
 #pragma unroll
@@ -228,18 +228,18 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
     }
   };
 
-  // ---- fragments and products: rows 16 i + lr of the wavefront's 64, columns through j --------------------------
+  // ---- fragments and products: rows 16 i + lr of the wavefront's 16 TM, columns through j --------------------------
   const int frag = (lq ^ ((lr >> 1) & 7)) * 16;
-  const int x_off[2] = {(wm * 64 + lr) * 128 + frag, (wm * 64 + lr) * 128 + (frag ^ 64)};
+  const int x_off[2] = {(wm * 16 * TM + lr) * 128 + frag, (wm * 16 * TM + lr) * 128 + (frag ^ 64)};
   const int w_off[2] = {(P::BM + wn * 16 * TN + lr) * 128 + frag, (P::BM + wn * 16 * TN + lr) * 128 + (frag ^ 64)};
-  i32x4 fx[2][4], fw[2][H];
-  typename E::acc_t acc[4][TN];
+  i32x4 fx[2][TM], fw[2][H];
+  typename E::acc_t acc[TM][TN];
   auto read = [&](int turn, int stage) __attribute__((always_inline)) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       if (turn == 0)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) fx[k][i] = *reinterpret_cast<const i32x4*>(lds + stage + x_off[k] + i * 2048);
+        for (int i = 0; i < TM; ++i) fx[k][i] = *reinterpret_cast<const i32x4*>(lds + stage + x_off[k] + i * 2048);
 #pragma unroll
       for (int j = 0; j < H; ++j) fw[k][j] = *reinterpret_cast<const i32x4*>(lds + stage + w_off[k] + (turn * H + j) * 2048);
     }
@@ -250,7 +250,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
 #pragma unroll
     for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int jj = 0; jj < H; ++jj) {
           const int j = i & 1 ? H - 1 - jj : jj;  // one operand stays from each instruction to the next
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
         }
     // (the products are pure values to the compiler; this pins them to their turn)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < H; ++j) asm volatile("" : "+v"(acc[i][T * H + j]));
     __builtin_amdgcn_s_setprio(0);
@@ -270,11 +270,11 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // ---- output: rows wm * 64 + 16 i + 4 lq + r, quads and pair of columns from col0 on ------------------------------
+  // ---- output: rows 16 (TM wm + i) + 4 lq + r, quads and pair of columns from col0 on ------------------------------
   typedef __attribute__((address_space(1))) unsigned char* gbyte_t;
   const int col0 = wn * 16 * TN;
   // address of row 16 i + r, group g of this lane in the tile at `tile` (uniform base, 32-bit lane offset; the pitch is
-  // made opaque at every use: as loop invariants the 16 row offsets would be kept in registers)
+  // made opaque at every use: as loop invariants the row offsets would be kept in registers)
   auto lane_again = [&]() __attribute__((always_inline)) {  // (made again at every use: kept, it would be spilled)
     int l = lane;
     asm volatile("" : "+v"(l));
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
     const int l = lane_again();
     unsigned int pitch = (unsigned int)ld * 2u;
     asm volatile("" : "+s"(pitch));
-    const unsigned char* p = reinterpret_cast<const unsigned char*>(tile) + (unsigned int)(wm * 64 + 16 * i + r) * pitch + (col0 + 64 * g) * 2;
+    const unsigned char* p = reinterpret_cast<const unsigned char*>(tile) + (unsigned int)(wm * 16 * TM + 16 * i + r) * pitch + (col0 + 64 * g) * 2;
     asm volatile("" : "+s"(p));
     unsigned int lane_off = (unsigned int)(4 * (l >> 4)) * pitch + (g < P::NQ ? 8 : 4) * (l & 15);
     asm volatile("" : "+v"(lane_off));
@@ -292,9 +292,11 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
   };
   typedef __attribute__((address_space(1))) u32x2* gquad_t;
   typedef __attribute__((address_space(1))) unsigned int* gpair_t;
-  constexpr int EARLY = P::NQ * 4 + (P::PAIR ? 4 : 0);  // residual values of the first row group: requested in the last k tile
-  u32x2 res[RES ? 4 : 1][4][P::NQ];
-  unsigned int res_pair[RES && P::PAIR ? 4 : 1][4];
+  // residual values of the first row group: requested in the last k tile (where the operands leave registers for them)
+  constexpr bool AHEAD = RES && TM == 4;
+  constexpr int EARLY = P::NQ * 4 + (P::PAIR ? 4 : 0);
+  u32x2 res[RES ? TM : 1][4][P::NQ];
+  unsigned int res_pair[RES && P::PAIR ? TM : 1][4];
   auto load_residual = [&](int i) __attribute__((always_inline)) {
     const unsigned short* tile = a.residual + (int64_t)m0 * a.ld_res + n0;
 #pragma unroll
@@ -308,6 +310,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
     constexpr bool FULL = decltype(whole)::value;
     const int l = lane_again(), lr = l & 15, lq = l >> 4;
     if constexpr (RES) {
+      if constexpr (!AHEAD) load_residual(0);
       load_residual(1);
       load_residual(2);
       __builtin_amdgcn_sched_barrier(0);
@@ -330,11 +333,11 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
     }
     unsigned short* const tile = a.out + (int64_t)m0 * a.ldo + n0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < TM; ++i) {
       if constexpr (RES)
-        if (i == 1) load_residual(3);  // (three of the four row groups at a time: registers)
+        if (i >= 1 && i + 2 < TM) load_residual(i + 2);  // (three of the row groups at a time: registers)
       f32x4 sx;
-      if constexpr (E::SCALED) sx = *reinterpret_cast<const f32x4*>(sc + (wm * 64 + 16 * i + 4 * lq) * 4);
+      if constexpr (E::SCALED) sx = *reinterpret_cast<const f32x4*>(sc + (wm * 16 * TM + 16 * i + 4 * lq) * 4);
       // two adjacent columns of row r, rounded; group g, elements e and e + 1, plus the residual pair v
       auto two = [&](int r, int g, int e, unsigned int v) __attribute__((always_inline)) {
         float y[2];
@@ -361,7 +364,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
       };
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = wm * 64 + 16 * i + 4 * lq + r;
+        const int row = wm * 16 * TM + 16 * i + 4 * lq + r;
 #pragma unroll
         for (int g = 0; g < P::NQ; ++g) {
           const u32x2 v = RES ? res[RES ? i : 0][r][g] : u32x2{0u, 0u};
@@ -406,7 +409,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
     using T0 = std::integral_constant<int, 0>;
     using T1 = std::integral_constant<int, 1>;
     constexpr int EXTRA = decltype(extra_n)::value;
-    constexpr bool LAST = RES && !decltype(zero)::value && EXTRA > 0;
+    constexpr bool LAST = AHEAD && !decltype(zero)::value && EXTRA > 0;
     const int other = stage ^ P::STAGE;
     read(0, stage);
     load_w(1, other);
@@ -433,8 +436,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
   bool stored = false;  // a whole tile's stores are on their way
   for (int ti = 0; ti < nt; ++ti) {
     ktile(Yes{}, std::integral_constant<int, P::NSTORES>{}, stored);
-    for (int k = 1; k < a.nk - (RES ? 1 : 0); ++k) ktile(No{}, std::integral_constant<int, 0>{}, false);
-    if constexpr (RES) ktile(No{}, std::integral_constant<int, EARLY>{}, true);
+    for (int k = 1; k < a.nk - (AHEAD ? 1 : 0); ++k) ktile(No{}, std::integral_constant<int, 0>{}, false);
+    if constexpr (AHEAD) ktile(No{}, std::integral_constant<int, EARLY>{}, true);
     stored = skip_m == 0 && skip_n == 0;
     if (stored) finish(Yes{});
     else finish(No{});
@@ -715,29 +718,35 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_split_kernel(PPArgs a) {
 }
 
 // ---- host side ---------------------------------------------------------------------------------------------------------
-// Time of a launch in units of one 16-column fragment for one k tile: rounds of the CUs, each as long as its k tiles and a start
-// and an end worth eight more of them, a tile two or three and a half fragments more expensive than its columns.  The width with the
+// Time of a launch in units of one 16-column fragment of 64 rows for one k tile: rounds of the CUs, each as long as its k tiles and a start
+// and an end worth eight more of them, a tile two or three and a half fragments more expensive than its columns.  The tile with the
 // least; `used`: the share of those CU-cycles that makes output.
 // us, 256 / 320 columns: int8 inside the encoder 65536 x 1280 -> 3840 263 / 301; 4096 x 1280 -> 5120 (320 / 256 tiles) 33.0 / 28.1, 8192 x 1280 ->
 // 5120 (three / two rounds) 57.7 / 52.6, 20480 x 1280 -> 5120 (seven / five) 129.5 / 124.1.  (192 columns, at an
 // equal number of columns per CU, lost: 65536 x 1280 -> 3840 284 / 305, 4096 x 1024 -> 3072 17.5 / 18.3.)
+// The residual's registers leave no room for 320 columns, but for 320 rows, which few columns and many rows fill better.  256 / 320
+// rows: int8 20480 x 4096 -> 1024 (two rounds / one) 97.1 / 72.6, 24576 x 3072 -> 768 76.8 / 55.6, 53248 x 4096 -> 1024 (four / three) 220.6 /
+// 203.2, in equal rounds 16384 x 4096 -> 1024 60.2 / 64.4, 65536 x 5120 -> 1280 337 / 372.
 struct PPChoice {
-  int tn;
+  int tm, tn;
   int64_t rounds;
   double used;
 };
-static inline PPChoice pp_choose(int64_t M, int N, int nk, bool wide) {
-  PPChoice best = {0, 0, 0.0};
+static inline PPChoice pp_choose(int64_t M, int N, int nk, bool residual) {
+  PPChoice best = {0, 0, 0, 0.0};
   double least = 0.0;
-  for (int tn = 8; tn <= (wide ? 10 : 8); tn += 2) {
-    if (N < 32 * tn || M < 256) continue;
-    const int64_t rounds = (((M + 255) / 256) * ((N + 32 * tn - 1) / (32 * tn)) + 255) / 256;
-    const double cost = (double)rounds * (tn == 8 ? 10.0 : 13.5) * (nk + 8);
+  auto candidate = [&](int tm, int tn, double fragments) {
+    if (N < 32 * tn || M < 64 * tm) return;
+    const int64_t rounds = (((M + 64 * tm - 1) / (64 * tm)) * ((N + 32 * tn - 1) / (32 * tn)) + 255) / 256;
+    const double cost = (double)rounds * fragments * (nk + 8);
     if (best.tn == 0 || cost < least) {
-      best = PPChoice{tn, rounds, (double)M * N / (256.0 * rounds * 256 * 32 * tn)};
+      best = PPChoice{tm, tn, rounds, (double)M * N / (256.0 * rounds * 64 * tm * 32 * tn)};
       least = cost;
     }
-  }
+  };
+  candidate(4, 8, 10.0);
+  if (residual) candidate(5, 8, 12.5);
+  else candidate(4, 10, 13.5);
   return best;
 }
 

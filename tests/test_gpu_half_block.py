@@ -31,6 +31,8 @@ def test_add_layernorm_and_gelu_rows(M, K, dtype):
     (256, 256, 320, 0, 8), (700, 520, 384, 1, 8), (4096, 3840, 320, 2, 8), (20000, 1032, 320, 0, 8),
     (256, 320, 320, 1, 10), (900, 648, 448, 0, 10), (9000, 1288, 320, 1, 10),
     (256, 96, 320, 2, 3), (700, 200, 832, 0, 3), (300, 128, 320, 1, 4), (4096, 1024, 1024, 2, 4), (256, 160, 320, 0, 5), (4000, 1288, 1280, 2, 5),
+    # 320 rows by 256 columns
+    (320, 256, 320, 2, 58), (700, 520, 384, 2, 58), (40900, 1016, 320, 2, 58),
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_half_linear_with_its_epilogues(M, N, K, epi, tile, dtype):

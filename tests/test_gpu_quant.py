@@ -662,10 +662,12 @@ def test_gelu_quantiser_is_the_epilogue_and_the_quantiser(M, K, layout):
     # (chosen width) one tile and the shortest loop; ragged rows and columns, moved back tiles; lists of two tiles, whole and not
     (256, 256, 640, 0), (256, 320, 768, 0), (300, 264, 1280, 2), (1000, 1288, 896, 0), (2433, 2056, 1536, 2),
     (4096, 5120, 768, 0), (20480, 1024, 640, 2), (17000, 1288, 768, 2), (33000, 648, 768, 0),
+    # (320 rows by 256 columns) ragged, lists of two tiles
+    (20400, 1000, 640, 2), (40900, 1016, 768, 2),
 ])
 @pytest.mark.parametrize("layout", [0, 1])
 def test_gemm_by_turns_agrees(M, N, K, epi, layout):
-    """256 x {256, 320} tiles whose two halves take turns: the bits of the 64 x 128 tiles; residual also in place."""
+    """256 x {256, 320} and 320 x 256 tiles whose two halves take turns: the bits of the 64 x 128 tiles; residual also in place."""
     from samfast_amd import _lib, ops
     print(f"case gemm by turns M={M} N={N} K={K} epi={epi} layout={layout}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
