@@ -868,11 +868,15 @@ static int launch_hd(const AttnArgs& a, bool global_path, hipStream_t stream) {
       const unsigned int grid = (unsigned int)(((total + 7) / 8) * 8);
       hipLaunchKernelGGL((attn_global_kernel<T, HD, QT, WAVES>), dim3(grid), dim3(64 * WAVES), 0, stream, a);
     };
-    // 256 queries per workgroup when that still gives every CU several workgroups
-    // (SAMFAST_ATTN_WAVES=4 / 8 overrides the choice where the shape allows it)
-    const int64_t wg8 = (int64_t)a.B * a.nH * (a.N / 256);
+    // 256 queries per workgroup (one per CU) or 128 (two), which agree bit for bit, by how they divide among the 256 CUs
+    // (SAMFAST_ATTN_WAVES=4 / 8 overrides the choice where the shape allows it).  The prices are microseconds of a full round over 64
+    // key rows and, of 128 queries, of a last one with one workgroup per CU.  us, 128 / 256: 1 x 12 x 64 84 / 80, 1 x 16 x 64 91 / 88, 2 x 12 x 64
+    // 137 / 162, 8 x 16 x 64 682 / 687, 1 x 16 x 80 104 / 99, 2 x 16 x 80 202 / 195, 16 x 16 x 80 1612 / 1592.
+    const int64_t wgs4 = (int64_t)a.B * a.nH * (a.N / 128), wgs8 = (int64_t)a.B * a.nH * (a.N / 256), rest4 = wgs4 % 512;
+    const int full4 = HD == 64 ? 91 : 104, one4 = HD == 64 ? 46 : 52, full8 = HD == 64 ? 88 : 98;
+    const int64_t price4 = wgs4 / 512 * full4 + (rest4 == 0 ? 0 : rest4 <= 256 ? one4 : full4);
     const int force = knob(KNOB_ATTN_WAVES);
-    const bool want8 = force != kKnobUnset ? force == 8 : wg8 >= 1024;
+    const bool want8 = force != kKnobUnset ? force == 8 : (wgs8 + 255) / 256 * full8 <= price4;
     if (a.N % 256 == 0 && want8) launch(std::integral_constant<int, 8>{});
     else launch(std::integral_constant<int, 4>{});
     return check_launch("attn_global_kernel");
