@@ -46,7 +46,7 @@ PEAK = {"op": ("mfma", 5.0e15, "TOP/s"),       # int8 dense MFMA
 # workload (vit_h, batch 16, dense int8 linears) and only while the kernel family's source files
 # still have the hash they had when the counters were taken (otherwise `traffic` is null).
 TRAFFIC_SOURCE = "profiles/bench_vit_h_bs16_pmc_traffic.txt"
-TRAFFIC = {"gemm_i8_kernel": (1.0211e9, "gemm_i8.hip+gemm_i8_persist.hip+gemm_i8_shared.hpp", "502c262514342481")}
+TRAFFIC = {"gemm_i8_kernel": (1.0085e9, "gemm_i8.hip+gemm_i8_pingpong.hip+gemm_pingpong.hpp+gemm_i8_shared.hpp", "50e0bb8a7fe682e8")}
 
 
 def parse():
@@ -335,13 +335,14 @@ def gemm_variants(batch=16, width=1280):
     dev = torch.device("cuda:0")
     M = batch * 4096
     g = torch.Generator(device="cuda").manual_seed(11)
-    variants = [("three_workgroups_per_cu", {"SAMFAST_GEMM_PERSIST": 0}),
+    variants = [("256-row tiles by turns, where they pay (the default)", {}),
+                ("three_workgroups_per_cu", {"SAMFAST_GEMM_PINGPONG": 0, "SAMFAST_GEMM_PERSIST": 0}),
                 ("two_workgroups_per_cu", {"SAMFAST_GEMM_PERSIST": 0, "SAMFAST_GEMM_WG3": 0}),
                 ("persistent, all workgroups start together", {"SAMFAST_GEMM_PERSIST": 2, "SAMFAST_GEMM_PERSIST_SKEW": 0}),
                 ("persistent, every second workgroup starts a tile late", {"SAMFAST_GEMM_PERSIST": 2}),
                 ("persistent, skewed, no wave priorities", {"SAMFAST_GEMM_PERSIST": 2, "SAMFAST_GEMM_PERSIST_PRIO": 0})]
     shapes = [("qkv", 3 * width, width, _lib.EPILOGUE_NONE), ("proj", width, width, _lib.EPILOGUE_RESIDUAL),
-              ("lin1", 4 * width, width, _lib.EPILOGUE_GELU), ("lin2", width, 4 * width, _lib.EPILOGUE_RESIDUAL)]
+              ("lin1", 4 * width, width, _lib.EPILOGUE_NONE), ("lin2", width, 4 * width, _lib.EPILOGUE_RESIDUAL)]
     res = {"what": f"gemm_i8 at M={M}, us per launch (10 back to back) and TOP/s, per variant knob, on "
                    "all-zero / Gaussian int8 codes", "rows": {}}
     for name, N, K, epi in shapes:
