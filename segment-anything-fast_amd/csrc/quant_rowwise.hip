@@ -62,8 +62,9 @@ __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowwise_bf16_k
 
 // WPR wavefronts share a row: fewer registers per lane for long rows (one wavefront with 4096 values needs 238: two
 // per SIMD and 2.2 TB/s at 65536 rows, 5.1 TB/s with four sharing), and for few rows more wavefronts with
-// fewer loads each to wait for.  The shares' maxima meet in LDS.  Bound: HBM, at the rate of a copy, from 8192 rows on.
-template <int NCH, int EPC, int WPR, bool ACT>
+// fewer loads each to wait for.  The shares' maxima meet in LDS.  Bound: memory, at the rate of a copy, from 8192 rows on.
+// NTL: rows larger than the cache, read past it.
+template <int NCH, int EPC, int WPR, bool ACT, bool NTL>
 __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowshare_bf16_kernel(QuantArgs a) {
   constexpr int RPB = kQuantWavesPerBlock / WPR;  // rows per workgroup
   using RQ = RowQuantizer<NCH, EPC, false>;
@@ -84,7 +85,10 @@ __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowshare_bf16_
     const int c = (i * WPR + sub) * 64 + lane;
     const in_t z = {};
     xw[i] = z;
-    if (live && c < nchunk) xw[i] = __builtin_nontemporal_load(reinterpret_cast<const in_t*>(a.x + row * a.ldx) + c);
+    if (live && c < nchunk) {
+      const in_t* src = reinterpret_cast<const in_t*>(a.x + row * a.ldx) + c;
+      xw[i] = NTL ? __builtin_nontemporal_load(src) : *src;
+    }
   }
   if (ACT) gelu_chunks(xw);
 #pragma unroll
@@ -125,10 +129,10 @@ __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowshare_bf16_
   }
 }
 
-template <int NCH, int EPC, int WPR, bool ACT>
+template <int NCH, int EPC, int WPR, bool ACT, bool NTL>
 static int launch_rowshare(const QuantArgs& a, hipStream_t stream) {
   constexpr int RPB = kQuantWavesPerBlock / WPR;
-  hipLaunchKernelGGL((quant_rowshare_bf16_kernel<NCH, EPC, WPR, ACT>), dim3((unsigned int)((a.M + RPB - 1) / RPB)), dim3(64 * kQuantWavesPerBlock), 0, stream, a);
+  hipLaunchKernelGGL((quant_rowshare_bf16_kernel<NCH, EPC, WPR, ACT, NTL>), dim3((unsigned int)((a.M + RPB - 1) / RPB)), dim3(64 * kQuantWavesPerBlock), 0, stream, a);
   return check_launch("quant_rowshare_bf16_kernel");
 }
 
@@ -140,16 +144,16 @@ static int launch_quant(const QuantArgs& a, hipStream_t stream) {
   return check_launch("quant_rowwise_bf16_kernel");
 }
 
-template <int WPR, bool ACT>
+template <int WPR, bool ACT, bool NTL>
 static int launch_shares(const QuantArgs& a, hipStream_t s) {
   // shares that 4-element chunks divide among the 64 lanes exactly and 8-element chunks do not
-  if (a.K == 3 * 256 * WPR) return launch_rowshare<3, 4, WPR, ACT>(a, s);
-  if (a.K == 5 * 256 * WPR) return launch_rowshare<5, 4, WPR, ACT>(a, s);
+  if (a.K == 3 * 256 * WPR) return launch_rowshare<3, 4, WPR, ACT, NTL>(a, s);
+  if (a.K == 5 * 256 * WPR) return launch_rowshare<5, 4, WPR, ACT, NTL>(a, s);
   const int need = (a.K / 8 + 64 * WPR - 1) / (64 * WPR);
-  if (need <= 1) return launch_rowshare<1, 8, WPR, ACT>(a, s);
-  if (need <= 2) return launch_rowshare<2, 8, WPR, ACT>(a, s);
-  if (WPR == 2 || need <= 3) return launch_rowshare<3, 8, WPR, ACT>(a, s);
-  return launch_rowshare<4, 8, WPR, ACT>(a, s);
+  if (need <= 1) return launch_rowshare<1, 8, WPR, ACT, NTL>(a, s);
+  if (need <= 2) return launch_rowshare<2, 8, WPR, ACT, NTL>(a, s);
+  if (WPR == 2 || need <= 3) return launch_rowshare<3, 8, WPR, ACT, NTL>(a, s);
+  return launch_rowshare<4, 8, WPR, ACT, NTL>(a, s);
 }
 
 template <bool LN, bool ACT>
@@ -159,22 +163,24 @@ static int dispatch_quant(const QuantArgs& a, hipStream_t s) {
   if (a.K == 1280) return launch_quant<5, 4, LN, ACT>(a, s);
   const int need = (a.K / 8 + 63) / 64;
   if constexpr (!LN) {
-    // Rows of more than 1024: wavefronts that share a row (us, one wavefront a row / two / four).
-    //   Where one wavefront would need 128 registers and more, at any M: 65536 x 4096: 308 / 166 / 159, 16384 x 3072:
-    //   38 / 32 / 30, 65536 x 2560: 115 / 102 / 105, 4096 x 2048: 9.2 / 8.0 / 9.0.
-    //   Else while the rows are too few to fill the GPU with one wavefront each: 512 x 5120: 6.5 / 5.4 / 4.1, 1000 x 1536: 3.9 / 3.6 /
-    //   3.2, 8192 x 1536: 12.1 / 11.3 / 12.9.
-    //   K > 4096 beyond that (one / four): where quarters fill their lanes (K % 1024 == 0) the sharing form is the faster one as
-    //   long as its stores spread: 4096 x 5120 row-major 15.4 / 12.8, 16384 x 5120 43.7 / 40.6, K-block major 5003 x 5120 18.5 / 16.9,
-    //   8001 x 5120 26.5 / 23.4, 6001 x 6144 26.0 / 25.3.  K-block major codes of M % 16 == 0 rows have their K blocks a multiple of
-    //   1 KB apart, and the four stores meet: 4096 x 5120 15.2 / 16.6, 8192 x 5120 27.4 / 27.9.  Quarters that do not fill: 4001 x 4608
-    //   14.1 / 16.2.  From 11 chunks per lane on one wavefront is short of registers: 8192 x 8192 46.3 / 43.5.  At 32768 rows one
-    //   wavefront is ahead in either layout (K-block major 85.6 / 104.7 at K = 5120).
-    if (need == 3 && a.M <= 8192) return a.M <= 1024 ? launch_shares<4, ACT>(a, s) : launch_shares<2, ACT>(a, s);
-    if (need == 4 || need == 5) return a.M <= 1024 ? launch_shares<4, ACT>(a, s) : launch_shares<2, ACT>(a, s);
-    if (need >= 6 && need <= 8) return launch_shares<4, ACT>(a, s);
+    // Rows of more than 1024.  Where the rows and their codes fit the 256 MB last-level cache together (a producer has just put
+    // them there), they are read as such and shared: by two wavefronts up to 2560 values, by four above and for few rows, in which the
+    // wavefronts, not their loads, are scarce.  us, streamed and by the rules below / so: 4096 x 3072 10.8 / 9.5, 20480 x 3072 37.5 / 31.4, 4096 x 5120 15.6 /
+    // 13.1, 5003 x 5120 17.3 / 15.4, 8192 x 5120 27.9 / 21.9, 16384 x 5120 46.6 / 40.2, 20480 x 4096 47.5 / 40.0, 12288 x 1536 14.7 / 12.2, 32768 x
+    // 2048 42.3 / 32.8, 8192 x 8192 44.0 / 37.5 (168 MB of rows: the last that gain; inside an
+    // encoder, where lin1 has just written them, neither way is ahead); beyond, 20480 x 5120 56.2 / 68.7, 65536 x 5120 198 / 248.
+    // (Three loads of a wavefront, the third less than three quarters full, are as well alone from 8192 rows on: 12000 x 1152 12.6 / 13.0.)
+    if (need >= 3 && a.M * a.K * 3 <= (256ll << 20) && (a.K >= 1408 || a.M <= 8192))
+      return need >= 6 || a.M <= 1024 ? launch_shares<4, ACT, false>(a, s) : launch_shares<2, ACT, false>(a, s);
+    // Larger ones are streamed past the cache, and shared where one wavefront would need 128 registers and more (us, one wavefront a
+    // row / two / four: 65536 x 4096: 308 / 166 / 159, 65536 x 2560: 115 / 102 / 105).
+    if (need == 4 || need == 5) return launch_shares<2, ACT, true>(a, s);
+    if (need >= 6 && need <= 8) return launch_shares<4, ACT, true>(a, s);
+    // K > 4096: quarters that fill their lanes (K % 1024 == 0), while their stores spread.  K-block major codes of M % 16 == 0 rows have
+    // their K blocks a multiple of 1 KB apart, and the four stores meet.  From 11 chunks per lane on one wavefront is short of
+    // registers: 16384 x 8192 82 / 77.5; not at more rows: 32768 x 5120 87 / 105 (one / four).
     const bool spread = !a.kb64 || a.M % 16 != 0;
-    if (need > 8 && (a.M <= 2048 || (a.M <= 16384 && (need > 12 || (a.K % 1024 == 0 && spread))))) return launch_shares<4, ACT>(a, s);
+    if (need > 8 && a.M <= 16384 && (need > 12 || (a.K % 1024 == 0 && spread))) return launch_shares<4, ACT, true>(a, s);
   } else {
     if (need == 4) return launch_quant<4, 8, LN, ACT>(a, s);
     if (need > 4 && need <= 6) return launch_quant<6, 8, LN, ACT>(a, s);

@@ -658,6 +658,28 @@ def test_gelu_quantiser_is_the_epilogue_and_the_quantiser(M, K, layout):
     assert torch.equal(a[1:], b[1:])
 
 
+@pytest.mark.parametrize("K", [1152, 1536, 2560, 3072, 5120, 8192])
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_quantiser_on_both_sides_of_the_cache(K, layout, gelu):
+    """Rows that fit the last-level cache beside their codes and one row more (read past it, and shared otherwise): the codes and
+    scales that the first and the last rows have in a call of their own."""
+    from samfast_amd import _lib, ops
+    print(f"case quantiser cache line K={K} layout={layout} gelu={gelu}", flush=True)
+    fits = (256 << 20) // (3 * K)
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn((fits + 1, K), generator=g, device="cuda").to(torch.bfloat16)
+    x[0, 1] = float("nan")
+    x[-1] = 0.0
+    rows = (lambda c: ops.from_kb64(c)) if layout == _lib.LAYOUT_KB64 else (lambda c: c)
+    for M in (fits, fits + 1):
+        codes, scales = ops.quant_rowwise(x[:M], layout, gelu=gelu)
+        assert torch.isnan(scales[0]) and not torch.isnan(scales[1:]).any()
+        for part in (slice(1, 70), slice(M - 33, M)):
+            want_codes, want_scales = ops.quant_rowwise(x[:M][part], layout, gelu=gelu)
+            assert torch.equal(rows(codes)[part], rows(want_codes)) and torch.equal(scales[part], want_scales)
+
+
 @pytest.mark.parametrize("M,N,K,epi", [
     # (chosen width) one tile and the shortest loop; ragged rows and columns, moved back tiles; lists of two tiles, whole and not
     (256, 256, 640, 0), (256, 320, 768, 0), (300, 264, 1280, 2), (1000, 1288, 896, 0), (2433, 2056, 1536, 2),
