@@ -236,7 +236,7 @@ int samfast_preprocess(
  * An int8 block's middle in one launch: tokens = proj(quantise(x)) + residual and xq, sx = quantise(norm2(tokens)), with the
  * bits of samfast_quant_rowwise_i8, samfast_gemm_i8_fused (RESIDUAL) and samfast_layernorm_quant_i8
  * (modeling/image_encoder.py:178-181, 251).  x (M, C) with row stride ldx, wq (C/64, C, 64) K-block major, residual and tokens
- * (M, C) contiguous, possibly the same buffer, xq K-block major.  C is 768; samfast_proj_block_pays says at how many rows it is
+ * (M, C) contiguous, possibly the same buffer, xq K-block major.  C is 768 or 1024; samfast_proj_block_pays says at how many rows it is
  * ahead of the three launches.
  */
 int samfast_proj_block_pays(int64_t M, int C);

@@ -3,12 +3,14 @@
 //
 // At 4096 rows the three launches of it (5.0, 8.7 and 5.4 us at width 768) are mostly starts, ends and latency.  Here a workgroup
 // owns 16 whole rows (32 from 4097 rows on), so nothing between the quantisers leaves the CU: eight wavefronts quantise the rows into LDS,
-// multiply them by all of W - each its own eighth of the columns, fragments straight from the K-block-major weight into
-// registers, 1 KB a load, requested before the rows are there - and finish whole rows again, one wavefront each, with the quantiser's
-// own code.  What bounds it is W through the load path of every CU, 0.6 MB at 56 bytes a cycle: 4.5 us of the 16 (1.6 MB and 12 us at width
-// 1280, where the three launches stay ahead, 27.5 / 35.3 us at 4096 rows; 24.7 / 25.0 at width 1024: only 768 is built).
+// multiply them by all of W - each its own eighth of the columns, through a ring of 14 to 16 KB of its own in LDS that is requested before the
+// rows are there - and finish whole rows again, one wavefront each, with the quantiser's own code.  What bounds it is W through
+// the load path of every CU, 0.6 MB at 56 bytes a cycle: 4.7 us of the 13.6 at width 768 (fragments straight into registers, 16 bytes of each
+// of 16 rows to a quarter of the lanes, came at 33 bytes a cycle: 16.3 us).  Width 1280, 1.6 MB, is no faster than the three
+// launches (4096 rows 26.6 / 26.8) and not built.
 //
 // Codes, sums, roundings and scales are those of the separate launches: the same bits.
+#include "attn_relpos_shared.hpp"
 #include "gemm_i8_shared.hpp"
 #include "quant_row.hpp"
 
@@ -27,6 +29,17 @@ struct ProjBlockArgs {
   QuantArgs q;                     // x unused; gamma, beta, eps, xq (K-block major), sx of the output
 };
 
+// at most n vector memory operations of this wavefront outstanding (n constant at every use)
+SF_DEVICE void proj_wait(int n) {
+  switch (n) {
+#define SF_CASE(H) case H: __builtin_amdgcn_s_waitcnt(0x0F70 | (H)); break
+    SF_CASE(0); SF_CASE(1); SF_CASE(2); SF_CASE(3); SF_CASE(4); SF_CASE(5); SF_CASE(6); SF_CASE(7);
+    SF_CASE(8); SF_CASE(9); SF_CASE(10); SF_CASE(11); SF_CASE(12); SF_CASE(13); SF_CASE(14); SF_CASE(15);
+#undef SF_CASE
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 template <int C, int RT>
 __global__ __launch_bounds__(512) void proj_block_i8_kernel(ProjBlockArgs a) {
   constexpr int EPC = quant_epc_for(C), NCH = quant_nch_for(C), NCHUNK = C / EPC;
@@ -34,14 +47,15 @@ __global__ __launch_bounds__(512) void proj_block_i8_kernel(ProjBlockArgs a) {
   using Ln = RowQuantizer<NCH, EPC, true>;
   typedef typename In::in_t in_t;
   constexpr int R = 16 * RT, RPW = 2 * RT;      // rows of the workgroup, of a wavefront
-  constexpr int NF = C / 128, NK = C / 64;      // column fragments of a wavefront, k steps
-  constexpr int AHEAD = 7;                      // k steps of W in registers
+  constexpr int NF = C / 128, NK = C / 64;      // column fragments of a wavefront (16 columns x 64 bytes, 1 KB), k steps
+  constexpr int RING = RT == 1 ? 16 : 14;       // fragments of a wavefront in LDS
   constexpr int CP = C + 16, OP = 2 * C + 16;   // LDS row pitches: codes, Linear output
-  __shared__ __attribute__((aligned(16))) unsigned char lds[R * (CP > OP ? CP : OP) + R * CP];
+  static_assert(RING >= NF && RING - NF < 16, "wait thresholds");
+  static_assert(R * OP <= 8 * RING * 1024, "the output rows take the ring's place");
+  __shared__ __attribute__((aligned(16))) unsigned char lds[8 * RING * 1024 + R * CP];
   __shared__ float scales[R];
-  unsigned char* codes = lds;                   // R rows
-  unsigned char* rows = lds + R * CP;           // R rows of bf16
-  static_assert(R * CP + R * OP <= (int)sizeof(lds), "codes and rows side by side");
+  unsigned char* rows = lds;                    // R rows of bf16, behind the products
+  unsigned char* codes = lds + 8 * RING * 1024; // R rows
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -49,21 +63,35 @@ __global__ __launch_bounds__(512) void proj_block_i8_kernel(ProjBlockArgs a) {
   const int64_t row0 = (int64_t)blockIdx.x * R;
   const int64_t last = a.q.M - 1;
 
-  // ---- loads that wait for nothing: the rows to quantise, W's first k steps, the residual rows, gamma and beta ----------------------
+  // ---- loads that wait for nothing: the rows to quantise, then everything that is needed behind the products, then W ----------------
   in_t xw[RPW][NCH], res[RPW][NCH], gw[NCH], bw[NCH];
 #pragma unroll
   for (int r = 0; r < RPW; ++r) In::template load_row<false>(a.x + min(row0 + wave * RPW + r, last) * a.ldx, NCHUNK, lane, xw[r]);
-  const int8_t* wlane = a.w + (int64_t)(wave * (C / 8) + lr) * 64 + lq * 16;
-  i32x4 wf[AHEAD][NF];
-  auto load_w = [&](int k, i32x4 (&f)[NF]) __attribute__((always_inline)) {
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < NF; ++j) f[j] = *reinterpret_cast<const i32x4*>(wlane + (int64_t)k * C * 64 + j * 1024);
+  for (int r = 0; r < RPW; ++r) Ln::template load_row<false>(a.residual + min(row0 + wave * RPW + r, last) * C, NCHUNK, lane, res[r]);
+  Ln::load_affine(a.q.gamma, a.q.beta, NCHUNK, lane, gw, bw);
+  f32x4 sw[NF], bias[NF];
+  const float* bias_or_sw = a.bias ? a.bias : a.sw;  // (a load under a branch would make the compiler wait here)
+#pragma unroll
+  for (int j = 0; j < NF; ++j) {
+    const int n = wave * (C / 8) + 16 * j + 4 * lq;
+    sw[j] = *reinterpret_cast<const f32x4*>(a.sw + n);
+    bias[j] = *reinterpret_cast<const f32x4*>(bias_or_sw + n);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // Through LDS, although no other wavefront reads these columns: a fragment as the instruction takes it is 16 bytes of each of 16
+  // rows to a quarter of the lanes, which the load path serves at 33 bytes a cycle, in the order of memory at 56.
+  const unsigned int w_lane = (unsigned int)((lane >> 2) * 64 + (((lane & 3) ^ (-(lane >> 4) & 3)) * 16));
+  unsigned char* ring = lds + wave * RING * 1024;
+  const unsigned int ring_at = (unsigned int)(uintptr_t)((__attribute__((address_space(3))) unsigned char*)ring);
+  const unsigned char* wbase = reinterpret_cast<const unsigned char*>(a.w) + (int64_t)wave * (C / 8) * 64;
+  auto load_w = [&](int f) __attribute__((always_inline)) {
+    lds_dma16(wbase + (int64_t)(f / NF) * C * 64 + (f % NF) * 1024, w_lane, ring_at + f % RING * 1024);
   };
 #pragma unroll
-  for (int k = 0; k < AHEAD; ++k) {
-    load_w(k, wf[k]);
-    __builtin_amdgcn_sched_barrier(0);
-  }
+  for (int f = 0; f < RING; ++f) load_w(f);
+  __builtin_amdgcn_sched_barrier(0);
 
   // LDS written by all is visible to all; loads stay in flight (a __syncthreads would wait for them)
   auto meet = [] __device__ () __attribute__((always_inline)) {
@@ -91,40 +119,44 @@ __global__ __launch_bounds__(512) void proj_block_i8_kernel(ProjBlockArgs a) {
   for (int t = 0; t < RT; ++t)
 #pragma unroll
     for (int j = 0; j < NF; ++j) acc[t][j] = i32x4{0, 0, 0, 0};
+  const unsigned char* wfrag = ring + lr * 64 + ((lq ^ (-(lr >> 2) & 3)) * 16);
 #pragma unroll
   for (int k = 0; k < NK; ++k) {
-    i32x4 f[RT];
+    proj_wait((k * NF + RING < NK * NF ? k * NF + RING : NK * NF) - (k + 1) * NF);
+    i32x4 f[RT], w[NF];
 #pragma unroll
     for (int t = 0; t < RT; ++t) f[t] = *reinterpret_cast<const i32x4*>(codes + (16 * t + lr) * CP + k * 64 + lq * 16);
 #pragma unroll
+    for (int j = 0; j < NF; ++j) w[j] = *reinterpret_cast<const i32x4*>(wfrag + (k * NF + j) % RING * 1024);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // the fragments are in registers: their places are requested anew
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < NF; ++j)
+      if (k * NF + j + RING < NK * NF) load_w(k * NF + j + RING);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
     for (int j = 0; j < NF; ++j)
 #pragma unroll
-      for (int t = 0; t < RT; ++t) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[k % AHEAD][j], f[t], acc[t][j], 0, 0, 0);
-    if (k + AHEAD < NK) load_w(k + AHEAD, wf[k % AHEAD]);
-    __builtin_amdgcn_sched_barrier(0);  // (products and loads in this order: gathered, the loads behind would wait for all in front)
-    if (k == NK - AHEAD) {
-      // the residual rows and norm2's parameters travel under the last products
-#pragma unroll
-      for (int r = 0; r < RPW; ++r) Ln::template load_row<false>(a.residual + min(row0 + wave * RPW + r, last) * C, NCHUNK, lane, res[r]);
-      Ln::load_affine(a.q.gamma, a.q.beta, NCHUNK, lane, gw, bw);
-    }
+      for (int t = 0; t < RT; ++t) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[j], f[t], acc[t][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
   }
+  meet();  // nobody reads the ring any more
+  if (!a.bias)  // uniform
+#pragma unroll
+    for (int j = 0; j < NF; ++j) bias[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
     const float sx = scales[16 * t + lr];
 #pragma unroll
     for (int j = 0; j < NF; ++j) {
       const int n = wave * (C / 8) + 16 * j + 4 * lq;
-      const f32x4 sw = *reinterpret_cast<const f32x4*>(a.sw + n);
-      f32x4 bias = {0.f, 0.f, 0.f, 0.f};
-      if (a.bias) bias = *reinterpret_cast<const f32x4*>(a.bias + n);
       float y[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         // three separately rounded fp32 operations (no fused multiply-add)
         float v = (float)acc[t][j][e] * sx;
-        v = v * sw[e];
-        y[e] = v + bias[e];
+        v = v * sw[j][e];
+        y[e] = v + bias[j][e];
       }
       *reinterpret_cast<u32x2*>(rows + (16 * t + lr) * OP + n * 2) = u32x2{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
     }
@@ -156,12 +188,12 @@ __global__ __launch_bounds__(512) void proj_block_i8_kernel(ProjBlockArgs a) {
 
 }  // namespace samfast
 
-// A workgroup's time is the same for one row and for sixteen, so the three launches are ahead while they leave CUs idle and the one where its
-// grid is most of a round of 256 workgroups, of 16 rows up to 4096 and of 32 up to 8192.  us, three launches / one: 16 rows
-// 11.6 / 14.3, 2048 15.2 / 15.7, 2560 16.5 / 15.8, 4096 20.2 / 16.3, 4100 20.2 / 20.9, 5000 22.1 / 21.5, 6144 23.9 / 22.1, 8192
-// 25.7 / 23.0.
+// While one workgroup per CU does it; the time hardly depends on the rows, so the wider W needs enough of them to be ahead.  us, three launches /
+// one: width 768, 16 rows 11.5 / 11.3, 1024 13.0 / 12.0, 2048 15.0 / 12.5, 4096 20.0 / 13.6, 4100 19.7 / 18.2, 8192 25.5 / 20.4, 8200 26.5 / 33.0; width 1024, 1024
+// rows 15.8 / 17.2, 2048 18.8 / 17.7, 4096 24.0 / 19.5, 4100 25.5 / 25.7, 5121 27.1 / 26.4, 8192 31.9 / 29.3, 8200 35.4 / 48.3.
 extern "C" int samfast_proj_block_pays(int64_t M, int C) {
-  return C == 768 && ((M > 2304 && M <= 4096) || (M > 5120 && M <= 8192));
+  if (C == 768) return M <= 8192;
+  return C == 1024 && ((M > 1536 && M <= 4096) || (M > 4608 && M <= 8192));
 }
 
 extern "C" int samfast_proj_block_i8(const void* x, int64_t ldx, const int8_t* wq, const float* sw, const float* bias,
@@ -169,7 +201,7 @@ extern "C" int samfast_proj_block_i8(const void* x, int64_t ldx, const int8_t* w
                                      int8_t* xq, float* sx, int64_t M, int C, int dtype, void* stream) {
   using namespace samfast;
   if (dtype != SAMFAST_BF16) SF_FAIL(SAMFAST_E_UNSUPPORTED, "proj_block: only bf16");
-  if (C != 768) SF_FAIL(SAMFAST_E_UNSUPPORTED, "proj_block: width %d, only 768 is built", C);
+  if (C != 768 && C != 1024) SF_FAIL(SAMFAST_E_UNSUPPORTED, "proj_block: width %d, 768 and 1024 are built", C);
   SF_REQUIRE(M >= 0 && M * (int64_t)C < (1ll << 31), "proj_block: bad M=%lld", (long long)M);
   if (M == 0) return SAMFAST_OK;
   SF_REQUIRE(x && wq && sw && residual && tokens && gamma && beta && xq && sx, "proj_block: null pointer");
@@ -196,7 +228,10 @@ extern "C" int samfast_proj_block_i8(const void* x, int64_t ldx, const int8_t* w
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int rt = M <= 4096 ? 1 : 2;
   const dim3 grid((unsigned int)((M + 16 * rt - 1) / (16 * rt)));
-  if (rt == 1) hipLaunchKernelGGL((proj_block_i8_kernel<768, 1>), grid, dim3(512), 0, s, a);
-  else hipLaunchKernelGGL((proj_block_i8_kernel<768, 2>), grid, dim3(512), 0, s, a);
+#define SF_PROJ(W) do { if (rt == 1) hipLaunchKernelGGL((proj_block_i8_kernel<W, 1>), grid, dim3(512), 0, s, a); \
+                        else hipLaunchKernelGGL((proj_block_i8_kernel<W, 2>), grid, dim3(512), 0, s, a); } while (0)
+  if (C == 768) SF_PROJ(768);
+  else SF_PROJ(1024);
+#undef SF_PROJ
   return check_launch("proj_block_i8_kernel");
 }

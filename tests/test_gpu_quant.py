@@ -713,14 +713,15 @@ def test_gemm_by_turns_agrees(M, N, K, epi, layout):
             assert torch.equal(got, want)
 
 
-@pytest.mark.parametrize("M,bias,pitch", [(1, True, 768), (15, False, 776), (17, True, 2304), (2305, True, 768), (4096, False, 768), (4097, True, 1536),
-                                          (5121, True, 768), (8191, False, 768)])
-def test_proj_block_is_its_three_launches(M, bias, pitch):
+@pytest.mark.parametrize("M,bias,pitch,C", [(1, True, 768, 768), (15, False, 776, 768), (17, True, 2304, 768), (2305, True, 768, 768), (4096, False, 768, 768),
+                                            (4097, True, 1536, 768), (5121, True, 768, 768), (8191, False, 768, 768), (8193, True, 768, 768),
+                                            (7, False, 1032, 1024), (1537, True, 1024, 1024), (4096, True, 3072, 1024), (4100, False, 1024, 1024), (8190, True, 1024, 1024)])
+def test_proj_block_is_its_three_launches(M, bias, pitch, C):
     """Quantiser, proj + residual, norm2 and the next quantiser in one launch (16 rows a workgroup, 32 from 4097 on): the bits of
     the separate launches, also for rows with NaN, zeros and infinities and with the tokens written in place."""
     from samfast_amd import _lib, ops
-    print(f"case proj block M={M} bias={bias} pitch={pitch}", flush=True)
-    C, L = 768, _lib.LAYOUT_KB64
+    print(f"case proj block M={M} bias={bias} pitch={pitch} C={C}", flush=True)
+    L = _lib.LAYOUT_KB64
     g = torch.Generator(device="cuda").manual_seed(M)
     x = torch.randn((M, pitch), generator=g, device="cuda").to(torch.bfloat16)[:, :C]
     x[M // 2], x[0, 5] = 0.0, float("nan")
