@@ -1010,6 +1010,9 @@ static int gemm_common(int epi, const int8_t* xq, const float* sx, const int8_t*
   // (not where one of the other members is asked for)
   const bool unasked = !tail && tm == 2 && knob(KNOB_GEMM_TILE) == kKnobUnset && knob(KNOB_GEMM_WG3) != 0 &&
                        knob_or(KNOB_GEMM_PERSIST, 1) < 2 && knob_or(KNOB_GEMM_SPLITK, 1) < 2;
+  // GELU outputs the GPU holds once, K = 768: one tile per CU
+  if (unasked && knob_or(KNOB_GEMM_ONCE, 1) <= 1 && knob_or(KNOB_GEMM_PINGPONG, 1) <= 1 && gemm_i8_strip_covers(epi, a))
+    return gemm_i8_strip_launch(a, stream);
   // whole rounds of 256 x 256 or 256 x 320 tiles: the halves of a workgroup by turns
   if (unasked && knob_or(KNOB_GEMM_ONCE, 1) <= 1 && gemm_i8_pingpong_covers(epi, a)) return gemm_i8_pingpong_launch(epi, a, stream);
   // outputs the GPU holds once, K >= 1280: one tile per CU

@@ -60,4 +60,8 @@ bool gemm_i8_pingpong_reads_rows(int64_t M, int N, int K);
 bool gemm_i8_once_covers(int epi, const GemmArgs& a);
 int gemm_i8_once_launch(int epi, const GemmArgs& a, hipStream_t stream);
 
+// One tile per CU with GELU on loops of K = 768 (gemm_i8_strip.hip), the same way.
+bool gemm_i8_strip_covers(int epi, const GemmArgs& a);
+int gemm_i8_strip_launch(const GemmArgs& a, hipStream_t stream);
+
 }  // namespace samfast

@@ -713,6 +713,27 @@ def test_gemm_by_turns_agrees(M, N, K, epi, layout):
             assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("M,N,pitch", [(128, 384, 384), (300, 400, 400), (129, 1160, 1168), (4096, 3072, 3072), (4900, 2304, 2304), (9000, 776, 776)])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_gelu_strips_agree(M, N, pitch, layout):
+    """128 x 384 tiles over the whole of K = 768: the bits of the 64 x 128 tiles, edges moved back inside, with and without a bias."""
+    from samfast_amd import _lib, ops
+    print(f"case gelu strip M={M} N={N} pitch={pitch} layout={layout}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    xk, wk = (torch.randint(-127, 128, (n, 768), generator=g, dtype=torch.int8, device="cuda") for n in (M, N))
+    sx, sw = (torch.rand(n, generator=g, device="cuda") * 1e-2 for n in (M, N))
+    bias = torch.randn(N, generator=g, device="cuda") if M % 2 == 0 else None
+    if layout == _lib.LAYOUT_KB64:
+        xk, wk = ops.to_kb64(xk), ops.to_kb64(wk)
+    outs = []
+    for knobs in (dict(SAMFAST_GEMM_TILE=64, SAMFAST_GEMM_SKINNY=0), dict(SAMFAST_GEMM_STRIP=2, SAMFAST_GEMM_SKINNY=0)):
+        with _lib.knobs(**knobs):
+            buf = torch.zeros((M, pitch), dtype=torch.bfloat16, device="cuda")
+            ops.gemm_i8_fused(xk, sx, wk, sw, bias, _lib.EPILOGUE_GELU, out=buf[:, :N], layout=layout)
+            outs.append(buf)
+    assert torch.equal(*outs)
+
+
 @pytest.mark.parametrize("M,bias,pitch,C", [(1, True, 768, 768), (15, False, 776, 768), (17, True, 2304, 768), (2305, True, 768, 768), (4096, False, 768, 768),
                                             (4097, True, 1536, 768), (5121, True, 768, 768), (8191, False, 768, 768), (8193, True, 768, 768),
                                             (7, False, 1032, 1024), (1537, True, 1024, 1024), (4096, True, 3072, 1024), (4100, False, 1024, 1024), (8190, True, 1024, 1024)])
