@@ -218,7 +218,7 @@ int samfast_linear_half(
  * A convolution of the neck (modeling/image_encoder.py:88-104) over channels-last half-type images: y (B, H, W, Cout) of x
  * (B, H, W, Cin), stride 1, no bias; taps = 1: 1 x 1, w (Cout, Cin); taps = 9: 3 x 3 with zero padding of one, w (Cout, 9, Cin).
  * With relay_src the launch also writes relay_dst (relay_rows, 9, relay_cin) from a 3 x 3 weight (relay_rows, relay_cin, 3, 3): the
- * order a following call with taps = 9 wants.  Cin and Cout multiples of 64, pointers 16-byte aligned.
+ * order a following call with taps = 9 wants.  Cin and Cout multiples of 64, pointers 16-byte aligned.  Nothing is written for B = 0.
  */
 int samfast_neck_conv(
     const void* x, const void* w, void* y, int64_t B, int H, int W, int Cin, int Cout, int taps,

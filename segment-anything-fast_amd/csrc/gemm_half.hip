@@ -88,7 +88,8 @@ extern "C" int samfast_linear_half(const void* x, int64_t ldx, const void* w, co
     case SAMFAST_EPILOGUE_RESIDUAL: epi = PP_RESIDUAL; break;
     default: SF_FAIL(SAMFAST_E_INVALID, "linear_half: unknown epilogue %d", epilogue);
   }
-  SF_REQUIRE(M > 0 && N > 0 && K > 0 && N % 8 == 0, "linear_half: bad shape M=%lld N=%d K=%d (N must be a multiple of 8)", (long long)M, N, K);
+  SF_REQUIRE(M >= 0 && N > 0 && K > 0 && N % 8 == 0, "linear_half: bad shape M=%lld N=%d K=%d (N must be a multiple of 8)", (long long)M, N, K);
+  if (M == 0) return SAMFAST_OK;
   SF_REQUIRE(x && w && y && (epi != PP_RESIDUAL || residual), "linear_half: null pointer");
   SF_REQUIRE(aligned16(x) && aligned16(w) && aligned16(y) && aligned16(residual) && (reinterpret_cast<uintptr_t>(bias) & 3u) == 0,
              "linear_half: operands must be 16-byte aligned, the bias 4-byte");

@@ -146,9 +146,10 @@ extern "C" int samfast_neck_conv(const void* x, const void* w, void* y, int64_t 
   using namespace samfast;
   if (dtype != SAMFAST_BF16 && dtype != SAMFAST_F16) SF_FAIL(SAMFAST_E_UNSUPPORTED, "neck_conv: element type %d is neither SAMFAST_BF16 nor SAMFAST_F16", dtype);
   SF_REQUIRE(taps == 1 || taps == 9, "neck_conv: %d taps, 1 or 9 are built", taps);
-  SF_REQUIRE(B > 0 && H > 0 && W > 0 && Cin > 0 && Cout > 0 && Cin % CV == 0 && Cout % CV == 0,
+  SF_REQUIRE(B >= 0 && H > 0 && W > 0 && Cin > 0 && Cout > 0 && Cin % CV == 0 && Cout % CV == 0,
              "neck_conv: bad shape B=%lld H=%d W=%d Cin=%d Cout=%d (channels must be multiples of %d)", (long long)B, H, W, Cin, Cout, CV);
   SF_REQUIRE((int64_t)H * W < (1ll << 30) && B * H * W < (1ll << 30) && Cin <= (1 << 16) && Cout <= (1 << 16), "neck_conv: too large");
+  if (B == 0) return SAMFAST_OK;
   SF_REQUIRE(x && w && y && aligned16(x) && aligned16(w) && aligned16(y), "neck_conv: null or unaligned pointer");
   SF_REQUIRE((relay_src == nullptr) == (relay_dst == nullptr), "neck_conv: both ends of the reordered weight or none");
   SF_REQUIRE(!relay_src || (relay_rows > 0 && relay_rows <= (1 << 16) && relay_cin > 0 && relay_cin * 18 <= CVNST * CVSTAGE), "neck_conv: bad reordered weight");

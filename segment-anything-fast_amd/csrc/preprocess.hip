@@ -53,7 +53,8 @@ extern "C" int samfast_preprocess(const void* x, int x_is_u8, const float* mean,
                                   int dtype, void* stream) {
   using namespace samfast;
   if (dtype != SAMFAST_BF16 && dtype != SAMFAST_F16) SF_FAIL(SAMFAST_E_UNSUPPORTED, "preprocess: element type %d is neither SAMFAST_BF16 nor SAMFAST_F16", dtype);
-  SF_REQUIRE(B > 0 && h > 0 && w > 0 && S > 0 && S % 8 == 0 && h <= S && w <= S && S <= (1 << 16), "preprocess: bad shape B=%lld %dx%d in %d", (long long)B, h, w, S);
+  SF_REQUIRE(B >= 0 && h > 0 && w > 0 && S > 0 && S % 8 == 0 && h <= S && w <= S && S <= (1 << 16), "preprocess: bad shape B=%lld %dx%d in %d", (long long)B, h, w, S);
+  if (B == 0) return SAMFAST_OK;
   SF_REQUIRE(x && mean && std && y && aligned16(y) && (x_is_u8 || (reinterpret_cast<uintptr_t>(x) & 3u) == 0), "preprocess: null or unaligned pointer");
   PreprocessArgs a = {x, mean, std, reinterpret_cast<unsigned short*>(y), B * 3 * S * (S / 8), h, w, S};
   SF_REQUIRE((a.chunks + 255) / 256 < (1ll << 31), "preprocess: too large");

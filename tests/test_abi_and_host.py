@@ -109,6 +109,22 @@ def test_empty_calls_are_no_ops_without_gpu():
                                        *strides, 0, 0.125, None) == -1
 
 
+def test_empty_calls_of_block_neck_and_image_are_no_ops_without_gpu():
+    """The same for the half-type Linear, the int8 block's middle, the neck's convolutions and the image's preparation."""
+    from samfast_amd import _lib
+    lib = _lib.load()
+    for epilogue in (0, 1, 2):
+        assert lib.samfast_linear_half(None, 768, None, None, None, 3072, 0, 3072, 768, 0, epilogue, None, 3072, None) == 0
+        assert lib.samfast_linear_half(None, 768, None, None, None, 3072, -1, 3072, 768, 0, epilogue, None, 3072, None) == -1
+    proj = lambda M: lib.samfast_proj_block_i8(None, 768, None, None, None, None, None, None, None, 1e-6, None, None, M, 768, 0, None)
+    assert proj(0) == 0 and proj(-1) == -1
+    for taps in (1, 9):
+        conv = lambda B, channels=768: lib.samfast_neck_conv(None, None, None, B, 64, 64, channels, 256, taps, 0, None, None, 0, 0, None)
+        assert conv(0) == 0 and conv(-1) == -1 and conv(0, 100) == -1
+    image = lambda B, size=1024: lib.samfast_preprocess(None, 1, None, None, None, B, 700, 1024, size, 0, None)
+    assert image(0) == 0 and image(-1) == -1 and image(0, 1001) == -1
+
+
 def test_argument_validation_without_gpu():
     """Validation runs on the host before any launch, so error codes are testable here."""
     from samfast_amd import _lib

@@ -565,3 +565,17 @@ def test_predictor_keeps_a_model_s_own_preprocess_and_writes_where_the_recording
     sam.__class__ = Other
     pred.set_torch_image(images[0], (700, 1024))
     assert not torch.equal(pred.get_image_embedding(), want[0])
+
+
+@pytest.mark.parametrize("width,dtype,int8", [(128, torch.bfloat16, False), (128, torch.float16, False), (768, torch.bfloat16, True)])
+def test_an_empty_batch_gives_an_empty_embedding(width, dtype, int8):
+    import samfast_amd
+    from samfast_amd.modeling import ImageEncoderViT
+    print(f"case empty batch {width} {dtype} int8={int8}", flush=True)
+    enc = ImageEncoderViT(img_size=1024, embed_dim=width, depth=2, num_heads=width // 64, use_rel_pos=True, window_size=14, global_attn_indexes=(1,))
+    enc = enc.cuda().to(dtype).eval()
+    if int8:
+        samfast_amd.apply_dynamic_quant(enc)
+    with torch.no_grad():
+        y = enc(torch.empty((0, 3, 1024, 1024), device="cuda", dtype=dtype))
+    assert y.shape == (0, 256, 64, 64) and y.dtype == dtype
