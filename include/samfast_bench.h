@@ -20,9 +20,11 @@ extern "C" {
  * SAMFAST_GEMM_PINGPONG, SAMFAST_GEMM_HALF, SAMFAST_GEMM_SPLITK, SAMFAST_GEMM_ONCE, SAMFAST_GEMM_STRIP, SAMFAST_GEMM_LINEAR_SMALL, SAMFAST_GEMM_SKINNY,
  * SAMFAST_ATTN_WAVES, SAMFAST_ATTN_SPLIT, SAMFAST_ATTN_WINDOW_ROWS, SAMFAST_SPARSE_PERSIST.  This
  * call sets one (`unset` != 0: back to "not given", `value` ignored).  The knobs move time; every
- * variant of a kernel returns the same bits, with two exceptions that sum in another order:
- * SAMFAST_ATTN_SPLIT and SAMFAST_ATTN_WINDOW_ROWS.  (Neither default looks at the number of slices:
- * a slice's result does not depend on its batch.)  Returns SAMFAST_E_INVALID for an unknown name.
+ * variant of a kernel returns the same bits, with three exceptions that sum in another order:
+ * SAMFAST_ATTN_SPLIT, SAMFAST_ATTN_WINDOW_ROWS and SAMFAST_GEMM_HALF (the framework's products, tiles that sum K in one
+ * order, tiles that sum its halves apart).  The first two defaults do not look at the number of slices: a slice's
+ * attention does not depend on its batch.  A half-type product's kernel does follow its rows (samfast_linear_half_pays).
+ * Returns SAMFAST_E_INVALID for an unknown name.
  */
 int samfast_bench_set_knob(const char* name, int value, int unset);
 

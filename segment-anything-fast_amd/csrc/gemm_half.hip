@@ -23,7 +23,10 @@ static int half_choose(int64_t M, int N, int K, int epi) {
   const int force = knob_or(KNOB_GEMM_HALF, 1);
   if (force <= 0 || K % 64 != 0 || K < 320 || M < 256 || N < 96) return 0;
   if (force == kHalfTall) return epi == PP_RESIDUAL && N >= 256 && M >= 320 ? force : 0;
-  if (force >= 3) return N >= 32 * force && (force != 10 || epi != PP_RESIDUAL) ? force : 0;
+  if (force >= 3) {
+    const bool built = (force <= 5 || force == 8 || (force == 10 && epi != PP_RESIDUAL)) && N >= 32 * force;
+    return built ? force : 0;
+  }
   if (epi == PP_RESIDUAL)
     for (int tn = 3; tn <= 5; ++tn) {
       const int64_t tiles = ((M + 127) / 128) * ((N + 32 * tn - 1) / (32 * tn));

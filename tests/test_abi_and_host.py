@@ -66,6 +66,17 @@ def test_knobs_are_named_and_bounded_without_gpu():
     assert b"2^27" in lib.samfast_last_error()
 
 
+def test_the_half_product_knob_names_built_tiles_only():
+    """A tile that is not built is left to the framework's product, whatever number the knob holds."""
+    from samfast_amd import _lib
+    lib = _lib.load()
+    built = {_lib.EPILOGUE_NONE: {3, 4, 5, 8, 10}, _lib.EPILOGUE_GELU: {3, 4, 5, 8, 10}, _lib.EPILOGUE_RESIDUAL: {3, 4, 5, 8, 58}}
+    for value in (-1, 0, *range(3, 80)):
+        with _lib.knobs(SAMFAST_GEMM_HALF=value):
+            for epilogue, tiles in built.items():
+                assert lib.samfast_linear_half_pays(4096, 4096, 1280, epilogue) == (value in tiles), (value, epilogue)
+
+
 def test_fused_quant_gemm_refuses_outputs_its_quantiser_cannot_address():
     """lin1-shaped call with M * N >= 2^31: the in-kernel quantiser's 32-bit offsets would wrap, so
     the entry point (and its allocation-free form) refuses before anything is launched."""
