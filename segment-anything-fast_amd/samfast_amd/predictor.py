@@ -57,7 +57,7 @@ class SamPredictor:
         if type(model).preprocess is not Sam.preprocess or "preprocess" in model.__dict__:
             return None
         buffer, encoder = None, model.image_encoder
-        if type(encoder) is ReplayedEncoder and not encoder._forward_hooks and not encoder._forward_pre_hooks:
+        if isinstance(encoder, ReplayedEncoder):
             buffer = encoder.input_buffer((image.shape[0], 3, size, size), dtype, image.device)
         return ops.preprocess(image, model.pixel_mean, model.pixel_std, size, dtype, buffer)
 

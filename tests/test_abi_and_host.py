@@ -491,3 +491,37 @@ def test_copies_derived_from_a_buffer_are_kept_only_while_they_hold():
         c += 1
         assert torch.equal(copy_of(c), c) and len(made) == 7
     assert copy_of(a) is made[4]
+
+
+@pytest.mark.parametrize("who", ["nobody", "hook", "pre-hook", "global hook", "global pre-hook", "own forward", "subclass"])
+def test_a_recording_s_input_buffer_is_written_only_where_nobody_is_handed_it(who, monkeypatch):
+    """A predictor writes the image straight into the buffer that a recorded encoder reads; whoever else would see that
+    tensor, overwritten by the next image, makes it a tensor of its own."""
+    from types import SimpleNamespace
+    from samfast_amd import SamPredictor, ops
+    from samfast_amd.graphs import ReplayedEncoder
+    from samfast_amd.modeling import Sam
+    inner = torch.nn.Linear(1, 1)
+    inner.img_size = 64
+    encoder = ReplayedEncoder(inner).eval()
+    sam, device = Sam(encoder), torch.device("cuda", 0)
+    buffer = SimpleNamespace(is_cuda=True, shape=(1, 3, 64, 64), dim=lambda: 4)
+    encoder._graphs[((1, 3, 64, 64), torch.bfloat16, device)] = SimpleNamespace(_in=buffer)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(ops, "preprocess", lambda image, mean, std, size, dtype, out: out)
+    image = SimpleNamespace(shape=(1, 3, 40, 64), device=device)
+    from torch.nn.modules import module
+    handle = {"hook": encoder.register_forward_hook, "pre-hook": encoder.register_forward_pre_hook,
+              "global hook": module.register_module_forward_hook,
+              "global pre-hook": module.register_module_forward_pre_hook}.get(who, lambda f: None)(lambda *a: None)
+    if who == "own forward":
+        encoder.forward = lambda x: x
+    elif who == "subclass":
+        encoder.__class__ = type("Mine", (ReplayedEncoder,), {})
+    try:
+        with torch.no_grad():
+            got = SamPredictor(sam)._preprocessed(image, 64, torch.bfloat16)
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert got is (buffer if who == "nobody" else None)
