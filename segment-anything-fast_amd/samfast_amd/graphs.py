@@ -117,12 +117,14 @@ class ReplayedEncoder(nn.Module):
     def input_buffer(self, shape, dtype, device) -> Optional[torch.Tensor]:
         """The buffer that the recording for such an input reads, if there is one: an input written there on the current stream,
         and then passed to forward, is not copied.  None where somebody beside forward is handed the input - a hook on this
-        module or on every module, a forward of a subclass's or an instance's own - and might keep what the next image overwrites."""
+        module or on every module, a forward of a subclass's or an instance's own - and might keep what the next image overwrites,
+        and where forward would not replay: the encoder's own launches, recorded by the caller, would hold the address of a buffer
+        that goes with this recording."""
         if (type(self) is not ReplayedEncoder or "forward" in self.__dict__ or self._forward_hooks or self._forward_pre_hooks
                 or nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks):
             return None
         graph = self._graphs.get((tuple(shape), dtype, device))
-        return None if graph is None else graph._in
+        return None if graph is None or not self.replays(graph._in) else graph._in
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not self.replays(x):

@@ -493,7 +493,7 @@ def test_copies_derived_from_a_buffer_are_kept_only_while_they_hold():
     assert copy_of(a) is made[4]
 
 
-@pytest.mark.parametrize("who", ["nobody", "hook", "pre-hook", "global hook", "global pre-hook", "own forward", "subclass"])
+@pytest.mark.parametrize("who", ["nobody", "hook", "pre-hook", "global hook", "global pre-hook", "own forward", "subclass", "capture", "eager"])
 def test_a_recording_s_input_buffer_is_written_only_where_nobody_is_handed_it(who, monkeypatch):
     """A predictor writes the image straight into the buffer that a recorded encoder reads; whoever else would see that
     tensor, overwritten by the next image, makes it a tensor of its own."""
@@ -507,7 +507,7 @@ def test_a_recording_s_input_buffer_is_written_only_where_nobody_is_handed_it(wh
     sam, device = Sam(encoder), torch.device("cuda", 0)
     buffer = SimpleNamespace(is_cuda=True, shape=(1, 3, 64, 64), dim=lambda: 4)
     encoder._graphs[((1, 3, 64, 64), torch.bfloat16, device)] = SimpleNamespace(_in=buffer)
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: who == "capture")
     monkeypatch.setattr(ops, "preprocess", lambda image, mean, std, size, dtype, out: out)
     image = SimpleNamespace(shape=(1, 3, 40, 64), device=device)
     from torch.nn.modules import module
@@ -518,6 +518,8 @@ def test_a_recording_s_input_buffer_is_written_only_where_nobody_is_handed_it(wh
         encoder.forward = lambda x: x
     elif who == "subclass":
         encoder.__class__ = type("Mine", (ReplayedEncoder,), {})
+    elif who == "eager":
+        encoder.compile_mode = None
     try:
         with torch.no_grad():
             got = SamPredictor(sam)._preprocessed(image, 64, torch.bfloat16)

@@ -579,3 +579,31 @@ def test_an_empty_batch_gives_an_empty_embedding(width, dtype, int8):
     with torch.no_grad():
         y = enc(torch.empty((0, 3, 1024, 1024), device="cuda", dtype=dtype))
     assert y.shape == (0, 256, 64, 64) and y.dtype == dtype
+
+
+def test_a_caller_s_own_capture_outlives_the_recordings():
+    """set_torch_image under a graph of the caller's: nothing in it belongs to a recording that may be dropped."""
+    import samfast_amd
+    from samfast_amd.modeling import ImageEncoderViT, Sam
+    from samfast_amd.graphs import ReplayedEncoder
+    torch.manual_seed(2)
+    enc = ImageEncoderViT(img_size=1024, embed_dim=128, depth=2, num_heads=2, use_rel_pos=True, window_size=14, global_attn_indexes=(1,))
+    sam = Sam(ReplayedEncoder(enc.to(torch.bfloat16).eval())).cuda().eval()
+    images = [torch.randint(0, 256, (1, 3, 700, 1024), device="cuda", dtype=torch.uint8) for _ in range(3)]
+    with torch.no_grad():
+        want = [sam.image_encoder._orig_mod(sam.preprocess(i).to(torch.bfloat16)) for i in images]
+    pred = samfast_amd.SamPredictor(sam)
+    pred.set_torch_image(images[0], (700, 1024))  # records
+    image, graph = images[0].clone(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        pred.set_torch_image(image, (700, 1024))
+    out = pred.get_image_embedding()
+    sam.image_encoder.invalidate()
+    torch.cuda.synchronize()
+    kept = [torch.full((1, 3, 1024, 1024), float("nan"), device="cuda", dtype=torch.bfloat16) for _ in range(4)]
+    for i in (1, 2, 0, 1):
+        image.copy_(images[i])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[i])
+    assert all(k.isnan().all() for k in kept)
