@@ -627,6 +627,8 @@ def linear_half(x: torch.Tensor, linear: torch.nn.Linear, epilogue: int = _lib.E
     are left to the framework's product."""
     w, b = linear.weight, linear.bias
     M, K = x.shape
+    if w.dim() != 2 or w.shape[1] != K or (b is not None and b.shape != w.shape[:1]):
+        return None  # (the framework's product says what is wrong)
     N = w.shape[0]
     lib = _lib.load()
     if not lib.samfast_linear_half_pays(M, N, K, int(epilogue)):
@@ -637,6 +639,9 @@ def linear_half(x: torch.Tensor, linear: torch.nn.Linear, epilogue: int = _lib.E
             return None
     if not x.is_contiguous() or x.data_ptr() % 16 != 0 or x.device.index != torch.cuda.current_device():
         return None
+    for t in (residual, out):
+        if t is not None and (t.shape != (M, N) or t.dtype != x.dtype or t.device != x.device or not t.is_contiguous()):
+            raise RuntimeError("samfast: residual and out must be contiguous (rows, N) tensors of x's dtype and device")
     if out is None:
         out = torch.empty((M, N), dtype=x.dtype, device=x.device)
     code = _timed(

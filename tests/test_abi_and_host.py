@@ -6,6 +6,7 @@ import ctypes
 import inspect
 import re
 from pathlib import Path
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -497,7 +498,6 @@ def test_copies_derived_from_a_buffer_are_kept_only_while_they_hold():
 def test_a_recording_s_input_buffer_is_written_only_where_nobody_is_handed_it(who, monkeypatch):
     """A predictor writes the image straight into the buffer that a recorded encoder reads; whoever else would see that
     tensor, overwritten by the next image, makes it a tensor of its own."""
-    from types import SimpleNamespace
     from samfast_amd import SamPredictor, ops
     from samfast_amd.graphs import ReplayedEncoder
     from samfast_amd.modeling import Sam
@@ -527,3 +527,52 @@ def test_a_recording_s_input_buffer_is_written_only_where_nobody_is_handed_it(wh
         if handle is not None:
             handle.remove()
     assert got is (buffer if who == "nobody" else None)
+
+
+class _Recorder:
+    """A library whose entry points launch nothing: the names called, in order."""
+
+    def __init__(self):
+        self.called = []
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.called.append(name)
+            return 1 if name.endswith("_pays") else 0
+        return call
+
+    def launches(self):
+        return [n for n in self.called if not n.endswith("_pays")]
+
+
+@pytest.fixture
+def recorder(monkeypatch):
+    """ops on CPU tensors, up to the call into the library."""
+    from samfast_amd import _lib, ops
+    lib = _Recorder()
+    monkeypatch.setattr(_lib, "load", lambda: lib)
+    monkeypatch.setattr(_lib, "check", lambda code, what: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_require_gpu", lambda *tensors: None)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: None)
+    return lib
+
+
+def test_half_linear_launches_nothing_on_other_shapes(recorder):
+    """What the kernel would read past its end never reaches it: a weight or bias of another shape is the framework's
+    product's to refuse, a residual or output of another shape, type or stride an error."""
+    from samfast_amd import _lib, ops
+    half = lambda *shape: torch.zeros(shape, dtype=torch.bfloat16)
+    make = lambda w, b: SimpleNamespace(weight=w, bias=b)
+    x, linear = half(256, 320), make(half(96, 320), half(96))
+    assert ops.linear_half(x, linear).shape == (256, 96) and recorder.launches() == ["samfast_linear_half"]
+    recorder.called.clear()
+    for other in (make(half(96, 256), half(96)), make(half(96, 384), None), make(half(96, 320), half(95)), make(half(96, 320), half(1)),
+                  make(half(320), None)):
+        assert ops.linear_half(x, other) is None
+    for bad in (half(255, 96), half(256, 104), half(96), half(256, 96).float(), half(96, 256).t()):
+        with pytest.raises(RuntimeError):
+            ops.linear_half(x, linear, _lib.EPILOGUE_RESIDUAL, residual=bad)
+        with pytest.raises(RuntimeError):
+            ops.linear_half(x, linear, _lib.EPILOGUE_RESIDUAL, residual=half(256, 96), out=bad)
+    assert recorder.launches() == []
