@@ -567,6 +567,9 @@ def proj_block(x: torch.Tensor, wq: torch.Tensor, sw: torch.Tensor, bias: Option
         return None
     if gamma.dtype != x.dtype or beta.dtype != x.dtype or (bias is not None and not rows_launchable(bias)):
         return None
+    if any(t.numel() != C for t in (sw, gamma, beta)) or wq.dtype != torch.int8 or sw.dtype != torch.float32 \
+            or (bias is not None and (bias.numel() != C or bias.dtype != torch.float32)):
+        return None  # (the three launches' own checks say what is wrong)
     _require_gpu(x, wq, sw, bias, residual, gamma, beta)
     tokens = torch.empty_like(residual)
     xq = _xq_empty(M, C, _lib.LAYOUT_KB64, x.device)

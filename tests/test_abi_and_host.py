@@ -576,3 +576,20 @@ def test_half_linear_launches_nothing_on_other_shapes(recorder):
         with pytest.raises(RuntimeError):
             ops.linear_half(x, linear, _lib.EPILOGUE_RESIDUAL, residual=half(256, 96), out=bad)
     assert recorder.launches() == []
+
+
+def test_proj_block_launches_nothing_on_other_shapes(recorder):
+    """Scales, bias or norm parameters of another length or type are left to the checks of the separate launches."""
+    from samfast_amd import ops
+    C, M = 768, 32
+    x, res = (torch.zeros((M, C), dtype=torch.bfloat16) for _ in range(2))
+    wq, sw, bias = torch.zeros((C // 64, C, 64), dtype=torch.int8), torch.ones(C), torch.zeros(C)
+    norm = torch.ones(C, dtype=torch.bfloat16)
+    assert ops.proj_block(x, wq, sw, bias, res, (norm, norm, 1e-6)) is not None and recorder.launches() == ["samfast_proj_block_i8"]
+    recorder.called.clear()
+    short = norm[:C - 8].clone()
+    for args in ((wq, sw, bias, res, (short, norm, 1e-6)), (wq, sw, bias, res, (norm, short, 1e-6)), (wq, sw[:8].clone(), bias, res, (norm, norm, 1e-6)),
+                 (wq, sw, bias[:8].clone(), res, (norm, norm, 1e-6)), (wq, sw.bfloat16(), bias, res, (norm, norm, 1e-6)),
+                 (wq, sw, bias.bfloat16(), res, (norm, norm, 1e-6)), (wq[1:].clone(), sw, bias, res, (norm, norm, 1e-6))):
+        assert ops.proj_block(x, *args) is None
+    assert recorder.launches() == []
