@@ -156,12 +156,14 @@ class ImageEncoderViT(nn.Module):
         for m, size in ((conv1, 1), (conv3, 3)):
             if not (m.kernel_size == (size, size) and m.padding == (size // 2, size // 2) and m.stride == m.dilation == (1, 1)
                     and m.groups == 1 and m.bias is None and m.padding_mode == "zeros"
+                    and m.weight.shape == (m.out_channels, m.in_channels, size, size)
                     and m.in_channels % 64 == 0 and m.out_channels % 64 == 0 and m.in_channels <= 4096 and m.out_channels <= 4096):
                 return False
         tensors = (x, conv1.weight, norm1.weight, norm1.bias, conv3.weight, norm2.weight, norm2.bias)
         return (all(type(t) in (torch.Tensor, nn.Parameter) and t.dtype == x.dtype for t in tensors) and ops.rows_launchable(*tensors)
-                and conv1.in_channels == x.shape[3] and norm1.weight.numel() == conv1.out_channels == conv3.in_channels
-                and conv3.in_channels * 18 <= 96 * 1024 and norm2.weight.numel() == conv3.out_channels
+                and conv1.in_channels == x.shape[3] and conv1.out_channels == conv3.in_channels and conv3.in_channels * 18 <= 96 * 1024
+                and norm1.weight.numel() == norm1.bias.numel() == conv1.out_channels
+                and norm2.weight.numel() == norm2.bias.numel() == conv3.out_channels
                 and norm1.eps >= 0 and norm2.eps >= 0)
 
 

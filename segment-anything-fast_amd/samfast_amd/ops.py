@@ -662,6 +662,9 @@ def neck_convs(x: torch.Tensor, w1: torch.Tensor, norm, w3: torch.Tensor) -> tor
     _require_gpu(x, w1, w3)
     B, H, W, C = x.shape
     mid, out = w1.shape[0], w3.shape[0]
+    if w1.shape != (mid, C, 1, 1) or w3.shape != (out, mid, 3, 3) or w1.dtype != x.dtype or w3.dtype != x.dtype \
+            or not (x.is_contiguous() and w1.is_contiguous() and w3.is_contiguous()):
+        raise RuntimeError("samfast: neck_convs needs contiguous images and (mid, C, 1, 1), (out, mid, 3, 3) weights of one dtype")
     lib = _lib.load()
     y = torch.empty((B, H, W, mid), dtype=x.dtype, device=x.device)
     taps = torch.empty((out, 9, mid), dtype=x.dtype, device=x.device)
@@ -669,6 +672,8 @@ def neck_convs(x: torch.Tensor, w1: torch.Tensor, norm, w3: torch.Tensor) -> tor
         x.data_ptr(), w1.data_ptr(), y.data_ptr(), B, H, W, C, mid, 1, _dtype_code(x), w3.data_ptr(), taps.data_ptr(), out, mid, _stream()))
     _lib.check(code, "neck_conv")
     y = norm(y)
+    if y.shape != (B, H, W, mid) or y.dtype != x.dtype or not y.is_contiguous():
+        raise RuntimeError("samfast: the rows between the convolutions must keep their shape, dtype and order")
     z = torch.empty((B, H, W, out), dtype=x.dtype, device=x.device)
     code = _timed("neck_conv", 2.0 * B * H * W * out * 9 * mid, "flop", lambda: lib.samfast_neck_conv(
         y.data_ptr(), taps.data_ptr(), z.data_ptr(), B, H, W, mid, out, 9, _dtype_code(x), None, None, 0, 0, _stream()))

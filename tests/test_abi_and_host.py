@@ -593,3 +593,19 @@ def test_proj_block_launches_nothing_on_other_shapes(recorder):
                  (wq, sw, bias.bfloat16(), res, (norm, norm, 1e-6)), (wq[1:].clone(), sw, bias, res, (norm, norm, 1e-6))):
         assert ops.proj_block(x, *args) is None
     assert recorder.launches() == []
+
+
+def test_neck_launches_nothing_on_other_shapes(recorder):
+    from samfast_amd import ops
+    half = lambda *shape: torch.zeros(shape, dtype=torch.bfloat16)
+    x, w1, w3 = half(1, 4, 4, 128), half(64, 128, 1, 1), half(64, 64, 3, 3)
+    assert ops.neck_convs(x, w1, lambda y: y, w3).shape == (1, 4, 4, 64) and recorder.launches() == ["samfast_neck_conv"] * 2
+    recorder.called.clear()
+    for args in ((x, half(64, 64, 1, 1), w3), (x, half(64, 128, 3, 3), w3), (x, w1, half(64, 128, 3, 3)), (x, w1, half(64, 64, 1, 1)),
+                 (x, w1.float(), w3), (x.transpose(1, 2), w1, w3), (x, w1, w3.to(memory_format=torch.channels_last))):
+        with pytest.raises(RuntimeError):
+            ops.neck_convs(args[0], args[1], lambda y: y, args[2])
+    assert recorder.launches() == []
+    with pytest.raises(RuntimeError):
+        ops.neck_convs(x, w1, lambda y: y[:, :2], w3)
+    assert recorder.launches() == ["samfast_neck_conv"]

@@ -607,3 +607,16 @@ def test_a_caller_s_own_capture_outlives_the_recordings():
         torch.cuda.synchronize()
         assert torch.equal(out, want[i])
     assert all(k.isnan().all() for k in kept)
+
+
+@pytest.mark.parametrize("part,shape", [(0, (256, 64, 1, 1)), (0, (192, 128, 1, 1)), (2, (256, 192, 3, 3)), (2, (256, 256, 1, 1)), (1, (128,)), (3, (1,))])
+def test_neck_with_parameters_of_another_shape_is_called_as_modules(part, shape):
+    """Whatever the modules' own attributes say of them."""
+    from samfast_amd.modeling import ImageEncoderViT
+    enc = ImageEncoderViT(img_size=1024, embed_dim=128, depth=0, num_heads=2, use_rel_pos=True, window_size=14).cuda().to(torch.bfloat16).eval()
+    x = torch.zeros((1, 64, 64, 128), device="cuda", dtype=torch.bfloat16)
+    other = torch.nn.Parameter(torch.ones(shape, device="cuda", dtype=torch.bfloat16))
+    with torch.no_grad():
+        assert enc._neck_launchable(x)
+        setattr(enc.neck[part], "weight" if len(shape) > 1 else "bias", other)
+        assert not enc._neck_launchable(x)
