@@ -11,6 +11,7 @@ Nothing in the reference corresponds to this (it relies on torch.compile's CUDA 
 build_sam.py:95-141 `mode='max-autotune'`); it is the same idea without a tracing compiler.
 """
 
+import threading
 from collections import OrderedDict
 from typing import Optional
 
@@ -30,6 +31,7 @@ class GraphedEncoder(nn.Module):
         self.encoder = encoder
         self._in = example.clone()
         self._out: Optional[torch.Tensor] = None
+        self._stream = torch.cuda.current_stream()  # of the last call
         self._graph = torch.cuda.CUDAGraph()
         side = torch.cuda.Stream()  # default priority
         side.wait_stream(torch.cuda.current_stream())
@@ -41,11 +43,20 @@ class GraphedEncoder(nn.Module):
         with torch.no_grad(), torch.cuda.graph(self._graph):
             self._out = self.encoder(self._in)
 
+    def follow(self) -> None:
+        """Work enqueued on the current stream from here on comes behind the last call's, whichever stream that was on: the
+        buffers are the same ones."""
+        stream = torch.cuda.current_stream()
+        if stream != self._stream:
+            stream.wait_stream(self._stream)
+            self._stream = stream
+
     @torch.no_grad()
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if x.shape != self._in.shape or x.dtype != self._in.dtype:
             raise RuntimeError(f"samfast: GraphedEncoder was recorded for {tuple(self._in.shape)} "
                                f"{self._in.dtype}, got {tuple(x.shape)} {x.dtype}")
+        self.follow()
         if x is not self._in:
             self._in.copy_(x)
         self._graph.replay()
@@ -77,6 +88,9 @@ class ReplayedEncoder(nn.Module):
 
     max_rows = 4 * 4096
     max_graphs = 4
+    # Held by the thread that has a recording's buffers, from writing the input until the copy of the output is enqueued
+    # (one for all encoders: a module with a lock of its own could not be copied)
+    turn = threading.RLock()
 
     def __init__(self, encoder: nn.Module, compile_mode: Optional[str] = "max-autotune") -> None:
         super().__init__()
@@ -116,7 +130,7 @@ class ReplayedEncoder(nn.Module):
 
     def input_buffer(self, shape, dtype, device) -> Optional[torch.Tensor]:
         """The buffer that the recording for such an input reads, if there is one: an input written there on the current stream,
-        and then passed to forward, is not copied.  None where somebody beside forward is handed the input - a hook on this
+        and then passed to forward, is not copied (in one `turn`).  None where somebody beside forward is handed the input - a hook on this
         module or on every module, a forward of a subclass's or an instance's own - and might keep what the next image overwrites,
         and where forward would not replay: the encoder's own launches, recorded by the caller, would hold the address of a buffer
         that goes with this recording."""
@@ -124,21 +138,25 @@ class ReplayedEncoder(nn.Module):
                 or nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks):
             return None
         graph = self._graphs.get((tuple(shape), dtype, device))
-        return None if graph is None or not self.replays(graph._in) else graph._in
+        if graph is None or not self.replays(graph._in):
+            return None
+        graph.follow()
+        return graph._in
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not self.replays(x):
             return self._orig_mod(x)
         key = (tuple(x.shape), x.dtype, x.device)
-        graph = self._graphs.get(key)
-        if graph is None:
-            graph = GraphedEncoder(self._orig_mod, x)
-            self._graphs[key] = graph
-            while len(self._graphs) > self.max_graphs:
-                self._graphs.popitem(last=False)
-        else:
-            self._graphs.move_to_end(key)
-        return graph(x).clone()
+        with self.turn:
+            graph = self._graphs.get(key)
+            if graph is None:
+                graph = GraphedEncoder(self._orig_mod, x)
+                self._graphs[key] = graph
+                while len(self._graphs) > self.max_graphs:
+                    self._graphs.popitem(last=False)
+            else:
+                self._graphs.move_to_end(key)
+            return graph(x).clone()
 
 
 def invalidate_recordings(model: nn.Module) -> None:

@@ -45,20 +45,25 @@ class SamPredictor:
         self.input_size = tuple(transformed_image.shape[-2:])
         encoder = self.model.image_encoder
         dtype = next(encoder.parameters()).dtype
-        x = self._preprocessed(transformed_image, size, dtype)
-        self.features = encoder(self.model.preprocess(transformed_image).to(dtype) if x is None else x)
+        self.features = self._encoded(transformed_image, size, dtype)
         self.is_image_set = True
 
-    def _preprocessed(self, image: torch.Tensor, size: int, dtype: torch.dtype) -> Optional[torch.Tensor]:
-        """The encoder's input in one launch, in the buffer that a recorded encoder reads where there is one; None where
-        the model's own preprocess has to run (a class of its own, a method put in its place, an input the kernel
-        does not read)."""
+    def _encoded(self, image: torch.Tensor, size: int, dtype: torch.dtype) -> torch.Tensor:
+        encoder = self.model.image_encoder
+        if isinstance(encoder, ReplayedEncoder):
+            with encoder.turn:
+                buffer = encoder.input_buffer((image.shape[0], 3, size, size), dtype, image.device)
+                if buffer is not None and self._preprocessed(image, size, dtype, buffer) is buffer:
+                    return encoder(buffer)
+        x = self._preprocessed(image, size, dtype)
+        return encoder(self.model.preprocess(image).to(dtype) if x is None else x)
+
+    def _preprocessed(self, image: torch.Tensor, size: int, dtype: torch.dtype, buffer: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+        """The encoder's input in one launch, in `buffer` where given; None where the model's own preprocess has to run (a class
+        of its own, a method put in its place, an input the kernel does not read)."""
         model = self.model
         if type(model).preprocess is not Sam.preprocess or "preprocess" in model.__dict__:
             return None
-        buffer, encoder = None, model.image_encoder
-        if isinstance(encoder, ReplayedEncoder):
-            buffer = encoder.input_buffer((image.shape[0], 3, size, size), dtype, image.device)
         return ops.preprocess(image, model.pixel_mean, model.pixel_std, size, dtype, buffer)
 
     def get_image_embedding(self) -> torch.Tensor:

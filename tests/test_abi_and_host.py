@@ -5,6 +5,8 @@ reference's names and signatures; the product refuses to run without its kernels
 import ctypes
 import inspect
 import re
+import threading
+import time
 from pathlib import Path
 from types import SimpleNamespace
 
@@ -494,39 +496,87 @@ def test_copies_derived_from_a_buffer_are_kept_only_while_they_hold():
     assert copy_of(a) is made[4]
 
 
-@pytest.mark.parametrize("who", ["nobody", "hook", "pre-hook", "global hook", "global pre-hook", "own forward", "subclass", "capture", "eager"])
-def test_a_recording_s_input_buffer_is_written_only_where_nobody_is_handed_it(who, monkeypatch):
-    """A predictor writes the image straight into the buffer that a recorded encoder reads; whoever else would see that
-    tensor, overwritten by the next image, makes it a tensor of its own."""
+class _Recording:
+    """A GraphedEncoder's buffer and replay, without a GPU: the embedding is what the buffer holds."""
+
+    def __init__(self, shape):
+        self._in = SimpleNamespace(is_cuda=True, shape=shape, dim=lambda: 4, value=None, dtype=torch.bfloat16, device=torch.device("cuda", 0))
+
+    def follow(self):
+        pass
+
+    def __call__(self, x):
+        if x is not self._in:
+            self._in.value = x.value
+        time.sleep(1e-3)
+        value = self._in.value
+        return SimpleNamespace(clone=lambda: value)
+
+
+@pytest.fixture
+def predictor(monkeypatch):
+    """A predictor over an encoder with such a recording of one image; an image of value v gives the embedding v."""
     from samfast_amd import SamPredictor, ops
     from samfast_amd.graphs import ReplayedEncoder
     from samfast_amd.modeling import Sam
-    inner = torch.nn.Linear(1, 1)
-    inner.img_size = 64
-    encoder = ReplayedEncoder(inner).eval()
-    sam, device = Sam(encoder), torch.device("cuda", 0)
-    buffer = SimpleNamespace(is_cuda=True, shape=(1, 3, 64, 64), dim=lambda: 4)
-    encoder._graphs[((1, 3, 64, 64), torch.bfloat16, device)] = SimpleNamespace(_in=buffer)
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: who == "capture")
-    monkeypatch.setattr(ops, "preprocess", lambda image, mean, std, size, dtype, out: out)
-    image = SimpleNamespace(shape=(1, 3, 40, 64), device=device)
+    inner = torch.nn.Linear(1, 1, dtype=torch.bfloat16)
+    inner.img_size, inner.forward = 64, lambda x: x.value
+    encoder, recording = ReplayedEncoder(inner).eval(), _Recording((1, 3, 64, 64))
+    encoder._graphs[((1, 3, 64, 64), torch.bfloat16, torch.device("cuda", 0))] = recording
+
+    def preprocess(image, mean, std, size, dtype, out):
+        out = _Recording((1, 3, size, size))._in if out is None else out
+        out.value = image.value
+        written.append(out)
+        return out
+
+    written = []
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(ops, "preprocess", preprocess)
+    predictor = SamPredictor(Sam(encoder))
+    predictor.encode = lambda value: predictor._encoded(SimpleNamespace(shape=(1, 3, 40, 64), device=torch.device("cuda", 0), value=value), 64, torch.bfloat16)
+    predictor.written, predictor.buffer = written, recording._in
+    return predictor
+
+
+@pytest.mark.parametrize("who", ["nobody", "hook", "pre-hook", "global hook", "global pre-hook", "own forward", "subclass", "capture", "eager"])
+def test_a_recording_s_input_buffer_is_written_only_where_nobody_is_handed_it(who, predictor, monkeypatch):
+    """A predictor writes the image straight into the buffer that a recorded encoder reads; whoever else would see that
+    tensor, overwritten by the next image, makes it a tensor of its own."""
     from torch.nn.modules import module
+    encoder = predictor.model.image_encoder
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: who == "capture")
     handle = {"hook": encoder.register_forward_hook, "pre-hook": encoder.register_forward_pre_hook,
               "global hook": module.register_module_forward_hook,
               "global pre-hook": module.register_module_forward_pre_hook}.get(who, lambda f: None)(lambda *a: None)
     if who == "own forward":
-        encoder.forward = lambda x: x
+        encoder.forward = lambda x: x.value
     elif who == "subclass":
-        encoder.__class__ = type("Mine", (ReplayedEncoder,), {})
+        encoder.__class__ = type("Mine", (type(encoder),), {})
     elif who == "eager":
         encoder.compile_mode = None
     try:
         with torch.no_grad():
-            got = SamPredictor(sam)._preprocessed(image, 64, torch.bfloat16)
+            assert predictor.encode(7) == 7
     finally:
         if handle is not None:
             handle.remove()
-    assert got is (buffer if who == "nobody" else None)
+    assert [w is predictor.buffer for w in predictor.written] == [who == "nobody"]
+
+
+def test_threads_that_share_a_recorded_encoder_get_their_own_embeddings(predictor):
+    wrong = []
+
+    def work(value):
+        with torch.no_grad():
+            wrong.extend(i for i in range(20) if predictor.encode((value, i)) != (value, i))
+
+    threads = [threading.Thread(target=work, args=(v,)) for v in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == []
 
 
 class _Recorder:

@@ -620,3 +620,47 @@ def test_neck_with_parameters_of_another_shape_is_called_as_modules(part, shape)
         assert enc._neck_launchable(x)
         setattr(enc.neck[part], "weight" if len(shape) > 1 else "bias", other)
         assert not enc._neck_launchable(x)
+
+
+def test_streams_and_threads_that_share_a_recorded_encoder_get_their_own_embeddings():
+    import copy
+    import threading
+    import samfast_amd
+    from samfast_amd.modeling import ImageEncoderViT, Sam
+    from samfast_amd.graphs import ReplayedEncoder
+    torch.manual_seed(4)
+    enc = ImageEncoderViT(img_size=1024, embed_dim=128, depth=2, num_heads=2, use_rel_pos=True, window_size=14, global_attn_indexes=(1,))
+    sam = Sam(ReplayedEncoder(enc.to(torch.bfloat16).eval())).cuda().eval()
+    copy.deepcopy(sam)
+    images = [torch.randint(0, 256, (1, 3, 700, 1024), device="cuda", dtype=torch.uint8) for _ in range(3)]
+    with torch.no_grad():
+        want = [sam.image_encoder._orig_mod(sam.preprocess(i).to(torch.bfloat16)) for i in images]
+    pred = samfast_amd.SamPredictor(sam)
+    pred.set_torch_image(images[0], (700, 1024))  # records
+    torch.cuda.synchronize()
+    # one thread, two streams in turn, the host far ahead of either
+    streams, got = [torch.cuda.Stream() for _ in range(2)], []
+    for i in range(12):
+        with torch.cuda.stream(streams[i % 2]):
+            pred.set_torch_image(images[i % 3], (700, 1024))
+            got.append((i % 3, pred.get_image_embedding()))
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, want[i]) for i, y in got)
+    # a thread to a stream
+    got.clear()
+
+    def work(i):
+        mine = samfast_amd.SamPredictor(sam)
+        with torch.cuda.stream(streams[i]):
+            for _ in range(10):
+                mine.set_torch_image(images[i], (700, 1024))
+                got.append((i, mine.get_image_embedding()))
+            streams[i].synchronize()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert len(got) == 20 and all(torch.equal(y, want[i]) for i, y in got)
