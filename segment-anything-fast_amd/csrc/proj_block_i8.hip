@@ -189,11 +189,11 @@ __global__ __launch_bounds__(512) void proj_block_i8_kernel(ProjBlockArgs a) {
 }  // namespace samfast
 
 // While one workgroup per CU does it; the time hardly depends on the rows, so the wider W needs enough of them to be ahead.  us, three launches /
-// one: width 768, 16 rows 11.5 / 11.3, 1024 13.0 / 12.0, 2048 15.0 / 12.5, 4096 20.0 / 13.6, 4100 19.7 / 18.2, 8192 25.5 / 20.4, 8200 26.5 / 33.0; width 1024, 1024
-// rows 15.8 / 17.2, 2048 18.8 / 17.7, 4096 24.0 / 19.5, 4100 25.5 / 25.7, 5121 27.1 / 26.4, 8192 31.9 / 29.3, 8200 35.4 / 48.3.
+// one (medians of nine recordings of twenty, which spread by 1 %): width 768, 16 rows 11.1 / 11.0, 1024 12.5 / 11.8, 2048 14.5 / 12.3, 4096 19.7 / 13.3, 4097 19.8 / 17.8,
+// 6144 23.8 / 19.4, 8192 25.3 / 20.6, two rounds from 8193 on (8200 26.5 / 33.0); width 1024, 1024 rows 15.3 / 17.0, 1536 17.1 / 17.2, 1664 17.3 / 17.4, 1792 18.2 / 17.4, 3072 22.2 /
+// 18.5, 4096 24.2 / 20.3, 4100 26.0 / 26.0, 4224 26.3 / 25.5, 4608 26.9 / 26.3, 5120 26.7 / 25.6, 6144 28.5 / 27.3, 8192 32.7 / 30.2 (8200 35.4 / 48.3).
 extern "C" int samfast_proj_block_pays(int64_t M, int C) {
-  if (C == 768) return M <= 8192;
-  return C == 1024 && ((M > 1536 && M <= 4096) || (M > 4608 && M <= 8192));
+  return (C == 768 || (C == 1024 && M > 1664)) && M <= 8192;
 }
 
 extern "C" int samfast_proj_block_i8(const void* x, int64_t ldx, const int8_t* wq, const float* sw, const float* bias,

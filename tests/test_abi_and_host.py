@@ -496,6 +496,14 @@ def test_copies_derived_from_a_buffer_are_kept_only_while_they_hold():
     assert copy_of(a) is made[4]
 
 
+def test_proj_block_pays_on_one_range_of_rows():
+    from samfast_amd import _lib
+    lib = _lib.load()
+    for width, first in ((768, 0), (1024, 1665)):
+        assert [m for m in range(9000) if lib.samfast_proj_block_pays(m, width)] == list(range(first, 8193))
+    assert not any(lib.samfast_proj_block_pays(m, 1280) for m in (1, 4096))
+
+
 class _Recording:
     """A GraphedEncoder's buffer and replay, without a GPU: the embedding is what the buffer holds."""
 
