@@ -18,7 +18,7 @@
 // (2500 cycles) to arrive although only two are held.
 //
 // Epilogues: int8 (float(acc) * sx[m]) * sw[n] + bias[n] in three separately rounded fp32 operations, the half
-// types acc + bias[n]; rounded to the output type; then nothing, GELU of the rounded value, or + residual (one more
+// types acc + bias[n]; rounded to the output type; then nothing, (half types) GELU of the rounded value, or + residual (one more
 // rounding).  A wavefront's columns are dealt to the LDS rows so that a lane ends with four adjacent ones and stores
 // 128-byte segments straight from the accumulators, between the turns.  (Held in registers and sent out a few per turn of
 // the next tile, as gemm_i8_persist_kernel does, the stores lengthened every turn: 65536 x 1280 -> 3840 took 363 us for 310.)
@@ -356,8 +356,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
         unsigned int o = Out::pack2(y[0], y[1]);
         if constexpr (EPI == PP_GELU) {
           // activation of the rounded Linear output, as a separate GELU would see it
-          if constexpr (E::SCALED) o = Out::pack2(gelu_erf(Out::lo(o)), gelu_erf(Out::hi(o)));
-          else o = Out::pack2(gelu_value(Out::lo(o)), gelu_value(Out::hi(o)));
+          static_assert(!E::SCALED, "int8 products with GELU are other kernels'");
+          o = Out::pack2(gelu_value(Out::lo(o)), gelu_value(Out::hi(o)));
         }
         if constexpr (RES) o = Out::pack2(Out::lo(o) + Out::lo(v), Out::hi(o) + Out::hi(v));
         return o;
@@ -461,10 +461,10 @@ struct PPSplitTile {
   static constexpr int BM = 128, BN = 32 * TN;
   static constexpr int STAGE = (BM + BN) * 128;
   static constexpr int NST = TN == 3 ? 5 : 4;
-  static constexpr int SCALES = BM * 4 + 2 * ((BN + 63) / 64 * 64) * 4;
+  static constexpr int BIAS = 512;                    // bytes, two requests of 64 lanes
   static constexpr int LO = (TN + 1) / 2;             // loads of W per k tile for wavefronts 0-3 (two of X); 4-7: TN - LO
   static constexpr int N0 = TN == 3 ? 2 : 4;          // adjacent columns of a lane; the others (TN - N0: none or one) follow 16 N0 further on
-  static_assert(NST * STAGE + SCALES <= 160 * 1024 && 16 * TN * 1024 <= NST * STAGE, "LDS of a CU");
+  static_assert(NST * STAGE + BIAS <= 160 * 1024 && 16 * TN * 1024 <= NST * STAGE, "LDS of a CU");
 };
 
 template <class E, int EPI, int TN>
@@ -472,8 +472,9 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_split_kernel(PPArgs a) {
   typedef typename E::Out Out;
   using P = PPSplitTile<TN>;
   constexpr bool RES = EPI == PP_RESIDUAL, ONE = TN > P::N0;
+  static_assert(!E::SCALED, "half types");
   constexpr int NST = P::NST, N0 = P::N0, NP = N0 / 2;  // NP: pairs of a lane's adjacent columns
-  __shared__ __attribute__((aligned(16))) unsigned char lds[NST * P::STAGE + P::SCALES];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[NST * P::STAGE + P::BIAS];
   unsigned char* sc = lds + NST * P::STAGE;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -527,16 +528,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_split_kernel(PPArgs a) {
     __builtin_amdgcn_sched_barrier(0);  // the oldest operations in flight: no threshold below counts them
   }
 
-  // ---- scales and bias, 64 lanes of 4 bytes an instruction -----------------------------------------------------------
-  if constexpr (E::SCALED) {
-    constexpr int XS = P::BM / 64, WS = (P::BN + 63) / 64, SLICES = XS + 2 * WS;
-    static_assert(SLICES <= 8, "one slice per wavefront");
-    const int s = wave % SLICES, part = s < XS ? 0 : s < XS + WS ? 1 : 2, q = (part == 0 ? s : (s - XS) % WS) * 64;
-    const float* src = part == 0 ? a.sx + m0 : (part == 1 || !a.bias ? a.sw : reinterpret_cast<const float*>(a.bias)) + n0;
-    const int limit = part == 0 ? P::BM - 1 : P::BN - 1;
-    const int dst = (part == 0 ? 0 : P::BM * 4 + (part - 1) * WS * 256) + q * 4;
-    __builtin_amdgcn_global_load_lds((gptr_t)(src + min(q + lane, limit)), (lptr_t)(sc + dst), 4, 0, 0);
-  } else if (a.bias) {
+  // ---- bias, 64 lanes of 4 bytes an instruction ----------------------------------------------------------------------
+  if (a.bias) {
     // columns in pairs (N is even)
     const int q = (wave & 1) * 128;
     __builtin_amdgcn_global_load_lds((gptr_t)(reinterpret_cast<const unsigned short*>(a.bias) + n0 + min(q + 2 * lane, P::BN - 2)), (lptr_t)(sc + q * 2), 4, 0, 0);
@@ -658,37 +651,17 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_split_kernel(PPArgs a) {
 
   // ---- output ----------------------------------------------------------------------------------------------------------
   const bool full = skip_m == 0 && skip_n == 0;
-  constexpr int WPAD = (P::BN + 63) / 64 * 64;
-  float sw[TN], bias[TN];
+  float bias[TN];
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     const int col = j < N0 ? col0 + j : wn * 16 * TN + 16 * N0 + lr;
-    if constexpr (E::SCALED) {
-      sw[j] = reinterpret_cast<const float*>(sc + P::BM * 4)[col];
-      bias[j] = a.bias ? reinterpret_cast<const float*>(sc + P::BM * 4)[WPAD + col] : 0.f;
-    } else {
-      bias[j] = a.bias ? Out::lo((unsigned int)reinterpret_cast<const unsigned short*>(sc)[col]) : 0.f;
-    }
+    bias[j] = a.bias ? Out::lo((unsigned int)reinterpret_cast<const unsigned short*>(sc)[col]) : 0.f;
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    f32x4 sx;
-    if constexpr (E::SCALED) sx = *reinterpret_cast<const f32x4*>(sc + (row0 + 16 * i) * 4);
-    auto value = [&](int j, int r) __attribute__((always_inline)) {
-      if constexpr (E::SCALED) {
-        // three separately rounded fp32 operations (no fused multiply-add)
-        float t = (float)acc[i][j][r] * sx[r];
-        t = t * sw[j];
-        return t + bias[j];
-      } else {
-        return acc[i][j][r] + bias[j];
-      }
-    };
+    auto value = [&](int j, int r) __attribute__((always_inline)) { return acc[i][j][r] + bias[j]; };
     auto last_step = [&](unsigned int o, unsigned int v) __attribute__((always_inline)) {
-      if constexpr (EPI == PP_GELU) {
-        if constexpr (E::SCALED) o = Out::pack2(gelu_erf(Out::lo(o)), gelu_erf(Out::hi(o)));
-        else o = Out::pack2(gelu_value(Out::lo(o)), gelu_value(Out::hi(o)));
-      }
+      if constexpr (EPI == PP_GELU) o = Out::pack2(gelu_value(Out::lo(o)), gelu_value(Out::hi(o)));
       if constexpr (RES) o = Out::pack2(Out::lo(o) + Out::lo(v), Out::hi(o) + Out::hi(v));
       return o;
     };
