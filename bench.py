@@ -239,9 +239,16 @@ def mfma_ceiling():
     res = {"what": "8 independent MFMAs per round and wavefront, operands in registers, 512 workgroups of "
                    "4 wavefronts (2 wavefronts per SIMD on 256 CUs), ~40 ms per launch, events on the launch stream",
            "int8_v_mfma_i32_32x32x32_i8": {"unit": "POP/s", "published_peak": 5.0},
-           "bf16_v_mfma_f32_32x32x16_bf16": {"unit": "PFLOP/s", "published_peak": 2.5}}
+           "bf16_v_mfma_f32_32x32x16_bf16": {"unit": "PFLOP/s", "published_peak": 2.5},
+           "int8_v_mfma_i32_16x16x64_i8": {"unit": "POP/s", "published_peak": 5.0},
+           "bf16_v_mfma_f32_16x16x32_bf16": {"unit": "PFLOP/s", "published_peak": 2.5}}
+    operands[1]["random_normal_half"] = operands[1]["random_normal"] * 0.5
+    for small, instr in ((2, 0), (3, 1)):  # the 16 x 16 forms, on the same buffers
+        operands[small] = {name: operands[instr][name] for name in ("zeros", "gaussian_codes", "random_normal", "random_normal_half")
+                           if name in operands[instr]}
     stream = torch.cuda.current_stream().cuda_stream
-    for instr, key, iters in ((0, "int8_v_mfma_i32_32x32x32_i8", 120000), (1, "bf16_v_mfma_f32_32x32x16_bf16", 100000)):
+    for instr, key, iters in ((0, "int8_v_mfma_i32_32x32x32_i8", 120000), (1, "bf16_v_mfma_f32_32x32x16_bf16", 100000),
+                              (2, "int8_v_mfma_i32_16x16x64_i8", 240000), (3, "bf16_v_mfma_f32_16x16x32_bf16", 200000)):
         for name, buf in operands[instr].items():
             ops = ctypes.c_int64(0)
             launch = lambda: _lib.check(lib.samfast_bench_mfma_ceiling(

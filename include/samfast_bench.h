@@ -33,7 +33,7 @@ int samfast_bench_set_knob(const char* name, int value, int unset);
  * but matrix instructions on operands held in registers (no global loads, no LDS, no barriers)
  * - the rate a GEMM or attention kernel built from the same instruction can approach at best
  * on the same kind of data.  instruction 0 = v_mfma_i32_32x32x32_i8, 1 =
- * v_mfma_f32_32x32x16_bf16.  `operands` holds 4 (A, B) pairs of 16 bytes for each of 256 lanes
+ * v_mfma_f32_32x32x16_bf16, 2 = v_mfma_i32_16x16x64_i8, 3 = v_mfma_f32_16x16x32_bf16.  `operands` holds 4 (A, B) pairs of 16 bytes for each of 256 lanes
  * (8 * 256 * 16 bytes, [pair][A|B][lane]); their values decide what the multipliers toggle.
  * `workgroups` of 256 threads run `iters` rounds of 8 independent instructions per wavefront
  * (workgroups * iters <= 2^27, about a second of GPU time; more returns SAMFAST_E_INVALID);

@@ -20,10 +20,42 @@ namespace samfast {
 constexpr int kCeilSets = 8;   // independent accumulator sets per wavefront
 constexpr int kCeilPairs = 4;  // distinct (A, B) operand pairs per lane
 
+// The instructions, by the number the entry point takes: result type, its words, operations of one instruction.
+template <int> struct CeilInstr;
+template <> struct CeilInstr<0> {
+  typedef i32x16 acc_t;
+  static constexpr int WORDS = 16, OPS = 2 * 32 * 32 * 32;
+  static SF_DEVICE acc_t mma(u32x4 a, u32x4 b, acc_t c) {
+    return __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, a), __builtin_bit_cast(i32x4, b), c, 0, 0, 0);
+  }
+};
+template <> struct CeilInstr<1> {
+  typedef f32x16 acc_t;
+  static constexpr int WORDS = 16, OPS = 2 * 32 * 32 * 16;
+  static SF_DEVICE acc_t mma(u32x4 a, u32x4 b, acc_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+};
+template <> struct CeilInstr<2> {
+  typedef i32x4 acc_t;
+  static constexpr int WORDS = 4, OPS = 2 * 16 * 16 * 64;
+  static SF_DEVICE acc_t mma(u32x4 a, u32x4 b, acc_t c) {
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, a), __builtin_bit_cast(i32x4, b), c, 0, 0, 0);
+  }
+};
+template <> struct CeilInstr<3> {
+  typedef f32x4 acc_t;
+  static constexpr int WORDS = 4, OPS = 2 * 16 * 16 * 32;
+  static SF_DEVICE acc_t mma(u32x4 a, u32x4 b, acc_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+};
+
 // operands: (kCeilPairs, 2, 256) 16-byte vectors, indexed [pair][a|b][thread of the workgroup]
-template <bool INT8>
+template <int I>
 __global__ __launch_bounds__(256, 2) void mfma_ceiling_kernel(const u32x4* __restrict__ operands,
                                                                int iters, int* out) {
+  using L = CeilInstr<I>;
   const int tid = threadIdx.x;
   u32x4 av[kCeilPairs], bv[kCeilPairs];
 #pragma unroll
@@ -32,41 +64,20 @@ __global__ __launch_bounds__(256, 2) void mfma_ceiling_kernel(const u32x4* __res
     bv[p] = operands[(2 * p + 1) * 256 + tid];
   }
   int check = 0;
-  if constexpr (INT8) {
-    i32x16 acc[kCeilSets];
+  typename L::acc_t acc[kCeilSets];
 #pragma unroll
-    for (int j = 0; j < kCeilSets; ++j)
+  for (int j = 0; j < kCeilSets; ++j) acc[j] = typename L::acc_t{};
+  for (int it = 0; it < iters; ++it) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[j][r] = 0;
-    for (int it = 0; it < iters; ++it) {
-#pragma unroll
-      for (int j = 0; j < kCeilSets; ++j)
-        acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, av[j % kCeilPairs]),
-                                                       __builtin_bit_cast(i32x4, bv[(j + j / kCeilPairs) % kCeilPairs]),
-                                                       acc[j], 0, 0, 0);
-    }
-#pragma unroll
-    for (int j = 0; j < kCeilSets; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) check ^= acc[j][r];
-  } else {
-    f32x16 acc[kCeilSets];
-#pragma unroll
-    for (int j = 0; j < kCeilSets; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
-    for (int it = 0; it < iters; ++it) {
-#pragma unroll
-      for (int j = 0; j < kCeilSets; ++j)
-        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av[j % kCeilPairs]),
-                                                         __builtin_bit_cast(bf16x8, bv[(j + j / kCeilPairs) % kCeilPairs]),
-                                                         acc[j], 0, 0, 0);
-    }
-#pragma unroll
-    for (int j = 0; j < kCeilSets; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) check ^= __float_as_int(acc[j][r]);
+    for (int j = 0; j < kCeilSets; ++j) acc[j] = L::mma(av[j % kCeilPairs], bv[(j + j / kCeilPairs) % kCeilPairs], acc[j]);
   }
+#pragma unroll
+  for (int j = 0; j < kCeilSets; ++j)
+#pragma unroll
+    for (int r = 0; r < L::WORDS; ++r) {
+      const auto v = acc[j][r];
+      check ^= __builtin_bit_cast(int, v);
+    }
   if (check == 0x5a17c0de) out[tid] = check;
 }
 
@@ -145,7 +156,7 @@ extern "C" int samfast_bench_mfma_valu_overlap(int vector_kind, const void* oper
 extern "C" int samfast_bench_mfma_ceiling(int instruction, const void* operands, int workgroups,
                                           int iters, int64_t* host_ops_out, void* scratch_out, void* stream) {
   using namespace samfast;
-  SF_REQUIRE(instruction == 0 || instruction == 1, "bench_mfma_ceiling: instruction must be 0 (int8) or 1 (bf16)");
+  SF_REQUIRE(instruction >= 0 && instruction <= 3, "bench_mfma_ceiling: instruction must be 0 or 2 (int8), 1 or 3 (bf16)");
   SF_REQUIRE(operands && scratch_out && aligned16(operands), "bench_mfma_ceiling: null or unaligned buffer");
   SF_REQUIRE(workgroups > 0 && workgroups <= (1 << 20) && iters > 0 && iters <= (1 << 24),
              "bench_mfma_ceiling: bad workgroup or iteration count");
@@ -153,12 +164,20 @@ extern "C" int samfast_bench_mfma_ceiling(int instruction, const void* operands,
   SF_REQUIRE((int64_t)workgroups * iters <= (1ll << 27), "bench_mfma_ceiling: workgroups * iters must not exceed 2^27");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const u32x4* ops = reinterpret_cast<const u32x4*>(operands);
-  if (instruction == 0)
-    hipLaunchKernelGGL((mfma_ceiling_kernel<true>), dim3(workgroups), dim3(256), 0, s, ops, iters, (int*)scratch_out);
-  else
-    hipLaunchKernelGGL((mfma_ceiling_kernel<false>), dim3(workgroups), dim3(256), 0, s, ops, iters, (int*)scratch_out);
-  // arithmetic operations the launch executes: 2 * 32 * 32 * k per MFMA, k = 32 (int8) or 16 (bf16)
-  if (host_ops_out)
-    *host_ops_out = (int64_t)workgroups * 4 * iters * kCeilSets * 2 * 32 * 32 * (instruction == 0 ? 32 : 16);
+  int instruction_ops = 0;
+#define SF_CEIL(I)                                                                                             \
+  case I:                                                                                                      \
+    hipLaunchKernelGGL((mfma_ceiling_kernel<I>), dim3(workgroups), dim3(256), 0, s, ops, iters, (int*)scratch_out); \
+    instruction_ops = CeilInstr<I>::OPS;                                                                       \
+    break
+  switch (instruction) {
+    SF_CEIL(0);
+    SF_CEIL(1);
+    SF_CEIL(2);
+    SF_CEIL(3);
+  }
+#undef SF_CEIL
+  // arithmetic operations the launch executes
+  if (host_ops_out) *host_ops_out = (int64_t)workgroups * 4 * iters * kCeilSets * instruction_ops;
   return check_launch("mfma_ceiling_kernel");
 }

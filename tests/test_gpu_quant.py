@@ -840,3 +840,21 @@ def test_measurement_aids_run_and_check_their_arguments():
     assert lib.samfast_bench_mfma_valu_overlap(2, buf.data_ptr(), 8, 1, 1, out.data_ptr(), stream) == -1  # SAMFAST_E_INVALID
     assert lib.samfast_bench_mfma_valu_overlap(0, None, 8, 1, 1, out.data_ptr(), stream) == -1  # SAMFAST_E_INVALID
     assert lib.samfast_bench_mfma_valu_overlap(0, buf.data_ptr(), 8, -1, 1, out.data_ptr(), stream) == -1  # SAMFAST_E_INVALID
+
+
+def test_matrix_loops_of_either_shape_count_their_operations():
+    import ctypes
+    from samfast_amd import _lib
+    lib = _lib.load()
+    buf = torch.randn(8 * 256 * 8, device="cuda").to(torch.bfloat16)
+    out = torch.zeros(1024, dtype=torch.int32, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    done = ctypes.c_int64(0)
+    for instr, per in enumerate((2 * 32 * 32 * 32, 2 * 32 * 32 * 16, 2 * 16 * 16 * 64, 2 * 16 * 16 * 32)):
+        print(f"case matrix loop {instr}", flush=True)
+        assert lib.samfast_bench_mfma_ceiling(instr, buf.data_ptr(), 8, 10, ctypes.byref(done), out.data_ptr(), stream) == 0
+        assert done.value == 8 * 4 * 10 * 8 * per
+    torch.cuda.synchronize()
+    assert not out.any()  # the kernels write nothing
+    for bad in (-1, 4):
+        assert lib.samfast_bench_mfma_ceiling(bad, buf.data_ptr(), 8, 10, None, out.data_ptr(), stream) == -1
