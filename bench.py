@@ -335,12 +335,32 @@ def mfma_ceiling():
 def gemm_variants(batch=16, width=1280):
     """The four Linears of a ViT-H block at batch * 4096 rows (K-block major operands, the epilogue the
     encoder uses) under each variant of the int8 GEMM kernel, ten launches back to back after three
-    warm-up launches, events on the launch stream; on all-zero codes (no operand toggling: the clock
+    warm-up launches, events on the launch stream, the variants in turn and the median of five turns (the clock
+    a variant meets depends on what ran before it); on all-zero codes (no operand toggling: the clock
     stays up, what is left is the kernel's structure) and on Gaussian codes like the encoder's."""
     import torch
     from samfast_amd import _lib, ops
     dev = torch.device("cuda:0")
     M = batch * 4096
+
+    def in_turn(variants, run):
+        """{variant: us per launch}"""
+        us = {label: [] for label, _ in variants}
+        for _ in range(5):
+            for label, knobs in variants:
+                with _lib.knobs(**knobs):
+                    for _ in range(3):
+                        run()
+                    torch.cuda.synchronize()
+                    e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                    e0.record()
+                    for _ in range(10):
+                        run()
+                    e1.record()
+                    torch.cuda.synchronize()
+                us[label].append(e0.elapsed_time(e1) * 100.0)
+        return {label: sorted(v)[2] for label, v in us.items()}
+
     g = torch.Generator(device="cuda").manual_seed(11)
     variants = [("256-row tiles by turns, where they pay (the default)", {}),
                 ("three_workgroups_per_cu", {"SAMFAST_GEMM_PINGPONG": 0, "SAMFAST_GEMM_PERSIST": 0}),
@@ -350,7 +370,7 @@ def gemm_variants(batch=16, width=1280):
                 ("persistent, skewed, no wave priorities", {"SAMFAST_GEMM_PERSIST": 2, "SAMFAST_GEMM_PERSIST_PRIO": 0})]
     shapes = [("qkv", 3 * width, width, _lib.EPILOGUE_NONE), ("proj", width, width, _lib.EPILOGUE_RESIDUAL),
               ("lin1", 4 * width, width, _lib.EPILOGUE_NONE), ("lin2", width, 4 * width, _lib.EPILOGUE_RESIDUAL)]
-    res = {"what": f"gemm_i8 at M={M}, us per launch (10 back to back) and TOP/s, per variant knob, on "
+    res = {"what": f"gemm_i8 at M={M}, us per launch (10 back to back, median of 5 in turn) and TOP/s, per variant knob, on "
                    "all-zero / Gaussian int8 codes", "rows": {}}
     for name, N, K, epi in shapes:
         sx = torch.full((M,), 0.01, device=dev)
@@ -367,18 +387,7 @@ def gemm_variants(batch=16, width=1280):
                 xq = (torch.randn((K // 64, M, 64), device=dev, generator=g) * 28).round().clamp(-127, 127).to(torch.int8)
                 wq = (torch.randn((K // 64, N, 64), device=dev, generator=g) * 28).round().clamp(-127, 127).to(torch.int8)
             run = lambda: ops.gemm_i8_fused(xq, sx, wq, sw, bias, epi, residual=resid, out=y, layout=_lib.LAYOUT_KB64)
-            for label, knobs in variants:
-                with _lib.knobs(**knobs):
-                    for _ in range(3):
-                        run()
-                    torch.cuda.synchronize()
-                    e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-                    e0.record()
-                    for _ in range(10):
-                        run()
-                    e1.record()
-                    torch.cuda.synchronize()
-                us = e0.elapsed_time(e1) * 100.0
+            for label, us in in_turn(variants, run).items():
                 row.setdefault(label, {})[data] = {"us": round(us, 1), "TOP/s": round(2.0 * M * N * K / us / 1e6, 1)}
             del xq, wq
         res["rows"][f"{name} {M}x{N}x{K}"] = row
@@ -399,20 +408,8 @@ def gemm_variants(batch=16, width=1280):
         xq = (torch.randn((K // 64, M, 64), device=dev, generator=g) * 28).round().clamp(-127, 127).to(torch.int8)
         run = lambda: ops.gemm_i8_sparse24_fused(xq, sx, wc, widx, sw, bias, epi, residual=resid, out=y,
                                                  layout=_lib.LAYOUT_KB64)
-        row = {}
-        for label, knobs in sparse_variants:
-            with _lib.knobs(**knobs):
-                for _ in range(3):
-                    run()
-                torch.cuda.synchronize()
-                e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-                e0.record()
-                for _ in range(10):
-                    run()
-                e1.record()
-                torch.cuda.synchronize()
-            us = e0.elapsed_time(e1) * 100.0
-            row[label] = {"gaussian": {"us": round(us, 1), "TOP/s executed": round(1.0 * M * N * K / us / 1e6, 1)}}
+        row = {label: {"gaussian": {"us": round(us, 1), "TOP/s executed": round(1.0 * M * N * K / us / 1e6, 1)}}
+               for label, us in in_turn(sparse_variants, run).items()}
         res["rows"][f"2:4 {name} {M}x{N}x{K}"] = row
         del y, resid, xq, wc, widx
     torch.cuda.empty_cache()
