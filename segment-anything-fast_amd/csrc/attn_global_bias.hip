@@ -6,9 +6,9 @@
 // matrix instructions of the next half row's scores and of the previous one's P V, and the LDS reads that feed
 // them.  No running maximum is taken in the common case, LDS reads meet no bank twice (GridRow), and the
 // workgroups of a head touch its K and V ahead, so that the rows come out of their XCD's L2.
-//   Bound: at 8 x 16 x 4096 x 80 (fp16 760 us, 900 TFLOP/s, bf16 710; fp16 805 with attn_global_kernel) the power limit:
-//   the same loop with its MFMAs alone, on the same values, takes 666 us - 429 on zeros.  At one image of 12 heads
-//   (65 us against 83) the last, half-empty round and the prologue.
+//   Bound: at 8 x 16 x 4096 x 80 (fp16 785 us, 875 TFLOP/s, bf16 711; attn_global_kernel 803 and 763) the power limit:
+//   the same loop with its MFMAs alone, on the same values, took 666 us - 429 on zeros (probes that are not kept).  At one image of
+//   12 heads (65 us against 82) the last, half-empty round and the prologue.
 //   (The encoder, which hands over tables, keeps attn_global_kernel: its int8 Linears turn any other order of these
 //   roundings into other codes.)
 //

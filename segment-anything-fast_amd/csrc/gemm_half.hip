@@ -18,6 +18,9 @@ namespace samfast {
 //     Else 256 x 256, on long loops within one round from 0.7 on (12288 x 5120 -> 1280 138 / 132; 0.5: 8192 x 4096 -> 1024 69 / 83, two
 //     rounds: 32768 x 4096 -> 1024 236 / 248), on short ones up to four rounds from 0.75 on (12288 x 1024 -> 1024 42.6 / 40.4, 32768 x
 //     1280 -> 1280 181 / 147; 0.5: 8192 x 1024 -> 1024 31.1 / 33.9, five rounds: 65536 x 1280 -> 1280 276 / 284).
+// The rows decide, so the order in which a product's terms are summed, and with it the last bits of an image's embedding in the half
+// types, follows the batch, as it does with the library's kernels (one ViT-H image: 3-5 split K, five ViT-L images: 320-row tiles, the
+// library in between; 0.016 and 2e-4 of the embedding's norm).  int8 sums are integers: an image comes out the same in any batch.
 constexpr int kHalfTall = 58;  // 320 rows, 256 columns
 static int half_choose(int64_t M, int N, int K, int epi) {
   const int force = knob_or(KNOB_GEMM_HALF, 1);

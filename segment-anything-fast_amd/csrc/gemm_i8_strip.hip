@@ -7,7 +7,7 @@
 // gives 56 bytes a cycle; fragments straight into registers, 16 bytes of each of 16 rows to a quarter of the lanes, 33).
 // The columns of a fragment pair are dealt so that a lane ends with eight adjacent ones: stores without a turn through LDS.
 // us, 64 x 128 tiles / this one, K-block-major operands: 4096 x 768 -> 3072 18.9 / 16.8, 4900 x 768 -> 2304 17.8 / 16.4, 8192 x 768 -> 1536 18.6 /
-// 16.7; one image of ViT-B 1396 / 1378.  Without GELU the other members are level (15.4 / 15.2, 13.9 / 14.1, 14.9 / 14.6): not built.
+// 16.7; one image of ViT-B, twelve of these launches, 1474 / 1466 (medians of fifteen turns).  Without GELU the other members are level (15.4 / 15.2, 13.9 / 14.1, 14.9 / 14.6): not built.
 // Integer sums and the epilogue's arithmetic are those of the other members: the same bits.
 #include "attn_relpos_shared.hpp"
 #include "gemm_i8_shared.hpp"

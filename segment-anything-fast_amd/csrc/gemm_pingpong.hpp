@@ -1,13 +1,15 @@
 // One matrix product y = x . w^T for the element types of this library (int8, bf16, fp16): output tiles of 256 rows and 256 or 320
 // columns, or 320 rows and 256 columns, one resident workgroup of eight wavefronts per CU, two per SIMD that take turns at the matrix pipe.
 //
-// What bounds it is power, not the matrix pipe.  The pipe is busy 0.93-0.96 of the loop's cycles, and on operands
-// like an encoder's the clock settles at 1.5-1.7 GHz of 2.4, so every choice here is about energy per product or
-// about cycles in which nothing is multiplied:
-//   * v_mfma_*_16x16x(64 bytes): bare loops of them sustain 3.9 POP/s on Gaussian codes (bf16: 1.93 PFLOP/s) where the
-//     32x32 forms sustain 3.5 (1.8): half the accumulator bytes per product cross the register file;
-//   * 256 x 256 tiles: a third fewer operand bytes from the L2s than 128 x 256 (the loads are 17 % of the energy, the
-//     LDS reads 7 %: loops without them run that much faster at the same pipe occupancy);
+// What bounds it, at 65536 x 1280 -> 3840 in int8 (284 us inside an encoder; 215 on all-zero codes, where no power limit acts): the products
+// alone are 163 us at the rate that bare loops of the same instruction sustain under the power limit on codes like an encoder's
+// (139 on zeros), and the rest is the tiles' ends, in which nothing is multiplied: every CU rounds and stores its tile at the same time, 0.5 GB
+// in fifteen bursts.  (The pipe is busy 0.56 of whole launches, at 2.0 GHz of 2.4, and 0.93-0.96 of the loop: the latter by a
+// cycle counter in a probe that is not kept.)  So the choices here are about energy per product, or about cycles without products:
+//   * v_mfma_*_16x16x(64 bytes): bare loops of them (bench.py --mfma-ceiling) sustain 3.95 POP/s on Gaussian codes (bf16: 1.93 PFLOP/s)
+//     where the 32x32 forms sustain 3.5 (1.8): half the accumulator bytes per product cross the register file;
+//   * 256 x 256 tiles: a third fewer operand bytes from the L2s than 128 x 256 (loops without the loads ran 17 % faster at the
+//     same pipe occupancy, without the LDS reads 7 %: probes that are not kept);
 //   * turns: the wavefronts 0-3 multiply while 4-7 (their SIMD partners) read fragments and request tiles, and
 //     the other way round, a barrier between turns of 32 matrix instructions.  The same code with both halves in
 //     step keeps the pipe busy 0.59 of the time.
@@ -23,8 +25,8 @@
 // 128-byte segments straight from the accumulators, between the turns.  (Held in registers and sent out a few per turn of
 // the next tile, as gemm_i8_persist_kernel does, the stores lengthened every turn: 65536 x 1280 -> 3840 took 363 us for 310.)
 //
-// Inside the ViT-H encoder at 65536 rows, us per launch, before / with this kernel: 1280 -> 3840 309 / 263 (2.45 POP/s), 5120 -> 1280 with
-// the residual 404 / 337 (2.55), 1280 -> 1280 with it 136 / 135 (0.4 GB of rows through HBM).
+// Inside the ViT-H encoder at 65536 rows, us per launch (means of a kernel trace), before / with this kernel: 1280 -> 3840 309 / 284 (2.27 POP/s),
+// 1280 -> 5120 376 (2.28), 5120 -> 1280 with the residual 404 / 335 (2.56), 1280 -> 1280 with it 136 / 137 (0.4 GB of rows through HBM).
 #pragma once
 
 #include "gemm_i8_shared.hpp"
@@ -694,7 +696,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_split_kernel(PPArgs a) {
 // Time of a launch in units of one 16-column fragment of 64 rows for one k tile: rounds of the CUs, each as long as its k tiles and a start
 // and an end worth eight more of them, a tile two or three and a half fragments more expensive than its columns.  The tile with the
 // least; `used`: the share of those CU-cycles that makes output.
-// us, 256 / 320 columns: int8 inside the encoder 65536 x 1280 -> 3840 263 / 301; 4096 x 1280 -> 5120 (320 / 256 tiles) 33.0 / 28.1, 8192 x 1280 ->
+// us, 256 / 320 columns: int8 inside the encoder 65536 x 1280 -> 3840 284 / 301; 4096 x 1280 -> 5120 (320 / 256 tiles) 33.0 / 28.1, 8192 x 1280 ->
 // 5120 (three / two rounds) 57.7 / 52.6, 20480 x 1280 -> 5120 (seven / five) 129.5 / 124.1.  (192 columns, at an
 // equal number of columns per CU, lost: 65536 x 1280 -> 3840 284 / 305, 4096 x 1024 -> 3072 17.5 / 18.3.)
 // The residual's registers leave no room for 320 columns, but for 320 rows, which few columns and many rows fill better.  256 / 320
