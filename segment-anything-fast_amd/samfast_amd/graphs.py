@@ -49,6 +49,7 @@ class GraphedEncoder(nn.Module):
         stream = torch.cuda.current_stream()
         if stream != self._stream:
             stream.wait_stream(self._stream)
+            self._in.record_stream(stream)  # (a recording may be dropped while its last replay is under way)
             self._stream = stream
 
     @torch.no_grad()

@@ -667,3 +667,22 @@ def test_neck_launches_nothing_on_other_shapes(recorder):
     with pytest.raises(RuntimeError):
         ops.neck_convs(x, w1, lambda y: y[:, :2], w3)
     assert recorder.launches() == ["samfast_neck_conv"]
+
+
+def test_a_recording_follows_the_stream_of_its_last_call(monkeypatch):
+    """Another stream waits for the last one's work, and the input buffer is known to the allocator as used there."""
+    from samfast_amd.graphs import GraphedEncoder
+
+    class Stream:
+        def wait_stream(self, other):
+            seen.append(("waits for", self, other))
+
+    seen, streams = [], [Stream(), Stream()]
+    recording = GraphedEncoder.__new__(GraphedEncoder)
+    nn.Module.__init__(recording)
+    recording._in, recording._stream = SimpleNamespace(record_stream=lambda s: seen.append(("used on", s))), streams[0]
+    for i in (0, 1, 1, 0):
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda: streams[i])
+        recording.follow()
+    assert seen == [("waits for", streams[1], streams[0]), ("used on", streams[1]),
+                    ("waits for", streams[0], streams[1]), ("used on", streams[0])]
