@@ -1,11 +1,12 @@
 // One matrix product y = x . w^T for the element types of this library (int8, bf16, fp16): output tiles of 256 rows and 256 or 320
 // columns, or 320 rows and 256 columns, one resident workgroup of eight wavefronts per CU, two per SIMD that take turns at the matrix pipe.
 //
-// What bounds it, at 65536 x 1280 -> 3840 in int8 (284 us inside an encoder; 215 on all-zero codes, where no power limit acts): the products
+// What bounds it, at 65536 x 1280 -> 3840 in int8 (265 us; 197 on all-zero codes, where no power limit acts): the products
 // alone are 163 us at the rate that bare loops of the same instruction sustain under the power limit on codes like an encoder's
-// (139 on zeros), and the rest is the tiles' ends, in which nothing is multiplied: every CU rounds and stores its tile at the same time, 0.5 GB
-// in fifteen bursts.  (The pipe is busy 0.56 of whole launches, at 2.0 GHz of 2.4, and 0.93-0.96 of the loop: the latter by a
-// cycle counter in a probe that is not kept.)  So the choices here are about energy per product, or about cycles without products:
+// (139 on zeros), and the rest is the tiles' ends, in which hardly anything is multiplied: four and a half vector instructions per value
+// (eight with the residual), four cycles each, are 5400 cycles of a SIMD beside the loop's 21000.  (Not the burst of stores: the CUs or
+// XCDs started up to half a tile's time apart took the same 198-206 us on zeros.  Cycle counts by probes that are not kept; the
+// pipe is busy 0.93-0.96 of the loop.)  So the choices here are about energy per product, or about cycles without products:
 //   * v_mfma_*_16x16x(64 bytes): bare loops of them (bench.py --mfma-ceiling) sustain 3.95 POP/s on Gaussian codes (bf16: 1.93 PFLOP/s)
 //     where the 32x32 forms sustain 3.5 (1.8): half the accumulator bytes per product cross the register file;
 //   * 256 x 256 tiles: a third fewer operand bytes from the L2s than 128 x 256 (loops without the loads ran 17 % faster at the
@@ -22,11 +23,14 @@
 // Epilogues: int8 (float(acc) * sx[m]) * sw[n] + bias[n] in three separately rounded fp32 operations, the half
 // types acc + bias[n]; rounded to the output type; then nothing, (half types) GELU of the rounded value, or + residual (one more
 // rounding).  A wavefront's columns are dealt to the LDS rows so that a lane ends with four adjacent ones and stores
-// 128-byte segments straight from the accumulators, between the turns.  (Held in registers and sent out a few per turn of
+// 128-byte segments straight from the accumulators, between the turns, both sides at once: a wavefront alone issues an instruction every
+// 5.2 cycles, two together one every 4.3.  (One side behind the other, and with every store's address made anew, 1045 instead of 676
+// instructions, an end was 10800 cycles for now 6300: 65536 x 1280 -> 3840 292 -> 265 us, -> 5120 373 -> 347, 1280 -> 1280 with the residual
+// 134.5 -> 126, 20480 x 1024 -> 3072 70 -> 60, bf16 20480 x 1024 -> 4096 with GELU 167 -> 155.)  (Held in registers and sent out a few per turn of
 // the next tile, as gemm_i8_persist_kernel does, the stores lengthened every turn: 65536 x 1280 -> 3840 took 363 us for 310.)
 //
-// Inside the ViT-H encoder at 65536 rows, us per launch (means of a kernel trace), before / with this kernel: 1280 -> 3840 309 / 284 (2.27 POP/s),
-// 1280 -> 5120 376 (2.28), 5120 -> 1280 with the residual 404 / 335 (2.56), 1280 -> 1280 with it 136 / 137 (0.4 GB of rows through HBM).
+// Inside the ViT-H encoder at 65536 rows, us per launch (means of a kernel trace), before / with this kernel: 1280 -> 3840 309 / 261 (2.47 POP/s),
+// 1280 -> 5120 345 (2.49), 5120 -> 1280 with the residual 404 / 324 (2.65), 1280 -> 1280 with it 136 / 127 (0.4 GB of rows through HBM).
 #pragma once
 
 #include "gemm_i8_shared.hpp"
@@ -275,22 +279,33 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
   // ---- output: rows 16 (TM wm + i) + 4 lq + r, quads and pair of columns from col0 on ------------------------------
   typedef __attribute__((address_space(1))) unsigned char* gbyte_t;
   const int col0 = wn * 16 * TN;
-  // address of row 16 i + r, group g of this lane in the tile at `tile` (uniform base, 32-bit lane offset; the pitch is
-  // made opaque at every use: as loop invariants the row offsets would be kept in registers)
   auto lane_again = [&]() __attribute__((always_inline)) {  // (made again at every use: kept, it would be spilled)
     int l = lane;
     asm volatile("" : "+v"(l));
     return l;
   };
-  auto at = [&](const unsigned short* tile, int64_t ld, int i, int r, int g) __attribute__((always_inline)) {
+  // Walks the rows of the tile at `tile` in the order in which they are finished: a uniform base that moves by the pitch and a 32-bit
+  // lane offset made once per tile (as loop invariants of the kernel the offsets of all rows would be kept in registers).
+  struct Walk {
+    const unsigned char* p;
+    unsigned int pitch, quad, pair;
+    SF_DEVICE gbyte_t at(int g) const { return (gbyte_t)(uintptr_t)p + (g < P::NQ ? quad : pair) + 128 * g; }
+    SF_DEVICE void down(int rows) {
+      p += rows * pitch;
+      asm volatile("" : "+s"(p));
+    }
+  };
+  auto walk = [&](const unsigned short* tile, int64_t ld, int i) __attribute__((always_inline)) {
     const int l = lane_again();
-    unsigned int pitch = (unsigned int)ld * 2u;
-    asm volatile("" : "+s"(pitch));
-    const unsigned char* p = reinterpret_cast<const unsigned char*>(tile) + (unsigned int)(wm * 16 * TM + 16 * i + r) * pitch + (col0 + 64 * g) * 2;
-    asm volatile("" : "+s"(p));
-    unsigned int lane_off = (unsigned int)(4 * (l >> 4)) * pitch + (g < P::NQ ? 8 : 4) * (l & 15);
-    asm volatile("" : "+v"(lane_off));
-    return (gbyte_t)(uintptr_t)p + lane_off;
+    Walk w;
+    w.pitch = (unsigned int)ld * 2u;
+    asm volatile("" : "+s"(w.pitch));
+    w.p = reinterpret_cast<const unsigned char*>(tile + col0) + (int64_t)(wm * 16 * TM + 16 * i) * w.pitch;
+    asm volatile("" : "+s"(w.p));
+    w.quad = (unsigned int)(4 * (l >> 4)) * w.pitch + 8 * (l & 15);
+    asm volatile("" : "+v"(w.quad));
+    w.pair = P::PAIR ? w.quad - 4 * (l & 15) : 0;
+    return w;
   };
   typedef __attribute__((address_space(1))) u32x2* gquad_t;
   typedef __attribute__((address_space(1))) unsigned int* gpair_t;
@@ -299,22 +314,29 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
   constexpr int EARLY = P::NQ * 4 + (P::PAIR ? 4 : 0);
   u32x2 res[RES ? TM : 1][4][P::NQ];
   unsigned int res_pair[RES && P::PAIR ? TM : 1][4];
-  auto load_residual = [&](int i) __attribute__((always_inline)) {
-    const unsigned short* tile = a.residual + (int64_t)m0 * a.ld_res + n0;
+  auto residual_walk = [&](int i) __attribute__((always_inline)) { return walk(a.residual + (int64_t)m0 * a.ld_res + n0, a.ld_res, i); };
+  auto load_residual = [&](Walk& w, int i) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
 #pragma unroll
-      for (int g = 0; g < P::NQ; ++g) res[i][r][g] = *(gquad_t)at(tile, a.ld_res, i, r, g);
-      if constexpr (P::PAIR) res_pair[i][r] = *(gpair_t)at(tile, a.ld_res, i, r, P::NQ);
+      for (int g = 0; g < P::NQ; ++g) res[i][r][g] = *(gquad_t)w.at(g);
+      if constexpr (P::PAIR) res_pair[i][r] = *(gpair_t)w.at(P::NQ);
+      w.down(r < 3 ? 1 : 13);
     }
   };
+  // Both sides finish between the same two barriers, the lower one ahead by what it converts under the upper one's last products: two
+  // wavefronts share a SIMD's vector unit.  Where the conversion is an add and half a pack per value, they finish one behind the other,
+  // each under a turn of the other's products.
+  constexpr bool TOGETHER = E::SCALED || EPI != PP_PLAIN;
   auto finish = [&](auto whole) __attribute__((always_inline)) {
     constexpr bool FULL = decltype(whole)::value;
     const int l = lane_again(), lr = l & 15, lq = l >> 4;
+    Walk from = {};
     if constexpr (RES) {
-      if constexpr (!AHEAD) load_residual(0);
-      load_residual(1);
-      load_residual(2);
+      from = residual_walk(AHEAD ? 1 : 0);
+      if constexpr (!AHEAD) load_residual(from, 0);
+      load_residual(from, 1);
+      load_residual(from, 2);
       __builtin_amdgcn_sched_barrier(0);
     }
     // column scales and bias of the quads and the pair
@@ -333,11 +355,11 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
         }
       }
     }
-    unsigned short* const tile = a.out + (int64_t)m0 * a.ldo + n0;
+    Walk to = walk(a.out + (int64_t)m0 * a.ldo + n0, a.ldo, 0);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       if constexpr (RES)
-        if (i >= 1 && i + 2 < TM) load_residual(i + 2);  // (three of the row groups at a time: registers)
+        if (i >= 1 && i + 2 < TM) load_residual(from, i + 2);  // (three of the row groups at a time: registers)
       f32x4 sx;
       if constexpr (E::SCALED) sx = *reinterpret_cast<const f32x4*>(sc + (wm * 16 * TM + 16 * i + 4 * lq) * 4);
       // two adjacent columns of row r, rounded; group g, elements e and e + 1, plus the residual pair v
@@ -371,7 +393,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
         for (int g = 0; g < P::NQ; ++g) {
           const u32x2 v = RES ? res[RES ? i : 0][r][g] : u32x2{0u, 0u};
           const u32x2 o = {two(r, g, 0, v[0]), two(r, g, 2, v[1])};
-          const gquad_t dst = (gquad_t)at(tile, a.ldo, i, r, g);
+          const gquad_t dst = (gquad_t)to.at(g);
           if (FULL || (row >= skip_m && col0 + 64 * g + 4 * lr >= skip_n)) {
             if (NT) __builtin_nontemporal_store(o, dst);
             else *dst = o;
@@ -379,14 +401,16 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
         }
         if constexpr (P::PAIR) {
           const unsigned int o = two(r, P::NQ, 0, RES ? res_pair[RES ? i : 0][r] : 0u);
-          const gpair_t dst = (gpair_t)at(tile, a.ldo, i, r, P::NQ);
+          const gpair_t dst = (gpair_t)to.at(P::NQ);
           if (FULL || (row >= skip_m && col0 + 64 * P::NQ + 2 * lr >= skip_n)) {
             if (NT) __builtin_nontemporal_store(o, dst);
             else *dst = o;
           }
         }
+        to.down(r < 3 ? 1 : 13);
         __builtin_amdgcn_sched_barrier(0);  // keep the conversion narrow
       }
+      if (TOGETHER && i == 0 && wn == 0) meet();
     }
   };
 
@@ -416,7 +440,10 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
     read(0, stage);
     load_w(1, other);
     next_ktile();
-    if constexpr (LAST) load_residual(0);
+    if constexpr (LAST) {
+      Walk w = residual_walk(0);
+      load_residual(w, 0);
+    }
     if (EXTRA > 0 && extra) pp_wait<P::NLOADS + EXTRA>();
     else pp_wait<P::NLOADS>();
     meet();
@@ -443,6 +470,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
     stored = skip_m == 0 && skip_n == 0;
     if (stored) finish(Yes{});
     else finish(No{});
+    if (TOGETHER && wn == 1) meet();
     if (ti + 1 < nt) tile_origin(ti + 1, m0, n0, skip_m, skip_n);
   }
   if (wn == 0) meet();
