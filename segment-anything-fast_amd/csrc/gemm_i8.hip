@@ -1227,7 +1227,7 @@ extern "C" int64_t samfast_linear_i8_workspace(int64_t M, int N, int K, int layo
   using namespace samfast;
   SF_REQUIRE(M > 0 && N > 0 && K > 0 && layout >= SAMFAST_LAYOUT_ROWMAJOR && layout <= SAMFAST_LAYOUT_SPARSE24,
              "linear_i8_workspace: bad shape M=%lld N=%d K=%d or layout %d", (long long)M, N, K, layout);
-  if (layout != SAMFAST_LAYOUT_SPARSE24 && linear_i8_small_covers(M, N, K)) return 0;
+  if (linear_i8_small_covers(M, N, K, layout == SAMFAST_LAYOUT_SPARSE24)) return 0;
   const int64_t weights = layout == SAMFAST_LAYOUT_ROWMAJOR && linear_reorders_weights(M, N, K) ? (int64_t)N * K : 0;
   return linear_codes_bytes(M, K) + linear_scales_bytes(M) + weights;
 }
@@ -1237,11 +1237,12 @@ extern "C" int samfast_linear_i8(const void* x, int64_t ldx, const int8_t* wq, c
                                  int layout, void* stream) {
   using namespace samfast;
   SF_REQUIRE(layout == SAMFAST_LAYOUT_ROWMAJOR || layout == SAMFAST_LAYOUT_KB64, "linear_i8: unknown layout %d", layout);
-  if (M > 0 && linear_i8_small_covers(M, N, K)) {
+  if (M > 0 && linear_i8_small_covers(M, N, K, false)) {
     SF_REQUIRE(dtype == SAMFAST_BF16, "linear_i8: only bf16");
-    SF_REQUIRE(x && wq && sw && y && aligned16(x) && aligned16(wq) && aligned16(y), "linear_i8: null or unaligned pointer");
+    SF_REQUIRE(x && wq && sw && y && aligned16(x) && aligned16(wq) && aligned16(y) && (linear_i8_small_any_alignment(M, K) || (aligned16(sw) && aligned16(bias))),
+               "linear_i8: null or unaligned pointer");
     SF_REQUIRE(ldx >= K && ldx % 8 == 0 && ldy >= N && ldy % 8 == 0, "linear_i8: row strides must be multiples of 8, >= K and >= N");
-    return linear_i8_small_launch(reinterpret_cast<const unsigned short*>(x), ldx, wq, sw, bias, reinterpret_cast<unsigned short*>(y), ldy,
+    return linear_i8_small_launch(reinterpret_cast<const unsigned short*>(x), ldx, wq, nullptr, sw, bias, reinterpret_cast<unsigned short*>(y), ldy,
                                   (int)M, N, K, layout, reinterpret_cast<hipStream_t>(stream));
   }
   SF_REQUIRE(M == 0 || (workspace && aligned16(workspace)), "linear_i8: the workspace must be non-null and 16-byte aligned");
@@ -1267,6 +1268,15 @@ extern "C" int samfast_linear_i8_sparse24(const void* x, int64_t ldx, const int8
                                           const float* sw, const float* bias, void* y, int64_t ldy, void* workspace,
                                           int64_t M, int N, int K, int dtype, void* stream) {
   using namespace samfast;
+  if (M > 0 && linear_i8_small_covers(M, N, K, true)) {
+    SF_REQUIRE(dtype == SAMFAST_BF16, "linear_i8_sparse24: only bf16");
+    SF_REQUIRE(x && wc && widx && sw && y && aligned16(x) && aligned16(wc) && aligned16(widx) && aligned16(y) && aligned16(sw) && aligned16(bias),
+               "linear_i8_sparse24: null or unaligned pointer");
+    SF_REQUIRE(ldx >= K && ldx % 8 == 0 && ldy >= N && ldy % 8 == 0 && (int64_t)N * 32 < (1ll << 31),
+               "linear_i8_sparse24: row strides must be multiples of 8, >= K and >= N");
+    return linear_i8_small_launch(reinterpret_cast<const unsigned short*>(x), ldx, wc, widx, sw, bias, reinterpret_cast<unsigned short*>(y), ldy,
+                                  (int)M, N, K, 0, reinterpret_cast<hipStream_t>(stream));
+  }
   SF_REQUIRE(M == 0 || (workspace && aligned16(workspace)), "linear_i8_sparse24: the workspace must be non-null and 16-byte aligned");
   int8_t* xq = reinterpret_cast<int8_t*>(workspace);
   float* sx = reinterpret_cast<float*>(xq + linear_codes_bytes(M, K));

@@ -1,16 +1,17 @@
-// A whole quantised Linear over a handful of rows in one launch: row quantiser, int8 product and
+// A whole quantised Linear over few rows in one launch: row quantiser, int8 product and
 // the scale + bias epilogue (what quant_rowwise.hip + gemm_i8.hip do in two).
 //
 // Such a call is latency: the two launches and their gap, a row's way through memory twice, and a
 // K loop that a 64 x 128 tile walks serially on a GPU it leaves empty.  Here a 512-thread workgroup
-// owns 16 * NT output columns and ALL rows (MT tiles of 16):
+// owns 16 * NT output columns (2:4: 32) of 8 or 16 rows:
 //   * every wavefront first requests its share of the weight columns straight into registers (the K
 //     range is dealt out to the eight wavefronts in steps of 64, at most NCH each), so that the
 //     weights travel while the rows are quantised;
 //   * the workgroup quantises the rows itself - each workgroup repeats that for its own columns, which
-//     is why the form ends at a few dozen rows - and leaves the codes in LDS;
+//     is why the form ends at a few hundred rows - and leaves the codes in LDS; one row to a wavefront: what bounds it is that
+//     chain of 50 to 200 vector instructions per 512 values (blocks of 32 rows took 1-3 us more throughout);
 //   * v_mfma_i32_16x16x64_i8, codes as A and weights as B (both take 16 consecutive k bytes of one
-//     row per lane), then the eight partial sums meet in LDS: integer sums, so the order is free
+//     row per lane; 2:4: v_smfmac_i32_32x32x64_i8), then the eight partial sums meet in LDS: integer sums, so the order is free
 //     and the results have the bits of the two-launch form.
 #include "gemm_i8_shared.hpp"
 #include "linear_i8_small.hpp"
@@ -34,7 +35,8 @@ struct SmallArgs {
   int M, N, K;
   int x_pitch, w_pitch;      // bytes between consecutive code / weight rows: K, or 64 (K-block major)
   int64_t x_kstep, w_kstep;  // bytes between consecutive 64-byte k steps: 64, or rows * 64
-  int tiles_m, tiles;  // product alone: row tiles, tiles
+  int tiles_m, tiles;  // row blocks or row tiles, all tiles
+  const int32_t* widx;  // 2:4 weights: `w` holds (K/64, N, 32) bytes, this (K/64, N, 2) words
 };
 
 constexpr int kSmallWaves = 8;
@@ -77,37 +79,15 @@ SF_DEVICE void finish_tile(const SmallArgs& a, const i32x4 (&acc)[MT][NT], unsig
   }
 }
 
-template <int NCH, int RPW, int NT>  // RPW: rows per wavefront, so 8, 16 or 32 rows in all
-__global__ __launch_bounds__(64 * kSmallWaves, 2) void linear_i8_small_kernel(SmallArgs a) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  constexpr int MT = (RPW + 1) / 2, ROWS = 16 * MT;
-  float* sx = reinterpret_cast<float*>(lds);          // ROWS scales
-  unsigned char* codes = lds + ROWS * 4;              // ROWS x (K + 16) bytes; later the partial sums
-  const int pitch = a.K + 16;                         // an odd number of 16-byte pieces: operand reads spread over the banks
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n0 = blockIdx.x * 16 * NT;
-  const int nk = a.K / 64;
-  const int lr = lane & 15, lq = lane >> 4;
-
-  // weights first: step wave + 8 i, columns n0 + 16 t + lr, k bytes 16 lq .. +15
-  i32x4 wf[NCH][NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int8_t* wrow = a.w + (int64_t)min(n0 + 16 * t + lr, a.N - 1) * a.w_pitch + 16 * lq;
-#pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-      const int step = wave + kSmallWaves * i;
-      if (step < nk) wf[i][t] = *reinterpret_cast<const i32x4*>(wrow + step * a.w_kstep);  // uniform
-    }
-  }
-
-  // rows wave, wave + 8, ...: the arithmetic of RowQuantizer::finish_row, codes into LDS
+// The eight wavefronts quantise rows m0 .. m0 + 8 RPW - 1 (wave + 8 j of them is a wavefront's) into `codes`, their scales into `sx`.
+template <int NCH, int RPW>
+SF_DEVICE void quantize_rows(const SmallArgs& a, int m0, float* sx, unsigned char* codes, int pitch, int wave, int lane) {
+  // the arithmetic of RowQuantizer::finish_row
   const int nchunk = a.K / 8;
   u32x4 xw[RPW][NCH];
 #pragma unroll
   for (int j = 0; j < RPW; ++j) {
-    const int row = wave + kSmallWaves * j;
+    const int row = m0 + wave + kSmallWaves * j;
     const u32x4* src = reinterpret_cast<const u32x4*>(a.x + row * a.ldx);
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
@@ -156,28 +136,136 @@ __global__ __launch_bounds__(64 * kSmallWaves, 2) void linear_i8_small_kernel(Sm
     const bool row_nan = __any(saw_nan);
     if (lane == 0) sx[row] = row_nan ? __uint_as_float(0x7fc00000u) : scale[j];
   }
+}
+
+template <int NCH, int RPW, int NT>  // RPW: rows per wavefront, so blocks of 8 or 16 rows
+__global__ __launch_bounds__(64 * kSmallWaves, 2) void linear_i8_small_kernel(SmallArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  constexpr int ROWS = 16;
+  float* sx = reinterpret_cast<float*>(lds);          // ROWS scales
+  unsigned char* codes = lds + ROWS * 4;              // ROWS x (K + 16) bytes; later the partial sums
+  const int pitch = a.K + 16;                         // an odd number of 16-byte pieces: operand reads spread over the banks
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // row blocks of one column panel next to each other on an XCD
+  const unsigned int pid = xcd_contiguous_id(blockIdx.x, a.tiles);
+  if (pid >= (unsigned int)a.tiles) return;  // uniform
+  const int m0 = (int)(pid % a.tiles_m) * 8 * RPW, n0 = (int)(pid / a.tiles_m) * 16 * NT;
+  const int nk = a.K / 64;
+  const int lr = lane & 15, lq = lane >> 4;
+
+  // weights first: step wave + 8 i, columns n0 + 16 t + lr, k bytes 16 lq .. +15
+  i32x4 wf[NCH][NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int8_t* wrow = a.w + (int64_t)min(n0 + 16 * t + lr, a.N - 1) * a.w_pitch + 16 * lq;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int step = wave + kSmallWaves * i;
+      if (step < nk) wf[i][t] = *reinterpret_cast<const i32x4*>(wrow + step * a.w_kstep);  // uniform
+    }
+  }
+  quantize_rows<NCH, RPW>(a, m0, sx, codes, pitch, wave, lane);
   __syncthreads();
 
-  i32x4 acc[MT][NT];
+  i32x4 acc[1][NT];
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[m][t] = i32x4{0, 0, 0, 0};
+  for (int t = 0; t < NT; ++t) acc[0][t] = i32x4{0, 0, 0, 0};
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     const int step = wave + kSmallWaves * i;
     if (step < nk) {
+      const i32x4 xf = *reinterpret_cast<const i32x4*>(codes + lr * pitch + step * 64 + 16 * lq);
 #pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        const i32x4 xf = *reinterpret_cast<const i32x4*>(codes + (16 * m + lr) * pitch + step * 64 + 16 * lq);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[m][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xf, wf[i][t], acc[m][t], 0, 0, 0);
-      }
+      for (int t = 0; t < NT; ++t) acc[0][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xf, wf[i][t], acc[0][t], 0, 0, 0);
     }
   }
 
   __syncthreads();  // nobody reads the codes any more
-  finish_tile<MT, NT>(a, acc, codes, 0, n0, tid, [&](int row) { return sx[row]; });
+  // (of a block of 8 rows the upper half of the product's 16 is whatever stood in LDS, and nobody's)
+  SmallArgs b = a;
+  b.M = min(a.M, m0 + 8 * RPW);
+  finish_tile<1, NT>(b, acc, codes, m0, n0, tid, [&](int row) { return sx[row - m0]; });
+}
+
+// The same with 2:4 weights, in the packed order of gemm_i8_sparse24.hip: v_smfmac_i32_32x32x64_i8, weights (the sparse operand)
+// as the rows, tokens as the columns.  A workgroup owns 32 channels of 8 rows.
+template <int NCH>
+__global__ __launch_bounds__(64 * kSmallWaves, 2) void linear_i8_sp24_small_kernel(SmallArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  typedef int i32x8 __attribute__((ext_vector_type(8)));
+  constexpr int ROWS = 8;
+  float* sx = reinterpret_cast<float*>(lds);          // ROWS scales, in the first 64 bytes
+  unsigned char* codes = lds + 64;
+  const int pitch = a.K + 16;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const unsigned int pid = xcd_contiguous_id(blockIdx.x, a.tiles);
+  if (pid >= (unsigned int)a.tiles) return;  // uniform
+  const int m0 = (int)(pid % a.tiles_m) * ROWS, n0 = (int)(pid / a.tiles_m) * 32;
+  const int nk = a.K / 64;
+  const int lr = lane & 31, lh = lane >> 5;
+
+  i32x4 wf[NCH];
+  int ix[NCH];
+  {
+    const int nc = min(n0 + lr, a.N - 1);
+    const int8_t* wrow = a.w + (int64_t)nc * 32 + 16 * lh;
+    const int32_t* irow = a.widx + (int64_t)nc * 2 + lh;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int64_t step = wave + kSmallWaves * i;
+      if (step < nk) {  // uniform
+        wf[i] = *reinterpret_cast<const i32x4*>(wrow + step * a.N * 32);
+        ix[i] = irow[step * a.N * 2];
+      }
+    }
+  }
+  quantize_rows<NCH, 1>(a, m0, sx, codes, pitch, wave, lane);
+  __syncthreads();
+
+  i32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int step = wave + kSmallWaves * i;
+    if (step < nk) {
+      // (the columns beyond the eight tokens repeat the last one; nobody reads them)
+      const unsigned char* p = codes + min(lr, ROWS - 1) * pitch + step * 64 + 32 * lh;
+      const i32x4 lo = *reinterpret_cast<const i32x4*>(p), hi = *reinterpret_cast<const i32x4*>(p + 16);
+      const i32x8 xf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      acc = __builtin_amdgcn_smfmac_i32_32x32x64_i8(wf[i], xf, acc, ix[i], 0, 0);
+    }
+  }
+  __syncthreads();  // nobody reads the codes any more
+
+  // partial sums [wave][register][token], two runs of eight tokens a register: lane = token + 32 h, channels 8 (r/4) + 4 h + r%4
+  int* red = reinterpret_cast<int*>(codes);
+  if (lr < ROWS) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) red[wave * 256 + r * 16 + 8 * lh + lr] = acc[r];
+  }
+  __syncthreads();
+  // a thread finishes two adjacent channels of one token; 16 consecutive threads: one token row
+  if (tid >= 16 * ROWS) return;
+  const int tok = tid >> 4, c = 2 * (tid & 15);
+  const int row = m0 + tok, n = n0 + c;
+  if (row >= a.M || n >= a.N) return;  // N % 8 == 0: a pair is in or out together
+  const int at = (4 * (c >> 3) + (c & 3)) * 16 + 8 * ((c >> 2) & 1) + tok;
+  int s0 = 0, s1 = 0;
+#pragma unroll
+  for (int w = 0; w < kSmallWaves; ++w) {
+    s0 += red[w * 256 + at];
+    s1 += red[w * 256 + at + 16];
+  }
+  const float s = sx[tok];
+  float b0 = 0.f, b1 = 0.f;
+  if (a.bias) { b0 = a.bias[n]; b1 = a.bias[n + 1]; }
+  float t0 = (float)s0 * s, t1 = (float)s1 * s;
+  t0 = t0 * a.sw[n];
+  t1 = t1 * a.sw[n + 1];
+  *reinterpret_cast<unsigned int*>(a.y + (int64_t)row * a.ldy + n) = pack_bf16x2(t0 + b0, t1 + b1);
 }
 
 // The product alone, on codes that a quantiser launch has written: the same dealing of the K range over
@@ -234,48 +322,79 @@ __global__ __launch_bounds__(64 * kSmallWaves, 2) void gemm_i8_skinny_kernel(Sma
   finish_tile<MT, NT>(a, acc, lds, m0, n0, tid, [&](int row) { return a.sx[row]; });
 }
 
-bool linear_i8_small_covers(int64_t M, int N, int K) {
-  if (knob_or(KNOB_LINEAR_SMALL, 1) <= 0 || K % 64 != 0 || N % 8 != 0 || K > 5120) return false;
-  // every workgroup quantises every row, 0.3 us per 8 rows of 1280: past these lines the separate quantiser
-  // and the small-tile product take less GPU time than the repetition (16 x 3072: 9.1 us against 8.6), below
-  // them one launch also saves the host the second one (7 x 256 -> 2048: 6.7 us a call against 8.7)
-  return M <= 8 || (M <= 16 && K <= 2048) || (M <= 32 && K <= 768);
+bool linear_i8_small_any_alignment(int64_t M, int K) { return M <= 8 || (M <= 16 && K <= 2048) || (M <= 32 && K <= 768); }
+
+// Rows per wavefront * 8 + column tiles (16 columns each; 2:4: 32) of a workgroup; 0 = not this form.
+// A call of one launch costs the host 6.3 us, of two 9.7, whatever the GPU does meanwhile; on the GPU every workgroup quantises its
+// rows (8 of 768: 0.5 us, of 3072: 3), so the form ends where that repetition, or a second workgroup on a CU, makes it longer than the
+// quantiser and the small-tile product by more than about a microsecond.  GPU time in us, two launches / one (shape):
+//   int8  24 x 768 -> 2304 5.8 / 4.4 (8 rows, 2 tiles), 64 x 1024 -> 1024 6.1 / 4.9, 128 x 1024 -> 1024 6.6 / 5.5 (4 tiles), 256 x 1024 -> 1024 6.9 /
+//         6.9 (16 rows, 4), 192 x 1280 -> 1280 7.6 / 8.2 (16, 4), 256 x 768 -> 768 6.4 / 6.7 (8, 4), 64 x 2048 -> 1024 6.5 / 7.2 (8, 2); beyond: 384 x
+//         1024 -> 1024 8.0 / 9.3, 96 x 2048 -> 1024 7.3 / 8.9, 12 x 3072 -> 768 7.1 / 8.0, 256 x 1280 -> 1280 8.5 / 11.3
+//   2:4   64 x 768 -> 768 7.1 / 4.6, 128 x 1024 -> 1024 7.8 / 6.1, 96 x 1280 -> 1280 7.9 / 7.3, 64 x 2048 -> 1024 8.1 / 6.8, 64 x 3072 -> 768 9.1 / 9.1;
+//         beyond: 256 x 1024 -> 1024 7.7 / 8.1, 128 x 1280 -> 1280 8.0 / 9.1, 48 x 4096 -> 1024 10.2 / 10.0 (rows at or past M cost less: 4 x 5120 -> 1280 8.5 / 7.7), 96 x 2048 -> 1024 8.0 / 8.5
+// A call, launches included (7 x 256 -> 2048 6.7 us a call, two launches 8.7): 64 x 1024 -> 1024 9.8 / 6.4, 2:4 64 x 1024 -> 1024 9.8 / 6.4.
+static int small_shape(int64_t M, int N, int K, bool sparse) {
+  if (knob_or(KNOB_LINEAR_SMALL, 1) <= 0 || K % 64 != 0 || N % 8 != 0 || N <= 0 || K <= 0 || K > 5120 || M <= 0 || M > 4096) return 0;
+  const int64_t eights = (M + 7) / 8;
+  if (sparse) {
+    const int64_t tiles = eights * ((N + 31) / 32);
+    return K % 128 == 0 && K >= 256 && (K <= 3072 || M <= 4) && tiles <= (K <= 1024 ? 768 : K <= 1536 ? 512 : 256) ? 8 + 1 : 0;
+  }
+  auto tiles = [&](int nt) { return eights * ((N + 16 * nt - 1) / (16 * nt)); };
+  if (M <= 8 || K <= 2048) {
+    if (tiles(1) <= 256) return 8 + 1;
+    if (tiles(2) <= 256) return 8 + 2;
+    if (K <= 1536 && tiles(4) <= 256) return 8 + 4;
+    if (M <= 8) return 8 + 2;
+  }
+  if (K <= 1536 && ((M + 15) / 16) * ((N + 63) / 64) <= 256) return 16 + 4;
+  if (K <= 768 && tiles(4) <= 512) return 8 + 4;
+  return linear_i8_small_any_alignment(M, K) ? (K <= 1536 ? 16 + 4 : 8 + 2) : 0;
 }
 
-template <int NCH, int RPW, int NT>
-static int launch_small(const SmallArgs& a, hipStream_t stream) {
-  constexpr int MT = (RPW + 1) / 2;
-  const int codes = 16 * MT * (a.K + 16), red = kSmallWaves * MT * NT * 1024;
-  const size_t lds = 16 * MT * 4 + (codes > red ? codes : red);
-  hipLaunchKernelGGL((linear_i8_small_kernel<NCH, RPW, NT>), dim3((a.N + 16 * NT - 1) / (16 * NT)), dim3(64 * kSmallWaves), lds, stream, a);
+bool linear_i8_small_covers(int64_t M, int N, int K, bool sparse) { return small_shape(M, N, K, sparse) != 0; }
+
+template <typename Kernel>
+static int launch_small(Kernel kernel, SmallArgs a, int rows, int cols, int lds, hipStream_t stream) {
+  a.tiles_m = (a.M + rows - 1) / rows;
+  a.tiles = a.tiles_m * ((a.N + cols - 1) / cols);
+  hipLaunchKernelGGL(kernel, dim3((unsigned int)((a.tiles + 7) / 8 * 8)), dim3(64 * kSmallWaves), (size_t)lds, stream, a);
   return check_launch("linear_i8_small_kernel");
 }
 
-int linear_i8_small_launch(const unsigned short* x, int64_t ldx, const int8_t* wq, const float* sw, const float* bias, unsigned short* y,
-                           int64_t ldy, int M, int N, int K, int layout, hipStream_t stream) {
+template <int NCH>
+static int launch_shape(const SmallArgs& a, int shape, hipStream_t stream) {
+  auto lds = [&](int scales, int rows, int sums) { return scales + max(rows * (a.K + 16), sums); };
+  if (a.widx) {
+    if (shape == 8 + 1) return launch_small(linear_i8_sp24_small_kernel<NCH>, a, 8, 32, lds(64, 8, kSmallWaves * 1024), stream);
+  } else {
+    if (shape == 8 + 1) return launch_small(linear_i8_small_kernel<NCH, 1, 1>, a, 8, 16, lds(64, 16, kSmallWaves * 1024), stream);
+    if (shape == 8 + 2) return launch_small(linear_i8_small_kernel<NCH, 1, 2>, a, 8, 32, lds(64, 16, kSmallWaves * 2048), stream);
+    if constexpr (NCH <= 3) {
+      if (shape == 8 + 4) return launch_small(linear_i8_small_kernel<NCH, 1, 4>, a, 8, 64, lds(64, 16, kSmallWaves * 4096), stream);
+      if (shape == 16 + 4) return launch_small(linear_i8_small_kernel<NCH, 2, 4>, a, 16, 64, lds(64, 16, kSmallWaves * 4096), stream);
+    }
+  }
+  set_error("linear_i8_small: %d rows of %d values are not covered", a.M, a.K);
+  return SAMFAST_E_UNSUPPORTED;
+}
+
+int linear_i8_small_launch(const unsigned short* x, int64_t ldx, const int8_t* w, const int32_t* widx, const float* sw, const float* bias,
+                           unsigned short* y, int64_t ldy, int M, int N, int K, int layout, hipStream_t stream) {
   SmallArgs a = {};
-  a.x = x; a.ldx = ldx; a.w = wq; a.sw = sw; a.bias = bias; a.y = y; a.ldy = ldy; a.M = M; a.N = N; a.K = K;
+  a.x = x; a.ldx = ldx; a.w = w; a.widx = widx; a.sw = sw; a.bias = bias; a.y = y; a.ldy = ldy; a.M = M; a.N = N; a.K = K;
   const bool kb = layout == SAMFAST_LAYOUT_KB64;
   a.w_pitch = kb ? 64 : K;
   a.w_kstep = kb ? (int64_t)N * 64 : 64;
-  // two column tiles per workgroup once single ones are more than the GPU has CUs: half the repeated
-  // row work for the same number of rounds
-  const bool wide = N > 16 * 256;
-  auto by_rows = [&](auto nch) {
-    constexpr int NCH = decltype(nch)::value;
-    if (M <= 8) return wide ? launch_small<NCH, 1, 2>(a, stream) : launch_small<NCH, 1, 1>(a, stream);
-    if (M <= 16) return wide ? launch_small<NCH, 2, 2>(a, stream) : launch_small<NCH, 2, 1>(a, stream);
-    if constexpr (NCH <= 2) return wide ? launch_small<NCH, 4, 2>(a, stream) : launch_small<NCH, 4, 1>(a, stream);
-    set_error("linear_i8_small: %d rows of %d values are not covered", M, K);
-    return (int)SAMFAST_E_UNSUPPORTED;
-  };
-  if (K <= 512) return by_rows(std::integral_constant<int, 1>{});
-  if (K <= 1024) return by_rows(std::integral_constant<int, 2>{});
-  if (K <= 1536) return by_rows(std::integral_constant<int, 3>{});
-  if (K <= 2048) return by_rows(std::integral_constant<int, 4>{});
-  if (K <= 3072) return by_rows(std::integral_constant<int, 6>{});
-  if (K <= 4096) return by_rows(std::integral_constant<int, 8>{});
-  return by_rows(std::integral_constant<int, 10>{});
+  const int shape = small_shape(M, N, K, widx != nullptr);
+  if (K <= 512) return launch_shape<1>(a, shape, stream);
+  if (K <= 1024) return launch_shape<2>(a, shape, stream);
+  if (K <= 1536) return launch_shape<3>(a, shape, stream);
+  if (K <= 2048) return launch_shape<4>(a, shape, stream);
+  if (K <= 3072) return launch_shape<6>(a, shape, stream);
+  if (K <= 4096) return launch_shape<8>(a, shape, stream);
+  return launch_shape<10>(a, shape, stream);
 }
 
 // The smallest tile whose tiles still fit the GPU's CUs once: a smaller tile means a shorter chain, a second

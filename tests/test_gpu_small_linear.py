@@ -217,3 +217,30 @@ def test_one_tile_per_cu_agrees_with_the_small_tiles(bm, tn, M, N, K, epi, layou
             assert run(residual=inplace, out=inplace) is not None and torch.equal(inplace, y)
     with _lib.knobs(SAMFAST_GEMM_TILE=64, SAMFAST_GEMM_SKINNY=0):
         assert torch.equal(run(residual=res), y)
+
+
+@pytest.mark.parametrize("sparse,M,N,K", [
+    # workgroups of 8 rows and one, two, four column tiles, of 16 rows; the last calls of each, remainders of rows, columns and k steps
+    (False, 63, 488, 64), (False, 64, 512, 512), (False, 65, 1000, 576), (False, 121, 1024, 1024), (False, 128, 1032, 1088), (False, 250, 1016, 1536),
+    (False, 79, 760, 2048), (False, 405, 632, 704), (False, 9, 8200, 1600), (False, 31, 13000, 768),
+    (True, 1, 8, 256), (True, 63, 1000, 512), (True, 128, 1536, 1024), (True, 77, 1632, 1152), (True, 57, 1016, 2048), (True, 81, 712, 3072), (True, 4, 1288, 5120),
+])
+def test_one_launch_agrees_with_two(sparse, M, N, K):
+    from samfast_amd import Int8DynamicLinear, Int8Sparse24Linear, _lib
+    print(f"case one launch sparse={sparse} M={M} N={N} K={K}", flush=True)
+    x, w, b = linear_inputs(M, K, N, seed=M + N + K)
+    x[M // 2] = 0
+    x[M - 1, K // 3] = float("nan")
+    lin = torch.nn.Linear(K, N, bias=M % 2 == 1, dtype=torch.bfloat16)
+    with torch.no_grad():
+        lin.weight.copy_(w)
+        if lin.bias is not None:
+            lin.bias.copy_(b)
+    lin, x = (Int8Sparse24Linear if sparse else Int8DynamicLinear).from_float(lin.cuda()), x.cuda()
+    layout = 2 if sparse else _lib.LAYOUT_ROWMAJOR
+    assert _lib.load().samfast_linear_i8_workspace(M, N, K, layout) == 0
+    one = lin(x)
+    with _lib.knobs(SAMFAST_GEMM_LINEAR_SMALL=0):
+        assert _lib.load().samfast_linear_i8_workspace(M, N, K, layout) > 0
+        two = lin(x)
+    assert torch.equal(one.view(torch.int16), two.view(torch.int16))
