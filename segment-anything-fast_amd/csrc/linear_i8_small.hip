@@ -98,43 +98,28 @@ SF_DEVICE void quantize_rows(const SmallArgs& a, int m0, float* sx, unsigned cha
   }
   // (rows at or past M hold zeros: they are quantised along, which keeps the rows' serial chains -
   // maximum, lane reduction, two divisions - independent and in flight together)
-  float amax[RPW], scale[RPW], inv_scale[RPW];
-#pragma unroll
-  for (int j = 0; j < RPW; ++j) {
-    amax[j] = 0.f;
-#pragma unroll
-    for (int i = 0; i < NCH; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        amax[j] = fmaxf(amax[j], fmaxf(fabsf(bf16_lo_to_f32(xw[j][i][e])), fabsf(bf16_hi_to_f32(xw[j][i][e]))));
-  }
-#pragma unroll
-  for (int j = 0; j < RPW; ++j) amax[j] = wave_max_nonneg(amax[j]);
-#pragma unroll
-  for (int j = 0; j < RPW; ++j) {
-    scale[j] = fmaxf(amax[j], 1e-5f) / 127.0f;
-    inv_scale[j] = 1.0f / scale[j];
-  }
 #pragma unroll
   for (int j = 0; j < RPW; ++j) {
     const int row = wave + kSmallWaves * j;
-    bool saw_nan = false;
+    float f[NCH][8], amax;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f[i][2 * e] = bf16_lo_to_f32(xw[j][i][e]);
+        f[i][2 * e + 1] = bf16_hi_to_f32(xw[j][i][e]);
+      }
+    const bool row_nan = wave_absmax(f, amax);
+    const QuantScale q(amax);
 #pragma unroll
     for (int i = 0; i < NCH; ++i)
       if (lane + 64 * i < nchunk) {
-        float f[8];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          f[2 * e] = bf16_lo_to_f32(xw[j][i][e]);
-          f[2 * e + 1] = bf16_hi_to_f32(xw[j][i][e]);
-        }
         unsigned int c[2];
-        saw_nan |= quantize_chunk<8>(f, scale[j], inv_scale[j], c);
+        quantize_chunk<8>(f[i], q, c);
         const u32x2 o = {c[0], c[1]};
         *reinterpret_cast<u32x2*>(codes + row * pitch + (lane + 64 * i) * 8) = o;
       }
-    const bool row_nan = __any(saw_nan);
-    if (lane == 0) sx[row] = row_nan ? __uint_as_float(0x7fc00000u) : scale[j];
+    if (lane == 0) sx[row] = row_nan ? __uint_as_float(0x7fc00000u) : q.scale;
   }
 }
 

@@ -105,9 +105,9 @@ __global__ __launch_bounds__(512) void proj_block_i8_kernel(ProjBlockArgs a) {
 #pragma unroll
   for (int r = 0; r < RPW; ++r) {
     const int row = wave * RPW + r;
-    const float scale = In::finish(a.q, NCHUNK, lane, xw[r], gw, bw, [&](int c, const unsigned int (&v)[EPC / 4]) {
+    const float scale = In::finish(a.q, NCHUNK, lane, xw[r], gw, bw, [&](int i, const unsigned int (&v)[EPC / 4]) {
 #pragma unroll
-      for (int e = 0; e < EPC / 4; ++e) reinterpret_cast<unsigned int*>(codes + row * CP + c * EPC)[e] = v[e];
+      for (int e = 0; e < EPC / 4; ++e) reinterpret_cast<unsigned int*>(codes + row * CP + (64 * i + lane) * EPC)[e] = v[e];
     });
     if (lane == 0) scales[row] = scale;
   }

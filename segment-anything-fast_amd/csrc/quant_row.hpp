@@ -60,46 +60,70 @@ SF_DEVICE float wave_max_nonneg(float v) {
   });
 }
 
+// A row's scale and what its values are multiplied by: 1 / scale a little short of it and a little past it.
+struct QuantScale {
+  float scale, below, above;
+  SF_DEVICE explicit QuantScale(float amax) {
+    scale = fmaxf(amax, 1e-5f) / 127.0f;
+    const float inv = 1.0f / scale;
+    below = inv * (1.0f - 0x1p-22f);
+    above = inv * (1.0f + 0x1p-22f);
+  }
+};
+
 // EPC (4 or 8) values -> EPC int8 codes packed in EPC bytes.
-// The code wanted is rint(fl(v / scale)) with the correctly rounded IEEE quotient.  The cheap
-// route works on p = v * inv_scale (inv_scale = fl(1 / scale)), taken exactly inside fused
-// multiply-adds: m = fl(p + 1.5 * 2^23) holds rint(p) - half to even - in its low mantissa bits
-// (|p| <= 127 (1 + 2^-23)), so the low byte of m's bit pattern is the int8 code of p, and
-// d = fl(p - (m - 1.5 * 2^23)) is p - rint(p) to 3e-8.  p differs from v / scale by at most
-// 127 * 2^-24 (the rounding of inv_scale) and fl(v / scale) from v / scale by as much: 1.6e-5
-// together.  Unless p lies within that distance of a half-integer, rint(p) is the wanted code;
-// chunks with a |d| above 0.5 - 2.5e-5 are redone with the true division.
-// Returns true when the chunk holds a NaN: the comparison that finds near-ties is written so
-// that a NaN product also takes the slow path, where the chunk's values are looked at once more;
-// the common path pays nothing for it.
+// The code wanted is rint(fl(v / scale)) with the correctly rounded IEEE quotient.  The cheap route brackets it: below and
+// above are 1 / scale to within three roundings (2^-24 each) of 1 -+ 2^-22 times it, so v / scale, and its rounding, lies between
+// the exact products v * below and v * above.  m = fl(v * below + 1.5 * 2^23), a fused multiply-add, holds rint(v * below) - half to
+// even - in its low mantissa bits (|v / scale| <= 127 (1 + 2^-23)); rint is monotone: where the same with `above` is the same,
+// so is the code.  Chunks with a value for which it is not - one within 3e-5 of a half-integer - are redone with the true division.
+// Per value two fused multiply-adds and one bit operation (product, its distance from the integer and a comparison before: one
+// more vector and one more scalar instruction, of which this kernel's time consists).
 template <int EPC>
-SF_DEVICE bool quantize_chunk(const float (&v)[EPC], float scale, float inv_scale, unsigned int (&out)[EPC / 4]) {
+SF_DEVICE void quantize_chunk(const float (&v)[EPC], const QuantScale& s, unsigned int (&out)[EPC / 4]) {
   constexpr float kMagic = 12582912.0f;  // 1.5 * 2^23
   float m[EPC];
-  bool near_tie = false, saw_nan = false;
+  unsigned int differ = 0u;
 #pragma unroll
   for (int e = 0; e < EPC; ++e) {
-    m[e] = fmaf(v[e], inv_scale, kMagic);
-    const float d = fmaf(v[e], inv_scale, kMagic - m[e]);  // kMagic - m[e] = -rint(p), exact
-    near_tie |= !(fabsf(d) <= 0.5f - 2.5e-5f);  // also true for a NaN
+    m[e] = fmaf(v[e], s.below, kMagic);
+    // differ | (a ^ b), one instruction (written with operators the compiler would compare value by value)
+    differ = __builtin_amdgcn_bitop3_b32(differ, __float_as_uint(m[e]), __float_as_uint(fmaf(v[e], s.above, kMagic)), 0xf6);
   }
-  if (near_tie) {
+  if (differ != 0u) {
 #pragma unroll
-    for (int e = 0; e < EPC; ++e) {
-      m[e] = v[e] / scale + kMagic;  // IEEE division
-      saw_nan |= v[e] != v[e];
-    }
+    for (int e = 0; e < EPC; ++e) m[e] = v[e] / s.scale + kMagic;  // IEEE division
   }
 #pragma unroll
   for (int g = 0; g < EPC / 4; ++g) {
-    const unsigned int w0 = __builtin_bit_cast(unsigned int, m[4 * g]), w1 = __builtin_bit_cast(unsigned int, m[4 * g + 1]);
-    const unsigned int w2 = __builtin_bit_cast(unsigned int, m[4 * g + 2]), w3 = __builtin_bit_cast(unsigned int, m[4 * g + 3]);
+    const unsigned int w0 = __float_as_uint(m[4 * g]), w1 = __float_as_uint(m[4 * g + 1]);
+    const unsigned int w2 = __float_as_uint(m[4 * g + 2]), w3 = __float_as_uint(m[4 * g + 3]);
     // byte 0 of each of four words -> one word (v_perm_b32: selector bytes pick from {hi, lo})
     const unsigned int lo = __builtin_amdgcn_perm(w1, w0, 0x0c0c0400u);  // [w0.b0, w1.b0, 0, 0]
     const unsigned int hi = __builtin_amdgcn_perm(w3, w2, 0x04000c0cu);  // [0, 0, w2.b0, w3.b0]
     out[g] = lo | hi;
   }
-  return saw_nan;
+}
+
+// Absolute maximum of what the wavefront's lanes hold, without NaNs; returns whether there was one.  The maximum of the common path
+// hands NaNs on, which costs nothing; a row with one is looked through again.
+template <int N, int EPC>
+SF_DEVICE bool wave_absmax(const float (&f)[N][EPC], float& amax) {
+  amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < EPC; ++e) amax = __builtin_elementwise_maximum(amax, fabsf(f[i][e]));
+  amax = wave_max_nonneg(fabsf(amax));
+  if (__builtin_amdgcn_readfirstlane(__float_as_uint(amax)) <= 0x7f800000u) return false;
+  asm volatile("");  // (not to be run ahead of the branch)
+  amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < EPC; ++e) amax = fmaxf(amax, fabsf(f[i][e]));
+  amax = wave_max_nonneg(amax);
+  return true;
 }
 
 // A lane holds chunks lane, lane + 64, ... of EPC elements (NCH of them: K <= NCH * 64 * EPC).
@@ -138,19 +162,19 @@ struct RowQuantizer {
     }
   }
 
-  // chunk c of output row `row`: row-major at row*K + EPC*c; K-block major at
-  // ((c*EPC/64)*M + row)*64 + (c*EPC)%64.  Written as a uniform base (the row is the same for the
-  // whole wavefront) plus an unsigned 32-bit lane offset - M*K < 2^31 is checked on the host - so
-  // that the stores take the scalar-base form and no 64-bit arithmetic runs per lane.
-  static SF_DEVICE void store_chunk(const QuantArgs& a, int64_t row, int c, const unsigned int (&codes)[EPC / 4]) {
-    const unsigned int k = (unsigned int)c * EPC;
+  // chunk 64 i + lane of output row `row` (i uniform): row-major at row*K + EPC*c; K-block major at
+  // ((c*EPC/64)*M + row)*64 + (c*EPC)%64.  Written as a uniform base plus an unsigned 32-bit lane offset - M*K < 2^31 is
+  // checked on the host - that is the same for every i: the stores take the scalar-base form and nothing of the address is
+  // computed per chunk and lane.
+  static SF_DEVICE void store_chunk(const QuantArgs& a, int64_t row, int i, int lane, const unsigned int (&codes)[EPC / 4]) {
+    const unsigned int k = (unsigned int)lane * EPC;
     int8_t* base;
     unsigned int off;
     if (a.kb64) {
-      base = a.xq + row * 64;
+      base = a.xq + row * 64 + (int64_t)(i * EPC) * (a.M * 64);
       off = (k >> 6) * ((unsigned int)a.M * 64u) + (k & 63u);
     } else {
-      base = a.xq + row * (int64_t)a.K;
+      base = a.xq + row * (int64_t)a.K + i * (64 * EPC);
       off = k;
     }
     unsigned int* dst = reinterpret_cast<unsigned int*>(base + off);
@@ -168,7 +192,7 @@ struct RowQuantizer {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const int c = lane + i * 64;
-      if (c < nchunk) store_chunk(a, row, c, z);
+      if (c < nchunk) store_chunk(a, row, i, lane, z);
     }
     if (lane == 0) a.sx[row] = 1e-5f / 127.0f;
   }
@@ -176,11 +200,11 @@ struct RowQuantizer {
   // Everything after the loads: (LayerNorm,) absmax, scale, codes of output row `row`.
   static SF_DEVICE void finish_row(const QuantArgs& a, int64_t row, int nchunk, int lane,
                                    const in_t (&xw)[NCH], const in_t (&gw)[NCH], const in_t (&bw)[NCH]) {
-    const float scale = finish(a, nchunk, lane, xw, gw, bw, [&](int c, const unsigned int (&codes)[EPC / 4]) { store_chunk(a, row, c, codes); });
+    const float scale = finish(a, nchunk, lane, xw, gw, bw, [&](int i, const unsigned int (&codes)[EPC / 4]) { store_chunk(a, row, i, lane, codes); });
     if (lane == 0) a.sx[row] = scale;
   }
 
-  // The same with the chunks' codes handed to store(chunk, codes); returns the row's scale (in every lane).
+  // The same with the codes of chunk 64 i + lane handed to store(i, codes); returns the row's scale (in every lane).
   template <typename Store>
   static SF_DEVICE float finish(const QuantArgs& a, int nchunk, int lane, const in_t (&xw)[NCH], const in_t (&gw)[NCH], const in_t (&bw)[NCH],
                                 Store store) {
@@ -236,30 +260,18 @@ struct RowQuantizer {
       }
     }
 
-    float amax = 0.f;
+    float amax;
+    // a row that holds a NaN gets a NaN scale, so that the Linear reading it returns NaN for this row as a float Linear would
+    const bool row_nan = wave_absmax(f, amax);
+    const QuantScale q(amax);
 #pragma unroll
     for (int i = 0; i < NCH; ++i)
-#pragma unroll
-      for (int e = 0; e < EPC; ++e) amax = fmaxf(amax, fabsf(f[i][e]));
-    amax = wave_max_nonneg(amax);
-
-    const float scale = fmaxf(amax, 1e-5f) / 127.0f;
-    const float inv_scale = 1.0f / scale;
-
-    bool saw_nan = false;
-#pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-      const int c = lane + i * 64;
-      if (c < nchunk) {
+      if (lane + i * 64 < nchunk) {
         unsigned int codes[EPC / 4];
-        saw_nan |= quantize_chunk<EPC>(f[i], scale, inv_scale, codes);
-        store(c, codes);
+        quantize_chunk<EPC>(f[i], q, codes);
+        store(i, codes);
       }
-    }
-    // the maximum above drops NaNs (fmaxf returns its other operand); a row that holds one gets a
-    // NaN scale, so that the Linear reading it returns NaN for this row as a float Linear would
-    const bool row_nan = __any(saw_nan);
-    return row_nan ? __uint_as_float(0x7fc00000u) : scale;
+    return row_nan ? __uint_as_float(0x7fc00000u) : q.scale;
   }
 };
 

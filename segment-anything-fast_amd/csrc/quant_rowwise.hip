@@ -1,7 +1,9 @@
 // Per-row symmetric int8 quantiser (bf16 -> int8 + fp32 scale), optionally preceded
-// by LayerNorm over the row and a row gather (window partition).  HBM-bound for long rows
-// (K = 5120); for K = 1280, whose tensors sit in the last-level cache, the vector ALU is the
-// limit (310 vector instructions per row plain, 530 with LayerNorm, by the hardware counters).
+// by LayerNorm over the row and a row gather (window partition).  HBM-bound: 65536 rows of 5120 through GELU 209 us, of 1280
+// plain 38, with LayerNorm 48 (4.8, 6.6 and 5.2 TB/s; a copy reaches 4.9 from HBM), and the vector ALU close behind: 254 vector
+// instructions per row of 1280 plain, 448 with LayerNorm, 1764 per row of 5120 with GELU, by the hardware counters (297, 515 and 1949 with
+// a product, its distance from the integer and a comparison per value, and every chunk's address made per lane: 20480 x 4096 with
+// GELU 57.3 -> 53.3 us, 4096 x 5120 17.6 -> 16.7).
 //
 // One wavefront owns one output row: the source row is read once with 16- or 8-byte loads
 // and unpacked to fp32 registers, (normalised,) reduced to its absmax across the 64 lanes
@@ -10,9 +12,8 @@
 // Algorithmic traffic: 2 bytes read + 1 byte written per element + 4 bytes of scale.
 //
 // q = rint(x / s) must equal the IEEE division bit for bit.  Most elements take a
-// cheap route: the exact product x * fl(1/s) differs from fl(x / s) by at most 1.6e-5, so
-// its rint can only differ when it lies within that distance of a half-integer; only those
-// elements (and their 8-element chunk) are redone with the true division (quant_row.hpp).
+// cheap route: rint of a product a little below the quotient and of one a little above it; only where those differ
+// is the element's chunk redone with the true division (quant_row.hpp).
 // |x| <= absmax makes |x / s| <= 127 by construction, so no clamp is needed.
 #include "quant_row.hpp"
 
@@ -32,7 +33,8 @@ SF_DEVICE void gelu_chunks(in_t (&xw)[NCH]) {
 // ACT: the values are GELU's of what lies in memory.  Between an MLP's two Linears the activation runs here rather than in
 // the first one's epilogue: this kernel waits for memory and the vector ALU is free (65536 x 5120: 175 us without, 215 with it),
 // while a GEMM's wavefronts multiply nothing in the meantime (65536 x 1280 -> 5120: 465 us with GELU, 375 without).
-template <int NCH, int EPC, bool LN, bool ACT>
+// EXACT: the row fills every lane's chunks (nothing is tested per chunk, and the loads' addresses are one and constants).
+template <int NCH, int EPC, bool LN, bool ACT, bool EXACT>
 __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowwise_bf16_kernel(QuantArgs a) {
   using RQ = RowQuantizer<NCH, EPC, LN>;
   const int lane = threadIdx.x & 63;
@@ -40,7 +42,7 @@ __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowwise_bf16_k
   // (row pointers, output offsets) in scalar registers instead of 64-bit arithmetic per lane
   const int64_t row = (int64_t)blockIdx.x * kQuantWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= a.M) return;  // whole wavefront leaves together
-  const int nchunk = a.K / EPC;
+  const int nchunk = EXACT ? 64 * NCH : a.K / EPC;
 
   int64_t srow = row;
   if (LN && a.src_row) {
@@ -79,7 +81,7 @@ __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowshare_bf16_
   const int nchunk = a.K / EPC;
   // chunk i of the lane: (i * WPR + sub) * 64 + lane, so that the wavefronts of a row read it side by side
   in_t xw[NCH];
-  float amax = 0.f;
+  float amax;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     const int c = (i * WPR + sub) * 64 + lane;
@@ -91,42 +93,35 @@ __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowshare_bf16_
     }
   }
   if (ACT) gelu_chunks(xw);
+  float f[NCH][EPC];
 #pragma unroll
   for (int i = 0; i < NCH; ++i)
 #pragma unroll
-    for (int e = 0; e < RQ::W; ++e) amax = fmaxf(amax, fmaxf(fabsf(bf16_lo_to_f32(xw[i][e])), fabsf(bf16_hi_to_f32(xw[i][e]))));
-  amax = wave_max_nonneg(amax);
-  if (lane == 0) part[wave] = amax;
-  __syncthreads();
-#pragma unroll
-  for (int w = 0; w < WPR; ++w) amax = fmaxf(amax, part[wave / WPR * WPR + w]);
-  const float scale = fmaxf(amax, 1e-5f) / 127.0f;
-  const float inv_scale = 1.0f / scale;
-  bool saw_nan = false;
-#pragma unroll
-  for (int i = 0; i < NCH; ++i) {
-    const int c = (i * WPR + sub) * 64 + lane;
-    if (live && c < nchunk) {
-      float f[EPC];
-#pragma unroll
-      for (int e = 0; e < RQ::W; ++e) {
-        f[2 * e] = bf16_lo_to_f32(xw[i][e]);
-        f[2 * e + 1] = bf16_hi_to_f32(xw[i][e]);
-      }
-      unsigned int codes[EPC / 4];
-      saw_nan |= quantize_chunk<EPC>(f, scale, inv_scale, codes);
-      RQ::store_chunk(a, row, c, codes);
+    for (int e = 0; e < RQ::W; ++e) {
+      f[i][2 * e] = bf16_lo_to_f32(xw[i][e]);
+      f[i][2 * e + 1] = bf16_hi_to_f32(xw[i][e]);
     }
+  const bool own_nan = wave_absmax(f, amax);
+  if (lane == 0) {
+    part[wave] = amax;
+    nan_seen[wave] = own_nan;
   }
-  const bool any_nan = __any(saw_nan);  // (the maximum drops NaNs: see RowQuantizer::finish_row)
-  if (lane == 0) nan_seen[wave] = any_nan;
   __syncthreads();
-  if (live && sub == 0 && lane == 0) {
-    int n = 0;
+  int any_nan = 0;
 #pragma unroll
-    for (int w = 0; w < WPR; ++w) n |= nan_seen[wave + w];
-    a.sx[row] = n ? __uint_as_float(0x7fc00000u) : scale;
+  for (int w = 0; w < WPR; ++w) {
+    amax = fmaxf(amax, part[wave / WPR * WPR + w]);
+    any_nan |= nan_seen[wave / WPR * WPR + w];
   }
+  const QuantScale q(amax);
+#pragma unroll
+  for (int i = 0; i < NCH; ++i)
+    if (live && (i * WPR + sub) * 64 + lane < nchunk) {
+      unsigned int codes[EPC / 4];
+      quantize_chunk<EPC>(f[i], q, codes);
+      RQ::store_chunk(a, row, i * WPR + sub, lane, codes);
+    }
+  if (live && sub == 0 && lane == 0) a.sx[row] = any_nan ? __uint_as_float(0x7fc00000u) : q.scale;
 }
 
 template <int NCH, int EPC, int WPR, bool ACT, bool NTL>
@@ -138,9 +133,11 @@ static int launch_rowshare(const QuantArgs& a, hipStream_t stream) {
 
 template <int NCH, int EPC, bool LN, bool ACT>
 static int launch_quant(const QuantArgs& a, hipStream_t stream) {
-  const int64_t blocks = (a.M + kQuantWavesPerBlock - 1) / kQuantWavesPerBlock;
-  hipLaunchKernelGGL((quant_rowwise_bf16_kernel<NCH, EPC, LN, ACT>), dim3((unsigned int)blocks),
-                     dim3(64 * kQuantWavesPerBlock), 0, stream, a);
+  const dim3 grid((unsigned int)((a.M + kQuantWavesPerBlock - 1) / kQuantWavesPerBlock)), block(64 * kQuantWavesPerBlock);
+  // (the widths of the encoders' rows: built for those)
+  constexpr bool MAY_FIT = EPC == 4 || NCH == 2 || NCH == 10;
+  if (MAY_FIT && a.K == 64 * EPC * NCH) hipLaunchKernelGGL((quant_rowwise_bf16_kernel<NCH, EPC, LN, ACT, MAY_FIT>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((quant_rowwise_bf16_kernel<NCH, EPC, LN, ACT, false>), grid, block, 0, stream, a);
   return check_launch("quant_rowwise_bf16_kernel");
 }
 
