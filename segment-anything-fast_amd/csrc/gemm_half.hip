@@ -7,17 +7,19 @@ namespace samfast {
 // The kernel for a product: columns / 32 of a tile; 8 and 10 the resident kernel (kHalfTall: with 320 rows and 256 columns), 3 to 5 the
 // split one, 0 none (the library's product and a pass of its own for GELU or residual are ahead).  The lines, by the rounds of the
 // CUs and the share of their time that makes output (us, library with its pass / here, residuals with the LayerNorm behind them):
-//   GELU: from half of the CUs on.  4096 x 768 -> 3072 33.8 / 28.7, 4096 x 1280 -> 5120 75.3 / 51.8, 20480 x 1024 -> 4096 188 / 165,
-//     65536 x 1280 -> 5120 863 / 768.
-//   plain: up to 8 rounds, 0.7.  4096 x 1024 -> 3072 27.7 / 26.2, 8192 x 768 -> 2304 35.8 / 30.7, 20480 x 1024 -> 3072 107 / 102, 32768 x 768 ->
-//     2304 119 / 104; but 4096 x 768 -> 2304 (0.56) 19.8 / 20.2, 65536 x 768 -> 2304 (9 rounds) 201 / 221.
-//   residual: 128-row tiles where the CUs hold them all at once.  4096 x 1280 -> 1280 31.1 / 23.6, 4096 x 5120 -> 1280 61.3 / 55.9.
-//     Else 320 x 256 where that fills its rounds from 0.8 on: 20480 x 4096 -> 1024 (1.0) 171 / 142, 20480 x 1024 -> 1024 76.6 / 56.3, 24576 x 3072
-//     -> 768 (0.9) 148 / 109, 40960 x 5120 -> 1280 (three rounds, 0.83) 553 / 472, 57344 x 5120 -> 1280 (four, 0.88) 702 / 628, 36864 x
-//     4096 -> 1024 (two, 0.9) 290 / 259.
-//     Else 256 x 256, on long loops within one round from 0.7 on (12288 x 5120 -> 1280 138 / 132; 0.5: 8192 x 4096 -> 1024 69 / 83, two
-//     rounds: 32768 x 4096 -> 1024 236 / 248), on short ones up to four rounds from 0.75 on (12288 x 1024 -> 1024 42.6 / 40.4, 32768 x
-//     1280 -> 1280 181 / 147; 0.5: 8192 x 1024 -> 1024 31.1 / 33.9, five rounds: 65536 x 1280 -> 1280 276 / 284).
+//   GELU: from half of the CUs on.  4096 x 768 -> 3072 34.2 / 27.6, 4096 x 1280 -> 5120 77.1 / 50.1, 20480 x 1024 -> 4096 188 / 152,
+//     65536 x 1280 -> 5120 856 / 729.
+//   plain: from 0.7 on, on loops shorter than 1024 up to 8 rounds.  4096 x 1024 -> 3072 28.5 / 26.6, 8192 x 768 -> 2304 38.8 / 30.8, 20480 x 1024 -> 3072
+//     106 / 99.5, 32768 x 768 -> 2304 120 / 101, 57344 x 1024 -> 3072 (11 rounds) 299 / 280, 49152 x 1280 -> 3840 (12) 370 / 361; but 4096 x 768 -> 2304
+//     (0.56) 20.1 / 21.0, 65536 x 768 -> 2304 (9 rounds) 196 / 213.
+//   residual: 128-row tiles where the CUs hold them all at once.  4096 x 1280 -> 1280 28.6 / 24.9, 4096 x 5120 -> 1280 61 / 53.
+//     Else 320 x 256 where that fills its rounds from 0.8 on: 20480 x 4096 -> 1024 (1.0) 164 / 137, 20480 x 1024 -> 1024 74.3 / 52.7, 24576 x 3072
+//     -> 768 (0.9) 146 / 102, 40960 x 5120 -> 1280 (three rounds, 0.83) 545 / 450, 57344 x 5120 -> 1280 (four, 0.88) 700 / 622, 57344 x
+//     1280 -> 1280 (four, 0.88) 255 / 233.
+//     Else 256 x 256, on long loops within one round from 0.7 on (12288 x 5120 -> 1280 140 / 126; 0.62: 8192 x 5120 -> 1280 alone 104 / 104, an
+//     encoder of two images 4 % slower; two rounds: 32768 x 4096 -> 1024 231 / 238), on short ones up to four rounds from 0.55 on (0.56: 12288
+//     x 768 -> 768 39.8 / 30.5, 0.62: 8192 x 1280 -> 1280 45.2 / 40.2, 16384 x 1280 -> 1280 88.3 / 75.4, 0.75: 12288 x 1024 -> 1024 42.4 / 38.3; 0.5: 8192 x 1024 -> 1024
+//     32.2 / 33.6, five rounds: 65536 x 1280 -> 1280 276 / 278).
 // The rows decide, so the order in which a product's terms are summed, and with it the last bits of an image's embedding in the half
 // types, follows the batch, as it does with the library's kernels (one ViT-H image: 3-5 split K, five ViT-L images: 320-row tiles, the
 // library in between; 0.016 and 2e-4 of the embedding's norm).  int8 sums are integers: an image comes out the same in any batch.
@@ -38,8 +40,8 @@ static int half_choose(int64_t M, int N, int K, int epi) {
   const PPChoice c = pp_choose(M, N, K / 64, epi == PP_RESIDUAL);
   if (c.tn == 0) return 0;
   bool pays = c.used >= 0.5;
-  if (epi == PP_PLAIN) pays = c.rounds <= 8 && c.used >= 0.7;
-  if (epi == PP_RESIDUAL) pays = c.tm == 5 ? c.used >= 0.8 : K >= 2048 ? c.rounds == 1 && c.used >= 0.7 : c.rounds <= 4 && c.used >= 0.75;
+  if (epi == PP_PLAIN) pays = c.used >= 0.7 && (c.rounds <= 8 || K >= 1024);
+  if (epi == PP_RESIDUAL) pays = c.tm == 5 ? c.used >= 0.8 : K >= 2048 ? c.rounds == 1 && c.used >= 0.7 : c.rounds <= 4 && c.used >= 0.55;
   return pays ? (c.tm == 5 ? kHalfTall : c.tn) : 0;
 }
 

@@ -26,17 +26,20 @@ static PPArgs pp_args(const GemmArgs& g) {
 
 static bool pays(int epi, int K, const PPChoice& c) {
   // The lines, by the share of the CUs' time that makes output (us, the other members / this one, K-block major, random codes):
-  //   plain, K >= 1280, 0.75: 0.78 (5000 rows -> 5120) 43.1 / 38.1, 0.94 (4096 -> 3840) 27.1 / 22.4, 1.0 (65536 -> 3840) 310 / 284,
+  //   plain, K >= 1280, 0.75: 0.78 (5000 rows -> 5120) 43.1 / 38.1, 0.94 (4096 -> 3840) 26.9 / 21.0, 1.0 (65536 -> 3840) 309 / 263,
   //     K = 5120, 1.0 (65536 -> 3840) 1126 / 994; but 0.59 (5000 -> 3840) 30.0 / 37.6
-  //   shorter loops, 0.85, and at K = 768 not within one round: 0.94 (20480 x 768 -> 3072) 58.7 / 56.4, 1.0 (4096 x 1024 -> 4096) 23.4 /
-  //     20.3; but 0.75 (12288 x 768 -> 3072) 38.0 / 40.5, 0.94 (5000 x 768 -> 3072, one round) 19.1 / 18.9
-  //   residual, K >= 2048, 0.7: 0.75 (12288 x 4096 -> 1024) 58.4 / 51.9, 0.94 (12288 x 5120 -> 1280) 85.0 / 68.6, 1.0 (20480 x 4096 -> 1024, 320
-  //     rows) 93.9 / 72.6, (65536 x 5120 -> 1280) 401 / 337, 0.88 (28672 x 5120 -> 1280, 320 rows) 200 / 161; but 0.66 (28672 x 3072 -> 768) 75.5 / 80.1
-  //   residual, K from 1280 on, 0.9, from 1024 on within one round: 0.94 (24576 x 1280 -> 1280) 53.7 / 53.6, 1.0 (65536) 138 / 135, 1.0 (20480 x
-  //     1024 -> 1024, 320 rows) 35.6 / 31.7; but 0.88 (57344 x 1280 -> 1280) 123.9 / 126.6, K = 1024 in two rounds (40960 -> 1024) 57.2 / 61.9, and
-  //     inside an encoder 0.75 (12288 x 1024 -> 1024) and K = 768 (24576 -> 768) cost 1 % of it (alone 32.0 / 24.0 and 30.4 / 28.0)
-  if (epi == EPI_RESIDUAL_BF16) return K >= 2048 ? c.used >= 0.7 : c.used >= 0.9 && (K >= 1280 || (K >= 1024 && c.rounds == 1));
-  return K >= 1280 ? c.used >= 0.75 : c.used >= 0.85 && (K >= 1024 || c.rounds > 1);
+  //   shorter loops, 0.8: 0.84 (12288 x 768 -> 2304) 31.0 / 26.5, 0.9 (8192 x 768 -> 2304) 23.4 / 20.4, 0.84 in four rounds (24576 x 768 -> 2304) 52.3 /
+  //     50.1, 1.0 (4096 x 1024 -> 4096) 23.1 / 20.1; but 0.75 (8192 x 768 -> 3072) 25.7 / 25.8, and 0.75 at K = 1024 (8192 -> 3072, alone 31.0 / 30.2)
+  //     cost an encoder of two images 1 %
+  //   residual, K >= 2048, 0.7, within one round 0.55: 0.56 (12288 x 3072 -> 768) 38.6 / 36.6, 0.62 (8192 x 5120 -> 1280) 59.5 / 54.6, 0.75 (12288 x 4096 ->
+  //     1024) 54.1 / 49.8, 1.0 (20480 x 4096 -> 1024, 320 rows) 86.5 / 64.3, (65536 x 5120 -> 1280) 402 / 336, 0.88 (28672 x 5120 -> 1280, 320 rows) 190 /
+  //     149; but 0.5 (8192 x 4096 -> 1024) 40.6 / 45.5, 0.66 in two rounds (28672 x 3072 -> 768) 70.4 / 71.1
+  //   residual, shorter loops, 0.85: 0.94 (20480 x 768 -> 768) 22.4 / 19.8, two rounds (40960 x 768 -> 768) 41.3 / 34.4, 0.88 (28672 x 1024 -> 1024) 43.9 / 38.5, 1.0
+  //     (20480 x 1024 -> 1024, 320 rows) 31.9 / 28.4, 0.88 in five rounds (57344 x 1280 -> 1280) 124.2 / 117.2; but 0.75 (24576 x 1024 -> 1024) 35.7 / 37.5, 0.83
+  //     (32768 x 1280 -> 1280) 63.2 / 66.3; from K = 1280 on 0.77 in up to two rounds: 0.78 (20480 -> 1280) 48.5 / 41.5
+  if (epi != EPI_RESIDUAL_BF16) return c.used >= (K >= 1280 ? 0.75 : 0.8);
+  if (K >= 2048) return c.used >= (c.rounds == 1 ? 0.55 : 0.7);
+  return c.used >= (K >= 1280 && c.rounds <= 2 ? 0.77 : 0.85);
 }
 
 bool gemm_i8_pingpong_reads_rows(int64_t M, int N, int K) {

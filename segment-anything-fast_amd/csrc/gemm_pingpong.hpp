@@ -722,14 +722,16 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_split_kernel(PPArgs a) {
 
 // ---- host side ---------------------------------------------------------------------------------------------------------
 // Time of a launch in units of one 16-column fragment of 64 rows for one k tile: rounds of the CUs, each as long as its k tiles and a start
-// and an end worth eight more of them, a tile two or three and a half fragments more expensive than its columns.  The tile with the
+// and an end worth eight more of them, a tile two to three fragments more expensive than its columns.  The tile with the
 // least; `used`: the share of those CU-cycles that makes output.
-// us, 256 / 320 columns: int8 inside the encoder 65536 x 1280 -> 3840 284 / 301; 4096 x 1280 -> 5120 (320 / 256 tiles) 33.0 / 28.1, 8192 x 1280 ->
-// 5120 (three / two rounds) 57.7 / 52.6, 20480 x 1280 -> 5120 (seven / five) 129.5 / 124.1.  (192 columns, at an
-// equal number of columns per CU, lost: 65536 x 1280 -> 3840 284 / 305, 4096 x 1024 -> 3072 17.5 / 18.3.)
+// us, 256 / 320 columns: int8 4096 x 1280 -> 5120 (two rounds / one) 33.1 / 27.6, 8192 x 1280 -> 5120 (three / two) 53.5 / 52.1, 32768 x 1280 -> 3840 (eight /
+// six) 151 / 139, 24576 x 1280 -> 5120 (eight / six) 145 / 138, but 24576 x 1280 -> 3840 (six / five) 110.5 / 112.4, at equal numbers of columns
+// per CU 65536 x 1280 -> 3840 276 / 275; loops under ten k tiles pay more for the wide tile's end: 24576 x 768 -> 3072 (five / four)
+// 64.4 / 70.3, 24576 x 1024 -> 3072 (five / four) 77.7 / 81.3, 12288 x 1024 -> 3072 (three / two) 44.4 / 42.1.  bf16 12288 x 1280 -> 5120 (four / three) 141 / 134,
+// 24576 x 1280 -> 5120 276 / 261, but 24576 x 1024 -> 3072 121 / 124.  (192 columns, at an equal number of columns per CU, lost.)
 // The residual's registers leave no room for 320 columns, but for 320 rows, which few columns and many rows fill better.  256 / 320
-// rows: int8 20480 x 4096 -> 1024 (two rounds / one) 97.1 / 72.6, 24576 x 3072 -> 768 76.8 / 55.6, 53248 x 4096 -> 1024 (four / three) 220.6 /
-// 203.2, in equal rounds 16384 x 4096 -> 1024 60.2 / 64.4, 65536 x 5120 -> 1280 337 / 372.
+// rows: int8 20480 x 4096 -> 1024 (two rounds / one) 89.2 / 67.6, 24576 x 3072 -> 768 69.6 / 51.0, 57344 x 4096 -> 1024 (four / three) 215 /
+// 203, 57344 x 5120 -> 1280 (five / four) 315 / 313, bf16 696 / 622; in equal rounds 16384 x 4096 -> 1024 bf16 103 / 112.
 struct PPChoice {
   int tm, tn;
   int64_t rounds;
@@ -748,8 +750,8 @@ static inline PPChoice pp_choose(int64_t M, int N, int nk, bool residual) {
     }
   };
   candidate(4, 8, 10.0);
-  if (residual) candidate(5, 8, 12.5);
-  else candidate(4, 10, 13.5);
+  if (residual) candidate(5, 8, 12.4);
+  else candidate(4, 10, nk < 10 ? 13.2 : 12.5);
   return best;
 }
 

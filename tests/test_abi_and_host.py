@@ -80,6 +80,18 @@ def test_the_half_product_knob_names_built_tiles_only():
                 assert lib.samfast_linear_half_pays(4096, 4096, 1280, epilogue) == (value in tiles), (value, epilogue)
 
 
+def test_the_half_products_lines():
+    """Both sides of each line between the library's kernels and the framework's: (M, N, K, epilogue, paid)."""
+    from samfast_amd import _lib
+    lib = _lib.load()
+    none, gelu, residual = _lib.EPILOGUE_NONE, _lib.EPILOGUE_GELU, _lib.EPILOGUE_RESIDUAL
+    for *call, paid in ((4096, 2304, 768, none, 0), (4096, 3072, 768, none, 1), (57344, 2304, 768, none, 1), (65536, 2304, 768, none, 0),
+                        (65536, 3072, 1024, none, 1), (4096, 2304, 768, gelu, 1), (2048, 2304, 768, gelu, 0),
+                        (8192, 1024, 1024, residual, 0), (12288, 768, 768, residual, 1), (65536, 1280, 1280, residual, 0),
+                        (57344, 1280, 1280, residual, 1), (8192, 1280, 5120, residual, 0), (12288, 1280, 5120, residual, 1)):
+        assert lib.samfast_linear_half_pays(*call) == paid, call
+
+
 def test_fused_quant_gemm_refuses_outputs_its_quantiser_cannot_address():
     """lin1-shaped call with M * N >= 2^31: the in-kernel quantiser's 32-bit offsets would wrap, so
     the entry point (and its allocation-free form) refuses before anything is launched."""
