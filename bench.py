@@ -392,9 +392,10 @@ def gemm_variants(batch=16, width=1280):
             del xq, wq
         res["rows"][f"{name} {M}x{N}x{K}"] = row
         del y, resid
-    # the 2:4-sparse kernel's two forms on the MLP shapes (weights pruned to 2:4, Gaussian codes)
-    sparse_variants = [("one workgroup per tile", {"SAMFAST_SPARSE_PERSIST": 0}),
-                       ("resident workgroups", {"SAMFAST_SPARSE_PERSIST": 2})]
+    # the 2:4-sparse kernels on the MLP shapes (weights pruned to 2:4, Gaussian codes)
+    sparse_variants = [("one workgroup per tile", {"SAMFAST_SPARSE_TURNS": 0}),
+                       ("resident workgroups", {"SAMFAST_SPARSE_PERSIST": 2}),
+                       ("by turns (default)", {"SAMFAST_SPARSE_TURNS": 1})]
     for name, N, K, epi in shapes[2:]:
         w = (torch.randn((N, K), device=dev, generator=g) * 28).round().clamp(-127, 127)
         w4 = w.view(N, K // 4, 4)

@@ -20,6 +20,7 @@
 //   wc   (K/64, N, 32) int8   byte 16*h + 2*g + e of row n, block kb = W[n, 64*kb + k(g,h) + p_e]
 //   widx (K/64, N, 2)  int32  word h of row n, block kb = the eight position nibbles
 //
+// Outputs of whole rounds of larger tiles are another kernel's (gemm_i8_sp24_turns.hip); this one takes the others.
 // Tiling: a 256-thread workgroup owns 256 W rows x 128 X rows; its four wavefronts sit
 // 2x2, each holding 128 x 64 as 4x2 MFMA tiles (128 accumulators), two workgroups per CU.
 // One k-step of 64 dense k per tile; tiles travel global memory -> LDS directly
@@ -538,6 +539,7 @@ static int sparse_common(int epi, const int8_t* xq, const float* sx, const int8_
   SF_REQUIRE(total < (1ll << 30), "gemm_i8_sparse24: too many tiles");
   if (gemm_i8_sp24_skinny_covers(epi, a)) return gemm_i8_sp24_skinny_launch(a, stream);
   if (gemm_i8_sp24_persist_covers(epi, a)) return gemm_i8_sp24_persist_launch(epi, a, stream);
+  if (gemm_i8_sp24_turns_covers(epi, a)) return gemm_i8_sp24_turns_launch(epi, a, stream);
   const unsigned int grid = (unsigned int)(((total + 7) / 8) * 8);
   // The K split where a CU has one tile and the loop is long (us, one group / two; SAMFAST_GEMM_SPLITK=0 off, 2
   // wherever it is built).  K = 5120, while every tile has a CU: 60 tiles (1500 x 5120 -> 1280) 24.9 / 22.0, 160 (4096) 29.5 /

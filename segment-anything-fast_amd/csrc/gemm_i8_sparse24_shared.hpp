@@ -52,6 +52,10 @@ SF_DEVICE int sp_slot_to_row(int slot) {
 bool gemm_i8_sp24_persist_covers(int epi, const SparseArgs& a);
 int gemm_i8_sp24_persist_launch(int epi, const SparseArgs& a, hipStream_t stream);
 
+// Large tiles, two wavefronts per SIMD by turns (gemm_i8_sp24_turns.hip): scale + bias and residual epilogues.  tiles_x / tiles_w are recomputed.
+bool gemm_i8_sp24_turns_covers(int epi, const SparseArgs& a);
+int gemm_i8_sp24_turns_launch(int epi, const SparseArgs& a, hipStream_t stream);
+
 // Small tiles with the K range dealt out over eight wavefronts (gemm_i8_sp24_skinny.hip): scale + bias
 // epilogue, few rows.  tiles_x / tiles_w are recomputed.
 bool gemm_i8_sp24_skinny_covers(int epi, const SparseArgs& a);

@@ -42,6 +42,7 @@ enum Knob {
   KNOB_ATTN_SPLIT,        // SAMFAST_ATTN_SPLIT: global attention with the keys split between two wavefronts (other bits), 0 = never, 1 = head_dim 64, 2 = always
   KNOB_ATTN_WINDOW_ROWS,  // SAMFAST_ATTN_WINDOW_ROWS: 1 = window keys as grid rows padded to 16 (attn_window_rows_kernel) where built
   KNOB_SPARSE_PERSIST,    // SAMFAST_SPARSE_PERSIST: 2:4 GEMM, 0 = one workgroup per tile (default), 1 = resident workgroups from two tiles each on, 2 wherever built
+  KNOB_SPARSE_TURNS,      // SAMFAST_SPARSE_TURNS: 2:4 GEMM by turns (gemm_i8_sp24_turns.hip), 0 off, 1 where it pays, 8 / 10 wherever built, channels / 32 of the tile
   KNOB_COUNT
 };
 constexpr int kKnobUnset = INT32_MIN;

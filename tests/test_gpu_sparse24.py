@@ -147,6 +147,51 @@ def test_sparse24_resident_form_agrees(M, N, K, layout):
         assert torch.equal(dense.view(torch.int16), want.view(torch.int16)), epi
 
 
+@pytest.mark.parametrize("M,N,K,layout", [
+    (256, 256, 640, "kb64"),        # one tile of the narrow form, the shortest loop; the wide one does not fit
+    (257, 328, 640, "rows"),        # tiles moved back over one row and over 8 channels
+    (300, 640, 1280, "kb64"),
+    (2001, 1288, 768, "kb64"),      # both edges ragged
+    (511, 320, 5120, "rows"),
+    (20500, 1288, 640, "kb64"),     # more tiles than CUs: one tile's output under the next one's first products
+    (26300, 5120, 640, "rows"),     # 269 MB of output: streamed stores
+])
+def test_sparse24_by_turns_agrees(M, N, K, layout):
+    """The 256-row tiles by turns against the 128-row kernel, bit for bit: scale + bias, without bias, residual, residual in place, rows
+    of the output further apart than its columns (what lies between them stays)."""
+    from samfast_amd import _lib, ops
+    print(f"case sparse turns M={M} N={N} K={K} {layout}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    xq = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8, device="cuda")
+    wq = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device="cuda")
+    sx = torch.rand(M, generator=g, device="cuda") * 1e-2 + 1e-3
+    sw = torch.rand(N, generator=g, device="cuda") * 1e-3 + 1e-4
+    bias = torch.randn(N, generator=g, device="cuda") * 0.1
+    res = torch.randn((M, N), generator=g, device="cuda").to(torch.bfloat16)
+    wc, widx = ops.prune24_pack(wq)
+    L = _lib.LAYOUT_ROWMAJOR
+    if layout == "kb64":
+        L = _lib.LAYOUT_KB64
+        xq = ops.to_kb64(xq)
+
+    def run(turns, epi, b, residual=None, out=None):
+        with _lib.knobs(SAMFAST_SPARSE_TURNS=turns, SAMFAST_GEMM_SKINNY=0):
+            return ops.gemm_i8_sparse24_fused(xq, sx, wc, widx, sw, b, epi, residual=residual, out=out, layout=L)
+
+    plain = run(0, _lib.EPILOGUE_NONE, bias)
+    bare = run(0, _lib.EPILOGUE_NONE, None)
+    summed = run(0, _lib.EPILOGUE_RESIDUAL, bias, res)
+    for turns in (8, 10):
+        assert torch.equal(run(turns, _lib.EPILOGUE_NONE, bias), plain), turns
+        assert torch.equal(run(turns, _lib.EPILOGUE_NONE, None), bare), turns
+        assert torch.equal(run(turns, _lib.EPILOGUE_RESIDUAL, bias, res), summed), turns
+        inplace = res.clone()
+        assert torch.equal(run(turns, _lib.EPILOGUE_RESIDUAL, bias, inplace, inplace), summed), turns
+        wide = torch.full((M, N + 24), 7.0, dtype=torch.bfloat16, device="cuda")
+        run(turns, _lib.EPILOGUE_NONE, bias, None, wide[:, 8:8 + N])
+        assert torch.equal(wide[:, 8:8 + N], plain) and bool((wide[:, :8] == 7).all()) and bool((wide[:, 8 + N:] == 7).all()), turns
+
+
 def test_sparse24_full_size_equals_dense_kernel():
     """lin1 of ViT-H at batch 16 (65536 x 5120 x 1280): accumulators of the sparse kernel
     equal those of the dense kernel on the pruned weight, compared on the GPU."""
