@@ -192,7 +192,9 @@ int samfast_gemm_i8_scale_bias(
  * samfast_linear_i8_workspace(M, N, K, layout) bytes of device memory, 16-byte aligned, contents
  * irrelevant before and after; may be NULL where that is 0.  The size function returns
  * SAMFAST_E_INVALID for a negative or zero dimension or an unknown layout; with
- * SAMFAST_LAYOUT_SPARSE24 it answers for samfast_linear_i8_sparse24.
+ * SAMFAST_LAYOUT_SPARSE24 it answers for samfast_linear_i8_sparse24.  Where
+ * samfast_linear_i8_one_launch(M, N, K, layout) is 1, a call whose x and y do not share memory uses no
+ * workspace either: it may be NULL.
  */
 #define SAMFAST_LAYOUT_SPARSE24 2  /* samfast_linear_i8_workspace only */
 int samfast_linear_i8(
@@ -200,6 +202,7 @@ int samfast_linear_i8(
     void* y, int64_t ldy, void* workspace,
     int64_t M, int N, int K, int dtype, int layout, void* stream);
 int64_t samfast_linear_i8_workspace(int64_t M, int N, int K, int layout);
+int samfast_linear_i8_one_launch(int64_t M, int N, int K, int layout);
 
 /*
  * A block's Linear in the half types: y = x w^T + bias (summed in fp32, rounded to `dtype`), then by `epilogue`

@@ -17,7 +17,7 @@ extern "C" {
  * Kernel variants are chosen by knobs, each named like the environment variable that gives its
  * initial value (read once per process): SAMFAST_GEMM_TM, SAMFAST_GEMM_WG3, SAMFAST_GEMM_TILE,
  * SAMFAST_GEMM_PERSIST, SAMFAST_GEMM_PERSIST_SKEW, SAMFAST_GEMM_PERSIST_PRIO,
- * SAMFAST_GEMM_PINGPONG, SAMFAST_GEMM_HALF, SAMFAST_GEMM_SPLITK, SAMFAST_GEMM_ONCE, SAMFAST_GEMM_STRIP, SAMFAST_GEMM_LINEAR_SMALL, SAMFAST_GEMM_SKINNY,
+ * SAMFAST_GEMM_PINGPONG, SAMFAST_GEMM_HALF, SAMFAST_GEMM_SPLITK, SAMFAST_GEMM_ONCE, SAMFAST_GEMM_STRIP, SAMFAST_GEMM_LINEAR_SMALL, SAMFAST_GEMM_LINEAR_BAND, SAMFAST_GEMM_SKINNY,
  * SAMFAST_ATTN_WAVES, SAMFAST_ATTN_SPLIT, SAMFAST_ATTN_WINDOW_ROWS, SAMFAST_SPARSE_PERSIST, SAMFAST_SPARSE_TURNS.  This
  * call sets one (`unset` != 0: back to "not given", `value` ignored).  The knobs move time; every
  * variant of a kernel returns the same bits, with three exceptions that sum in another order:

@@ -30,7 +30,7 @@ int check_launch(const char* what) {
 
 static const char* const kKnobNames[KNOB_COUNT] = {
     "SAMFAST_GEMM_TM",      "SAMFAST_GEMM_WG3",    "SAMFAST_GEMM_TILE",
-    "SAMFAST_GEMM_PERSIST", "SAMFAST_GEMM_PERSIST_SKEW", "SAMFAST_GEMM_PERSIST_PRIO", "SAMFAST_GEMM_PINGPONG", "SAMFAST_GEMM_HALF", "SAMFAST_GEMM_SPLITK", "SAMFAST_GEMM_ONCE", "SAMFAST_GEMM_STRIP", "SAMFAST_GEMM_LINEAR_SMALL", "SAMFAST_GEMM_SKINNY", "SAMFAST_ATTN_WAVES", "SAMFAST_ATTN_SPLIT", "SAMFAST_ATTN_WINDOW_ROWS",
+    "SAMFAST_GEMM_PERSIST", "SAMFAST_GEMM_PERSIST_SKEW", "SAMFAST_GEMM_PERSIST_PRIO", "SAMFAST_GEMM_PINGPONG", "SAMFAST_GEMM_HALF", "SAMFAST_GEMM_SPLITK", "SAMFAST_GEMM_ONCE", "SAMFAST_GEMM_STRIP", "SAMFAST_GEMM_LINEAR_SMALL", "SAMFAST_GEMM_LINEAR_BAND", "SAMFAST_GEMM_SKINNY", "SAMFAST_ATTN_WAVES", "SAMFAST_ATTN_SPLIT", "SAMFAST_ATTN_WINDOW_ROWS",
     "SAMFAST_SPARSE_PERSIST", "SAMFAST_SPARSE_TURNS"};
 static int g_knobs[KNOB_COUNT];
 static pthread_once_t g_knobs_once = PTHREAD_ONCE_INIT;

@@ -1227,9 +1227,21 @@ extern "C" int64_t samfast_linear_i8_workspace(int64_t M, int N, int K, int layo
   using namespace samfast;
   SF_REQUIRE(M > 0 && N > 0 && K > 0 && layout >= SAMFAST_LAYOUT_ROWMAJOR && layout <= SAMFAST_LAYOUT_SPARSE24,
              "linear_i8_workspace: bad shape M=%lld N=%d K=%d or layout %d", (long long)M, N, K, layout);
-  if (linear_i8_small_covers(M, N, K, layout == SAMFAST_LAYOUT_SPARSE24)) return 0;
+  if (layout != SAMFAST_LAYOUT_SPARSE24 && linear_i8_small_any_alignment(M, K) && linear_i8_small_covers(M, N, K, false)) return 0;
   const int64_t weights = layout == SAMFAST_LAYOUT_ROWMAJOR && linear_reorders_weights(M, N, K) ? (int64_t)N * K : 0;
   return linear_codes_bytes(M, K) + linear_scales_bytes(M) + weights;
+}
+
+extern "C" int samfast_linear_i8_one_launch(int64_t M, int N, int K, int layout) {
+  using namespace samfast;
+  if (layout == SAMFAST_LAYOUT_SPARSE24) return linear_i8_small_covers(M, N, K, true);
+  return linear_i8_small_covers(M, N, K, false) || linear_i8_band_covers(M, N, K);
+}
+
+// Whether rows of x and of y may share memory: one launch reads some while it writes others.
+static bool rows_may_meet(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t M, int N, int K) {
+  const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
+  return x0 < y0 + 2 * (uintptr_t)((M - 1) * ldy + N) && y0 < x0 + 2 * (uintptr_t)((M - 1) * ldx + K);
 }
 
 extern "C" int samfast_linear_i8(const void* x, int64_t ldx, const int8_t* wq, const float* sw, const float* bias,
@@ -1237,11 +1249,15 @@ extern "C" int samfast_linear_i8(const void* x, int64_t ldx, const int8_t* wq, c
                                  int layout, void* stream) {
   using namespace samfast;
   SF_REQUIRE(layout == SAMFAST_LAYOUT_ROWMAJOR || layout == SAMFAST_LAYOUT_KB64, "linear_i8: unknown layout %d", layout);
-  if (M > 0 && linear_i8_small_covers(M, N, K, false)) {
+  const bool small = M > 0 && linear_i8_small_covers(M, N, K, false), any_alignment = small && linear_i8_small_any_alignment(M, K);
+  if (any_alignment || (M > 0 && (small || linear_i8_band_covers(M, N, K)) && !rows_may_meet(x, ldx, y, ldy, M, N, K))) {
     SF_REQUIRE(dtype == SAMFAST_BF16, "linear_i8: only bf16");
-    SF_REQUIRE(x && wq && sw && y && aligned16(x) && aligned16(wq) && aligned16(y) && (linear_i8_small_any_alignment(M, K) || (aligned16(sw) && aligned16(bias))),
+    SF_REQUIRE(x && wq && sw && y && aligned16(x) && aligned16(wq) && aligned16(y) && (any_alignment || (aligned16(sw) && aligned16(bias))),
                "linear_i8: null or unaligned pointer");
     SF_REQUIRE(ldx >= K && ldx % 8 == 0 && ldy >= N && ldy % 8 == 0, "linear_i8: row strides must be multiples of 8, >= K and >= N");
+    if (!small)
+      return linear_i8_band_launch(reinterpret_cast<const unsigned short*>(x), ldx, wq, sw, bias, reinterpret_cast<unsigned short*>(y), ldy,
+                                   (int)M, N, K, layout, reinterpret_cast<hipStream_t>(stream));
     return linear_i8_small_launch(reinterpret_cast<const unsigned short*>(x), ldx, wq, nullptr, sw, bias, reinterpret_cast<unsigned short*>(y), ldy,
                                   (int)M, N, K, layout, reinterpret_cast<hipStream_t>(stream));
   }
@@ -1268,7 +1284,7 @@ extern "C" int samfast_linear_i8_sparse24(const void* x, int64_t ldx, const int8
                                           const float* sw, const float* bias, void* y, int64_t ldy, void* workspace,
                                           int64_t M, int N, int K, int dtype, void* stream) {
   using namespace samfast;
-  if (M > 0 && linear_i8_small_covers(M, N, K, true)) {
+  if (M > 0 && linear_i8_small_covers(M, N, K, true) && !rows_may_meet(x, ldx, y, ldy, M, N, K)) {
     SF_REQUIRE(dtype == SAMFAST_BF16, "linear_i8_sparse24: only bf16");
     SF_REQUIRE(x && wc && widx && sw && y && aligned16(x) && aligned16(wc) && aligned16(widx) && aligned16(y) && aligned16(sw) && aligned16(bias),
                "linear_i8_sparse24: null or unaligned pointer");

@@ -27,6 +27,7 @@ namespace {
 
 decltype(&samfast_linear_i8) p_linear_i8;
 decltype(&samfast_linear_i8_workspace) p_linear_i8_workspace;
+decltype(&samfast_linear_i8_one_launch) p_linear_i8_one_launch;
 decltype(&samfast_linear_i8_sparse24) p_linear_i8_sparse24;
 decltype(&samfast_attn_relpos_bias_fwd) p_attn_bias;
 
@@ -34,6 +35,7 @@ struct Bound { const char* name; void** slot; };
 const Bound kBound[] = {
     {"samfast_linear_i8", reinterpret_cast<void**>(&p_linear_i8)},
     {"samfast_linear_i8_workspace", reinterpret_cast<void**>(&p_linear_i8_workspace)},
+    {"samfast_linear_i8_one_launch", reinterpret_cast<void**>(&p_linear_i8_one_launch)},
     {"samfast_linear_i8_sparse24", reinterpret_cast<void**>(&p_linear_i8_sparse24)},
     {"samfast_attn_relpos_bias_fwd", reinterpret_cast<void**>(&p_attn_bias)},
 };
@@ -106,6 +108,12 @@ struct LinearCall {
   }
 };
 
+// bytes of workspace of a call whose output is its own
+int64_t workspace(const LinearCall& c, int layout) {
+  const int N = static_cast<int>(c.N), K = static_cast<int>(c.K);
+  return p_linear_i8_one_launch(c.M, N, K, layout) ? 0 : p_linear_i8_workspace(c.M, N, K, layout);
+}
+
 // linear(x, wq, layout, sw_bits, bias_bits or None): the whole int8 Linear on bf16 rows.
 // wq is (N, K), or (K/64, N, 64) for layout 1.
 PyObject* host_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -122,7 +130,7 @@ PyObject* host_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   c.K = kb ? wq->size(0) * 64 : wq->size(1);
   if (!c.accept(dev)) Py_RETURN_NONE;
   c.M = c.x->numel() / c.K;
-  const int64_t need = p_linear_i8_workspace(c.M, static_cast<int>(c.N), static_cast<int>(c.K), layout);
+  const int64_t need = workspace(c, layout);
   if (need < 0) Py_RETURN_NONE;
   c.allocate(need);
   const int rc = p_linear_i8(ptr(*c.x), c.K, static_cast<const int8_t*>(ptr(*wq)), c.sw_ptr(), c.bias_ptr(), c.y.data_ptr(), c.N,
@@ -148,7 +156,7 @@ PyObject* host_sparse_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   c.K = wc->size(0) * 64;
   if (!c.accept(dev)) Py_RETURN_NONE;
   c.M = c.x->numel() / c.K;
-  const int64_t need = p_linear_i8_workspace(c.M, static_cast<int>(c.N), static_cast<int>(c.K), SAMFAST_LAYOUT_SPARSE24);
+  const int64_t need = workspace(c, SAMFAST_LAYOUT_SPARSE24);
   if (need < 0) Py_RETURN_NONE;
   c.allocate(need);
   const int rc = p_linear_i8_sparse24(ptr(*c.x), c.K, static_cast<const int8_t*>(ptr(*wc)), static_cast<const int32_t*>(ptr(*widx)),

@@ -1,0 +1,347 @@
+// A whole quantised Linear over a band of rows and a range of columns per workgroup: row quantiser, int8 product and the scale + bias
+// epilogue in one launch, for the row counts between linear_i8_small.hip's and those whose products fill the GPU in rounds.
+//
+// Two launches of such a call are mostly starts and ends (4096 x 768 -> 3072: 5 and 15 us for 4.5 us of matrix pipe), the codes go through
+// memory between them, and the host pays for both.  Here every workgroup quantises its 32 or 64 rows itself - once per range of columns,
+// 2 to 14 times in all, which is why ranges are wide, at 64 rows 640 or 768 columns, and why sixteen lanes take a row (one reduction and
+// one division serve four rows) - keeps the codes in LDS for the whole of K and runs on W alone: a ring per wavefront in LDS, a
+// 16-column x 128-byte fragment at a time, whole lines of row-major weights as well as of K-block-major ones; one barrier before the
+// products, one behind them.  Bound (4096 x 768 -> 3072, cycles of a workgroup's 28800): rows and first W through the load path
+// 4000, codes 6000 of vector work, products 11400 (9200 of matrix pipe), scales and output 7300; little of it overlaps, 160 KB of LDS being one workgroup per CU.
+// us on the GPU, two launches / this one: 4096 x 768 -> 3072 22.9 / 18.9, 4096 x 768 -> 768 13 / 8.7, 2048 x 768 -> 3072 16 / 13.1, 16384 x 768 -> 768 34 / 20, 1024 x 1024 -> 3072
+// 13 / 9.7, 512 x 1280 -> 1280 12.1 / 9.2.  Integer sums and the epilogue's arithmetic are those of the other forms: the same bits.
+#include "attn_relpos_shared.hpp"
+#include "gemm_i8_shared.hpp"
+#include "linear_i8_small.hpp"
+#include "quant_row.hpp"
+
+// every fp32 step below is rounded on its own (no fused multiply-add), as in the other forms
+#pragma clang fp contract(off)
+
+namespace samfast {
+
+struct BandArgs {
+  const unsigned short* x;
+  int64_t ldx;
+  const int8_t* w;
+  const float* sw;
+  const float* bias;
+  unsigned short* y;
+  int64_t ldy;
+  int M, N, K;
+  int tiles_m, tiles_n, tiles;
+  int group_m;  // row tiles per scheduling group
+  unsigned int w_pitch, w_kstep;  // bytes between weight rows / between 64-byte k steps: K and 64, or 64 and 64 N (K-block major)
+};
+
+// at most n vector memory operations of this wavefront outstanding (n constant at every use)
+SF_DEVICE void band_wait(int n) {
+  switch (n) {
+#define SF_CASE(H) case H: __builtin_amdgcn_s_waitcnt(0x0F70 | (H)); break
+    SF_CASE(0); SF_CASE(1); SF_CASE(2); SF_CASE(3); SF_CASE(4); SF_CASE(5); SF_CASE(6); SF_CASE(7);
+    SF_CASE(8); SF_CASE(9); SF_CASE(10); SF_CASE(11); SF_CASE(12); SF_CASE(13); SF_CASE(14); SF_CASE(15);
+#undef SF_CASE
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// KMAX: 128 * the chunks of 8 values a lane holds of a row; RF: fragments of 16 rows; NF: fragments of 16 columns of a wavefront;
+// DEPTH: k steps of 128 in a wavefront's ring.  K % 128 == 0, 128 * DEPTH <= K <= KMAX, M >= 16 RF, N >= 128 NF.
+template <int KMAX, int RF, int NF, int DEPTH>
+__global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
+  constexpr int R = 16 * RF, BN = 128 * NF, RPW = 2 * RF, NB = RPW / 4;  // rows, columns; rows of a wavefront, quantised four at a time
+  constexpr int NCH = KMAX / 128;
+  constexpr int SLOT = 2048, RING = NF * DEPTH * SLOT;  // a column fragment: 16 columns x 128 bytes
+  constexpr int CODES = R * KMAX;
+  static_assert(CODES + 8 * RING <= 160 * 1024, "LDS of a CU");
+  static_assert(2 * (NF * DEPTH - 1) <= 15, "wait thresholds");
+  __shared__ __attribute__((aligned(16))) unsigned char lds[CODES + 8 * RING];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lq = lane >> 4;
+  const unsigned int pid = xcd_contiguous_id(blockIdx.x, (unsigned int)a.tiles);
+  if (pid >= (unsigned int)a.tiles) return;  // uniform over the workgroup
+  const unsigned int per_group = (unsigned int)(a.group_m * a.tiles_n);
+  const unsigned int first_m = pid / per_group * a.group_m, in_group = pid % per_group;
+  const unsigned int gsz = min((unsigned int)a.tiles_m - first_m, (unsigned int)a.group_m);
+  // the last tiles are moved back inside (M >= R, N >= BN): rows and columns of two tiles get the same bits twice
+  const int m0 = min((int)(first_m + in_group % gsz) * R, a.M - R);
+  const int n0 = min((int)(in_group / gsz) * BN, a.N - BN) + wave * 16 * NF;
+  const int steps = a.K / 128;
+
+  // ---- the rows: sixteen lanes to a row, chunks lr, lr + 16, .. of eight values (past the row's end: its last ones once more) -----------
+  u32x4 xw[NB][NCH];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const unsigned short* src = a.x + (int64_t)(m0 + wave * RPW + 4 * b + lq) * a.ldx + 8 * lr;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) xw[b][i] = *reinterpret_cast<const u32x4*>(src + 128 * min(i, steps - 1));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // (column scales and bias, needed last, stand between the rows and W: the compiler's waits for the rows, which do not count the
+  // requests of W, then leave those in flight)
+  f32x4 sw[NF], bias[NF];
+  const float* bias_or_sw = a.bias ? a.bias : a.sw;  // (a load under a branch would make the compiler wait here)
+#pragma unroll
+  for (int j = 0; j < NF; ++j) {
+    const int n = n0 + (NF % 2 == 1 && j == NF - 1 ? 16 * j + 4 * lq : 32 * (j / 2) + 8 * lq + 4 * (j & 1));
+    sw[j] = *reinterpret_cast<const f32x4*>(a.sw + n);
+    bias[j] = *reinterpret_cast<const f32x4*>(bias_or_sw + n);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- W: row r of fragment j is 128 bytes at 128 r in its slot, 16-byte chunk c at position c ^ (r / 2 % 8).  Of a pair of fragments
+  // row r is column 8 (r / 4) + 4 (j % 2) + r % 4, so that a lane ends with eight adjacent columns; of a last one alone column r ------------
+  unsigned int w_off[NF][2];
+#pragma unroll
+  for (int j = 0; j < NF; ++j)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int r = 8 * h + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+      const int col = NF % 2 == 1 && j == NF - 1 ? 16 * j + r : 32 * (j / 2) + 8 * (r >> 2) + 4 * (j & 1) + (r & 3);
+      w_off[j][h] = (unsigned int)col * a.w_pitch + (unsigned int)(c >> 2) * a.w_kstep + (unsigned int)(c & 3) * 16u;
+    }
+  unsigned char* ring = lds + CODES + wave * RING;
+  const unsigned int ring_at = (unsigned int)(uintptr_t)((__attribute__((address_space(3))) unsigned char*)ring);
+  const unsigned char* wbase = reinterpret_cast<const unsigned char*>(a.w) + (int64_t)n0 * a.w_pitch;
+  const int64_t w_step = 2 * (int64_t)a.w_kstep;
+  auto load_w = [&](const unsigned char* from, int j, unsigned int slots) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) lds_dma16(from, w_off[j][h], ring_at + slots + j * SLOT + h * 1024);
+  };
+  // request i of the first DEPTH k steps' 2 NF DEPTH, between the rows' chunks
+  auto first_w = [&](int i) __attribute__((always_inline)) {
+    const int d = i / (2 * NF), j = i / 2 % NF, h = i % 2;
+    lds_dma16(wbase + d * w_step, w_off[j][h], ring_at + d * NF * SLOT + j * SLOT + h * 1024);
+  };
+
+  // ---- codes: 128 bytes of every row to a block, chunks at the same positions as W's.  The code wanted is rint(fl(v / scale)) (quant_row.hpp).
+  // q = fl(v * inv), then fl(q + fl(v - q * scale) * inv) with fused multiply-adds is that quotient to its last bit wherever it is
+  // not tiny, without the branch, whose other side, met once per chunk in code that runs once, costs more than the arithmetic here (64
+  // rows of 768 13700 cycles with it, 6000 without).  All pairs of a bf16 row maximum and a bf16 value give the same code both ways. --------
+  float scale[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    float f[NCH][8];
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f[i][2 * e] = bf16_lo_to_f32(xw[b][i][e]);
+        f[i][2 * e + 1] = bf16_hi_to_f32(xw[b][i][e]);
+        amax = __builtin_elementwise_maximum(amax, __builtin_elementwise_maximum(fabsf(f[i][2 * e]), fabsf(f[i][2 * e + 1])));
+      }
+    // over the row's sixteen lanes; a NaN has the largest pattern
+    auto row_max = [](float v) __attribute__((always_inline)) {
+      auto larger = [](float p, float q) { return __uint_as_float(max(__float_as_uint(p), __float_as_uint(q))); };
+      v = larger(v, dpp_f32<0xB1>(v));
+      v = larger(v, dpp_f32<0x4E>(v));
+      v = larger(v, dpp_f32<0x141>(v));
+      return larger(v, dpp_f32<0x140>(v));
+    };
+    amax = row_max(fabsf(amax));
+    const bool row_nan = __float_as_uint(amax) > 0x7f800000u;
+    if (__any(row_nan)) {  // the maximum without them
+      float m = 0.f;
+#pragma unroll
+      for (int i = 0; i < NCH; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(f[i][e]));
+      amax = row_max(m);
+    }
+    const float sc = fmaxf(amax, 1e-5f) / 127.0f;
+    float div = sc;
+    if (__any(__float_as_uint(amax) >= 0x7f800000u)) {  // an infinity in the row: every quotient is 0 or NaN, every code 0
+      const bool inf = __float_as_uint(amax) >= 0x7f800000u;
+      div = inf ? 1.0f : sc;
+#pragma unroll
+      for (int i = 0; i < NCH; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[i][e] = inf ? 0.f : f[i][e];
+    }
+    const float inv = 1.0f / div;
+    const int row = wave * RPW + 4 * b + lq;
+    unsigned char* at = lds + row * 128 + (((lr >> 1) ^ ((row >> 1) & 7)) * 16) + (lr & 1) * 8;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      constexpr int FIRST = 2 * NF * DEPTH, CHUNKS = NB * NCH;
+#pragma unroll
+      for (int w = FIRST * (b * NCH + i) / CHUNKS; w < FIRST * (b * NCH + i + 1) / CHUNKS; ++w) first_w(w);
+      if (i < steps) {  // uniform
+        unsigned int m[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float q = f[i][e] * inv;
+          m[e] = __float_as_uint(fmaf(fmaf(-q, div, f[i][e]), inv, q) + 12582912.0f);  // 1.5 * 2^23: the code in the low byte
+        }
+        u32x2 c;
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+          c[g] = __builtin_amdgcn_perm(m[4 * g + 1], m[4 * g], 0x0c0c0400u) | __builtin_amdgcn_perm(m[4 * g + 3], m[4 * g + 2], 0x04000c0cu);
+        *reinterpret_cast<u32x2*>(at + i * (R * 128)) = c;
+      }
+    }
+    scale[b] = row_nan ? __uint_as_float(0x7fc00000u) : sc;
+  }
+  // LDS written by all is visible to all; W stays in flight (a __syncthreads would wait for it)
+  auto meet = [] __device__ () __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  meet();
+
+  // ---- products: every wavefront runs on its own ring, a column fragment at a time -----------------------------------------------------
+  i32x4 acc[RF][NF];
+#pragma unroll
+  for (int t = 0; t < RF; ++t)
+#pragma unroll
+    for (int j = 0; j < NF; ++j) acc[t][j] = i32x4{0, 0, 0, 0};
+  int frag[2];  // of the 64-byte halves of a block
+#pragma unroll
+  for (int h = 0; h < 2; ++h) frag[h] = lr * 128 + (((4 * h + lq) ^ ((lr >> 1) & 7)) * 16);
+  // k step k out of the slots at `slots`; LEFT: k steps behind it whose W has been requested; `from`: W of step k + DEPTH
+  auto step = [&](int k, unsigned int slots, auto left_c, const unsigned char* from) __attribute__((always_inline)) {
+    constexpr int LEFT = decltype(left_c)::value;
+    constexpr bool REQUEST = LEFT == DEPTH;
+    i32x4 xf[RF][2];
+#pragma unroll
+    for (int t = 0; t < RF; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) xf[t][h] = *reinterpret_cast<const i32x4*>(lds + k * (R * 128) + t * 2048 + frag[h]);
+#pragma unroll
+    for (int j = 0; j < NF; ++j) {
+      band_wait(REQUEST ? 2 * (NF * DEPTH - 1) : 2 * (NF * (LEFT + 1) - 1 - j));
+      i32x4 wf[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) wf[h] = *reinterpret_cast<const i32x4*>(ring + slots + j * SLOT + frag[h]);
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // the fragment is in registers: its slot is requested anew
+      __builtin_amdgcn_sched_barrier(0);
+      if (REQUEST) load_w(from, j, slots);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int t = 0; t < RF; ++t) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[h], xf[t][h], acc[t][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  unsigned int slots = 0;
+  const unsigned char* from = wbase + DEPTH * w_step;
+  int k = 0;
+  for (; k + DEPTH < steps; ++k) {
+    step(k, slots, std::integral_constant<int, DEPTH>{}, from);
+    from += w_step;
+    slots = DEPTH == 1 || slots == (DEPTH - 1) * NF * SLOT ? 0 : slots + NF * SLOT;
+  }
+  if (DEPTH == 2) {
+    step(k++, slots, std::integral_constant<int, DEPTH - 1>{}, from);
+    slots = slots == 0 ? NF * SLOT : 0;
+  }
+  step(k, slots, std::integral_constant<int, 0>{}, from);
+
+  // ---- row scales change hands in the rings, which nobody loads into any more; then (float(acc) * sx) * sw + bias ------------------------
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+    if (lr == 0) reinterpret_cast<float*>(ring)[4 * b + lq] = scale[b];
+  if (!a.bias)  // uniform
+#pragma unroll
+    for (int j = 0; j < NF; ++j) bias[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  meet();
+  const int64_t out_off = lr * a.ldy * 2;
+  unsigned char* out = reinterpret_cast<unsigned char*>(a.y + (int64_t)m0 * a.ldy + n0);
+#pragma unroll
+  for (int t = 0; t < RF; ++t) {
+    const int row = 16 * t + lr;
+    const float sx = *reinterpret_cast<const float*>(lds + CODES + row / RPW * RING + row % RPW * 4);
+    unsigned int o[NF][2];
+#pragma unroll
+    for (int j = 0; j < NF; ++j)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        float v[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          // three separately rounded fp32 operations (no fused multiply-add)
+          v[e] = (float)acc[t][j][2 * c + e] * sx;
+          v[e] = v[e] * sw[j][2 * c + e];
+          v[e] = v[e] + bias[j][2 * c + e];
+        }
+        o[j][c] = pack_bf16x2(v[0], v[1]);
+      }
+    unsigned char* to = out + (int64_t)(16 * t) * a.ldy * 2 + out_off;
+#pragma unroll
+    for (int j = 0; j + 1 < NF; j += 2) *reinterpret_cast<u32x4*>(to + 32 * j + 16 * lq) = u32x4{o[j][0], o[j][1], o[j + 1][0], o[j + 1][1]};
+    if (NF % 2 == 1) *reinterpret_cast<u32x2*>(to + 32 * (NF - 1) + 8 * lq) = u32x2{o[NF - 1][0], o[NF - 1][1]};
+  }
+}
+
+// Row fragments * 8 + column fragments of a wavefront in the tile; 0 = not this form.
+// The smallest tile whose tiles fit the CUs once; a second round costs more than the smaller tile gains (4096 x 768 -> 2304: 32 x 384 tiles, three
+// rounds, 21.7 us, 64 x 384, two, 21.5, 64 x 768 17.3), and beyond one round of the largest the two launches are ahead (6000 x 768 -> 2304 30 / 31,
+// 2700 x 1024 -> 4096 28.7 / 36).  On longer rows the quantiser's share grows with the rows a workgroup has: 64 x 384 tiles only from about 180 of
+// them on (us, two launches / one: 1024 x 1280 -> 3840, 160 tiles, 14.9 / 15.4, 1200 x 1280 -> 3840, 190, 17.3 / 15.7, 1024 x 1024 -> 4096, 176, 14.2 / 13.6), and
+// behind 1280 values the small-tile product's rows stay with it (300 x 1280 -> 1280 8.4 / 9.0, 400, beyond them, 11.9 / 9.2).
+static int band_shape(int64_t M, int N, int K) {
+  const int mode = knob_or(KNOB_LINEAR_BAND, 1);
+  if (mode <= 0 || knob_or(KNOB_LINEAR_SMALL, 1) <= 0 || K % 128 != 0 || K < 256 || K > 1280 || N % 8 != 0 || M < 32 || N < 384 || M > (1 << 20) || (int64_t)N * K >= (1ll << 31)) return 0;
+  auto tiles = [&](int rf, int nf) { return (M + 16 * rf - 1) / (16 * rf) * ((N + 128 * nf - 1) / (128 * nf)); };
+  auto fits = [&](int rf, int nf) { return M >= 16 * rf && N >= 128 * nf && tiles(rf, nf) <= 256; };
+  const int wide = K <= 1024 ? 6 : 5;
+  if (mode > 1) return (mode == 2 * 8 + 3 || mode == 4 * 8 + 3 || mode == 4 * 8 + wide) && M >= 16 * (mode / 8) && N >= 128 * (mode % 8) ? mode : 0;
+  if (K > 1024 && (M + 63) / 64 * ((N + 31) / 32) <= 256) return 0;
+  if (fits(2, 3)) return 2 * 8 + 3;
+  if (fits(4, 3)) return K <= 768 || tiles(4, 3) >= 176 ? 4 * 8 + 3 : 0;
+  return fits(4, wide) ? 4 * 8 + wide : 0;
+}
+
+bool linear_i8_band_covers(int64_t M, int N, int K) { return band_shape(M, N, K) != 0; }
+
+template <int KMAX, int RF, int NF, int DEPTH>
+static int launch_band(BandArgs a, hipStream_t stream) {
+  a.tiles_n = (a.N + 128 * NF - 1) / (128 * NF);
+  a.tiles_m = (a.M + 16 * RF - 1) / (16 * RF);
+  a.tiles = a.tiles_m * a.tiles_n;
+  // An XCD's eighth of the tiles is to be g row tiles by t / g column tiles with g * R rows of two bytes about as many bytes as the
+  // columns' weights: what its L2 fetches is least there
+  // (256 x 1280 -> 5120, whose 6.5 MB of weights every XCD would read otherwise, 12.8 -> 9.8 us).
+  const int t = (a.tiles + 7) / 8;
+  int g = 1;
+  while (g < a.tiles_m && (g + 1) * (g + 1) * 2 * 16 * RF <= t * 128 * NF) ++g;
+  a.group_m = g;
+  hipLaunchKernelGGL((linear_i8_band_kernel<KMAX, RF, NF, DEPTH>), dim3((unsigned int)((a.tiles + 7) / 8 * 8)), dim3(512), 0, stream, a);
+  return check_launch("linear_i8_band_kernel");
+}
+
+template <int KMAX>
+static int launch_band_shape(const BandArgs& a, int shape, hipStream_t stream) {
+  if (shape == 2 * 8 + 3) return launch_band<KMAX, 2, 3, 2>(a, stream);
+  if constexpr (KMAX <= 1024) {
+    if (shape == 4 * 8 + 3) return launch_band<KMAX, 4, 3, 2>(a, stream);
+    if (shape == 4 * 8 + 6) return launch_band<KMAX, 4, 6, 1>(a, stream);
+  } else {
+    if (shape == 4 * 8 + 3) return launch_band<KMAX, 4, 3, 1>(a, stream);
+    if (shape == 4 * 8 + 5) return launch_band<KMAX, 4, 5, 1>(a, stream);
+  }
+  set_error("linear_i8_band: %d x %d values to %d are not covered", a.M, a.K, a.N);
+  return SAMFAST_E_UNSUPPORTED;
+}
+
+int linear_i8_band_launch(const unsigned short* x, int64_t ldx, const int8_t* w, const float* sw, const float* bias, unsigned short* y,
+                          int64_t ldy, int M, int N, int K, int layout, hipStream_t stream) {
+  BandArgs a = {};
+  a.x = x; a.ldx = ldx; a.w = w; a.sw = sw; a.bias = bias; a.y = y; a.ldy = ldy; a.M = M; a.N = N; a.K = K;
+  const bool kb = layout == SAMFAST_LAYOUT_KB64;
+  a.w_pitch = kb ? 64 : (unsigned int)K;
+  a.w_kstep = kb ? (unsigned int)N * 64u : 64u;
+  const int shape = band_shape(M, N, K);
+  if (K <= 768) return launch_band_shape<768>(a, shape, stream);
+  if (K <= 1024) return launch_band_shape<1024>(a, shape, stream);
+  return launch_band_shape<1280>(a, shape, stream);
+}
+
+}  // namespace samfast

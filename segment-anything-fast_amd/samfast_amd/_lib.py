@@ -44,6 +44,7 @@ _SIGNATURES = {
     "samfast_layernorm": (_i32, [_ptr] * 4 + [_f32, _ptr, _ptr, _i64, _i32, _i32, _ptr]),
     "samfast_gelu": (_i32, [_ptr, _ptr, _i64, _i32, _ptr]),
     "samfast_linear_i8_workspace": (_i64, [_i64, _i32, _i32, _i32]),
+    "samfast_linear_i8_one_launch": (_i32, [_i64, _i32, _i32, _i32]),
     "samfast_gemm_i8_i32": (_i32, [_ptr, _ptr, _ptr, _i64, _i32, _i32, _ptr]),
     "samfast_gemm_i8_scale_bias": (
         _i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i32, _i32, _i32, _ptr]),

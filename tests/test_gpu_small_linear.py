@@ -238,9 +238,65 @@ def test_one_launch_agrees_with_two(sparse, M, N, K):
             lin.bias.copy_(b)
     lin, x = (Int8Sparse24Linear if sparse else Int8DynamicLinear).from_float(lin.cuda()), x.cuda()
     layout = 2 if sparse else _lib.LAYOUT_ROWMAJOR
-    assert _lib.load().samfast_linear_i8_workspace(M, N, K, layout) == 0
+    assert _lib.load().samfast_linear_i8_one_launch(M, N, K, layout) == 1
     one = lin(x)
     with _lib.knobs(SAMFAST_GEMM_LINEAR_SMALL=0):
-        assert _lib.load().samfast_linear_i8_workspace(M, N, K, layout) > 0
+        assert _lib.load().samfast_linear_i8_one_launch(M, N, K, layout) == 0
         two = lin(x)
     assert torch.equal(one.view(torch.int16), two.view(torch.int16))
+
+
+@pytest.mark.parametrize("M,N,K", [
+    # each tile at its smallest, with rows and columns moved back inside, the shortest, odd and longest K; then what the rule takes
+    (32, 384, 256), (33, 392, 384), (64, 768, 256), (65, 776, 640), (127, 1528, 768), (100, 1160, 896), (200, 2304, 1024), (95, 640, 1152), (129, 1288, 1280),
+    (4096, 768, 768), (2100, 2304, 768), (5300, 2304, 768), (1100, 4096, 1024), (700, 3080, 1024), (1990, 3840, 1280), (450, 1280, 1280),
+])
+def test_a_band_of_rows_in_one_launch_agrees_with_two(M, N, K):
+    """Every tile that the shape admits and the rule's choice, weights in both layouts; rows with a NaN, an infinity, zeros and ties."""
+    from samfast_amd import Int8DynamicLinear, _lib, ops
+    print(f"case band M={M} N={N} K={K}", flush=True)
+    lib = _lib.load()
+    x, w, b = linear_inputs(M, K, N, seed=M + N + K)
+    x[M // 2] = 0
+    x[M - 1, K // 3] = float("nan")
+    x[1, K - 1] = float("inf")
+    x[2] = torch.arange(K).remainder(255).sub(127).to(torch.bfloat16) / 2  # a maximum of 63.5: every second value a tie
+    lin = torch.nn.Linear(K, N, dtype=torch.bfloat16)
+    with torch.no_grad():
+        lin.weight.copy_(w)
+        lin.bias.copy_(b)
+    lin, x = Int8DynamicLinear.from_float(lin.cuda()), x.cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+    with _lib.knobs(SAMFAST_GEMM_LINEAR_SMALL=0):
+        two = lin(x)
+    assert torch.isnan(two[M - 1]).all()
+    wk = ops.to_kb64(lin.wq)
+    for tile in (1, 2 * 8 + 3, 4 * 8 + 3, 4 * 8 + (6 if K <= 1024 else 5)):
+        rows, cols = (16 * (tile // 8), 128 * (tile % 8)) if tile > 1 else (M, N)
+        if M < rows or N < cols:
+            continue
+        with _lib.knobs(SAMFAST_GEMM_LINEAR_BAND=tile):
+            if tile > 1:
+                assert lib.samfast_linear_i8_one_launch(M, N, K, 0) == 1
+            assert torch.equal(lin(x).view(torch.int16), two.view(torch.int16)), tile
+            if lib.samfast_linear_i8_one_launch(M, N, K, 1):
+                y = torch.empty_like(two)
+                assert lib.samfast_linear_i8(x.data_ptr(), K, wk.data_ptr(), lin.sw.data_ptr(), lin.bias_f32.data_ptr(), y.data_ptr(), N, None,
+                                             M, N, K, _lib.SAMFAST_BF16, _lib.LAYOUT_KB64, stream) == 0
+                assert torch.equal(y.view(torch.int16), two.view(torch.int16)), tile
+
+
+def test_a_linear_into_its_own_rows():
+    """y may be x where the caller brings the workspace: two launches, the quantiser has read every row before one is written."""
+    from samfast_amd import _lib
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    for M, K in ((64, 512), (4096, 768)):
+        lin = _linear(K, K, M)
+        x = torch.randn((M, K), device="cuda").to(torch.bfloat16)
+        want = lin(x)
+        need = lib.samfast_linear_i8_workspace(M, K, K, 0)
+        assert need > 0 and lib.samfast_linear_i8_one_launch(M, K, K, 0) == 1
+        work = torch.empty(need, dtype=torch.int8, device="cuda")
+        assert lib.samfast_linear_i8(x.data_ptr(), K, lin.wq.data_ptr(), lin.sw.data_ptr(), lin.bias_f32.data_ptr(), x.data_ptr(), K,
+                                     work.data_ptr(), M, K, K, _lib.SAMFAST_BF16, 0, stream) == 0
+        assert torch.equal(x, want)
