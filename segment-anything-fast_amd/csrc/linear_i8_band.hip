@@ -117,10 +117,7 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
     lds_dma16(wbase + d * w_step, w_off[j][h], ring_at + d * NF * SLOT + j * SLOT + h * 1024);
   };
 
-  // ---- codes: 128 bytes of every row to a block, chunks at the same positions as W's.  The code wanted is rint(fl(v / scale)) (quant_row.hpp).
-  // q = fl(v * inv), then fl(q + fl(v - q * scale) * inv) with fused multiply-adds is that quotient to its last bit wherever it is
-  // not tiny, without the branch, whose other side, met once per chunk in code that runs once, costs more than the arithmetic here (64
-  // rows of 768 13700 cycles with it, 6000 without).  All pairs of a bf16 row maximum and a bf16 value give the same code both ways. --------
+  // ---- codes: 128 bytes of every row to a block, chunks at the same positions as W's. -------------------------------------------------
   float scale[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
@@ -152,17 +149,7 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
         for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(f[i][e]));
       amax = row_max(m);
     }
-    const float sc = fmaxf(amax, 1e-5f) / 127.0f;
-    float div = sc;
-    if (__any(__float_as_uint(amax) >= 0x7f800000u)) {  // an infinity in the row: every quotient is 0 or NaN, every code 0
-      const bool inf = __float_as_uint(amax) >= 0x7f800000u;
-      div = inf ? 1.0f : sc;
-#pragma unroll
-      for (int i = 0; i < NCH; ++i)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) f[i][e] = inf ? 0.f : f[i][e];
-    }
-    const float inv = 1.0f / div;
+    const QuantScale q(amax);
     const int row = wave * RPW + 4 * b + lq;
     unsigned char* at = lds + row * 128 + (((lr >> 1) ^ ((row >> 1) & 7)) * 16) + (lr & 1) * 8;
 #pragma unroll
@@ -171,20 +158,12 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
 #pragma unroll
       for (int w = FIRST * (b * NCH + i) / CHUNKS; w < FIRST * (b * NCH + i + 1) / CHUNKS; ++w) first_w(w);
       if (i < steps) {  // uniform
-        unsigned int m[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float q = f[i][e] * inv;
-          m[e] = __float_as_uint(fmaf(fmaf(-q, div, f[i][e]), inv, q) + 12582912.0f);  // 1.5 * 2^23: the code in the low byte
-        }
-        u32x2 c;
-#pragma unroll
-        for (int g = 0; g < 2; ++g)
-          c[g] = __builtin_amdgcn_perm(m[4 * g + 1], m[4 * g], 0x0c0c0400u) | __builtin_amdgcn_perm(m[4 * g + 3], m[4 * g + 2], 0x04000c0cu);
-        *reinterpret_cast<u32x2*>(at + i * (R * 128)) = c;
+        unsigned int c[2];
+        quantize_chunk<8>(f[i], q, c);
+        *reinterpret_cast<u32x2*>(at + i * (R * 128)) = u32x2{c[0], c[1]};
       }
     }
-    scale[b] = row_nan ? __uint_as_float(0x7fc00000u) : sc;
+    scale[b] = row_nan ? __uint_as_float(0x7fc00000u) : q.scale;
   }
   // LDS written by all is visible to all; W stays in flight (a __syncthreads would wait for it)
   auto meet = [] __device__ () __attribute__((always_inline)) {

@@ -1,9 +1,9 @@
 // Per-row symmetric int8 quantiser (bf16 -> int8 + fp32 scale), optionally preceded
-// by LayerNorm over the row and a row gather (window partition).  HBM-bound: 65536 rows of 5120 through GELU 209 us, of 1280
-// plain 38, with LayerNorm 48 (4.8, 6.6 and 5.2 TB/s; a copy reaches 4.9 from HBM), and the vector ALU close behind: 254 vector
-// instructions per row of 1280 plain, 448 with LayerNorm, 1764 per row of 5120 with GELU, by the hardware counters (297, 515 and 1949 with
-// a product, its distance from the integer and a comparison per value, and every chunk's address made per lane: 20480 x 4096 with
-// GELU 57.3 -> 53.3 us, 4096 x 5120 17.6 -> 16.7).
+// by LayerNorm over the row and a row gather (window partition).  HBM-bound: 65536 rows of 5120 through GELU 216 us, of 1280
+// plain 46, with LayerNorm 63, codes written into new memory each time (4.7, 5.5 and 4.0 TB/s; a copy reaches 4.9 from HBM), and with LayerNorm the
+// vector ALU close behind: 188 vector instructions per row of 1280 plain, 382 with LayerNorm, 1593 per row of 5120 with GELU, by the hardware counters.  us with a
+// branch per chunk / without (quant_row.hpp): 4096 x 1024 4.7 / 3.5, with LayerNorm 5.8 / 4.6, 4096 x 4096 11.4 / 9.8, with GELU 15.9 / 14.4, 20480 x 1024 with
+// LayerNorm 19.1 / 15.4, 65536 x 5120 with GELU 228 / 216, 65536 x 1280 with LayerNorm 61.7 / 63.2.
 //
 // One wavefront owns one output row: the source row is read once with 16- or 8-byte loads
 // and unpacked to fp32 registers, (normalised,) reduced to its absmax across the 64 lanes
@@ -11,9 +11,7 @@
 // half-to-even and written back as 8- or 4-byte packs of int8.
 // Algorithmic traffic: 2 bytes read + 1 byte written per element + 4 bytes of scale.
 //
-// q = rint(x / s) must equal the IEEE division bit for bit.  Most elements take a
-// cheap route: rint of a product a little below the quotient and of one a little above it; only where those differ
-// is the element's chunk redone with the true division (quant_row.hpp).
+// q = rint(x / s) must equal the IEEE division bit for bit (quant_row.hpp).
 // |x| <= absmax makes |x / s| <= 127 by construction, so no clamp is needed.
 #include "quant_row.hpp"
 
