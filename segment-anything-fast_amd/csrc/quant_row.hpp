@@ -187,10 +187,34 @@ struct RowQuantizer {
     if (lane == 0) a.sx[row] = 1e-5f / 127.0f;
   }
 
+  // gamma and beta (LN) as they were loaded, unpacked where they are used, or unpacked once for many rows
+  struct PackedAffine {
+    const in_t (&g)[NCH];
+    const in_t (&b)[NCH];
+    SF_DEVICE float gamma(int i, int e) const { return e % 2 ? bf16_hi_to_f32(g[i][e / 2]) : bf16_lo_to_f32(g[i][e / 2]); }
+    SF_DEVICE float beta(int i, int e) const { return e % 2 ? bf16_hi_to_f32(b[i][e / 2]) : bf16_lo_to_f32(b[i][e / 2]); }
+  };
+  struct PlainAffine {
+    float g[NCH][EPC], b[NCH][EPC];
+    SF_DEVICE PlainAffine(const in_t (&gw)[NCH], const in_t (&bw)[NCH]) {
+      const PackedAffine p = {gw, bw};
+#pragma unroll
+      for (int i = 0; i < NCH; ++i)
+#pragma unroll
+        for (int e = 0; e < EPC; ++e) g[i][e] = p.gamma(i, e), b[i][e] = p.beta(i, e);
+    }
+    SF_DEVICE float gamma(int i, int e) const { return g[i][e]; }
+    SF_DEVICE float beta(int i, int e) const { return b[i][e]; }
+  };
+
   // Everything after the loads: (LayerNorm,) absmax, scale, codes of output row `row`.
   static SF_DEVICE void finish_row(const QuantArgs& a, int64_t row, int nchunk, int lane,
                                    const in_t (&xw)[NCH], const in_t (&gw)[NCH], const in_t (&bw)[NCH]) {
-    const float scale = finish(a, nchunk, lane, xw, gw, bw, [&](int i, const unsigned int (&codes)[EPC / 4]) { store_chunk(a, row, i, lane, codes); });
+    finish_row(a, row, nchunk, lane, xw, PackedAffine{gw, bw});
+  }
+  template <typename Affine>
+  static SF_DEVICE void finish_row(const QuantArgs& a, int64_t row, int nchunk, int lane, const in_t (&xw)[NCH], const Affine& affine) {
+    const float scale = finish(a, nchunk, lane, xw, affine, [&](int i, const unsigned int (&codes)[EPC / 4]) { store_chunk(a, row, i, lane, codes); });
     if (lane == 0) a.sx[row] = scale;
   }
 
@@ -198,6 +222,10 @@ struct RowQuantizer {
   template <typename Store>
   static SF_DEVICE float finish(const QuantArgs& a, int nchunk, int lane, const in_t (&xw)[NCH], const in_t (&gw)[NCH], const in_t (&bw)[NCH],
                                 Store store) {
+    return finish(a, nchunk, lane, xw, PackedAffine{gw, bw}, store);
+  }
+  template <typename Affine, typename Store>
+  static SF_DEVICE float finish(const QuantArgs& a, int nchunk, int lane, const in_t (&xw)[NCH], const Affine& affine, Store store) {
     // the row as floats, unpacked once
     float f[NCH][EPC];
 #pragma unroll
@@ -236,12 +264,11 @@ struct RowQuantizer {
       for (int i = 0; i < NCH; ++i) {
         const int c = lane + i * 64;
         if (c < nchunk) {
-          const in_t g = gw[i], b = bw[i];
 #pragma unroll
           for (int j = 0; j < W; ++j) {
             // (x - mean) * rstd, then one fused multiply-add with gamma and beta
-            const float y0 = fmaf(f[i][2 * j] * rstd, bf16_lo_to_f32(g[j]), bf16_lo_to_f32(b[j]));
-            const float y1 = fmaf(f[i][2 * j + 1] * rstd, bf16_hi_to_f32(g[j]), bf16_hi_to_f32(b[j]));
+            const float y0 = fmaf(f[i][2 * j] * rstd, affine.gamma(i, 2 * j), affine.beta(i, 2 * j));
+            const float y1 = fmaf(f[i][2 * j + 1] * rstd, affine.gamma(i, 2 * j + 1), affine.beta(i, 2 * j + 1));
             const unsigned int y = pack_bf16x2(y0, y1);  // the bf16 values a separate LayerNorm would have stored
             f[i][2 * j] = bf16_lo_to_f32(y);
             f[i][2 * j + 1] = bf16_hi_to_f32(y);

@@ -1,7 +1,7 @@
 // Per-row symmetric int8 quantiser (bf16 -> int8 + fp32 scale), optionally preceded
 // by LayerNorm over the row and a row gather (window partition).  HBM-bound: 65536 rows of 5120 through GELU 216 us, of 1280
-// plain 46, with LayerNorm 63, codes written into new memory each time (4.7, 5.5 and 4.0 TB/s; a copy reaches 4.9 from HBM), and with LayerNorm the
-// vector ALU close behind: 188 vector instructions per row of 1280 plain, 382 with LayerNorm, 1593 per row of 5120 with GELU, by the hardware counters.  us with a
+// plain 46, with LayerNorm 54, codes written into new memory each time (4.7, 5.5 and 4.6 TB/s; a copy reaches 4.9 from HBM), and with LayerNorm the
+// vector ALU close behind: 188 vector instructions per row of 1280 plain, 382 with LayerNorm, 1593 per row of 5120 with GELU, by the hardware counters, for a wavefront per row.  us with a
 // branch per chunk / without (quant_row.hpp): 4096 x 1024 4.7 / 3.5, with LayerNorm 5.8 / 4.6, 4096 x 4096 11.4 / 9.8, with GELU 15.9 / 14.4, 20480 x 1024 with
 // LayerNorm 19.1 / 15.4, 65536 x 5120 with GELU 228 / 216, 65536 x 1280 with LayerNorm 61.7 / 63.2.
 //
@@ -58,6 +58,30 @@ __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowwise_bf16_k
   if (LN) RQ::load_affine(a.gamma, a.beta, nchunk, lane, gw, bw);
   if (ACT) gelu_chunks(xw);
   RQ::finish_row(a, row, nchunk, lane, xw, gw, bw);
+}
+
+// Many rows with LayerNorm: the wavefronts stay and walk the rows, gamma and beta unpacked once, the next row's loads under the
+// present one's arithmetic: five workgroups per CU, what 84 registers a lane admit.  Bound: memory and the vector ALU level.  us, a wavefront per row / so
+// (8 workgroups per CU): 65536 x 1280 62.7 / 54.2 (55.4), 131072 x 1280 128 / 118 (115), 32768 x 1280 32.9 / 29.2, 16384 x 1280 15.7 / 15.3, 65536 x 768 37.1 / 34.8, 65536 x 1024
+// 43.3 / 42.2, 20480 x 1024 15.6 / 15.6; fewer values than that are no faster (16384 x 768 11.8 / 12.1, 8192 x 1024 7.9 / 8.0).
+template <int NCH, int EPC>
+__global__ __launch_bounds__(64 * kQuantWavesPerBlock) void layernorm_quant_rows_kernel(QuantArgs a) {
+  using RQ = RowQuantizer<NCH, EPC, true>;
+  const int lane = threadIdx.x & 63;
+  constexpr int NCHUNK = 64 * NCH;
+  const int64_t step = (int64_t)gridDim.x * kQuantWavesPerBlock;
+  int64_t row = (int64_t)blockIdx.x * kQuantWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  typename RQ::in_t xw[NCH], next[NCH], gw[NCH], bw[NCH];
+  const int64_t last = a.M - 1;
+  RQ::template load_row<false>(a.x + min(row, last) * a.ldx, NCHUNK, lane, xw);
+  RQ::load_affine(a.gamma, a.beta, NCHUNK, lane, gw, bw);
+  const typename RQ::PlainAffine affine(gw, bw);
+  for (; row < a.M; row += step) {
+    RQ::template load_row<false>(a.x + min(row + step, last) * a.ldx, NCHUNK, lane, next);
+    RQ::finish_row(a, row, NCHUNK, lane, xw, affine);
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) xw[i] = next[i];
+  }
 }
 
 // WPR wavefronts share a row: fewer registers per lane for long rows (one wavefront with 4096 values needs 238: two
@@ -134,6 +158,12 @@ static int launch_quant(const QuantArgs& a, hipStream_t stream) {
   const dim3 grid((unsigned int)((a.M + kQuantWavesPerBlock - 1) / kQuantWavesPerBlock)), block(64 * kQuantWavesPerBlock);
   // (the widths of the encoders' rows: built for those)
   constexpr bool MAY_FIT = EPC == 4 || NCH == 2 || NCH == 10;
+  if constexpr (LN && (EPC == 4 || NCH == 2)) {
+    if (a.K == 64 * EPC * NCH && !a.src_row && a.M * a.K >= (20ll << 20)) {
+      hipLaunchKernelGGL((layernorm_quant_rows_kernel<NCH, EPC>), dim3(min(grid.x, 256u * 5u)), block, 0, stream, a);
+      return check_launch("layernorm_quant_rows_kernel");
+    }
+  }
   if (MAY_FIT && a.K == 64 * EPC * NCH) hipLaunchKernelGGL((quant_rowwise_bf16_kernel<NCH, EPC, LN, ACT, MAY_FIT>), grid, block, 0, stream, a);
   else hipLaunchKernelGGL((quant_rowwise_bf16_kernel<NCH, EPC, LN, ACT, false>), grid, block, 0, stream, a);
   return check_launch("quant_rowwise_bf16_kernel");

@@ -858,3 +858,23 @@ def test_matrix_loops_of_either_shape_count_their_operations():
     assert not out.any()  # the kernels write nothing
     for bad in (-1, 4):
         assert lib.samfast_bench_mfma_ceiling(bad, buf.data_ptr(), 8, 10, None, out.data_ptr(), stream) == -1
+
+
+@pytest.mark.parametrize("M,K", [(16384, 1280), (16389, 1280), (27310, 768), (20481, 1024)])
+def test_layernorm_quant_of_many_rows_agrees_with_few(M, K):
+    """Wavefronts that walk the rows (from 20 M values on) against the wavefront per row of shorter calls, bit for bit: a strided
+    input, a NaN row, a constant row."""
+    from samfast_amd import _lib, ops
+    print(f"case layernorm rows M={M} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn((M, K + 8), generator=g, device="cuda").to(torch.bfloat16)[:, :K]
+    x[M - 1, 3] = float("nan")
+    x[M // 2] = 0.5
+    gamma, beta = (torch.randn(K, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    for layout in (_lib.LAYOUT_ROWMAJOR, _lib.LAYOUT_KB64):
+        q, s = ops.layernorm_quant(x, gamma, beta, 1e-6, layout=layout)
+        q = ops.from_kb64(q) if layout == _lib.LAYOUT_KB64 else q
+        few = [ops.layernorm_quant(x[i:i + 4000], gamma, beta, 1e-6) for i in range(0, M, 4000)]
+        assert torch.equal(q, torch.cat([f[0] for f in few]))
+        assert torch.equal(s.view(torch.int32), torch.cat([f[1] for f in few]).view(torch.int32))
+        assert torch.isnan(s[M - 1])
