@@ -409,17 +409,17 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void attn_global_ke
 // window kernel: gh <= 15, gw <= 16, N = gh*gw <= 208; one workgroup per (window, head), or two
 // or three for those that are left over beside whole rounds of 256
 // =============================================================================
-// Eight wavefronts: all of them stage K / V, wavefront w then owns query tile w (32 queries;
-// 7 tiles for 196 tokens).  Registers are kept under 128 per lane (online softmax over the
+// Eight wavefronts (small windows: as many as query tiles): all of them stage K / V, wavefront w then owns
+// query tile w (32 queries; 7 tiles for 196 tokens).  Registers are kept under 128 per lane (online softmax over the
 // key tiles instead of holding all scores) so that two workgroups = four wavefronts per SIMD
 // are resident and fill each other's pipeline gaps.
-template <int HD>
+template <int HD, int TILES>
 struct WindowCfg {
   static constexpr int KS = HD / 16;
   static constexpr int DT = (HD + 31) / 32;
-  static constexpr int NMAX = 208;
-  static constexpr int NT = 7;                 // key tiles of 32
-  static constexpr int WAVES = 8;
+  static constexpr int NT = TILES;             // key tiles of 32
+  static constexpr int NMAX = NT == 7 ? 208 : 32 * NT;
+  static constexpr int WAVES = NT == 7 ? 8 : NT;
   static constexpr int THREADS = 64 * WAVES;
   // K and V rows travel global memory -> LDS directly, row-major, in 16-byte pieces; a staged
   // row is HD/8 data pieces and one spare piece that no load writes (rows HD + 8 elements apart)
@@ -445,9 +445,9 @@ struct WindowCfg {
   static_assert(NT <= WAVES, "one query tile per wavefront");
 };
 
-template <typename T, int HD, bool FUSED>
-__global__ __launch_bounds__(WindowCfg<HD>::THREADS, 2) void attn_window_kernel(AttnArgs a) {
-  using C = WindowCfg<HD>;
+template <typename T, int HD, bool FUSED, int TILES>
+__global__ __launch_bounds__((WindowCfg<HD, TILES>::THREADS), 2) void attn_window_kernel(AttnArgs a) {
+  using C = WindowCfg<HD, TILES>;
   __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS_BYTES];
   unsigned char* kl = lds;
   unsigned char* vl = lds + C::KBYTES;
@@ -884,19 +884,45 @@ static int launch_hd(const AttnArgs& a, bool global_path, hipStream_t stream) {
   const int64_t wins = a.ws > 0 ? (int64_t)a.B * a.wins_x * a.wins_y : a.B;
   const int64_t total = wins * a.nH;
   AttnArgs b = a;
+  const int ntq = (a.N + 31) / 32;
+  // Windows of up to four query tiles whose factors the caller brings (grids of other sizes than the encoder's 14 x 14): workgroups of as many wavefronts as
+  // tiles and LDS for as many keys, so that four to sixteen of them share a CU where two of eight mostly idle wavefronts did.  The tiles and their
+  // order are the same, and so are the bits.  us, eight wavefronts / so, 400 x 12 x 64: 5 x 5 40.2 / 15.9, 8 x 8 49.4 / 31.6, 6 x 11 57 / 37.7, 10 x 10 67.9 / 53.8, 9 x
+  // 13 79.7 / 65.1, of 80 channels 42.7 / 18.9, 55.1 / 42.1, 61 / 46, 73.9 / 71.6, 87.1 / 80.2 (floors at a copy's rate 13, 34, 35, 54, 64; 16, 42, 44, 67, 78).  Up to two
+  // workgroups a CU four wavefronts stage faster (25 x 12 x 64, 8 x 8: 7.9 / 7.6, with four 7.2), up to half a one eight, cut up as below (4 x 12 x 80,
+  // 8 x 8: 6.4 / 6.9, 6.6).  Five and six are slower: 12 x 12 97 / 117.
+  if constexpr (!FUSED) {
+    if (ntq <= 4 && total > 128) {
+      b.whole = (int)(total & ~(int64_t)7);
+      b.part_tiles = ntq;
+      b.parts = 1;
+      const dim3 grid((unsigned int)((total + 7) / 8 * 8));
+      auto launch = [&](auto tiles) {
+        constexpr int TILES = decltype(tiles)::value;
+        hipLaunchKernelGGL((attn_window_kernel<T, HD, FUSED, TILES>), grid, dim3(WindowCfg<HD, TILES>::THREADS), 0, stream, b);
+        return check_launch("attn_window_kernel");
+      };
+      switch (total <= 512 ? 4 : ntq) {
+        case 1: return launch(std::integral_constant<int, 1>{});
+        case 2: return launch(std::integral_constant<int, 2>{});
+        case 3: return launch(std::integral_constant<int, 3>{});
+        default: return launch(std::integral_constant<int, 4>{});
+      }
+    }
+  }
   // Whole rounds of 256 items get a workgroup each; what is left over is cut into halves or thirds, by query tiles, while that makes at most
   // a workgroup more per CU: otherwise a few CUs run two workgroups side by side and the others wait for them (the
   // staging is done again, by CUs that would idle).  us, before / whole / halves / thirds, windows of 14 x 14: 25 x 12 x 64 15.9 / 15.9 / 13.4 /
   // 13.3, in an image 18.1 / 15.2 / 15.0 / 14.6, 5 x 12 x 64 9.4 / 9.4 / 8.0 / 7.9, 30 x 12 x 64 (104 left) 16.2 / 15.8 / 13.8 / 17.7, 2 images x 12 x
   // 64 (88 left) 24.6 / 24.0 / 22.5 / 24.5, 2 images x 16 x 80 (32 left) 32.6 / 29.8 / 29.4 / 29.5; 25 x 16 x 80 (144 left) 19.0 / 18.7 / 21.5 / 20.8.
   // (Before: contiguous eighths of all items, padding tiles computed as well.)
-  const int ntq = (a.N + 31) / 32, left = (int)(total % 256);
+  const int left = (int)(total % 256);
   const int parts = left * 3 <= 256 ? 3 : left * 2 <= 256 ? 2 : 1;
   b.whole = (int)(total - left);
   b.part_tiles = (ntq + parts - 1) / parts;
   b.parts = (ntq + b.part_tiles - 1) / b.part_tiles;
   const unsigned int grid = (unsigned int)((b.whole + ((total - b.whole) * b.parts + 7) / 8 * 8));
-  hipLaunchKernelGGL((attn_window_kernel<T, HD, FUSED>), dim3(grid), dim3(WindowCfg<HD>::THREADS), 0, stream, b);
+  hipLaunchKernelGGL((attn_window_kernel<T, HD, FUSED, 7>), dim3(grid), dim3(WindowCfg<HD, 7>::THREADS), 0, stream, b);
   return check_launch("attn_window_kernel");
 }
 

@@ -232,3 +232,27 @@ def test_window_factors_read_in_pairs_or_one_by_one(gh, gw, hd, dtype):
     # probabilities and result in the half type, as the operator's other tests
     eps = torch.finfo(dtype).eps
     assert (y.cpu().double() - ref).abs().max() <= 4 * eps * v.abs().max().item()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hd", [64, 80])
+@pytest.mark.parametrize("gh,gw", [(1, 1), (5, 5), (2, 16), (3, 11), (8, 8), (5, 13), (6, 16), (7, 14), (9, 13), (8, 16), (10, 13)])
+def test_small_windows_same_bits_in_any_batch(gh, gw, hd, dtype):
+    """Workgroups sized to the window (many windows), of four wavefronts (some) and of eight (few) at the edges of 32-token tiles,
+    strided operands; the few against the oracle."""
+    from samfast_amd import ops
+    print(f"case small windows {gh}x{gw} hd={hd} {dtype}", flush=True)
+    nH, N = 4, gh * gw
+    g = torch.Generator(device="cuda").manual_seed(N + hd)
+    qkv = (torch.randn((140, N, 3, nH, hd), generator=g, device="cuda") * 0.5).to(dtype)
+    q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
+    rel_h, rel_w = ((torch.randn((140, nH, N, n), generator=g, device="cuda") * 0.5).to(dtype) for n in (gh, gw))
+    rel_h[1, :, :, 0] = float("-inf") if gh > 1 else 0
+    run = lambda b: ops.attn_relpos_bias(q[b], k[b], v[b], rel_h[b], rel_w[b])
+    many, some, few = run(slice(0, 140)), run(slice(0, 60)), run(slice(0, 3))  # 560, 240 and 12 items
+    assert torch.equal(many[:60], some) and torch.equal(some[:3], few)
+    last = run(slice(130, 140))
+    assert torch.equal(many[130:], last)
+    ref = ora.attention_rel_h_rel_w(*(t[:3].cpu() for t in (q, k, v)), rel_h[:3, ..., None].cpu(), rel_w[:3, :, :, None].cpu(), compute_dtype=torch.float32)
+    diff = (few.float().cpu() - ref.float()).abs()
+    assert diff.max().item() <= 2e-2 and diff.mean().item() <= 1e-3
