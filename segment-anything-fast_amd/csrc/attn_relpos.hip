@@ -460,7 +460,7 @@ __global__ __launch_bounds__((WindowCfg<HD, TILES>::THREADS), 2) void attn_windo
   // the indicator table (read only after the barrier that follows the arrival of K)
   if (tid < 2 * C::HOT_ENTRIES) *reinterpret_cast<u32x4*>(hot + tid * 16) = onehot_x8<T>(tid >> 1, tid & 1);
   // all heads of a window run on one XCD: their 2*HD-byte slices of a token share cache lines
-  const unsigned int total = (unsigned int)((a.ws > 0 ? a.B * a.wins_x * a.wins_y : a.B) * a.nH);
+  const unsigned int total = (unsigned int)((FUSED && a.ws > 0 ? a.B * a.wins_x * a.wins_y : a.B) * a.nH);
   // every XCD has a contiguous range of the items with one workgroup (a.whole, a multiple of 8) and one of the others' parts
   const unsigned int xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
   const unsigned int whole_x = (unsigned int)a.whole >> 3;
@@ -478,7 +478,8 @@ __global__ __launch_bounds__((WindowCfg<HD, TILES>::THREADS), 2) void attn_windo
   const int bwin = bh / a.nH, h = bh % a.nH;
   // image-ordered mode: bwin = (image, window row, window column)
   int b = bwin, win_y0 = 0, win_x0 = 0;
-  if (a.ws > 0) {
+  const bool in_image = FUSED && a.ws > 0;  // the other form is launched on windows alone: no geometry in it
+  if (in_image) {
     const int per_img = a.wins_x * a.wins_y;
     b = bwin / per_img;
     const int wi = bwin - b * per_img;
@@ -492,7 +493,7 @@ __global__ __launch_bounds__((WindowCfg<HD, TILES>::THREADS), 2) void attn_windo
   auto div_gw = [&](int n) { return (int)(__umul24((unsigned int)n, (unsigned int)gw_magic) >> 16); };
   auto times_gw = [&](int r) { return (int)__umul24((unsigned int)r, (unsigned int)a.gw); };
   auto tok_of = [&](int n) {
-    if (a.ws <= 0) return n;
+    if (!in_image) return n;
     const int ny = div_gw(n);
     const int y = win_y0 + ny, x = win_x0 + n - times_gw(ny);
     return (y < a.img_h && x < a.img_w) ? y * a.img_w + x : -1;
@@ -501,14 +502,14 @@ __global__ __launch_bounds__((WindowCfg<HD, TILES>::THREADS), 2) void attn_windo
   const unsigned short* kbase = a.k + b * a.k_sb + h * a.k_sh;
   const unsigned short* vbase = a.v + b * a.v_sb + h * a.v_sh;
   const unsigned short* qbase = a.q + b * a.q_sb + h * a.q_sh;
-  const unsigned short* kpad = a.ws > 0 ? a.pad_k + h * HD : kbase;
-  const unsigned short* vpad = a.ws > 0 ? a.pad_v + h * HD : vbase;
+  const unsigned short* kpad = in_image ? a.pad_k + h * HD : kbase;
+  const unsigned short* vpad = in_image ? a.pad_v + h * HD : vbase;
 
   const int ntq = (N + 31) / 32;
   const int nsteps = (N + 15) / 16;
   // uniform per wavefront; tiles of padding tokens alone (a window over the image's lower edge) are left out
   const int tile = tile0 + wave;
-  const bool has_tile = wave < tiles && tile < ntq && (a.ws <= 0 || win_y0 + div_gw(32 * tile) < a.img_h);
+  const bool has_tile = wave < tiles && tile < ntq && (!in_image || win_y0 + div_gw(32 * tile) < a.img_h);
   const int qi = 32 * tile + lr;
   const int qc = min(qi, N - 1);
 
