@@ -5,11 +5,13 @@
 // memory between them, and the host pays for both.  Here every workgroup quantises its 32 or 64 rows itself - once per range of columns,
 // 2 to 14 times in all, which is why ranges are wide, at 64 rows 640 or 768 columns, and why sixteen lanes take a row (one reduction and
 // one division serve four rows) - keeps the codes in LDS for the whole of K and runs on W alone: a ring per wavefront in LDS, a
-// 16-column x 128-byte fragment at a time, whole lines of row-major weights as well as of K-block-major ones; one barrier before the
-// products, one behind them.  Bound (4096 x 768 -> 3072, cycles of a workgroup's 28800): rows and first W through the load path
-// 4000, codes 6000 of vector work, products 11400 (9200 of matrix pipe), scales and output 7300; little of it overlaps, 160 KB of LDS being one workgroup per CU.
-// us on the GPU, two launches / this one: 4096 x 768 -> 3072 22.9 / 18.9, 4096 x 768 -> 768 13 / 8.7, 2048 x 768 -> 3072 16 / 13.1, 16384 x 768 -> 768 34 / 20, 1024 x 1024 -> 3072
-// 13 / 9.7, 512 x 1280 -> 1280 12.1 / 9.2.  Integer sums and the epilogue's arithmetic are those of the other forms: the same bits.
+// 16-column x 128-byte fragment at a time, whole lines of row-major weights as well as of K-block-major ones.  Wavefronts meet in front of the
+// products and never again: the row scales are in registers by then, so that one that is through converts and stores under the others'
+// products (with the scales fetched behind a barrier at the end 28900 cycles instead of 26500).  Bound (4096 x 768 -> 3072, cycles of a workgroup's
+// 26500): rows and first W through the load path 4000, codes 6000 of vector work, products 12700 (9200 of matrix pipe), output 3700; little of it
+// overlaps, 160 KB of LDS being one workgroup per CU.
+// us on the GPU, two launches / this one: 4096 x 768 -> 3072 21.9 / 18.3, 4096 x 768 -> 768 12.2 / 8.7, 2048 x 768 -> 3072 15.6 / 12.2, 16384 x 768 -> 768 26.9 / 19.5, 1024 x 1024
+// -> 3072 12.8 / 9.3, 512 x 1280 -> 5120 12.3 / 9.9.  Integer sums and the epilogue's arithmetic are those of the other forms: the same bits.
 #include "attn_relpos_shared.hpp"
 #include "gemm_i8_shared.hpp"
 #include "linear_i8_small.hpp"
@@ -55,7 +57,8 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
   constexpr int CODES = R * KMAX;
   static_assert(CODES + 8 * RING <= 160 * 1024, "LDS of a CU");
   static_assert(2 * (NF * DEPTH - 1) <= 15, "wait thresholds");
-  __shared__ __attribute__((aligned(16))) unsigned char lds[CODES + 8 * RING];
+  constexpr bool ROOM = CODES + 8 * RING + R * 4 <= 160 * 1024;  // for the row scales beside codes and rings
+  __shared__ __attribute__((aligned(16))) unsigned char lds[CODES + 8 * RING + (ROOM ? R * 4 : 0)];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -118,7 +121,10 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
   };
 
   // ---- codes: 128 bytes of every row to a block, chunks at the same positions as W's. -------------------------------------------------
-  float scale[NB];
+  // Row scales: beside the rings, or, where LDS is full, in the place of each ring's last KB, whose request then waits for them to be read
+  auto scale_of = [&](int row) __attribute__((always_inline)) {
+    return reinterpret_cast<float*>(ROOM ? lds + CODES + 8 * RING + row * 4 : lds + CODES + row / RPW * RING + RING - 1024 + row % RPW * 4);
+  };
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
     float f[NCH][8];
@@ -156,14 +162,15 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
     for (int i = 0; i < NCH; ++i) {
       constexpr int FIRST = 2 * NF * DEPTH, CHUNKS = NB * NCH;
 #pragma unroll
-      for (int w = FIRST * (b * NCH + i) / CHUNKS; w < FIRST * (b * NCH + i + 1) / CHUNKS; ++w) first_w(w);
+      for (int w = FIRST * (b * NCH + i) / CHUNKS; w < FIRST * (b * NCH + i + 1) / CHUNKS; ++w)
+        if (ROOM || w < FIRST - 1) first_w(w);
       if (i < steps) {  // uniform
         unsigned int c[2];
         quantize_chunk<8>(f[i], q, c);
         *reinterpret_cast<u32x2*>(at + i * (R * 128)) = u32x2{c[0], c[1]};
       }
     }
-    scale[b] = row_nan ? __uint_as_float(0x7fc00000u) : q.scale;
+    if (lr == 0) *scale_of(row) = row_nan ? __uint_as_float(0x7fc00000u) : q.scale;
   }
   // LDS written by all is visible to all; W stays in flight (a __syncthreads would wait for it)
   auto meet = [] __device__ () __attribute__((always_inline)) {
@@ -173,6 +180,13 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
     __builtin_amdgcn_sched_barrier(0);
   };
   meet();
+  float sx[RF];
+#pragma unroll
+  for (int t = 0; t < RF; ++t) sx[t] = *scale_of(16 * t + lr);
+  if constexpr (!ROOM) {
+    meet();
+    first_w(2 * NF * DEPTH - 1);
+  }
 
   // ---- products: every wavefront runs on its own ring, a column fragment at a time -----------------------------------------------------
   i32x4 acc[RF][NF];
@@ -223,20 +237,14 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
   }
   step(k, slots, std::integral_constant<int, 0>{}, from);
 
-  // ---- row scales change hands in the rings, which nobody loads into any more; then (float(acc) * sx) * sw + bias ------------------------
-#pragma unroll
-  for (int b = 0; b < NB; ++b)
-    if (lr == 0) reinterpret_cast<float*>(ring)[4 * b + lq] = scale[b];
+  // ---- (float(acc) * sx) * sw + bias; a wavefront that is through finishes under the others' products ------------------------------------
   if (!a.bias)  // uniform
 #pragma unroll
     for (int j = 0; j < NF; ++j) bias[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  meet();
   const int64_t out_off = lr * a.ldy * 2;
   unsigned char* out = reinterpret_cast<unsigned char*>(a.y + (int64_t)m0 * a.ldy + n0);
 #pragma unroll
   for (int t = 0; t < RF; ++t) {
-    const int row = 16 * t + lr;
-    const float sx = *reinterpret_cast<const float*>(lds + CODES + row / RPW * RING + row % RPW * 4);
     unsigned int o[NF][2];
 #pragma unroll
     for (int j = 0; j < NF; ++j)
@@ -246,7 +254,7 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           // three separately rounded fp32 operations (no fused multiply-add)
-          v[e] = (float)acc[t][j][2 * c + e] * sx;
+          v[e] = (float)acc[t][j][2 * c + e] * sx[t];
           v[e] = v[e] * sw[j][2 * c + e];
           v[e] = v[e] + bias[j][2 * c + e];
         }
@@ -261,10 +269,10 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
 
 // Row fragments * 8 + column fragments of a wavefront in the tile; 0 = not this form.
 // The smallest tile whose tiles fit the CUs once; a second round costs more than the smaller tile gains (4096 x 768 -> 2304: 32 x 384 tiles, three
-// rounds, 21.7 us, 64 x 384, two, 21.5, 64 x 768 17.3), and beyond one round of the largest the two launches are ahead (6000 x 768 -> 2304 30 / 31,
-// 2700 x 1024 -> 4096 28.7 / 36).  On longer rows the quantiser's share grows with the rows a workgroup has: 64 x 384 tiles only from about 180 of
-// them on (us, two launches / one: 1024 x 1280 -> 3840, 160 tiles, 14.9 / 15.4, 1200 x 1280 -> 3840, 190, 17.3 / 15.7, 1024 x 1024 -> 4096, 176, 14.2 / 13.6), and
-// behind 1280 values the small-tile product's rows stay with it (300 x 1280 -> 1280 8.4 / 9.0, 400, beyond them, 11.9 / 9.2).
+// rounds, 20.7 us, 64 x 384, two, 19.6, 64 x 768 16.9), and beyond one round of the largest the two launches are ahead (6000 x 768 -> 2304 26.6 / 29.3,
+// 2700 x 1024 -> 4096 27.2 / 34.5).  On longer rows the quantiser's share grows with the rows a workgroup has: 64 x 384 tiles only from about 180 of
+// them on (us, two launches / one: 1024 x 1280 -> 3840, 160 tiles, 14.1 / 14.8, 1200 x 1280 -> 3840, 190, 17.2 / 15.2, 900 x 1024 -> 4096, 165, 13.0 / 12.5, a call 12.6 / 12.1), and
+// behind 1280 values the small-tile product's rows stay with it (300 x 1280 -> 1280 8.0 / 8.4, 400, beyond them, 11.9 / 9.0).
 static int band_shape(int64_t M, int N, int K) {
   const int mode = knob_or(KNOB_LINEAR_BAND, 1);
   if (mode <= 0 || knob_or(KNOB_LINEAR_SMALL, 1) <= 0 || K % 128 != 0 || K < 256 || K > 1280 || N % 8 != 0 || M < 32 || N < 384 || M > (1 << 20) || (int64_t)N * K >= (1ll << 31)) return 0;
