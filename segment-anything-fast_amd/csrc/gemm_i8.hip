@@ -1234,8 +1234,8 @@ extern "C" int64_t samfast_linear_i8_workspace(int64_t M, int N, int K, int layo
 
 extern "C" int samfast_linear_i8_one_launch(int64_t M, int N, int K, int layout) {
   using namespace samfast;
-  if (layout == SAMFAST_LAYOUT_SPARSE24) return linear_i8_small_covers(M, N, K, true);
-  return linear_i8_small_covers(M, N, K, false) || linear_i8_band_covers(M, N, K);
+  const bool sparse = layout == SAMFAST_LAYOUT_SPARSE24;
+  return linear_i8_small_covers(M, N, K, sparse) || linear_i8_band_covers(M, N, K, sparse);
 }
 
 // Whether rows of x and of y may share memory: one launch reads some while it writes others.
@@ -1250,13 +1250,13 @@ extern "C" int samfast_linear_i8(const void* x, int64_t ldx, const int8_t* wq, c
   using namespace samfast;
   SF_REQUIRE(layout == SAMFAST_LAYOUT_ROWMAJOR || layout == SAMFAST_LAYOUT_KB64, "linear_i8: unknown layout %d", layout);
   const bool small = M > 0 && linear_i8_small_covers(M, N, K, false), any_alignment = small && linear_i8_small_any_alignment(M, K);
-  if (any_alignment || (M > 0 && (small || linear_i8_band_covers(M, N, K)) && !rows_may_meet(x, ldx, y, ldy, M, N, K))) {
+  if (any_alignment || (M > 0 && (small || linear_i8_band_covers(M, N, K, false)) && !rows_may_meet(x, ldx, y, ldy, M, N, K))) {
     SF_REQUIRE(dtype == SAMFAST_BF16, "linear_i8: only bf16");
     SF_REQUIRE(x && wq && sw && y && aligned16(x) && aligned16(wq) && aligned16(y) && (any_alignment || (aligned16(sw) && aligned16(bias))),
                "linear_i8: null or unaligned pointer");
     SF_REQUIRE(ldx >= K && ldx % 8 == 0 && ldy >= N && ldy % 8 == 0, "linear_i8: row strides must be multiples of 8, >= K and >= N");
     if (!small)
-      return linear_i8_band_launch(reinterpret_cast<const unsigned short*>(x), ldx, wq, sw, bias, reinterpret_cast<unsigned short*>(y), ldy,
+      return linear_i8_band_launch(reinterpret_cast<const unsigned short*>(x), ldx, wq, nullptr, sw, bias, reinterpret_cast<unsigned short*>(y), ldy,
                                    (int)M, N, K, layout, reinterpret_cast<hipStream_t>(stream));
     return linear_i8_small_launch(reinterpret_cast<const unsigned short*>(x), ldx, wq, nullptr, sw, bias, reinterpret_cast<unsigned short*>(y), ldy,
                                   (int)M, N, K, layout, reinterpret_cast<hipStream_t>(stream));
@@ -1284,12 +1284,16 @@ extern "C" int samfast_linear_i8_sparse24(const void* x, int64_t ldx, const int8
                                           const float* sw, const float* bias, void* y, int64_t ldy, void* workspace,
                                           int64_t M, int N, int K, int dtype, void* stream) {
   using namespace samfast;
-  if (M > 0 && linear_i8_small_covers(M, N, K, true) && !rows_may_meet(x, ldx, y, ldy, M, N, K)) {
+  const bool small = M > 0 && linear_i8_small_covers(M, N, K, true);
+  if (M > 0 && (small || linear_i8_band_covers(M, N, K, true)) && !rows_may_meet(x, ldx, y, ldy, M, N, K)) {
     SF_REQUIRE(dtype == SAMFAST_BF16, "linear_i8_sparse24: only bf16");
     SF_REQUIRE(x && wc && widx && sw && y && aligned16(x) && aligned16(wc) && aligned16(widx) && aligned16(y) && aligned16(sw) && aligned16(bias),
                "linear_i8_sparse24: null or unaligned pointer");
     SF_REQUIRE(ldx >= K && ldx % 8 == 0 && ldy >= N && ldy % 8 == 0 && (int64_t)N * 32 < (1ll << 31),
                "linear_i8_sparse24: row strides must be multiples of 8, >= K and >= N");
+    if (!small)
+      return linear_i8_band_launch(reinterpret_cast<const unsigned short*>(x), ldx, wc, widx, sw, bias, reinterpret_cast<unsigned short*>(y), ldy,
+                                   (int)M, N, K, 0, reinterpret_cast<hipStream_t>(stream));
     return linear_i8_small_launch(reinterpret_cast<const unsigned short*>(x), ldx, wc, widx, sw, bias, reinterpret_cast<unsigned short*>(y), ldy,
                                   (int)M, N, K, 0, reinterpret_cast<hipStream_t>(stream));
   }

@@ -1,5 +1,5 @@
-// A whole quantised Linear over a band of rows and a range of columns per workgroup: row quantiser, int8 product and the scale + bias
-// epilogue in one launch, for the row counts between linear_i8_small.hip's and those whose products fill the GPU in rounds.
+// A whole quantised Linear, 2:4 ones too, over a band of rows and a range of columns per workgroup: row quantiser, int8 product and the scale +
+// bias epilogue in one launch, for the row counts between linear_i8_small.hip's and those whose products fill the GPU in rounds.
 //
 // Two launches of such a call are mostly starts and ends (4096 x 768 -> 3072: 5 and 15 us for 4.5 us of matrix pipe), the codes go through
 // memory between them, and the host pays for both.  Here every workgroup quantises its 32 or 64 rows itself - once per range of columns,
@@ -22,10 +22,13 @@
 
 namespace samfast {
 
+typedef int i32x8 __attribute__((ext_vector_type(8)));
+
 struct BandArgs {
   const unsigned short* x;
   int64_t ldx;
   const int8_t* w;
+  const int32_t* widx;  // 2:4 weights: `w` holds (K/64, N, 32) bytes, this (K/64, N, 2) words
   const float* sw;
   const float* bias;
   unsigned short* y;
@@ -48,12 +51,13 @@ SF_DEVICE void band_wait(int n) {
 }
 
 // KMAX: 128 * the chunks of 8 values a lane holds of a row; RF: fragments of 16 rows; NF: fragments of 16 columns of a wavefront;
-// DEPTH: k steps of 128 in a wavefront's ring.  K % 128 == 0, 128 * DEPTH <= K <= KMAX, M >= 16 RF, N >= 128 NF.
-template <int KMAX, int RF, int NF, int DEPTH>
+// DEPTH: k steps of 128 in a wavefront's ring; SPARSE: packed 2:4 weights (gemm_i8_sparse24.hip), v_smfmac_i32_16x16x128_i8.  K % 128 == 0, 128 * DEPTH <= K <= KMAX, M >= 16 RF, N >= 128 NF.
+template <int KMAX, int RF, int NF, int DEPTH, bool SPARSE>
 __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
   constexpr int R = 16 * RF, BN = 128 * NF, RPW = 2 * RF, NB = RPW / 4;  // rows, columns; rows of a wavefront, quantised four at a time
   constexpr int NCH = KMAX / 128;
-  constexpr int SLOT = 2048, RING = NF * DEPTH * SLOT;  // a column fragment: 16 columns x 128 bytes
+  // a column fragment: 16 columns x 128 bytes; SPARSE: 16 x 64 and their index words.  Requested in two parts
+  constexpr int PART = SPARSE ? 256 : 1024, SLOT = 1024 + PART, RING = NF * DEPTH * SLOT;
   constexpr int CODES = R * KMAX;
   static_assert(CODES + 8 * RING <= 160 * 1024, "LDS of a CU");
   static_assert(2 * (NF * DEPTH - 1) <= 15, "wait thresholds");
@@ -102,28 +106,30 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
   for (int j = 0; j < NF; ++j)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int r = 8 * h + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+      // SPARSE: 64-k block by block, the 32 bytes of every row; then, sixteen lanes, the 8 bytes of indices of two rows each
+      const int r = SPARSE ? (h == 0 ? (lane & 31) >> 1 : 2 * (lane & 7)) : 8 * h + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
       const int col = NF % 2 == 1 && j == NF - 1 ? 16 * j + r : 32 * (j / 2) + 8 * (r >> 2) + 4 * (j & 1) + (r & 3);
-      w_off[j][h] = (unsigned int)col * a.w_pitch + (unsigned int)(c >> 2) * a.w_kstep + (unsigned int)(c & 3) * 16u;
+      if (!SPARSE) w_off[j][h] = (unsigned int)col * a.w_pitch + (unsigned int)(c >> 2) * a.w_kstep + (unsigned int)(c & 3) * 16u;
+      else if (h == 0) w_off[j][h] = (unsigned int)((lane >> 5) * a.N + col) * 32u + (lane & 1) * 16u;
+      else w_off[j][h] = (unsigned int)((lane >> 3 & 1) * a.N + col) * 8u;
     }
   unsigned char* ring = lds + CODES + wave * RING;
   const unsigned int ring_at = (unsigned int)(uintptr_t)((__attribute__((address_space(3))) unsigned char*)ring);
-  const unsigned char* wbase = reinterpret_cast<const unsigned char*>(a.w) + (int64_t)n0 * a.w_pitch;
-  const int64_t w_step = 2 * (int64_t)a.w_kstep;
-  auto load_w = [&](const unsigned char* from, int j, unsigned int slots) __attribute__((always_inline)) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) lds_dma16(from, w_off[j][h], ring_at + slots + j * SLOT + h * 1024);
+  const unsigned char* wbase = reinterpret_cast<const unsigned char*>(a.w) + (int64_t)n0 * (SPARSE ? 32 : a.w_pitch);
+  const unsigned char* ibase = reinterpret_cast<const unsigned char*>(a.widx) + (int64_t)n0 * 8;
+  const int64_t w_step = SPARSE ? (int64_t)a.N * 64 : 2 * (int64_t)a.w_kstep, i_step = (int64_t)a.N * 16;
+  // part h of fragment j of k step k
+  auto load_w = [&](int k, int j, int h, unsigned int slot) __attribute__((always_inline)) {
+    if (!SPARSE || h == 0) lds_dma16(wbase + k * w_step, w_off[j][h], ring_at + slot + h * 1024);
+    else if (lane < 16) lds_dma16(ibase + k * i_step, w_off[j][h], ring_at + slot + 1024);
   };
   // request i of the first DEPTH k steps' 2 NF DEPTH, between the rows' chunks
-  auto first_w = [&](int i) __attribute__((always_inline)) {
-    const int d = i / (2 * NF), j = i / 2 % NF, h = i % 2;
-    lds_dma16(wbase + d * w_step, w_off[j][h], ring_at + d * NF * SLOT + j * SLOT + h * 1024);
-  };
+  auto first_w = [&](int i) __attribute__((always_inline)) { load_w(i / (2 * NF), i / 2 % NF, i % 2, i / 2 * SLOT); };
 
   // ---- codes: 128 bytes of every row to a block, chunks at the same positions as W's. -------------------------------------------------
-  // Row scales: beside the rings, or, where LDS is full, in the place of each ring's last KB, whose request then waits for them to be read
+  // Row scales: beside the rings, or, where LDS is full, in the place of each ring's last part, whose request then waits for them to be read
   auto scale_of = [&](int row) __attribute__((always_inline)) {
-    return reinterpret_cast<float*>(ROOM ? lds + CODES + 8 * RING + row * 4 : lds + CODES + row / RPW * RING + RING - 1024 + row % RPW * 4);
+    return reinterpret_cast<float*>(ROOM ? lds + CODES + 8 * RING + row * 4 : lds + CODES + row / RPW * RING + RING - PART + row % RPW * 4);
   };
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
@@ -194,11 +200,16 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
   for (int t = 0; t < RF; ++t)
 #pragma unroll
     for (int j = 0; j < NF; ++j) acc[t][j] = i32x4{0, 0, 0, 0};
-  int frag[2];  // of the 64-byte halves of a block
+  // Of a 128-byte row of codes the two 16-byte chunks of the lane, of a fragment its bytes.  SPARSE: lane (i, q) holds the stored half q % 2 of
+  // 64-k block q / 2 of weight row i, so that lane (j, Q) of the codes wants chunks 2 (Q % 2) + Q / 2 and four more (gemm_i8_sp24_turns.hip)
+  int frag[2], wfrag[2];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) frag[h] = lr * 128 + (((4 * h + lq) ^ ((lr >> 1) & 7)) * 16);
-  // k step k out of the slots at `slots`; LEFT: k steps behind it whose W has been requested; `from`: W of step k + DEPTH
-  auto step = [&](int k, unsigned int slots, auto left_c, const unsigned char* from) __attribute__((always_inline)) {
+  for (int h = 0; h < 2; ++h) {
+    frag[h] = lr * 128 + (((4 * h + (SPARSE ? 2 * (lq & 1) + (lq >> 1) : lq)) ^ ((lr >> 1) & 7)) * 16);
+    wfrag[h] = !SPARSE ? frag[h] : h == 0 ? (lq >> 1) * 512 + lr * 32 + (lq & 1) * 16 : 1024 + (lq >> 1) * 128 + lr * 8 + (lq & 1) * 4;
+  }
+  // k step k out of the slots at `slots`; LEFT: k steps behind it whose W has been requested
+  auto step = [&](int k, unsigned int slots, auto left_c) __attribute__((always_inline)) {
     constexpr int LEFT = decltype(left_c)::value;
     constexpr bool REQUEST = LEFT == DEPTH;
     i32x4 xf[RF][2];
@@ -209,33 +220,45 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
 #pragma unroll
     for (int j = 0; j < NF; ++j) {
       band_wait(REQUEST ? 2 * (NF * DEPTH - 1) : 2 * (NF * (LEFT + 1) - 1 - j));
+      const unsigned char* f = ring + slots + j * SLOT;
       i32x4 wf[2];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) wf[h] = *reinterpret_cast<const i32x4*>(ring + slots + j * SLOT + frag[h]);
+      int index = 0;
+      wf[0] = *reinterpret_cast<const i32x4*>(f + wfrag[0]);
+      if (SPARSE) index = *reinterpret_cast<const int*>(f + wfrag[1]);
+      else wf[1] = *reinterpret_cast<const i32x4*>(f + wfrag[1]);
       __builtin_amdgcn_s_waitcnt(0xC07F);  // the fragment is in registers: its slot is requested anew
       __builtin_amdgcn_sched_barrier(0);
-      if (REQUEST) load_w(from, j, slots);
+      if (REQUEST) {
+        load_w(k + DEPTH, j, 0, slots + j * SLOT);
+        load_w(k + DEPTH, j, 1, slots + j * SLOT);
+      }
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (SPARSE) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+        for (int t = 0; t < RF; ++t) {
+          const i32x8 x8 = {xf[t][0][0], xf[t][0][1], xf[t][0][2], xf[t][0][3], xf[t][1][0], xf[t][1][1], xf[t][1][2], xf[t][1][3]};
+          acc[t][j] = __builtin_amdgcn_smfmac_i32_16x16x128_i8(wf[0], x8, acc[t][j], index, 0, 0);
+        }
+      } else {
 #pragma unroll
-        for (int t = 0; t < RF; ++t) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[h], xf[t][h], acc[t][j], 0, 0, 0);
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int t = 0; t < RF; ++t) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[h], xf[t][h], acc[t][j], 0, 0, 0);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
   unsigned int slots = 0;
-  const unsigned char* from = wbase + DEPTH * w_step;
   int k = 0;
   for (; k + DEPTH < steps; ++k) {
-    step(k, slots, std::integral_constant<int, DEPTH>{}, from);
-    from += w_step;
+    step(k, slots, std::integral_constant<int, DEPTH>{});
     slots = DEPTH == 1 || slots == (DEPTH - 1) * NF * SLOT ? 0 : slots + NF * SLOT;
   }
   if (DEPTH == 2) {
-    step(k++, slots, std::integral_constant<int, DEPTH - 1>{}, from);
+    step(k++, slots, std::integral_constant<int, DEPTH - 1>{});
     slots = slots == 0 ? NF * SLOT : 0;
   }
-  step(k, slots, std::integral_constant<int, 0>{}, from);
+  step(k, slots, std::integral_constant<int, 0>{});
 
   // ---- (float(acc) * sx) * sw + bias; a wavefront that is through finishes under the others' products ------------------------------------
   if (!a.bias)  // uniform
@@ -273,20 +296,25 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
 // 2700 x 1024 -> 4096 27.2 / 34.5).  On longer rows the quantiser's share grows with the rows a workgroup has: 64 x 384 tiles only from about 180 of
 // them on (us, two launches / one: 1024 x 1280 -> 3840, 160 tiles, 14.1 / 14.8, 1200 x 1280 -> 3840, 190, 17.2 / 15.2, 900 x 1024 -> 4096, 165, 13.0 / 12.5, a call 12.6 / 12.1), and
 // behind 1280 values the small-tile product's rows stay with it (300 x 1280 -> 1280 8.0 / 8.4, 400, beyond them, 11.9 / 9.0).
-static int band_shape(int64_t M, int N, int K) {
+// 2:4 weights: the two launches take longer (the quantiser is the same, the products are bound by what they load) and win nowhere below one round,
+// but for 64 x 640 tiles on the longest rows, level up to about 200 of them (1800 x 1280 -> 3840, 174, 18.3 / 18.5): us, two / one, 4096 x 768 -> 3072 20.5 / 16.2, 4096 x 768 -> 768 13.3 / 8.7, 1024 x 768 -> 3072 11.9 / 8.2, 1024 x 1024 -> 1024
+// 11.6 / 7.8, 512 x 1280 -> 5120 13.9 / 10.3, 200 x 1280 -> 1280 9.5 / 8.4, 700 x 1280 -> 5120 14.9 / 13.8, 2048 x 1280 -> 5120 (256 tiles) 22.7 / 19.3; 2048 x 1280 -> 3840 (192)
+// 18.8 / 19.0, a call 17.5 / 18.3.
+static int band_shape(int64_t M, int N, int K, bool sparse) {
   const int mode = knob_or(KNOB_LINEAR_BAND, 1);
   if (mode <= 0 || knob_or(KNOB_LINEAR_SMALL, 1) <= 0 || K % 128 != 0 || K < 256 || K > 1280 || N % 8 != 0 || M < 32 || N < 384 || M > (1 << 20) || (int64_t)N * K >= (1ll << 31)) return 0;
   auto tiles = [&](int rf, int nf) { return (M + 16 * rf - 1) / (16 * rf) * ((N + 128 * nf - 1) / (128 * nf)); };
   auto fits = [&](int rf, int nf) { return M >= 16 * rf && N >= 128 * nf && tiles(rf, nf) <= 256; };
   const int wide = K <= 1024 ? 6 : 5;
   if (mode > 1) return (mode == 2 * 8 + 3 || mode == 4 * 8 + 3 || mode == 4 * 8 + wide) && M >= 16 * (mode / 8) && N >= 128 * (mode % 8) ? mode : 0;
-  if (K > 1024 && (M + 63) / 64 * ((N + 31) / 32) <= 256) return 0;
+  if (!sparse && K > 1024 && (M + 63) / 64 * ((N + 31) / 32) <= 256) return 0;
   if (fits(2, 3)) return 2 * 8 + 3;
-  if (fits(4, 3)) return K <= 768 || tiles(4, 3) >= 176 ? 4 * 8 + 3 : 0;
+  if (fits(4, 3)) return sparse || K <= 768 || tiles(4, 3) >= 176 ? 4 * 8 + 3 : 0;
+  if (sparse && K > 1152 && tiles(4, wide) < 208) return 0;
   return fits(4, wide) ? 4 * 8 + wide : 0;
 }
 
-bool linear_i8_band_covers(int64_t M, int N, int K) { return band_shape(M, N, K) != 0; }
+bool linear_i8_band_covers(int64_t M, int N, int K, bool sparse) { return band_shape(M, N, K, sparse) != 0; }
 
 template <int KMAX, int RF, int NF, int DEPTH>
 static int launch_band(BandArgs a, hipStream_t stream) {
@@ -300,7 +328,9 @@ static int launch_band(BandArgs a, hipStream_t stream) {
   int g = 1;
   while (g < a.tiles_m && (g + 1) * (g + 1) * 2 * 16 * RF <= t * 128 * NF) ++g;
   a.group_m = g;
-  hipLaunchKernelGGL((linear_i8_band_kernel<KMAX, RF, NF, DEPTH>), dim3((unsigned int)((a.tiles + 7) / 8 * 8)), dim3(512), 0, stream, a);
+  const dim3 grid((unsigned int)((a.tiles + 7) / 8 * 8));
+  if (a.widx) hipLaunchKernelGGL((linear_i8_band_kernel<KMAX, RF, NF, DEPTH, true>), grid, dim3(512), 0, stream, a);
+  else hipLaunchKernelGGL((linear_i8_band_kernel<KMAX, RF, NF, DEPTH, false>), grid, dim3(512), 0, stream, a);
   return check_launch("linear_i8_band_kernel");
 }
 
@@ -318,14 +348,14 @@ static int launch_band_shape(const BandArgs& a, int shape, hipStream_t stream) {
   return SAMFAST_E_UNSUPPORTED;
 }
 
-int linear_i8_band_launch(const unsigned short* x, int64_t ldx, const int8_t* w, const float* sw, const float* bias, unsigned short* y,
+int linear_i8_band_launch(const unsigned short* x, int64_t ldx, const int8_t* w, const int32_t* widx, const float* sw, const float* bias, unsigned short* y,
                           int64_t ldy, int M, int N, int K, int layout, hipStream_t stream) {
   BandArgs a = {};
-  a.x = x; a.ldx = ldx; a.w = w; a.sw = sw; a.bias = bias; a.y = y; a.ldy = ldy; a.M = M; a.N = N; a.K = K;
+  a.x = x; a.ldx = ldx; a.w = w; a.widx = widx; a.sw = sw; a.bias = bias; a.y = y; a.ldy = ldy; a.M = M; a.N = N; a.K = K;
   const bool kb = layout == SAMFAST_LAYOUT_KB64;
   a.w_pitch = kb ? 64 : (unsigned int)K;
   a.w_kstep = kb ? (unsigned int)N * 64u : 64u;
-  const int shape = band_shape(M, N, K);
+  const int shape = band_shape(M, N, K, widx != nullptr);
   if (K <= 768) return launch_band_shape<768>(a, shape, stream);
   if (K <= 1024) return launch_band_shape<1024>(a, shape, stream);
   return launch_band_shape<1280>(a, shape, stream);

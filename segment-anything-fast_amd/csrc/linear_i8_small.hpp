@@ -15,8 +15,8 @@ int linear_i8_small_launch(const unsigned short* x, int64_t ldx, const int8_t* w
                            unsigned short* y, int64_t ldy, int M, int N, int K, int layout, hipStream_t stream);
 
 // The same over more rows, a band of them and a range of columns per workgroup (linear_i8_band.hip).
-bool linear_i8_band_covers(int64_t M, int N, int K);
-int linear_i8_band_launch(const unsigned short* x, int64_t ldx, const int8_t* w, const float* sw, const float* bias, unsigned short* y,
+bool linear_i8_band_covers(int64_t M, int N, int K, bool sparse);
+int linear_i8_band_launch(const unsigned short* x, int64_t ldx, const int8_t* w, const int32_t* widx, const float* sw, const float* bias, unsigned short* y,
                           int64_t ldy, int M, int N, int K, int layout, hipStream_t stream);
 
 // The product with scale + bias epilogue for few rows (the codes come from a quantiser launch).

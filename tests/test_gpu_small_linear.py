@@ -286,6 +286,34 @@ def test_a_band_of_rows_in_one_launch_agrees_with_two(M, N, K):
                 assert torch.equal(y.view(torch.int16), two.view(torch.int16)), tile
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (32, 384, 256), (33, 392, 384), (64, 768, 256), (65, 776, 640), (127, 1528, 768), (200, 2304, 1024), (95, 640, 1152), (129, 1288, 1280),
+    (2100, 2304, 768), (1100, 4096, 1024), (1990, 3840, 1280), (450, 1280, 1280),
+])
+def test_a_band_of_rows_with_sparse_weights(M, N, K):
+    """2:4 weights in every tile that the shape admits and by the rule, against two launches; a row with a NaN and one of zeros."""
+    from samfast_amd import Int8Sparse24Linear, _lib
+    print(f"case sparse band M={M} N={N} K={K}", flush=True)
+    x, w, b = linear_inputs(M, K, N, seed=M + N + K)
+    x[M // 2] = 0
+    x[M - 1, K // 3] = float("nan")
+    lin = torch.nn.Linear(K, N, bias=M % 2 == 1, dtype=torch.bfloat16)
+    with torch.no_grad():
+        lin.weight.copy_(w)
+        if lin.bias is not None:
+            lin.bias.copy_(b)
+    lin, x = Int8Sparse24Linear.from_float(lin.cuda()), x.cuda()
+    with _lib.knobs(SAMFAST_GEMM_LINEAR_SMALL=0):
+        two = lin(x)
+    for tile in (1, 2 * 8 + 3, 4 * 8 + 3, 4 * 8 + (6 if K <= 1024 else 5)):
+        if tile > 1 and (M < 16 * (tile // 8) or N < 128 * (tile % 8)):
+            continue
+        with _lib.knobs(SAMFAST_GEMM_LINEAR_BAND=tile):
+            if tile > 1:
+                assert _lib.load().samfast_linear_i8_one_launch(M, N, K, 2) == 1
+            assert torch.equal(lin(x).view(torch.int16), two.view(torch.int16)), tile
+
+
 def test_a_linear_into_its_own_rows():
     """y may be x where the caller brings the workspace: two launches, the quantiser has read every row before one is written."""
     from samfast_amd import _lib
