@@ -96,6 +96,9 @@ __global__ __launch_bounds__(512, 2) void gemm_i8_strip_kernel(GemmArgs a) {
   const int frag = lr * 64 + ((lq ^ (-(lr >> 2) & 3)) * 16);
   const unsigned char* xfrag = lds + frag;
   const unsigned char* wfrag = lds + NK * BLOCK + wave * RING * 1024 + frag;
+  // of a SIMD's two wavefronts one multiplies ahead of the other and runs its GELU under the other's products (4096 x 768 -> 3072 19.4 / 19.1 us)
+  if (wave < 4) __builtin_amdgcn_s_setprio(3);
+  else __builtin_amdgcn_s_setprio(2);
 #pragma unroll
   for (int k = 0; k < NK; ++k) {
     // outstanding behind what step k reads, of X 0, W 0-2, X 1, W 3-5, X 2, W 6, X 3, .. X 11, W 7, ..: in step 0 X 0 and 1 (and W 0-2), in step 1 W 3-5, from
@@ -125,6 +128,7 @@ __global__ __launch_bounds__(512, 2) void gemm_i8_strip_kernel(GemmArgs a) {
     __builtin_amdgcn_sched_barrier(0);
   }
 
+  __builtin_amdgcn_s_setprio(0);
   if (!a.bias)  // uniform
 #pragma unroll
     for (int j = 0; j < NF; ++j) bias[j] = f32x4{0.f, 0.f, 0.f, 0.f};
