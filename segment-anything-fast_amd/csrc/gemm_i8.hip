@@ -1238,10 +1238,24 @@ extern "C" int samfast_linear_i8_one_launch(int64_t M, int N, int K, int layout)
   return linear_i8_small_covers(M, N, K, sparse) || linear_i8_band_covers(M, N, K, sparse);
 }
 
-// Whether rows of x and of y may share memory: one launch reads some while it writes others.
-static bool rows_may_meet(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t M, int N, int K) {
-  const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
-  return x0 < y0 + 2 * (uintptr_t)((M - 1) * ldy + N) && y0 < x0 + 2 * (uintptr_t)((M - 1) * ldx + K);
+// Whether a row of x and a row of y share memory: one launch reads some while it writes others.  Column ranges of one buffer do not.
+// (Rows shorter than their stride allows: false, for the launch's own checks to refuse.)
+static bool rows_share_memory(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t M, int N, int K) {
+  const int64_t x0 = (int64_t)reinterpret_cast<uintptr_t>(x), y0 = (int64_t)reinterpret_cast<uintptr_t>(y);
+  const int64_t xs = 2 * ldx, ys = 2 * ldy, xw = 2 * (int64_t)K, yw = 2 * (int64_t)N;  // bytes from row to row, of a row
+  if (ldx < K || ldy < N || x0 >= y0 + (M - 1) * ys + yw || y0 >= x0 + (M - 1) * xs + xw) return false;
+  if (xs == ys) {  // y lies at the same offset to the x row in front of it everywhere
+    const int64_t d = ((y0 - x0) % xs + xs) % xs;
+    return d < xw || d + yw > xs;
+  }
+  int64_t j = 0;  // first row of y that ends behind the start of x's row i
+  for (int64_t i = 0; i < M; ++i) {
+    const int64_t at = x0 + i * xs;
+    while (j < M && y0 + j * ys + yw <= at) ++j;
+    if (j == M) return false;
+    if (y0 + j * ys < at + xw) return true;
+  }
+  return false;
 }
 
 extern "C" int samfast_linear_i8(const void* x, int64_t ldx, const int8_t* wq, const float* sw, const float* bias,
@@ -1250,7 +1264,7 @@ extern "C" int samfast_linear_i8(const void* x, int64_t ldx, const int8_t* wq, c
   using namespace samfast;
   SF_REQUIRE(layout == SAMFAST_LAYOUT_ROWMAJOR || layout == SAMFAST_LAYOUT_KB64, "linear_i8: unknown layout %d", layout);
   const bool small = M > 0 && linear_i8_small_covers(M, N, K, false), any_alignment = small && linear_i8_small_any_alignment(M, K);
-  if (any_alignment || (M > 0 && (small || linear_i8_band_covers(M, N, K, false)) && !rows_may_meet(x, ldx, y, ldy, M, N, K))) {
+  if (any_alignment || (M > 0 && (small || linear_i8_band_covers(M, N, K, false)) && !rows_share_memory(x, ldx, y, ldy, M, N, K))) {
     SF_REQUIRE(dtype == SAMFAST_BF16, "linear_i8: only bf16");
     SF_REQUIRE(x && wq && sw && y && aligned16(x) && aligned16(wq) && aligned16(y) && (any_alignment || (aligned16(sw) && aligned16(bias))),
                "linear_i8: null or unaligned pointer");
@@ -1285,7 +1299,7 @@ extern "C" int samfast_linear_i8_sparse24(const void* x, int64_t ldx, const int8
                                           int64_t M, int N, int K, int dtype, void* stream) {
   using namespace samfast;
   const bool small = M > 0 && linear_i8_small_covers(M, N, K, true);
-  if (M > 0 && (small || linear_i8_band_covers(M, N, K, true)) && !rows_may_meet(x, ldx, y, ldy, M, N, K)) {
+  if (M > 0 && (small || linear_i8_band_covers(M, N, K, true)) && !rows_share_memory(x, ldx, y, ldy, M, N, K)) {
     SF_REQUIRE(dtype == SAMFAST_BF16, "linear_i8_sparse24: only bf16");
     SF_REQUIRE(x && wc && widx && sw && y && aligned16(x) && aligned16(wc) && aligned16(widx) && aligned16(y) && aligned16(sw) && aligned16(bias),
                "linear_i8_sparse24: null or unaligned pointer");

@@ -698,3 +698,41 @@ def test_a_recording_follows_the_stream_of_its_last_call(monkeypatch):
         recording.follow()
     assert seen == [("waits for", streams[1], streams[0]), ("used on", streams[1]),
                     ("waits for", streams[0], streams[1]), ("used on", streams[0])]
+
+
+def _linear_route(M, N, K, x_at, ldx, y_at, ldy, sparse=False):
+    """Which launches a call without a workspace would be: "one", or "two" (refused then).  The type is one that no kernel
+    takes, so that nothing is launched: the one launch refuses it, the two ask for their workspace first."""
+    from samfast_amd import _lib
+    lib = _lib.load()
+    base = 1 << 40  # elements are 2 bytes; weights, scales and bias lie elsewhere
+    weights = (base - (1 << 30),) + ((base - (1 << 29),) if sparse else ())
+    args = (base + 2 * x_at, ldx) + weights + (base - (1 << 28), base - (1 << 27), base + 2 * y_at, ldy, None, M, N, K, _lib.SAMFAST_F16)
+    assert (lib.samfast_linear_i8_sparse24(*args, None) if sparse else lib.samfast_linear_i8(*args, 0, None)) == -1
+    error = lib.samfast_last_error()
+    assert b"only bf16" in error or b"workspace must be" in error, error
+    return "one" if b"only bf16" in error else "two"
+
+
+@pytest.mark.parametrize("sparse", [False, True])
+@pytest.mark.parametrize("M,N,K", [(40, 384, 256), (600, 640, 256), (64, 64, 256)])  # few rows, a band of rows, N under K
+def test_a_linear_is_one_launch_unless_its_rows_share_memory(M, N, K, sparse):
+    """x and y as column ranges of one buffer do not; one element in common does.  Against a count of the elements."""
+    import random
+    rng = random.Random(M + N)
+    assert _linear_route(M, N, K, 0, K, 0, N, sparse) == "two"  # y over x
+    ld = K + N
+    assert _linear_route(M, N, K, 0, ld, K, ld, sparse) == "one"
+    assert _linear_route(M, N, K, N, ld, 0, ld, sparse) == "one"
+    assert _linear_route(M, N, K, 0, ld, K - 8, ld, sparse) == "two"
+    assert _linear_route(M, N, K, N - 8, ld, 0, ld, sparse) == "two"
+    assert _linear_route(M, N, K, 0, ld, K + M * ld, ld, sparse) == "one"  # behind one another
+    for _ in range(40):
+        ldx, ldy = K + 8 * rng.randint(0, 90), N + 8 * rng.randint(0, 90)
+        ldy = ldx if rng.random() < 0.5 and ldx >= N else ldy
+        x_at, y_at = 0, 8 * rng.randint(0, (M * ldx) // 8)
+        if rng.random() < 0.5:
+            x_at, y_at = y_at, x_at
+        taken = {e for i in range(M) for e in range((x_at + i * ldx) // 8, (x_at + i * ldx + K) // 8)}
+        shared = any(e in taken for i in range(M) for e in range((y_at + i * ldy) // 8, (y_at + i * ldy + N) // 8))
+        assert _linear_route(M, N, K, x_at, ldx, y_at, ldy, sparse) == ("two" if shared else "one"), (x_at, ldx, y_at, ldy)
