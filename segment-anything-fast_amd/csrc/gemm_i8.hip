@@ -1227,7 +1227,6 @@ extern "C" int64_t samfast_linear_i8_workspace(int64_t M, int N, int K, int layo
   using namespace samfast;
   SF_REQUIRE(M > 0 && N > 0 && K > 0 && layout >= SAMFAST_LAYOUT_ROWMAJOR && layout <= SAMFAST_LAYOUT_SPARSE24,
              "linear_i8_workspace: bad shape M=%lld N=%d K=%d or layout %d", (long long)M, N, K, layout);
-  if (layout != SAMFAST_LAYOUT_SPARSE24 && linear_i8_small_any_alignment(M, K) && linear_i8_small_covers(M, N, K, false)) return 0;
   const int64_t weights = layout == SAMFAST_LAYOUT_ROWMAJOR && linear_reorders_weights(M, N, K) ? (int64_t)N * K : 0;
   return linear_codes_bytes(M, K) + linear_scales_bytes(M) + weights;
 }
@@ -1239,7 +1238,7 @@ extern "C" int samfast_linear_i8_one_launch(int64_t M, int N, int K, int layout)
 }
 
 // Whether a row of x and a row of y share memory: one launch reads some while it writes others.  Column ranges of one buffer do not.
-// (Rows shorter than their stride allows: false, for the launch's own checks to refuse.)
+// (A stride shorter than its rows: false, for the one launch to refuse.)
 static bool rows_share_memory(const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t M, int N, int K) {
   const int64_t x0 = (int64_t)reinterpret_cast<uintptr_t>(x), y0 = (int64_t)reinterpret_cast<uintptr_t>(y);
   const int64_t xs = 2 * ldx, ys = 2 * ldy, xw = 2 * (int64_t)K, yw = 2 * (int64_t)N;  // bytes from row to row, of a row
@@ -1264,7 +1263,7 @@ extern "C" int samfast_linear_i8(const void* x, int64_t ldx, const int8_t* wq, c
   using namespace samfast;
   SF_REQUIRE(layout == SAMFAST_LAYOUT_ROWMAJOR || layout == SAMFAST_LAYOUT_KB64, "linear_i8: unknown layout %d", layout);
   const bool small = M > 0 && linear_i8_small_covers(M, N, K, false), any_alignment = small && linear_i8_small_any_alignment(M, K);
-  if (any_alignment || (M > 0 && (small || linear_i8_band_covers(M, N, K, false)) && !rows_share_memory(x, ldx, y, ldy, M, N, K))) {
+  if (M > 0 && (small || linear_i8_band_covers(M, N, K, false)) && !rows_share_memory(x, ldx, y, ldy, M, N, K)) {
     SF_REQUIRE(dtype == SAMFAST_BF16, "linear_i8: only bf16");
     SF_REQUIRE(x && wq && sw && y && aligned16(x) && aligned16(wq) && aligned16(y) && (any_alignment || (aligned16(sw) && aligned16(bias))),
                "linear_i8: null or unaligned pointer");

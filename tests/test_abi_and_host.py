@@ -736,3 +736,15 @@ def test_a_linear_is_one_launch_unless_its_rows_share_memory(M, N, K, sparse):
         taken = {e for i in range(M) for e in range((x_at + i * ldx) // 8, (x_at + i * ldx + K) // 8)}
         shared = any(e in taken for i in range(M) for e in range((y_at + i * ldy) // 8, (y_at + i * ldy + N) // 8))
         assert _linear_route(M, N, K, x_at, ldx, y_at, ldy, sparse) == ("two" if shared else "one"), (x_at, ldx, y_at, ldy)
+
+
+@pytest.mark.parametrize("M,K", [(1, 256), (8, 1024), (8, 5120), (9, 2048), (16, 2048), (17, 768), (32, 768)])
+def test_a_linear_over_a_handful_of_rows_into_those_rows_takes_a_workspace(M, K):
+    """The sizes at which scales of any alignment are taken: one launch reads rows of x in every workgroup while others write y, so
+    that y over x is two launches there too, refused without a workspace, and the size of one is told."""
+    from samfast_amd import _lib
+    lib = _lib.load()
+    assert lib.samfast_linear_i8_one_launch(M, K, K, 0) == 1
+    assert lib.samfast_linear_i8_workspace(M, K, K, 0) >= M * K + 4 * M
+    assert _linear_route(M, K, K, 0, K, 0, K) == "two"
+    assert _linear_route(M, K, K, 0, 2 * K, K, 2 * K) == "one"

@@ -328,3 +328,17 @@ def test_a_linear_into_its_own_rows():
         assert lib.samfast_linear_i8(x.data_ptr(), K, lin.wq.data_ptr(), lin.sw.data_ptr(), lin.bias_f32.data_ptr(), x.data_ptr(), K,
                                      work.data_ptr(), M, K, K, _lib.SAMFAST_BF16, 0, stream) == 0
         assert torch.equal(x, want)
+
+
+@pytest.mark.parametrize("M,K", [(1, 768), (8, 1024), (8, 5120), (16, 2048), (32, 768)])
+def test_a_linear_over_a_handful_of_rows_into_those_rows(M, K):
+    """The same where one launch takes scales of any alignment."""
+    from samfast_amd import _lib
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    lin = _linear(K, K, M)
+    x = torch.randn((M, K), device="cuda").to(torch.bfloat16)
+    want = lin(x)
+    work = torch.empty(lib.samfast_linear_i8_workspace(M, K, K, 0), dtype=torch.int8, device="cuda")
+    assert lib.samfast_linear_i8(x.data_ptr(), K, lin.wq.data_ptr(), lin.sw.data_ptr(), lin.bias_f32.data_ptr(), x.data_ptr(), K,
+                                 work.data_ptr(), M, K, K, _lib.SAMFAST_BF16, 0, stream) == 0
+    assert torch.equal(x, want)
