@@ -190,14 +190,14 @@ int samfast_gemm_i8_scale_bias(
  * samfast_gemm_i8_scale_bias, same codes, accumulators and result.  `layout` is the layout of wq;
  * nothing of the weights is kept from one call for the next.  `workspace`: at least
  * samfast_linear_i8_workspace(M, N, K, layout) bytes of device memory, 16-byte aligned, contents
- * irrelevant before and after.  The size function returns
+ * irrelevant before and after.  This and samfast_linear_i8_one_launch return
  * SAMFAST_E_INVALID for a negative or zero dimension or an unknown layout; with
- * SAMFAST_LAYOUT_SPARSE24 it answers for samfast_linear_i8_sparse24.  Where
+ * SAMFAST_LAYOUT_SPARSE24 they answer for samfast_linear_i8_sparse24.  Where
  * samfast_linear_i8_one_launch(M, N, K, layout) is 1, a call in which no row of x shares memory with a row of y
  * uses no workspace: it may be NULL.  Rows of y may lie over rows of x at any size; with the workspace, which is
  * then needed, every row of x has been read before one of y is written.
  */
-#define SAMFAST_LAYOUT_SPARSE24 2  /* samfast_linear_i8_workspace only */
+#define SAMFAST_LAYOUT_SPARSE24 2  /* samfast_linear_i8_workspace and samfast_linear_i8_one_launch only */
 int samfast_linear_i8(
     const void* x, int64_t ldx, const int8_t* wq, const float* sw, const float* bias,
     void* y, int64_t ldy, void* workspace,

@@ -1221,18 +1221,23 @@ static bool linear_reorders_weights(int64_t M, int N, int K) { return M >= 16384
 static int64_t linear_codes_bytes(int64_t M, int K) { return (M * K + 15) & ~(int64_t)15; }
 static int64_t linear_scales_bytes(int64_t M) { return (M * 4 + 15) & ~(int64_t)15; }
 
+// what the two questions about a Linear (workspace, launches) answer
+static bool linear_shape_ok(int64_t M, int N, int K, int layout) {
+  return M > 0 && N > 0 && K > 0 && layout >= SAMFAST_LAYOUT_ROWMAJOR && layout <= SAMFAST_LAYOUT_SPARSE24;
+}
+
 }  // namespace samfast
 
 extern "C" int64_t samfast_linear_i8_workspace(int64_t M, int N, int K, int layout) {
   using namespace samfast;
-  SF_REQUIRE(M > 0 && N > 0 && K > 0 && layout >= SAMFAST_LAYOUT_ROWMAJOR && layout <= SAMFAST_LAYOUT_SPARSE24,
-             "linear_i8_workspace: bad shape M=%lld N=%d K=%d or layout %d", (long long)M, N, K, layout);
+  SF_REQUIRE(linear_shape_ok(M, N, K, layout), "linear_i8_workspace: bad shape M=%lld N=%d K=%d or layout %d", (long long)M, N, K, layout);
   const int64_t weights = layout == SAMFAST_LAYOUT_ROWMAJOR && linear_reorders_weights(M, N, K) ? (int64_t)N * K : 0;
   return linear_codes_bytes(M, K) + linear_scales_bytes(M) + weights;
 }
 
 extern "C" int samfast_linear_i8_one_launch(int64_t M, int N, int K, int layout) {
   using namespace samfast;
+  SF_REQUIRE(linear_shape_ok(M, N, K, layout), "linear_i8_one_launch: bad shape M=%lld N=%d K=%d or layout %d", (long long)M, N, K, layout);
   const bool sparse = layout == SAMFAST_LAYOUT_SPARSE24;
   return linear_i8_small_covers(M, N, K, sparse) || linear_i8_band_covers(M, N, K, sparse);
 }

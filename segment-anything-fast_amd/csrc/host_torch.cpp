@@ -111,7 +111,7 @@ struct LinearCall {
 // bytes of workspace of a call whose output is its own
 int64_t workspace(const LinearCall& c, int layout) {
   const int N = static_cast<int>(c.N), K = static_cast<int>(c.K);
-  return p_linear_i8_one_launch(c.M, N, K, layout) ? 0 : p_linear_i8_workspace(c.M, N, K, layout);
+  return p_linear_i8_one_launch(c.M, N, K, layout) == 1 ? 0 : p_linear_i8_workspace(c.M, N, K, layout);
 }
 
 // linear(x, wq, layout, sw_bits, bias_bits or None): the whole int8 Linear on bf16 rows.

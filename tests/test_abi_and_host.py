@@ -748,3 +748,13 @@ def test_a_linear_over_a_handful_of_rows_into_those_rows_takes_a_workspace(M, K)
     assert lib.samfast_linear_i8_workspace(M, K, K, 0) >= M * K + 4 * M
     assert _linear_route(M, K, K, 0, K, 0, K) == "two"
     assert _linear_route(M, K, K, 0, 2 * K, K, 2 * K) == "one"
+
+
+@pytest.mark.parametrize("M,N,K,layout", [(0, 768, 768, 0), (-1, 768, 768, 0), (8, 0, 768, 1), (8, -8, 768, 2), (8, 768, 0, 0), (8, 768, -64, 2), (8, 768, 768, 3),
+                                          (8, 768, 768, -1), (4096, 768, 768, 7)])
+def test_questions_about_no_linear_are_refused(M, N, K, layout):
+    from samfast_amd import _lib
+    lib = _lib.load()
+    for name in ("samfast_linear_i8_workspace", "samfast_linear_i8_one_launch"):
+        assert getattr(lib, name)(M, N, K, layout) == -1, name
+        assert name[8:].encode() in lib.samfast_last_error()
