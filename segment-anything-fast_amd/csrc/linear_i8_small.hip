@@ -319,8 +319,9 @@ bool linear_i8_small_any_alignment(int64_t M, int K) { return M <= 8 || (M <= 16
 //   2:4   64 x 768 -> 768 7.1 / 4.6, 128 x 1024 -> 1024 7.8 / 6.1, 96 x 1280 -> 1280 7.9 / 7.3, 64 x 2048 -> 1024 8.1 / 6.8, 64 x 3072 -> 768 9.1 / 9.1;
 //         beyond: 256 x 1024 -> 1024 7.7 / 8.1, 128 x 1280 -> 1280 8.0 / 9.1, 48 x 4096 -> 1024 10.2 / 10.0 (rows at or past M cost less: 4 x 5120 -> 1280 8.5 / 7.7), 96 x 2048 -> 1024 8.0 / 8.5
 // A call, launches included (7 x 256 -> 2048 6.7 us a call, two launches 8.7): 64 x 1024 -> 1024 9.8 / 6.4, 2:4 64 x 1024 -> 1024 9.8 / 6.4.
+// (A forced tile of the band kernel turns this form off.)
 static int small_shape(int64_t M, int N, int K, bool sparse) {
-  if (knob_or(KNOB_LINEAR_SMALL, 1) <= 0 || K % 64 != 0 || N % 8 != 0 || N <= 0 || K <= 0 || K > 5120 || M <= 0 || M > 4096) return 0;
+  if (knob_or(KNOB_LINEAR_SMALL, 1) <= 0 || knob_or(KNOB_LINEAR_BAND, 1) > 1 || K % 64 != 0 || N % 8 != 0 || N <= 0 || K <= 0 || K > 5120 || M <= 0 || M > 4096) return 0;
   const int64_t eights = (M + 7) / 8;
   if (sparse) {
     const int64_t tiles = eights * ((N + 31) / 32);

@@ -36,8 +36,8 @@ enum Knob {
   KNOB_GEMM_SPLITK,       // SAMFAST_GEMM_SPLITK: 0 off, 1 where it pays (launches that leave the GPU half empty; 2:4: one tile per CU), 2 wherever built
   KNOB_GEMM_ONCE,         // SAMFAST_GEMM_ONCE: 0 = off, 1 where it pays, rows * 16 + columns / 32 = that tile of the one-tile-per-CU kernel
   KNOB_GEMM_STRIP,        // SAMFAST_GEMM_STRIP: 0 = off, 1 where it pays, 2 = wherever built (gemm_i8_strip.hip)
-  KNOB_LINEAR_SMALL,      // SAMFAST_GEMM_LINEAR_SMALL: 0 = whole Linears (2:4 ones too) over few rows as two launches as well
-  KNOB_LINEAR_BAND,       // SAMFAST_GEMM_LINEAR_BAND: whole Linears over a band of rows in one launch, 0 off, 1 where it pays, row tiles * 8 + column tiles (of 16) of a wavefront: that tile
+  KNOB_LINEAR_SMALL,      // SAMFAST_GEMM_LINEAR_SMALL: 0 = whole Linears (2:4 ones too) as two launches throughout: over few rows and over a band of rows
+  KNOB_LINEAR_BAND,       // SAMFAST_GEMM_LINEAR_BAND: whole Linears over a band of rows in one launch, 0 off, 1 where it pays, row tiles * 8 + column tiles (of 16) of a wavefront: that tile, and no Linear by the few-row form
   KNOB_GEMM_SKINNY,       // SAMFAST_GEMM_SKINNY: 0 = products over few rows through the tiled kernels
   KNOB_ATTN_WAVES,        // SAMFAST_ATTN_WAVES: 4 / 8 wavefronts per global-attention workgroup
   KNOB_ATTN_SPLIT,        // SAMFAST_ATTN_SPLIT: global attention with the keys split between two wavefronts (other bits), 0 = never, 1 = head_dim 64, 2 = always

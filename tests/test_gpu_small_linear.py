@@ -276,7 +276,8 @@ def test_a_band_of_rows_in_one_launch_agrees_with_two(M, N, K):
         if M < rows or N < cols:
             continue
         with _lib.knobs(SAMFAST_GEMM_LINEAR_BAND=tile):
-            if tile > 1:
+            if tile > 1:  # this tile: the few-row form is off
+                assert lib.samfast_linear_i8_one_launch(8, 768, 768, 0) == 0
                 assert lib.samfast_linear_i8_one_launch(M, N, K, 0) == 1
             assert torch.equal(lin(x).view(torch.int16), two.view(torch.int16)), tile
             if lib.samfast_linear_i8_one_launch(M, N, K, 1):
@@ -309,9 +310,44 @@ def test_a_band_of_rows_with_sparse_weights(M, N, K):
         if tile > 1 and (M < 16 * (tile // 8) or N < 128 * (tile % 8)):
             continue
         with _lib.knobs(SAMFAST_GEMM_LINEAR_BAND=tile):
-            if tile > 1:
+            if tile > 1:  # this tile: the few-row form is off
+                assert _lib.load().samfast_linear_i8_one_launch(4, 768, 768, 2) == 0
                 assert _lib.load().samfast_linear_i8_one_launch(M, N, K, 2) == 1
             assert torch.equal(lin(x).view(torch.int16), two.view(torch.int16)), tile
+
+
+@pytest.mark.parametrize("layout", [0, 1, 2])
+@pytest.mark.parametrize("M,N,K", [
+    # tiles of 32 x 384, 64 x 384 and the wide one, on rows that are shorter than a lane's chunks: two k steps, three, odd counts
+    (512, 1024, 256), (600, 1000, 640), (1500, 2000, 384), (700, 512, 512), (3000, 1280, 896), (4900, 1536, 256), (5000, 2304, 384), (1100, 4096, 896),
+    (500, 1288, 1152), (1900, 2600, 1152),
+])
+def test_short_rows_by_the_bands_rule(M, N, K, layout):
+    """Calls that the rule gives to the band kernel (not to the few-row form), whose rows do not fill what its lanes hold."""
+    from samfast_amd import Int8DynamicLinear, Int8Sparse24Linear, _lib, ops
+    print(f"case band rule M={M} N={N} K={K} layout={layout}", flush=True)
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    assert lib.samfast_linear_i8_one_launch(M, N, K, layout) == 1
+    with _lib.knobs(SAMFAST_GEMM_LINEAR_BAND=0):
+        assert lib.samfast_linear_i8_one_launch(M, N, K, layout) == 0
+    x, w, b = linear_inputs(M, K, N, seed=M + N + K)
+    x[M // 2] = 0
+    x[M - 1, K - 1] = float("nan")
+    lin = torch.nn.Linear(K, N, dtype=torch.bfloat16)
+    with torch.no_grad():
+        lin.weight.copy_(w)
+        lin.bias.copy_(b)
+    lin, x = (Int8Sparse24Linear if layout == 2 else Int8DynamicLinear).from_float(lin.cuda()), x.cuda()
+    if layout == 1:
+        wk, one = ops.to_kb64(lin.wq), torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+        assert lib.samfast_linear_i8(x.data_ptr(), K, wk.data_ptr(), lin.sw.data_ptr(), lin.bias_f32.data_ptr(), one.data_ptr(), N, None,
+                                     M, N, K, _lib.SAMFAST_BF16, layout, stream) == 0
+    else:
+        one = lin(x)
+    with _lib.knobs(SAMFAST_GEMM_LINEAR_SMALL=0):
+        two = lin(x)
+    assert torch.isnan(two[M - 1]).all()
+    assert torch.equal(one.view(torch.int16), two.view(torch.int16))
 
 
 def test_a_linear_into_its_own_rows():
