@@ -378,3 +378,50 @@ def test_a_linear_over_a_handful_of_rows_into_those_rows(M, K):
     assert lib.samfast_linear_i8(x.data_ptr(), K, lin.wq.data_ptr(), lin.sw.data_ptr(), lin.bias_f32.data_ptr(), x.data_ptr(), K,
                                  work.data_ptr(), M, K, K, _lib.SAMFAST_BF16, 0, stream) == 0
     assert torch.equal(x, want)
+
+
+def _into(lin, layout, x, y, work):
+    """The C call on rows of x and y that may lie apart, in either layout of the weights or 2:4."""
+    from samfast_amd import _lib, ops
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    (M, K), N = x.shape, y.shape[1]
+    tail = (lin.sw.data_ptr(), lin.bias_f32.data_ptr(), y.data_ptr(), y.stride(0), work, M, N, K, _lib.SAMFAST_BF16)
+    if layout == 2:
+        return lib.samfast_linear_i8_sparse24(x.data_ptr(), x.stride(0), lin.wc.data_ptr(), lin.widx.data_ptr(), *tail, stream)
+    w = ops.to_kb64(lin.wq) if layout == 1 else lin.wq
+    return lib.samfast_linear_i8(x.data_ptr(), x.stride(0), w.data_ptr(), *tail, layout, stream)
+
+
+@pytest.mark.parametrize("layout", [0, 1, 2])
+@pytest.mark.parametrize("M,N,K,form", [(63, 488, 512, "few"), (57, 520, 1280, "few"), (600, 1000, 640, "band"), (3001, 1288, 768, "band"), (1990, 3840, 1152, "band")])
+def test_rows_of_one_launch_further_apart(M, N, K, form, layout):
+    """x and y as column ranges of one buffer, without a workspace: the bits of contiguous rows, and nothing beside y is written.
+    Then y over x, with a workspace: the same."""
+    from samfast_amd import Int8Sparse24Linear, _lib
+    print(f"case strides {form} M={M} N={N} K={K} layout={layout}", flush=True)
+    lib = _lib.load()
+    assert lib.samfast_linear_i8_one_launch(M, N, K, layout) == 1
+    with _lib.knobs(SAMFAST_GEMM_LINEAR_BAND=0):
+        assert lib.samfast_linear_i8_one_launch(M, N, K, layout) == (form == "few")
+    lin = _linear(N, K, M)
+    if layout == 2:
+        lin = Int8Sparse24Linear.from_int8(lin.wq, lin.sw, lin.bias_f32)
+    x = torch.randn((M, K), device="cuda").to(torch.bfloat16)
+    want = lin(x)
+    buf = torch.full((M, 8 + K + 16 + N + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+    for x_at, y_at in ((8, 8 + K + 16), (8 + N + 16, 8)):
+        buf.fill_(7.0)
+        buf[:, x_at:x_at + K] = x
+        expected = buf.clone()
+        expected[:, y_at:y_at + N] = want
+        assert _into(lin, layout, buf[:, x_at:x_at + K], buf[:, y_at:y_at + N], None) == 0
+        assert torch.equal(buf, expected)
+    work = torch.empty(lib.samfast_linear_i8_workspace(M, N, K, layout), dtype=torch.int8, device="cuda")
+    for shift in (0, 8):  # the same columns, and columns that overlap
+        buf.fill_(7.0)
+        buf[:, 8:8 + K] = x
+        expected = buf.clone()
+        expected[:, 8 + shift:8 + shift + N] = want
+        assert _into(lin, layout, buf[:, 8:8 + K], buf[:, 8 + shift:8 + shift + N], None) == -1  # refused without it
+        assert _into(lin, layout, buf[:, 8:8 + K], buf[:, 8 + shift:8 + shift + N], work.data_ptr()) == 0
+        assert torch.equal(buf, expected)
