@@ -29,6 +29,13 @@ extern "C" {
 int samfast_bench_set_knob(const char* name, int value, int unset);
 
 /*
+ * Channels of the tile (256 or 320) in which samfast_gemm_i8_sparse24_fused forms this output by turns, 0 where another
+ * kernel does: the dispatch's rule, without a launch, for rows of the output and the residual `row_stride` elements
+ * apart that start on a cache line.  SAMFAST_E_INVALID for a bad shape.
+ */
+int samfast_bench_sparse24_turns(int64_t M, int N, int K, int epilogue, int64_t row_stride);
+
+/*
  * Measurement aid, no counterpart in the reference: one launch of a kernel that does nothing
  * but matrix instructions on operands held in registers (no global loads, no LDS, no barriers)
  * - the rate a GEMM or attention kernel built from the same instruction can approach at best

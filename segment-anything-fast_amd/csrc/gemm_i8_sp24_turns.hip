@@ -16,6 +16,7 @@
 // Inside the ViT-H encoder, both Linears of the MLP 2:4, 32 images 115.7 -> 111.2 ms, 16 58.6 -> 55.5, one 5.52 -> 5.22.
 #include "gemm_i8_sparse24_shared.hpp"
 #include "gemm_pingpong.hpp"
+#include "samfast_bench.h"
 
 // every fp32 step below is rounded on its own
 #pragma clang fp contract(off)
@@ -405,6 +406,8 @@ static STChoice st_choose(const SparseArgs& a) {
   return best;
 }
 
+static bool whole_lines(const void* p, int64_t ld) { return reinterpret_cast<uintptr_t>(p) % 128 == 0 && ld % 64 == 0; }
+
 bool gemm_i8_sp24_turns_covers(int epi, const SparseArgs& a) {
   const int mode = knob_or(KNOB_SPARSE_TURNS, 1);
   if (mode <= 0 || (epi != SEPI_SCALE_BIAS && epi != SEPI_RESIDUAL)) return false;
@@ -412,16 +415,38 @@ bool gemm_i8_sp24_turns_covers(int epi, const SparseArgs& a) {
   if (a.K % 128 != 0 || a.K < 640 || a.ldo >= (1ll << 22) || (epi == SEPI_RESIDUAL && a.ld_res >= (1ll << 22))) return false;
   const STChoice c = st_choose(a);
   if (c.tn == 0 || mode >= 8) return c.tn != 0;
-  // The lines, by `used` (us, the other kernels / this one, K-block major, random codes):
-  //   plain, 0.85: 0.87 (13406 x 1024 -> 4096, 320 channels, three rounds) 59.6 / 57.4, 0.88 (8633 x 1280 -> 5120) 55.4 / 51.6, 0.94 (4826 x 1024 -> 4096)
-  //     26.6 / 23.2, 1.0 (4096 x 1280 -> 5120) 27.8 / 24.6, (65536 x 1280 -> 5120) 358 / 302; but 0.84 in three rounds (17277 x 1024 -> 3072) 55.9 /
-  //     57.0; 320 channels within two rounds 0.8: 0.80 (7319 x 768 -> 2304) 23.0 / 19.7, 0.83 (8525 x 1024 -> 4096) 42.6 / 37.1, but 0.75 (4096 x 768
-  //     -> 3072) 14.5 / 15.9; loops shorter than 1024 0.91: 0.92 (40166 x 768 -> 3072) 101.6 / 97.1, 0.92 (60082 x 768 -> 2304) 128 / 107,
-  //     but 0.9 (24576 x 768 -> 3072) 60.7 / 62.1
-  //   residual, 320 channels 0.8: 0.83 (40960 x 5120 -> 1280) 198 / 184, 1.0 (16384) 77.4 / 63.8; 256 channels from three rounds on 0.85: 0.88 (57344 x
-  //     3072 -> 768) 118.7 / 110.8, 1.0 (49152 x 4096 -> 1024) 154 / 142; but 0.83 (40960 x 4096 -> 1024) 128 / 132, two rounds (32768 x 4096 -> 1024) 91.4 / 91.2
-  if (epi == SEPI_RESIDUAL) return c.tn == 10 ? c.used >= 0.8 : c.rounds >= 3 && c.used >= 0.85;
-  return c.used >= (c.tn == 10 && c.rounds <= 2 ? 0.8 : a.K >= 1024 ? 0.85 : 0.91);
+  // The lines (us, the 128-token kernel / this one, Gaussian codes, K-block major; 2700 products of 640 to 5120 by 768 to 8192, half
+  // of them drawn at random, stand behind them).
+  // Rows that are whole cache lines: eight lanes hold 128 bytes of a row, and where its lines lie elsewhere every store, and the residual's
+  // loads, are two of them in part.  Streamed ones 32288 x 640 -> 4904 112 / 252, else 8012 x 1024 -> 4904 39.8 / 51.2, 38665 x 640 -> 1992 63.2 / 68.9,
+  // with the residual 20496 x 640 -> 5096 122 / 177, 47794 x 768 -> 1992 120 / 163; nothing at the longest loops (24143 x 4096 -> 1992 122.0 / 122.0).
+  if (!whole_lines(a.out, a.ldo) || (epi == SEPI_RESIDUAL && !whole_lines(a.residual, a.ld_res))) return false;
+  if (epi == SEPI_RESIDUAL) {
+    // The residual's loads lengthen every tile's end, in which nothing is multiplied, so that loops have to be the longer the more
+    // ends there are, and the column tiles few:
+    //   256 channels, from three rounds on, 0.85 of them used: up to 1280 columns and from 2560 on 131072 x 4096 -> 1024 411 / 384, 65536 x 3072 -> 1024
+    //     173 / 164; but 57344 x 2048 -> 768 89.5 / 89.3, 40960 x 3072 -> 3072 283 / 289
+    //   320, 0.8 used: one round from 1024 on or up to 1280 columns 8192 x 1024 -> 2304 28.0 / 26.9, 13632 x 896 -> 1280 26.5 / 24.6; but 11654 x 640 -> 1536 24.0 / 24.7.
+    //     Two rounds, or up to 1280 columns: from 2048 on 10317 x 2048 -> 3840 70.0 / 68.5, 65536 x 2560 -> 1280 187 / 173, 40960 x 5120 -> 1280 201 / 193; but
+    //     16338 x 1280 -> 2304 51.2 / 53.3, 69627 x 640 -> 1280 109 / 119.  Others from nine rounds and 3072 on: 40504 x 4096 -> 5120 561 / 531; but five
+    //     rounds 40960 x 2560 -> 2560 213 / 216, 16943 x 1536 -> 8192 194 / 212
+    const bool narrow = a.N <= 1280;
+    if (c.tn == 8) return c.rounds >= 3 && c.used >= 0.85 && narrow && a.K >= 2560;
+    if (c.used < 0.8) return false;
+    if (c.rounds == 1) return narrow || a.K >= 1024;
+    return narrow || c.rounds == 2 ? a.K >= 2048 : c.rounds >= 9 && a.K >= 3072;
+  }
+  // Outputs that the 128-token kernel's tiles hold in one round, two of them on a CU, are its own: 4096 x 1024 -> 4096 (512 tiles) 18.5 / 19.7, 16384 x
+  // 1280 -> 1024 20.8 / 22.1, 4096 x 640 -> 3840 13.9 / 15.5; but 528 (4200 x 1024 -> 4096) 24.6 / 21.2.
+  if (((int64_t)a.M + 127) / 128 * ((a.N + 255) / 256) <= 512) return false;
+  // By `used`:
+  //   256 channels 0.92, on loops beyond 1536 0.95: 0.98 (36149 x 768 -> 4096) 120 / 117, 0.94 (28672 x 896 -> 3840) 95.0 / 94.4, 1.0 (16384 x 2560 -> 3072) 86.9 / 86.9;
+  //     but 0.9 (27377 x 768 -> 3840) 85.2 / 86.2, 0.94 (16453 x 2560 -> 3840) 111 / 113
+  //   320 0.88: 0.89 (14612 x 3072 -> 5120) 144 / 139, 1.0 (65536 x 1280 -> 5120) 358 / 302; but 0.86 (23968 x 1280 -> 3840) 99.3 / 101.3.  Within two rounds
+  //     0.8: 0.83 (4261 x 768 -> 4096) 21.8 / 19.1, 0.84 (11496 x 5120 -> 3072) 119 / 106, but 0.75 (4096 x 768 -> 3072) 14.5 / 15.9.  Beyond them on loops
+  //     shorter than 1024 0.91: 0.92 (30232 x 640 -> 5120) 116 / 108, but 0.9 (24576 x 768 -> 3072) 60.7 / 62.1
+  if (c.tn == 8) return c.used >= (a.K <= 1536 ? 0.92 : 0.95);
+  return c.used >= (c.rounds <= 2 ? 0.8 : a.K >= 1024 ? 0.88 : 0.91);
 }
 
 int gemm_i8_sp24_turns_launch(int epi, const SparseArgs& args, hipStream_t stream) {
@@ -441,3 +466,12 @@ int gemm_i8_sp24_turns_launch(int epi, const SparseArgs& args, hipStream_t strea
 }
 
 }  // namespace samfast
+
+extern "C" int samfast_bench_sparse24_turns(int64_t M, int N, int K, int epilogue, int64_t row_stride) {
+  using namespace samfast;
+  SF_REQUIRE(M > 0 && M < (1ll << 31) - 256 && N > 0 && K > 0 && row_stride >= N, "bench_sparse24_turns: bad shape M=%lld N=%d K=%d", (long long)M, N, K);
+  SparseArgs a = {};
+  a.M = (int)M; a.N = N; a.K = K; a.ldo = a.ld_res = row_stride;
+  const int epi = epilogue == SAMFAST_EPILOGUE_NONE ? SEPI_SCALE_BIAS : epilogue == SAMFAST_EPILOGUE_RESIDUAL ? SEPI_RESIDUAL : SEPI_GELU;
+  return gemm_i8_sp24_turns_covers(epi, a) ? 32 * st_choose(a).tn : 0;
+}

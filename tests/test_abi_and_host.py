@@ -758,3 +758,25 @@ def test_questions_about_no_linear_are_refused(M, N, K, layout):
     for name in ("samfast_linear_i8_workspace", "samfast_linear_i8_one_launch"):
         assert getattr(lib, name)(M, N, K, layout) == -1, name
         assert name[8:].encode() in lib.samfast_last_error()
+
+
+def test_the_sparse_products_lines():
+    """Both sides of each line between the 128-token kernel and the tiles by turns: (M, N, K, epilogue, channels of the tile)."""
+    from samfast_amd import _lib
+    lib = _lib.load()
+    none, gelu, residual = _lib.EPILOGUE_NONE, _lib.EPILOGUE_GELU, _lib.EPILOGUE_RESIDUAL
+    turns = lambda M, N, K, epilogue, stride=None: lib.samfast_bench_sparse24_turns(M, N, K, epilogue, stride or N)
+    for *call, channels in ((4096, 4096, 1024, none, 0), (4200, 4096, 1024, none, 320), (16384, 1024, 1280, none, 0), (4096, 5120, 1280, none, 320),
+                            (36149, 4096, 768, none, 256), (27377, 3840, 768, none, 0), (16384, 3072, 2560, none, 256), (16453, 3840, 2560, none, 0),
+                            (14612, 5120, 3072, none, 320), (23968, 3840, 1280, none, 0), (4261, 4096, 768, none, 320), (4096, 3072, 768, none, 0),
+                            (30232, 5120, 640, none, 320), (4096, 5120, 512, none, 0), (65536, 5120, 1280, none, 320), (65536, 5120, 1280, gelu, 0),
+                            (131072, 1024, 4096, residual, 256), (57344, 768, 2048, residual, 0), (40960, 3072, 3072, residual, 0),
+                            (8192, 2304, 1024, residual, 320), (11654, 1536, 640, residual, 0), (13632, 1280, 896, residual, 320),
+                            (10317, 3840, 2048, residual, 320), (16338, 2304, 1280, residual, 0), (40960, 1280, 5120, residual, 320),
+                            (69627, 1280, 640, residual, 0), (40504, 5120, 4096, residual, 320), (40960, 2560, 2560, residual, 0)):
+        assert turns(*call) == channels, call
+    # rows that are no whole cache lines, at sizes that are otherwise taken
+    for M, N, K, epilogue in ((32288, 4904, 640, none), (38665, 1992, 640, none), (20496, 5096, 640, residual), (24576, 1288, 5120, residual)):
+        assert turns(M, N, K, epilogue) == 0
+    assert turns(65536, 5120, 1280, none, 5128) == 0 and turns(65536, 5120, 1280, none, 5184) == 320
+    assert turns(0, 5120, 1280, none) == -1 and turns(65536, 5120, 1280, none, 5112) == -1
