@@ -29,10 +29,11 @@ extern "C" {
 int samfast_bench_set_knob(const char* name, int value, int unset);
 
 /*
- * Channels of the tile (256 or 320) in which samfast_gemm_i8_sparse24_fused forms this output by turns, 0 where another
- * kernel does: the dispatch's rule, without a launch, for rows of the output and the residual `row_stride` elements
- * apart that start on a cache line.  SAMFAST_E_INVALID for a bad shape.
+ * Columns of the tile (256 or 320) in which samfast_gemm_i8_fused or samfast_gemm_i8_sparse24_fused forms this output by
+ * turns, 0 where the rule leaves it to other kernels: no launch, for rows of the output and the residual
+ * `row_stride` elements apart that start on a cache line.  SAMFAST_E_INVALID for a bad shape.
  */
+int samfast_bench_gemm_i8_turns(int64_t M, int N, int K, int epilogue, int64_t row_stride);
 int samfast_bench_sparse24_turns(int64_t M, int N, int K, int epilogue, int64_t row_stride);
 
 /*

@@ -1,5 +1,6 @@
 // int8 GEMM for outputs of whole rounds of wide tiles: the turn-taking kernel of gemm_pingpong.hpp.
 #include "gemm_pingpong.hpp"
+#include "samfast_bench.h"
 
 namespace samfast {
 
@@ -24,7 +25,8 @@ static PPArgs pp_args(const GemmArgs& g) {
   return a;
 }
 
-static bool pays(int epi, int K, const PPChoice& c) {
+// lines: rows of the output and the residual are whole cache lines (residual products)
+static bool pays(int epi, int K, const PPChoice& c, bool lines) {
   // The lines, by the share of the CUs' time that makes output (us, the other members / this one, K-block major, random codes):
   //   plain, K >= 1280, 0.75: 0.78 (5000 rows -> 5120) 43.1 / 38.1, 0.94 (4096 -> 3840) 26.9 / 21.0, 1.0 (65536 -> 3840) 309 / 263,
   //     K = 5120, 1.0 (65536 -> 3840) 1126 / 994; but 0.59 (5000 -> 3840) 30.0 / 37.6
@@ -37,15 +39,18 @@ static bool pays(int epi, int K, const PPChoice& c) {
   //   residual, shorter loops, 0.85: 0.94 (20480 x 768 -> 768) 22.4 / 19.8, two rounds (40960 x 768 -> 768) 41.3 / 34.4, 0.88 (28672 x 1024 -> 1024) 43.9 / 38.5, 1.0
   //     (20480 x 1024 -> 1024, 320 rows) 31.9 / 28.4, 0.88 in five rounds (57344 x 1280 -> 1280) 124.2 / 117.2; but 0.75 (24576 x 1024 -> 1024) 35.7 / 37.5, 0.83
   //     (32768 x 1280 -> 1280) 63.2 / 66.3; from K = 1280 on 0.77 in up to two rounds: 0.78 (20480 -> 1280) 48.5 / 41.5
+  //     Rows that are no whole lines, whose segments each touch two, only within two rounds: 7556 x 1024 -> 1992 31.4 / 28.3, 16384 x 640 -> 1992 47.4 / 44.6; but
+  //     four 28672 x 640 -> 1992 72.4 / 78.1, five 14563 x 640 -> 4904 102 / 114, thirteen 40960 x 1024 -> 4904 309 / 321 (28672 x 1280 -> 1992 110 / 101)
   if (epi != EPI_RESIDUAL_BF16) return c.used >= (K >= 1280 ? 0.75 : 0.8);
   if (K >= 2048) return c.used >= (c.rounds == 1 ? 0.55 : 0.7);
+  if (K < 1280 && c.rounds > 2 && !lines) return false;
   return c.used >= (K >= 1280 && c.rounds <= 2 ? 0.77 : 0.85);
 }
 
 bool gemm_i8_pingpong_reads_rows(int64_t M, int N, int K) {
   if (K % 128 != 0 || K < 640) return false;  // (no knob: a workspace sized by this answer must fit the call that follows)
   const PPChoice c = pp_choose(M, N, K / 128, false);
-  return c.tn != 0 && pays(EPI_SCALE_BIAS_BF16, K, c);
+  return c.tn != 0 && pays(EPI_SCALE_BIAS_BF16, K, c, true);
 }
 
 bool gemm_i8_pingpong_covers(int epi, const GemmArgs& g) {
@@ -55,7 +60,8 @@ bool gemm_i8_pingpong_covers(int epi, const GemmArgs& g) {
   const PPChoice c = pp_choose(g.M, g.N, g.K / 128, epi == EPI_RESIDUAL_BF16);
   if (c.tn == 0) return false;
   if (mode >= 2) return true;
-  return pays(epi, g.K, c);
+  const auto whole_lines = [](const void* p, int64_t ld) { return reinterpret_cast<uintptr_t>(p) % 128 == 0 && ld % 64 == 0; };
+  return pays(epi, g.K, c, whole_lines(g.out, g.ldo) && whole_lines(g.residual, g.ld_res));
 }
 
 int gemm_i8_pingpong_launch(int epi, const GemmArgs& g, hipStream_t stream) {
@@ -80,3 +86,12 @@ int gemm_i8_pingpong_launch(int epi, const GemmArgs& g, hipStream_t stream) {
 }
 
 }  // namespace samfast
+
+extern "C" int samfast_bench_gemm_i8_turns(int64_t M, int N, int K, int epilogue, int64_t row_stride) {
+  using namespace samfast;
+  SF_REQUIRE(M > 0 && M < (1ll << 31) - 256 && N > 0 && K > 0 && row_stride >= N, "bench_gemm_i8_turns: bad shape M=%lld N=%d K=%d", (long long)M, N, K);
+  GemmArgs g = {};
+  g.M = (int)M; g.N = N; g.K = K; g.ldo = g.ld_res = row_stride;
+  const int epi = epilogue == SAMFAST_EPILOGUE_NONE ? EPI_SCALE_BIAS_BF16 : epilogue == SAMFAST_EPILOGUE_RESIDUAL ? EPI_RESIDUAL_BF16 : EPI_GELU_BF16;
+  return gemm_i8_pingpong_covers(epi, g) ? 32 * pp_choose(M, N, K / 128, epi == EPI_RESIDUAL_BF16).tn : 0;
+}

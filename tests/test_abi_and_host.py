@@ -780,3 +780,16 @@ def test_the_sparse_products_lines():
         assert turns(M, N, K, epilogue) == 0
     assert turns(65536, 5120, 1280, none, 5128) == 0 and turns(65536, 5120, 1280, none, 5184) == 320
     assert turns(0, 5120, 1280, none) == -1 and turns(65536, 5120, 1280, none, 5112) == -1
+
+
+def test_the_dense_residual_products_lines_where_rows_are_no_whole_lines():
+    """Loops under 1280 beyond two rounds are left to the smaller tiles there, others by turns as on whole lines: (M, N, K, columns)."""
+    from samfast_amd import _lib
+    turns = lambda M, N, K, epilogue, stride=None: _lib.load().samfast_bench_gemm_i8_turns(M, N, K, epilogue, stride or N)
+    residual = _lib.EPILOGUE_RESIDUAL
+    for *call, columns in ((28672, 1992, 640, 0), (14563, 4904, 640, 0), (40960, 4904, 1024, 0), (16384, 1992, 640, 256), (7556, 1992, 1024, 256),
+                           (28672, 1992, 1280, 256)):
+        assert turns(*call, residual) == columns, call
+    assert turns(28672, 1992, 640, residual, 2048) == 256 and turns(28672, 1024, 1024, residual) == 256  # whole lines
+    assert turns(65536, 3840, 1280, _lib.EPILOGUE_NONE) in (256, 320) and turns(65536, 3840, 1280, _lib.EPILOGUE_GELU) == 0
+    assert turns(-1, 3840, 1280, residual) == -1
