@@ -304,9 +304,25 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
 // them on (us, two launches / one: 1024 x 1280 -> 3840, 160 tiles, 14.1 / 14.8, 1200 x 1280 -> 3840, 190, 17.2 / 15.2, 900 x 1024 -> 4096, 165, 13.0 / 12.5, a call 12.6 / 12.1), and
 // behind 1280 values the small-tile product's rows stay with it (300 x 1280 -> 1280 8.0 / 8.4, 400, beyond them, 11.9 / 9.0).
 // 2:4 weights: the two launches take longer (the quantiser is the same, the products are bound by what they load) and win nowhere below one round,
-// but for 64 x 640 tiles on the longest rows, level up to about 200 of them (1800 x 1280 -> 3840, 174, 18.3 / 18.5): us, two / one, 4096 x 768 -> 3072 20.5 / 16.2, 4096 x 768 -> 768 13.3 / 8.7, 1024 x 768 -> 3072 11.9 / 8.2, 1024 x 1024 -> 1024
-// 11.6 / 7.8, 512 x 1280 -> 5120 13.9 / 10.3, 200 x 1280 -> 1280 9.5 / 8.4, 700 x 1280 -> 5120 14.9 / 13.8, 2048 x 1280 -> 5120 (256 tiles) 22.7 / 19.3; 2048 x 1280 -> 3840 (192)
-// 18.8 / 19.0, a call 17.5 / 18.3.
+// but for the wide tiles below: us, two / one, 4096 x 768 -> 3072 20.5 / 16.2, 4096 x 768 -> 768 13.3 / 8.7, 1024 x 768 -> 3072 11.9 / 8.2, 1024 x 1024 -> 1024
+// 11.6 / 7.8, 512 x 1280 -> 5120 13.9 / 10.3, 700 x 1280 -> 5120 14.9 / 13.8, 2048 x 1280 -> 5120 (256 tiles) 22.7 / 19.3.  (On rows of 1152 and 1280 and up to 24
+// tiles of 32 x 384 the two are the shorter ones on the GPU by up to half a microsecond, and no shorter as calls: 48 x 1280 -> 3840 7.95 / 8.4, a call 8.75 / 8.5.)
+// Wide tiles (us, two / one).  A workgroup takes as long however few there are, so that they pay from 180 of 64 x 768 on: 200 x 1024 -> 32000 (168) 17.8 / 19.0, 481 x
+// 1024 -> 16384 (176) 1.06 times as long, 2:4 1024 x 1024 -> 8192 (176) 16.6 / 18.1; from 180 on nowhere longer.  The more rows, the longer the quantiser that is
+// saved: over more than 2048 at any number (2256 x 1024 -> 3072, 144, 0.96, 2:4 2980 x 512 -> 2048, 141, 0.92 times), over more than 1024 on rows up to 768 at any
+// number (2:4: 152), up to 1024 from 156 on (1497 x 1024 -> 4096, 144, 19.1 / 20.0; 1933 x 896 -> 3584, 155, 18.5 / 19.2), 2:4 not (1540 x 1024 -> 4096, 150, 16.8 / 17.5).
+// 64 x 640 over more than 1024 rows at any number, else from 205 on (351 x 1280 -> 16384, 156, 1.06 times; 229 x 1280 -> 32000, 200, 1.03 times); 2:4 from 212
+// on (492 x 1280 -> 16384, 208, 1.08 times), on rows up to 1152 sooner: over more than 2048 at any number, more than 1024 from 176 on (331 x 1152 -> 20680, 198, 15.7 / 17.2).
+static bool wide_pays(int64_t M, int K, bool sparse, int64_t tiles) {
+  if (tiles >= (K <= 1024 ? 180 : sparse ? 212 : 205)) return true;
+  if (sparse && K > 1152) return false;
+  if (M > 2048) return true;
+  if (M <= 1024) return false;
+  if (K <= 768) return !sparse || tiles >= 152;
+  if (K <= 1024) return !sparse && tiles >= 156;
+  return !sparse || tiles >= 176;
+}
+
 static int band_shape(int64_t M, int N, int K, bool sparse) {
   const int mode = knob_or(KNOB_LINEAR_BAND, 1);
   if (mode <= 0 || knob_or(KNOB_LINEAR_SMALL, 1) <= 0 || K % 128 != 0 || K < 256 || K > 1280 || N % 8 != 0 || M < 32 || N < 384 || M > (1 << 20) || (int64_t)N * K >= (1ll << 31)) return 0;
@@ -317,8 +333,7 @@ static int band_shape(int64_t M, int N, int K, bool sparse) {
   if (!sparse && K > 1024 && (M + 63) / 64 * ((N + 31) / 32) <= 256) return 0;
   if (fits(2, 3)) return 2 * 8 + 3;
   if (fits(4, 3)) return sparse || K <= 768 || tiles(4, 3) >= 176 ? 4 * 8 + 3 : 0;
-  if (sparse && K > 1152 && tiles(4, wide) < 208) return 0;
-  return fits(4, wide) ? 4 * 8 + wide : 0;
+  return fits(4, wide) && wide_pays(M, K, sparse, tiles(4, wide)) ? 4 * 8 + wide : 0;
 }
 
 bool linear_i8_band_covers(int64_t M, int N, int K, bool sparse) { return band_shape(M, N, K, sparse) != 0; }
