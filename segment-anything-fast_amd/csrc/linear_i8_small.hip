@@ -318,6 +318,8 @@ bool linear_i8_small_any_alignment(int64_t M, int K) { return M <= 8 || (M <= 16
 //         1024 -> 1024 8.0 / 9.3, 96 x 2048 -> 1024 7.3 / 8.9, 12 x 3072 -> 768 7.1 / 8.0, 256 x 1280 -> 1280 8.5 / 11.3
 //   2:4   64 x 768 -> 768 7.1 / 4.6, 128 x 1024 -> 1024 7.8 / 6.1, 96 x 1280 -> 1280 7.9 / 7.3, 64 x 2048 -> 1024 8.1 / 6.8, 64 x 3072 -> 768 9.1 / 9.1;
 //         beyond: 256 x 1024 -> 1024 7.7 / 8.1, 128 x 1280 -> 1280 8.0 / 9.1, 48 x 4096 -> 1024 10.2 / 10.0 (rows at or past M cost less: 4 x 5120 -> 1280 8.5 / 7.7), 96 x 2048 -> 1024 8.0 / 8.5
+//   Up to four short rows are quantised in no time, and two column tiles on more workgroups than CUs are ahead of four: 1 x 256 -> 8200 3.07 / 3.64 (two / four),
+//         4 x 128 -> 10240 3.2 / 3.5, 1 x 512 -> 16384 3.83 / 3.98, 1 x 1024 -> 8200 4.46 / 4.75; but 8 x 256 -> 10240 3.8 / 3.6, 4 x 768 -> 12288 4.8 / 4.5.
 // A call, launches included (7 x 256 -> 2048 6.7 us a call, two launches 8.7): 64 x 1024 -> 1024 9.8 / 6.4, 2:4 64 x 1024 -> 1024 9.8 / 6.4.
 // (A forced tile of the band kernel turns this form off.)
 static int small_shape(int64_t M, int N, int K, bool sparse) {
@@ -331,6 +333,7 @@ static int small_shape(int64_t M, int N, int K, bool sparse) {
   if (M <= 8 || K <= 2048) {
     if (tiles(1) <= 256) return 8 + 1;
     if (tiles(2) <= 256) return 8 + 2;
+    if (M <= 4 && (K <= 512 || tiles(2) <= 288)) return 8 + 2;
     if (K <= 1536 && tiles(4) <= 256) return 8 + 4;
     if (M <= 8) return 8 + 2;
   }

@@ -222,7 +222,7 @@ def test_one_tile_per_cu_agrees_with_the_small_tiles(bm, tn, M, N, K, epi, layou
 @pytest.mark.parametrize("sparse,M,N,K", [
     # workgroups of 8 rows and one, two, four column tiles, of 16 rows; the last calls of each, remainders of rows, columns and k steps
     (False, 63, 488, 64), (False, 64, 512, 512), (False, 65, 1000, 576), (False, 121, 1024, 1024), (False, 128, 1032, 1088), (False, 250, 1016, 1536),
-    (False, 79, 760, 2048), (False, 405, 632, 704), (False, 9, 8200, 1600), (False, 31, 13000, 768),
+    (False, 79, 760, 2048), (False, 405, 632, 704), (False, 9, 8200, 1600), (False, 31, 13000, 768), (False, 4, 8200, 512), (False, 1, 9000, 1088), (False, 5, 8200, 256),
     (True, 1, 8, 256), (True, 63, 1000, 512), (True, 128, 1536, 1024), (True, 77, 1632, 1152), (True, 57, 1016, 2048), (True, 81, 712, 3072), (True, 4, 1288, 5120),
 ])
 def test_one_launch_agrees_with_two(sparse, M, N, K):
