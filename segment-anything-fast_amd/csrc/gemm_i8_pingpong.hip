@@ -25,6 +25,8 @@ static PPArgs pp_args(const GemmArgs& g) {
   return a;
 }
 
+static bool whole_lines(const void* p, int64_t ld) { return reinterpret_cast<uintptr_t>(p) % 128 == 0 && ld % 64 == 0; }
+
 // lines: rows of the output and the residual are whole cache lines (residual products)
 static bool pays(int epi, int K, const PPChoice& c, bool lines) {
   // The lines, by the share of the CUs' time that makes output (us, the other members / this one, K-block major, random codes):
@@ -60,7 +62,6 @@ bool gemm_i8_pingpong_covers(int epi, const GemmArgs& g) {
   const PPChoice c = pp_choose(g.M, g.N, g.K / 128, epi == EPI_RESIDUAL_BF16);
   if (c.tn == 0) return false;
   if (mode >= 2) return true;
-  const auto whole_lines = [](const void* p, int64_t ld) { return reinterpret_cast<uintptr_t>(p) % 128 == 0 && ld % 64 == 0; };
   return pays(epi, g.K, c, whole_lines(g.out, g.ldo) && whole_lines(g.residual, g.ld_res));
 }
 
@@ -71,8 +72,9 @@ int gemm_i8_pingpong_launch(int epi, const GemmArgs& g, hipStream_t stream) {
   a.group_m = 4;
   a.tiles_m = (a.M + 64 * c.tm - 1) / (64 * c.tm);
   a.tiles_n = (a.N + 32 * tn - 1) / (32 * tn);
-  // an output larger than the last-level cache that is read once (qkv, lin1) is streamed out
-  const bool nt = g.stream_out != 0;
+  // an output larger than the last-level cache that is read once (qkv, lin1) is streamed out; not where rows are no whole cache lines,
+  // whose two halves two stores bring (streamed / not, us: 31790 x 640 -> 4904 186 / 128, 55833 x 768 -> 4904 318 / 279, 40000 x 1280 -> 5096 299 / 280)
+  const bool nt = g.stream_out != 0 && whole_lines(g.out, g.ldo);
 #define SF_PP(E, TN, NT) hipLaunchKernelGGL((gemm_pingpong_kernel<PPInt8, E, TN, NT>), dim3(pp_grid(a)), dim3(512), 0, stream, a)
 #define SF_PP_PLAIN(TN) do { if (nt) SF_PP(PP_PLAIN, TN, true); else SF_PP(PP_PLAIN, TN, false); } while (0)
   if (epi == EPI_RESIDUAL_BF16 && c.tm == 5)

@@ -686,6 +686,8 @@ def test_quantiser_on_both_sides_of_the_cache(K, layout, gelu):
     (4096, 5120, 768, 0), (20480, 1024, 640, 2), (17000, 1288, 768, 2), (33000, 648, 768, 0),
     # (320 rows by 256 columns) ragged, lists of two tiles
     (20400, 1000, 640, 2), (40900, 1016, 768, 2),
+    # outputs beyond the last-level cache: streamed, and, of rows that are no whole cache lines, not
+    (26300, 5120, 640, 0), (27500, 4904, 640, 0),
 ])
 @pytest.mark.parametrize("layout", [0, 1])
 def test_gemm_by_turns_agrees(M, N, K, epi, layout):
