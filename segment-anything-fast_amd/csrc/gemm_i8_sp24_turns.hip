@@ -4,8 +4,8 @@
 // What bounds it is memory, not products: at 131072 x 1280 -> 5120 (600 us, 455 on zeros) 304 on zeros are the loop with its loads, most of the
 // rest 1.3 GB of output; without the products it takes the same time, without the loads 160 less (timings of patched copies that are not
 // kept, counters beside them).  So the choices are about bytes and about the units they pass:
-//   * 256 x 320 tiles: 58 KB of operands per 1280 cycles of products, 44.5 bytes per clock, for 72 in the 128-token kernel and 52 in
-//     256 x 256 (taken where 320 channels fit badly);
+//   * 256 x 320 tiles: 58368 bytes of operands per 1280 cycles of products, 45.6 a clock (46.4 with the padded piece of the index words), for 72
+//     in the 128-token kernel and 52 in 256 x 256 (taken where 320 channels fit badly);
 //   * the index words as 16-byte loads, behind the weights that they belong to: 4 bytes a lane, each cost as much as 16;
 //   * the output through LDS.  The sparse operand has to be the instruction's rows, so a lane ends with channels of one token and its
 //     neighbours have other tokens: stored from there, 16 bytes are an access of their own, 10000 of them per tile at one a cycle, twice
@@ -31,12 +31,11 @@ struct STTile {
   static constexpr int BM = 256, BN = 32 * TN, H = TN / 2;
   static constexpr int WUNITS = 2 * H, IUNITS = (2 * H + 3) / 4, UNITS = WUNITS + IUNITS;  // a turn's pieces of 1 KB: weights, indices
   static constexpr int TURN = UNITS * 1024;
-  static constexpr int STAGE = BM * 128 + 2 * TURN;
-  static constexpr int NST = 2;                        // k tiles held
+  static constexpr int STAGE = BM * 128 + 2 * TURN;   // a k tile, of which two are held
   static constexpr int SCALES = BM * 4 + 2 * BN * 4;
   static constexpr int NSTORES = 4 * H;
   static_assert(UNITS > 8 && UNITS <= 16, "one or two pieces for each wavefront");
-  static_assert(NST * STAGE + SCALES + 8 * 4096 + 16 <= 160 * 1024, "LDS of a CU");
+  static_assert(2 * STAGE + SCALES + 8 * 4096 + 16 <= 160 * 1024, "LDS of a CU");
   static constexpr int PAIRS = H / 2 * 2, UNITS_OUT = PAIRS + H % 2;
   // first channel of a half's pairs of fragment pairs, of its odd one
   static SF_DEVICE int first(int half) { return half * (TN == 10 ? 192 : 128); }
@@ -58,8 +57,8 @@ __global__ __launch_bounds__(512, 2) void gemm_i8_sp24_turns_kernel(SparseArgs a
   using P = STTile<TN>;
   constexpr bool RES = EPI == SEPI_RESIDUAL;
   constexpr int H = P::H;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[P::NST * P::STAGE + P::SCALES + 8 * 4096 + 16];
-  unsigned char* sc = lds + P::NST * P::STAGE;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * P::STAGE + P::SCALES + 8 * 4096 + 16];
+  unsigned char* sc = lds + 2 * P::STAGE;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -213,13 +212,12 @@ __global__ __launch_bounds__(512, 2) void gemm_i8_sp24_turns_kernel(SparseArgs a
   };
   auto arrive = [&](auto extra_n, bool extra) __attribute__((always_inline)) {
     constexpr int EXTRA = decltype(extra_n)::value;
-    constexpr int A = P::NST - 1;
     if (EXTRA > 0 && extra) {
-      if (two) pp_wait<8 * A + EXTRA>();
-      else pp_wait<6 * A + EXTRA>();
+      if (two) pp_wait<8 + EXTRA>();
+      else pp_wait<6 + EXTRA>();
     } else {
-      if (two) pp_wait<8 * A>();
-      else pp_wait<6 * A>();
+      if (two) pp_wait<8>();
+      else pp_wait<6>();
     }
   };
 
@@ -322,14 +320,12 @@ __global__ __launch_bounds__(512, 2) void gemm_i8_sp24_turns_kernel(SparseArgs a
   if (tid == 0) *reinterpret_cast<u32x4*>(sc + P::SCALES + 8 * 4096) = u32x4{0u, 0u, 0u, 0u};
 
   // ---- prologue: k tile 0, and of k tile 1 what the first turn of a k tile needs ---------------------------------
-#pragma unroll
-  for (int k = 0; k < P::NST; ++k) {
-    load_x(k * P::STAGE);
-    load_w(0, k * P::STAGE);
-    if (k + 1 == P::NST) break;
-    load_w(1, k * P::STAGE);
-    next_ktile();
-  }
+  load_x(0);
+  load_w(0, 0);
+  load_w(1, 0);
+  next_ktile();
+  load_x(P::STAGE);
+  load_w(0, P::STAGE);
   arrive(std::integral_constant<int, 0>{}, false);  // X and the first channels of k tile 0
   meet();
   if (wn == 1) meet();  // from here on the upper half is one turn behind
@@ -340,7 +336,7 @@ __global__ __launch_bounds__(512, 2) void gemm_i8_sp24_turns_kernel(SparseArgs a
     using T0 = std::integral_constant<int, 0>;
     using T1 = std::integral_constant<int, 1>;
     constexpr bool ZERO = decltype(first_of_tile)::value;
-    const int before = stage == 0 ? (P::NST - 1) * P::STAGE : stage - P::STAGE;
+    const int other = P::STAGE - stage;
     auto clear = [&](int turn) __attribute__((always_inline)) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -348,7 +344,7 @@ __global__ __launch_bounds__(512, 2) void gemm_i8_sp24_turns_kernel(SparseArgs a
         for (int j = 0; j < H; ++j) acc[i][turn * H + j] = i32x4{0, 0, 0, 0};
     };
     read(0, stage);
-    load_w(1, before);
+    load_w(1, other);
     next_ktile();
     if constexpr (ZERO) clear(0);
     arrive(extra_n, extra);
@@ -366,7 +362,7 @@ __global__ __launch_bounds__(512, 2) void gemm_i8_sp24_turns_kernel(SparseArgs a
     meet();
     multiply(T1{});
     meet();
-    stage = stage == (P::NST - 1) * P::STAGE ? 0 : stage + P::STAGE;
+    stage = other;
   };
   using Yes = std::true_type;
   using No = std::false_type;
