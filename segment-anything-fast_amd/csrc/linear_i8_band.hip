@@ -3,13 +3,13 @@
 //
 // Two launches of such a call are mostly starts and ends (4096 x 768 -> 3072: 5 and 15 us for 4.5 us of matrix pipe), the codes go through
 // memory between them, and the host pays for both.  Here every workgroup quantises its 32 or 64 rows itself - once per range of columns,
-// 2 to 14 times in all, which is why ranges are wide, at 64 rows 640 or 768 columns, and why sixteen lanes take a row (one reduction and
-// one division serve four rows) - keeps the codes in LDS for the whole of K and runs on W alone: a ring per wavefront in LDS, a
+// at the encoders' widths 2 to 14 times in all, at N = 32000 up to 84, which is why ranges are wide, at 64 rows 640 or 768 columns, and why sixteen
+// lanes take a row (one reduction and one division serve four rows) - keeps the codes in LDS for the whole of K and runs on W alone: a ring per wavefront in LDS, a
 // 16-column x 128-byte fragment at a time, whole lines of row-major weights as well as of K-block-major ones.  Wavefronts meet in front of the
 // products and never again: the row scales are in registers by then, so that one that is through converts and stores under the others'
 // products (with the scales fetched behind a barrier at the end 28900 cycles instead of 26500).  Bound (4096 x 768 -> 3072, cycles of a workgroup's
-// 26500): rows and first W through the load path 4000, codes 6000 of vector work, products 12700 (9200 of matrix pipe), output 3700; little of it
-// overlaps, 160 KB of LDS being one workgroup per CU.
+// 26500, by a cycle counter in probes that are not kept): rows and first W through the load path 4000, codes 6000 of vector work, products 12700 (9200
+// of matrix pipe), output 3700; little of it overlaps, 160 KB of LDS being one workgroup per CU.
 // us on the GPU, two launches / this one: 4096 x 768 -> 3072 21.9 / 18.3, 4096 x 768 -> 768 12.2 / 8.7, 2048 x 768 -> 3072 15.6 / 12.2, 16384 x 768 -> 768 26.9 / 19.5, 1024 x 1024
 // -> 3072 12.8 / 9.3, 512 x 1280 -> 5120 12.3 / 9.9.  Integer sums and the epilogue's arithmetic are those of the other forms: the same bits.
 #include "attn_relpos_shared.hpp"
@@ -307,15 +307,17 @@ __global__ __launch_bounds__(512, 2) void linear_i8_band_kernel(BandArgs a) {
 // but for the wide tiles below: us, two / one, 4096 x 768 -> 3072 20.5 / 16.2, 4096 x 768 -> 768 13.3 / 8.7, 1024 x 768 -> 3072 11.9 / 8.2, 1024 x 1024 -> 1024
 // 11.6 / 7.8, 512 x 1280 -> 5120 13.9 / 10.3, 700 x 1280 -> 5120 14.9 / 13.8, 2048 x 1280 -> 5120 (256 tiles) 22.7 / 19.3.  (On rows of 1152 and 1280 and up to 24
 // tiles of 32 x 384 the two are the shorter ones on the GPU by up to half a microsecond, and no shorter as calls: 48 x 1280 -> 3840 7.95 / 8.4, a call 8.75 / 8.5.)
-// Wide tiles (us, two / one).  A workgroup takes as long however few there are, so that they pay from 180 of 64 x 768 on: 200 x 1024 -> 32000 (168) 17.8 / 19.0, 481 x
-// 1024 -> 16384 (176) 1.06 times as long, 2:4 1024 x 1024 -> 8192 (176) 16.6 / 18.1; from 180 on nowhere longer.  The more rows, the longer the quantiser that is
+// Wide tiles (us, two / one).  A workgroup takes as long however few there are, so that they pay from 181 of 64 x 768 on: 200 x 1024 -> 32000 (168) 17.8 / 19.0, 481 x
+// 1024 -> 16384 (176) 1.06 times as long, 761 x 512 -> 10880 (180) 13.9 / 14.6, 2:4 1024 x 1024 -> 8192 (176) 16.6 / 18.1.  The more rows, the longer the quantiser that is
 // saved: over more than 2048 at any number (2256 x 1024 -> 3072, 144, 0.96, 2:4 2980 x 512 -> 2048, 141, 0.92 times), over more than 1024 on rows up to 768 at any
-// number (2:4: 152), up to 1024 from 156 on (1497 x 1024 -> 4096, 144, 19.1 / 20.0; 1933 x 896 -> 3584, 155, 18.5 / 19.2), 2:4 not (1540 x 1024 -> 4096, 150, 16.8 / 17.5).
+// number (2:4: 152), up to 1024 from 156 on (1497 x 1024 -> 4096, 144, 19.1 / 20.0; 1933 x 896 -> 3584, 155, 18.5 / 19.2), 2:4 not (1540 x 1024 -> 4096, 150, 16.8 / 17.5);
+// up to 3072 rows of 256 from 168 on (1451 x 256 -> 5120, 161, 11.3 / 11.9, 2616 x 256 -> 3072, 164, 11.8 / 12.3; 3490 x 256 -> 2048, 165, 0.98 times).
 // 64 x 640 over more than 1024 rows at any number, else from 205 on (351 x 1280 -> 16384, 156, 1.06 times; 229 x 1280 -> 32000, 200, 1.03 times); 2:4 from 212
 // on (492 x 1280 -> 16384, 208, 1.08 times), on rows up to 1152 sooner: over more than 2048 at any number, more than 1024 from 176 on (331 x 1152 -> 20680, 198, 15.7 / 17.2).
 static bool wide_pays(int64_t M, int K, bool sparse, int64_t tiles) {
-  if (tiles >= (K <= 1024 ? 180 : sparse ? 212 : 205)) return true;
+  if (tiles >= (K <= 1024 ? 181 : sparse ? 212 : 205)) return true;
   if (sparse && K > 1152) return false;
+  if (!sparse && K <= 256 && M <= 3072) return M > 1024 && tiles >= 168;
   if (M > 2048) return true;
   if (M <= 1024) return false;
   if (K <= 768) return !sparse || tiles >= 152;

@@ -799,9 +799,9 @@ def test_the_lines_of_a_linear_in_one_launch_on_wide_tiles():
     """Both sides of each line of the band's widest tiles: (M, N, K, layout, one launch)."""
     from samfast_amd import _lib
     one = _lib.load().samfast_linear_i8_one_launch
-    for *call, taken in ((200, 32000, 1024, 0, 0), (200, 32000, 1024, 2, 0), (64, 138240, 1024, 0, 1), (1024, 8192, 1024, 2, 0), (1100, 8192, 1024, 2, 1),
+    for *call, taken in ((200, 32000, 1024, 0, 0), (200, 32000, 1024, 2, 0), (64, 139008, 1024, 0, 1), (1024, 8192, 1024, 2, 0), (1100, 8192, 1024, 2, 1),
                          (2256, 3072, 1024, 0, 1), (2980, 2048, 512, 2, 1), (1497, 4096, 1024, 0, 0), (1650, 4096, 1024, 0, 1), (1540, 4096, 1024, 2, 0),
-                         (1486, 4016, 256, 0, 1), (1500, 5120, 768, 2, 1), (1300, 5120, 768, 2, 0), (351, 16384, 1280, 0, 0), (480, 16384, 1280, 0, 1),
+                         (761, 10880, 512, 0, 0), (1451, 5120, 256, 0, 0), (1651, 5120, 256, 0, 1), (3490, 2048, 256, 0, 1), (1500, 5120, 768, 2, 1), (1300, 5120, 768, 2, 0), (351, 16384, 1280, 0, 0), (480, 16384, 1280, 0, 1),
                          (1600, 3840, 1280, 0, 1), (492, 16384, 1280, 2, 0), (520, 16384, 1280, 2, 1), (331, 20680, 1152, 2, 0),
                          (1900, 3456, 1152, 2, 1), (4630, 1280, 1152, 2, 1), (4096, 3072, 768, 0, 1)):
         assert one(*call) == taken, call
