@@ -723,8 +723,10 @@ __global__ __launch_bounds__((WindowCfg<HD, TILES>::THREADS), 2) void attn_windo
     const u32x4 bh_op = bias_hv, bw_op = bias_wv;
 
     // Where whole items share the CUs with the cut ones of one round, half of a workgroup's wavefronts are let ahead, so that a SIMD's do not multiply
-    // and take exponentials in step (us, 25 x 12 x 64, 14 x 14: 17.0 / 16.4, 30 x 12 17.5 / 16.9; without cut ones nothing, 16 x 16 13.7 / 13.7, and with
-    // more rounds they are out of step by themselves: 100 x 12 41.1 / 43.4)
+    // and take exponentials in step: 257 to 384 items of 14 x 14.  us, all alike / so, inputs that a cache holds and ones that none does: the caller's factors
+    // 25 x 12 x 64 13.5 / 12.7 and 16.0 / 15.6, 30 x 12 x 80 16.4 / 16.0 and 18.6 / 18.1; with tables in an image of 12 heads of 64 channels 16.0 / 15.4 and 16.5 / 16.3, of
+    // 80 15.5 / 14.9 and 17.5 / 16.9 (0.95 to 0.99 throughout, ten counts of items, both types).  Without cut ones nothing, 16 x 16 13.7 / 13.7, and with more
+    // rounds they are out of step by themselves: 100 x 12 41.1 / 43.4.
     const bool ahead = a.whole == 256 && a.parts > 1 && wave_u < 4;  // uniform
     if (ahead) __builtin_amdgcn_s_setprio(1);
     // ---- online softmax over the key tiles: S^T tile, running max, P, O^T += V^T P^T --------
