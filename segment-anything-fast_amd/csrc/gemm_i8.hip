@@ -1269,7 +1269,7 @@ extern "C" int samfast_linear_i8(const void* x, int64_t ldx, const int8_t* wq, c
   SF_REQUIRE(layout == SAMFAST_LAYOUT_ROWMAJOR || layout == SAMFAST_LAYOUT_KB64, "linear_i8: unknown layout %d", layout);
   const bool small = M > 0 && linear_i8_small_covers(M, N, K, false), any_alignment = small && linear_i8_small_any_alignment(M, K);
   if (M > 0 && (small || linear_i8_band_covers(M, N, K, false)) && !rows_share_memory(x, ldx, y, ldy, M, N, K)) {
-    SF_REQUIRE(dtype == SAMFAST_BF16, "linear_i8: only bf16");
+    if (dtype != SAMFAST_BF16) SF_FAIL(SAMFAST_E_UNSUPPORTED, "linear_i8: only bf16");
     SF_REQUIRE(x && wq && sw && y && aligned16(x) && aligned16(wq) && aligned16(y) && (any_alignment || (aligned16(sw) && aligned16(bias))),
                "linear_i8: null or unaligned pointer");
     SF_REQUIRE(ldx >= K && ldx % 8 == 0 && ldy >= N && ldy % 8 == 0, "linear_i8: row strides must be multiples of 8, >= K and >= N");
@@ -1304,7 +1304,7 @@ extern "C" int samfast_linear_i8_sparse24(const void* x, int64_t ldx, const int8
   using namespace samfast;
   const bool small = M > 0 && linear_i8_small_covers(M, N, K, true);
   if (M > 0 && (small || linear_i8_band_covers(M, N, K, true)) && !rows_share_memory(x, ldx, y, ldy, M, N, K)) {
-    SF_REQUIRE(dtype == SAMFAST_BF16, "linear_i8_sparse24: only bf16");
+    if (dtype != SAMFAST_BF16) SF_FAIL(SAMFAST_E_UNSUPPORTED, "linear_i8_sparse24: only bf16");
     SF_REQUIRE(x && wc && widx && sw && y && aligned16(x) && aligned16(wc) && aligned16(widx) && aligned16(y) && aligned16(sw) && aligned16(bias),
                "linear_i8_sparse24: null or unaligned pointer");
     SF_REQUIRE(ldx >= K && ldx % 8 == 0 && ldy >= N && ldy % 8 == 0 && (int64_t)N * 32 < (1ll << 31),

@@ -708,10 +708,10 @@ def _linear_route(M, N, K, x_at, ldx, y_at, ldy, sparse=False):
     base = 1 << 40  # elements are 2 bytes; weights, scales and bias lie elsewhere
     weights = (base - (1 << 30),) + ((base - (1 << 29),) if sparse else ())
     args = (base + 2 * x_at, ldx) + weights + (base - (1 << 28), base - (1 << 27), base + 2 * y_at, ldy, None, M, N, K, _lib.SAMFAST_F16)
-    assert (lib.samfast_linear_i8_sparse24(*args, None) if sparse else lib.samfast_linear_i8(*args, 0, None)) == -1
+    code = lib.samfast_linear_i8_sparse24(*args, None) if sparse else lib.samfast_linear_i8(*args, 0, None)
     error = lib.samfast_last_error()
-    assert b"only bf16" in error or b"workspace must be" in error, error
-    return "one" if b"only bf16" in error else "two"
+    assert (code == -2 and b"only bf16" in error) or (code == -1 and b"workspace must be" in error), (code, error)
+    return "one" if code == -2 else "two"
 
 
 @pytest.mark.parametrize("sparse", [False, True])
@@ -805,3 +805,11 @@ def test_the_lines_of_a_linear_in_one_launch_on_wide_tiles():
                          (1600, 3840, 1280, 0, 1), (492, 16384, 1280, 2, 0), (520, 16384, 1280, 2, 1), (331, 20680, 1152, 2, 0),
                          (1900, 3456, 1152, 2, 1), (4630, 1280, 1152, 2, 1), (4096, 3072, 768, 0, 1)):
         assert one(*call) == taken, call
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 1024, 1024), (64, 1024, 1024), (4096, 3072, 768), (5000, 1280, 5120)])  # few rows, more, a band, two launches
+def test_a_linear_of_another_type_is_unsupported_in_every_form(M, N, K):
+    from samfast_amd import _lib
+    lib, p = _lib.load(), [1 << 40 + i for i in range(7)]  # (refused before anything is launched)
+    assert lib.samfast_linear_i8(p[0], K, p[1], p[2], p[3], p[4], N, p[5], M, N, K, _lib.SAMFAST_F16, 0, None) == -2
+    assert lib.samfast_linear_i8_sparse24(p[0], K, p[1], p[2], p[3], p[4], p[5], N, p[6], M, N, K, _lib.SAMFAST_F16, None) == -2
