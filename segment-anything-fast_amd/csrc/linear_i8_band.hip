@@ -8,9 +8,9 @@
 // 16-column x 128-byte fragment at a time, whole lines of row-major weights as well as of K-block-major ones.  Wavefronts meet in front of the
 // products and never again: the row scales are in registers by then, so that one that is through converts and stores under the others'
 // products (with the scales fetched behind a barrier at the end 28900 cycles instead of 26500).  Bound (4096 x 768 -> 3072, cycles of a workgroup's
-// 26500, by a cycle counter in probes that are not kept): rows and first W through the load path 4000, codes 6000 of vector work, products 12700 (9200
-// of matrix pipe), output 3700; little of it overlaps, 160 KB of LDS being one workgroup per CU.
-// us on the GPU, two launches / this one: 4096 x 768 -> 3072 21.9 / 18.3, 4096 x 768 -> 768 12.2 / 8.7, 2048 x 768 -> 3072 15.6 / 12.2, 16384 x 768 -> 768 26.9 / 19.5, 1024 x 1024
+// 26500, by a cycle counter in probes that are not kept, with four instructions per code; with one, quant_row.hpp, 0.7 us less): rows and first W through the load path
+// 4000, codes 6000 of vector work, products 12700 (9200 of matrix pipe), output 3700; little of it overlaps, 160 KB of LDS being one workgroup per CU.
+// us on the GPU, two launches / this one: 4096 x 768 -> 3072 21.9 / 17.6, 4096 x 768 -> 768 12.2 / 8.7, 2048 x 768 -> 3072 15.6 / 12.2, 16384 x 768 -> 768 26.9 / 19.5, 1024 x 1024
 // -> 3072 12.8 / 9.3, 512 x 1280 -> 5120 12.3 / 9.9.  Integer sums and the epilogue's arithmetic are those of the other forms: the same bits.
 #include "attn_relpos_shared.hpp"
 #include "gemm_i8_shared.hpp"

@@ -60,32 +60,35 @@ SF_DEVICE float wave_max_nonneg(float v) {
   });
 }
 
-// A row's scale and its reciprocal.
+// A row's scale and the factor that codes are made with: code = rint(v * factor), rounded once.
+// The code wanted is rint(fl(v / scale)) with the correctly rounded IEEE quotient.  Values and maximum are bf16, so the exact
+// 127 v / amax is a tie (k + 1/2) only at v = amax / 2, where it is 63.5, and, if 127 divides amax's significand (254), at ties of both parities for which
+// scale and 1 / scale are powers of two; elsewhere it stays 2^-16 of its size and more away from one, beyond what the roundings of scale, quotient and
+// factor (2^-24 each) move.  So any factor within a few units of 1 / scale gives the division's codes but for v = amax / 2, and there the
+// factor is moved by one unit to the side on which the division lies: its quotient is 63.5 or more (code 64) where m >= scale * (127 - 2^-18), m being
+// the maximum at its floor; the residual of m / scale is exact in one fused multiply-add.  All pairs of a bf16 row maximum and a bf16 value up to it
+// (5.3e8) give the division's code.  In a row with an infinity the factor is 0: the codes are 0, as the low byte of the division's NaN.
 struct QuantScale {
-  float scale, inv;
+  float scale, factor;
   SF_DEVICE explicit QuantScale(float amax) {
-    scale = fmaxf(amax, 1e-5f) / 127.0f;
-    inv = 1.0f / scale;
+    const float m = fmaxf(amax, 1e-5f);
+    scale = m / 127.0f;
+    const float inv = 1.0f / scale;
+    const bool up = fmaf(-scale, 127.0f, m) >= scale * -0x1p-18f;  // the division gives 64
+    const float over = fmaf(0.5f * m, inv, -63.5f);                // (exact in its sign)
+    factor = __uint_as_float(__float_as_uint(inv) + (up && over < 0.f ? 1u : !up && over >= 0.f ? -1u : 0u));
   }
 };
 
 // EPC (4 or 8) values -> EPC int8 codes packed in EPC bytes.
-// The code wanted is rint(fl(v / scale)) with the correctly rounded IEEE quotient.  q = fl(v * inv), then fl(q + fl(v - q * scale) * inv)
-// with fused multiply-adds has its last bit right wherever that can matter: all pairs of a bf16 row maximum and a bf16 value, and values
-// are never anything else here, give the code of the division.  Adding 1.5 * 2^23 rounds half to even and leaves the code in the low
-// byte (|v / scale| <= 127 (1 + 2^-23)).  In a row with an infinity every quotient comes out NaN, whose low byte is 0: the codes
-// the division gives there.  Four instructions per value and no branch.
-// (Two products bracketing the quotient, and the division in chunks where they round apart, was one instruction fewer per value,
-// but a branch per chunk, and its other side ran often enough: 254 / 448 / 1764 vector instructions per row of 1280 plain / 1280 with LayerNorm /
-// 5120 with GELU, 188 / 382 / 1593 now.)
+// Adding 1.5 * 2^23 in the same fused multiply-add rounds the exact product half to even and leaves the code in the low
+// byte (|v * factor| <= 127 (1 + 2^-22)).  One instruction per value; with the quotient itself made exact (q = v * inv, then q + (v - q * scale) *
+// inv, then the addition: four) 188 / 341 / 1593 vector instructions per row of 1280 plain / 1280 with LayerNorm / 5120 with GELU.
 template <int EPC>
 SF_DEVICE void quantize_chunk(const float (&v)[EPC], const QuantScale& s, unsigned int (&out)[EPC / 4]) {
   unsigned int m[EPC];
 #pragma unroll
-  for (int e = 0; e < EPC; ++e) {
-    const float q = v[e] * s.inv;
-    m[e] = __float_as_uint(fmaf(fmaf(-q, s.scale, v[e]), s.inv, q) + 12582912.0f);
-  }
+  for (int e = 0; e < EPC; ++e) m[e] = __float_as_uint(fmaf(v[e], s.factor, 12582912.0f));
 #pragma unroll
   for (int g = 0; g < EPC / 4; ++g) {
     // byte 0 of each of four words -> one word (v_perm_b32: selector bytes pick from {hi, lo})

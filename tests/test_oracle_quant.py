@@ -153,3 +153,23 @@ def test_quotient_in_three_steps_gives_every_code():
         q = v * inv
         code = np.rint(fma(fma(-q, scale, v), inv, q))
         assert np.array_equal(code, np.rint(v / scale)), i
+
+
+def test_one_product_gives_every_code():
+    """rint(v * factor) with one rounding, as quant_row.hpp forms codes (a fused multiply-add with 1.5 * 2^23): the oracle's code for the same
+    maxima and values, the factor being 1 / scale or its neighbour, on the side where the division puts half of the maximum."""
+    f32 = np.float32
+    values = (np.arange(0x7f80, dtype=np.uint32) << 16).view(f32)
+    moved = 0
+    for i in [1, 0x80, 0x3700, 0x3727, 0x3728, 0x7f7f] + [e * 128 + m for e in (110, 127, 140, 253) for m in range(128)]:
+        v = values[max(0, i - 9 * 128):i + 1]
+        m = max(values[i], f32(1e-5))
+        scale = m / f32(127)
+        inv = f32(1) / scale
+        up = float(m) - 127.0 * float(scale) >= float(scale) * -2.0 ** -18  # exact in float64
+        over = 0.5 * float(m) * float(inv) - 63.5
+        factor = np.nextafter(inv, f32(np.inf)) if up and over < 0 else np.nextafter(inv, f32(0)) if not up and over >= 0 else inv
+        moved += factor != inv
+        product = v.astype(np.float64) * np.float64(factor)  # 8 and 24 bits: exact
+        assert np.array_equal(np.rint(product), np.rint(v / scale)), i
+    assert moved > 0
