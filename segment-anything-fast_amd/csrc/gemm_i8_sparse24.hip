@@ -32,6 +32,7 @@
 // holds W row 32g + 16*(ta/2) + 8h + 4*(ta%2) + e; the lane then writes 8 adjacent bf16 per
 // 16-byte store.
 #include "gemm_i8_sparse24_shared.hpp"
+#include "gemm_pingpong.hpp"
 #include <type_traits>
 
 // every fp32 step below is rounded on its own (no fused multiply-add), so results
@@ -220,20 +221,14 @@ SF_DEVICE void sp24_epilogue_staged(const SparseArgs& a, i32x16 (&acc)[4][2 / KS
   }
 }
 
-// KS = 2: two groups of four wavefronts per tile, each on every second k tile with stages of its own; the
-// integer sums meet in LDS and each group finishes one of a wavefront's two X tiles.  For outputs of so
-// few tiles that a CU has one: its SIMDs would hold one wavefront, whose every barrier and fragment read is waited for.
-template <int EPI, int KS = 1>
-__global__ __launch_bounds__(256 * KS, 2) void gemm_i8_sp24_kernel(SparseArgs a) {
+template <int EPI>
+__global__ __launch_bounds__(256, 2) void gemm_i8_sp24_kernel(SparseArgs a) {
   constexpr int NST = S_NST;
   constexpr bool STAGED = EPI != SEPI_I32;  // epilogue through LDS
   static_assert(128 * SEP_STRIDE <= NST * S_STAGE, "output tile must fit in the operand stages");
-  static_assert(KS == 1 || (KS == 2 && STAGED), "the K split is built for the staged epilogues");
-  __shared__ __attribute__((aligned(16))) unsigned char lds_all[KS * NST * S_STAGE + (STAGED ? SEP_SCALE_BYTES : 0)];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[NST * S_STAGE + (STAGED ? SEP_SCALE_BYTES : 0)];
 
-  const int tid = threadIdx.x & 255;  // inside the group
-  const int grp = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
-  unsigned char* lds = lds_all + grp * (NST * S_STAGE);  // the group's operand stages
+  const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wa = wave >> 1, wb = wave & 1;  // position along W rows / X rows
@@ -250,27 +245,28 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_i8_sp24_kernel(SparseArgs a)
   const int x0 = (int)(first_x + in_group % gsz) * SBX;
   const int w0 = (int)(in_group / gsz) * SBW;
 
-  // ---- global -> LDS: per tile and wave 2 x (X, 16 B) + 2 x (Wc, 16 B) + 2 x (index, 4 B) ----
-  constexpr int NLD = 6;
+  // ---- global -> LDS, 16 bytes a lane: per tile and wave 2 x X + 2 x Wc + 1 x index words (half of them: the same twice, rather than a
+  // request of 4 bytes a lane that costs as much or a branch between the products) ----
+  constexpr int NLD = 5;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  unsigned int off_x[2], off_w[2], off_i[2];  // unsigned lane offsets: scalar-base load form
+  unsigned int off_x[2], off_w[2];  // unsigned lane offsets: scalar-base load form
+  // two slots' words are those of adjacent rows
+  const unsigned int off_i = (unsigned int)min(w0 + sp_slot_to_row(128 * (wave_u & 1) + 2 * lane), a.N - 2) * 8u;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int blk = wave_u + 4 * i;  // 1 KB block of the X / Wc tile, 256 B block of the index tile
+    const int blk = wave_u + 4 * i;  // 1 KB block of the X / Wc tile
     const int xr = 16 * blk + (lane >> 2);
     off_x[i] = (unsigned int)(min(x0 + xr, a.M - 1) * a.x_row_pitch + (((lane & 3) ^ sp_swizzle_x(xr)) * 16));
     const int slot = 32 * blk + (lane >> 1);
     const int gn = min(w0 + sp_slot_to_row(slot), a.N - 1);
     off_w[i] = (unsigned int)(gn * 32 + (((lane & 1) ^ sp_swizzle_w(slot)) * 16));
-    off_i[i] = (unsigned int)(gn * 8 + (lane & 1) * 4);
   }
   typedef __attribute__((address_space(1))) const void* gptr_t;
   typedef __attribute__((address_space(3))) void* lptr_t;
   auto dma_issue = [&](int kt, int stage_off) {
-    const int k = kt * KS + grp;
-    const int8_t* xb = a.x + k * a.x_kstep;
-    const int8_t* wb_ = a.wc + (int64_t)k * a.N * 32;
-    const int8_t* ib = reinterpret_cast<const int8_t*>(a.widx) + (int64_t)k * a.N * 8;
+    const int8_t* xb = a.x + kt * a.x_kstep;
+    const int8_t* wb_ = a.wc + (int64_t)kt * a.N * 32;
+    const int8_t* ib = reinterpret_cast<const int8_t*>(a.widx) + (int64_t)kt * a.N * 8;
     // tile bases stay in scalar registers and the lane offsets 32-bit at the point of use, so the
     // loads take the scalar-base form (the 64-bit per-lane address form costs the MFMA stream
     // several times more per load)
@@ -278,14 +274,15 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_i8_sp24_kernel(SparseArgs a)
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int blk = wave_u + 4 * i;
-      unsigned int ox = off_x[i], ow = off_w[i], oi = off_i[i];
-      asm volatile("" : "+v"(ox), "+v"(ow), "+v"(oi));
+      unsigned int ox = off_x[i], ow = off_w[i];
+      asm volatile("" : "+v"(ox), "+v"(ow));
       __builtin_amdgcn_global_load_lds((gptr_t)(xb + ox), (lptr_t)(lds + stage_off + blk * 1024), 16, 0, 0);
       __builtin_amdgcn_global_load_lds((gptr_t)(wb_ + ow),
                                        (lptr_t)(lds + stage_off + S_OFF_W + blk * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((gptr_t)(ib + oi),
-                                       (lptr_t)(lds + stage_off + S_OFF_I + blk * 256), 4, 0, 0);
     }
+    unsigned int oi = off_i;
+    asm volatile("" : "+v"(oi));
+    __builtin_amdgcn_global_load_lds((gptr_t)(ib + oi), (lptr_t)(lds + stage_off + S_OFF_I + (wave_u & 1) * 1024), 16, 0, 0);
   };
 
   // ---- operand fragments ----
@@ -335,7 +332,7 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_i8_sp24_kernel(SparseArgs a)
   if constexpr (STAGED) {
     // row scales, column scales and bias of this tile, 4 bytes per lane, straight into LDS; they
     // are the oldest loads in flight, so every later vmcnt wait covers them
-    unsigned char* sc = lds_all + KS * NST * S_STAGE;  // (both groups fetch the same)
+    unsigned char* sc = lds + NST * S_STAGE;
     const int mm = min(x0 + (wave_u & 1) * 64 + lane, a.M - 1);
     const int nn = min(w0 + wave_u * 64 + lane, a.N - 1);
     __builtin_amdgcn_global_load_lds((gptr_t)(a.sx + mm), (lptr_t)(sc + (wave_u & 1) * 256), 4, 0, 0);
@@ -343,7 +340,7 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_i8_sp24_kernel(SparseArgs a)
     __builtin_amdgcn_global_load_lds((gptr_t)((a.bias ? a.bias : a.sw) + nn),
                                      (lptr_t)(sc + 1536 + wave_u * 256), 4, 0, 0);
   }
-  const int nk = a.K / SBK / KS;  // even and >= NST (checked by the host)
+  const int nk = a.K / SBK;  // even and >= NST (checked by the host)
   int st[NST];  // st[j] = LDS offset of the stage holding tile kt + j (uniform, rotated)
 #pragma unroll
   for (int j = 0; j < NST; ++j) {
@@ -374,7 +371,7 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_i8_sp24_kernel(SparseArgs a)
       frags_at(st[1], fa[1 - P], fi[1 - P], fb[1 - P]);
     }
     mma(fa[P], fi[P], fb[P]);
-    // 12 LDS reads and 6 global->LDS loads spread over the 8 MFMAs
+    // 12 LDS reads and 5 global->LDS loads spread over the 8 MFMAs
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -386,7 +383,7 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_i8_sp24_kernel(SparseArgs a)
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       if constexpr (NEXT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       if constexpr (ISSUE)
-        if (g < 2) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        if (g < 1) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
     const int t = st[0];
@@ -409,39 +406,203 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_i8_sp24_kernel(SparseArgs a)
   iteration(kt + 2, C0{}, C0{}, C1{}, C0{});
   iteration(kt + 3, C1{}, C0{}, C0{}, C0{});
 
-  if constexpr (KS == 2) {
-    // group g finishes X tile g: the other group's share of it comes through LDS
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    __builtin_amdgcn_s_barrier();  // nobody reads operand stages any more
-    __builtin_amdgcn_sched_barrier(0);
-    i32x4* red = reinterpret_cast<i32x4*>(lds_all);
-    static_assert(2 * 256 * 16 * 16 <= KS * NST * S_STAGE, "the partial sums must fit in the operand stages");
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        i32x4 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = grp == 0 ? acc[i][1][4 * r + e] : acc[i][0][4 * r + e];
-        red[((1 - grp) * 16 + 4 * i + r) * 256 + tid] = v;
-      }
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    i32x16 sum[4][1];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const i32x4 v = red[(grp * 16 + 4 * i + r) * 256 + tid];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) sum[i][0][4 * r + e] = v[e] + (grp == 0 ? acc[i][0][4 * r + e] : acc[i][1][4 * r + e]);
-      }
-    sp24_epilogue_staged<EPI, KS>(a, sum, lds_all, lds_all + KS * NST * S_STAGE, x0, w0, wa, wb, lr, lh, threadIdx.x, grp);
-  } else if constexpr (STAGED)
-    sp24_epilogue_staged<EPI, KS>(a, acc, lds_all, lds_all + NST * S_STAGE, x0, w0, wa, wb, lr, lh, tid, 0);
+  if constexpr (STAGED)
+    sp24_epilogue_staged<EPI, 1>(a, acc, lds, lds + NST * S_STAGE, x0, w0, wa, wb, lr, lh, tid, 0);
   else
     sp24_epilogue<EPI>(a, acc, x0, w0, wa, wb, lr, lh);
+}
+
+// ---- outputs the GPU holds once -----------------------------------------------------------------------------------------
+// Tiles of 128 tokens x 256 channels, one workgroup of two sides per CU, K dealt to the sides in tiles of 128: while one side multiplies its 16
+// matrix instructions, 512 cycles, the other reads its fragments, 340 cycles; a barrier between turns; the sides' integer sums meet in LDS.
+// What bounds it is the load path: 36.9 KB of X, W and index words per turn are 576 cycles at the 64 bytes a clock that a CU takes in, and a wavefront that
+// requests them waits in line.  All behind the fragments' reads they made a turn 1065 cycles, all under the products 775, dealt to both 700 (by a
+// cycle counter in probes that are not kept).  Index words as 16-byte loads: 4 bytes a lane cost as much.
+// 5003 x 5120 -> 1280, us: four wavefronts 31.2, two groups of four on alternate 64-byte tiles in step (1100 cycles per 128 bytes) 30.5, this 29.1; of its 25 inside the kernel
+// 2 go before the first tile, 4.5 behind the last.
+template <int EPI>
+__global__ __launch_bounds__(512, 2) void gemm_i8_sp24_split_kernel(SparseArgs a) {
+  constexpr int OFF_W = SBX * 128, OFF_I = OFF_W + SBW * 64, STAGE = OFF_I + SBW * 16, NST = 4;
+  constexpr int LOADS = 9;  // of a wavefront in two turns
+  __shared__ __attribute__((aligned(16))) unsigned char lds[NST * STAGE + SEP_SCALE_BYTES];
+  unsigned char* sc = lds + NST * STAGE;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int side = wave >> 2, wq = wave & 3, wa = wq >> 1, wb = wq & 1;  // position along W rows / X rows
+  const int lr = lane & 31, lh = lane >> 5;
+  const unsigned int total = (unsigned int)a.tiles_x * (unsigned int)a.tiles_w;
+  const unsigned int pid = xcd_contiguous_id(blockIdx.x, total);
+  if (pid >= total) return;  // uniform over the workgroup
+  const unsigned int per_group = (unsigned int)a.group_x * a.tiles_w;
+  const unsigned int first_x = (pid / per_group) * a.group_x;
+  const unsigned int gsz = min((unsigned int)a.tiles_x - first_x, (unsigned int)a.group_x);
+  const unsigned int in_group = pid % per_group;
+  const int x0 = (int)(first_x + in_group % gsz) * SBX;
+  const int w0 = (int)(in_group / gsz) * SBW;
+
+  // ---- a tile's loads, wave instructions of 1 KB.  X: 128 bytes of a row, 16-byte chunk c at position c ^ (row / 2 % 8).  W and
+  // its index words 64-k block by block, in the slots of the 128-token kernel; two slots' words, 16 bytes, are those of adjacent rows ------
+  unsigned int off_x[4], off_w[4], off_i;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int u = wq + 4 * i;
+    const int r = 8 * u + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+    off_x[i] = (unsigned int)min(x0 + r, a.M - 1) * (unsigned int)a.x_row_pitch + (unsigned int)(c >> 2) * (unsigned int)a.x_kstep + (c & 3) * 16;
+    const int slot = 32 * (u & 7) + (lane >> 1);
+    off_w[i] = ((unsigned int)((u >> 3) * a.N) + min(w0 + sp_slot_to_row(slot), a.N - 1)) * 32u + ((lane & 1) ^ sp_swizzle_w(slot)) * 16;
+  }
+  off_i = ((unsigned int)((wq >> 1) * a.N) + min(w0 + sp_slot_to_row(128 * (wq & 1) + 2 * lane), a.N - 2)) * 8u;
+  typedef __attribute__((address_space(1))) const void* gptr_t;
+  typedef __attribute__((address_space(3))) void* lptr_t;
+  auto load = [&](const int8_t* base, unsigned int o, int dst) __attribute__((always_inline)) {
+    asm volatile("" : "+s"(base));  // uniform base, 32-bit lane offset
+    asm volatile("" : "+v"(o));
+    __builtin_amdgcn_global_load_lds((gptr_t)(base + o), (lptr_t)(lds + dst), 16, 0, 0);
+  };
+  // piece i of this wavefront's shares of tile t: of X and, last, the index words; of W
+  auto load_x = [&](int t, int i) __attribute__((always_inline)) {
+    const int at = (t & 3) * STAGE + wq * 1024;
+    if (i < 4) load(a.x + (int64_t)(2 * t) * a.x_kstep, off_x[i], at + i * 4096);
+    else load(reinterpret_cast<const int8_t*>(a.widx) + (int64_t)t * a.N * 16, off_i, at + OFF_I);
+  };
+  auto load_w = [&](int t, int i) __attribute__((always_inline)) {
+    load(a.wc + (int64_t)t * a.N * 64, off_w[i], (t & 3) * STAGE + OFF_W + (wq + 4 * i) * 1024);
+  };
+  auto share = [&](int t, bool x) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      if (x) load_x(t, i);
+      else if (i < 4) load_w(t, i);
+    }
+  };
+  auto meet = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // ---- fragments and products --------------------------------------------------------------------------------------------
+  const int fa_off = OFF_W + (wa * 128 + lr) * 32 + (lh ^ sp_swizzle_w(lr)) * 16;
+  const int fi_off = OFF_I + (wa * 128 + lr) * 8 + lh * 4;
+  const int fb_row = (wb * 64 + lr) * 128, fb_c = (2 * lh) ^ ((lr >> 1) & 7);  // chunks 2 lh, 2 lh + 1 and four more
+  i32x4 fa[2][4];
+  int fi[2][4];
+  i32x8 fb[2][2];
+  i32x16 acc[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+  // A tile is requested in two parts at once, W by the side that reads its fragments, X and the index words by the one that multiplies
+  auto read = [&](int t, bool request) __attribute__((always_inline)) {
+    const unsigned char* src = lds + (t & 3) * STAGE;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (request) load_w(t + 3, 2 * k + h);
+#pragma unroll
+        for (int i = 2 * h; i < 2 * h + 2; ++i) {
+          fa[k][i] = *reinterpret_cast<const i32x4*>(src + fa_off + k * (SBW * 32) + i * 1024);
+          fi[k][i] = *reinterpret_cast<const int*>(src + fi_off + k * (SBW * 8) + i * 256);
+        }
+        const i32x4 lo = *reinterpret_cast<const i32x4*>(src + fb_row + h * 4096 + (fb_c ^ (4 * k)) * 16);
+        const i32x4 hi = *reinterpret_cast<const i32x4*>(src + fb_row + h * 4096 + (fb_c ^ (4 * k + 1)) * 16);
+        fb[k][h] = i32x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      }
+  };
+  auto multiply = [&](int t, bool request) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          acc[i][j] = __builtin_amdgcn_smfmac_i32_32x32x64_i8(fa[k][i], fb[k][j], acc[i][j], fi[k][i], 0, 0);
+          const int at = 8 * k + 2 * i + j;
+          __builtin_amdgcn_sched_barrier(0);
+          if (request && at % 3 == 0 && at < 15) load_x(t + 4, at / 3);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    // (the products are pure values to the compiler; this pins them to their turn)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) asm volatile("" : "+v"(acc[i][j]));
+    __builtin_amdgcn_s_setprio(0);
+  };
+
+  // ---- scales and bias, the oldest loads in flight (both sides fetch the same), then the first three tiles ------------------
+  {
+    const int mm = min(x0 + (wq & 1) * 64 + lane, a.M - 1), nn = min(w0 + wq * 64 + lane, a.N - 1);
+    __builtin_amdgcn_global_load_lds((gptr_t)(a.sx + mm), (lptr_t)(sc + (wq & 1) * 256), 4, 0, 0);
+    __builtin_amdgcn_global_load_lds((gptr_t)(a.sw + nn), (lptr_t)(sc + 512 + wq * 256), 4, 0, 0);
+    __builtin_amdgcn_global_load_lds((gptr_t)((a.bias ? a.bias : a.sw) + nn), (lptr_t)(sc + 1536 + wq * 256), 4, 0, 0);
+  }
+  const int nt = a.K / 128;  // >= 3
+  share(0, side == 0);
+  share(2 - side, true);
+  share(2 - side, false);
+  pp_wait<LOADS>();  // tile 0
+  meet();
+  if (side == 1) {  // turn 0 of this side: one turn behind from here on
+    if (nt > 3) {
+      share(3, true);
+      pp_wait<5>();  // tile 1
+    } else {
+      pp_wait<0>();
+    }
+    meet();
+  }
+  // Turn t: one side reads tile t, the other one multiplies tile t - 1, both request tile t + 3 into the place that tile t - 1 was read from in the turn
+  // before.  A side's nine youngest requests, of this turn and the one before, stay in flight: tile t + 1 is there.
+  auto arrive = [&](bool requested) __attribute__((always_inline)) {
+    if (requested) pp_wait<LOADS>();
+    else pp_wait<0>();
+    meet();
+  };
+  for (int t = side; t < nt; t += 2) {
+    read(t, t + 3 < nt);
+    arrive(t + 3 < nt);
+    multiply(t, t + 4 < nt);
+    arrive(t + 4 < nt);
+  }
+  if (side == 0) meet();
+  else if (nt & 1) {  // the other side had one tile more
+    meet();
+    meet();
+  }
+  meet();  // nobody reads operand stages any more
+
+  // side g finishes X tile g: the other side's share of it comes through LDS
+  i32x4* red = reinterpret_cast<i32x4*>(lds);
+  static_assert(2 * 256 * 16 * 16 <= NST * STAGE, "the partial sums must fit in the operand stages");
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      i32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = side == 0 ? acc[i][1][4 * r + e] : acc[i][0][4 * r + e];
+      red[((1 - side) * 16 + 4 * i + r) * 256 + (tid & 255)] = v;
+    }
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  i32x16 sum[4][1];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const i32x4 v = red[(side * 16 + 4 * i + r) * 256 + (tid & 255)];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[i][0][4 * r + e] = v[e] + (side == 0 ? acc[i][0][4 * r + e] : acc[i][1][4 * r + e]);
+    }
+  sp24_epilogue_staged<EPI, 2>(a, sum, lds, sc, x0, w0, wa, wb, lr, lh, tid, side);
 }
 
 // ---- 2:4 pruning + packing --------------------------------------------------------
@@ -541,17 +702,16 @@ static int sparse_common(int epi, const int8_t* xq, const float* sx, const int8_
   if (gemm_i8_sp24_persist_covers(epi, a)) return gemm_i8_sp24_persist_launch(epi, a, stream);
   if (gemm_i8_sp24_turns_covers(epi, a)) return gemm_i8_sp24_turns_launch(epi, a, stream);
   const unsigned int grid = (unsigned int)(((total + 7) / 8) * 8);
-  // The K split where a CU has one tile and the loop is long (us, one group / two; SAMFAST_GEMM_SPLITK=0 off, 2
-  // wherever it is built).  K = 5120, while every tile has a CU: 60 tiles (1500 x 5120 -> 1280) 24.9 / 22.0, 160 (4096) 29.5 /
-  // 25.5, 200 (5003) 28.4 / 26.8, 220 28.9 / 28.0, 255 (6528) 31.7 / 30.8; 265 40.1 / 47.2, 320 42.8 / 48.6.  K = 3072 and 4096 pay
-  // less for the meeting in LDS the more CUs there are to feed, and nothing from 192 tiles on: 96 (4096 x 3072 -> 768) 17.8 /
-  // 16.4, 144 18.4 / 17.1, 192 19.1 / 19.0 and (2048 x 3072 -> 3072) 19.0 / 19.6, 225 20.8 / 21.1; 128 (4096 x 4096 -> 1024) 22.0 / 20.3, 192
-  // 23.0 / 22.9.  Shorter loops do not pay (6500 x 1280 -> 1280: 13.5 / 14.2).  What bounds both is operand delivery.
+  // K dealt to two sides where a CU has one tile and the loop is long enough for the meeting of their sums, 1.4 us, the more CUs there are to feed
+  // the longer (700 products of 1280 to 5120 values, one side / two, us; SAMFAST_GEMM_SPLITK=0 off, 2 wherever it is built): K = 5120 on 200 tiles (5003 ->
+  // 1280) 31.2 / 29.1, on 225 to 255 0.97 times as long; 4096 on 160 to 192 0.96 times, on 225 to 256 1.01; 3072 on 160 to 191 0.985, on 192 to 224 1.00;
+  // 2560 on 128 to 159 0.994, on 160 to 191 1.00; 2304 on 64 to 95 0.987, on 96 to 127 0.996; 2048 on 40 to 63 0.988, on 96 to 127 1.01; 1792 on 40 to 63 1.006.
   const int sk = knob_or(KNOB_GEMM_SPLITK, 1);
-  const bool ksplit = epi != SEPI_I32 && K % (4 * SBK) == 0 && K / SBK >= 2 * S_NST && (sk >= 2 || (sk == 1 && K >= 3072 && total <= (K >= 5120 ? 256 : 160)));
+  const int most = K >= 5120 ? 256 : K >= 4096 ? 224 : K >= 3072 ? 192 : K >= 2560 ? 144 : K >= 2304 ? 96 : K >= 2048 ? 64 : 0;
+  const bool ksplit = epi != SEPI_I32 && K / SBK >= 2 * S_NST && (sk >= 2 || (sk == 1 && total <= most));
 #define SF_SP24(E)                                                                                              \
   do {                                                                                                          \
-    if (ksplit) hipLaunchKernelGGL((gemm_i8_sp24_kernel<E, 2>), dim3(grid), dim3(512), 0, stream, a);           \
+    if (ksplit) hipLaunchKernelGGL((gemm_i8_sp24_split_kernel<E>), dim3(grid), dim3(512), 0, stream, a);        \
     else hipLaunchKernelGGL((gemm_i8_sp24_kernel<E>), dim3(grid), dim3(256), 0, stream, a);                     \
   } while (0)
   switch (epi) {

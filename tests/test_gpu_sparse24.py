@@ -334,3 +334,10 @@ def test_sparse24_split_k_loop_agrees(M, N, K, epi, layout):
             buf = res.clone()
             run(residual=buf, out=buf)
             assert torch.equal(buf, want)
+
+
+@pytest.mark.parametrize("M,N,K,epi", [(300, 264, 640, 0), (129, 8, 896, 2), (1000, 776, 1152, 1), (4090, 1280, 2560, 2)])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_sparse24_two_sides_with_any_number_of_k_tiles(M, N, K, epi, layout):
+    """K in an odd number of the sides' 128-value tiles, and rows and channels that end inside a tile's pieces."""
+    test_sparse24_split_k_loop_agrees(M, N, K, epi, layout)
