@@ -13,6 +13,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -83,6 +84,12 @@ void* stream_of(c10::DeviceIndex dev) { return c10::hip::getCurrentHIPStream(dev
 
 const void* ptr(const at::Tensor& t) { return t.const_data_ptr(); }
 
+// at::empty without its way through the dispatcher (0.72 -> 0.49 us): whoever has to see the allocation there is one of those whose
+// calls are declined above, and what is allocated here is written in full.
+at::Tensor new_tensor(at::IntArrayRef sizes, at::ScalarType type, c10::DeviceIndex dev) {
+  return at::detail::empty_cuda(sizes, type, c10::Device(c10::kCUDA, dev), std::nullopt);
+}
+
 // What the dense and the sparse Linear share: x is (..., K) contiguous bf16, sw_bits / bias_bits are
 // the fp32 scales and bias as the modules hold them (int32 bit patterns).  Fills y and the workspace.
 struct LinearCall {
@@ -100,11 +107,11 @@ struct LinearCall {
            sw->scalar_type() == at::kInt && sw->is_contiguous() && sw->numel() == N &&
            (!bias || (bias->scalar_type() == at::kInt && bias->is_contiguous() && bias->numel() == N));
   }
-  void allocate(int64_t need) {
+  void allocate(int64_t need, c10::DeviceIndex dev) {
     c10::SmallVector<int64_t, 5> shape(x->sizes().begin(), x->sizes().end());
     shape.back() = N;
-    y = at::empty(shape, x->options().requires_grad(false));
-    if (need > 0) work = at::empty({need}, x->options().dtype(at::kByte).requires_grad(false));
+    y = new_tensor(shape, at::kBFloat16, dev);
+    if (need > 0) work = new_tensor({need}, at::kByte, dev);
   }
 };
 
@@ -113,6 +120,14 @@ int64_t workspace(const LinearCall& c, int layout) {
   const int N = static_cast<int>(c.N), K = static_cast<int>(c.K);
   return p_linear_i8_one_launch(c.M, N, K, layout) == 1 ? 0 : p_linear_i8_workspace(c.M, N, K, layout);
 }
+
+// The entry of a module's buffers by that name, borrowed; None where there is none
+PyObject* buffer(PyObject* buffers, PyObject* name) {
+  PyObject* v = PyDict_GetItemWithError(buffers, name);
+  if (!v && PyErr_Occurred()) throw python_error();
+  return v ? v : Py_None;
+}
+PyObject* name_of(const char* s) { return PyUnicode_InternFromString(s); }
 
 // linear(x, wq, layout, sw_bits, bias_bits or None): the whole int8 Linear on bf16 rows.
 // wq is (N, K), or (K/64, N, 64) for layout 1.
@@ -132,7 +147,7 @@ PyObject* host_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   c.M = c.x->numel() / c.K;
   const int64_t need = workspace(c, layout);
   if (need < 0) Py_RETURN_NONE;
-  c.allocate(need);
+  c.allocate(need, dev);
   const int rc = p_linear_i8(ptr(*c.x), c.K, static_cast<const int8_t*>(ptr(*wq)), c.sw_ptr(), c.bias_ptr(), c.y.data_ptr(), c.N,
                              c.work_ptr(), c.M, static_cast<int>(c.N), static_cast<int>(c.K), SAMFAST_BF16, layout, stream_of(dev));
   if (rc != SAMFAST_OK) Py_RETURN_NONE;
@@ -158,12 +173,30 @@ PyObject* host_sparse_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   c.M = c.x->numel() / c.K;
   const int64_t need = workspace(c, SAMFAST_LAYOUT_SPARSE24);
   if (need < 0) Py_RETURN_NONE;
-  c.allocate(need);
+  c.allocate(need, dev);
   const int rc = p_linear_i8_sparse24(ptr(*c.x), c.K, static_cast<const int8_t*>(ptr(*wc)), static_cast<const int32_t*>(ptr(*widx)),
                                       c.sw_ptr(), c.bias_ptr(), c.y.data_ptr(), c.N, c.work_ptr(), c.M, static_cast<int>(c.N),
                                       static_cast<int>(c.K), SAMFAST_BF16, stream_of(dev));
   if (rc != SAMFAST_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(c.y));
+  END_HANDLE_TH_ERRORS
+}
+
+// module_linear(x, buffers), module_sparse_linear(x, buffers): the same with the buffers of the module as they stand
+PyObject* host_module_linear(PyObject* self, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  static PyObject *const wq = name_of("wq"), *const sw = name_of("sw_bits"), *const bias = name_of("bias_bits"), *const layout = PyLong_FromLong(SAMFAST_LAYOUT_ROWMAJOR);
+  if (n != 2 || !PyDict_Check(args[1])) Py_RETURN_NONE;
+  PyObject* const call[5] = {args[0], buffer(args[1], wq), layout, buffer(args[1], sw), buffer(args[1], bias)};
+  return host_linear(self, call, 5);
+  END_HANDLE_TH_ERRORS
+}
+PyObject* host_module_sparse_linear(PyObject* self, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  static PyObject *const wc = name_of("wc"), *const widx = name_of("widx"), *const sw = name_of("sw_bits"), *const bias = name_of("bias_bits");
+  if (n != 2 || !PyDict_Check(args[1])) Py_RETURN_NONE;
+  PyObject* const call[5] = {args[0], buffer(args[1], wc), buffer(args[1], widx), buffer(args[1], sw), buffer(args[1], bias)};
+  return host_sparse_linear(self, call, 5);
   END_HANDLE_TH_ERRORS
 }
 
@@ -189,7 +222,7 @@ PyObject* host_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (rh.size(4) != 1 || rw.size(3) != 1 || q.stride(3) != 1 || k.stride(3) != 1 || v.stride(3) != 1 || rh.stride(3) != 1 || rw.stride(4) != 1)
     Py_RETURN_NONE;
   const double scale = PyFloat_AsDouble(args[5]);
-  at::Tensor out = at::empty({B, nH, N, hd}, q.options().requires_grad(false));
+  at::Tensor out = new_tensor({B, nH, N, hd}, q.scalar_type(), dev);
   const int rc = p_attn_bias(ptr(q), ptr(k), ptr(v), ptr(rh), ptr(rw), out.data_ptr(), static_cast<int>(B), static_cast<int>(nH),
                              static_cast<int>(gh), static_cast<int>(gw), static_cast<int>(hd), q.stride(0), q.stride(1), q.stride(2),
                              k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2), nH * N * hd, N * hd, hd,
@@ -244,6 +277,8 @@ PyMethodDef kMethods[] = {
     {"plain", host_plain, METH_O, nullptr},
     {"linear", fastcall(host_linear), METH_FASTCALL, nullptr},
     {"sparse_linear", fastcall(host_sparse_linear), METH_FASTCALL, nullptr},
+    {"module_linear", fastcall(host_module_linear), METH_FASTCALL, nullptr},
+    {"module_sparse_linear", fastcall(host_module_sparse_linear), METH_FASTCALL, nullptr},
     {"attention", fastcall(host_attention), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

@@ -90,7 +90,7 @@ def _attention_rel_h_rel_w(q_, k_, v_, rel_h_, rel_w_):
         # one native call on the factors as they are: the operator below wants them packed side by
         # side (flash_4.py:352), a copy that costs an eighth of the attention itself.  Where a tracer,
         # a transform or a mode is to see the operator, the call declines.
-        out = _lib.host().attention(q_, k_, v_, rel_h_, rel_w_, 1.0 / math.sqrt(hd))
+        out = (_lib._host or _lib.host()).attention(q_, k_, v_, rel_h_, rel_w_, 1.0 / math.sqrt(hd))
         if out is not None:
             return out
     k_h, k_w = rel_h_.size(3), rel_w_.size(4)

@@ -153,17 +153,10 @@ class Int8LinearBase(nn.Module):
             yq, sy = ops.quant_rowwise(y, layout=out_layout)
         return y, yq, sy
 
-    def _forward_native(self, x: torch.Tensor) -> Optional[torch.Tensor]:
-        """The whole Linear through the native host module; None for a call it does not cover."""
-        return None
-
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """The kernels compute on bf16 rows; any other floating input is cast on the way in and
-        the result cast back, so the module keeps its input's dtype as nn.Linear does."""
-        if ops._launch_log is None and x.is_cuda:
-            y = self._forward_native(x)
-            if y is not None:
-                return y
+        the result cast back, so the module keeps its input's dtype as nn.Linear does.  The
+        subclasses try the native host module first, which does the whole Linear of a call that it covers."""
         lead = x.shape[:-1]
         x2 = x.reshape(-1, self.in_features)
         if x2.dtype != torch.bfloat16:
@@ -198,9 +191,13 @@ class Int8DynamicLinear(Int8LinearBase):
         wq = self._buffers["wq"]
         return wq if layout != LAYOUT_KB64 else kept_copy(self, "_kb64", wq, lambda: ops.to_kb64(wq))
 
-    def _forward_native(self, x: torch.Tensor) -> Optional[torch.Tensor]:
-        buffers = self._buffers  # the weights as they stand: no copy that could be behind them
-        return _lib.host().linear(x, buffers["wq"], LAYOUT_ROWMAJOR, buffers["sw_bits"], buffers.get("bias_bits"))
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if ops._launch_log is None and x.is_cuda:
+            # the weights as they stand: no copy that could be behind them
+            y = (_lib._host or _lib.host()).module_linear(x, self._buffers)
+            if y is not None:
+                return y
+        return super().forward(x)
 
     def linear_fused_quant(self, xq, sx, epilogue, residual=None, out=None, layout=LAYOUT_ROWMAJOR,
                            ln=None, out_layout=LAYOUT_ROWMAJOR):

@@ -96,9 +96,12 @@ class Int8Sparse24Linear(Int8LinearBase):
         return ops.gemm_i8_sparse24_fused(xq, sx, self.wc, self.widx, self.sw, self.bias_f32,
                                           epilogue, residual=residual, out=out, layout=layout)
 
-    def _forward_native(self, x: torch.Tensor) -> Optional[torch.Tensor]:
-        b = self._buffers
-        return _lib.host().sparse_linear(x, b["wc"], b["widx"], b["sw_bits"], b.get("bias_bits"))
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if ops._launch_log is None and x.is_cuda:
+            y = (_lib._host or _lib.host()).module_sparse_linear(x, self._buffers)
+            if y is not None:
+                return y
+        return super().forward(x)
 
     def extra_repr(self) -> str:
         return (f"in_features={self.in_features}, out_features={self.out_features}, "

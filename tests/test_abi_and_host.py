@@ -813,3 +813,19 @@ def test_a_linear_of_another_type_is_unsupported_in_every_form(M, N, K):
     lib, p = _lib.load(), [1 << 40 + i for i in range(7)]  # (refused before anything is launched)
     assert lib.samfast_linear_i8(p[0], K, p[1], p[2], p[3], p[4], N, p[5], M, N, K, _lib.SAMFAST_F16, 0, None) == -2
     assert lib.samfast_linear_i8_sparse24(p[0], K, p[1], p[2], p[3], p[4], p[5], N, p[6], M, N, K, _lib.SAMFAST_F16, None) == -2
+
+
+def test_the_native_modules_entries_decline_what_they_do_not_cover():
+    """A module's Linear on the CPU, with a buffer missing or none at all, is left to the Python route."""
+    from samfast_amd import _lib
+    from samfast_amd.quant import Int8DynamicLinear
+    host = _lib.host()
+    lin = Int8DynamicLinear.from_float(torch.nn.Linear(256, 16))
+    x = torch.randn(3, 256).to(torch.bfloat16)
+    for entry in (host.module_linear, host.module_sparse_linear):
+        assert entry(x, lin._buffers) is None
+        assert entry(x, {}) is None
+        assert entry(x, None) is None
+        assert entry(x) is None
+    with pytest.raises(RuntimeError):
+        lin(x)
