@@ -138,7 +138,7 @@ PyObject* host_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int layout = static_cast<int>(PyLong_AsLong(args[2]));
   const bool kb = layout == SAMFAST_LAYOUT_KB64;
   LinearCall c = {tensor_arg(args[0]), tensor_arg(args[3]), tensor_arg(args[4])};
-  if (!c.x || !wq || !c.sw || (args[4] != Py_None && !c.bias)) Py_RETURN_NONE;
+  if (!c.x || !c.x->is_cuda() || !wq || !c.sw || (args[4] != Py_None && !c.bias)) Py_RETURN_NONE;
   const c10::DeviceIndex dev = c10::hip::current_device();
   if (!on_current_gpu(*wq, dev) || wq->scalar_type() != at::kChar || wq->dim() != (kb ? 3 : 2) || !wq->is_contiguous()) Py_RETURN_NONE;
   c.N = wq->size(kb ? 1 : 0);
@@ -161,7 +161,7 @@ PyObject* host_sparse_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (n != 5 || !plain_call()) Py_RETURN_NONE;
   const at::Tensor *wc = tensor_arg(args[1]), *widx = tensor_arg(args[2]);
   LinearCall c = {tensor_arg(args[0]), tensor_arg(args[3]), tensor_arg(args[4])};
-  if (!c.x || !wc || !widx || !c.sw || (args[4] != Py_None && !c.bias)) Py_RETURN_NONE;
+  if (!c.x || !c.x->is_cuda() || !wc || !widx || !c.sw || (args[4] != Py_None && !c.bias)) Py_RETURN_NONE;
   const c10::DeviceIndex dev = c10::hip::current_device();
   if (!on_current_gpu(*wc, dev) || !on_current_gpu(*widx, dev) || wc->scalar_type() != at::kChar || widx->scalar_type() != at::kInt ||
       wc->dim() != 3 || widx->dim() != 3 || !wc->is_contiguous() || !widx->is_contiguous() || wc->size(2) != 32 ||
