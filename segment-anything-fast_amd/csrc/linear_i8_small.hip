@@ -260,7 +260,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 2) void linear_i8_sp24_small_kern
 template <int MT, int NT>
 __global__ __launch_bounds__(64 * kSmallWaves, 2) void gemm_i8_skinny_kernel(SmallArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  constexpr int DEPTH = MT + NT <= 4 ? 4 : MT + NT <= 6 ? 3 : 2;
+  constexpr int DEPTH = MT + NT <= 4 ? 4 : 3;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lq = lane >> 4;
@@ -388,16 +388,16 @@ int linear_i8_small_launch(const unsigned short* x, int64_t ldx, const int8_t* w
 
 // The smallest tile whose tiles still fit the GPU's CUs once: a smaller tile means a shorter chain, a second
 // round costs more than that gains.  Measured on K-block major codes, us, against the tiled kernels:
-// 128 x 3840 x 1280 in 64 x 32 tiles 4.7 (6.3), 64 x 1280 x 5120 in 16 x 32 5.6 (14.6), 512 x 1280 x 5120 in
-// 64 x 64 12.8 (21.9); the largest tile only pays on a long K loop (512 x 1280 x 1280: 6.3 against 6.4).
+// 128 x 3840 x 1280 in 64 x 32 tiles 4.7 (6.3), 64 x 1280 x 5120 in 16 x 32 5.6 (14.6).  From 2304 values on 64 x 32 tiles are slower than
+// 64 x 64 ones whose operands come through LDS (gemm_i8_once.hip; 278 x 1280 x 3072 8.3 / 7.6, 0.96 times as long over 70 shapes, below 2240 1.04 to 1.07), and
+// 64 x 64 tiles straight into registers were at any length (512 x 1280 x 3072 10.6 / 8.4).
 // Returns 16-row tiles * 8 + 16-column tiles, 0 = none.
 static int skinny_shape(int M, int N, int K) {
   auto fits = [&](int mt, int nt) { return (int64_t)((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * nt - 1) / (16 * nt)) <= 256; };
   if (fits(1, 1)) return 1 * 8 + 1;
   if (fits(1, 2)) return 1 * 8 + 2;
   if (fits(2, 2)) return 2 * 8 + 2;
-  if (fits(4, 2)) return 4 * 8 + 2;
-  if (K >= 2048 && fits(4, 4)) return 4 * 8 + 4;
+  if (K < 2304 && fits(4, 2)) return 4 * 8 + 2;
   return 0;
 }
 
@@ -424,8 +424,7 @@ int gemm_i8_skinny_launch(const GemmArgs& g, hipStream_t stream) {
     case 1 * 8 + 1: return launch_skinny<1, 1>(a, stream);
     case 1 * 8 + 2: return launch_skinny<1, 2>(a, stream);
     case 2 * 8 + 2: return launch_skinny<2, 2>(a, stream);
-    case 4 * 8 + 2: return launch_skinny<4, 2>(a, stream);
-    default: return launch_skinny<4, 4>(a, stream);
+    default: return launch_skinny<4, 2>(a, stream);
   }
 }
 

@@ -219,6 +219,34 @@ def test_one_tile_per_cu_agrees_with_the_small_tiles(bm, tn, M, N, K, epi, layou
         assert torch.equal(run(residual=res), y)
 
 
+@pytest.mark.parametrize("bm,tn,M,N,K,epi", [
+    # 64-row tiles, K dealt to four groups: the shortest loop, one to three k tiles behind the last whole round of the groups, edges of rows and columns
+    (64, 2, 64, 64, 1280, 0), (64, 2, 1, 8, 1344, 0), (64, 2, 633, 1288, 5120, 2), (64, 2, 130, 200, 1408, 1),
+    (64, 3, 65, 96, 1472, 0), (64, 3, 1000, 776, 3072, 2), (64, 3, 63, 104, 1280, 1),
+    (64, 4, 129, 128, 1280, 2), (64, 4, 1321, 1280, 4096, 0), (64, 4, 200, 136, 1600, 1),
+])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_one_tile_of_64_rows_agrees_with_the_small_tiles(bm, tn, M, N, K, epi, layout):
+    test_one_tile_per_cu_agrees_with_the_small_tiles(bm, tn, M, N, K, epi, layout)
+
+
+@pytest.mark.parametrize("M,N,K", [(278, 1280, 3072), (900, 768, 3072), (1638, 768, 4096), (1327, 1280, 4096), (2000, 1280, 4096)])
+def test_linears_over_some_hundred_long_rows_against_their_codes(M, N, K):
+    """Two launches through the tile that the rule takes, against the product of the quantiser's own codes in 64 bits."""
+    from samfast_amd import Int8DynamicLinear, ops
+    print(f"case long rows M={M} N={N} K={K}", flush=True)
+    x, w, b = linear_inputs(M, K, N, seed=M)
+    lin = torch.nn.Linear(K, N, dtype=torch.bfloat16)
+    with torch.no_grad():
+        lin.weight.copy_(w)
+        lin.bias.copy_(b)
+    lin, x = Int8DynamicLinear.from_float(lin.cuda()), x.cuda()
+    y = lin(x)
+    xq, sx = ops.quant_rowwise(x)
+    acc = (xq.double() @ lin.wq.double().t()).float()  # (integers below 2^53: exact)
+    assert torch.equal(y, (acc * sx[:, None] * lin.sw + lin.bias_f32).to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("sparse,M,N,K", [
     # workgroups of 8 rows and one, two, four column tiles, of 16 rows; the last calls of each, remainders of rows, columns and k steps
     (False, 63, 488, 64), (False, 64, 512, 512), (False, 65, 1000, 576), (False, 121, 1024, 1024), (False, 128, 1032, 1088), (False, 250, 1016, 1536),
