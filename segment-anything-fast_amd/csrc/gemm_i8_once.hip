@@ -243,9 +243,17 @@ __global__ __launch_bounds__(512, 2) void gemm_i8_once_kernel(GemmArgs a) {
       constexpr bool STEADY = decltype(steady)::value;
       if constexpr (STEADY) arrive(NST - 2);
       else arrive(t == 0 ? NST - 1 : min(nt - 1 - t, NST - 2));
-      if (STEADY || (t > 0 && t - 1 + NST < nt)) fill(t - 1 + NST, st == 0 ? NST - 1 : st - 1);
       read(f, st);
       multiply(f);
+      if (STEADY || (t > 0 && t - 1 + NST < nt)) fill(t - 1 + NST, st == 0 ? NST - 1 : st - 1);
+      if (STEADY) {
+        __builtin_amdgcn_sched_group_barrier(0x100, TM + TN, 0);
+#pragma unroll
+        for (int g = 0; g < NLD; ++g) {
+          __builtin_amdgcn_sched_group_barrier(0x008, TM * TN / (NLD + 1), 0);
+          __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        }
+      }
       st = next_stage(st);
       __builtin_amdgcn_sched_barrier(0);
     };
