@@ -11,8 +11,11 @@
 //     neighbours have other tokens: stored from there, 16 bytes are an access of their own, 10000 of them per tile at one a cycle, twice
 //     that with the residual.  Turned round in 4 KB that the wavefront owns, eight lanes hold a whole line;
 //   * outputs beyond the last-level cache streamed: left in the L2s they pushed the operands out.
+//   * scales and bias of a lane's channels kept over the units of its output that share them.
 // us, 128-token kernel / stored from the accumulators / turned round / streamed / whole lines: 131072 x 1280 -> 5120 704 / 702 / 684 / 598 / 578,
-// 131072 x 5120 -> 1280 with the residual 605 / 547 / 545 / - / 516.  A third k tile in LDS (256 x 256): nothing.
+// 131072 x 5120 -> 1280 with the residual 605 / 547 / 545 / - / 516.  Scales read anew for every 16 tokens / kept: 131072 x 1280 -> 5120 597 / 567, 131072 x
+// 1024 -> 3072 325 / 308, 65536 x 1280 -> 5120 303 / 290, 131072 x 5120 -> 1280 with the residual 515 / 512.  A third k tile in LDS (256 x 256): nothing.  Three k tiles of X, its
+// fragments read under the products before theirs (the output turned round where a k tile was): on zeros 5120 -> 1280 471 / 453, on codes 518 / 535 and 1280 -> 5120 571 / 599.
 // Inside the ViT-H encoder, both Linears of the MLP 2:4, 32 images 115.7 -> 111.2 ms, 16 58.6 -> 55.5, one 5.52 -> 5.22.
 #include "gemm_i8_sparse24_shared.hpp"
 #include "gemm_pingpong.hpp"
@@ -256,34 +259,56 @@ __global__ __launch_bounds__(512, 2) void gemm_i8_sp24_turns_kernel(SparseArgs a
     float sx[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) sx[i] = *reinterpret_cast<const float*>(sc + (row0 + 16 * i + lr) * 4);
+    // Scales and bias of a lane's eight channels of a pair: kept while the two wide units that share 64 channels need them, or, where the
+    // residual leaves no registers for both pairs, read for twice 16 tokens.  Read anew for every 16 tokens they were two thirds of an end's LDS
+    // operations.
+    constexpr bool KEEP = !RES || TN == 8;
+    f32x4 scale[1 + KEEP][1 + KEEP], shift[1 + KEEP][1 + KEEP];
+    auto constants = [&](int slot, int t, int channel) __attribute__((always_inline)) {
+      const int at = P::BM * 4 + (channel + 8 * lq + 4 * t) * 4;
+      scale[slot][KEEP ? t : 0] = *reinterpret_cast<const f32x4*>(sc + at);
+      shift[slot][KEEP ? t : 0] = *reinterpret_cast<const f32x4*>(sc + (a.bias ? P::BN * 4 + at : P::SCALES + 8 * 4096));
+    };
 #pragma unroll
     for (int u = 0; u <= P::UNITS_OUT; ++u) {
       if (u < P::UNITS_OUT) {
+        if (KEEP && !(wide(u) && u & 1)) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          // 16 tokens by 32 channels: token fragment i, channel pair p
-          const int i = wide(u) ? 2 * (u & 1) + (e & 1) : e, p = wide(u) ? (u & ~1) + (e >> 1) : P::PAIRS;
-          const int at = P::BM * 4 + (column(u) + (wide(u) ? 32 * (e >> 1) : 0) + 8 * lq) * 4;
-          u32x4 v4;
+          for (int d = 0; d < (wide(u) ? 2 : 1); ++d)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) constants(d, t, column(u) + 32 * d);
+        }
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+          // twice 16 tokens by 32 channels: token fragments i0 and i0 + 1, channel pair p
+          const int i0 = wide(u) ? 2 * (u & 1) : 2 * d, p = wide(u) ? (u & ~1) + d : P::PAIRS;
+          u32x4 v4[2];
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
-            const f32x4 sw = *reinterpret_cast<const f32x4*>(sc + at + 16 * t);
-            const f32x4 bias = *reinterpret_cast<const f32x4*>(sc + (a.bias ? P::BN * 4 + at + 16 * t : P::SCALES + 8 * 4096));
-            float y[4];
+            const int k = KEEP && wide(u) ? d : 0, kt = KEEP ? t : 0;
+            if (!KEEP) constants(0, t, column(u) + (wide(u) ? 32 * d : 0));
+            const f32x4 sw = scale[k][kt], bias = shift[k][kt];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              // three separately rounded fp32 operations (no fused multiply-add)
-              float v = (float)acc[i][2 * p + t][r] * sx[i];
-              v = v * sw[r];
-              y[r] = v + bias[r];
+            for (int j = 0; j < 2; ++j) {
+              float y[4];
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                // three separately rounded fp32 operations (no fused multiply-add)
+                float v = (float)acc[i0 + j][2 * p + t][r] * sx[i0 + j];
+                v = v * sw[r];
+                y[r] = v + bias[r];
+              }
+              v4[j][2 * t] = pack_bf16x2(y[0], y[1]);
+              v4[j][2 * t + 1] = pack_bf16x2(y[2], y[3]);
             }
-            v4[2 * t] = pack_bf16x2(y[0], y[1]);
-            v4[2 * t + 1] = pack_bf16x2(y[2], y[3]);
           }
           // through the wavefront's own 4 KB: a lane has 16 bytes of a token, neighbouring lanes other tokens
-          const int in = wide(u) ? (e & 1) * 2048 + lr * 128 + (((4 * (e >> 1) + lq) ^ (lr >> 1)) * 16) : e * 1024 + lr * 64 + ((lq ^ (-(lr >> 2) & 3)) * 16);
-          *reinterpret_cast<u32x4*>(turn + in) = v4;
-          if (e & 1) __builtin_amdgcn_sched_barrier(0);  // keep the conversion narrow
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int in = wide(u) ? j * 2048 + lr * 128 + (((4 * d + lq) ^ (lr >> 1)) * 16) : (2 * d + j) * 1024 + lr * 64 + ((lq ^ (-(lr >> 2) & 3)) * 16);
+            *reinterpret_cast<u32x4*>(turn + in) = v4[j];
+          }
+          __builtin_amdgcn_sched_barrier(0);  // keep the conversion narrow
         }
       }
       if (u > 0) {
