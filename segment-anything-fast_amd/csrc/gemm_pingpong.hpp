@@ -479,12 +479,19 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
 
 // ---- outputs the GPU holds once: 128-row tiles, K shared between the sides ------------------------------------------
 // An image's products onto few columns: 4096 rows and 768, 1024 or 1280 columns are exactly 256 tiles of 128 x {96, 128, 160}.  The
-// wavefronts 0-3 multiply the lower 64 bytes of every k tile, 4-7 the upper ones, by turns as above; each holds 64 rows and half
-// of the columns, and the two sides' sums meet in LDS at the end, where each side finishes half of the rows.  What bounds it is
-// the load path: 288 rows of 128 bytes for 640 cycles of products are 58 of the 64 bytes per clock that a CU takes in (bf16 4096 x 5120
-// -> 1280: 61 us, 41 without the products, 37 without the loads).  With the residual, us, library's product + residual in the
-// next LayerNorm / this + LayerNorm: 4096 x 5120 -> 1280 61.3 / 55.9, 4096 x 1280 -> 1280 31.1 / 23.6, 4096 x 768 -> 768 31.6 / 18.6.
-// (int8 keeps gemm_i8_once.hip: 4096 x 5120 -> 1280 30.0 there, 32.7 here.)
+// wavefronts 0-3 multiply the lower 64 bytes of every k tile, 4-7 the upper ones; each holds 64 rows and half
+// of the columns, and the two sides' sums meet in LDS at the end, where each side finishes half of the rows.  So few columns leave a
+// wavefront registers for two k tiles' fragments: it reads the next ones, and requests a k tile, between its products, with one barrier per k tile.
+// (The sides by turns as above, one multiplying while the other read, were two barriers and two latencies of the LDS around 320 cycles of
+// products.  bf16 with the residual, us, by turns / so, operands in the caches: 4096 x 5120 -> 1280 53.3 / 48.1, 4096 x 4096 -> 1024 36.5 / 32.4, 4096 x 3072 -> 768 27.0 / 22.0,
+// 4096 x 1280 -> 1280 18.3 / 17.4, 4096 x 768 -> 768 9.9 / 8.5.)  What bounds it now is how the operands come: 288 rows of 128 bytes for
+// 640 cycles of products are 58 of the 64 bytes per clock that a CU takes in.
+// Long loops' weights, which come from HBM in an encoder whose weights exceed the last-level cache, are touched once, a line by each
+// thread of the grid, row by row: the loop asks all CUs' rows for one line each at a time, and waited for HBM at every k tile
+// (weights and rows not in the L2s: 4096 x 5120 -> 1280 60.2 / 50.3, 4096 x 4096 -> 1024 39.0 / 34.0, 4096 x 3072 -> 768 29.8 / 25.0, 2048 x 5120 -> 1280 45.1 / 36.2; all of it in
+// them: 49.0 / 49.0, 32.4 / 33.0, 21.9 / 22.4, 31.5 / 32.6).  At 20 k tiles and fewer it is level or slower (4096 x 1280 -> 1280 20.7 / 21.3).
+// Library's product + residual in the next LayerNorm / by turns + LayerNorm: 4096 x 5120 -> 1280 61.3 / 55.9, 4096 x 1280 -> 1280
+// 31.1 / 23.6, 4096 x 768 -> 768 31.6 / 18.6.  (int8 keeps gemm_i8_once.hip.)
 template <int TN>
 struct PPSplitTile {
   static_assert(TN >= 3 && TN <= 5, "widths built: 96, 128, 160");
@@ -588,12 +595,12 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_split_kernel(PPArgs a) {
     asm volatile("" : "+v"(o));
     __builtin_amdgcn_global_load_lds((gptr_t)(base + o), (lptr_t)(lds + stage + row * 128), 16, 0, 0);
   };
-  auto fill = [&](int stage) __attribute__((always_inline)) {
-    load(xk, off_x, wave * 8, stage);
-    load(xk + (int64_t)64 * a.x_pitch, off_x, (wave + 8) * 8, stage);
-#pragma unroll
-    for (int i = 0; i < P::LO; ++i)
-      if (i < nw) load(wk, off_w[i], P::BM + at_w[i], stage);
+  // load l of this wavefront's 2 + nw for a k tile
+  auto fill = [&](int l, int stage) __attribute__((always_inline)) {
+    if (l < 2) load(xk + (int64_t)(64 * l) * a.x_pitch, off_x, (wave + 8 * l) * 8, stage);
+    else if (l - 2 < TN - P::LO || l - 2 < nw) load(wk, off_w[l < 2 ? 0 : l - 2], P::BM + at_w[l < 2 ? 0 : l - 2], stage);
+  };
+  auto advance = [&]() __attribute__((always_inline)) {
     xk += 2 * a.x_kstep;
     wk += 2 * a.w_kstep;
   };
@@ -618,49 +625,83 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_split_kernel(PPArgs a) {
     for (int j = 0; j < TN; ++j) acc[i][j] = typename E::acc_t{};
   const int nk = a.nk;  // >= NST
 #pragma unroll
-  for (int p = 0; p < NST - 1; ++p) fill(p * P::STAGE);
-  arrive(std::integral_constant<int, NST - 2>{});
-  meet();
-  if (side == 1) meet();  // one turn behind
-  // k tile t: fragments read, k tile t + NST - 1 requested into the stage that both sides have left, t + 1 awaited; then the products
-  auto ktile = [&](int t, int rd, int wr, bool steady) __attribute__((always_inline)) {
-    i32x4 fx[4], fw[TN];
+  for (int p = 0; p < NST; ++p) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) fx[i] = *reinterpret_cast<const i32x4*>(lds + rd + x_off + i * 2048);
+    for (int l = 0; l < 2 + P::LO; ++l) fill(l, p * P::STAGE);
+    advance();
+  }
+  unsigned int touched = 0;
+  if (nk >= 32) {  // this thread's line of W
+    const unsigned int line = min(blockIdx.x * 512u + tid, (unsigned int)a.N * nk - 1u), row = line / (unsigned int)nk;
+    touched = *(gword_t)((gbyte_t)(uintptr_t)a.w + (int64_t)row * a.w_pitch + (line - row * nk) * 128);
+  }
+  i32x4 fx[2][4], fw[2][TN];
+  constexpr int READS = 4 + TN;
+  auto read = [&](int buf, int r, int stage) __attribute__((always_inline)) {
+    if (r < TN) fw[buf][r < TN ? r : 0] = *reinterpret_cast<const i32x4*>(lds + stage + w_off + r * 2048);
+    else fx[buf][r < TN ? 0 : r - TN] = *reinterpret_cast<const i32x4*>(lds + stage + x_off + (r - TN) * 2048);
+  };
+  // k tile t: its products; between them its stage, whose fragments every wavefront holds, is requested anew for t + NST (`more`), and t + 1's
+  // fragments are read (`next`); t + 2 is awaited
+  auto ktile = [&](auto buf, auto more, auto next, int here, int ahead) __attribute__((always_inline)) {
+    constexpr int B = decltype(buf)::value;
+    int slot = 0;
 #pragma unroll
-    for (int j = 0; j < TN; ++j) fw[j] = *reinterpret_cast<const i32x4*>(lds + rd + w_off + j * 2048);
-    if (steady) {
-      fill(wr);
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int jj = 0; jj < TN; ++jj, ++slot) {
+        const int j = i & 1 ? TN - 1 - jj : jj;
+        acc[i][j] = E::mma(fx[B][i], fw[B][j], acc[i][j]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (decltype(next)::value && slot < READS) read(1 - B, slot, ahead);
+        if (decltype(more)::value && slot >= 4 * TN - 2 - P::LO) fill(slot - (4 * TN - 2 - P::LO), here);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    if constexpr (decltype(more)::value) {
+      advance();
       arrive(std::integral_constant<int, NST - 2>{});
     } else {
       pp_wait<0>();
     }
-    meet();
-    __builtin_amdgcn_s_setprio(1);
+    if constexpr (decltype(next)::value) meet();
+  };
+  using B0 = std::integral_constant<int, 0>;
+  using B1 = std::integral_constant<int, 1>;
+  using Yes = std::true_type;
+  using No = std::false_type;
+  auto up = [&](int s) __attribute__((always_inline)) { return s == (NST - 1) * P::STAGE ? 0 : s + P::STAGE; };
+  auto begin = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int jj = 0; jj < TN; ++jj) {
-        const int j = i & 1 ? TN - 1 - jj : jj;
-        acc[i][j] = E::mma(fx[i], fw[j], acc[i][j]);
-      }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(acc[i][j]));
-    __builtin_amdgcn_s_setprio(0);
+    for (int r = 0; r < READS; ++r) read(buf, r, 0);
+    arrive(std::integral_constant<int, NST - 2>{});
     meet();
   };
-  auto up = [&](int s) __attribute__((always_inline)) { return s == (NST - 1) * P::STAGE ? 0 : s + P::STAGE; };
-  int rd = 0, wr = (NST - 1) * P::STAGE;
-  for (int t = 0; t < nk; ++t) {
-    ktile(t, rd, wr, t + NST - 1 < nk);
-    rd = up(rd);
-    wr = up(wr);
+  int here = 0, left = nk;
+  arrive(std::integral_constant<int, NST - 1>{});
+  meet();
+  // two at a time, so that the fragments' two places are known; an odd one first
+  if ((nk - NST) & 1) {
+    begin(1);
+    ktile(B1{}, Yes{}, Yes{}, here, up(here));
+    here = up(here);
+    --left;
+  } else {
+    begin(0);
   }
-  if (side == 0) meet();
-  meet();  // nobody reads operand stages any more
+  for (; left > NST; left -= 2) {
+    const int there = up(here);
+    ktile(B0{}, Yes{}, Yes{}, here, there);
+    here = up(there);
+    ktile(B1{}, Yes{}, Yes{}, there, here);
+  }
+#pragma unroll
+  for (int p = 0; p < NST; ++p) {
+    if (p == NST - 1) p & 1 ? ktile(B1{}, No{}, No{}, here, here) : ktile(B0{}, No{}, No{}, here, here);
+    else p & 1 ? ktile(B1{}, No{}, Yes{}, here, up(here)) : ktile(B0{}, No{}, Yes{}, here, up(here));
+    here = up(here);
+  }
 
+  asm volatile("" : : "v"(touched));
   // ---- the sides' sums meet: side 0 finishes row groups 0 and 1, side 1 the other two -----------------------------------
   typedef typename E::acc_t acc_t;
   acc_t* red = reinterpret_cast<acc_t*>(lds) + (wave & 3) * 2 * TN * 64 + lane;

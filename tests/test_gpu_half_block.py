@@ -64,6 +64,13 @@ def test_half_linear_with_its_epilogues(M, N, K, epi, tile, dtype):
     assert ((outs[0].double() - ref).abs() <= bound * 1.0001).all()
 
 
+# as few k tiles of 64 values as there are stages (tile 3: five, else four) and one to three more, both sides of the touched weights (32)
+@pytest.mark.parametrize("K", [320, 384, 448, 512, 1984, 2048, 2112])
+@pytest.mark.parametrize("tile", [3, 4, 5])
+def test_split_half_linear_at_the_ends_of_its_loop(tile, K):
+    test_half_linear_with_its_epilogues(301, 32 * tile + 40, K, 2, tile, torch.bfloat16)
+
+
 def test_half_linear_leaves_what_it_does_not_take():
     from samfast_amd import ops
     linear = torch.nn.Linear(1024, 4096, device="cuda", dtype=torch.bfloat16).requires_grad_(False)
