@@ -310,30 +310,36 @@ __global__ __launch_bounds__(64 * kSmallWaves, 2) void gemm_i8_skinny_kernel(Sma
 bool linear_i8_small_any_alignment(int64_t M, int K) { return M <= 8 || (M <= 16 && K <= 2048) || (M <= 32 && K <= 768); }
 
 // Rows per wavefront * 8 + column tiles (16 columns each; 2:4: 32) of a workgroup; 0 = not this form.
-// A call of one launch costs the host 6.3 us, of two 9.7, whatever the GPU does meanwhile; on the GPU every workgroup quantises its
-// rows (8 of 768: 0.5 us, of 3072: 3), so the form ends where that repetition, or a second workgroup on a CU, makes it longer than the
-// quantiser and the small-tile product by more than about a microsecond.  GPU time in us, two launches / one (shape):
-//   int8  24 x 768 -> 2304 5.8 / 4.4 (8 rows, 2 tiles), 64 x 1024 -> 1024 6.1 / 4.9, 128 x 1024 -> 1024 6.6 / 5.5 (4 tiles), 256 x 1024 -> 1024 6.9 /
-//         6.9 (16 rows, 4), 192 x 1280 -> 1280 7.6 / 8.2 (16, 4), 256 x 768 -> 768 6.4 / 6.7 (8, 4), 64 x 2048 -> 1024 6.5 / 7.2 (8, 2); beyond: 384 x
-//         1024 -> 1024 8.0 / 9.3, 96 x 2048 -> 1024 7.3 / 8.9, 12 x 3072 -> 768 7.1 / 8.0, 256 x 1280 -> 1280 8.5 / 11.3
-//   2:4   64 x 768 -> 768 7.1 / 4.6, 128 x 1024 -> 1024 7.8 / 6.1, 96 x 1280 -> 1280 7.9 / 7.3, 64 x 2048 -> 1024 8.1 / 6.8, 64 x 3072 -> 768 9.1 / 9.1;
-//         beyond: 256 x 1024 -> 1024 7.7 / 8.1, 128 x 1280 -> 1280 8.0 / 9.1, 48 x 4096 -> 1024 10.2 / 10.0 (rows at or past M cost less: 4 x 5120 -> 1280 8.5 / 7.7), 96 x 2048 -> 1024 8.0 / 8.5
+// A call of one launch costs the host 4.5 to 6.3 us, of two 7.3 to 9.7, whatever the GPU does meanwhile; on the GPU every workgroup quantises its
+// rows, so the form ends where that repetition, or another workgroup on a CU, makes it longer than the quantiser and the small-tile
+// product.  GPU time in us, two launches / one (shape), at the last calls of each line and beyond:
+//   int8, one column tile  up to 256 tiles, at any length 9 x 5120 -> 1280 8.2 / 6.5, 22 x 5120 -> 1280 8.4 / 6.6, 40 x 3072 -> 768 7.1 / 5.3, 58 x 2560 -> 264 6.6 / 5.0,
+//         12 x 3072 -> 768 6.6 / 5.0; with rows of up to 1024 values three on a CU are ahead of wider ones (four column tiles / one: 168 x 1024 -> 488 5.0 / 4.7, 203 x 768 -> 424 4.6 / 4.4,
+//         259 x 384 -> 288 3.9 / 3.65; 780 tiles: 158 x 1024 -> 624 5.10 / 5.13, 200 x 768 -> 512 4.6 / 4.8; at 1152 to 1536 values level)
+//   two column tiles  up to 256 tiles and 4096 values 254 x 2304 -> 240 7.0 / 5.7, 124 x 2816 -> 496 7.0 / 6.3, 120 x 3072 -> 512 7.2 / 6.5, 144 x 3584 -> 432 7.8 / 7.2, 51 x
+//         4096 -> 840 7.75 / 7.7; beyond: 67 x 2816 -> 1048 (297) 8.1 / 8.9, 32 x 5120 -> 1280 8.3 / 8.7; up to 512 short rows 223 x 256 -> 520 3.8 / 3.65 (four column tiles / two)
+//   others  128 x 1024 -> 1024 6.6 / 5.5 (4 tiles), 256 x 1024 -> 1024 6.9 / 6.9 (16 rows, 4)
+//   2:4   to 2048 values up to 1024 tiles 117 x 1024 -> 2064 6.95 / 5.6, 165 x 1280 -> 1504 7.9 / 6.5, 174 x 1536 -> 1000 7.6 / 6.2, 318 x 1792 -> 776 8.3 / 7.5, 258 x 2048 -> 976 10.2 / 7.6;
+//         beyond: 109 x 768 -> 2992 (1316) 6.15 / 6.6, 251 x 1280 -> 1304 (1312) 7.9 / 8.5; to 3072 up to 512 290 x 2560 -> 352 9.1 / 6.7, 90 x 3072 -> 1304 9.0 / 7.4; beyond: 42 x 2304 -> 2984
+//         (564) 8.2 / 8.8; else up to 256 31 x 5120 -> 1280 10.4 / 6.3, 48 x 4096 -> 1024 9.0 / 6.6; beyond: 119 x 3328 -> 680 (330) 9.1 / 11.4
 //   Up to four short rows are quantised in no time, and two column tiles on more workgroups than CUs are ahead of four: 1 x 256 -> 8200 3.07 / 3.64 (two / four),
 //         4 x 128 -> 10240 3.2 / 3.5, 1 x 512 -> 16384 3.83 / 3.98, 1 x 1024 -> 8200 4.46 / 4.75; but 8 x 256 -> 10240 3.8 / 3.6, 4 x 768 -> 12288 4.8 / 4.5.
-// A call, launches included (7 x 256 -> 2048 6.7 us a call, two launches 8.7): 64 x 1024 -> 1024 9.8 / 6.4, 2:4 64 x 1024 -> 1024 9.8 / 6.4.
+// A call, launches included: 64 x 1024 -> 1024 9.8 / 6.4, 12 x 3072 -> 768 7.5 / 5.6, 2:4 48 x 5120 -> 1280 10.8 / 6.3, 16 x 4096 -> 1024 8.7 / 6.8.
 // (A forced tile of the band kernel turns this form off.)
 static int small_shape(int64_t M, int N, int K, bool sparse) {
   if (knob_or(KNOB_LINEAR_SMALL, 1) <= 0 || knob_or(KNOB_LINEAR_BAND, 1) > 1 || K % 64 != 0 || N % 8 != 0 || N <= 0 || K <= 0 || K > 5120 || M <= 0 || M > 4096) return 0;
   const int64_t eights = (M + 7) / 8;
   if (sparse) {
     const int64_t tiles = eights * ((N + 31) / 32);
-    return K % 128 == 0 && K >= 256 && (K <= 3072 || M <= 4) && tiles <= (K <= 1024 ? 768 : K <= 1536 ? 512 : 256) ? 8 + 1 : 0;
+    return K % 128 == 0 && K >= 256 && tiles <= (K <= 2048 ? 1024 : K <= 3072 ? 512 : 256) ? 8 + 1 : 0;
   }
   auto tiles = [&](int nt) { return eights * ((N + 16 * nt - 1) / (16 * nt)); };
-  if (M <= 8 || K <= 2048) {
-    if (tiles(1) <= 256) return 8 + 1;
+  if (tiles(1) <= 256) return 8 + 1;
+  if (M <= 8 || K <= 4096) {
     if (tiles(2) <= 256) return 8 + 2;
     if (M <= 4 && (K <= 512 || tiles(2) <= 288)) return 8 + 2;
+    if (M > 8 && K <= 1024 && tiles(1) <= 768) return 8 + 1;
+    if (M > 8 && K <= 512 && tiles(2) <= 512) return 8 + 2;
     if (K <= 1536 && tiles(4) <= 256) return 8 + 4;
     if (M <= 8) return 8 + 2;
   }

@@ -807,6 +807,15 @@ def test_the_lines_of_a_linear_in_one_launch_on_wide_tiles():
         assert one(*call) == taken, call
 
 
+def test_the_lines_of_a_linear_in_one_launch_over_few_rows():
+    """Both sides of each line of long rows (shorter ones may be the band's): (M, N, K, layout, one launch)."""
+    from samfast_amd import _lib
+    one = _lib.load().samfast_linear_i8_one_launch
+    for *call, taken in ((24, 1280, 5120, 0, 1), (32, 1280, 5120, 0, 0), (64, 1024, 4096, 0, 1), (65, 1024, 4096, 0, 0), (64, 1024, 4160, 0, 0), (128, 512, 2112, 1, 1), (129, 512, 2112, 1, 0),
+                         (256, 1024, 2048, 2, 1), (257, 1024, 2048, 2, 0), (128, 1024, 3072, 2, 1), (129, 1024, 3072, 2, 0), (64, 1024, 5120, 2, 1), (65, 1024, 5120, 2, 0)):
+        assert one(*call) == taken, call
+
+
 @pytest.mark.parametrize("M,N,K", [(8, 1024, 1024), (64, 1024, 1024), (4096, 3072, 768), (5000, 1280, 5120)])  # few rows, more, a band, two launches
 def test_a_linear_of_another_type_is_unsupported_in_every_form(M, N, K):
     from samfast_amd import _lib
