@@ -294,10 +294,10 @@ class Block(nn.Module):
                 tokens, hq, sh = attn.proj.linear_fused_quant(oq, so, _lib.EPILOGUE_RESIDUAL, residual=tokens,
                                                               layout=L, ln=norm2, out_layout=L)
         # lin1, GELU, lin2's quantiser, lin2 + `x + mlp(...)` (+ the next block's norm1 and quantiser).  GELU runs in the
-        # quantiser, except where lin1 is short: there the product hides some of it and the quantiser nothing
-        # (lin1 + quantiser, us, GELU in lin1 / in the quantiser: 4096 x 1280 51.7 / 47.4, 65536 x 1280 661 / 601, 65536 x 768 335 /
-        # 313; but 20480 x 768 105 / 107, and a ViT-B image 1693 / 1746 for all twelve blocks)
-        if quant.FUSED_QUANT or (C < 1024 and tokens.shape[0] < 32768):
+        # quantiser, which waits for memory, except where an image's lin1 is short (lin1 + quantiser, us, GELU in lin1 / in the quantiser:
+        # 8192 x 768 45.9 / 42.7, 12288 x 768 66.6 / 57.8, 4096 x 1024 34.9 / 31.4, 4096 x 1280 51.7 / 47.4, 65536 x 1280 661 / 601, 65536 x
+        # 768 335 / 313, 4096 x 768 29.1 / 28.1; all twelve blocks of a ViT-B, one image 1404 / 1412, two 2261 / 2222, five 4897 / 4722)
+        if quant.FUSED_QUANT or (C < 1024 and tokens.shape[0] < 8192):
             _, gq, sg = mlp.lin1.linear_fused_quant(hq, sh, _lib.EPILOGUE_GELU, layout=L, out_layout=L)
         else:
             gq, sg = ops.quant_rowwise(mlp.lin1.linear_fused(hq, sh, _lib.EPILOGUE_NONE, layout=L), layout=L, gelu=True)
