@@ -4,7 +4,7 @@
 
 namespace samfast {
 
-// The kernel for a product: columns / 32 of a tile; 8 and 10 the resident kernel (kHalfTall: with 320 rows and 256 columns), 3 to 5 the
+// The kernel for a product: columns / 32 of a tile; 6, 8 and 10 the resident kernel (kHalfTall: with 320 rows and 256 columns), 3 to 5 the
 // split one, 0 none (the library's product and a pass of its own for GELU or residual are ahead).  The lines, by the rounds of the
 // CUs and the share of their time that makes output (us, library with its pass / here, residuals with the LayerNorm behind them):
 //   GELU: from half of the CUs on.  4096 x 768 -> 3072 34.2 / 27.6, 4096 x 1280 -> 5120 77.1 / 50.1, 20480 x 1024 -> 4096 188 / 152,
@@ -29,7 +29,7 @@ static int half_choose(int64_t M, int N, int K, int epi) {
   if (force <= 0 || K % 64 != 0 || K < 320 || M < 256 || N < 96) return 0;
   if (force == kHalfTall) return epi == PP_RESIDUAL && N >= 256 && M >= 320 ? force : 0;
   if (force >= 3) {
-    const bool built = (force <= 5 || force == 8 || (force == 10 && epi != PP_RESIDUAL)) && N >= 32 * force;
+    const bool built = (force <= 5 || force == 8 || ((force == 6 || force == 10) && epi != PP_RESIDUAL)) && N >= 32 * force;
     return built ? force : 0;
   }
   if (epi == PP_RESIDUAL)
@@ -42,7 +42,10 @@ static int half_choose(int64_t M, int N, int K, int epi) {
   bool pays = c.used >= 0.5;
   if (epi == PP_PLAIN) pays = c.used >= 0.7 && (c.rounds <= 8 || K >= 1024);
   if (epi == PP_RESIDUAL) pays = c.tm == 5 ? c.used >= 0.8 : K >= 2048 ? c.rounds == 1 && c.used >= 0.7 : c.rounds <= 4 && c.used >= 0.55;
-  return pays ? (c.tm == 5 ? kHalfTall : c.tn) : 0;
+  if (!pays) return 0;
+  if (c.tm == 5) return kHalfTall;
+  // (192 columns are no reason to leave the library's product, whose order of K is another: all of these sum in the same one)
+  return epi == PP_RESIDUAL ? c.tn : pp_choose(M, N, K / 64, false, true).tn;
 }
 
 template <class E>
@@ -55,13 +58,13 @@ static int half_launch(PPArgs a, int tn, int epi, hipStream_t stream) {
     return check_launch("gemm_pingpong_kernel");
   }
   a.tiles_n = (a.N + 32 * tn - 1) / (32 * tn);
-  if (tn >= 8) {
+  if (tn >= 6) {
     a.tiles_m = (a.M + 255) / 256;
     const dim3 grid(pp_grid(a));
 #define SF_PP(EPI, TN) hipLaunchKernelGGL((gemm_pingpong_kernel<E, EPI, TN, false>), grid, dim3(512), 0, stream, a)
-    if (epi == PP_GELU) { if (tn == 8) SF_PP(PP_GELU, 8); else SF_PP(PP_GELU, 10); }
+    if (epi == PP_GELU) { if (tn == 6) SF_PP(PP_GELU, 6); else if (tn == 8) SF_PP(PP_GELU, 8); else SF_PP(PP_GELU, 10); }
     else if (epi == PP_RESIDUAL) SF_PP(PP_RESIDUAL, 8);
-    else { if (tn == 8) SF_PP(PP_PLAIN, 8); else SF_PP(PP_PLAIN, 10); }
+    else { if (tn == 6) SF_PP(PP_PLAIN, 6); else if (tn == 8) SF_PP(PP_PLAIN, 8); else SF_PP(PP_PLAIN, 10); }
 #undef SF_PP
     return check_launch("gemm_pingpong_kernel");
   }

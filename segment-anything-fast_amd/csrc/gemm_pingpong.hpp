@@ -1,5 +1,5 @@
 // One matrix product y = x . w^T for the element types of this library (int8, bf16, fp16): output tiles of 256 rows and 256 or 320
-// columns, or 320 rows and 256 columns, one resident workgroup of eight wavefronts per CU, two per SIMD that take turns at the matrix pipe.
+// columns, or 320 rows and 256 columns (half types also 256 rows and 192 columns), one resident workgroup of eight wavefronts per CU, two per SIMD that take turns at the matrix pipe.
 //
 // What bounds it, at 65536 x 1280 -> 3840 in int8 (265 us; 197 on all-zero codes, where no power limit acts): the products
 // alone are 163 us at the rate that bare loops of the same instruction sustain under the power limit on codes like an encoder's
@@ -94,7 +94,7 @@ SF_DEVICE void pp_wait() {
 // element e of a quad q is column 64 q + 4 lr + e of the half, of the pair 64 NQ + 2 lr + e.
 template <int TN, int TM>
 struct PPTile {
-  static_assert((TN == 8 || TN == 10) && TM + TN / 2 <= 9 && TM >= 4, "tiles built: 256 x {256, 320}, 320 x 256");
+  static_assert((TN == 6 || TN == 8 || TN == 10) && TM + TN / 2 <= 9 && TM >= 4, "tiles built: 256 x {192, 256, 320}, 320 x 256");
   static constexpr int BM = 64 * TM, BN = 32 * TN, H = TN / 2;
   static constexpr int NQ = TN / 4;
   static constexpr bool PAIR = TN % 4 != 0;
@@ -105,10 +105,13 @@ struct PPTile {
   static_assert(2 * STAGE + SCALES <= 160 * 1024, "LDS of a CU");
   static_assert(NLOADS + NSTORES < 64, "vmcnt threshold");
   // column of the half that fragment j of a turn holds in its row r
-  static SF_DEVICE int column(int turn, int j, int r) { return j < 4 ? 64 * turn + 4 * r + j : 64 * NQ + 2 * r + turn; }
+  static SF_DEVICE int column(int turn, int j, int r) {
+    if (TN == 6) return 3 * turn + j < 4 ? 4 * r + 3 * turn + j : 64 + 2 * r + 3 * turn + j - 4;  // (the quad's last element is the second turn's)
+    return j < 4 ? 64 * turn + 4 * r + j : 64 * NQ + 2 * r + turn;
+  }
   // fragment (of both turns) of element e of quad q / of the pair
   static constexpr int quad(int q, int e) { return q * H + e; }
-  static constexpr int pair(int e) { return e * H + H - 1; }
+  static constexpr int pair(int e) { return TN == 6 ? 4 + e : e * H + H - 1; }
 };
 
 // NT: non-temporal stores
@@ -228,8 +231,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
         __builtin_amdgcn_global_load_lds((gptr_t)(src + q + lane), (lptr_t)(sc + dst), 4, 0, 0);
       }
     } else {
-      // columns in pairs (N is even); 320 columns are two and a half slices: they overlap
-      const int q = P::BN == 320 ? (wave % 3) * 96 : (wave & 1) * 128;
+      // columns in pairs (N is even); 320 columns are two and a half slices, 192 one and a half: they overlap
+      const int q = P::BN == 320 ? (wave % 3) * 96 : (wave & 1) * (P::BN - 128);
       if (a.bias) __builtin_amdgcn_global_load_lds((gptr_t)(reinterpret_cast<const unsigned short*>(a.bias) + n0 + q + 2 * lane), (lptr_t)(sc + q * 2), 4, 0, 0);
     }
   };
@@ -769,7 +772,10 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_split_kernel(PPArgs a) {
 // six) 151 / 139, 24576 x 1280 -> 5120 (eight / six) 145 / 138, but 24576 x 1280 -> 3840 (six / five) 110.5 / 112.4, at equal numbers of columns
 // per CU 65536 x 1280 -> 3840 276 / 275; loops under ten k tiles pay more for the wide tile's end: 24576 x 768 -> 3072 (five / four)
 // 64.4 / 70.3, 24576 x 1024 -> 3072 (five / four) 77.7 / 81.3, 12288 x 1024 -> 3072 (three / two) 44.4 / 42.1.  bf16 12288 x 1280 -> 5120 (four / three) 141 / 134,
-// 24576 x 1280 -> 5120 276 / 261, but 24576 x 1024 -> 3072 121 / 124.  (192 columns, at an equal number of columns per CU, lost.)
+// 24576 x 1280 -> 5120 276 / 261, but 24576 x 1024 -> 3072 121 / 124.
+// `narrow`: 192 columns as well (built for the half types without residual), 0.81 of a round of 256 (0.88 of the first).  bf16, 256 / 192, rounds: 4096 x 768 -> 3072 with
+// GELU (one / one) 27.0 / 23.9, 4096 x 1024 -> 3072 25.9 / 23.7, 8192 x 768 -> 3072 with GELU (two / two) 45.6 / 40.0, 28672 x 1024 -> 3072 (six / seven) 141 / 133; but 20480 x 1024 ->
+// 3072 (four / five) 96.7 / 96.9, 32768 x 768 -> 3072 with GELU (six / eight) 145 / 152; 320 / 192: 12288 x 1024 -> 3072 (two / three) 61.0 / 58.5, but 24576 x 768 -> 2304 (three / five) 73.1 / 73.4.
 // The residual's registers leave no room for 320 columns, but for 320 rows, which few columns and many rows fill better.  256 / 320
 // rows: int8 20480 x 4096 -> 1024 (two rounds / one) 89.2 / 67.6, 24576 x 3072 -> 768 69.6 / 51.0, 57344 x 4096 -> 1024 (four / three) 215 /
 // 203, 57344 x 5120 -> 1280 (five / four) 315 / 313, bf16 696 / 622; in equal rounds 16384 x 4096 -> 1024 bf16 103 / 112.
@@ -778,7 +784,7 @@ struct PPChoice {
   int64_t rounds;
   double used;
 };
-static inline PPChoice pp_choose(int64_t M, int N, int nk, bool residual) {
+static inline PPChoice pp_choose(int64_t M, int N, int nk, bool residual, bool narrow = false) {
   PPChoice best = {0, 0, 0, 0.0};
   double least = 0.0;
   auto candidate = [&](int tm, int tn, double fragments) {
@@ -793,6 +799,7 @@ static inline PPChoice pp_choose(int64_t M, int N, int nk, bool residual) {
   candidate(4, 8, 10.0);
   if (residual) candidate(5, 8, 12.4);
   else candidate(4, 10, nk < 10 ? 13.2 : 12.5);
+  if (narrow) candidate(4, 6, 8.1);
   return best;
 }
 
