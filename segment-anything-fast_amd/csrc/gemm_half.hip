@@ -24,12 +24,14 @@ namespace samfast {
 // types, follows the batch, as it does with the library's kernels (one ViT-H image: 3-5 split K, five ViT-L images: 320-row tiles, the
 // library in between; 0.016 and 2e-4 of the embedding's norm).  int8 sums are integers: an image comes out the same in any batch.
 constexpr int kHalfTall = 58;  // 320 rows, 256 columns
+constexpr int kHalfNarrow = 192;  // the knob's number for 192 columns
 static int half_choose(int64_t M, int N, int K, int epi) {
   const int force = knob_or(KNOB_GEMM_HALF, 1);
   if (force <= 0 || K % 64 != 0 || K < 320 || M < 256 || N < 96) return 0;
+  if (force == kHalfNarrow) return epi != PP_RESIDUAL && N >= 192 ? 6 : 0;
   if (force == kHalfTall) return epi == PP_RESIDUAL && N >= 256 && M >= 320 ? force : 0;
   if (force >= 3) {
-    const bool built = (force <= 5 || force == 8 || ((force == 6 || force == 10) && epi != PP_RESIDUAL)) && N >= 32 * force;
+    const bool built = (force <= 5 || force == 8 || (force == 10 && epi != PP_RESIDUAL)) && N >= 32 * force;
     return built ? force : 0;
   }
   if (epi == PP_RESIDUAL)

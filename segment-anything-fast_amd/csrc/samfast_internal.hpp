@@ -32,7 +32,7 @@ enum Knob {
   KNOB_GEMM_PERSIST_SKEW, // SAMFAST_GEMM_PERSIST_SKEW: start delay of every second resident workgroup, 64 cycles per k tile
   KNOB_GEMM_PERSIST_PRIO, // SAMFAST_GEMM_PERSIST_PRIO: 0 = no wave priority changes in the persistent kernel
   KNOB_GEMM_PINGPONG,     // SAMFAST_GEMM_PINGPONG: 256-row tiles by turns (gemm_pingpong.hpp), 0 off, 1 where it pays, 2 wherever built
-  KNOB_GEMM_HALF,         // SAMFAST_GEMM_HALF: the half types' products, 0 the library's, 1 ours where they pay; 3, 4, 5 (K halves summed apart), 8, 10: columns / 32 of the tile, 58: 320 x 256; others: the library's
+  KNOB_GEMM_HALF,         // SAMFAST_GEMM_HALF: the half types' products, 0 the library's, 1 ours where they pay; 3, 4, 5 (K halves summed apart), 8, 10: columns / 32 of the tile, 58: 320 x 256, 192: 256 x 192; others: the library's
   KNOB_GEMM_SPLITK,       // SAMFAST_GEMM_SPLITK: 0 off, 1 where it pays (launches that leave the GPU half empty; 2:4: one tile per CU), 2 wherever built
   KNOB_GEMM_ONCE,         // SAMFAST_GEMM_ONCE: 0 = off, 1 where it pays, rows * 16 + columns / 32 = that tile of the one-tile-per-CU kernel
   KNOB_GEMM_STRIP,        // SAMFAST_GEMM_STRIP: 0 = off, 1 where it pays, 2 = wherever built (gemm_i8_strip.hip)
