@@ -47,7 +47,7 @@ static int half_choose(int64_t M, int N, int K, int epi) {
   if (!pays) return 0;
   if (c.tm == 5) return kHalfTall;
   // (192 columns are no reason to leave the library's product, whose order of K is another: all of these sum in the same one)
-  return epi == PP_RESIDUAL ? c.tn : pp_choose(M, N, K / 64, false, true).tn;
+  return epi == PP_RESIDUAL ? c.tn : pp_choose(M, N, K / 64, false, 8.1).tn;
 }
 
 template <class E>

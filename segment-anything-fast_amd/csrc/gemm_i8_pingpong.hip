@@ -25,6 +25,12 @@ static PPArgs pp_args(const GemmArgs& g) {
   return a;
 }
 
+// SAMFAST_GEMM_PINGPONG = 1 chooses among all tiles, 6 takes 192 columns wherever they are built, other numbers the wider ones.
+static PPChoice choose(int epi, int64_t M, int N, int K) {
+  const int mode = knob_or(KNOB_GEMM_PINGPONG, 1);
+  return pp_choose(M, N, K / 128, epi == EPI_RESIDUAL_BF16, mode == 1 ? 8.7 : mode == 6 ? 0.1 : 0.0);
+}
+
 static bool whole_lines(const void* p, int64_t ld) { return reinterpret_cast<uintptr_t>(p) % 128 == 0 && ld % 64 == 0; }
 
 // lines: rows of the output and the residual are whole cache lines (residual products)
@@ -33,8 +39,9 @@ static bool pays(int epi, int K, const PPChoice& c, bool lines) {
   //   plain, K >= 1280, 0.75: 0.78 (5000 rows -> 5120) 43.1 / 38.1, 0.94 (4096 -> 3840) 26.9 / 21.0, 1.0 (65536 -> 3840) 309 / 263,
   //     K = 5120, 1.0 (65536 -> 3840) 1126 / 994; but 0.59 (5000 -> 3840) 30.0 / 37.6
   //   shorter loops, 0.8: 0.84 (12288 x 768 -> 2304) 31.0 / 26.5, 0.9 (8192 x 768 -> 2304) 23.4 / 20.4, 0.84 in four rounds (24576 x 768 -> 2304) 52.3 /
-  //     50.1, 1.0 (4096 x 1024 -> 4096) 23.1 / 20.1; but 0.75 (8192 x 768 -> 3072) 25.7 / 25.8, and 0.75 at K = 1024 (8192 -> 3072, alone 31.0 / 30.2)
-  //     cost an encoder of two images 1 %
+  //     50.1, 1.0 (4096 x 1024 -> 4096) 23.1 / 20.1; but 0.75 (8192 x 768 -> 3072 in 256 columns) 25.7 / 25.8, (4096 x 768 -> 2304 in 192) 15.8 / 16.2.  Tiles of 192
+  //     columns fill rounds that the wider ones leave out: 90 products drawn where they are taken are 0.68 to 0.99 times as long, one of them 1.015 (26317 x 896 -> 1280):
+  //     8192 x 768 -> 3072 25.0 / 22.7, 8192 x 1024 -> 3072 29.6 / 26.6, 2820 x 3584 -> 3840 42.4 / 35.4, 11268 x 3456 -> 2080 96.7 / 65.9, 32355 x 3072 -> 768 72.9 / 60.9
   //   residual, K >= 2048, 0.7, within one round 0.55: 0.56 (12288 x 3072 -> 768) 38.6 / 36.6, 0.62 (8192 x 5120 -> 1280) 59.5 / 54.6, 0.75 (12288 x 4096 ->
   //     1024) 54.1 / 49.8, 1.0 (20480 x 4096 -> 1024, 320 rows) 86.5 / 64.3, (65536 x 5120 -> 1280) 402 / 336, 0.88 (28672 x 5120 -> 1280, 320 rows) 190 /
   //     149; but 0.5 (8192 x 4096 -> 1024) 40.6 / 45.5, 0.66 in two rounds (28672 x 3072 -> 768) 70.4 / 71.1
@@ -59,7 +66,7 @@ bool gemm_i8_pingpong_covers(int epi, const GemmArgs& g) {
   const int mode = knob_or(KNOB_GEMM_PINGPONG, 1);
   if (mode <= 0 || (epi != EPI_SCALE_BIAS_BF16 && epi != EPI_RESIDUAL_BF16) || g.dst_row || g.tile_counters) return false;
   if (g.K % 128 != 0 || !pp_addressable(pp_args(g))) return false;
-  const PPChoice c = pp_choose(g.M, g.N, g.K / 128, epi == EPI_RESIDUAL_BF16);
+  const PPChoice c = choose(epi, g.M, g.N, g.K);
   if (c.tn == 0) return false;
   if (mode >= 2) return true;
   return pays(epi, g.K, c, whole_lines(g.out, g.ldo) && whole_lines(g.residual, g.ld_res));
@@ -67,7 +74,7 @@ bool gemm_i8_pingpong_covers(int epi, const GemmArgs& g) {
 
 int gemm_i8_pingpong_launch(int epi, const GemmArgs& g, hipStream_t stream) {
   PPArgs a = pp_args(g);
-  const PPChoice c = pp_choose(g.M, g.N, a.nk, epi == EPI_RESIDUAL_BF16);
+  const PPChoice c = choose(epi, g.M, g.N, g.K);
   const int tn = c.tn;
   a.group_m = 4;
   a.tiles_m = (a.M + 64 * c.tm - 1) / (64 * c.tm);
@@ -80,6 +87,7 @@ int gemm_i8_pingpong_launch(int epi, const GemmArgs& g, hipStream_t stream) {
   if (epi == EPI_RESIDUAL_BF16 && c.tm == 5)
     hipLaunchKernelGGL((gemm_pingpong_kernel<PPInt8, PP_RESIDUAL, 8, false, 5>), dim3(pp_grid(a)), dim3(512), 0, stream, a);
   else if (epi == EPI_RESIDUAL_BF16) SF_PP(PP_RESIDUAL, 8, false);
+  else if (tn == 6) SF_PP_PLAIN(6);
   else if (tn == 8) SF_PP_PLAIN(8);
   else SF_PP_PLAIN(10);
 #undef SF_PP_PLAIN
@@ -95,5 +103,5 @@ extern "C" int samfast_bench_gemm_i8_turns(int64_t M, int N, int K, int epilogue
   GemmArgs g = {};
   g.M = (int)M; g.N = N; g.K = K; g.ldo = g.ld_res = row_stride;
   const int epi = epilogue == SAMFAST_EPILOGUE_NONE ? EPI_SCALE_BIAS_BF16 : epilogue == SAMFAST_EPILOGUE_RESIDUAL ? EPI_RESIDUAL_BF16 : EPI_GELU_BF16;
-  return gemm_i8_pingpong_covers(epi, g) ? 32 * pp_choose(M, N, K / 128, epi == EPI_RESIDUAL_BF16).tn : 0;
+  return gemm_i8_pingpong_covers(epi, g) ? 32 * choose(epi, M, N, K).tn : 0;
 }

@@ -782,6 +782,14 @@ def test_the_sparse_products_lines():
     assert turns(0, 5120, 1280, none) == -1 and turns(65536, 5120, 1280, none, 5112) == -1
 
 
+def test_the_dense_products_lines_between_widths():
+    """Tiles of 192, 256 and 320 columns by the price of their rounds, 0 for the smaller members: (M, N, K, columns)."""
+    from samfast_amd import _lib
+    for M, N, K, columns in ((4096, 3072, 1024, 192), (4096, 2304, 768, 0), (8192, 3072, 768, 192), (8192, 2304, 768, 320), (12288, 3072, 1024, 192), (12288, 2304, 768, 256),
+                             (28672, 3072, 768, 256), (6144, 3840, 1280, 192), (16384, 3840, 1280, 320), (65536, 3840, 1280, 256)):
+        assert _lib.load().samfast_bench_gemm_i8_turns(M, N, K, _lib.EPILOGUE_NONE, N) == columns, (M, N, K)
+
+
 def test_the_dense_residual_products_lines_where_rows_are_no_whole_lines():
     """Loops under 1280 beyond two rounds are left to the smaller tiles there, others by turns as on whole lines: (M, N, K, columns)."""
     from samfast_amd import _lib

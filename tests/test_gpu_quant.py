@@ -715,6 +715,31 @@ def test_gemm_by_turns_agrees(M, N, K, epi, layout):
             assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("M,N,K,strided", [(256, 192, 640, False), (301, 200, 640, False), (700, 392, 768, True), (4100, 3072, 1024, False), (9001, 1288, 896, True), (45001, 3072, 640, False)])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_gemm_by_turns_of_192_columns_agrees(M, N, K, strided, layout):
+    """One tile, moved back rows and columns, one round, several, streamed; rows of a wider buffer: the bits of the 64 x 128 tiles."""
+    from samfast_amd import _lib, ops
+    print(f"case gemm by turns of 192 columns M={M} N={N} K={K} layout={layout}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    xk = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8, device="cuda")
+    wk = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device="cuda")
+    sx, sw = (torch.rand(n, generator=g, device="cuda") * 1e-2 for n in (M, N))
+    bias = torch.randn(N, generator=g, device="cuda") if M % 2 == 0 else None
+    if layout == _lib.LAYOUT_KB64:
+        xk, wk = ops.to_kb64(xk), ops.to_kb64(wk)
+    out = torch.full((M, N + 24), 7.0, dtype=torch.bfloat16, device="cuda") if strided else None
+    run = lambda **kw: ops.gemm_i8_fused(xk, sx, wk, sw, bias, _lib.EPILOGUE_NONE, layout=layout, **kw)
+    with _lib.knobs(SAMFAST_GEMM_TILE=64, SAMFAST_GEMM_SKINNY=0):
+        want = run()
+    with _lib.knobs(SAMFAST_GEMM_PINGPONG=6, SAMFAST_GEMM_SKINNY=0):
+        assert _lib.load().samfast_bench_gemm_i8_turns(M, N, K, _lib.EPILOGUE_NONE, N) == 192
+        for _ in range(2):
+            got = run() if out is None else run(out=out[:, :N])
+            assert torch.equal(got, want)
+    assert out is None or (out[:, N:] == 7).all()
+
+
 @pytest.mark.parametrize("M,N,pitch", [(128, 384, 384), (300, 400, 400), (129, 1160, 1168), (4096, 3072, 3072), (4900, 2304, 2304), (9000, 776, 776)])
 @pytest.mark.parametrize("layout", [0, 1])
 def test_gelu_strips_agree(M, N, pitch, layout):
