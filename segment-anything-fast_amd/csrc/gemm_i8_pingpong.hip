@@ -25,10 +25,13 @@ static PPArgs pp_args(const GemmArgs& g) {
   return a;
 }
 
-// SAMFAST_GEMM_PINGPONG = 1 chooses among all tiles, 6 takes 192 columns wherever they are built, other numbers the wider ones.
+// SAMFAST_GEMM_PINGPONG = 1 chooses among all tiles, 6 takes 192 columns wherever they fit, other numbers the wider ones.  With the residual short loops have nothing from 192 columns
+// (12288 x 768 -> 768 15.5 / 15.9, 28672 x 768 -> 768 28.6 / 28.8), and below 4096 values two rounds of them are ahead alone (28672 x 3072 -> 768 72.1 / 65.2) but not in an
+// encoder (seven images of ViT-B 7.08 / 7.11 ms; one round, three images 3.40 / 3.38; K = 5120, four of ViT-H 16.99 / 16.66).
 static PPChoice choose(int epi, int64_t M, int N, int K) {
   const int mode = knob_or(KNOB_GEMM_PINGPONG, 1);
-  return pp_choose(M, N, K / 128, epi == EPI_RESIDUAL_BF16, mode == 1 ? 8.7 : mode == 6 ? 0.1 : 0.0);
+  const bool residual = K >= 4096 || (K >= 2048 && (M + 255) / 256 * ((N + 191) / 192) <= 256);
+  return pp_choose(M, N, K / 128, epi == EPI_RESIDUAL_BF16, mode == 6 ? 0.1 : mode != 1 ? 0.0 : epi != EPI_RESIDUAL_BF16 ? 8.7 : residual ? 9.0 : 0.0);
 }
 
 static bool whole_lines(const void* p, int64_t ld) { return reinterpret_cast<uintptr_t>(p) % 128 == 0 && ld % 64 == 0; }
@@ -42,8 +45,9 @@ static bool pays(int epi, int K, const PPChoice& c, bool lines) {
   //     50.1, 1.0 (4096 x 1024 -> 4096) 23.1 / 20.1; but 0.75 (8192 x 768 -> 3072 in 256 columns) 25.7 / 25.8, (4096 x 768 -> 2304 in 192) 15.8 / 16.2.  Tiles of 192
   //     columns fill rounds that the wider ones leave out: 90 products drawn where they are taken are 0.68 to 0.99 times as long, one of them 1.015 (26317 x 896 -> 1280):
   //     8192 x 768 -> 3072 25.0 / 22.7, 8192 x 1024 -> 3072 29.6 / 26.6, 2820 x 3584 -> 3840 42.4 / 35.4, 11268 x 3456 -> 2080 96.7 / 65.9, 32355 x 3072 -> 768 72.9 / 60.9
-  //   residual, K >= 2048, 0.7, within one round 0.55: 0.56 (12288 x 3072 -> 768) 38.6 / 36.6, 0.62 (8192 x 5120 -> 1280) 59.5 / 54.6, 0.75 (12288 x 4096 ->
-  //     1024) 54.1 / 49.8, 1.0 (20480 x 4096 -> 1024, 320 rows) 86.5 / 64.3, (65536 x 5120 -> 1280) 402 / 336, 0.88 (28672 x 5120 -> 1280, 320 rows) 190 /
+  //   residual, K >= 2048, 0.7, within one round of 256 columns 0.55: 0.56 (12288 x 3072 -> 768) 38.6 / 36.6, 0.62 (8192 x 5120 -> 1280) 59.5 / 54.6, 0.75 (12288 x 4096 ->
+  //     1024) 54.1 / 49.8, (192 columns) 0.83 (16384 x 5120 -> 1280) 108 / 96, 0.75 (12288 x 3072 ->
+  //     768) 36.5 / 32.6, but 0.66 (10771 x 3200 -> 768) 31.7 / 32.4, 1.0 (20480 x 4096 -> 1024, 320 rows) 86.5 / 64.3, (65536 x 5120 -> 1280) 402 / 336, 0.88 (28672 x 5120 -> 1280, 320 rows) 190 /
   //     149; but 0.5 (8192 x 4096 -> 1024) 40.6 / 45.5, 0.66 in two rounds (28672 x 3072 -> 768) 70.4 / 71.1
   //   residual, shorter loops, 0.85: 0.94 (20480 x 768 -> 768) 22.4 / 19.8, two rounds (40960 x 768 -> 768) 41.3 / 34.4, 0.88 (28672 x 1024 -> 1024) 43.9 / 38.5, 1.0
   //     (20480 x 1024 -> 1024, 320 rows) 31.9 / 28.4, 0.88 in five rounds (57344 x 1280 -> 1280) 124.2 / 117.2; but 0.75 (24576 x 1024 -> 1024) 35.7 / 37.5, 0.83
@@ -51,7 +55,7 @@ static bool pays(int epi, int K, const PPChoice& c, bool lines) {
   //     Rows that are no whole lines, whose segments each touch two, only within two rounds: 7556 x 1024 -> 1992 31.4 / 28.3, 16384 x 640 -> 1992 47.4 / 44.6; but
   //     four 28672 x 640 -> 1992 72.4 / 78.1, five 14563 x 640 -> 4904 102 / 114, thirteen 40960 x 1024 -> 4904 309 / 321 (28672 x 1280 -> 1992 110 / 101)
   if (epi != EPI_RESIDUAL_BF16) return c.used >= (K >= 1280 ? 0.75 : 0.8);
-  if (K >= 2048) return c.used >= (c.rounds == 1 ? 0.55 : 0.7);
+  if (K >= 2048) return c.used >= (c.rounds == 1 && c.tn != 6 ? 0.55 : 0.7);
   if (K < 1280 && c.rounds > 2 && !lines) return false;
   return c.used >= (K >= 1280 && c.rounds <= 2 ? 0.77 : 0.85);
 }
@@ -86,6 +90,7 @@ int gemm_i8_pingpong_launch(int epi, const GemmArgs& g, hipStream_t stream) {
 #define SF_PP_PLAIN(TN) do { if (nt) SF_PP(PP_PLAIN, TN, true); else SF_PP(PP_PLAIN, TN, false); } while (0)
   if (epi == EPI_RESIDUAL_BF16 && c.tm == 5)
     hipLaunchKernelGGL((gemm_pingpong_kernel<PPInt8, PP_RESIDUAL, 8, false, 5>), dim3(pp_grid(a)), dim3(512), 0, stream, a);
+  else if (epi == EPI_RESIDUAL_BF16 && tn == 6) SF_PP(PP_RESIDUAL, 6, false);
   else if (epi == EPI_RESIDUAL_BF16) SF_PP(PP_RESIDUAL, 8, false);
   else if (tn == 6) SF_PP_PLAIN(6);
   else if (tn == 8) SF_PP_PLAIN(8);

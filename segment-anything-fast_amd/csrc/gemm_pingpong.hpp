@@ -1,5 +1,5 @@
 // One matrix product y = x . w^T for the element types of this library (int8, bf16, fp16): output tiles of 256 rows and 256 or 320
-// columns, or 320 rows and 256 columns (without a residual also 256 rows and 192 columns), one resident workgroup of eight wavefronts per CU, two per SIMD that take turns at the matrix pipe.
+// columns, or 320 rows and 256 columns (int8, and the half types without a residual, also 256 rows and 192 columns), one resident workgroup of eight wavefronts per CU, two per SIMD that take turns at the matrix pipe.
 //
 // What bounds it, at 65536 x 1280 -> 3840 in int8 (265 us; 197 on all-zero codes, where no power limit acts): the products
 // alone are 163 us at the rate that bare loops of the same instruction sustain under the power limit on codes like an encoder's
@@ -773,12 +773,14 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_split_kernel(PPArgs a) {
 // per CU 65536 x 1280 -> 3840 276 / 275; loops under ten k tiles pay more for the wide tile's end: 24576 x 768 -> 3072 (five / four)
 // 64.4 / 70.3, 24576 x 1024 -> 3072 (five / four) 77.7 / 81.3, 12288 x 1024 -> 3072 (three / two) 44.4 / 42.1.  bf16 12288 x 1280 -> 5120 (four / three) 141 / 134,
 // 24576 x 1280 -> 5120 276 / 261, but 24576 x 1024 -> 3072 121 / 124.
-// `narrow`, unless 0: the price of 192 columns, where they are built (no residual): half types 8.1, int8 8.7 (both less in the first rounds).  256 / 192, rounds, bf16:
+// `narrow`, unless 0: the price of 192 columns, where the caller builds them: half types 8.1, int8 8.7 (both less in the first rounds), with the residual 9.  256 / 192, rounds, bf16:
 // 4096 x 768 -> 3072 with GELU (one / one) 27.0 / 23.9, 4096 x 1024 -> 3072 25.9 / 23.7, 8192 x 768 -> 3072 with GELU (two / two) 45.6 / 40.0, 28672 x 1024 ->
 // 3072 (six / seven) 141 / 133; but 20480 x 1024 -> 3072 (four / five) 96.7 / 96.9, 32768 x 768 -> 3072 with GELU (six / eight) 145 / 152; 320 / 192: 12288 x 1024 -> 3072 (two /
 // three) 61.0 / 58.5, but 24576 x 768 -> 2304 (three / five) 73.1 / 73.4.  int8, the smaller members / 192: 8192 x 768 -> 3072 25.0 / 22.7, 8192 x 1024 -> 3072 29.6 / 26.6, 6144 x
 // 1280 -> 3840 34.1 / 29.1, 4096 x 1024 -> 3072 18.3 / 16.9; 320 / 192 (two / three) 16384 x 768 -> 2304 32.6 / 31.0, 12288 x 1024 -> 3072 38.0 / 36.0; but 256 / 192 (six / seven)
 // 28672 x 768 -> 3072 67.6 / 71.4, (five / six) 32768 x 768 -> 2304 58.8 / 60.1.
+// With the residual, int8: 16384 x 5120 -> 1280 (two / two) 108 / 96, 12288 x 3072 -> 768 (one / one) 36.5 / 32.6, 8192 x 5120 -> 1280 52.5 / 50.6;
+// but 320 rows / 192 columns (one / two) 24576 x 3072 -> 768 50.2 / 59.2.
 // The residual's registers leave no room for 320 columns, but for 320 rows, which few columns and many rows fill better.  256 / 320
 // rows: int8 20480 x 4096 -> 1024 (two rounds / one) 89.2 / 67.6, 24576 x 3072 -> 768 69.6 / 51.0, 57344 x 4096 -> 1024 (four / three) 215 /
 // 203, 57344 x 5120 -> 1280 (five / four) 315 / 313, bf16 696 / 622; in equal rounds 16384 x 4096 -> 1024 bf16 103 / 112.
@@ -802,7 +804,7 @@ static inline PPChoice pp_choose(int64_t M, int N, int nk, bool residual, double
   candidate(4, 8, 10.0);
   if (residual) candidate(5, 8, 12.4);
   else candidate(4, 10, nk < 10 ? 13.2 : 12.5);
-  if (!residual && narrow > 0.0) candidate(4, 6, narrow);
+  if (narrow > 0.0) candidate(4, 6, narrow);
   return best;
 }
 

@@ -788,6 +788,8 @@ def test_the_dense_products_lines_between_widths():
     for M, N, K, columns in ((4096, 3072, 1024, 192), (4096, 2304, 768, 0), (8192, 3072, 768, 192), (8192, 2304, 768, 320), (12288, 3072, 1024, 192), (12288, 2304, 768, 256),
                              (28672, 3072, 768, 256), (6144, 3840, 1280, 192), (16384, 3840, 1280, 320), (65536, 3840, 1280, 256)):
         assert _lib.load().samfast_bench_gemm_i8_turns(M, N, K, _lib.EPILOGUE_NONE, N) == columns, (M, N, K)
+    for M, N, K, columns in ((12288, 768, 3072, 192), (10700, 768, 3200, 0), (16384, 1280, 5120, 192), (24576, 768, 3072, 256), (32768, 768, 3072, 256), (32768, 768, 768, 0)):
+        assert _lib.load().samfast_bench_gemm_i8_turns(M, N, K, _lib.EPILOGUE_RESIDUAL, N) == columns, (M, N, K)
 
 
 def test_the_dense_residual_products_lines_where_rows_are_no_whole_lines():

@@ -717,7 +717,8 @@ def test_gemm_by_turns_agrees(M, N, K, epi, layout):
 
 @pytest.mark.parametrize("M,N,K,strided", [(256, 192, 640, False), (301, 200, 640, False), (700, 392, 768, True), (4100, 3072, 1024, False), (9001, 1288, 896, True), (45001, 3072, 640, False)])
 @pytest.mark.parametrize("layout", [0, 1])
-def test_gemm_by_turns_of_192_columns_agrees(M, N, K, strided, layout):
+@pytest.mark.parametrize("epi", [0, 2])
+def test_gemm_by_turns_of_192_columns_agrees(M, N, K, strided, layout, epi):
     """One tile, moved back rows and columns, one round, several, streamed; rows of a wider buffer: the bits of the 64 x 128 tiles."""
     from samfast_amd import _lib, ops
     print(f"case gemm by turns of 192 columns M={M} N={N} K={K} layout={layout}", flush=True)
@@ -729,11 +730,12 @@ def test_gemm_by_turns_of_192_columns_agrees(M, N, K, strided, layout):
     if layout == _lib.LAYOUT_KB64:
         xk, wk = ops.to_kb64(xk), ops.to_kb64(wk)
     out = torch.full((M, N + 24), 7.0, dtype=torch.bfloat16, device="cuda") if strided else None
-    run = lambda **kw: ops.gemm_i8_fused(xk, sx, wk, sw, bias, _lib.EPILOGUE_NONE, layout=layout, **kw)
+    res = torch.randn((M, N), generator=g, device="cuda").to(torch.bfloat16) if epi == _lib.EPILOGUE_RESIDUAL else None
+    run = lambda **kw: ops.gemm_i8_fused(xk, sx, wk, sw, bias, epi, layout=layout, residual=res, **kw)
     with _lib.knobs(SAMFAST_GEMM_TILE=64, SAMFAST_GEMM_SKINNY=0):
         want = run()
     with _lib.knobs(SAMFAST_GEMM_PINGPONG=6, SAMFAST_GEMM_SKINNY=0):
-        assert _lib.load().samfast_bench_gemm_i8_turns(M, N, K, _lib.EPILOGUE_NONE, N) == 192
+        assert _lib.load().samfast_bench_gemm_i8_turns(M, N, K, epi, N) == 192
         for _ in range(2):
             got = run() if out is None else run(out=out[:, :N])
             assert torch.equal(got, want)
