@@ -8,15 +8,15 @@
 // workgroups of a head touch its K and V ahead, so that the rows come out of their XCD's L2.
 //   Bound: at 8 x 16 x 4096 x 80 (fp16 785 us, 875 TFLOP/s, bf16 711; attn_global_kernel 803 and 763) the power limit:
 //   the same loop with its MFMAs alone, on the same values, took 666 us - 429 on zeros (probes that are not kept).  At one image of
-//   12 heads (65 us against 82) the last, half-empty round and the prologue.
+//   12 heads (63.8 us against 82) the last, half-empty round and the prologue.
 //   (The encoder, which hands over tables, keeps attn_global_kernel: its int8 Linears turn any other order of these
 //   roundings into other codes.)
 //
-// Two kernels.  attn_global_bias_kernel: a wavefront owns 32 queries and walks whole key rows; workgroups of 8 (one
+// Three kernels.  attn_global_bias_kernel: a wavefront owns 32 queries and walks whole key rows; workgroups of 8 (one
 // per CU: every row staged once for 256 queries) or 4 wavefronts (two per CU).  attn_global_split_kernel: the keys
 // of every row are split between two wavefronts, whose results (maximum reference, denominator, output) meet in
 // LDS once, at the end; workgroups of two query tiles x two key halves (64 queries, under 54 KB of LDS), three per CU
-// at hd 64, so that one image's 12 heads are 768 workgroups: three on each of the 256 CUs, where 128-query
+// at hd 64 (attn_global_split16_kernel, on the smaller matrix instruction), so that one image's 12 heads are 768 workgroups: three on each of the 256 CUs, where 128-query
 // workgroups leave half of the CUs with one and half with two.  bias_form picks, by head_dim: the two kernels round
 // differently, and a slice's bits are not to depend on the batch.
 #include "attn_relpos_shared.hpp"
@@ -650,6 +650,297 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
     }
 }
 
+// The split form at hd 64 on 16 x 16 x 32 matrix instructions: half the accumulator bytes per product cross the register file, which counts because the
+// power limit is what a SIMD's matrix pipe and vector unit share (bare loops on N(0, 0.5) values 1.94 PFLOP/s for 1.77 of the 32 x 32 form).  A lane holds
+// two queries, lane % 16 and 16 more, and of every 16 keys the four from 4 (lane / 16) on; the packed pairs of a half row are the P V
+// operand as they stand, its k slots 8 q .. 8 q + 7 being the keys 4 q .. + 3 and 16 + 4 q .. + 3, and two transposing reads bring V in that order.
+// us, 32 x 32 x 16 / so (bf16; fp16): 1 x 8 heads 51.5 / 49.7; 50.9 / 47.9, 1 x 12 66.0 / 63.8; 69.3 / 66.3, 4 x 12 242 / 232; 259 / 244, 8 x 16 645 / 636; 675 / 658, 9 x 16 x 6 rows
+// of 64 19.2 / 18.1; 18.7 / 18.2.  The error against 64 bits is the same to three digits (2.35e-3, 2.94e-4 of the norm).
+struct Split16Cfg {
+  using R = GridRow<64>;
+  static constexpr int QW = 2, WAVES = 2 * QW, BM = 32 * QW;  // query tiles of 32 and two key halves
+  static constexpr int KTILE = R::KTILE, VTILE = R::VTILE, PW = R::KP / WAVES;  // PW: wave instructions of a tile
+  static constexpr int V_OFF = 2 * KTILE;       // LDS: K tiles of both stages, V tiles of both stages, rel_h
+  static constexpr int RELH_OFF = V_OFF + 2 * VTILE;
+  static constexpr int RH = 32;                 // key rows whose rel_h is at hand
+  static constexpr int LDS_BYTES = RELH_OFF + RH * BM * 4;
+  // V rows are 128 bytes; a transposing read takes 32 of them from each of 16 rows, eight rows at a time: 16-byte piece c of row r stands at c ^ v_swizzle(r)
+  static SF_DEVICE int v_swizzle(int row) { return 2 * ((row >> 1) & 3); }
+  static_assert(R::KP % WAVES == 0 && R::VP == R::KP, "whole wave instructions");
+  static_assert(3 * LDS_BYTES <= 160 * 1024, "three workgroups per CU");
+  static_assert(QW * 64 * 36 * 4 <= RELH_OFF, "the second halves' results");
+};
+
+template <typename T>
+__global__ __launch_bounds__(64 * Split16Cfg::WAVES, 3) void attn_global_split16_kernel(AttnArgs a) {
+  using C = Split16Cfg;
+  constexpr int HD = 64;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS_BYTES];
+  float* relhT = reinterpret_cast<float*>(lds + C::RELH_OFF);  // [kh % RH][BM], * log2(e)
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lq = lane >> 4;
+  const int qt = wave & (C::QW - 1), kg = wave / C::QW;  // query tile, key half
+
+  const unsigned int nqb = a.N / C::BM;
+  const unsigned int total = (unsigned int)(a.B * a.nH) * nqb;
+  const unsigned int pid = xcd_contiguous_id(blockIdx.x, total);
+  if (pid >= total) return;
+  const int bh = pid / nqb, qb = pid % nqb;
+  const int b = bh / a.nH, h = bh % a.nH;
+  const int q0 = qb * C::BM + 32 * qt;  // the wavefront's first query: half of one grid row
+
+  const unsigned short* kbase = a.k + b * a.k_sb + h * a.k_sh;
+  const unsigned short* vbase = a.v + b * a.v_sb + h * a.v_sh;
+
+  // ---- K / V rows: global memory -> LDS directly, wave instruction i of a tile fills pieces 64 i .. 64 i + 63 ----
+  unsigned int koff[C::PW], voff[C::PW];  // bytes, from the tile's first key row; unsigned: scalar-base load form
+#pragma unroll
+  for (int m = 0; m < C::PW; ++m) {
+    int row;
+    const int P = 64 * (wave + C::WAVES * m) + lane, at = C::R::k_source(P, row);
+    koff[m] = (unsigned int)(row * (int)a.k_sn) * 2u + at;
+    voff[m] = (unsigned int)(row * (int)a.v_sn) * 2u + ((P % 8) ^ C::v_swizzle(row)) * 16;
+  }
+  const unsigned int lds_base = (unsigned int)(uintptr_t)((__attribute__((address_space(3))) unsigned char*)lds);
+  auto k_dma = [&](int kt, int buf) __attribute__((always_inline)) {
+    const unsigned char* src = reinterpret_cast<const unsigned char*>(kbase + (int64_t)kt * 64 * a.k_sn);
+#pragma unroll
+    for (int m = 0; m < C::PW; ++m) lds_dma16(src, koff[m], lds_base + buf * C::KTILE + (wave + C::WAVES * m) * 1024);
+  };
+  auto v_dma = [&](int kt, int buf) __attribute__((always_inline)) {
+    const unsigned char* src = reinterpret_cast<const unsigned char*>(vbase + (int64_t)kt * 64 * a.v_sn);
+#pragma unroll
+    for (int m = 0; m < C::PW; ++m) lds_dma16(src, voff[m], lds_base + C::V_OFF + buf * C::VTILE + (wave + C::WAVES * m) * 1024);
+  };
+  k_dma(0, 0);
+  v_dma(0, 0);
+  k_dma(1, 1);  // N % 128 == 0: at least two key rows
+  v_dma(1, 1);
+  // operand reads of this wavefront's key half: K row lr, channels 32 s + 8 lq .. +7; V keys 4 lq + lr / 4, channels 16 ct + 4 (lr % 4) .. +3
+  int krd[2], vrd[4];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) krd[s] = (32 * kg + lr) * 128 + ((4 * s + lq) ^ C::R::k_swizzle(lr)) * 16;
+  {
+    const int key = 4 * lq + (lr >> 2);
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct)
+      vrd[ct] = C::V_OFF + (32 * kg + key) * 128 + ((2 * ct + ((lr & 3) >> 1)) ^ C::v_swizzle(key)) * 16 + 8 * (lr & 1);
+  }
+
+  // Each workgroup touches its own share of the head's K and V first (see above).
+  constexpr int NTOUCH = 2 * C::BM * (HD / 8) / (64 * C::WAVES);
+  unsigned int touched[NTOUCH];
+#pragma unroll
+  for (int i = 0; i < NTOUCH; ++i) {
+    const int P = (tid + 64 * C::WAVES * i) % (C::BM * (HD / 8)), row = P / (HD / 8), col = P % (HD / 8);
+    const bool is_v = 2 * i >= NTOUCH;
+    touched[i] = *reinterpret_cast<const unsigned int*>((is_v ? vbase : kbase) + (int64_t)(qb * C::BM + row) * (is_v ? a.v_sn : a.k_sn) + col * 8);
+  }
+
+  // ---- Q^T operands: queries lr and 16 + lr, channels 32 s + 8 lq .. +7 ----
+  u32x4 qf[2][2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const unsigned short* qp = a.q + b * a.q_sb + h * a.q_sh + (int64_t)(q0 + 16 * t + lr) * a.q_sn + 8 * lq;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) qf[t][s] = load_x8_global(qp + 32 * s);
+  }
+  // rel_h of key rows kh0 .. kh0 + 31, shared by the two key halves
+  auto fill_relh = [&](int kh0) __attribute__((always_inline)) {
+    const unsigned short* rhb = a.rh + b * a.rh_sb + h * a.rh_sh + (int64_t)(qb * C::BM) * a.rh_sn;
+    const int ql = tid / 4, part = tid % 4;  // 64 queries x 4 pieces of 8 key rows
+    static_assert(C::BM * 4 == 64 * C::WAVES, "one piece per thread");
+    unsigned short v8[8];
+    const unsigned short* src = rhb + (int64_t)ql * a.rh_sn + kh0 + 8 * part;
+    if (a.relh_x8) {
+      *reinterpret_cast<u32x4*>(v8) = load_x8_global(src);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v8[e] = kh0 + 8 * part + e < a.gh ? src[e] : (unsigned short)0;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) relhT[(8 * part + e) * C::BM + ql] = T::from_bits(v8[e]) * kLog2e;
+  };
+
+  // ---- rel_w / sm_scale of this wavefront's keys, the initial accumulator of every score tile: [16 keys][16 queries] ----
+  f32x4 b1[2][2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const unsigned short* rwp = a.rw + b * a.rw_sb + h * a.rw_sh + (int64_t)(q0 + 16 * t + lr) * a.rw_sn + 32 * kg + 4 * lq;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const u32x2 w = *reinterpret_cast<const u32x2*>(rwp + 16 * k);
+      b1[k][t] = f32x4{T::lo(w[0]) * a.inv_scale, T::hi(w[0]) * a.inv_scale, T::lo(w[1]) * a.inv_scale, T::hi(w[1]) * a.inv_scale};
+    }
+  }
+  fill_relh(0);
+#pragma unroll
+  for (int i = 0; i < NTOUCH; ++i) asm volatile("" : : "v"(touched[i]));
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of tile 0 has landed
+  __syncthreads();
+
+  // ---- main loop over key grid rows, pipelined inside a wavefront as attn_global_split_kernel's ----
+  f32x4 oacc[4][2];
+#pragma unroll
+  for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) oacc[ct][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_i[2] = {T::kLowest, T::kLowest}, l_i[2] = {0.f, 0.f};
+
+  const int nkt = a.N / 64;
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4* trptr_t;
+  struct Scores { f32x4 v[2][2]; };  // [16 keys][16 queries]
+  u32x4 kf[2][2], vf[4], pkA[2], pkB[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) pkA[t] = pkB[t] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int ct = 0; ct < 4; ++ct) vf[ct] = u32x4{0u, 0u, 0u, 0u};
+  auto read_k = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) kf[k][s] = *reinterpret_cast<const u32x4*>(lds + krd[s] + buf * C::KTILE + k * 16 * 128);
+  };
+  auto read_v = [&](int ct, int buf) __attribute__((always_inline)) {
+    const unsigned char* p = lds + vrd[ct] + buf * C::VTILE;
+    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((trptr_t)p));
+    const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((trptr_t)(p + 16 * 128)));
+    vf[ct] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+  };
+  // instruction n of the eight of a half row's scores (both of a k step's key tiles before the next step) / of its P V
+  auto score = [&](Scores& s, int n) __attribute__((always_inline)) {
+    const int ks = n >> 2, k = (n >> 1) & 1, t = n & 1;
+    s.v[k][t] = T::mfma16(kf[k][ks], qf[t][ks], ks == 0 ? b1[k][t] : s.v[k][t]);
+  };
+  auto pv = [&](const u32x4 (&pk)[2], int n) __attribute__((always_inline)) { oacc[n >> 1][n & 1] = T::mfma16(vf[n >> 1], pk[n & 1], oacc[n >> 1][n & 1]); };
+  auto row = [&](int kt, auto buf_c, Scores& s, Scores& s_next, u32x4 (&pk)[2], u32x4 (&pk_prev)[2]) __attribute__((always_inline)) {
+    constexpr int BUF = decltype(buf_c)::value;  // kt & 1, for constant LDS offsets
+    if (kt == C::RH) {  // uniform; everybody has left row kt - 1 (the barrier at its end)
+      fill_relh(kt);
+      __syncthreads();
+    }
+    const float* rh = relhT + (kt % C::RH) * C::BM + 32 * qt + lr;
+    const float b0[2] = {rh[0], rh[16]};
+    read_k(BUF ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (kt + 2 < nkt) k_dma(kt + 2, BUF);  // row kt's scores are made: its K buffer is free
+    __builtin_amdgcn_sched_barrier(0);
+
+    float neg_mrow[2] = {b0[0] - m_i[0], b0[1] - m_i[1]};
+    float l0[2] = {0.f, 0.f}, l1[2] = {0.f, 0.f};  // this row's share of the denominators, unrounded (two chains each)
+    float e0, e1;  // a pair is packed one step after its exponentials were issued
+    auto gather = [&](int w) __attribute__((always_inline)) {  // pair w: query w / 4, keys 16 (w / 2 % 2) + 4 lq + 2 (w % 2) and one more
+      pk[w >> 2][w & 3] = T::pack2(e0, e1);
+      l0[w >> 2] += e0;
+      l1[w >> 2] += e1;
+    };
+    // (the last row's kf is whatever the buffer holds: its product is not used)
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      const int t = g >> 2, k = (g >> 1) & 1, r = 2 * (g & 1);
+      const float x0 = fmaf(s.v[k][t][r], a.c, neg_mrow[t]), x1 = fmaf(s.v[k][t][r + 1], a.c, neg_mrow[t]);
+      if (g > 0) gather(g - 1);
+      e0 = fast_exp2(x0);
+      e1 = fast_exp2(x1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        if (g < 2) pv(pk_prev, 2 * g + n);
+        else if (g < 6) score(s_next, 2 * (g - 2) + n);
+        else pv(pk_prev, 2 * (g - 4) + n);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // this row's V for the next round
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct) read_v(ct, BUF);
+    gather(7);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) l0[t] += l1[t];
+    if (__any(l0[0] > kCeiling || l0[1] > kCeiling)) {  // move the references, as above
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        float mx = s.v[0][t][0];
+#pragma unroll
+        for (int w = 1; w < 8; ++w) mx = fmaxf(mx, s.v[w >> 2][t][w & 3]);
+        mx = max_with_lane_xor32(fmaxf(mx, __shfl_xor(mx, 16, 64)));
+        const float m_new = fmaxf(m_i[t], fmaf(mx, a.c, b0[t] + T::kMargin));
+        const float alpha = fast_exp2(m_i[t] - m_new);
+        m_i[t] = m_new;
+        l_i[t] *= alpha;
+        neg_mrow[t] = b0[t] - m_new;
+        l0[t] = 0.f;
+#pragma unroll
+        for (int ct = 0; ct < 4; ++ct) oacc[ct][t] *= alpha;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const f32x4 v = s.v[w >> 1][t];
+          const float p0 = fast_exp2(fmaf(v[2 * (w & 1)], a.c, neg_mrow[t])), p1 = fast_exp2(fmaf(v[2 * (w & 1) + 1], a.c, neg_mrow[t]));
+          pk[t][w] = T::pack2(p0, p1);
+          l0[t] += p0 + p1;
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) l_i[t] += l0[t];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of K row kt + 2 and V row kt + 1 has landed
+    __syncthreads();
+    if (kt + 2 < nkt) v_dma(kt + 2, BUF);  // row kt's V is in registers
+  };
+  Scores sA, sB;
+  read_k(0);
+#pragma unroll
+  for (int n = 0; n < 8; ++n) score(sA, n);
+  __syncthreads();  // K row 0 has been read by everyone: its buffer may be refilled
+  for (int kt = 0; kt < nkt; kt += 2) {  // nkt is even
+    row(kt, std::integral_constant<int, 0>{}, sA, sB, pkA, pkB);
+    row(kt + 1, std::integral_constant<int, 1>{}, sB, sA, pkB, pkA);
+  }
+#pragma unroll
+  for (int n = 0; n < 8; ++n) pv(pkB, n);  // of the last row
+
+  // ---- the two key halves meet: references, denominators and accumulators of half 1 through LDS ----
+  float* other = reinterpret_cast<float*>(lds) + qt * 64 * 36 + lane;  // word w of lane: 64 w + lane
+  if (kg == 1) {
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) other[64 * (8 * ct + 4 * t + r)] = oacc[ct][t][r];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      other[64 * (32 + t)] = m_i[t];
+      other[64 * (34 + t)] = l_i[t];
+    }
+  }
+  __syncthreads();
+  if (kg == 1) return;
+  unsigned short* op = a.out + b * a.o_sb + h * a.o_sh + (int64_t)(q0 + lr) * a.o_sn;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    // (a half all of whose keys are taken away: its reference is T::kLowest, its sums are zero)
+    const float m1 = other[64 * (32 + t)], l1 = other[64 * (34 + t)];
+    const float m = fmaxf(m_i[t], m1);
+    const float f0 = fast_exp2(m_i[t] - m), f1 = fast_exp2(m1 - m);
+    float l = l_i[t] * f0 + l1 * f1;
+    l += __shfl_xor(l, 16, 64);
+    l += xor32(l);
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct) {
+      float o[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = (oacc[ct][t][r] * f0 + other[64 * (8 * ct + 4 * t + r)] * f1) * inv;
+      *reinterpret_cast<u32x2*>(op + (int64_t)(16 * t) * a.o_sn + 16 * ct + 4 * lq) = u32x2{T::pack2(o[0], o[1]), T::pack2(o[2], o[3])};
+    }
+  }
+}
+
 // Which form of the global kernel.  Split keys round differently from unsplit ones, so that choice looks at head_dim
 // alone: a slice has the same bits whatever batch it travels in.  hd 64 is split (us, split / unsplit with 8 / with 4
 // wavefronts, 4096 tokens: 1 x 8 heads 48 / 73 / 53, 1 x 12: 66 / 71 / 76, 2 x 9: 102 / 142 / 116, 1 x 16: 87 / 79 / 82,
@@ -674,6 +965,7 @@ static void launch_bias(const AttnArgs& a, int form, hipStream_t stream) {
   auto grid = [&](int queries) { return dim3((unsigned int)(((int64_t)a.B * a.nH * (a.N / queries) + 7) / 8 * 8)); };
   if (form == 8) hipLaunchKernelGGL((attn_global_bias_kernel<T, HD, 8>), grid(256), dim3(512), 0, stream, a);
   else if (form == 4) hipLaunchKernelGGL((attn_global_bias_kernel<T, HD, 4>), grid(128), dim3(256), 0, stream, a);
+  else if constexpr (HD == 64) hipLaunchKernelGGL((attn_global_split16_kernel<T>), grid(64), dim3(256), 0, stream, a);
   else hipLaunchKernelGGL((attn_global_split_kernel<T, HD>), grid(64), dim3(256), 0, stream, a);
 }
 

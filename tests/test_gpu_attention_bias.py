@@ -79,6 +79,28 @@ def test_fp16_probabilities_far_below_the_maximum(form, hd, where):
     assert ((out.cpu().double() - ref).abs() / ref).max() <= 2.0 ** -10 + 2.0 ** -13
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("which", [0, 1])
+@pytest.mark.parametrize("gh", [2, 34, 64])
+def test_every_other_sixteen_queries_move_their_reference(gh, which, dtype):
+    """A lane of the split form has two queries, 16 apart: the logits of one rise along the keys, the other's do not."""
+    from samfast_amd import ops
+    print(f"case two queries gh={gh} which={which} {dtype}", flush=True)
+    q, k, v, rel_h, rel_w = bias_inputs(1, 2, gh, 64, 64, seed=gh + which, dtype=dtype)
+    n = torch.arange(gh * 64)
+    q = (q.float() + 0.5 * (n // 16 % 2 == which)[None, None, :, None]).to(dtype)
+    k = (k.float() + 3.75 * (n / (gh * 64))[None, None, :, None]).to(dtype)
+    out = ops.attn_relpos_bias(q.cuda(), k.cuda(), v.cuda(), rel_h.squeeze(-1).cuda(), rel_w.squeeze(-2).cuda()).double().cpu()
+    qd, kd, vd = q.double(), k.double(), v.double()
+    scores = qd @ kd.transpose(-1, -2) * 0.125 + (rel_h.double().reshape(1, 2, gh * 64, gh, 1) + rel_w.double().reshape(1, 2, gh * 64, 1, 64)).reshape(1, 2, gh * 64, gh * 64)
+    p = torch.softmax(scores, -1)
+    ref, weight = p @ vd, p @ vd.abs()
+    eps = torch.finfo(dtype).eps
+    # probabilities and output rounded to the type, scores and sums in fp32; fp16 probabilities below 2^-14 to 2^-25, the denominator being at least one
+    floor = gh * 64 * 2.0 ** -25 * vd.abs().amax() if dtype == torch.float16 else 0.0
+    assert ((out - ref).abs() <= 0.51 * eps * (weight + ref.abs()) + 1e-4 * weight + floor + 1e-6).all()
+
+
 @pytest.mark.parametrize("hd,dtype", [(64, torch.bfloat16), (80, torch.float16)])
 @pytest.mark.parametrize("gh", [64, 16, 6])
 def test_a_slice_has_the_same_bits_in_any_batch(hd, dtype, gh):
