@@ -29,12 +29,18 @@ extern "C" {
 int samfast_bench_set_knob(const char* name, int value, int unset);
 
 /*
- * Columns of the tile (256 or 320) in which samfast_gemm_i8_fused or samfast_gemm_i8_sparse24_fused forms this output by
+ * Columns of the tile (192, 256 or 320) in which samfast_gemm_i8_fused or samfast_gemm_i8_sparse24_fused forms this output by
  * turns, 0 where the rule leaves it to other kernels: no launch, for rows of the output and the residual
  * `row_stride` elements apart that start on a cache line.  SAMFAST_E_INVALID for a bad shape.
  */
 int samfast_bench_gemm_i8_turns(int64_t M, int N, int K, int epilogue, int64_t row_stride);
 int samfast_bench_sparse24_turns(int64_t M, int N, int K, int epilogue, int64_t row_stride);
+
+/*
+ * 1000 times the rows plus the columns of the tile in which samfast_gemm_i8_fused without a step behind it forms an output of few rows
+ * with K dealt over a workgroup's wavefronts, 0 where the rule leaves it to other kernels: no launch.  SAMFAST_E_INVALID for a bad shape.
+ */
+int samfast_bench_gemm_i8_few_rows(int64_t M, int N, int K, int x_layout, int w_layout);
 
 /*
  * Measurement aid, no counterpart in the reference: one launch of a kernel that does nothing

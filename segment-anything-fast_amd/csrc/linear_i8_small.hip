@@ -16,6 +16,7 @@
 #include "gemm_i8_shared.hpp"
 #include "linear_i8_small.hpp"
 #include "quant_row.hpp"
+#include "samfast_bench.h"
 
 // every fp32 step below is rounded on its own (no fused multiply-add), as in the other forms
 #pragma clang fp contract(off)
@@ -396,19 +397,23 @@ int linear_i8_small_launch(const unsigned short* x, int64_t ldx, const int8_t* w
 // round costs more than that gains.  Measured on K-block major codes, us, against the tiled kernels:
 // 128 x 3840 x 1280 in 64 x 32 tiles 4.7 (6.3), 64 x 1280 x 5120 in 16 x 32 5.6 (14.6).  From 2304 values on 64 x 32 tiles are slower than
 // 64 x 64 ones whose operands come through LDS (gemm_i8_once.hip; 278 x 1280 x 3072 8.3 / 7.6, 0.96 times as long over 70 shapes, below 2240 1.04 to 1.07), and
-// 64 x 64 tiles straight into registers were at any length (512 x 1280 x 3072 10.6 / 8.4).
+// 64 x 64 tiles straight into registers were at any length (512 x 1280 x 3072 10.6 / 8.4).  `w_splits_lines`: K-block-major codes beside row-major weights of an
+// odd multiple of 64 bytes, whose pieces of 64 bytes share cache lines with their neighbours: there 64 x 32 tiles stay ahead, each wavefront reading
+// its own part of a row (a Linear, 64 x 64 through LDS / 64 x 32, us: 39 x 3776 -> 5120 10.4 / 9.65, 194 x 3648 -> 1600 11.6 / 10.9, 331 x 5056 -> 1280 15.2 / 14.5; 1.03 times as long over
+// 170 shapes, over 360 of whole lines 0.89; with row-major codes as well 0.83, with both K-block major 0.94).
 // Returns 16-row tiles * 8 + 16-column tiles, 0 = none.
-static int skinny_shape(int M, int N, int K) {
+static int skinny_shape(int M, int N, int K, bool w_splits_lines) {
   auto fits = [&](int mt, int nt) { return (int64_t)((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * nt - 1) / (16 * nt)) <= 256; };
   if (fits(1, 1)) return 1 * 8 + 1;
   if (fits(1, 2)) return 1 * 8 + 2;
   if (fits(2, 2)) return 2 * 8 + 2;
-  if (K < 2304 && fits(4, 2)) return 4 * 8 + 2;
+  if ((K < 2304 || w_splits_lines) && fits(4, 2)) return 4 * 8 + 2;
   return 0;
 }
+static int skinny_shape(const GemmArgs& a) { return skinny_shape(a.M, a.N, a.K, a.x_pitch == GBK && a.w_pitch != GBK && a.K % 128 != 0); }
 
 bool gemm_i8_skinny_covers(const GemmArgs& a) {
-  return knob_or(KNOB_GEMM_SKINNY, 1) > 0 && skinny_shape(a.M, a.N, a.K) != 0;
+  return knob_or(KNOB_GEMM_SKINNY, 1) > 0 && skinny_shape(a) != 0;
 }
 
 template <int MT, int NT>
@@ -426,7 +431,7 @@ int gemm_i8_skinny_launch(const GemmArgs& g, hipStream_t stream) {
   a.y = reinterpret_cast<unsigned short*>(g.out);
   a.ldy = g.ldo; a.M = g.M; a.N = g.N; a.K = g.K;
   a.x_pitch = g.x_pitch; a.w_pitch = g.w_pitch; a.x_kstep = g.x_kstep; a.w_kstep = g.w_kstep;
-  switch (skinny_shape(a.M, a.N, a.K)) {
+  switch (skinny_shape(g)) {
     case 1 * 8 + 1: return launch_skinny<1, 1>(a, stream);
     case 1 * 8 + 2: return launch_skinny<1, 2>(a, stream);
     case 2 * 8 + 2: return launch_skinny<2, 2>(a, stream);
@@ -435,3 +440,14 @@ int gemm_i8_skinny_launch(const GemmArgs& g, hipStream_t stream) {
 }
 
 }  // namespace samfast
+
+extern "C" int samfast_bench_gemm_i8_few_rows(int64_t M, int N, int K, int x_layout, int w_layout) {
+  using namespace samfast;
+  SF_REQUIRE(M > 0 && M < (1ll << 31) && N > 0 && K > 0, "bench_gemm_i8_few_rows: bad shape M=%lld N=%d K=%d", (long long)M, N, K);
+  GemmArgs g = {};
+  g.M = (int)M; g.N = N; g.K = K;
+  g.x_pitch = x_layout == SAMFAST_LAYOUT_KB64 ? GBK : K;
+  g.w_pitch = w_layout == SAMFAST_LAYOUT_KB64 ? GBK : K;
+  const int s = gemm_i8_skinny_covers(g) ? skinny_shape(g) : 0;
+  return 16 * (s / 8) * 1000 + 16 * (s % 8);
+}

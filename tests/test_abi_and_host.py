@@ -792,6 +792,17 @@ def test_the_dense_products_lines_between_widths():
         assert _lib.load().samfast_bench_gemm_i8_turns(M, N, K, _lib.EPILOGUE_RESIDUAL, N) == columns, (M, N, K)
 
 
+def test_the_lines_of_the_products_of_few_rows():
+    """64 x 32 tiles end at 2304 values, but not where row-major weights of an odd multiple of 64 meet K-block-major codes: (M, N, K, codes' and weights'
+    layout, 1000 * rows + columns)."""
+    from samfast_amd import _lib
+    row, kb, tile = _lib.LAYOUT_ROWMAJOR, _lib.LAYOUT_KB64, _lib.load().samfast_bench_gemm_i8_few_rows
+    for *call, want in ((194, 1600, 2240, kb, row, 64032), (194, 1600, 2304, kb, row, 0), (194, 1600, 3648, kb, row, 64032), (39, 5120, 3776, kb, row, 64032), (39, 5120, 3840, kb, row, 0),
+                        (194, 1600, 3648, row, row, 0), (194, 1600, 3648, kb, kb, 0), (331, 1280, 5056, kb, row, 64032), (600, 1280, 5056, kb, row, 0), (64, 4096, 4096, kb, row, 32032)):
+        assert tile(*call) == want, call
+    assert tile(0, 1600, 2240, kb, row) == -1
+
+
 def test_the_dense_residual_products_lines_where_rows_are_no_whole_lines():
     """Loops under 1280 beyond two rounds are left to the smaller tiles there, others by turns as on whole lines: (M, N, K, columns)."""
     from samfast_amd import _lib

@@ -230,7 +230,7 @@ def test_one_tile_of_64_rows_agrees_with_the_small_tiles(bm, tn, M, N, K, epi, l
     test_one_tile_per_cu_agrees_with_the_small_tiles(bm, tn, M, N, K, epi, layout)
 
 
-@pytest.mark.parametrize("M,N,K", [(278, 1280, 3072), (900, 768, 3072), (1638, 768, 4096), (1327, 1280, 4096), (2000, 1280, 4096)])
+@pytest.mark.parametrize("M,N,K", [(278, 1280, 3072), (194, 1600, 3648), (39, 5120, 3776), (900, 768, 3072), (1638, 768, 4096), (1327, 1280, 4096), (2000, 1280, 4096)])
 def test_linears_over_some_hundred_long_rows_against_their_codes(M, N, K):
     """Two launches through the tile that the rule takes, against the product of the quantiser's own codes in 64 bits."""
     from samfast_amd import Int8DynamicLinear, ops
