@@ -43,6 +43,12 @@ int samfast_bench_sparse24_turns(int64_t M, int N, int K, int epilogue, int64_t 
 int samfast_bench_gemm_i8_few_rows(int64_t M, int N, int K, int x_layout, int w_layout);
 
 /*
+ * The same of a Linear (samfast_linear_i8, or samfast_linear_i8_sparse24 for `layout` SAMFAST_LAYOUT_SPARSE24) whose workgroups quantise
+ * a few rows themselves: 1000 times those rows plus the columns of one, 0 for other forms.
+ */
+int samfast_bench_linear_i8_few_rows(int64_t M, int N, int K, int layout);
+
+/*
  * Measurement aid, no counterpart in the reference: one launch of a kernel that does nothing
  * but matrix instructions on operands held in registers (no global loads, no LDS, no barriers)
  * - the rate a GEMM or attention kernel built from the same instruction can approach at best

@@ -316,7 +316,8 @@ bool linear_i8_small_any_alignment(int64_t M, int K) { return M <= 8 || (M <= 16
 // product.  GPU time in us, two launches / one (shape), at the last calls of each line and beyond:
 //   int8, one column tile  up to 256 tiles, at any length 9 x 5120 -> 1280 8.2 / 6.5, 22 x 5120 -> 1280 8.4 / 6.6, 40 x 3072 -> 768 7.1 / 5.3, 58 x 2560 -> 264 6.6 / 5.0,
 //         12 x 3072 -> 768 6.6 / 5.0; with rows of up to 1024 values three on a CU are ahead of wider ones (four column tiles / one: 168 x 1024 -> 488 5.0 / 4.7, 203 x 768 -> 424 4.6 / 4.4,
-//         259 x 384 -> 288 3.9 / 3.65; 780 tiles: 158 x 1024 -> 624 5.10 / 5.13, 200 x 768 -> 512 4.6 / 4.8; at 1152 to 1536 values level)
+//         259 x 384 -> 288 3.9 / 3.65; 780 tiles: 158 x 1024 -> 624 5.10 / 5.13, 200 x 768 -> 512 4.6 / 4.8; at 1152 to 1536 values level).  Nine k steps, of which one
+//         wavefront has two: not three workgroups on a CU (four column tiles / one: 829 x 576 -> 104, 728 tiles, 3.79 / 4.00, 66 x 576 -> 1280 3.80 / 3.99; on two 60 x 576 -> 1024 3.38 / 3.32)
 //   two column tiles  up to 256 tiles and 4096 values 254 x 2304 -> 240 7.0 / 5.7, 124 x 2816 -> 496 7.0 / 6.3, 120 x 3072 -> 512 7.2 / 6.5, 144 x 3584 -> 432 7.8 / 7.2, 51 x
 //         4096 -> 840 7.75 / 7.7; beyond: 67 x 2816 -> 1048 (297) 8.1 / 8.9, 32 x 5120 -> 1280 8.3 / 8.7; up to 512 short rows 223 x 256 -> 520 3.8 / 3.65 (four column tiles / two)
 //   others  128 x 1024 -> 1024 6.6 / 5.5 (4 tiles), 256 x 1024 -> 1024 6.9 / 6.9 (16 rows, 4)
@@ -339,7 +340,7 @@ static int small_shape(int64_t M, int N, int K, bool sparse) {
   if (M <= 8 || K <= 4096) {
     if (tiles(2) <= 256) return 8 + 2;
     if (M <= 4 && (K <= 512 || tiles(2) <= 288)) return 8 + 2;
-    if (M > 8 && K <= 1024 && tiles(1) <= 768) return 8 + 1;
+    if (M > 8 && K <= 1024 && tiles(1) <= (K == 576 ? 512 : 768)) return 8 + 1;
     if (M > 8 && K <= 512 && tiles(2) <= 512) return 8 + 2;
     if (K <= 1536 && tiles(4) <= 256) return 8 + 4;
     if (M <= 8) return 8 + 2;
@@ -450,4 +451,13 @@ extern "C" int samfast_bench_gemm_i8_few_rows(int64_t M, int N, int K, int x_lay
   g.w_pitch = w_layout == SAMFAST_LAYOUT_KB64 ? GBK : K;
   const int s = gemm_i8_skinny_covers(g) ? skinny_shape(g) : 0;
   return 16 * (s / 8) * 1000 + 16 * (s % 8);
+}
+
+extern "C" int samfast_bench_linear_i8_few_rows(int64_t M, int N, int K, int layout) {
+  using namespace samfast;
+  SF_REQUIRE(M > 0 && N > 0 && K > 0 && layout >= SAMFAST_LAYOUT_ROWMAJOR && layout <= SAMFAST_LAYOUT_SPARSE24,
+             "bench_linear_i8_few_rows: bad shape M=%lld N=%d K=%d or layout %d", (long long)M, N, K, layout);
+  const bool sparse = layout == SAMFAST_LAYOUT_SPARSE24;
+  const int s = small_shape(M, N, K, sparse);
+  return s / 8 * 8 * 1000 + s % 8 * (sparse ? 32 : 16);
 }

@@ -792,6 +792,16 @@ def test_the_dense_products_lines_between_widths():
         assert _lib.load().samfast_bench_gemm_i8_turns(M, N, K, _lib.EPILOGUE_RESIDUAL, N) == columns, (M, N, K)
 
 
+def test_the_lines_of_the_workgroups_of_a_linear_over_few_rows():
+    """One column tile each on up to 768 workgroups, nine k steps on up to 512: (M, N, K, layout, 1000 * rows + columns)."""
+    from samfast_amd import _lib
+    tile = _lib.load().samfast_bench_linear_i8_few_rows
+    for *call, want in ((576, 112, 576, 0, 8016), (599, 112, 576, 0, 8064), (66, 1280, 576, 0, 8064), (91, 776, 576, 1, 8064), (66, 1280, 512, 0, 8016), (66, 1280, 640, 0, 8016), (829, 104, 640, 0, 8016),
+                        (45, 2304, 576, 0, 8064), (13, 3840, 4096, 0, 8032), (24, 1280, 5120, 0, 8016), (32, 1280, 5120, 0, 0), (64, 1024, 5120, 2, 8032)):
+        assert tile(*call) == want, call
+    assert tile(0, 1024, 576, 0) == -1 and tile(8, 1024, 576, 3) == -1
+
+
 def test_the_lines_of_the_products_of_few_rows():
     """64 x 32 tiles end at 2304 values, but not where row-major weights of an odd multiple of 64 meet K-block-major codes: (M, N, K, codes' and weights'
     layout, 1000 * rows + columns)."""

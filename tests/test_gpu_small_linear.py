@@ -252,7 +252,7 @@ def test_linears_over_some_hundred_long_rows_against_their_codes(M, N, K):
     (False, 63, 488, 64), (False, 64, 512, 512), (False, 65, 1000, 576), (False, 121, 1024, 1024), (False, 128, 1032, 1088), (False, 250, 1016, 1536),
     (False, 79, 760, 2048), (False, 405, 632, 704), (False, 9, 8200, 1600), (False, 31, 13000, 768), (False, 4, 8200, 512), (False, 1, 9000, 1088), (False, 5, 8200, 256),
     # long rows, several short workgroups on a CU: the last calls of the lines
-    (False, 24, 1360, 5120), (False, 2041, 16, 2112), (False, 9, 4096, 4096), (False, 61, 1016, 4096), (False, 250, 256, 2112), (False, 379, 248, 1024),
+    (False, 24, 1360, 5120), (False, 2041, 16, 2112), (False, 9, 4096, 4096), (False, 61, 1016, 4096), (False, 250, 256, 2112), (False, 379, 248, 1024), (False, 576, 112, 576), (False, 599, 112, 576),
     (False, 92, 1024, 320), (False, 250, 512, 512), (False, 61, 2048, 128),
     (True, 256, 1024, 2048), (True, 59, 4096, 1920), (True, 125, 1016, 3072), (True, 61, 1016, 5120), (True, 250, 256, 3200),
     (True, 1, 8, 256), (True, 63, 1000, 512), (True, 128, 1536, 1024), (True, 77, 1632, 1152), (True, 57, 1016, 2048), (True, 81, 712, 3072), (True, 4, 1288, 5120),
