@@ -322,7 +322,8 @@ bool linear_i8_small_any_alignment(int64_t M, int K) { return M <= 8 || (M <= 16
 //         4096 -> 840 7.75 / 7.7; beyond: 67 x 2816 -> 1048 (297) 8.1 / 8.9, 32 x 5120 -> 1280 8.3 / 8.7; up to 512 short rows 223 x 256 -> 520 3.8 / 3.65 (four column tiles / two)
 //   others  128 x 1024 -> 1024 6.6 / 5.5 (4 tiles), 256 x 1024 -> 1024 6.9 / 6.9 (16 rows, 4)
 //   2:4   to 2048 values up to 1024 tiles 117 x 1024 -> 2064 6.95 / 5.6, 165 x 1280 -> 1504 7.9 / 6.5, 174 x 1536 -> 1000 7.6 / 6.2, 318 x 1792 -> 776 8.3 / 7.5, 258 x 2048 -> 976 10.2 / 7.6;
-//         beyond: 109 x 768 -> 2992 (1316) 6.15 / 6.6, 251 x 1280 -> 1304 (1312) 7.9 / 8.5; to 3072 up to 512 290 x 2560 -> 352 9.1 / 6.7, 90 x 3072 -> 1304 9.0 / 7.4; beyond: 42 x 2304 -> 2984
+//         but 256 values and more than 768 tiles are the band kernel's where it takes them, unless the columns are whole 128s, which it reads slower (it / this:
+//         480 -> 520 4.41 / 4.75, 241 -> 936 4.50 / 4.71; 60 -> 4096 4.94 / 4.68, 186 -> 1280 4.87 / 4.65); beyond: 109 x 768 -> 2992 (1316) 6.15 / 6.6, 251 x 1280 -> 1304 (1312) 7.9 / 8.5; to 3072 up to 512 290 x 2560 -> 352 9.1 / 6.7, 90 x 3072 -> 1304 9.0 / 7.4; beyond: 42 x 2304 -> 2984
 //         (564) 8.2 / 8.8; else up to 256 31 x 5120 -> 1280 10.4 / 6.3, 48 x 4096 -> 1024 9.0 / 6.6; beyond: 119 x 3328 -> 680 (330) 9.1 / 11.4
 //   Up to four short rows are quantised in no time, and two column tiles on more workgroups than CUs are ahead of four: 1 x 256 -> 8200 3.07 / 3.64 (two / four),
 //         4 x 128 -> 10240 3.2 / 3.5, 1 x 512 -> 16384 3.83 / 3.98, 1 x 1024 -> 8200 4.46 / 4.75; but 8 x 256 -> 10240 3.8 / 3.6, 4 x 768 -> 12288 4.8 / 4.5.
@@ -333,6 +334,7 @@ static int small_shape(int64_t M, int N, int K, bool sparse) {
   const int64_t eights = (M + 7) / 8;
   if (sparse) {
     const int64_t tiles = eights * ((N + 31) / 32);
+    if (K <= 256 && tiles > 768 && N % 128 != 0 && linear_i8_band_covers(M, N, K, true)) return 0;
     return K % 128 == 0 && K >= 256 && tiles <= (K <= 2048 ? 1024 : K <= 3072 ? 512 : 256) ? 8 + 1 : 0;
   }
   auto tiles = [&](int nt) { return eights * ((N + 16 * nt - 1) / (16 * nt)); };

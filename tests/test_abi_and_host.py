@@ -793,11 +793,13 @@ def test_the_dense_products_lines_between_widths():
 
 
 def test_the_lines_of_the_workgroups_of_a_linear_over_few_rows():
-    """One column tile each on up to 768 workgroups, nine k steps on up to 512: (M, N, K, layout, 1000 * rows + columns)."""
+    """One column tile each on up to 768 workgroups, nine k steps on up to 512; 2:4 up to 1024, 256 values on up to 768 where the band
+    kernel takes the others: (M, N, K, layout, 1000 * rows + columns)."""
     from samfast_amd import _lib
     tile = _lib.load().samfast_bench_linear_i8_few_rows
     for *call, want in ((576, 112, 576, 0, 8016), (599, 112, 576, 0, 8064), (66, 1280, 576, 0, 8064), (91, 776, 576, 1, 8064), (66, 1280, 512, 0, 8016), (66, 1280, 640, 0, 8016), (829, 104, 640, 0, 8016),
-                        (45, 2304, 576, 0, 8064), (13, 3840, 4096, 0, 8032), (24, 1280, 5120, 0, 8016), (32, 1280, 5120, 0, 0), (64, 1024, 5120, 2, 8032)):
+                        (45, 2304, 576, 0, 8064), (13, 3840, 4096, 0, 8032), (24, 1280, 5120, 0, 8016), (32, 1280, 5120, 0, 0), (64, 1024, 5120, 2, 8032),
+                        (472, 408, 256, 2, 8032), (480, 408, 256, 2, 0), (480, 520, 256, 2, 0), (480, 512, 256, 2, 8032), (480, 520, 384, 2, 8032), (60, 4096, 256, 2, 8032), (31, 6152, 256, 2, 8032), (1276, 144, 256, 2, 8032)):
         assert tile(*call) == want, call
     assert tile(0, 1024, 576, 0) == -1 and tile(8, 1024, 576, 3) == -1
 

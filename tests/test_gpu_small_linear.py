@@ -254,7 +254,7 @@ def test_linears_over_some_hundred_long_rows_against_their_codes(M, N, K):
     # long rows, several short workgroups on a CU: the last calls of the lines
     (False, 24, 1360, 5120), (False, 2041, 16, 2112), (False, 9, 4096, 4096), (False, 61, 1016, 4096), (False, 250, 256, 2112), (False, 379, 248, 1024), (False, 576, 112, 576), (False, 599, 112, 576),
     (False, 92, 1024, 320), (False, 250, 512, 512), (False, 61, 2048, 128),
-    (True, 256, 1024, 2048), (True, 59, 4096, 1920), (True, 125, 1016, 3072), (True, 61, 1016, 5120), (True, 250, 256, 3200),
+    (True, 480, 520, 256), (True, 256, 1024, 2048), (True, 59, 4096, 1920), (True, 125, 1016, 3072), (True, 61, 1016, 5120), (True, 250, 256, 3200),
     (True, 1, 8, 256), (True, 63, 1000, 512), (True, 128, 1536, 1024), (True, 77, 1632, 1152), (True, 57, 1016, 2048), (True, 81, 712, 3072), (True, 4, 1288, 5120),
 ])
 def test_one_launch_agrees_with_two(sparse, M, N, K):
