@@ -48,6 +48,9 @@ int samfast_bench_gemm_i8_few_rows(int64_t M, int N, int K, int x_layout, int w_
  */
 int samfast_bench_linear_i8_few_rows(int64_t M, int N, int K, int layout);
 
+/* 1000 times the rows plus the columns of the tile of samfast_linear_half, 0 where samfast_linear_half_pays says no. */
+int samfast_bench_linear_half(int64_t M, int N, int K, int epilogue);
+
 /*
  * Measurement aid, no counterpart in the reference: one launch of a kernel that does nothing
  * but matrix instructions on operands held in registers (no global loads, no LDS, no barriers)

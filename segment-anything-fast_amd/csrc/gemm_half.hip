@@ -1,6 +1,7 @@
 // bf16 / fp16 Linears of an encoder block: the turn-taking kernels of gemm_pingpong.hpp with the block's own epilogues, so that GELU and
 // the residual add cost no pass over memory of their own.
 #include "gemm_pingpong.hpp"
+#include "samfast_bench.h"
 
 namespace samfast {
 
@@ -47,7 +48,7 @@ static int half_choose(int64_t M, int N, int K, int epi) {
   if (!pays) return 0;
   if (c.tm == 5) return kHalfTall;
   // (192 columns are no reason to leave the library's product, whose order of K is another: all of these sum in the same one)
-  return epi == PP_RESIDUAL ? c.tn : pp_choose(M, N, K / 64, false, 8.1).tn;
+  return epi == PP_RESIDUAL ? c.tn : pp_choose(M, N, K / 64, false, epi == PP_GELU ? 8.4 : 8.1).tn;
 }
 
 template <class E>
@@ -88,6 +89,13 @@ extern "C" int samfast_linear_half_pays(int64_t M, int N, int K, int epilogue) {
   using namespace samfast;
   const int epi = epilogue == SAMFAST_EPILOGUE_GELU ? PP_GELU : epilogue == SAMFAST_EPILOGUE_RESIDUAL ? PP_RESIDUAL : PP_PLAIN;
   return N > 0 && N % 8 == 0 && half_choose(M, N, K, epi) != 0;
+}
+
+extern "C" int samfast_bench_linear_half(int64_t M, int N, int K, int epilogue) {
+  using namespace samfast;
+  SF_REQUIRE(M > 0 && N > 0 && K > 0 && N % 8 == 0, "bench_linear_half: bad shape M=%lld N=%d K=%d", (long long)M, N, K);
+  const int tn = half_choose(M, N, K, epilogue == SAMFAST_EPILOGUE_GELU ? PP_GELU : epilogue == SAMFAST_EPILOGUE_RESIDUAL ? PP_RESIDUAL : PP_PLAIN);
+  return tn == 0 ? 0 : tn == kHalfTall ? 320256 : (tn < 6 ? 128000 : 256000) + 32 * tn;
 }
 
 extern "C" int samfast_linear_half(const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t ldy,

@@ -773,7 +773,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_split_kernel(PPArgs a) {
 // per CU 65536 x 1280 -> 3840 276 / 275; loops under ten k tiles pay more for the wide tile's end: 24576 x 768 -> 3072 (five / four)
 // 64.4 / 70.3, 24576 x 1024 -> 3072 (five / four) 77.7 / 81.3, 12288 x 1024 -> 3072 (three / two) 44.4 / 42.1.  bf16 12288 x 1280 -> 5120 (four / three) 141 / 134,
 // 24576 x 1280 -> 5120 276 / 261, but 24576 x 1024 -> 3072 121 / 124.
-// `narrow`, unless 0: the price of 192 columns, where the caller builds them: half types 8.1, int8 8.7 (both less in the first rounds), with the residual 9.  256 / 192, rounds, bf16:
+// `narrow`, unless 0: the price of 192 columns, where the caller builds them: half types 8.1 (with GELU 8.4: a round more of them than of wider tiles, 0.97 of the price at 8.1, was 1.00 times as long over 15 products, 23243 x 5120 -> 1408
+// in three rounds for two 263 / 282; without GELU 0.976 over 20), int8 8.7 (both less in the first rounds), with the residual 9.  256 / 192, rounds, bf16:
 // 4096 x 768 -> 3072 with GELU (one / one) 27.0 / 23.9, 4096 x 1024 -> 3072 25.9 / 23.7, 8192 x 768 -> 3072 with GELU (two / two) 45.6 / 40.0, 28672 x 1024 ->
 // 3072 (six / seven) 141 / 133; but 20480 x 1024 -> 3072 (four / five) 96.7 / 96.9, 32768 x 768 -> 3072 with GELU (six / eight) 145 / 152; 320 / 192: 12288 x 1024 -> 3072 (two /
 // three) 61.0 / 58.5, but 24576 x 768 -> 2304 (three / five) 73.1 / 73.4.  int8, the smaller members / 192: 8192 x 768 -> 3072 25.0 / 22.7, 8192 x 1024 -> 3072 29.6 / 26.6, 6144 x

@@ -73,6 +73,7 @@ _BENCH_SIGNATURES = {
     "samfast_bench_sparse24_turns": (_i32, [_i64, _i32, _i32, _i32, _i64]),
     "samfast_bench_gemm_i8_few_rows": (_i32, [_i64, _i32, _i32, _i32, _i32]),
     "samfast_bench_linear_i8_few_rows": (_i32, [_i64, _i32, _i32, _i32]),
+    "samfast_bench_linear_half": (_i32, [_i64, _i32, _i32, _i32]),
     "samfast_bench_mfma_ceiling": (_i32, [_i32, _ptr, _i32, _i32, ctypes.POINTER(_i64), _ptr, _ptr]),
     "samfast_bench_mfma_valu_overlap": (_i32, [_i32, _ptr, _i32, _i32, _i32, _ptr, _ptr]),
 }

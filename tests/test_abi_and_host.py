@@ -782,6 +782,17 @@ def test_the_sparse_products_lines():
     assert turns(0, 5120, 1280, none) == -1 and turns(65536, 5120, 1280, none, 5112) == -1
 
 
+def test_the_half_type_products_lines_between_widths():
+    """Tiles of 192 columns among the wider ones by the price of their rounds, with GELU a little dearer: (M, N, K, epilogue, 1000 * rows + columns)."""
+    from samfast_amd import _lib
+    none, gelu, residual = _lib.EPILOGUE_NONE, _lib.EPILOGUE_GELU, _lib.EPILOGUE_RESIDUAL
+    for *call, tile in ((4096, 3072, 768, gelu, 256192), (8192, 3072, 768, gelu, 256192), (4096, 3072, 1024, none, 256192), (28672, 3072, 1024, none, 256192), (12288, 3072, 1024, none, 256192),
+                        (23243, 1408, 5120, none, 256192), (23243, 1408, 5120, gelu, 256320), (27762, 1280, 768, gelu, 256320), (17289, 4096, 1280, gelu, 256256), (28072, 3072, 1024, gelu, 256192),
+                        (4096, 5120, 1280, gelu, 256320), (4096, 1280, 5120, residual, 128160), (20480, 1024, 4096, residual, 320256), (4096, 2304, 768, none, 0)):
+        assert _lib.load().samfast_bench_linear_half(*call) == tile, call
+        assert _lib.load().samfast_linear_half_pays(*call) == (tile != 0), call
+
+
 def test_the_dense_products_lines_between_widths():
     """Tiles of 192, 256 and 320 columns by the price of their rounds, 0 for the smaller members: (M, N, K, columns)."""
     from samfast_amd import _lib
