@@ -492,7 +492,10 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(PPArgs a) {
 // Long loops' weights, which come from HBM in an encoder whose weights exceed the last-level cache, are touched once, a line by each
 // thread of the grid, row by row: the loop asks all CUs' rows for one line each at a time, and waited for HBM at every k tile
 // (weights and rows not in the L2s: 4096 x 5120 -> 1280 60.2 / 50.3, 4096 x 4096 -> 1024 39.0 / 34.0, 4096 x 3072 -> 768 29.8 / 25.0, 2048 x 5120 -> 1280 45.1 / 36.2; all of it in
-// them: 49.0 / 49.0, 32.4 / 33.0, 21.9 / 22.4, 31.5 / 32.6).  At 20 k tiles and fewer it is level or slower (4096 x 1280 -> 1280 20.7 / 21.3).
+// them: 49.0 / 49.0, 32.4 / 33.0, 21.9 / 22.4, 31.5 / 32.6; a ViT-H image with bf16 Linears 6640 / 6200, ViT-L 3810 / 3640, ViT-B 1650 / 1600).  At 20 k tiles and fewer it is
+// level or slower (4096 x 1280 -> 1280 20.7 / 21.3), and where the grid has fewer threads than W lines it costs more than the part that is touched
+// saves (touched / not, times as long as by turns: 113 products out of HBM 0.988 / 0.981, the worst twentieth 1.04 / 1.02; 21 out of the caches 0.885 / 0.850; a second
+// line a thread 1.02 times as long as touched): nothing is touched there.
 // Library's product + residual in the next LayerNorm / by turns + LayerNorm: 4096 x 5120 -> 1280 61.3 / 55.9, 4096 x 1280 -> 1280
 // 31.1 / 23.6, 4096 x 768 -> 768 31.6 / 18.6.  (int8 keeps gemm_i8_once.hip.)
 template <int TN>
@@ -634,8 +637,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_split_kernel(PPArgs a) {
     advance();
   }
   unsigned int touched = 0;
-  if (nk >= 32) {  // this thread's line of W
-    const unsigned int line = min(blockIdx.x * 512u + tid, (unsigned int)a.N * nk - 1u), row = line / (unsigned int)nk;
+  if (nk >= 32 && (unsigned int)a.N * nk <= total * 512u) {  // this thread's line of W
+    const unsigned int line = min(pid * 512u + tid, (unsigned int)a.N * nk - 1u), row = line / (unsigned int)nk;
     touched = *(gword_t)((gbyte_t)(uintptr_t)a.w + (int64_t)row * a.w_pitch + (line - row * nk) * 128);
   }
   i32x4 fx[2][4], fw[2][TN];

@@ -72,6 +72,12 @@ def test_split_half_linear_at_the_ends_of_its_loop(tile, K):
     test_half_linear_with_its_epilogues(301, 32 * tile + 40, K, 2, tile, torch.bfloat16)
 
 
+@pytest.mark.parametrize("M,N,tile", [(301, 100, 3), (1500, 104, 3), (1025, 136, 4), (3000, 768, 3), (2000, 160, 5)])
+def test_split_half_linear_whose_grid_touches_its_weights(M, N, tile):
+    """Threads of the grid fewer and more than the lines of W, tiles no multiple of eight."""
+    test_half_linear_with_its_epilogues(M, N // 8 * 8, 2048, 2, tile, torch.bfloat16)
+
+
 def test_half_linear_leaves_what_it_does_not_take():
     from samfast_amd import ops
     linear = torch.nn.Linear(1024, 4096, device="cuda", dtype=torch.bfloat16).requires_grad_(False)
