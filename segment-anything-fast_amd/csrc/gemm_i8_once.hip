@@ -14,7 +14,10 @@
 //   * a stage is global -> LDS loads only; the threshold of outstanding loads leaves NST - 2 stages in
 //     flight across the one barrier of an iteration.  The loads stand between the products: a wavefront waits in line with a load, 16 cycles
 //     for each that is ahead of it, and in front of the products they made an iteration of 4096 x 3072 -> 768 694 cycles, 384 of products and 448 of
-//     loads (us, in front / between: 4096 x 1280 -> 1280 14.9 / 14.4, 1024 x 5120 -> 1280 19.0 / 18.1, 3000 x 3072 -> 768 15.1 / 14.6);
+//     loads (us, in front / between: 4096 x 1280 -> 1280 14.9 / 14.4, 1024 x 5120 -> 1280 19.0 / 18.1, 3000 x 3072 -> 768 15.1 / 14.6).  Not so
+//     where an operand is row-major and the tile has 128 rows: the two groups' k tiles are halves of the same lines, and requests that go out together,
+//     in front of the products, share them (in front / between: both row-major 643 x 2176 -> 4952 14.1 / 15.0, 897 x 4992 -> 4096 with GELU 29.5 / 30.8; over 263 products 0.986 times as
+//     long; row-major weights alone, a Linear's, 250 of them 0.993; both K-block major, 137 of them, 1.017);
 //   * v_mfma_i32_16x16x64_i8 with W as A and X as B: a lane ends with four adjacent columns of one row.  The
 //     fragments of the next k tile are read while this one's MFMAs run, where registers allow (TN <= 5);
 //   * the residual rows are requested before the loop (128-row tiles), scales and bias land in LDS under it,
@@ -67,9 +70,11 @@ SF_DEVICE void load_lower_half(const int8_t* base, unsigned int off, unsigned in
   asm volatile("s_mov_b64 exec, 0xffffffff\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" : : "v"(off), "s"(base), "{m0}"(dst) : "memory");
 }
 
-template <int EPI, int BM, int TN>
+// FRONT: the loads in front of the products (see above)
+template <int EPI, int BM, int TN, bool FRONT = false>
 __global__ __launch_bounds__(512, 2) void gemm_i8_once_kernel(GemmArgs a) {
   using C = OnceCfg<BM, TN>;
+  static_assert(!FRONT || (BM == 128 && C::AHEAD), "built for 128 rows");
   constexpr int TM = C::TM, KG = C::KG, BN = C::BN, NST = C::NST, NLD = C::NLD;
   __shared__ __attribute__((aligned(16))) unsigned char lds[C::NST * C::STAGE + C::SC_BYTES];
   unsigned char* sc = lds + NST * C::STAGE;
@@ -205,13 +210,21 @@ __global__ __launch_bounds__(512, 2) void gemm_i8_once_kernel(GemmArgs a) {
       if constexpr (STEADY) arrive(NST - 2);
       else arrive(min(nt - 2 - t, NST - 2));
       const int free = st;
+      if (FRONT && (STEADY || t + NST < nt)) fill(t + NST, free);
       st = next_stage(st);
       if (STEADY || t + 1 < nt) read(next, st);
       if (STEADY || KG < 4 || t * KG + grp < nk) multiply(now);
-      if (STEADY || t + NST < nt) fill(t + NST, free);
-      // two fragment reads behind each of the first MFMAs, then the requests spread over the others: a wavefront waits in line with a
-      // request, 16 cycles for each that is ahead of it
-      if (STEADY) {
+      if (!FRONT && (STEADY || t + NST < nt)) fill(t + NST, free);
+      if (FRONT && STEADY) {
+        // one fragment read behind each of the first MFMAs
+#pragma unroll
+        for (int g = 0; g < TM + TN; ++g) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+      } else if (STEADY) {
+        // two fragment reads behind each of the first MFMAs, then the requests spread over the others: a wavefront waits in line with a
+        // request, 16 cycles for each that is ahead of it
         constexpr int READS = TM + TN, FIRST = (READS + 1) / 2, EACH = (TM * TN - FIRST) / NLD;
 #pragma unroll
         for (int g = 0; g < FIRST; ++g) {
@@ -417,12 +430,14 @@ int gemm_i8_once_launch(int epi, const GemmArgs& a0, hipStream_t stream) {
   a.tiles_n = (a.N + bn - 1) / bn;
   a.group_m = 4;  // an XCD's 32 tiles: 4 row tiles x 8 column tiles, 2 to 4 MB of operands in its L2
   const unsigned int grid = (unsigned int)((a.tiles_m * a.tiles_n + 7) / 8 * 8);
-#define SF_ONCE(E, B, T) hipLaunchKernelGGL((gemm_i8_once_kernel<E, B, T>), dim3(grid), dim3(512), 0, stream, a)
+  const bool front = a.x_pitch != GBK || a.w_pitch != GBK;  // a row-major operand
+#define SF_ONCE(E, B, ...) hipLaunchKernelGGL((gemm_i8_once_kernel<E, B, __VA_ARGS__>), dim3(grid), dim3(512), 0, stream, a)
+#define SF_ONCE_F(E, T) do { if (front) SF_ONCE(E, 128, T, true); else SF_ONCE(E, 128, T); } while (0)
 #define SF_ONCE_128(T)                                                              \
   case 128 * 16 + T:                                                                \
-    if (epi == EPI_GELU_BF16) SF_ONCE(EPI_GELU_BF16, 128, T);                       \
-    else if (epi == EPI_RESIDUAL_BF16) SF_ONCE(EPI_RESIDUAL_BF16, 128, T);          \
-    else SF_ONCE(EPI_SCALE_BIAS_BF16, 128, T);                                      \
+    if (epi == EPI_GELU_BF16) SF_ONCE_F(EPI_GELU_BF16, T);                          \
+    else if (epi == EPI_RESIDUAL_BF16) SF_ONCE_F(EPI_RESIDUAL_BF16, T);             \
+    else SF_ONCE_F(EPI_SCALE_BIAS_BF16, T);                                         \
     break
 #define SF_ONCE_64(T)                                                               \
   case 64 * 16 + T:                                                                 \
@@ -450,6 +465,7 @@ int gemm_i8_once_launch(int epi, const GemmArgs& a0, hipStream_t stream) {
 #undef SF_ONCE_256
 #undef SF_ONCE_64
 #undef SF_ONCE_128
+#undef SF_ONCE_F
 #undef SF_ONCE
   return check_launch("gemm_i8_once_kernel");
 }
