@@ -656,6 +656,10 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
 // operand as they stand, its k slots 8 q .. 8 q + 7 being the keys 4 q .. + 3 and 16 + 4 q .. + 3, and two transposing reads bring V in that order.
 // us, 32 x 32 x 16 / so (bf16; fp16): 1 x 8 heads 51.5 / 49.7; 50.9 / 47.9, 1 x 12 66.0 / 63.8; 69.3 / 66.3, 4 x 12 242 / 232; 259 / 244, 8 x 16 645 / 636; 675 / 658, 9 x 16 x 6 rows
 // of 64 19.2 / 18.1; 18.7 / 18.2.  The error against 64 bits is the same to three digits (2.35e-3, 2.94e-4 of the norm).
+// Up to 256 workgroups are one wavefront a SIMD, which waits for the matrix pipe between a step's two instructions if they stand side by side: there
+// they stand apart, one on either side of the exponentials (the same operations: the same bits.  us, 32 x 32 x 16 / side by side / apart, bf16; fp16: 2 x 1 heads 30.3 / 32.4 / 30.9;
+// 31.2 / 32.6 / 31.0, 2 x 3 x 40 rows 21.4 / 22.8 / 21.9, 4 x 1 x 40 fp16 21.8 / 22.8 / 21.8; over 61 calls 1.045 and 1.01 times as long as the 32 x 32 form, whose half as many
+// instructions that wavefront issues sooner).  From 257 to 384 the two are level, beyond, where other wavefronts fill the wait, side by side is ahead by up to 1.3 %.
 struct Split16Cfg {
   using R = GridRow<64>;
   static constexpr int QW = 2, WAVES = 2 * QW, BM = 32 * QW;  // query tiles of 32 and two key halves
@@ -671,7 +675,8 @@ struct Split16Cfg {
   static_assert(QW * 64 * 36 * 4 <= RELH_OFF, "the second halves' results");
 };
 
-template <typename T>
+// SPREAD: a step's two matrix instructions stand apart in its vector work (see above)
+template <typename T, bool SPREAD>
 __global__ __launch_bounds__(64 * Split16Cfg::WAVES, 3) void attn_global_split16_kernel(AttnArgs a) {
   using C = Split16Cfg;
   constexpr int HD = 64;
@@ -843,16 +848,22 @@ __global__ __launch_bounds__(64 * Split16Cfg::WAVES, 3) void attn_global_split16
     for (int g = 0; g < 8; ++g) {
       const int t = g >> 2, k = (g >> 1) & 1, r = 2 * (g & 1);
       const float x0 = fmaf(s.v[k][t][r], a.c, neg_mrow[t]), x1 = fmaf(s.v[k][t][r + 1], a.c, neg_mrow[t]);
-      if (g > 0) gather(g - 1);
-      e0 = fast_exp2(x0);
-      e1 = fast_exp2(x1);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int n = 0; n < 2; ++n) {
+      auto product = [&](int n) __attribute__((always_inline)) {
         if (g < 2) pv(pk_prev, 2 * g + n);
         else if (g < 6) score(s_next, 2 * (g - 2) + n);
         else pv(pk_prev, 2 * (g - 4) + n);
+      };
+      if (g > 0) gather(g - 1);
+      if constexpr (SPREAD) {
+        __builtin_amdgcn_sched_barrier(0);
+        product(0);
+        __builtin_amdgcn_sched_barrier(0);
       }
+      e0 = fast_exp2(x0);
+      e1 = fast_exp2(x1);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!SPREAD) product(0);
+      product(1);
       __builtin_amdgcn_sched_barrier(0);
     }
     // this row's V for the next round
@@ -965,7 +976,10 @@ static void launch_bias(const AttnArgs& a, int form, hipStream_t stream) {
   auto grid = [&](int queries) { return dim3((unsigned int)(((int64_t)a.B * a.nH * (a.N / queries) + 7) / 8 * 8)); };
   if (form == 8) hipLaunchKernelGGL((attn_global_bias_kernel<T, HD, 8>), grid(256), dim3(512), 0, stream, a);
   else if (form == 4) hipLaunchKernelGGL((attn_global_bias_kernel<T, HD, 4>), grid(128), dim3(256), 0, stream, a);
-  else if constexpr (HD == 64) hipLaunchKernelGGL((attn_global_split16_kernel<T>), grid(64), dim3(256), 0, stream, a);
+  else if constexpr (HD == 64) {
+    if ((int64_t)a.B * a.nH * (a.N / 64) <= 256) hipLaunchKernelGGL((attn_global_split16_kernel<T, true>), grid(64), dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((attn_global_split16_kernel<T, false>), grid(64), dim3(256), 0, stream, a);
+  }
   else hipLaunchKernelGGL((attn_global_split_kernel<T, HD>), grid(64), dim3(256), 0, stream, a);
 }
 

@@ -101,8 +101,8 @@ def test_every_other_sixteen_queries_move_their_reference(gh, which, dtype):
     assert ((out - ref).abs() <= 0.51 * eps * (weight + ref.abs()) + 1e-4 * weight + floor + 1e-6).all()
 
 
-@pytest.mark.parametrize("hd,dtype", [(64, torch.bfloat16), (80, torch.float16)])
-@pytest.mark.parametrize("gh", [64, 16, 6])
+@pytest.mark.parametrize("hd,dtype", [(64, torch.bfloat16), (64, torch.float16), (80, torch.float16)])
+@pytest.mark.parametrize("gh", [64, 16, 6])  # hd 64: up to 256 workgroups of 64 queries and more, two orders of one kernel's instructions
 def test_a_slice_has_the_same_bits_in_any_batch(hd, dtype, gh):
     from samfast_amd import ops
     print(f"case batch hd={hd} {dtype} gh={gh}", flush=True)
