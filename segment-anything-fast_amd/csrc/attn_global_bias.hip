@@ -13,17 +13,17 @@
 //   roundings into other codes.)
 //
 // Three kernels.  attn_global_bias_kernel: a wavefront owns 32 queries and walks whole key rows; workgroups of 8 (one
-// per CU: every row staged once for 256 queries) or 4 wavefronts (two per CU).  attn_global_split_kernel: the keys
-// of every row are split between two wavefronts, whose results (maximum reference, denominator, output) meet in
-// LDS once, at the end; workgroups of two query tiles x two key halves (64 queries, under 54 KB of LDS), three per CU
-// at hd 64 (attn_global_split16_kernel, on the smaller matrix instruction), so that one image's 12 heads are 768 workgroups: three on each of the 256 CUs, where 128-query
-// workgroups leave half of the CUs with one and half with two.  bias_form picks, by head_dim: the two kernels round
+// per CU: every row staged once for 256 queries) or 4 wavefronts (two per CU).  attn_global_split16_kernel (hd 64, on the smaller matrix
+// instruction): the keys of every row are split between two wavefronts, whose results (maximum reference, denominator, output) meet in
+// LDS once, at the end; workgroups of two query tiles x two key halves (64 queries, under 54 KB of LDS), three per CU, so that one image's 12 heads are
+// 768 workgroups: three on each of the 256 CUs, where 128-query workgroups leave half of the CUs with one and half with two.  attn_global_split_kernel:
+// the same at hd 80, on the larger instruction, where it is asked for.  bias_form picks, by head_dim: the kernels round
 // differently, and a slice's bits are not to depend on the batch.
 #include "attn_relpos_shared.hpp"
 
 namespace samfast {
 
-constexpr float kCeiling = 256.0f;  // of a half row's sum of probabilities: each stays far inside both types
+constexpr float kCeiling = 256.0f;  // of a lane's share of a half row's sum (16 of 32 keys, on the smaller instruction 8): each probability stays far inside both types
 
 template <int HD, int WAVES>
 struct BiasCfg : GridRow<HD> {
@@ -340,9 +340,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
     }
 }
 
-template <int HD>
-struct SplitCfg : GridRow<HD> {
-  using R = GridRow<HD>;
+// Split keys at hd 80 (SAMFAST_ATTN_SPLIT=2; hd 64 has a form of its own below).
+struct SplitCfg : GridRow<80> {
+  using R = GridRow<80>;
   static constexpr int QW = 2;                  // query tiles of 32 per workgroup
   static constexpr int WAVES = 2 * QW;
   static constexpr int BM = 32 * QW;
@@ -351,13 +351,14 @@ struct SplitCfg : GridRow<HD> {
   static constexpr int RELH_OFF = V_OFF + 2 * R::VTILE;
   static constexpr int RH = 32;                 // key rows whose rel_h is at hand
   static constexpr int LDS_BYTES = RELH_OFF + RH * BM * 4;
-  static_assert(3 * LDS_BYTES <= 160 * 1024, "three workgroups per CU");
-  static_assert(QW * 64 * (16 * R::DT + 2) * 4 <= RELH_OFF, "the second halves' results");
+  static_assert(2 * LDS_BYTES <= 160 * 1024, "two workgroups per CU");
+  static_assert(QW * 64 * (16 * R::DT + 1) * 4 <= RELH_OFF, "the second halves' results");
 };
 
-template <typename T, int HD>
-__global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void attn_global_split_kernel(AttnArgs a) {
-  using C = SplitCfg<HD>;
+template <typename T>
+__global__ __launch_bounds__(64 * SplitCfg::WAVES, 2) void attn_global_split_kernel(AttnArgs a) {
+  using C = SplitCfg;
+  constexpr int HD = 80;
   __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS_BYTES];
   float* relhT = reinterpret_cast<float*>(lds + C::RELH_OFF);  // [kh % RH][BM], * log2(e)
 
@@ -404,7 +405,7 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
     const unsigned char* src = reinterpret_cast<const unsigned char*>(vbase + (int64_t)kt * 64 * a.v_sn);
 #pragma unroll
     for (int m = 0; m < C::VDPW; ++m)
-      if (wave + C::WAVES * m < C::VP && (!C::ONES_ROW || voff[m] >= 0))
+      if (wave + C::WAVES * m < C::VP && voff[m] >= 0)
         lds_dma16(src, (unsigned int)voff[m], lds_base + C::V_OFF + buf * C::VTILE + (wave + C::WAVES * m) * 1024);
   };
   k_dma(0, 0);
@@ -440,7 +441,7 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
 
   // the spare pieces of V tile `buf`: (1, 0, ..) and zeros
   auto ones = [&](int buf) __attribute__((always_inline)) {
-    if (C::ONES_ROW && tid < 64) {
+    if (tid < 64) {
       u32x4* p = reinterpret_cast<u32x4*>(lds + C::V_OFF + buf * C::VTILE + tid * (C::VP * 16) + HD * 2);
       p[0] = u32x4{T::kOne, 0u, 0u, 0u};
       p[1] = u32x4{0u, 0u, 0u, 0u};
@@ -490,7 +491,7 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
   for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
-  float m_i = T::kLowest, l_i = 0.f;
+  float m_i = T::kLowest;
 
   const int nkt = a.N / 64;
   typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -524,11 +525,9 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
     __builtin_amdgcn_sched_barrier(0);
 
     unsigned int seen = 0u;
-    float l0 = 0.f, l1 = 0.f;  // this row's share of the denominator, unrounded (two chains)
     auto pair = [&](int w, float neg_mrow) __attribute__((always_inline)) {  // packed pair w of 8
       const float p0 = fast_exp2(fmaf(s[2 * w], a.c, neg_mrow)), p1 = fast_exp2(fmaf(s[2 * w + 1], a.c, neg_mrow));
       pk[w >> 2][w & 3] = T::pack2(p0, p1);
-      if (!C::ONES_ROW) l0 += p0 + p1;
     };
     auto score = [&](int ks) __attribute__((always_inline)) { s_next = T::mfma(kf[ks], qf[ks], ks == 0 ? b1 : s_next); };
     auto pv = [&](int j, int dt) __attribute__((always_inline)) { oacc[dt] = T::mfma(vf[j][dt], pk_prev[j], oacc[dt]); };
@@ -538,13 +537,10 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
 #pragma unroll
     for (int g = 0; g < 8; ++g) {
       const float x0 = fmaf(s[2 * g], a.c, neg_mrow), x1 = fmaf(s[2 * g + 1], a.c, neg_mrow);
-      if (g > 0) {
-        pk[(g - 1) >> 2][(g - 1) & 3] = T::pack2(e0, e1);
-        if (!C::ONES_ROW) l0 += e0, l1 += e1;
-      }
+      if (g > 0) pk[(g - 1) >> 2][(g - 1) & 3] = T::pack2(e0, e1);
       e0 = fast_exp2(x0);
       e1 = fast_exp2(x1);
-      if (C::ONES_ROW && g > 0 && !(g & 1)) seen = T::note(seen, pk[(g - 1) >> 2][(g - 2) & 3], pk[(g - 1) >> 2][(g - 1) & 3]);
+      if (g > 0 && !(g & 1)) seen = T::note(seen, pk[(g - 1) >> 2][(g - 2) & 3], pk[(g - 1) >> 2][(g - 1) & 3]);
       __builtin_amdgcn_sched_barrier(0);
       if (g == 0) pv(0, 0);
       if (g == 1) {
@@ -565,9 +561,8 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
 #pragma unroll
       for (int dt = 0; dt < C::DT; ++dt) read_v(j, dt, BUF);
     pk[1][3] = T::pack2(e0, e1);
-    if (C::ONES_ROW) seen = T::note(seen, pk[1][2], pk[1][3]);
-    else l0 = (l0 + e0) + (l1 + e1);
-    if (__any(C::ONES_ROW ? T::outgrown(seen) : l0 > kCeiling)) {  // move the reference, as above
+    seen = T::note(seen, pk[1][2], pk[1][3]);
+    if (__any(T::outgrown(seen))) {  // move the reference, as above
       float mx = s[0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
@@ -575,8 +570,6 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
       const float m_new = fmaxf(m_i, fmaf(mx, a.c, b0 + T::kMargin));
       const float alpha = fast_exp2(m_i - m_new);
       m_i = m_new;
-      l_i *= alpha;
-      l0 = 0.f;
 #pragma unroll
       for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
@@ -584,7 +577,6 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
 #pragma unroll
       for (int w = 0; w < 8; ++w) pair(w, b0 - m_i);
     }
-    if (!C::ONES_ROW) l_i += l0;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of K row kt + 2 and V row kt + 1 has landed
     __syncthreads();
     if (kt + 2 < nkt) v_dma(kt + 2, BUF);  // row kt's V is in registers
@@ -603,39 +595,31 @@ __global__ __launch_bounds__(64 * SplitCfg<HD>::WAVES, HD == 64 ? 3 : 2) void at
 #pragma unroll
     for (int dt = 0; dt < C::DT; ++dt) oacc[dt] = T::mfma(vf[j][dt], pkB[j], oacc[dt]);  // P V of the last row
 
-  // ---- the two key halves meet: reference, denominator and accumulators of half 1 through LDS ----
-  float* other = reinterpret_cast<float*>(lds) + qt * 64 * (16 * C::DT + 2) + lane;  // word w of lane: 64 w + lane
+  // ---- the two key halves meet: reference and accumulators (the denominator among them) of half 1 through LDS ----
+  float* other = reinterpret_cast<float*>(lds) + qt * 64 * (16 * C::DT + 1) + lane;  // word w of lane: 64 w + lane
   if (kg == 1) {
 #pragma unroll
     for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) other[64 * (16 * dt + r)] = oacc[dt][r];
     other[64 * 16 * C::DT] = m_i;
-    other[64 * (16 * C::DT + 1)] = l_i;
   }
   __syncthreads();
   if (kg == 1) return;
   {
     // (a half all of whose keys are taken away: its reference is T::kLowest, its sums are zero)
-    const float m1 = other[64 * 16 * C::DT], l1 = other[64 * (16 * C::DT + 1)];
+    const float m1 = other[64 * 16 * C::DT];
     const float m = fmaxf(m_i, m1);
     const float f0 = fast_exp2(m_i - m), f1 = fast_exp2(m1 - m);
-    l_i = l_i * f0 + l1 * f1;
 #pragma unroll
     for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) oacc[dt][r] = oacc[dt][r] * f0 + other[64 * (16 * dt + r)] * f1;
   }
-  float l;
-  if (C::ONES_ROW) {
-    constexpr int orow = HD % 32;
-    constexpr int oreg = 4 * (orow / 8) + orow % 4, olh = (orow / 4) % 2;
-    const float own = oacc[C::DT - 1][oreg], partner = xor32(own);
-    l = (lh == olh) ? own : partner;
-  } else {
-    l = l_i + xor32(l_i);
-  }
-  const float inv = 1.0f / l;
+  constexpr int orow = HD % 32;  // the denominator's row of the last channel tile
+  constexpr int oreg = 4 * (orow / 8) + orow % 4, olh = (orow / 4) % 2;
+  const float own = oacc[C::DT - 1][oreg], partner = xor32(own);
+  const float inv = 1.0f / (lh == olh ? own : partner);
   unsigned short* op = a.out + b * a.o_sb + h * a.o_sh + (int64_t)(q0 + lr) * a.o_sn;
 #pragma unroll
   for (int dt = 0; dt < C::DT; ++dt)
@@ -953,10 +937,10 @@ __global__ __launch_bounds__(64 * Split16Cfg::WAVES, 3) void attn_global_split16
 }
 
 // Which form of the global kernel.  Split keys round differently from unsplit ones, so that choice looks at head_dim
-// alone: a slice has the same bits whatever batch it travels in.  hd 64 is split (us, split / unsplit with 8 / with 4
-// wavefronts, 4096 tokens: 1 x 8 heads 48 / 73 / 53, 1 x 12: 66 / 71 / 76, 2 x 9: 102 / 142 / 116, 1 x 16: 87 / 79 / 82,
-// 8 x 16: 655 / 628 / 634), hd 80, where only two such workgroups fit a CU, is not (55 / 74 / 59, 84 / 78 / 83, 130 / 159 / 136,
-// 105 / 91 / 95, 851 / 714 / 730).  8 wavefronts or 4, which agree bit for bit: by how the workgroups of 256
+// alone: a slice has the same bits whatever batch it travels in.  hd 64 is split (us in bf16, split / unsplit with 8 / with 4
+// wavefronts, 4096 tokens: 1 x 8 heads 49 / 68 / 50, 1 x 12: 65 / 69 / 76, 2 x 9: 101 / 143 / 118, 1 x 16: 87 / 79 / 83, 4 x 12: 239 / 236 / 236,
+// 8 x 16: 629 / 622 / 617), hd 80, where only two such workgroups fit a CU, is not (55 / 73 / 56, 84 / 76 / 83, 130 / 159 / 136, 106 / 92 / 96, 307 / 272 / 274,
+// 818 / 715 / 718).  8 wavefronts or 4, which agree bit for bit: by how the workgroups of 256
 // queries (one per CU) and of 128 (two) divide among the 256 CUs.  The prices are microseconds of one full round over
 // 64 key rows and, of 128 queries, of a last one with one workgroup per CU.
 // Returns 8, 4, or 2 for the key-split form.
@@ -980,7 +964,7 @@ static void launch_bias(const AttnArgs& a, int form, hipStream_t stream) {
     if ((int64_t)a.B * a.nH * (a.N / 64) <= 256) hipLaunchKernelGGL((attn_global_split16_kernel<T, true>), grid(64), dim3(256), 0, stream, a);
     else hipLaunchKernelGGL((attn_global_split16_kernel<T, false>), grid(64), dim3(256), 0, stream, a);
   }
-  else hipLaunchKernelGGL((attn_global_split_kernel<T, HD>), grid(64), dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL((attn_global_split_kernel<T>), grid(64), dim3(256), 0, stream, a);
 }
 
 int attn_global_bias_launch(const AttnArgs& a0, int hd, int dtype, hipStream_t stream) {
