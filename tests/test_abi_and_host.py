@@ -868,8 +868,8 @@ def test_a_linear_of_another_type_is_unsupported_in_every_form(M, N, K):
     assert lib.samfast_linear_i8_sparse24(p[0], K, p[1], p[2], p[3], p[4], p[5], N, p[6], M, N, K, _lib.SAMFAST_F16, None) == -2
 
 
-def test_the_native_modules_entries_decline_what_they_do_not_cover():
-    """A module's Linear on the CPU, with a buffer missing or none at all, is left to the Python route."""
+def test_the_native_modules_entries_decline_rows_on_the_cpu():
+    """Such a call, or one without a module's buffers, is left to the Python route."""
     from samfast_amd import _lib
     from samfast_amd.quant import Int8DynamicLinear
     host = _lib.host()

@@ -65,6 +65,47 @@ def test_a_linear_reads_its_weights_as_they_stand(M, N, K):
     assert torch.equal(lin(x), _unfused(other, x))
 
 
+@pytest.mark.parametrize("sparse", [False, True])
+def test_the_native_modules_entries_look_buffers_up_by_name(sparse):
+    """Rows on the GPU: a buffer that is missing, None or of another type is declined, a missing bias is none, and a replaced buffer counts from the next call on."""
+    from samfast_amd import Int8DynamicLinear, Int8Sparse24Linear, _lib
+    print(f"case buffers by name sparse={sparse}", flush=True)
+    make = Int8Sparse24Linear if sparse else Int8DynamicLinear
+    entry = _lib.host().module_sparse_linear if sparse else _lib.host().module_linear
+    gen = torch.Generator().manual_seed(11)
+    floats = [torch.nn.Linear(256, 264, dtype=torch.bfloat16) for _ in range(2)]
+    for f in floats:
+        with torch.no_grad():
+            f.weight.copy_(torch.randn((264, 256), generator=gen) * 0.02)
+            f.bias.copy_(torch.randn(264, generator=gen))
+    lin, other = (make.from_float(f.cuda()) for f in floats)
+    x = torch.randn((9, 256), generator=gen).to(torch.bfloat16).cuda()
+    y = entry(x, lin._buffers)
+    assert y is not None and torch.equal(y, lin(x))
+    weights = ("wc", "widx", "sw_bits") if sparse else ("wq", "sw_bits")
+    for name in weights:
+        without = {k: v for k, v in lin._buffers.items() if k != name}
+        assert entry(x, without) is None, name
+        assert entry(x, {**without, name: None}) is None, name
+        assert entry(x, {**without, name: lin._buffers[name].cpu()}) is None, name
+        assert entry(x, {**without, name: lin._buffers[name].float()}) is None, name
+    floats[0].bias = None
+    unbiased = make.from_float(floats[0])(x)
+    assert not torch.equal(unbiased, y)
+    without = {k: v for k, v in lin._buffers.items() if k != "bias_bits"}
+    for buffers in (without, {**without, "bias_bits": None}):
+        assert torch.equal(entry(x, buffers), unbiased)
+    buffers = dict(lin._buffers)
+    for name in weights + ("bias_bits",):
+        buffers[name] = other._buffers[name]
+    assert torch.equal(entry(x, buffers), other(x))
+    lin.load_state_dict(other.state_dict())
+    assert torch.equal(lin(x), other(x))
+    for wrong in ({}, None, [], 5):
+        assert entry(x, wrong) is None
+    assert entry(x) is None
+
+
 @pytest.mark.parametrize("M", [7, 4096, 16384])
 def test_a_linears_first_call_anywhere(M):
     """Built in inference mode; first called while a graph is recorded; then called from another stream."""
