@@ -315,7 +315,7 @@ def test_seeded_sweep_of_ragged_shapes_sparse_bit_exact():
 @pytest.mark.parametrize("M,N,K,epi", [(1, 8, 512, 0), (5003, 1280, 5120, 0), (130, 264, 768, 1), (4096, 768, 3072, 2), (129, 1288, 512, 2), (257, 520, 1280, 1), (6528, 1280, 5120, 2)])
 @pytest.mark.parametrize("layout", [0, 1])
 def test_sparse24_split_k_loop_agrees(M, N, K, epi, layout):
-    """Two wavefront groups on alternate k tiles: the bits of one group walking them all."""
+    """Two sides that take turns on K tiles of 128 values, their integer sums joined at the end: the bits of one group walking them all."""
     from samfast_amd import _lib, ops
     print(f"case sparse split M={M} N={N} K={K} epi={epi} layout={layout}", flush=True)
     g = torch.Generator().manual_seed(M + N + K)

@@ -136,25 +136,6 @@ def test_pack_2_of_4_round_trip_and_invariants():
         assert np.array_equal(orq.unpack_2_of_4(wc2, widx2), pruned)
 
 
-def test_quotient_in_three_steps_gives_every_code():
-    """q = v * inv, q + (v - q * scale) * inv with fused multiply-adds, as linear_i8_band.hip forms codes: the oracle's code for
-    every bf16 row maximum of three exponents (and the smallest and largest) and every bf16 value down to 2^-9 of it."""
-    f32 = np.float32
-    values = (np.arange(0x7f80, dtype=np.uint32) << 16).view(f32)  # all finite ones that are not negative
-
-    def fma(a, b, c):  # the product of two float32 is exact in float64, the sum in an extended type but for bits far below
-        return (a.astype(np.float64) * b.astype(np.float64) + c.astype(np.longdouble)).astype(f32)
-
-    maxima = [1, 0x80, 0x3700, 0x3728, 0x7f7f] + [e * 128 + m for e in (110, 127, 140) for m in range(128)]
-    for i in maxima:
-        v = values[max(0, i - 9 * 128):i + 1]
-        scale = np.full_like(v, max(values[i], f32(1e-5)) / f32(127))
-        inv = f32(1) / scale
-        q = v * inv
-        code = np.rint(fma(fma(-q, scale, v), inv, q))
-        assert np.array_equal(code, np.rint(v / scale)), i
-
-
 def test_one_product_gives_every_code():
     """rint(v * factor) with one rounding, as quant_row.hpp forms codes (a fused multiply-add with 1.5 * 2^23): the oracle's code for the same
     maxima and values, the factor being 1 / scale or its neighbour, on the side where the division puts half of the maximum."""
