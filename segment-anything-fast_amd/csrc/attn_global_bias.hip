@@ -643,7 +643,9 @@ __global__ __launch_bounds__(64 * SplitCfg::WAVES, 2) void attn_global_split_ker
 // Up to 256 workgroups are one wavefront a SIMD, which waits for the matrix pipe between a step's two instructions if they stand side by side: there
 // they stand apart, one on either side of the exponentials (the same operations: the same bits.  us, 32 x 32 x 16 / side by side / apart, bf16; fp16: 2 x 1 heads 30.3 / 32.4 / 30.9;
 // 31.2 / 32.6 / 31.0, 2 x 3 x 40 rows 21.4 / 22.8 / 21.9, 4 x 1 x 40 fp16 21.8 / 22.8 / 21.8; over 61 calls 1.045 and 1.01 times as long as the 32 x 32 form, whose half as many
-// instructions that wavefront issues sooner).  From 257 to 384 the two are level, beyond, where other wavefronts fill the wait, side by side is ahead by up to 1.3 %.
+// instructions that wavefront issues sooner).  From 257 to 448, where other wavefronts fill the wait, side by side is up to 2 % ahead, beyond the two are level.
+// What the smaller instruction does not gain in bf16: one wavefront a SIMD on some CUs and two on others (1 x 5 heads 41.7 / 42.6, 1 x 6 42.6 / 42.8; fp16 42.7 / 42.4, 43.7 / 42.7), and
+// single calls on an idle GPU, which the power limit does not reach (1 x 5 51.5 / 53.0, 1 x 12 73.4 / 73.3, 8 x 16 665 / 670; fp16 53.0 / 53.2, 77.2 / 75.2, 704 / 685).
 struct Split16Cfg {
   using R = GridRow<64>;
   static constexpr int QW = 2, WAVES = 2 * QW, BM = 32 * QW;  // query tiles of 32 and two key halves

@@ -1,8 +1,8 @@
 // Per-row symmetric int8 quantiser (bf16 -> int8 + fp32 scale), optionally preceded
 // by LayerNorm over the row and a row gather (window partition).  HBM-bound: 65536 rows of 5120 through GELU 216 us, of 1280
 // plain 46, with LayerNorm 54, codes written into new memory each time (4.7, 5.5 and 4.6 TB/s; a copy reaches 4.9 from HBM); rows that lie in the
-// caches by the vector ALU as well: 144 vector instructions per row of 1280 plain, 291 with LayerNorm, 1374 per row of 5120 with GELU, by the hardware
-// counters, for a wavefront per row.  us with the quotient made exact in three steps / codes from one product (quant_row.hpp): 4096 x 1024 3.52 / 3.30, with LayerNorm
+// caches by the vector ALU as well: 144 vector instructions per row of 1280 plain, 338 with LayerNorm, 1374 per row of 5120 with GELU, by the hardware
+// counters, for a wavefront per row (with LayerNorm 291 where wavefronts walk the rows of 65536).  us with the quotient made exact in three steps / codes from one product (quant_row.hpp): 4096 x 1024 3.52 / 3.30, with LayerNorm
 // 4.63 / 4.36, 4096 x 4096 9.9 / 9.7, with GELU 14.6 / 13.8, 5003 x 5120 with GELU 20.1 / 18.9, 20480 x 1024 with LayerNorm 15.2 / 14.2, 65536 x 5120 with GELU 212 / 213,
 // 65536 x 1280 with LayerNorm 53.4 / 53.6.
 //
