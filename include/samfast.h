@@ -119,6 +119,25 @@ int samfast_attn_relpos_windowed_fwd(
     int dtype, float sm_scale, void* stream);
 
 /*
+ * The same, told what the launches behind it will read: soon_n buffers on the same GPU (at most
+ * SAMFAST_MAX_SOON; soon_bytes[i] bytes from soon[i]; the two arrays are read before the call returns).  Wavefronts that have no
+ * queries read a word of each of their cache lines while the others multiply, so that they come out of the last-level cache when
+ * they are wanted; results do not depend on it.  The buffers have to stay allocated as long as q does.
+ */
+#define SAMFAST_MAX_SOON 8
+int samfast_attn_relpos_windowed_soon_fwd(
+    const void* q, const void* k, const void* v,
+    const void* rel_pos_h, const void* rel_pos_w,
+    const void* pad_k, const void* pad_v, void* out,
+    int B, int nH, int img_h, int img_w, int ws, int hd,
+    int64_t q_sb, int64_t q_sh, int64_t q_sn,
+    int64_t k_sb, int64_t k_sh, int64_t k_sn,
+    int64_t v_sb, int64_t v_sh, int64_t v_sn,
+    int64_t o_sb, int64_t o_sh, int64_t o_sn,
+    int dtype, float sm_scale,
+    const void* const* soon, const int64_t* soon_bytes, int soon_n, void* stream);
+
+/*
  * Same attention with the two bias factors already computed by the caller:
  *   rel_h: (B, nH, N, gh) addressed ptr + b*rh_sb + h*rh_sh + n*rh_sn + j
  *   rel_w: (B, nH, N, gw) addressed ptr + b*rw_sb + h*rw_sh + n*rw_sn + j

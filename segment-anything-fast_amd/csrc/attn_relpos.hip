@@ -445,7 +445,8 @@ struct WindowCfg {
   static_assert(NT <= WAVES, "one query tile per wavefront");
 };
 
-template <typename T, int HD, bool FUSED, int TILES>
+// SOON: with AttnArgs::soon (a form of its own: the others' code stays as short as it is)
+template <typename T, int HD, bool FUSED, int TILES, bool SOON = false>
 __global__ __launch_bounds__((WindowCfg<HD, TILES>::THREADS), 2) void attn_window_kernel(AttnArgs a) {
   using C = WindowCfg<HD, TILES>;
   __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS_BYTES];
@@ -691,6 +692,13 @@ __global__ __launch_bounds__((WindowCfg<HD, TILES>::THREADS), 2) void attn_windo
   if (FUSED && !has_tile) {  // a wavefront without a query tile only helps with the staging and with the output
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();  // V complete (the barrier the others reach after their first score tile)
+    // The last wavefront of seven tiles' eight has none: it reads what comes next, while the others multiply, for 0.9 us of a launch of 20.  The
+    // words go behind the last key's row, where nobody looks: to registers, four at a time, an image's 38 MB took 7 us.  (The global kernel has no such
+    // wavefront: a chunk of each wavefront's every eight key rows, awaited with the next tile, lengthened it by 7 of 98 us.)
+    if constexpr (SOON)
+      if (wave_u == 7)
+        for (SoonWalk w(a, blockIdx.x); w.more(); w.on(gridDim.x))
+          __builtin_amdgcn_global_load_lds((gptr_t)w.word(lane), (lptr_t)(kl + N * C::KSTR * 2), 4, 0, 0);
   }
 
   if (has_tile) {
@@ -890,6 +898,7 @@ static int launch_hd(const AttnArgs& a, bool global_path, hipStream_t stream) {
     else launch(std::integral_constant<int, 4>{});
     return check_launch("attn_global_kernel");
   }
+  using C7 = WindowCfg<HD, 7>;
   const int64_t wins = a.ws > 0 ? (int64_t)a.B * a.wins_x * a.wins_y : a.B;
   const int64_t total = wins * a.nH;
   AttnArgs b = a;
@@ -931,7 +940,13 @@ static int launch_hd(const AttnArgs& a, bool global_path, hipStream_t stream) {
   b.part_tiles = (ntq + parts - 1) / parts;
   b.parts = (ntq + b.part_tiles - 1) / b.part_tiles;
   const unsigned int grid = (unsigned int)((b.whole + ((total - b.whole) * b.parts + 7) / 8 * 8));
-  hipLaunchKernelGGL((attn_window_kernel<T, HD, FUSED, 7>), dim3(grid), dim3(WindowCfg<HD, 7>::THREADS), 0, stream, b);
+  if constexpr (FUSED) {
+    if (a.soon_n > 0 && grid < (1u << 20) && (C7::NMAX - a.N) * C7::KSTR * 2 >= 256) {  // room for the words that are read
+      hipLaunchKernelGGL((attn_window_kernel<T, HD, FUSED, 7, true>), dim3(grid), dim3(C7::THREADS), 0, stream, b);
+      return check_launch("attn_window_kernel");
+    }
+  }
+  hipLaunchKernelGGL((attn_window_kernel<T, HD, FUSED, 7>), dim3(grid), dim3(C7::THREADS), 0, stream, b);
   return check_launch("attn_window_kernel");
 }
 
@@ -1003,6 +1018,21 @@ static int attn_dispatch(bool fused, AttnArgs& a, int hd, int dtype, float sm_sc
   return dtype == SAMFAST_F16 ? by_type(ElemF16{}) : by_type(ElemBf16{});
 }
 
+static int attn_soon(AttnArgs& a, const void* const* soon, const int64_t* bytes, int n) {
+  SF_REQUIRE(n >= 0 && n <= SAMFAST_MAX_SOON && (n == 0 || (soon && bytes)), "attn_relpos: bad list of buffers read soon");
+  a.soon_n = 0;
+  for (int i = 0; i < n; ++i) {
+    SF_REQUIRE(bytes[i] >= 0 && (bytes[i] == 0 || soon[i]), "attn_relpos: bad list of buffers read soon");
+    // words at multiples of a line from the first aligned one, all of them inside
+    const uintptr_t from = (reinterpret_cast<uintptr_t>(soon[i]) + 3u) & ~(uintptr_t)3u;
+    const int64_t inside = bytes[i] - (int64_t)(from - reinterpret_cast<uintptr_t>(soon[i]));
+    if (inside < 4) continue;
+    a.soon[a.soon_n] = reinterpret_cast<const unsigned int*>(from);
+    a.soon_lines[a.soon_n++] = (unsigned int)min((inside - 4) / kSoonLine + 1, (int64_t)1 << 28);
+  }
+  return SAMFAST_OK;
+}
+
 }  // namespace samfast
 
 extern "C" int samfast_attn_relpos_fwd(
@@ -1042,13 +1072,13 @@ extern "C" int samfast_attn_relpos_bias_fwd(
   return samfast::attn_dispatch(false, a, hd, dtype, sm_scale, reinterpret_cast<hipStream_t>(stream));
 }
 
-extern "C" int samfast_attn_relpos_windowed_fwd(
+extern "C" int samfast_attn_relpos_windowed_soon_fwd(
     const void* q, const void* k, const void* v, const void* rel_pos_h, const void* rel_pos_w,
     const void* pad_k, const void* pad_v, void* out,
     int B, int nH, int img_h, int img_w, int ws, int hd,
     int64_t q_sb, int64_t q_sh, int64_t q_sn, int64_t k_sb, int64_t k_sh, int64_t k_sn,
     int64_t v_sb, int64_t v_sh, int64_t v_sn, int64_t o_sb, int64_t o_sh, int64_t o_sn,
-    int dtype, float sm_scale, void* stream) {
+    int dtype, float sm_scale, const void* const* soon, const int64_t* soon_bytes, int soon_n, void* stream) {
   using us = unsigned short;
   samfast::AttnArgs a = {};
   if (ws <= 0) {
@@ -1061,5 +1091,18 @@ extern "C" int samfast_attn_relpos_windowed_fwd(
   a.q_sb = q_sb; a.q_sh = q_sh; a.q_sn = q_sn; a.k_sb = k_sb; a.k_sh = k_sh; a.k_sn = k_sn;
   a.v_sb = v_sb; a.v_sh = v_sh; a.v_sn = v_sn; a.o_sb = o_sb; a.o_sh = o_sh; a.o_sn = o_sn;
   a.B = B; a.nH = nH; a.gh = ws; a.gw = ws; a.img_h = img_h; a.img_w = img_w; a.ws = ws;
+  if (const int code = samfast::attn_soon(a, soon, soon_bytes, soon_n)) return code;
   return samfast::attn_dispatch(true, a, hd, dtype, sm_scale, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int samfast_attn_relpos_windowed_fwd(
+    const void* q, const void* k, const void* v, const void* rel_pos_h, const void* rel_pos_w,
+    const void* pad_k, const void* pad_v, void* out,
+    int B, int nH, int img_h, int img_w, int ws, int hd,
+    int64_t q_sb, int64_t q_sh, int64_t q_sn, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+    int64_t v_sb, int64_t v_sh, int64_t v_sn, int64_t o_sb, int64_t o_sh, int64_t o_sn,
+    int dtype, float sm_scale, void* stream) {
+  return samfast_attn_relpos_windowed_soon_fwd(
+      q, k, v, rel_pos_h, rel_pos_w, pad_k, pad_v, out, B, nH, img_h, img_w, ws, hd, q_sb, q_sh, q_sn, k_sb, k_sh,
+      k_sn, v_sb, v_sh, v_sn, o_sb, o_sh, o_sn, dtype, sm_scale, nullptr, nullptr, 0, stream);
 }

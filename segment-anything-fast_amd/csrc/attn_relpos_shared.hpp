@@ -31,8 +31,15 @@ struct AttnArgs {
   int relh_x8;  // attn_global_bias.hip: rel_h rows can be read 16 bytes at a time
   int rel_x2;   // window kernel: rows of the caller's factors can be read 4 bytes at a time
   int whole, parts, part_tiles;  // window kernel: items with a workgroup each; the others are `parts` workgroups of part_tiles query tiles
+  // Window kernel: operands of the launches behind this one.  One word of every kSoonLine bytes is read, by wavefronts that have nothing
+  // else to do, so that they stand in the last-level cache when they are wanted.  Nothing depends on it.
+  // (At the end: of the arguments every launch looks at, in memory of the host's, no cache line more.)
+  int soon_n;
+  unsigned int soon_lines[SAMFAST_MAX_SOON];
+  const unsigned int* soon[SAMFAST_MAX_SOON];
 };
 
+constexpr int kSoonLine = 64;  // what a miss of one word brings (at 128 the other halves still came from HBM)
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazyLog2 = 8.0f;  // softmax reference lags the running maximum by at most 2^8
 
@@ -94,6 +101,27 @@ struct ElemF16 {
   static SF_DEVICE float from_bits(unsigned short h) { return (float)__builtin_bit_cast(_Float16, h); }
   static SF_DEVICE float lo(unsigned int w) { return from_bits((unsigned short)(w & 0xffffu)); }
   static SF_DEVICE float hi(unsigned int w) { return from_bits((unsigned short)(w >> 16)); }
+};
+
+// Walks them (see AttnArgs::soon) in chunks of 64 lines, every `step`th one; all of it uniform.
+struct SoonWalk {
+  const AttnArgs& a;
+  int s = 0;
+  unsigned int line, lines;  // of operand s: the chunk's first, and all
+  const unsigned int* p;
+  SF_DEVICE SoonWalk(const AttnArgs& args, unsigned int chunk) : a(args), line(64u * chunk), lines(args.soon_lines[0]), p(args.soon[0]) {}
+  SF_DEVICE bool more() {
+    while (s < a.soon_n && line >= lines) {
+      line -= (lines + 63u) & ~63u;  // (to chunks: at least this much)
+      if (++s < a.soon_n) {
+        lines = a.soon_lines[s];
+        p = a.soon[s];
+      }
+    }
+    return s < a.soon_n;
+  }
+  SF_DEVICE const unsigned int* word(int lane) const { return p + (kSoonLine / 4) * min(line + lane, lines - 1u); }
+  SF_DEVICE void on(unsigned int step) { line += 64u * step; }
 };
 
 SF_DEVICE u32x4 load_x8_global(const unsigned short* p) { return *reinterpret_cast<const u32x4*>(p); }

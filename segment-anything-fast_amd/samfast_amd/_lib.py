@@ -29,6 +29,8 @@ _SIGNATURES = {
         _i32, [_ptr] * 6 + [_i32] * 5 + [_i64] * 12 + [_i32, _f32, _ptr]),
     "samfast_attn_relpos_windowed_fwd": (
         _i32, [_ptr] * 8 + [_i32] * 6 + [_i64] * 12 + [_i32, _f32, _ptr]),
+    "samfast_attn_relpos_windowed_soon_fwd": (
+        _i32, [_ptr] * 8 + [_i32] * 6 + [_i64] * 12 + [_i32, _f32, _ptr, _ptr, _i32, _ptr]),
     "samfast_attn_relpos_bias_fwd": (
         _i32, [_ptr] * 6 + [_i32] * 5 + [_i64] * 18 + [_i32, _f32, _ptr]),
     "samfast_quant_rowwise_i8": (_i32, [_ptr, _i64, _ptr, _ptr, _i64, _i32, _i32, _i32, _ptr]),
@@ -77,6 +79,8 @@ _BENCH_SIGNATURES = {
     "samfast_bench_mfma_ceiling": (_i32, [_i32, _ptr, _i32, _i32, ctypes.POINTER(_i64), _ptr, _ptr]),
     "samfast_bench_mfma_valu_overlap": (_i32, [_i32, _ptr, _i32, _i32, _i32, _ptr, _ptr]),
 }
+
+MAX_SOON = 8
 
 EPILOGUE_NONE, EPILOGUE_GELU, EPILOGUE_RESIDUAL = 0, 1, 2
 LAYOUT_ROWMAJOR, LAYOUT_KB64 = 0, 1

@@ -25,7 +25,7 @@ module-by-module composition.
 """
 
 import os
-from typing import Optional, Tuple, Type
+from typing import Optional, Sequence, Tuple, Type
 
 import torch
 import torch.nn as nn
@@ -40,7 +40,27 @@ WINDOWS_IN_PLACE = os.environ.get("SAMFAST_WINDOWS_IN_PLACE", "1") != "0"
 # The neck on the kernels here up to this many tokens; beyond, the library's larger convolution tiles are ahead (us, library / here,
 # width 1280: one image 107 / 45, four 198 / 102, eight 284 / 187, sixteen 261 / 365)
 NECK_TOKENS = 40960
+# Weights that a window attention kernel reads ahead of the products behind it (read_soon): up to this many tokens, this many
+# bytes a block, and from this many bytes over all blocks on
+SOON_TOKENS, SOON_BYTES, SOON_TOTAL = 8192, 9 << 20, 85 << 20
 FUSED_BLOCK = bool(int(os.environ.get("SAMFAST_FUSED_BLOCK", 1)))
+
+
+def read_soon(depth: int, tokens: int, weights: Sequence[torch.Tensor]) -> Sequence[torch.Tensor]:
+    """Of `weights`, those of the products behind one of `depth` blocks' attention, what the window kernel's idle wavefront reads
+    while the others multiply.  The weights of an encoder that exceeds the last-level cache come out of HBM in every pass, and an
+    image's products wait for them a k tile at a time: proj first, then lin2, whose loop is the longest, then the next
+    block's qkv, while they stay few enough to arrive under the attention; lin1's gains less than it costs there.  us a pass, none / so:
+    one image of ViT-L int8 3151 / 3024, ViT-H int8 4915 / 4788, with 2:4 MLPs 4833 / 4607, bf16 ViT-B 1512 / 1501, ViT-L 3494 / 3446,
+    ViT-H 6054 / 5947 (proj alone; with lin2 6135), two of ViT-L int8 5204 / 5081; all four Linears' ViT-H int8 4930, bf16 6160 (4949 and 6099
+    without on that box).  An encoder that the cache holds is slower by it (ViT-B int8 1324 / 1329), and from four images on it is
+    level (ViT-H int8 16284 / 16309)."""
+    if tokens > SOON_TOKENS:
+        return ()
+    sizes = [w.numel() * w.element_size() for w in weights]
+    if depth * sum(sizes) < SOON_TOTAL:
+        return ()
+    return [w for i, w in enumerate(weights) if sum(sizes[:i + 1]) <= SOON_BYTES]
 
 
 class ImageEncoderViT(nn.Module):
@@ -119,13 +139,13 @@ class ImageEncoderViT(nn.Module):
                     continue
                 nxt = self.blocks[i + 1] if i + 1 < len(self.blocks) else None
                 chained = nxt is not None and not nxt._int8_fused_ok(x) and nxt._half_fused_ok(x)
-                x, carry = blk._forward_half_fused(x, carry, nxt.norm1 if chained else None)
+                x, carry = blk._forward_half_fused(x, carry, nxt.norm1 if chained else None, nxt.attn.qkv if chained else None, len(self.blocks))
                 continue
             nxt = self.blocks[i + 1] if i + 1 < len(self.blocks) else None
-            next_norm = None
+            next_norm = next_qkv = None
             if nxt is not None and nxt._int8_fused_ok(x) and nxt._chains_from_previous():
-                next_norm = (nxt.norm1.weight, nxt.norm1.bias, nxt.norm1.eps)
-            x, carry = blk._forward_int8_fused(x, carry, next_norm)
+                next_norm, next_qkv = (nxt.norm1.weight, nxt.norm1.bias, nxt.norm1.eps), nxt.attn.qkv
+            x, carry = blk._forward_int8_fused(x, carry, next_norm, next_qkv, len(self.blocks))
         return x
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
@@ -236,12 +256,13 @@ class Block(nn.Module):
         its rows must be the image-ordered tokens (no window gather in front of qkv)."""
         return self.window_size == 0 or WINDOWS_IN_PLACE
 
-    def _forward_int8_fused(self, x: torch.Tensor, carry=None, next_norm=None):
+    def _forward_int8_fused(self, x: torch.Tensor, carry=None, next_norm=None, next_qkv=None, depth=0):
         """image_encoder.py:167-183 with every step on the HIP kernels.
 
         `carry` = (xq, sx): this block's norm1 output, already quantised by the previous block's
         lin2 launch.  `next_norm` = (gamma, beta, eps) of the next block's norm1: lin2 then
-        also returns that block's carry.  Returns (tokens (B, H, W, C), carry for the next block)."""
+        also returns that block's carry; `next_qkv`: that block's first Linear; `depth`: of how many
+        blocks this is one (0: of none).  Returns (tokens (B, H, W, C), carry for the next block)."""
         from .. import quant
         B, H, W, C = x.shape
         attn, mlp = self.attn, self.mlp
@@ -278,8 +299,9 @@ class Block(nn.Module):
                 # the attention kernel cuts the windows itself; the reference's zero-padded tokens
                 # enter as keys / values with the rows a zero input gives the qkv Linear: its bias
                 pad_k, pad_v = self._pad_rows(nH, hd, x.device)
+                soon = read_soon(depth, B * H * W, [t for m in (attn.proj, mlp.lin2, next_qkv) if m is not None for t in m.weight_operands(L)])
                 o = ops.attn_relpos_windowed(q, k, v, attn.rel_pos_h, attn.rel_pos_w, pad_k, pad_v,
-                                             (H, W), ws, attn.scale).view(B * H * W, C)
+                                             (H, W), ws, attn.scale, soon).view(B * H * W, C)
             else:
                 o = ops.attn_relpos(q, k, v, attn.rel_pos_h, attn.rel_pos_w, (H, W), attn.scale)
                 o = o.permute(0, 2, 1, 3).reshape(B * H * W, C)
@@ -347,13 +369,13 @@ class Block(nn.Module):
                 and ops.attn_supported(gh * gw, (gh, gw), C // attn.num_heads, x.dtype)
                 and (ws == 0 or ws * ws <= 208))
 
-    def _forward_half_fused(self, x: torch.Tensor, carry=None, next_norm=None):
+    def _forward_half_fused(self, x: torch.Tensor, carry=None, next_norm=None, next_qkv=None, depth=0):
         """image_encoder.py:167-183 with half-type Linears: four products, those that pay on this library's kernels with
         GELU or the residual add in them (ops.linear_half), and two or three launches around them.  The
         attention kernel cuts the windows out of the image-ordered tokens, so the products run on the image's tokens only
         (the zero-padded windows have a fifth more) and nothing is partitioned, padded or copied; a residual
         add that is in no product runs with the norm that follows it.
-        `carry`: norm1's output, where the previous block has made it; `next_norm`: the next block's norm1.
+        `carry`: norm1's output, where the previous block has made it; `next_norm`, `next_qkv`, `depth`: as above.
         Returns (tokens, carry for the next block)."""
         B, H, W, C = x.shape
         attn, mlp, ws = self.attn, self.mlp, self.window_size
@@ -368,7 +390,8 @@ class Block(nn.Module):
             # a zero-padded token's k and v rows: the qkv bias
             pads = (torch.zeros((2, nH, hd), dtype=x.dtype, device=x.device) if attn.qkv.bias is None
                     else attn.qkv.bias[C:].view(2, nH, hd))
-            o = ops.attn_relpos_windowed(q, k, v, attn.rel_pos_h, attn.rel_pos_w, pads[0], pads[1], (H, W), ws, attn.scale)
+            soon = read_soon(depth, B * H * W, [m.weight for m in (attn.proj, mlp.lin2, next_qkv) if m is not None])
+            o = ops.attn_relpos_windowed(q, k, v, attn.rel_pos_h, attn.rel_pos_w, pads[0], pads[1], (H, W), ws, attn.scale, soon)
         else:
             o = ops.attn_relpos(q, k, v, attn.rel_pos_h, attn.rel_pos_w, (H, W), attn.scale).permute(0, 2, 1, 3)
         o = o.reshape(B * H * W, C)

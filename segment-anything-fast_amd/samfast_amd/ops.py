@@ -5,8 +5,9 @@ Every function requires tensors on a GPU device and raises otherwise - there is
 no CPU or eager path behind these names.
 """
 
+import ctypes
 import math
-from typing import Optional, Tuple
+from typing import Optional, Sequence, Tuple
 
 import torch
 
@@ -101,6 +102,17 @@ def _check_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: Optional[
         raise RuntimeError("samfast: out must have the shape, dtype and device of q")
 
 
+def _soon(tensors: Sequence[torch.Tensor], device: torch.device):
+    """The list of buffers that the window kernel brings into the last-level cache while it multiplies: those of `tensors` that
+    are plain memory on this device."""
+    spans = [(t.data_ptr(), t.numel() * t.element_size()) for t in tensors
+             if type(t) in (torch.Tensor, torch.nn.Parameter) and t.device == device and t.is_contiguous()][:_lib.MAX_SOON]
+    if not spans:
+        return None, None, 0
+    n = len(spans)
+    return (ctypes.c_void_p * n)(*(p for p, _ in spans)), (ctypes.c_int64 * n)(*(b for _, b in spans)), n
+
+
 def attn_supported(N: int, grid_hw: Tuple[int, int], hd: int, dtype: torch.dtype) -> bool:
     """Shapes the HIP attention kernels cover (mirrors the checks in the library)."""
     gh, gw = grid_hw
@@ -149,10 +161,12 @@ def attn_relpos(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
 def attn_relpos_windowed(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                          rel_pos_h: torch.Tensor, rel_pos_w: torch.Tensor,
                          pad_k: torch.Tensor, pad_v: torch.Tensor,
-                         grid_hw: Tuple[int, int], window: int, scale: float) -> torch.Tensor:
+                         grid_hw: Tuple[int, int], window: int, scale: float,
+                         soon: Sequence[torch.Tensor] = ()) -> torch.Tensor:
     """Windowed attention on image-ordered tokens (partition + attention + unpartition).
     q, k, v: (B, nH, H*W, hd) views with contiguous hd; pad_k / pad_v: (nH, hd) rows standing
-    for the zero-padded tokens.  Returns (B, H*W, nH, hd) contiguous."""
+    for the zero-padded tokens.  `soon`: tensors that the launches
+    behind this one read (_soon).  Returns (B, H*W, nH, hd) contiguous."""
     H, W = grid_hw
     _check_qkv(q, k, v, None, H * W)
     _require_gpu(q, k, v, rel_pos_h, rel_pos_w, pad_k, pad_v)
@@ -172,12 +186,12 @@ def attn_relpos_windowed(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     nt = window * window
     code = _timed(
         "attn_window", 4.0 * nwin * nH * nt * nt * hd, "flop",
-        lambda: lib.samfast_attn_relpos_windowed_fwd(
+        lambda: lib.samfast_attn_relpos_windowed_soon_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), rel_pos_h.data_ptr(),
             rel_pos_w.data_ptr(), pad_k.data_ptr(), pad_v.data_ptr(), out.data_ptr(),
             B, nH, H, W, window, hd,
             *_bnhd_strides(q), *_bnhd_strides(k), *_bnhd_strides(v), *_bnhd_strides(o),
-            _dtype_code(q), float(scale), _stream()),
+            _dtype_code(q), float(scale), *_soon(soon, q.device), _stream()),
         nbytes=4.0 * nwin * nH * nt * hd * q.element_size())
     _lib.check(code, "attn_relpos_windowed_fwd")
     return out

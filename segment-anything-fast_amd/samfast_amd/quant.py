@@ -18,7 +18,7 @@ CPU route.
 """
 
 import os
-from typing import Callable, Optional
+from typing import Callable, Optional, Tuple
 
 import torch
 import torch.nn as nn
@@ -141,6 +141,10 @@ class Int8LinearBase(nn.Module):
                      layout=LAYOUT_ROWMAJOR):
         raise NotImplementedError
 
+    def weight_operands(self, layout: int) -> Tuple[torch.Tensor, ...]:
+        """The weight's tensors as linear_fused's kernel will read them beside rows in `layout`, as far as they are there already."""
+        return ()
+
     def linear_fused_quant(self, xq, sx, epilogue, residual=None, out=None, layout=LAYOUT_ROWMAJOR,
                            ln=None, out_layout=LAYOUT_ROWMAJOR):
         """linear_fused followed by the next Linear's row quantiser (behind a LayerNorm when
@@ -186,6 +190,12 @@ class Int8DynamicLinear(Int8LinearBase):
         the layout xq comes in.  The K-block major copy of the weight is made on first use."""
         return ops.gemm_i8_fused(xq, sx, self._weight_for(layout), self.sw, self.bias_f32, epilogue,
                                  residual=residual, dst_row=dst_row, out=out, layout=layout)
+
+    def weight_operands(self, layout: int) -> Tuple[torch.Tensor, ...]:
+        if layout != LAYOUT_KB64:
+            return (self._buffers["wq"],)
+        kept = self.__dict__.get("_kb64")
+        return () if kept is None else (kept[3],)
 
     def _weight_for(self, layout: int) -> torch.Tensor:
         wq = self._buffers["wq"]

@@ -89,6 +89,9 @@ class Int8Sparse24Linear(Int8LinearBase):
             out.scatter_(2, col, vals[..., e].permute(1, 0, 2, 3).reshape(N, KB, 16))
         return out.reshape(N, KB * 64)
 
+    def weight_operands(self, layout):
+        return self.wc, self.widx
+
     def linear_fused(self, xq, sx, epilogue, residual=None, dst_row=None, out=None,
                      layout=_lib.LAYOUT_ROWMAJOR):
         if dst_row is not None:

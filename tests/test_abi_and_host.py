@@ -135,6 +135,30 @@ def test_empty_calls_are_no_ops_without_gpu():
                                        *strides, 0, 0.125, None) == -1
 
 
+def test_lists_of_buffers_read_soon():
+    """The C entry takes up to eight buffers and refuses others before any launch; an encoder asks for what a window kernel can bring
+    in time, and for nothing where the cache holds its weights, for many tokens and outside an encoder."""
+    from samfast_amd import _lib
+    from samfast_amd.modeling.image_encoder import read_soon
+    lib = _lib.load()
+
+    def call(pointers, sizes, n):
+        ptrs = None if pointers is None else (ctypes.c_void_p * len(pointers))(*pointers)
+        return lib.samfast_attn_relpos_windowed_soon_fwd(
+            *([None] * 8), 0, 12, 64, 64, 14, 80, *([64] * 12), 0, 0.125, ptrs, None if sizes is None else (ctypes.c_int64 * len(sizes))(*sizes), n, None)
+
+    buf = ctypes.create_string_buffer(64)
+    p = ctypes.addressof(buf)
+    assert call([p] * 8, [64] * 8, 8) == call([None], [0], 1) == -1 and b"padding rows" in lib.samfast_last_error()  # (further on)
+    for bad in (([p] * 9, [1] * 9, 9), ([p], [-1], 1), ([None], [4], 1), (None, [4], 1), ([p], None, 1), ([p], [4], -1)):
+        assert call(*bad) == -1 and b"read soon" in lib.samfast_last_error(), bad
+    weights = lambda C, size: [torch.empty((n, C * size), dtype=torch.int8, device="meta") for n in (C, 4 * C, 3 * C)]
+    asked = lambda depth, tokens, C, size: len(read_soon(depth, tokens, weights(C, size)))
+    assert asked(24, 4096, 1024, 1) == 3 and asked(32, 4096, 1280, 1) == 2 and asked(32, 4096, 1280, 2) == 1
+    assert asked(12, 4096, 768, 1) == asked(24, 8193, 1024, 1) == asked(0, 4096, 1024, 1) == 0 and asked(24, 8192, 1024, 1) == 3
+    assert len(read_soon(24, 4096, [])) == 0
+
+
 def test_empty_calls_of_block_neck_and_image_are_no_ops_without_gpu():
     """The same for the half-type Linear, the int8 block's middle, the neck's convolutions and the image's preparation."""
     from samfast_amd import _lib

@@ -295,6 +295,29 @@ def test_image_windows_cut_into_parts_keep_their_bits(few, many, nH, H, W, hd):
     assert torch.isfinite(a.float()).all() and torch.equal(a, b[:few])
 
 
+@pytest.mark.parametrize("B,nH,H,W,ws,hd,sizes", [
+    (1, 2, 64, 64, 14, 80, (1, 0, 3, 5)),                   # no word, one word
+    (1, 12, 64, 64, 14, 64, (64 * 64, 64 * 64 + 4, 63)),    # whole chunks, a line more, a part of a line
+    (2, 3, 20, 17, 14, 64, (3 << 20, 100001)),              # many chunks of each workgroup
+    (1, 16, 64, 64, 14, 80, (4099,) * 8),                   # the longest list
+    (1, 2, 16, 13, 13, 64, (1 << 16,))])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_windows_that_read_ahead_keep_their_bits(B, nH, H, W, ws, hd, sizes, dtype):
+    """Buffers read for the launches behind: of any size and alignment, results are those without."""
+    from samfast_amd import ops
+    print(f"case soon B={B} nH={nH} H={H} W={W} ws={ws} hd={hd} {sizes}", flush=True)
+    g = torch.Generator().manual_seed(B + nH + H + ws + hd)
+    qkv = torch.randn((B, H * W, 3, nH, hd), generator=g).to(dtype).cuda()
+    q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
+    tables = [(torch.randn((2 * ws - 1, hd), generator=g) * 0.02).to(dtype).cuda() for _ in range(2)]
+    pads = [torch.randn((nH, hd), generator=g).to(dtype).cuda() for _ in range(2)]
+    soon = [torch.randint(-128, 128, (n + 1,), dtype=torch.int8, generator=g).cuda()[i % 2:n + i % 2] for i, n in enumerate(sizes)]
+    kept = [t.clone() for t in soon]
+    args = (q, k, v, *tables, *pads, (H, W), ws, hd ** -0.5)
+    assert torch.equal(ops.attn_relpos_windowed(*args, soon=soon), ops.attn_relpos_windowed(*args))
+    assert all(torch.equal(a, b) for a, b in zip(soon, kept))
+
+
 @pytest.mark.parametrize("batch", [1, 8])
 @pytest.mark.parametrize("head,hidden_dim", [(16, 80), (12, 64)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
