@@ -6,14 +6,15 @@
 // matrix instructions of the next half row's scores and of the previous one's P V, and the LDS reads that feed
 // them.  No running maximum is taken in the common case, LDS reads meet no bank twice (GridRow), and the
 // workgroups of a head touch its K and V ahead, so that the rows come out of their XCD's L2.
-//   Bound: at 8 x 16 x 4096 x 80 (fp16 785 us, 875 TFLOP/s, bf16 711; attn_global_kernel 803 and 763) the power limit:
-//   the same loop with its MFMAs alone, on the same values, took 666 us - 429 on zeros (probes that are not kept).  At one image of
+//   Bound: at 8 x 16 x 4096 x 80 (fp16 738 us, 931 TFLOP/s, bf16 691; attn_global_kernel 803 and 763) the power limit:
+//   the 32 x 32 loop with its MFMAs alone, on the same values, took 666 us - 429 on zeros (probes that are not kept).  At one image of
 //   12 heads (63.8 us against 82) the last, half-empty round and the prologue.
 //   (The encoder, which hands over tables, keeps attn_global_kernel: its int8 Linears turn any other order of these
 //   roundings into other codes.)
 //
-// Three kernels.  attn_global_bias_kernel: a wavefront owns 32 queries and walks whole key rows; workgroups of 8 (one
-// per CU: every row staged once for 256 queries) or 4 wavefronts (two per CU).  attn_global_split16_kernel (hd 64, on the smaller matrix
+// Four kernels.  attn_global_bias16_kernel (hd 80, on the smaller matrix instruction): a wavefront owns 32 queries and walks whole key rows; workgroups of 8 (one
+// per CU: every row staged once for 256 queries) or 4 wavefronts (two per CU).  attn_global_bias_kernel: the same at hd 64, on the larger
+// instruction, where it is asked for.  attn_global_split16_kernel (hd 64, on the smaller matrix
 // instruction): the keys of every row are split between two wavefronts, whose results (maximum reference, denominator, output) meet in
 // LDS once, at the end; workgroups of two query tiles x two key halves (64 queries, under 54 KB of LDS), three per CU, so that one image's 12 heads are
 // 768 workgroups: three on each of the 256 CUs, where 128-query workgroups leave half of the CUs with one and half with two.  attn_global_split_kernel:
@@ -938,11 +939,312 @@ __global__ __launch_bounds__(64 * Split16Cfg::WAVES, 3) void attn_global_split16
   }
 }
 
+// The unsplit form at hd 80 on 16 x 16 matrix instructions (see attn_global_split16_kernel for the lane's two queries and the order of its keys): 80 channels are two
+// k steps of 32 and one of 16, five channel tiles of V^T without padding, and a sixth tile whose channels are one for every key, from registers, the denominators: 24
+// instructions of 16 cycles a half row, where the 32 x 32 form (attn_global_bias_kernel, whose channels 80 to 95 were ones and zeros of V's rows) had 11 of 32.  What bounds it: the
+// power limit from about 256 workgroups of 256 queries on (it is 6 % behind alone at full clock, with the same waits), below that a wavefront's vector instructions, 64 a half row of which 16
+// are exponentials, and matrix instructions, issued one after another.  They stand one by one in turn: three side by side are 3 to 4 % slower.  A key row neither begins with a read
+// of its rel_h (read a row ahead) nor ends with a wait for the V fragments that are on their way (the barrier alone, behind vmcnt): 4 to 6 %.  The
+// denominators as 16 additions 2 %, as v_dot2 7 % slower.
+// us, 32 x 32 / so (bf16; fp16): 1 x 8 heads 63.1 / 61.7; 63.5 / 60.5, 1 x 12 77.6 / 78.0; 82.1 / 80.7, 1 x 16 91.1 / 86.9; 97.8 / 91.7, 2 x 16 181.7 / 173.0; 194.8 / 182.3, 4 x 12 268
+// / 257; 288 / 271, 8 x 16 720 / 691; 768 / 738, 16 x 16 1431 / 1381; 1533 / 1457, 3 x 13 x 24 rows 40.3 / 38.4; 42.2 / 40.0; up to a wavefront a SIMD it is level to
+// 2.5 % behind (1 x 16 x 4 rows 9.2 / 9.35; 9.05 / 9.2, 1 x 12 x 8 12.2 / 12.4; 12.1 / 12.3, 1 x 8 x 16 19.0 / 19.2; 18.7 / 19.2): twice the matrix instructions to issue (K read a half row
+// ahead where it has landed: 12.6, 19.5).  The error against 64 bits is the same to three digits (2.33e-3, 2.92e-4 of the norm).
+template <int WAVES>
+struct Bias16Cfg {
+  static constexpr int HD = 80, PIECES = HD / 8;        // 16-byte pieces of a row = wave instructions of a tile
+  static constexpr int BM = 32 * WAVES;                 // queries per workgroup
+  static constexpr int DPW = (PIECES + WAVES - 1) / WAVES;
+  static constexpr int PITCH = HD * 2, TILE = 64 * PITCH;
+  // LDS: two K tiles, three V tiles (of a row's V the second half is still to be read when the row two behind is requested), rel_h
+  static constexpr int V_OFF = 2 * TILE;
+  static constexpr int RH = 32;                         // key rows whose rel_h is at hand
+  static constexpr int RELH_OFF = V_OFF + 3 * TILE;
+  static constexpr int LDS_BYTES = RELH_OFF + RH * BM * 4;
+  static_assert(LDS_BYTES <= (WAVES == 4 ? 80 : 160) * 1024, "workgroups per CU");
+  // Rows lie as they come, but for the last two pieces of K, which are read eight bytes at a time and change places in eight rows of sixteen: 160
+  // bytes are ten sixteenths of the banks, so that eight rows of 32 bytes are all of them once, and sixteen rows of
+  // which half are read a piece further on (in the order in which reads of 16 bytes are served, once_swizzle's note).
+  static SF_DEVICE int k_swizzle(int piece, int row) { return piece >= 8 ? (row >> 3) & 1 : 0; }
+};
+
+template <typename T, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias16_kernel(AttnArgs a) {
+  using C = Bias16Cfg<WAVES>;
+  constexpr int HD = 80, CT = HD / 16;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS_BYTES];
+  float* relhT = reinterpret_cast<float*>(lds + C::RELH_OFF);  // [kh % RH][BM], * log2(e); a wavefront reads only its own columns
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lq = lane >> 4;
+
+  const unsigned int nqb = a.N / C::BM;
+  const unsigned int total = (unsigned int)(a.B * a.nH) * nqb;
+  const unsigned int pid = xcd_contiguous_id(blockIdx.x, total);
+  if (pid >= total) return;
+  const int bh = pid / nqb, qb = pid % nqb;
+  const int b = bh / a.nH, h = bh % a.nH;
+  const int q0 = qb * C::BM + 32 * wave;  // the wavefront's first query: half of one grid row
+
+  const unsigned short* kbase = a.k + b * a.k_sb + h * a.k_sh;
+  const unsigned short* vbase = a.v + b * a.v_sb + h * a.v_sh;
+
+  // ---- K / V rows: global memory -> LDS directly, wave instruction i of a tile fills pieces 64 i .. 64 i + 63 ----
+  unsigned int koff[C::DPW], voff[C::DPW];  // bytes, from the tile's first key row; unsigned: scalar-base load form
+#pragma unroll
+  for (int m = 0; m < C::DPW; ++m) {
+    const int P = 64 * (wave + WAVES * m) + lane, row = P / C::PIECES, piece = P % C::PIECES;
+    koff[m] = (unsigned int)(row * (int)a.k_sn) * 2u + (piece ^ C::k_swizzle(piece, row)) * 16;
+    voff[m] = (unsigned int)(row * (int)a.v_sn) * 2u + piece * 16;
+  }
+  const unsigned int lds_base = (unsigned int)(uintptr_t)((__attribute__((address_space(3))) unsigned char*)lds);
+  auto k_dma = [&](int kt, int buf) __attribute__((always_inline)) {
+    const unsigned char* src = reinterpret_cast<const unsigned char*>(kbase + (int64_t)kt * 64 * a.k_sn);
+#pragma unroll
+    for (int m = 0; m < C::DPW; ++m)
+      if (wave + WAVES * m < C::PIECES) lds_dma16(src, koff[m], lds_base + buf * C::TILE + (wave + WAVES * m) * 1024);
+  };
+  auto v_dma = [&](int kt, unsigned int buf_off) __attribute__((always_inline)) {
+    const unsigned char* src = reinterpret_cast<const unsigned char*>(vbase + (int64_t)kt * 64 * a.v_sn);
+#pragma unroll
+    for (int m = 0; m < C::DPW; ++m)
+      if (wave + WAVES * m < C::PIECES) lds_dma16(src, voff[m], lds_base + C::V_OFF + buf_off + (wave + WAVES * m) * 1024);
+  };
+  k_dma(0, 0);
+  v_dma(0, 0);
+  k_dma(1, 1);  // N % 128 == 0: at least two key rows
+  v_dma(1, C::TILE);
+
+  // ---- Q^T operands: queries lr and 16 + lr; channels 32 s + 8 lq .. +7 of two long k steps, 64 + 4 lq .. +3 of a short one ----
+  u32x4 qf[2][2];
+  u32x2 qs[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const unsigned short* qp = a.q + b * a.q_sb + h * a.q_sh + (int64_t)(q0 + 16 * t + lr) * a.q_sn;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) qf[t][s] = load_x8_global(qp + 32 * s + 8 * lq);
+    qs[t] = *reinterpret_cast<const u32x2*>(qp + 64 + 4 * lq);
+  }
+  // Each workgroup touches its own share of the head's K and V first (see above).
+  constexpr int NTOUCH = 2 * C::BM * C::PIECES / (64 * WAVES);
+  unsigned int touched[NTOUCH];
+#pragma unroll
+  for (int i = 0; i < NTOUCH; ++i) {
+    const int P = (tid + 64 * WAVES * i) % (C::BM * C::PIECES), row = P / C::PIECES, col = P % C::PIECES;
+    const bool is_v = 2 * i >= NTOUCH;
+    touched[i] = *reinterpret_cast<const unsigned int*>((is_v ? vbase : kbase) + (int64_t)(qb * C::BM + row) * (is_v ? a.v_sn : a.k_sn) + col * 8);
+  }
+
+  // operand reads: K row lr, its pieces 4 s + lq and, of eight bytes, 8 + lq / 2; V keys 4 lq + lr / 4, channels 16 ct + 4 (lr % 4) .. +3
+  int krd[2], krs;
+#pragma unroll
+  for (int s = 0; s < 2; ++s) krd[s] = lr * C::PITCH + (4 * s + lq) * 16;
+  krs = lr * C::PITCH + ((8 + (lq >> 1)) ^ C::k_swizzle(8, lr)) * 16 + 8 * (lq & 1);
+  const int vrd = C::V_OFF + (4 * lq + (lr >> 2)) * C::PITCH + 8 * (lr & 3);
+
+  // ---- bias: rel_w / sm_scale of the lane's queries is the initial accumulator of the score tiles of the two
+  //      half rows; rel_h * log2(e) stands in LDS, 32 key rows at a time ----
+  auto fill_relh = [&](int kh0) __attribute__((always_inline)) {
+    // lane: query lane % 32, key rows kh0 + 16 (lane / 32) .. +15
+    const int ql = lane & 31, part = 16 * (lane >> 5);
+    const unsigned short* src = a.rh + b * a.rh_sb + h * a.rh_sh + (int64_t)(q0 + ql) * a.rh_sn + kh0 + part;
+    unsigned short v[16];
+    if (a.relh_x8) {
+      *reinterpret_cast<u32x4*>(v) = load_x8_global(src);
+      *reinterpret_cast<u32x4*>(v + 8) = load_x8_global(src + 8);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) v[e] = kh0 + part + e < a.gh ? src[e] : (unsigned short)0;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) relhT[(part + e) * C::BM + 32 * wave + ql] = T::from_bits(v[e]) * kLog2e;
+  };
+  struct Scores { f32x4 v[2][2]; };  // [16 keys][16 queries]
+  Scores b1[2];                      // of the two half rows
+  fill_relh(0);
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const unsigned short* rwp = a.rw + b * a.rw_sb + h * a.rw_sh + (int64_t)(q0 + 16 * t + lr) * a.rw_sn + 4 * lq;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const u32x2 w = *reinterpret_cast<const u32x2*>(rwp + 16 * k);
+      b1[k >> 1].v[k & 1][t] = f32x4{T::lo(w[0]) * a.inv_scale, T::hi(w[0]) * a.inv_scale, T::lo(w[1]) * a.inv_scale, T::hi(w[1]) * a.inv_scale};
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NTOUCH; ++i) asm volatile("" : : "v"(touched[i]));
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of the first two rows has landed
+  __syncthreads();
+
+  // ---- main loop over half rows of 32 keys, pipelined inside a wavefront as attn_global_bias_kernel's ----
+  f32x4 oacc[CT][2];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) oacc[ct][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 lacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};  // denominators: a tile of channels that are one for every key
+  float m_i[2] = {T::kLowest, T::kLowest};
+  constexpr unsigned int ONES = T::kOne | T::kOne << 16;
+  u32x4 ones = {ONES, ONES, ONES, ONES};
+  asm volatile("" : "+v"(ones));
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4* trptr_t;
+  u32x4 kf[2][2], vf[CT], pkA[2], pkB[2];
+  u32x2 ks[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) pkA[t] = pkB[t] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) vf[ct] = u32x4{0u, 0u, 0u, 0u};
+  auto read_k = [&](int off) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) kf[k][s] = *reinterpret_cast<const u32x4*>(lds + krd[s] + off + k * 16 * C::PITCH);
+      ks[k] = *reinterpret_cast<const u32x2*>(lds + krs + off + k * 16 * C::PITCH);
+    }
+  };
+  auto read_v = [&](int ct, unsigned int off) __attribute__((always_inline)) {
+    const unsigned char* p = lds + vrd + off + 32 * ct;
+    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((trptr_t)p));
+    const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((trptr_t)(p + 16 * C::PITCH)));
+    vf[ct] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+  };
+  // instruction n of the twelve of a half row's scores (all four tiles of a k step before the next step) / of the ten of its P V
+  auto score = [&](Scores& s, const Scores& first, int n) __attribute__((always_inline)) {
+    const int step = n >> 2, k = (n >> 1) & 1, t = n & 1;
+    if (step < 2) s.v[k][t] = T::mfma16(kf[k][step & 1], qf[t][step & 1], step == 0 ? first.v[k][t] : s.v[k][t]);
+    else s.v[k][t] = T::mfma16_short(ks[k], qs[t], s.v[k][t]);
+  };
+  auto pv = [&](const u32x4 (&pk)[2], int n) __attribute__((always_inline)) { oacc[n >> 1][n & 1] = T::mfma16(vf[n >> 1], pk[n & 1], oacc[n >> 1][n & 1]); };
+  auto sum = [&](const u32x4 (&pk)[2], int t) __attribute__((always_inline)) { lacc[t] = T::mfma16(ones, pk[t], lacc[t]); };
+  // s, pk: scores and probabilities of this half row, its V at v_off, rel_h of its row b0; s_next: scores of the next one, from K at k_off with
+  // the initial accumulator `first`; pk_prev: the one before, whose V is in registers
+  auto half_row = [&](Scores& s, Scores& s_next, const Scores& first, u32x4 (&pk)[2], u32x4 (&pk_prev)[2], int k_off, unsigned int v_off,
+                      const float (&b0)[2]) __attribute__((always_inline)) {
+    read_k(k_off);
+    __builtin_amdgcn_sched_barrier(0);
+    float neg_mrow[2] = {b0[0] - m_i[0], b0[1] - m_i[1]};
+    unsigned int seen = 0u;
+    float e0, e1;  // a pair is packed one step after its exponentials were issued
+    auto gather = [&](int w) __attribute__((always_inline)) {  // pair w: query w / 4, keys 16 (w / 2 % 2) + 4 lq + 2 (w % 2) and one more
+      pk[w >> 2][w & 3] = T::pack2(e0, e1);
+      if (w & 1) seen = T::note(seen, pk[w >> 2][(w & 3) - 1], pk[w >> 2][w & 3]);
+    };
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      const int t = g >> 2, k = (g >> 1) & 1, r = 2 * (g & 1);
+      const float x0 = fmaf(s.v[k][t][r], a.c, neg_mrow[t]), x1 = fmaf(s.v[k][t][r + 1], a.c, neg_mrow[t]);
+      // three instructions a step, apart: P V of the one before on the first three channel tiles, the scores, P V on the other two and
+      // the denominators
+      auto product = [&](int n) __attribute__((always_inline)) {
+        if (g < 2) pv(pk_prev, 3 * g + n);
+        else if (g < 6) score(s_next, first, 3 * (g - 2) + n);
+        else if (n < 2) pv(pk_prev, 6 + 2 * (g - 6) + n);
+        else sum(pk_prev, g - 6);
+      };
+      if (g > 0) gather(g - 1);
+      __builtin_amdgcn_sched_barrier(0);
+      product(0);
+      __builtin_amdgcn_sched_barrier(0);
+      e0 = fast_exp2(x0);
+      __builtin_amdgcn_sched_barrier(0);
+      product(1);
+      __builtin_amdgcn_sched_barrier(0);
+      e1 = fast_exp2(x1);
+      __builtin_amdgcn_sched_barrier(0);
+      product(2);
+      if (g >= 2 && g < 5) read_v(g - 2, v_off);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    read_v(3, v_off);
+    read_v(4, v_off);
+    gather(7);
+    if (__any(T::outgrown(seen))) {  // move the references, as above
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        float mx = s.v[0][t][0];
+#pragma unroll
+        for (int w = 1; w < 8; ++w) mx = fmaxf(mx, s.v[w >> 2][t][w & 3]);
+        mx = max_with_lane_xor32(fmaxf(mx, __shfl_xor(mx, 16, 64)));
+        const float m_new = fmaxf(m_i[t], fmaf(mx, a.c, b0[t] + T::kMargin));
+        const float alpha = fast_exp2(m_i[t] - m_new);
+        m_i[t] = m_new;
+        lacc[t] *= alpha;
+        neg_mrow[t] = b0[t] - m_new;
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) oacc[ct][t] *= alpha;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const f32x4 v = s.v[w >> 1][t];
+          const float p0 = fast_exp2(fmaf(v[2 * (w & 1)], a.c, neg_mrow[t])), p1 = fast_exp2(fmaf(v[2 * (w & 1) + 1], a.c, neg_mrow[t]));
+          pk[t][w] = T::pack2(p0, p1);
+        }
+      }
+    }
+  };
+
+  const int nkt = a.N / 64;
+  // V tiles rotate: row kt's, and the one row kt + 2 goes to (row kt - 1's)
+  unsigned int v_cur = 0, v_free = 2 * C::TILE;
+  constexpr unsigned int HALF = 32 * C::PITCH;
+  Scores sA, sB;
+  float b_next[2];
+  auto read_relh = [&](int kt) __attribute__((always_inline)) {
+    const float* rh = relhT + (kt % C::RH) * C::BM + 32 * wave + lr;
+    b_next[0] = rh[0];
+    b_next[1] = rh[16];
+  };
+  read_relh(0);
+  read_k(0);
+#pragma unroll
+  for (int n = 0; n < 12; ++n) score(sA, b1[0], n);
+  auto key_row = [&](int kt, auto buf_c) __attribute__((always_inline)) {
+    constexpr int BUF = decltype(buf_c)::value;  // kt & 1, for constant LDS offsets
+    // rel_h of this row is at hand, the next row's is read now (the wavefront's own columns: no barrier)
+    const float b0[2] = {b_next[0], b_next[1]};
+    if (kt + 1 == C::RH && nkt > C::RH) fill_relh(C::RH);
+    read_relh(kt + 1);
+    half_row(sA, sB, b1[1], pkA, pkB, BUF * C::TILE + (int)HALF, v_cur, b0);
+    // row kt + 1 has landed (own share) and everybody has left K row kt and V row kt - 1: refill them.  (LDS reads are done in
+    // order, and the youngest four are the half row's last two V fragments, of row kt: those may be on their way.)
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(4)\n\ts_barrier" ::: "memory");
+    if (kt + 2 < nkt) {
+      k_dma(kt + 2, BUF);
+      v_dma(kt + 2, v_free);
+    }
+    // (after the last row kf is whatever the buffer holds: that product is not used)
+    half_row(sB, sA, b1[0], pkB, pkA, (BUF ^ 1) * C::TILE, v_cur + HALF, b0);
+    v_free = v_cur;
+    v_cur = v_cur == 2 * C::TILE ? 0 : v_cur + C::TILE;
+  };
+  for (int kt = 0; kt < nkt; kt += 2) {  // nkt is even
+    key_row(kt, std::integral_constant<int, 0>{});
+    key_row(kt + 1, std::integral_constant<int, 1>{});
+  }
+#pragma unroll
+  for (int n = 0; n < 2 * CT; ++n) pv(pkB, n);  // of the last half row
+  sum(pkB, 0);
+  sum(pkB, 1);
+
+  unsigned short* op = a.out + b * a.o_sb + h * a.o_sh + (int64_t)(q0 + lr) * a.o_sn + 4 * lq;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const float inv = 1.0f / lacc[t][0];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      const f32x4 o = oacc[ct][t];
+      *reinterpret_cast<u32x2*>(op + (int64_t)(16 * t) * a.o_sn + 16 * ct) = u32x2{T::pack2(o[0] * inv, o[1] * inv), T::pack2(o[2] * inv, o[3] * inv)};
+    }
+  }
+}
+
 // Which form of the global kernel.  Split keys round differently from unsplit ones, so that choice looks at head_dim
 // alone: a slice has the same bits whatever batch it travels in.  hd 64 is split (us in bf16, split / unsplit with 8 / with 4
 // wavefronts, 4096 tokens: 1 x 8 heads 49 / 68 / 50, 1 x 12: 65 / 69 / 76, 2 x 9: 101 / 143 / 118, 1 x 16: 87 / 79 / 83, 4 x 12: 239 / 236 / 236,
 // 8 x 16: 629 / 622 / 617), hd 80, where only two such workgroups fit a CU, is not (55 / 73 / 56, 84 / 76 / 83, 130 / 159 / 136, 106 / 92 / 96, 307 / 272 / 274,
-// 818 / 715 / 718).  8 wavefronts or 4, which agree bit for bit: by how the workgroups of 256
+// 818 / 715 / 718; 8 x 16 691 now, attn_global_bias16_kernel).  8 wavefronts or 4, which agree bit for bit: by how the workgroups of 256
 // queries (one per CU) and of 128 (two) divide among the 256 CUs.  The prices are microseconds of one full round over
 // 64 key rows and, of 128 queries, of a last one with one workgroup per CU.
 // Returns 8, 4, or 2 for the key-split form.
@@ -953,20 +1255,23 @@ static int bias_form(const AttnArgs& a, int hd) {
   const int split = knob_or(KNOB_ATTN_SPLIT, 1);
   if (split == 2 || (split != 0 && hd == 64)) return 2;
   const int64_t slices = (int64_t)a.B * a.nH, wgs4 = slices * (a.N / 128), wgs8 = slices * (a.N / 256), rest4 = wgs4 % 512;
-  const int full4 = hd == 64 ? 80 : 95, one4 = hd == 64 ? 53 : 59, full8 = hd == 64 ? 79 : 91;
+  const int full4 = hd == 64 ? 80 : 88, one4 = hd == 64 ? 53 : 56, full8 = hd == 64 ? 79 : 86;
   const int64_t p4 = wgs4 / 512 * full4 + (rest4 == 0 ? 0 : rest4 <= 256 ? one4 : full4);
   return by8 && (wgs8 + 255) / 256 * full8 <= p4 ? 8 : 4;
 }
 template <typename T, int HD>
 static void launch_bias(const AttnArgs& a, int form, hipStream_t stream) {
   auto grid = [&](int queries) { return dim3((unsigned int)(((int64_t)a.B * a.nH * (a.N / queries) + 7) / 8 * 8)); };
-  if (form == 8) hipLaunchKernelGGL((attn_global_bias_kernel<T, HD, 8>), grid(256), dim3(512), 0, stream, a);
-  else if (form == 4) hipLaunchKernelGGL((attn_global_bias_kernel<T, HD, 4>), grid(128), dim3(256), 0, stream, a);
-  else if constexpr (HD == 64) {
-    if ((int64_t)a.B * a.nH * (a.N / 64) <= 256) hipLaunchKernelGGL((attn_global_split16_kernel<T, true>), grid(64), dim3(256), 0, stream, a);
+  if constexpr (HD == 80) {
+    if (form == 8) hipLaunchKernelGGL((attn_global_bias16_kernel<T, 8>), grid(256), dim3(512), 0, stream, a);
+    else if (form == 4) hipLaunchKernelGGL((attn_global_bias16_kernel<T, 4>), grid(128), dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((attn_global_split_kernel<T>), grid(64), dim3(256), 0, stream, a);
+  } else {
+    if (form == 8) hipLaunchKernelGGL((attn_global_bias_kernel<T, HD, 8>), grid(256), dim3(512), 0, stream, a);
+    else if (form == 4) hipLaunchKernelGGL((attn_global_bias_kernel<T, HD, 4>), grid(128), dim3(256), 0, stream, a);
+    else if ((int64_t)a.B * a.nH * (a.N / 64) <= 256) hipLaunchKernelGGL((attn_global_split16_kernel<T, true>), grid(64), dim3(256), 0, stream, a);
     else hipLaunchKernelGGL((attn_global_split16_kernel<T, false>), grid(64), dim3(256), 0, stream, a);
   }
-  else hipLaunchKernelGGL((attn_global_split_kernel<T>), grid(64), dim3(256), 0, stream, a);
 }
 
 int attn_global_bias_launch(const AttnArgs& a0, int hd, int dtype, hipStream_t stream) {

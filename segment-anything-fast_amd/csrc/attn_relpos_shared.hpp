@@ -65,6 +65,11 @@ struct ElemBf16 {
   static SF_DEVICE f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
   }
+  // sixteen of k: four values a lane
+  static SF_DEVICE f32x4 mfma16_short(u32x2 a, u32x2 b, f32x4 c) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
+  }
   static SF_DEVICE unsigned int pack2(float lo, float hi) { return pack_bf16x2(lo, hi); }
   static SF_DEVICE float lo(unsigned int w) { return bf16_lo_to_f32(w); }
   static SF_DEVICE float hi(unsigned int w) { return bf16_hi_to_f32(w); }
@@ -93,6 +98,10 @@ struct ElemF16 {
   }
   static SF_DEVICE f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+  static SF_DEVICE f32x4 mfma16_short(u32x2 a, u32x2 b, f32x4 c) {
+    typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
   }
   static SF_DEVICE unsigned int pack2(float lo, float hi) {  // round to nearest even
     const f32x2 v = {lo, hi};

@@ -101,6 +101,31 @@ def test_every_other_sixteen_queries_move_their_reference(gh, which, dtype):
     assert ((out - ref).abs() <= 0.51 * eps * (weight + ref.abs()) + 1e-4 * weight + floor + 1e-6).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("which", [0, 1])
+@pytest.mark.parametrize("gh,form", [(2, "four"), (32, "four"), (34, "four"), (36, "eight wavefronts"), (64, "eight wavefronts")])
+def test_unsplit_keys_of_80_channels_near_64_bits(gh, form, which, dtype):
+    """The same where keys are not split, at 80 channels (whose last sixteen are a k step of their own): one query of a lane moves its reference, the
+    other does not, and rel_h is renewed at key row 32.  Larger values in the last channels, so that each of them counts."""
+    from samfast_amd import _lib, ops
+    print(f"case 80 channels gh={gh} {form} which={which} {dtype}", flush=True)
+    q, k, v, rel_h, rel_w = bias_inputs(1, 2, gh, 64, 80, seed=gh + which, dtype=dtype)
+    n = torch.arange(gh * 64)
+    last = 1.0 + (torch.arange(80) >= 64) * 1.0
+    q = (q.float() * last + 0.4 * (n // 16 % 2 == which)[None, None, :, None]).to(dtype)
+    k = (k.float() * last + 3.5 * (n / (gh * 64))[None, None, :, None]).to(dtype)
+    with _lib.knobs(**FORMS[form]):
+        out = ops.attn_relpos_bias(q.cuda(), k.cuda(), v.cuda(), rel_h.squeeze(-1).cuda(), rel_w.squeeze(-2).cuda()).double().cpu()
+    qd, kd, vd = q.double(), k.double(), v.double()
+    bias = (rel_h.double().reshape(1, 2, gh * 64, gh, 1) + rel_w.double().reshape(1, 2, gh * 64, 1, 64)).reshape(1, 2, gh * 64, gh * 64)
+    p = torch.softmax(qd @ kd.transpose(-1, -2) * 80 ** -0.5 + bias, -1)
+    ref, weight = p @ vd, p @ vd.abs()
+    eps = torch.finfo(dtype).eps
+    # as above; the denominator sums rounded probabilities, half an eps more
+    floor = gh * 64 * 2.0 ** -25 * vd.abs().amax() if dtype == torch.float16 else 0.0
+    assert ((out - ref).abs() <= 0.51 * eps * (weight + 2 * ref.abs()) + 1e-4 * weight + floor + 1e-6).all()
+
+
 @pytest.mark.parametrize("hd,dtype", [(64, torch.bfloat16), (64, torch.float16), (80, torch.float16)])
 @pytest.mark.parametrize("gh", [64, 16, 6])  # hd 64: up to 256 workgroups of 64 queries and more, two orders of one kernel's instructions
 def test_a_slice_has_the_same_bits_in_any_batch(hd, dtype, gh):
