@@ -775,9 +775,11 @@ __global__ __launch_bounds__((WindowCfg<HD, TILES>::THREADS), 2) void attn_windo
         if (32 * nt + 32 <= N) acc = score_tile(std::true_type{});  // uniform
         else acc = score_tile(std::false_type{});
 
+        // the seventh tile's upper sixteen keys are never there (N <= 208): no maximum, exponentials or products of theirs
+        const int R = C::NT == 7 && nt == 6 ? 8 : 16;
         float mx = acc[0];
 #pragma unroll
-        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, acc[r]);
+        for (int r = 1; r < R; ++r) mx = fmaxf(mx, acc[r]);
         mx = max_with_lane_xor32(mx);
         // lazy reference (see the global kernel): m_run follows the maximum in steps > 2^kLazyLog2
         const float m_new = fmaxf(m_run, mx);
@@ -790,7 +792,7 @@ __global__ __launch_bounds__((WindowCfg<HD, TILES>::THREADS), 2) void attn_windo
         const float neg_m = -m_run * a.c;
         float lsum = 0.f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
+        for (int r = 0; r < R; ++r) {
           const float p = fast_exp2(fmaf(acc[r], a.c, neg_m));
           acc[r] = p;
           if (!C::ONES_ROW) lsum += p;
@@ -808,7 +810,7 @@ __global__ __launch_bounds__((WindowCfg<HD, TILES>::THREADS), 2) void attn_windo
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
           const int j = 2 * nt + half;
-          if (j < nsteps) {  // uniform
+          if (8 * half < R && j < nsteps) {  // uniform
             const u32x4 pk = cvt_x8<T>(acc, 8 * half);
 #pragma unroll
             for (int dt = 0; dt < C::DT; ++dt) {
