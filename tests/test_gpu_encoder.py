@@ -493,6 +493,30 @@ def test_neck_convolutions_on_rows(B, H, W, C, mid, out, dtype):
         assert ((val.double() - ref).abs() <= bound * 1.0001).all()
 
 
+@pytest.mark.parametrize("B,H,W,C,mid,out", [
+    (1, 5, 7, 64, 64, 64),        # one k tile, nine
+    (1, 3, 70, 192, 192, 128),    # three, 27: the last stands alone between its barriers
+    (2, 20, 20, 448, 128, 64),    # seven; tiles over two images
+    (3, 64, 64, 128, 64, 256)])   # more tiles than CUs
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_neck_convolutions_two_k_tiles_between_barriers(B, H, W, C, mid, out, dtype):
+    test_neck_convolutions_on_rows(B, H, W, C, mid, out, dtype)
+
+
+@pytest.mark.parametrize("cin", [64, 4551, 4552, 5461])
+def test_weights_reordered_beside_a_convolution(cin):
+    """Output channels whose values fit the workgroup's LDS, and ones that are reordered in memory."""
+    from samfast_amd import _lib
+    print(f"case reordered weights {cin}", flush=True)
+    g = torch.Generator().manual_seed(cin)
+    x, w = (torch.randn((64, 64), generator=g).to(torch.bfloat16).cuda() for _ in range(2))
+    src = torch.randn((3, cin, 9), generator=g).to(torch.bfloat16).cuda()
+    y, dst = torch.empty_like(x), torch.empty((3, 9, cin), dtype=src.dtype, device="cuda")
+    _lib.check(_lib.load().samfast_neck_conv(x.data_ptr(), w.data_ptr(), y.data_ptr(), 1, 8, 8, 64, 64, 1, _lib.SAMFAST_BF16, src.data_ptr(), dst.data_ptr(),
+                                             3, cin, torch.cuda.current_stream().cuda_stream), "neck_conv")
+    assert torch.equal(dst, src.transpose(1, 2)) and torch.isfinite(y).all()
+
+
 def test_neck_with_a_hook_or_another_convolution_is_called_as_modules():
     from samfast_amd.modeling import ImageEncoderViT
     torch.manual_seed(1)
