@@ -37,9 +37,9 @@ from .common import LayerNorm2d, MLPBlock
 
 KB64_OPERANDS = os.environ.get("SAMFAST_KB64", "1") != "0"
 WINDOWS_IN_PLACE = os.environ.get("SAMFAST_WINDOWS_IN_PLACE", "1") != "0"
-# The neck on the kernels here up to this many tokens; beyond, the library's larger convolution tiles are ahead (us, library / here,
-# width 1280: one image 107 / 45, four 198 / 102, eight 284 / 187, sixteen 261 / 365)
-NECK_TOKENS = 40960
+# The neck on the kernels here up to this many tokens, the most that was measured (us with its LayerNorms, library / here: width 1280, one image 107 / 38, four 201
+# / 73, ten 202 / 152, sixteen 285 / 232, 32 541 / 499, 64 1057 / 999; width 768, sixteen 249 / 212, 64 925 / 853)
+NECK_TOKENS = 262144
 # Weights that a window attention kernel reads ahead of the products behind it (read_soon): up to this many tokens, this many
 # bytes a block, and from this many bytes over all blocks on
 SOON_TOKENS, SOON_BYTES, SOON_TOTAL = 8192, 9 << 20, 85 << 20
