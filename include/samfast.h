@@ -256,6 +256,12 @@ int samfast_preprocess(
     int dtype, void* stream);
 
 /*
+ * The 16 x 16 patches (modeling/image_encoder.py:375-406) of half-type images x (B, C, H, W), H and W multiples of 16, as rows
+ * y (B * H/16 * W/16, C * 256).
+ */
+int samfast_patch_rows(const void* x, void* y, int64_t B, int C, int H, int W, void* stream);
+
+/*
  * An int8 block's middle in one launch: tokens = proj(quantise(x)) + residual and xq, sx = quantise(norm2(tokens)), with the
  * bits of samfast_quant_rowwise_i8, samfast_gemm_i8_fused (RESIDUAL) and samfast_layernorm_quant_i8
  * (modeling/image_encoder.py:178-181, 251).  x (M, C) with row stride ldx, wq (C/64, C, 64) K-block major, residual and tokens

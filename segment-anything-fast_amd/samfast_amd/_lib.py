@@ -38,6 +38,7 @@ _SIGNATURES = {
     "samfast_proj_block_pays": (_i32, [_i64, _i32]),
     "samfast_proj_block_i8": (_i32, [_ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _f32, _ptr, _ptr, _i64, _i32, _i32, _ptr]),
     "samfast_preprocess": (_i32, [_ptr, _i32, _ptr, _ptr, _ptr, _i64, _i32, _i32, _i32, _i32, _ptr]),
+    "samfast_patch_rows": (_i32, [_ptr, _ptr, _i64, _i32, _i32, _i32, _ptr]),
     "samfast_linear_half_pays": (_i32, [_i64, _i32, _i32, _i32]),
     "samfast_linear_half": (_i32, [_ptr, _i64, _ptr, _ptr, _ptr, _i64, _i64, _i32, _i32, _i32, _i32, _ptr, _i64, _ptr]),
     "samfast_gelu_quant_rowwise_i8": (_i32, [_ptr, _i64, _ptr, _ptr, _i64, _i32, _i32, _i32, _ptr]),

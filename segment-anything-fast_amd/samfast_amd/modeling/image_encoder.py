@@ -569,7 +569,9 @@ class PatchEmbed(nn.Module):
             # output is already (B, H, W, C)
             B, C, H, W = x.shape
             gh, gw = H // kh, W // kw
-            cols = x.reshape(B, C, gh, kh, gw, kw).permute(0, 2, 4, 1, 3, 5).reshape(B * gh * gw, C * kh * kw)
+            cols = ops.patch_rows(x) if FUSED_BLOCK and kh == kw == 16 else None
+            if cols is None:
+                cols = x.reshape(B, C, gh, kh, gw, kw).permute(0, 2, 4, 1, 3, 5).reshape(B * gh * gw, C * kh * kw)
             y = F.linear(cols, p.weight.reshape(p.out_channels, C * kh * kw), p.bias)
             return y.view(B, gh, gw, p.out_channels)
         return self.proj(x).permute(0, 2, 3, 1)

@@ -717,6 +717,20 @@ def preprocess(x: torch.Tensor, mean: torch.Tensor, std: torch.Tensor, size: int
     return out
 
 
+def patch_rows(x: torch.Tensor) -> Optional[torch.Tensor]:
+    """The 16 x 16 patches of half-type images (B, C, H, W) as rows (B * H/16 * W/16, C * 256); None for what the kernel does not read."""
+    if not (x.is_cuda and x.dim() == 4 and x.dtype in (torch.bfloat16, torch.float16) and x.numel() > 0 and max(x.shape[1:]) <= 65536
+            and x.shape[2] % 16 == 0 and x.shape[3] % 16 == 0 and not torch.is_grad_enabled() and unwatched(x) and rows_launchable(x)):
+        return None
+    B, C, H, W = x.shape
+    out = torch.empty((B * (H // 16) * (W // 16), C * 256), dtype=x.dtype, device=x.device)
+    lib = _lib.load()
+    code = _timed("patch_rows", 4.0 * x.numel(), "byte",
+                  lambda: lib.samfast_patch_rows(x.data_ptr(), out.data_ptr(), B, C, H, W, _stream()))
+    _lib.check(code, "patch_rows")
+    return out
+
+
 def gelu_(x: torch.Tensor) -> torch.Tensor:
     """Exact-erf GELU of a contiguous half-type tensor, in place."""
     _require_gpu(x)

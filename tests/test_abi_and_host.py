@@ -175,6 +175,12 @@ def test_empty_calls_of_block_neck_and_image_are_no_ops_without_gpu():
     assert image(0) == 0 and image(-1) == -1 and image(0, 1001) == -1
 
 
+def test_patch_rows_refused_or_empty_without_gpu():
+    from samfast_amd import _lib
+    patches = lambda B, H=1024, W=1024, C=3: _lib.load().samfast_patch_rows(None, None, B, C, H, W, None)
+    assert patches(0) == 0 and patches(-1) == patches(0, 1000) == patches(0, 1024, 8) == patches(0, 1024, 0) == patches(0, C=0) == patches(1) == -1
+
+
 def test_argument_validation_without_gpu():
     """Validation runs on the host before any launch, so error codes are testable here."""
     from samfast_amd import _lib

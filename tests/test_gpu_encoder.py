@@ -517,6 +517,29 @@ def test_weights_reordered_beside_a_convolution(cin):
     assert torch.equal(dst, src.transpose(1, 2)) and torch.isfinite(y).all()
 
 
+@pytest.mark.parametrize("B,C,H,W", [(1, 3, 16, 16), (2, 1, 48, 80), (3, 5, 32, 112), (1, 3, 1024, 1024)])  # a row's last group of patches: 1, 1, 3, 4
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_patches_as_rows(B, C, H, W, dtype):
+    """A copy: the same bits as the permutation, and what the kernel does not read is left to that."""
+    from samfast_amd import ops
+    from samfast_amd.modeling.image_encoder import PatchEmbed
+    print(f"case patches {B} x {C} x {H} x {W} {dtype}", flush=True)
+    torch.manual_seed(C)
+    x = torch.randn((B, C, H, W), dtype=dtype, device="cuda")
+    x.view(torch.int16)[0, 0, 0, :2] = torch.tensor([0x7fff, -128], dtype=torch.int16)  # (NaNs move as they are)
+    expect = x.view(B, C, H // 16, 16, W // 16, 16).permute(0, 2, 4, 1, 3, 5).reshape(-1, C * 256)
+    embed = PatchEmbed(in_chans=C, embed_dim=64).to("cuda", dtype)
+    plain = torch.nn.functional.linear(expect, embed.proj.weight.view(64, -1), embed.proj.bias).view(B, H // 16, W // 16, 64)
+    with torch.no_grad():
+        assert torch.equal(ops.patch_rows(x).view(torch.int16), expect.view(torch.int16))
+        assert torch.equal(embed(x).view(torch.int16), plain.view(torch.int16))
+        for other in (x.transpose(2, 3), x.float(), x[..., :W - 8].contiguous(), x[0], x[:0], x.cpu()):
+            assert ops.patch_rows(other) is None
+        with torch.autocast("cuda", dtype=dtype):
+            assert ops.patch_rows(x) is None
+    assert ops.patch_rows(x) is None  # gradients are on
+
+
 def test_neck_with_a_hook_or_another_convolution_is_called_as_modules():
     from samfast_amd.modeling import ImageEncoderViT
     torch.manual_seed(1)
