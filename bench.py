@@ -542,7 +542,7 @@ def run_config(model, batch, steps, warmup, sparse_mlp=False, bf16_linears=False
                 "what": "sam_model_fast_registry[...]().image_encoder(images): HIP-graph replay behind the registry, "
                         "input copy and output clone included",
                 "value": round(batch / rsec, 3), "unit": "images/s", "ms_per_step": round(rsec * 1e3, 3),
-                "min_cosine_vs_eager": round(cos_r, 6)}  # (bit-equal up to the neck's MIOpen convolutions)
+                "min_cosine_vs_eager": round(cos_r, 6)}  # (bit-equal up to the library's patch product)
             del sam
         out = step()
         finite = bool(torch.isfinite(out.float()).all())
