@@ -742,6 +742,23 @@ def test_gemm_by_turns_of_192_columns_agrees(M, N, K, strided, layout, epi):
     assert out is None or (out[:, N:] == 7).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(4096, 2304, 896), (2437, 3584, 1024), (12973, 696, 1280), (2200, 3904, 5120)])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_one_round_of_192_columns_by_turns_agrees(M, N, K, layout):
+    """What the rule takes there against the 64-row tiles: the same bits, the last rows and columns of ragged outputs too."""
+    from samfast_amd import _lib, ops
+    print(f"case one round {M} x {K} -> {N} layout {layout}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    xk, wk = (torch.randint(-127, 128, (rows, K), generator=g, dtype=torch.int8, device="cuda") for rows in (M, N))
+    sx, sw = (torch.rand(n, generator=g, device="cuda") * 1e-2 for n in (M, N))
+    if layout == _lib.LAYOUT_KB64:
+        xk, wk = ops.to_kb64(xk), ops.to_kb64(wk)
+    assert _lib.load().samfast_bench_gemm_i8_turns(M, N, K, _lib.EPILOGUE_NONE, N) == 192
+    got = ops.gemm_i8_fused(xk, sx, wk, sw, None, _lib.EPILOGUE_NONE, layout=layout)
+    with _lib.knobs(SAMFAST_GEMM_TILE=64, SAMFAST_GEMM_SKINNY=0):
+        assert torch.equal(got, ops.gemm_i8_fused(xk, sx, wk, sw, None, _lib.EPILOGUE_NONE, layout=layout))
+
+
 @pytest.mark.parametrize("M,N,pitch", [(128, 384, 384), (300, 400, 400), (129, 1160, 1168), (4096, 3072, 3072), (4900, 2304, 2304), (9000, 776, 776)])
 @pytest.mark.parametrize("layout", [0, 1])
 def test_gelu_strips_agree(M, N, pitch, layout):
