@@ -47,8 +47,9 @@ static bool pays(int epi, int K, const PPChoice& c, bool lines) {
   //     8192 x 768 -> 3072 25.0 / 22.7, 8192 x 1024 -> 3072 29.6 / 26.6, 2820 x 3584 -> 3840 42.4 / 35.4, 11268 x 3456 -> 2080 96.7 / 65.9, 32355 x 3072 -> 768 72.9 / 60.9
   //   plain, one round of 192 columns, K above 768, 0.68: 0.75 (4096 x 1152 -> 2304) 18.6 / 15.8, (12288 x 1024 -> 768) 17.6 / 15.1, 0.69 (2437 x 1024 -> 3584) 16.3 / 14.6, (2200 x 5120 ->
   //     3904) 53.7 / 40.5, row-major 0.68 (2400 x 2432 -> 3552) 35.8 / 23.0, 85 products drawn between 0.68 and 0.8, K 896 to 5120, 0.62 to 1.005 times as long; but 0.67, where
-  //     512 tiles of 128 x 128 are two per CU, (8192 x 1024 -> 1024) 15.0 / 15.3, 0.66 (4604 x 1152 -> 1792) 14.6 / 15.2.  K of 640 and 768 keep 0.8 (0.94 to 1.0 in most there; 4096 x 768
-  //     -> 2304 14.5 / 12.9 in later measurements than the one above)
+  //     512 tiles of 128 x 128 are two per CU, (8192 x 1024 -> 1024) 15.0 / 15.3, 0.66 (4604 x 1152 -> 1792) 14.6 / 15.2.  From K = 2048 on 0.5: 0.51 (6262 x 4096 -> 1024) 33.9 / 31.9, 0.55 (8270 x 5120 -> 832) 43.6 / 39.8, 0.66 (3313 x
+  //     5120 -> 2488) 54.0 / 40.5, row-major 0.58 (1702 x 4096 -> 4280) 45.6 / 32.8, 32 drawn 0.63 to 0.95 times as long; but 0.55 (4025 x 1280 -> 1728) 15.1 / 15.5.  K of 640 and
+  //     768 keep 0.8 (0.94 to 1.0 in most there; 4096 x 768 -> 2304 14.5 / 12.9 in later measurements than the one above)
   //   residual, K >= 2048, 0.7, within one round of 256 columns 0.55: 0.56 (12288 x 3072 -> 768) 38.6 / 36.6, 0.62 (8192 x 5120 -> 1280) 59.5 / 54.6, 0.75 (12288 x 4096 ->
   //     1024) 54.1 / 49.8, (192 columns) 0.83 (16384 x 5120 -> 1280) 108 / 96, 0.75 (12288 x 3072 ->
   //     768) 36.5 / 32.6, but 0.66 (10771 x 3200 -> 768) 31.7 / 32.4, 1.0 (20480 x 4096 -> 1024, 320 rows) 86.5 / 64.3, (65536 x 5120 -> 1280) 402 / 336, 0.88 (28672 x 5120 -> 1280, 320 rows) 190 /
@@ -58,7 +59,7 @@ static bool pays(int epi, int K, const PPChoice& c, bool lines) {
   //     (32768 x 1280 -> 1280) 63.2 / 66.3; from K = 1280 on 0.77 in up to two rounds: 0.78 (20480 -> 1280) 48.5 / 41.5
   //     Rows that are no whole lines, whose segments each touch two, only within two rounds: 7556 x 1024 -> 1992 31.4 / 28.3, 16384 x 640 -> 1992 47.4 / 44.6; but
   //     four 28672 x 640 -> 1992 72.4 / 78.1, five 14563 x 640 -> 4904 102 / 114, thirteen 40960 x 1024 -> 4904 309 / 321 (28672 x 1280 -> 1992 110 / 101)
-  if (epi != EPI_RESIDUAL_BF16) return c.used >= (c.rounds == 1 && c.tn == 6 && K > 768 ? 0.68 : K >= 1280 ? 0.75 : 0.8);
+  if (epi != EPI_RESIDUAL_BF16) return c.used >= (c.rounds == 1 && c.tn == 6 && K > 768 ? (K >= 2048 ? 0.5 : 0.68) : K >= 1280 ? 0.75 : 0.8);
   if (K >= 2048) return c.used >= (c.rounds == 1 && c.tn != 6 ? 0.55 : 0.7);
   if (K < 1280 && c.rounds > 2 && !lines) return false;
   return c.used >= (K >= 1280 && c.rounds <= 2 ? 0.77 : 0.85);

@@ -857,9 +857,10 @@ def test_the_lines_of_the_products_of_few_rows():
 
 
 def test_the_dense_products_lines_within_one_round_of_192_columns():
-    """From two thirds of the CUs' time on where the loop is longer than 768: (M, N, K, columns)."""
+    """From two thirds of the CUs' time on where the loop is longer than 768, half of it from 2048 on: (M, N, K, columns)."""
     from samfast_amd import _lib
-    for M, N, K, columns in ((4096, 2304, 896, 192), (2437, 3584, 1024, 192), (2200, 3904, 5120, 192), (12973, 696, 1280, 192), (8192, 1024, 1024, 0), (4604, 1792, 1152, 0),
+    for M, N, K, columns in ((4096, 2304, 896, 192), (2437, 3584, 1024, 192), (2200, 3904, 5120, 192), (12973, 696, 1280, 192), (8192, 1024, 1024, 0), (4604, 1792, 1152, 0), (6262, 1024, 4096, 192),
+                             (5618, 1408, 2048, 192), (4025, 1728, 1280, 0), (1401, 3584, 4096, 0),
                              (4096, 2304, 640, 0), (4096, 2304, 960, 0), (16385, 768, 1024, 0)):
         assert _lib.load().samfast_bench_gemm_i8_turns(M, N, K, _lib.EPILOGUE_NONE, N) == columns, (M, N, K)
 

@@ -742,7 +742,7 @@ def test_gemm_by_turns_of_192_columns_agrees(M, N, K, strided, layout, epi):
     assert out is None or (out[:, N:] == 7).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(4096, 2304, 896), (2437, 3584, 1024), (12973, 696, 1280), (2200, 3904, 5120)])
+@pytest.mark.parametrize("M,N,K", [(4096, 2304, 896), (2437, 3584, 1024), (12973, 696, 1280), (2200, 3904, 5120), (6262, 1024, 2048)])
 @pytest.mark.parametrize("layout", [0, 1])
 def test_one_round_of_192_columns_by_turns_agrees(M, N, K, layout):
     """What the rule takes there against the 64-row tiles: the same bits, the last rows and columns of ragged outputs too."""
