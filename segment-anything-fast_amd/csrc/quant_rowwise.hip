@@ -28,6 +28,8 @@ __host__ SF_DEVICE unsigned int quant_blocks(int64_t M, int rpb) { return ((unsi
 // first here, and what is written last here is read first by the next one.  us in the ViT-H encoder, 16 images, row by row / so: rows with LayerNorm 53.2 / 51.9, proj
 // and lin2 behind them 232.8 / 227.4 on average, rows with GELU, whose producer streams past the cache, 176 / 179; the
 // whole 58541 / 58305, 32 images with 2:4 MLPs 109600 / 108660, ViT-L 16 images 35121 / 34917, five 12081 / 11980; single images level.
+// A Linear's own rows, without LayerNorm or GELU, are taken as they come by one wavefront (65536 x 1280 -> 3840 306.6 so, 309.4 from the ends) and by two through the cache (32768 x 2048
+// -> 2048 148 / 151); the other shared rows from the ends (65536 x 4096 -> 1024 378 / 338, 16384 x 5120 -> 1280 126.3 / 121.0, 65536 x 2560 -> 1280 268 / 260, 20480 x 3072 -> 768 72 / 69.8).
 SF_DEVICE unsigned int row_block(unsigned int b, int64_t M, int rpb) {
   const unsigned int eighth = quant_blocks(M, rpb) >> 3;
   return (b & 7u) * eighth + eighth - 1u - (b >> 3);
@@ -52,7 +54,8 @@ __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowwise_bf16_k
   const int lane = threadIdx.x & 63;
   // the wavefront index is uniform: telling the compiler so keeps the row and everything derived from it
   // (row pointers, output offsets) in scalar registers instead of 64-bit arithmetic per lane
-  const int64_t row = (int64_t)row_block(blockIdx.x, a.M, kQuantWavesPerBlock) * kQuantWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned int block = LN || ACT ? row_block(blockIdx.x, a.M, kQuantWavesPerBlock) : blockIdx.x;
+  const int64_t row = (int64_t)block * kQuantWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= a.M) return;  // whole wavefront leaves together
   const int nchunk = EXACT ? 64 * NCH : a.K / EPC;
 
@@ -119,7 +122,8 @@ __global__ __launch_bounds__(64 * kQuantWavesPerBlock) void quant_rowshare_bf16_
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = wave % WPR;
-  const int64_t row = (int64_t)row_block(blockIdx.x, a.M, RPB) * RPB + wave / WPR;
+  const unsigned int block = ACT || NTL || WPR == 4 ? row_block(blockIdx.x, a.M, RPB) : blockIdx.x;
+  const int64_t row = (int64_t)block * RPB + wave / WPR;
   const bool live = row < a.M;  // uniform over the wavefront
   const int nchunk = a.K / EPC;
   // chunk i of the lane: (i * WPR + sub) * 64 + lane, so that the wavefronts of a row read it side by side
