@@ -37,9 +37,10 @@ from .common import LayerNorm2d, MLPBlock
 
 KB64_OPERANDS = os.environ.get("SAMFAST_KB64", "1") != "0"
 WINDOWS_IN_PLACE = os.environ.get("SAMFAST_WINDOWS_IN_PLACE", "1") != "0"
-# The neck on the kernels here up to this many tokens, the most that was measured (us with its LayerNorms, library / here: width 1280, one image 107 / 38, four 201
-# / 73, ten 202 / 152, sixteen 285 / 232, 32 541 / 499, 64 1057 / 999; width 768, sixteen 249 / 212, 64 925 / 853)
-NECK_TOKENS = 262144
+# The neck on the kernels here up to this many tokens.  More are the library's convolutions, so that embeddings of large batches keep their bits: these kernels' differ by 5.4e-3
+# of the norm (against 64 bits, on the tokens of five encoders, library 3.4e-3, here 3.3e-3), for little time (us with its LayerNorms, library / here: width 1280, one image 107
+# / 38, four 201 / 73, ten 202 / 152, but sixteen 285 / 232 of an encoder's 58000, 32 541 / 499 of 109000)
+NECK_TOKENS = 40960
 # Weights that a window attention kernel reads ahead of the products behind it (read_soon): up to this many tokens, this many
 # bytes a block, and from this many bytes over all blocks on
 SOON_TOKENS, SOON_BYTES, SOON_TOTAL = 8192, 9 << 20, 85 << 20

@@ -540,6 +540,20 @@ def test_patches_as_rows(B, C, H, W, dtype):
     assert ops.patch_rows(x) is None  # gradients are on
 
 
+def test_neck_of_more_than_ten_images_is_the_librarys(monkeypatch):
+    """Ten images' convolutions run here, eleven's are the modules': the same bits as always on either side."""
+    from samfast_amd import ops
+    from samfast_amd.modeling import ImageEncoderViT
+    torch.manual_seed(1)
+    enc = ImageEncoderViT(img_size=1024, embed_dim=128, depth=0, num_heads=2).cuda().to(torch.bfloat16).eval()
+    calls, convs = [], ops.neck_convs
+    monkeypatch.setattr(ops, "neck_convs", lambda x, *args: calls.append(len(x)) or convs(x, *args))
+    for images in (10, 11):
+        with torch.no_grad():
+            assert enc(torch.zeros((images, 3, 1024, 1024), dtype=torch.bfloat16, device="cuda")).shape == (images, 256, 64, 64)
+    assert calls == [10]
+
+
 def test_neck_with_a_hook_or_another_convolution_is_called_as_modules():
     from samfast_amd.modeling import ImageEncoderViT
     torch.manual_seed(1)
