@@ -71,17 +71,24 @@ def quantize_weight_per_channel(weight: torch.Tensor, convention: str = "absmax1
     return q.contiguous(), scale.to(torch.float32).contiguous()
 
 
-def kept_copy(holder: nn.Module, name: str, source: torch.Tensor, make: Callable[[], object]):
-    """What make() derives from `source`, a buffer of the module: kept on `holder` and made anew when the
-    buffer is another one, elsewhere or written to (load_state_dict, .to()).  It is complete before
-    it is kept, so that any stream and thread may read it.  Made while a graph is recorded, it exists
-    at the replays only, and writes to inference tensors leave no trace: neither is kept."""
-    counted = not source.is_inference()
+def current_copy(holder: nn.Module, name: str, source: torch.Tensor):
+    """What kept_copy would hand out of `source` as it is now, None where it would make that anew: the buffer is another
+    one, elsewhere or written to since (load_state_dict, .to()), or an inference tensor, to which writes leave no trace."""
     hit = holder.__dict__.get(name)
-    if hit is not None and counted and hit[0] is source and hit[1] == source.data_ptr() and hit[2] == source._version:
-        return hit[3]
+    if hit is None or source.is_inference() or hit[0] is not source or hit[1] != source.data_ptr() or hit[2] != source._version:
+        return None
+    return hit[3]
+
+
+def kept_copy(holder: nn.Module, name: str, source: torch.Tensor, make: Callable[[], object]):
+    """What make() derives from `source`, a buffer of the module: kept on `holder` and made anew when it is no
+    longer current (current_copy).  It is complete before it is kept, so that any stream and thread may read it.  Made
+    while a graph is recorded, it exists at the replays only, and is not kept, nor is one of an inference tensor."""
+    current = current_copy(holder, name, source)
+    if current is not None:
+        return current
     made = make()
-    if not counted or (source.is_cuda and torch.cuda.is_current_stream_capturing()):
+    if source.is_inference() or (source.is_cuda and torch.cuda.is_current_stream_capturing()):
         return made
     if source.is_cuda:
         torch.cuda.current_stream(source.device).synchronize()
@@ -194,8 +201,9 @@ class Int8DynamicLinear(Int8LinearBase):
     def weight_operands(self, layout: int) -> Tuple[torch.Tensor, ...]:
         if layout != LAYOUT_KB64:
             return (self._buffers["wq"],)
-        kept = self.__dict__.get("_kb64")
-        return () if kept is None else (kept[3],)
+        # (the current copy alone: linear_fused reads no other, and a graph that is recorded now must not hold the address of one that the next pass frees)
+        kept = current_copy(self, "_kb64", self._buffers["wq"])
+        return () if kept is None else (kept,)
 
     def _weight_for(self, layout: int) -> torch.Tensor:
         wq = self._buffers["wq"]

@@ -159,6 +159,36 @@ def test_lists_of_buffers_read_soon():
     assert len(read_soon(24, 4096, [])) == 0
 
 
+def test_a_weight_that_is_read_ahead_is_the_one_that_the_product_reads():
+    """A K-block-major copy is named while it is current, and not once its weight was written to, moved or replaced: the next product
+    makes another, and the memory of the old one is given back, whoever still holds its address."""
+    from samfast_amd import _lib, quant
+    from samfast_amd.sparse import Int8Sparse24Linear
+    linear = quant.Int8DynamicLinear.from_float(torch.nn.Linear(128, 64))
+    copy = lambda: quant.kept_copy(linear, "_kb64", linear.wq, lambda: linear.wq.clone())
+    kb, row = _lib.LAYOUT_KB64, _lib.LAYOUT_ROWMAJOR
+    named = lambda: linear.weight_operands(kb)
+    assert named() == () and linear.weight_operands(row)[0] is linear.wq
+    first = copy()
+    assert copy() is first and len(named()) == 1 and named()[0] is first
+    linear.wq.copy_(linear.wq.flip(0))  # (in place, as load_state_dict does)
+    assert named() == () and linear.weight_operands(row)[0] is linear.wq
+    second = copy()
+    assert second is not first and named()[0] is second
+    linear.wq = linear.wq.clone()
+    assert named() == ()
+    third = copy()
+    assert named()[0] is third
+    linear.wq.data = linear.wq.data.clone()  # (elsewhere: the module's .to())
+    assert named() == ()
+    with torch.inference_mode():
+        linear.wq = linear.wq.clone()
+    copy()
+    assert named() == ()  # (writes to it leave no trace: none is kept)
+    packed = Int8Sparse24Linear(128, 64, torch.zeros((2, 64, 32), dtype=torch.int8), torch.zeros((2, 64, 2), dtype=torch.int32), torch.ones(64), None)
+    assert [t is b for t, b in zip(packed.weight_operands(kb), (packed.wc, packed.widx))] == [True, True]
+
+
 def test_empty_calls_of_block_neck_and_image_are_no_ops_without_gpu():
     """The same for the half-type Linear, the int8 block's middle, the neck's convolutions and the image's preparation."""
     from samfast_amd import _lib
