@@ -1214,7 +1214,8 @@ __global__ __launch_bounds__(256) void kblock_major_kernel(const int8_t* w, int8
 // 16384 x 1280 -> 3840: 105 / 102 / 98, 16384 x 5120 -> 1280: 136 / 137 / 133, 65536 x 1280 -> 3840: 380 / 352 / 348,
 // 65536 x 5120 -> 1280: 657 / 575 / 571.  (Row-major codes as well: 35, 65, 120, 140, 408, 640.)
 // The products by turns (gemm_pingpong.hpp) read 128 bytes of a row at a time: nothing to reorder there (the Linear 65536 x
-// 1280 -> 3840: 335 as they are, 339 reordered).
+// 1280 -> 3840: 335 as they are, 339 reordered; in tiles of 192 columns 57 Linears drawn 0.92 to 1.0 times as long as they are: 16404 x 1280 -> 1280 47.1 reordered,
+// 43.5 as they are, 28042 x 768 -> 768 38.6 / 36.0, 20000 x 2048 -> 400 48.2 / 45.8).
 static bool linear_reorders_weights(int64_t M, int N, int K) { return M >= 16384 && !gemm_i8_pingpong_reads_rows(M, N, K); }
 
 // bytes of the codes in a Linear's workspace; their row scales follow, then reordered weights

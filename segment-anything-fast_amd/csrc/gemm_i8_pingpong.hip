@@ -28,10 +28,11 @@ static PPArgs pp_args(const GemmArgs& g) {
 // SAMFAST_GEMM_PINGPONG = 1 chooses among all tiles, 6 takes 192 columns wherever they fit, other numbers the wider ones.  With the residual short loops have nothing from 192 columns
 // (12288 x 768 -> 768 15.5 / 15.9, 28672 x 768 -> 768 28.6 / 28.8), and below 4096 values two rounds of them are ahead alone (28672 x 3072 -> 768 72.1 / 65.2) but not in an
 // encoder (seven images of ViT-B 7.08 / 7.11 ms; one round, three images 3.40 / 3.38; K = 5120, four of ViT-H 16.99 / 16.66).
+constexpr double kNarrowPlain = 8.7;
 static PPChoice choose(int epi, int64_t M, int N, int K) {
   const int mode = knob_or(KNOB_GEMM_PINGPONG, 1);
   const bool residual = K >= 4096 || (K >= 2048 && (M + 255) / 256 * ((N + 191) / 192) <= 256);
-  return pp_choose(M, N, K / 128, epi == EPI_RESIDUAL_BF16, mode == 6 ? 0.1 : mode != 1 ? 0.0 : epi != EPI_RESIDUAL_BF16 ? 8.7 : residual ? 9.0 : 0.0);
+  return pp_choose(M, N, K / 128, epi == EPI_RESIDUAL_BF16, mode == 6 ? 0.1 : mode != 1 ? 0.0 : epi != EPI_RESIDUAL_BF16 ? kNarrowPlain : residual ? 9.0 : 0.0);
 }
 
 static bool whole_lines(const void* p, int64_t ld) { return reinterpret_cast<uintptr_t>(p) % 128 == 0 && ld % 64 == 0; }
@@ -67,7 +68,7 @@ static bool pays(int epi, int K, const PPChoice& c, bool lines) {
 
 bool gemm_i8_pingpong_reads_rows(int64_t M, int N, int K) {
   if (K % 128 != 0 || K < 640) return false;  // (no knob: a workspace sized by this answer must fit the call that follows)
-  const PPChoice c = pp_choose(M, N, K / 128, false);
+  const PPChoice c = pp_choose(M, N, K / 128, false, kNarrowPlain);  // choose's without a knob
   return c.tn != 0 && pays(EPI_SCALE_BIAS_BF16, K, c, true);
 }
 

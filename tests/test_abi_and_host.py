@@ -886,6 +886,22 @@ def test_the_lines_of_the_products_of_few_rows():
     assert tile(0, 1600, 2240, kb, row) == -1
 
 
+def test_a_linear_reorders_no_weights_for_products_by_turns():
+    """From 16384 rows on, the workspace holds reordered weights for the products that read them, and none for those by turns, whose tiles of 192
+    columns are among them."""
+    from samfast_amd import _lib
+    lib, seen = _lib.load(), set()
+    for M in (16384, 16404, 20000, 28042, 40000, 65536):
+        for K in (576, 640, 768, 1280, 2048, 5120):
+            for N in (128, 400, 496, 768, 1280, 2304, 3840):
+                turns = lib.samfast_bench_gemm_i8_turns(M, N, K, _lib.EPILOGUE_NONE, N)
+                spare = lib.samfast_linear_i8_workspace(M, N, K, 0) - M * K - 4 * M
+                assert spare < 32 if turns else N * K <= spare < N * K + 32, (M, N, K, turns)
+                seen.add(turns)
+    assert seen == {0, 192, 256, 320}
+    assert lib.samfast_linear_i8_workspace(16383, 400, 2048, 0) < 16383 * 2052 + 32
+
+
 def test_the_dense_products_lines_within_one_round_of_192_columns():
     """From two thirds of the CUs' time on where the loop is longer than 768, half of it from 2048 on: (M, N, K, columns)."""
     from samfast_amd import _lib
