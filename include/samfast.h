@@ -257,8 +257,9 @@ int samfast_preprocess(
 
 /*
  * The 16 x 16 patches (modeling/image_encoder.py:375-406) of half-type images x (B, C, H, W), H and W multiples of 16, as rows
- * y (B * H/16 * W/16, C * 256).
+ * y (B * H/16 * W/16, C * 256).  At most SAMFAST_PATCH_ROWS_MAX groups of four patches of one channel, B * C * H/16 * ceil(W/64).
  */
+#define SAMFAST_PATCH_ROWS_MAX ((1 << 26) - 4)
 int samfast_patch_rows(const void* x, void* y, int64_t B, int C, int H, int W, void* stream);
 
 /*

@@ -82,10 +82,11 @@ extern "C" int samfast_patch_rows(const void* x, void* y, int64_t B, int C, int 
   SF_REQUIRE(B >= 0 && C > 0 && C <= (1 << 16) && H > 0 && W > 0 && H % 16 == 0 && W % 16 == 0 && H <= (1 << 16) && W <= (1 << 16),
              "patch_rows: bad shape B=%lld C=%d %dx%d", (long long)B, C, H, W);
   if (B == 0) return SAMFAST_OK;
+  // a launch has fewer than 2^32 threads
+  const int64_t per_image = (int64_t)C * (H / 16) * ((W / 16 + 3) / 4);
+  SF_REQUIRE(B <= SAMFAST_PATCH_ROWS_MAX / per_image, "patch_rows: too large");
   SF_REQUIRE(x && y && aligned16(x) && aligned16(y), "patch_rows: null or unaligned pointer");
   PatchArgs a = {reinterpret_cast<const u32x4*>(x), reinterpret_cast<u32x4*>(y), 0, C, H / 16, W / 16, (W / 16 + 3) / 4};
-  const int64_t per_image = (int64_t)C * a.gh * a.groups;
-  SF_REQUIRE(B <= (int64_t)0x7fffffff / per_image, "patch_rows: too large");
   a.waves = (unsigned int)(B * per_image);
   hipLaunchKernelGGL(patch_rows_kernel, dim3((a.waves + 3u) / 4u), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), a);
   return check_launch("patch_rows_kernel");

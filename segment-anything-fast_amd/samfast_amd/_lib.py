@@ -82,6 +82,7 @@ _BENCH_SIGNATURES = {
 }
 
 MAX_SOON = 8
+PATCH_ROWS_MAX = (1 << 26) - 4
 
 EPILOGUE_NONE, EPILOGUE_GELU, EPILOGUE_RESIDUAL = 0, 1, 2
 LAYOUT_ROWMAJOR, LAYOUT_KB64 = 0, 1

@@ -723,6 +723,8 @@ def patch_rows(x: torch.Tensor) -> Optional[torch.Tensor]:
             and x.shape[2] % 16 == 0 and x.shape[3] % 16 == 0 and not torch.is_grad_enabled() and unwatched(x) and rows_launchable(x)):
         return None
     B, C, H, W = x.shape
+    if B * C * (H // 16) * -(-W // 64) > _lib.PATCH_ROWS_MAX:
+        return None
     out = torch.empty((B * (H // 16) * (W // 16), C * 256), dtype=x.dtype, device=x.device)
     lib = _lib.load()
     code = _timed("patch_rows", 4.0 * x.numel(), "byte",

@@ -211,6 +211,26 @@ def test_patch_rows_refused_or_empty_without_gpu():
     assert patches(0) == 0 and patches(-1) == patches(0, 1000) == patches(0, 1024, 8) == patches(0, 1024, 0) == patches(0, C=0) == patches(1) == -1
 
 
+@pytest.mark.parametrize("C,H,W,images", [(3, 1024, 1024, 21845), (1, 16, 16, (1 << 26) - 4), (3, 65536, 16, 5461), (2, 16, 80, 1 << 24)])
+def test_patches_beyond_one_launch_are_left_to_the_permutation(monkeypatch, C, H, W, images):
+    """The C entry refuses what a launch of under 2^32 threads does not cover, before it looks at a pointer, and the operator declines it."""
+    from samfast_amd import _lib, ops
+    most = _lib.PATCH_ROWS_MAX // (C * (H // 16) * ((W + 63) // 64))
+    assert abs(images - most) <= 1
+    for B, large in ((most, False), (most + 1, True)):
+        assert _lib.load().samfast_patch_rows(None, None, B, C, H, W, None) == -1
+        assert (b"too large" in _lib.load().samfast_last_error()) == large
+    monkeypatch.setattr(ops, "unwatched", lambda x: True)
+    monkeypatch.setattr(ops, "rows_launchable", lambda *tensors: True)
+    monkeypatch.setattr(torch, "empty", lambda *args, **kwargs: pytest.fail("not declined"))
+    x = SimpleNamespace(is_cuda=True, dim=lambda: 4, dtype=torch.bfloat16, numel=lambda: 1, shape=(most + 1, C, H, W), device=None)
+    with torch.no_grad():
+        assert ops.patch_rows(x) is None
+        x.shape = (most, C, H, W)
+        with pytest.raises(pytest.fail.Exception, match="not declined"):
+            ops.patch_rows(x)
+
+
 def test_argument_validation_without_gpu():
     """Validation runs on the host before any launch, so error codes are testable here."""
     from samfast_amd import _lib
