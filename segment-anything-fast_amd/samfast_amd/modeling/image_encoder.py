@@ -64,6 +64,10 @@ def read_soon(depth: int, tokens: int, weights: Sequence[torch.Tensor]) -> Seque
     return [w for i, w in enumerate(weights) if sum(sizes[:i + 1]) <= SOON_BYTES]
 
 
+def _recording(x: torch.Tensor) -> bool:
+    return x.is_cuda and torch.cuda.is_current_stream_capturing()
+
+
 class ImageEncoderViT(nn.Module):
     def __init__(
         self,
@@ -133,6 +137,9 @@ class ImageEncoderViT(nn.Module):
         if x.shape[0] > per_pass:
             return torch.cat([self.forward_blocks(x[i:i + per_pass]) for i in range(0, x.shape[0], per_pass)])
         carry = None
+        # Weights are read ahead (read_soon) in recordings.  Launches that the host issues one by one wait for it more than for the weights, and a list takes
+        # it 10 us a block (us a pass, none / so: ViT-L int8 4411 / 4618, ViT-H int8 6570 / 6864, ViT-B bf16 2493 / 2570; two of ViT-L int8 5418 / 5341).
+        depth = len(self.blocks) if x.shape[0] * x.shape[1] * x.shape[2] <= SOON_TOKENS and _recording(x) else 0
         for i, blk in enumerate(self.blocks):
             if not blk._int8_fused_ok(x):
                 if not blk._half_fused_ok(x):
@@ -140,13 +147,13 @@ class ImageEncoderViT(nn.Module):
                     continue
                 nxt = self.blocks[i + 1] if i + 1 < len(self.blocks) else None
                 chained = nxt is not None and not nxt._int8_fused_ok(x) and nxt._half_fused_ok(x)
-                x, carry = blk._forward_half_fused(x, carry, nxt.norm1 if chained else None, nxt.attn.qkv if chained else None, len(self.blocks))
+                x, carry = blk._forward_half_fused(x, carry, nxt.norm1 if chained else None, nxt.attn.qkv if chained else None, depth)
                 continue
             nxt = self.blocks[i + 1] if i + 1 < len(self.blocks) else None
             next_norm = next_qkv = None
             if nxt is not None and nxt._int8_fused_ok(x) and nxt._chains_from_previous():
                 next_norm, next_qkv = (nxt.norm1.weight, nxt.norm1.bias, nxt.norm1.eps), nxt.attn.qkv
-            x, carry = blk._forward_int8_fused(x, carry, next_norm, next_qkv, len(self.blocks))
+            x, carry = blk._forward_int8_fused(x, carry, next_norm, next_qkv, depth)
         return x
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
@@ -263,7 +270,7 @@ class Block(nn.Module):
         `carry` = (xq, sx): this block's norm1 output, already quantised by the previous block's
         lin2 launch.  `next_norm` = (gamma, beta, eps) of the next block's norm1: lin2 then
         also returns that block's carry; `next_qkv`: that block's first Linear; `depth`: of how many
-        blocks this is one (0: of none).  Returns (tokens (B, H, W, C), carry for the next block)."""
+        blocks this is one whose weights may be read ahead (0: of none).  Returns (tokens (B, H, W, C), carry for the next block)."""
         from .. import quant
         B, H, W, C = x.shape
         attn, mlp = self.attn, self.mlp
@@ -300,7 +307,7 @@ class Block(nn.Module):
                 # the attention kernel cuts the windows itself; the reference's zero-padded tokens
                 # enter as keys / values with the rows a zero input gives the qkv Linear: its bias
                 pad_k, pad_v = self._pad_rows(nH, hd, x.device)
-                soon = read_soon(depth, B * H * W, [t for m in (attn.proj, mlp.lin2, next_qkv) if m is not None for t in m.weight_operands(L)])
+                soon = () if depth == 0 else read_soon(depth, B * H * W, [t for m in (attn.proj, mlp.lin2, next_qkv) if m is not None for t in m.weight_operands(L)])
                 o = ops.attn_relpos_windowed(q, k, v, attn.rel_pos_h, attn.rel_pos_w, pad_k, pad_v,
                                              (H, W), ws, attn.scale, soon).view(B * H * W, C)
             else:
@@ -391,7 +398,7 @@ class Block(nn.Module):
             # a zero-padded token's k and v rows: the qkv bias
             pads = (torch.zeros((2, nH, hd), dtype=x.dtype, device=x.device) if attn.qkv.bias is None
                     else attn.qkv.bias[C:].view(2, nH, hd))
-            soon = read_soon(depth, B * H * W, [m.weight for m in (attn.proj, mlp.lin2, next_qkv) if m is not None])
+            soon = () if depth == 0 else read_soon(depth, B * H * W, [m.weight for m in (attn.proj, mlp.lin2, next_qkv) if m is not None])
             o = ops.attn_relpos_windowed(q, k, v, attn.rel_pos_h, attn.rel_pos_w, pads[0], pads[1], (H, W), ws, attn.scale, soon)
         else:
             o = ops.attn_relpos(q, k, v, attn.rel_pos_h, attn.rel_pos_w, (H, W), attn.scale).permute(0, 2, 1, 3)

@@ -159,6 +159,48 @@ def test_lists_of_buffers_read_soon():
     assert len(read_soon(24, 4096, [])) == 0
 
 
+@pytest.mark.parametrize("kind", ["int8", "half"])
+def test_weights_are_looked_up_to_be_read_ahead_in_recordings_of_few_tokens(monkeypatch, kind):
+    """Nothing is asked of a Linear, and no list is made, where the host issues the launches or the tokens are many: a block is told it is one of none."""
+    from samfast_amd import ops
+    from samfast_amd.modeling import ImageEncoderViT, image_encoder
+    enc = ImageEncoderViT(img_size=64, embed_dim=64, depth=3, num_heads=1, use_rel_pos=True, window_size=2).to(torch.bfloat16)
+    told, lists = [], []
+    monkeypatch.setattr(image_encoder.Block, "_int8_fused_ok", lambda self, x: kind == "int8")
+    monkeypatch.setattr(image_encoder.Block, "_half_fused_ok", lambda self, x: True)
+    name = f"_forward_{kind}_fused"
+    monkeypatch.setattr(image_encoder.Block, name, lambda self, x, carry=None, norm=None, qkv=None, depth=0: (told.append(depth), (x, None))[1])
+    x = torch.zeros((2, 4, 4, 64), dtype=torch.bfloat16)
+    for recorded, most, want in ((False, 32, 0), (True, 32, 3), (True, 31, 0)):
+        monkeypatch.setattr(image_encoder, "_recording", lambda x: recorded, raising=False)
+        monkeypatch.setattr(image_encoder, "SOON_TOKENS", most)
+        enc.forward_blocks(x)
+        assert told == [want] * 3, (recorded, most)
+        told.clear()
+    monkeypatch.undo()
+    # a block of none, as far as its attention
+    class Reached(Exception):
+        pass
+
+    def attention(*args):
+        raise Reached(args[-1])
+
+    monkeypatch.setattr(image_encoder, "read_soon", lambda *args: lists.append(args) or ())
+    monkeypatch.setattr(ops, "layernorm", lambda x, *args, **kwargs: x)
+    monkeypatch.setattr(ops, "layernorm_quant", lambda x, *args, **kwargs: (x, None))
+    monkeypatch.setattr(ops, "linear_half", lambda x, linear, *args, **kwargs: linear(x))
+    monkeypatch.setattr(ops, "attn_relpos_windowed", attention)
+    block = enc.blocks[0]
+    if kind == "int8":
+        block.attn.qkv.linear_fused = lambda x, *args, **kwargs: block.attn.qkv(x)
+        block._pad_rows = lambda *args: (None, None)
+        block.attn.proj.weight_operands = block.mlp.lin2.weight_operands = lambda layout: lists.append(layout) or ()
+    for depth in (0, 3):
+        with torch.no_grad(), pytest.raises(Reached) as reached:
+            getattr(block, name)(x, depth=depth)
+        assert reached.value.args == ((),) and bool(lists) == (depth > 0)
+
+
 def test_a_weight_that_is_read_ahead_is_the_one_that_the_product_reads():
     """A K-block-major copy is named while it is current, and not once its weight was written to, moved or replaced: the next product
     makes another, and the memory of the old one is given back, whoever still holds its address."""
