@@ -42,26 +42,29 @@ WINDOWS_IN_PLACE = os.environ.get("SAMFAST_WINDOWS_IN_PLACE", "1") != "0"
 # / 38, four 201 / 73, ten 202 / 152, but sixteen 285 / 232 of an encoder's 58000, 32 541 / 499 of 109000)
 NECK_TOKENS = 40960
 # Weights that a window attention kernel reads ahead of the products behind it (read_soon): up to this many tokens, this many
-# bytes a block, and from this many bytes over all blocks on
-SOON_TOKENS, SOON_BYTES, SOON_TOTAL = 8192, 9 << 20, 85 << 20
+# bytes a block, from this many bytes over all blocks on, and for more than half of the tokens from this many bytes a block on
+SOON_TOKENS, SOON_BYTES, SOON_TOTAL, SOON_LEAST = 8192, 9 << 20, 85 << 20, 3 << 20
 FUSED_BLOCK = bool(int(os.environ.get("SAMFAST_FUSED_BLOCK", 1)))
 
 
 def read_soon(depth: int, tokens: int, weights: Sequence[torch.Tensor]) -> Sequence[torch.Tensor]:
     """Of `weights`, those of the products behind one of `depth` blocks' attention, what the window kernel's idle wavefront reads
-    while the others multiply.  The weights of an encoder that exceeds the last-level cache come out of HBM in every pass, and an
-    image's products wait for them a k tile at a time: proj first, then lin2, whose loop is the longest, then the next
-    block's qkv, while they stay few enough to arrive under the attention; lin1's gains less than it costs there.  us a pass, none / so:
-    one image of ViT-L int8 3151 / 3024, ViT-H int8 4915 / 4788, with 2:4 MLPs 4833 / 4607, bf16 ViT-B 1512 / 1501, ViT-L 3494 / 3446,
-    ViT-H 6054 / 5947 (proj alone; with lin2 6135), two of ViT-L int8 5204 / 5081; all four Linears' ViT-H int8 4930, bf16 6160 (4949 and 6099
-    without on that box).  An encoder that the cache holds is slower by it (ViT-B int8 1324 / 1329), and from four images on it is
-    level (ViT-H int8 16284 / 16309)."""
+    while the others multiply.  Weights that were not read lately come out of HBM, and an image's products wait for them a k tile at a
+    time: proj first, then lin2, whose loop is the longest, then the next block's qkv, while they stay few enough to arrive under the attention; lin1's gains less than it
+    costs there.  us a recorded pass, none / so, the middle of four recordings of each by turns, the same to 0.3 % on two boxes: one image of ViT-L int8
+    3262 / 3168, with 2:4 MLPs 3271 / 3116, ViT-H int8 5138 / 5065, 5011 / 4842, bf16 ViT-B 1591 / 1568, ViT-L 3661 / 3635, ViT-H 6255 / 6185 (proj alone; with
+    lin2 6265 / 6309); two of ViT-B bf16 2670 / 2650, ViT-L int8 5396 / 5321, 4983 / 4921, ViT-H int8 level, bf16 11828 / 11669.
+    The form that reads costs a launch of 20 us 1.7: two images of ViT-L bf16, 2 MB a block, are 6475 / 6514 (SOON_LEAST).  Encoders of other
+    depths show where the weights of all blocks stay near enough without (MiB of the three Linears, times as long: width 768 int8 54 1.002, 81 0.999, 108 0.989, 135 0.985, bf16 72 1.002, 81
+    1.004, 108 0.995, width 1024 int8 64 0.997, 80 0.993, 96 0.985, width 1280 75 1.001, 100 0.999): SOON_TOTAL.
+    From four images on it is level (ViT-H int8 16284 / 16309)."""
     if tokens > SOON_TOKENS:
         return ()
     sizes = [w.numel() * w.element_size() for w in weights]
     if depth * sum(sizes) < SOON_TOTAL:
         return ()
-    return [w for i, w in enumerate(weights) if sum(sizes[:i + 1]) <= SOON_BYTES]
+    read = [w for i, w in enumerate(weights) if sum(sizes[:i + 1]) <= SOON_BYTES]
+    return read if 2 * tokens <= SOON_TOKENS or sum(sizes[:len(read)]) >= SOON_LEAST else ()
 
 
 def _recording(x: torch.Tensor) -> bool:

@@ -159,6 +159,14 @@ def test_lists_of_buffers_read_soon():
     assert len(read_soon(24, 4096, [])) == 0
 
 
+def test_two_images_weights_are_read_ahead_where_they_repay_it():
+    """A block's 2 MB do not, 3.3 MB do; one image's do either way: (depth, tokens, width, bytes a value, buffers named)."""
+    from samfast_amd.modeling.image_encoder import read_soon
+    for depth, tokens, C, size, want in ((24, 4096, 1024, 2, 1), (24, 4097, 1024, 2, 0), (24, 8192, 1024, 2, 0), (32, 8192, 1280, 2, 1), (12, 8192, 768, 2, 3), (24, 8192, 1024, 1, 3),
+                                         (32, 8192, 1280, 1, 2)):
+        assert len(read_soon(depth, tokens, [torch.empty((n, C * size), dtype=torch.int8, device="meta") for n in (C, 4 * C, 3 * C)])) == want, (depth, tokens, C, size)
+
+
 @pytest.mark.parametrize("kind", ["int8", "half"])
 def test_weights_are_looked_up_to_be_read_ahead_in_recordings_of_few_tokens(monkeypatch, kind):
     """Nothing is asked of a Linear, and no list is made, where the host issues the launches or the tokens are many: a block is told it is one of none."""
