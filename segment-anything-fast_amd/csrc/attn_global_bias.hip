@@ -6,9 +6,10 @@
 // matrix instructions of the next half row's scores and of the previous one's P V, and the LDS reads that feed
 // them.  No running maximum is taken in the common case, LDS reads meet no bank twice (GridRow), and the
 // workgroups of a head touch its K and V ahead, so that the rows come out of their XCD's L2.
-//   Bound: at 8 x 16 x 4096 x 80 (fp16 738 us, 931 TFLOP/s, bf16 691; attn_global_kernel 803 and 763) the power limit:
-//   the 32 x 32 loop with its MFMAs alone, on the same values, took 666 us - 429 on zeros (probes that are not kept).  At one image of
-//   12 heads (63.8 us against 82) the last, half-empty round and the prologue.
+//   Bound: at 8 x 16 x 4096 x 80 (fp16 738 us, 931 TFLOP/s, bf16 691; attn_global_kernel 803 and 763) first the instructions of the two pipes, then the power
+//   limit: the same launch on zeros takes 600 us in bf16 and 620 in fp16, on values 707 and 749 (one box; of the 42 between the types half is fp16's test of the packed pairs, half its values' power).  On the
+//   256 workgroups of 1 x 8 heads, where a SIMD has one wavefront, zeros are 2 to 5 % ahead (54.9 / 56.1, 54.9 / 57.9).  At one image of 12 heads of 64 channels
+//   (63.8 us against 82) the last, half-empty round and the prologue.
 //   (The encoder, which hands over tables, keeps attn_global_kernel: its int8 Linears turn any other order of these
 //   roundings into other codes.)
 //
@@ -26,9 +27,9 @@ namespace samfast {
 
 constexpr float kCeiling = 256.0f;  // of a lane's share of a half row's sum (16 of 32 keys, on the smaller instruction 8): each probability stays far inside both types
 
-template <int HD, int WAVES>
-struct BiasCfg : GridRow<HD> {
-  using R = GridRow<HD>;
+template <int WAVES>
+struct BiasCfg : GridRow<64> {
+  using R = GridRow<64>;
   static constexpr int BM = 32 * WAVES;       // queries per workgroup
   static constexpr int KDPW = (R::KP + WAVES - 1) / WAVES, VDPW = (R::VP + WAVES - 1) / WAVES;  // wave instructions per tile a wave issues at most
   // LDS: two K tiles, three V tiles (a row's V is still read while the next row's has to be there), rel_h
@@ -39,9 +40,10 @@ struct BiasCfg : GridRow<HD> {
   static_assert(LDS_BYTES <= (WAVES == 4 ? 80 : 160) * 1024, "workgroups per CU");
 };
 
-template <typename T, int HD, int WAVES>
+template <typename T, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArgs a) {
-  using C = BiasCfg<HD, WAVES>;
+  using C = BiasCfg<WAVES>;
+  constexpr int HD = 64;
   __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS_BYTES];
   float* relhT = reinterpret_cast<float*>(lds + C::RELH_OFF);  // [kh % RH][BM], * log2(e); a wave reads only its own columns
 
@@ -62,8 +64,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
   const unsigned short* vbase = a.v + b * a.v_sb + h * a.v_sh;
 
   // ---- K / V rows: global memory -> LDS directly, wave instruction i of a tile fills pieces 64 i .. 64 i + 63 ----
-  unsigned int koff[C::KDPW];  // bytes, from the tile's first key row; unsigned: scalar-base load form
-  int voff[C::VDPW];           // negative: a spare piece, the lane loads nothing
+  unsigned int koff[C::KDPW], voff[C::VDPW];  // bytes, from the tile's first key row; unsigned: scalar-base load form
 #pragma unroll
   for (int m = 0; m < C::KDPW; ++m) {
     int row;
@@ -74,7 +75,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
   for (int m = 0; m < C::VDPW; ++m) {
     int row;
     const int at = C::v_source(64 * (wave + WAVES * m) + lane, row);
-    voff[m] = at < 0 ? -1 : row * (int)a.v_sn * 2 + at;
+    voff[m] = (unsigned int)(row * (int)a.v_sn) * 2u + at;
   }
   const unsigned int lds_base = (unsigned int)(uintptr_t)((__attribute__((address_space(3))) unsigned char*)lds);
   auto k_dma = [&](int kt, int buf) __attribute__((always_inline)) {
@@ -87,8 +88,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
     const unsigned char* src = reinterpret_cast<const unsigned char*>(vbase + (int64_t)kt * 64 * a.v_sn);
 #pragma unroll
     for (int m = 0; m < C::VDPW; ++m)
-      if (wave + WAVES * m < C::VP && (!C::ONES_ROW || voff[m] >= 0))
-        lds_dma16(src, (unsigned int)voff[m], lds_base + C::V_OFF + buf_off + (wave + WAVES * m) * 1024);
+      if (wave + WAVES * m < C::VP) lds_dma16(src, voff[m], lds_base + C::V_OFF + buf_off + (wave + WAVES * m) * 1024);
   };
   k_dma(0, 0);
   v_dma(0, 0);
@@ -124,16 +124,6 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
   for (int dt = 0; dt < C::DT; ++dt) vrd[dt] = C::V_OFF + C::v_read(lane, dt);
 #pragma unroll
   for (int ks = 0; ks < C::KS; ++ks) krd[ks] = C::k_read(lr, lh, ks);
-  // the spare pieces of the three V tiles: (1, 0, ..) and zeros
-  auto ones = [&]() __attribute__((always_inline)) {
-    if (C::ONES_ROW)
-      for (int r = tid; r < 192; r += 64 * WAVES) {
-        u32x4* p = reinterpret_cast<u32x4*>(lds + C::V_OFF + r * (C::VP * 16) + HD * 2);
-        p[0] = u32x4{T::kOne, 0u, 0u, 0u};
-        p[1] = u32x4{0u, 0u, 0u, 0u};
-      }
-  };
-  ones();
 
   // ---- bias: rel_w / sm_scale of the lane's query is the initial accumulator of the score tiles of the two
   //      half rows; rel_h * log2(e) stands in LDS, 32 key rows at a time ----
@@ -212,17 +202,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
     // online softmax, one query per lane.  The exponent offset m_i is a reference, not the running
     // maximum (the final division by the denominator, accumulated with the same offsets, makes the
     // result independent of it): probabilities may sit anywhere below a ceiling, so no maximum of the scores is
-    // taken in the common case.  Whether one has grown too large shows where the denominator is summed here in the
-    // half row's sum, else (ONES_ROW) in the packed pairs (T::note, T::outgrown).  Then -
-    // always where the first keys are met, m_i being T::kLowest - the maximum is found, the accumulators are
+    // taken in the common case.  Whether one has grown too large shows in the half row's sum (in the kernels whose denominators are
+    // products, in the packed pairs: T::note, T::outgrown).  Then - always where the first keys are met, m_i being T::kLowest - the maximum is found, the accumulators are
     // rescaled and the probabilities formed once more.  m_i is finite throughout: keys that a factor of -inf, or of
     // the type's lowest value, has taken away have probabilities of zero whatever stands before or behind them.
-    unsigned int seen = 0u;
     float l0 = 0.f, l1 = 0.f;  // this half row's share of the denominator, unrounded (two chains)
     auto pair = [&](int w, float neg_mrow) __attribute__((always_inline)) {  // packed pair w of 8
       const float p0 = fast_exp2(fmaf(s[2 * w], a.c, neg_mrow)), p1 = fast_exp2(fmaf(s[2 * w + 1], a.c, neg_mrow));
       pk[w >> 2][w & 3] = T::pack2(p0, p1);
-      if (!C::ONES_ROW) l0 += p0 + p1;
+      l0 += p0 + p1;
     };
     auto score = [&](int ks) __attribute__((always_inline)) { s_next = T::mfma(kf[ks], qf[ks], ks == 0 ? b_next : s_next); };
     auto pv = [&](int j, int dt) __attribute__((always_inline)) { oacc[dt] = T::mfma(vf[j][dt], pk_prev[j], oacc[dt]); };
@@ -233,11 +221,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
       const float x0 = fmaf(s[2 * g], a.c, neg_mrow), x1 = fmaf(s[2 * g + 1], a.c, neg_mrow);
       if (g > 0) {
         pk[(g - 1) >> 2][(g - 1) & 3] = T::pack2(e0, e1);
-        if (!C::ONES_ROW) l0 += e0, l1 += e1;
+        l0 += e0, l1 += e1;
       }
       e0 = fast_exp2(x0);
       e1 = fast_exp2(x1);
-      if (C::ONES_ROW && g > 0 && !(g & 1)) seen = T::note(seen, pk[(g - 1) >> 2][(g - 2) & 3], pk[(g - 1) >> 2][(g - 1) & 3]);
       __builtin_amdgcn_sched_barrier(0);
       if (g == 0) pv(0, 0);
       if (g == 1) {
@@ -254,9 +241,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
       __builtin_amdgcn_sched_barrier(0);
     }
     pk[1][3] = T::pack2(e0, e1);
-    if (C::ONES_ROW) seen = T::note(seen, pk[1][2], pk[1][3]);
-    else l0 = (l0 + e0) + (l1 + e1);
-    if (__any(C::ONES_ROW ? T::outgrown(seen) : l0 > kCeiling)) {  // uniform; an infinity included
+    l0 = (l0 + e0) + (l1 + e1);
+    if (__any(l0 > kCeiling)) {  // uniform; an infinity included
       float mx = s[0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
@@ -273,7 +259,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
 #pragma unroll
       for (int w = 0; w < 8; ++w) pair(w, b0 - m_i);
     }
-    if (!C::ONES_ROW) l_i += l0;
+    l_i += l0;
   };
 
   const int nkt = a.N / 64;
@@ -315,29 +301,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_global_bias_kernel(AttnArg
     for (int dt = 0; dt < C::DT; ++dt) oacc[dt] = T::mfma(vf[j][dt], pkB[j], oacc[dt]);
 
   // ---- epilogue: O = acc / l, 4 adjacent channels per store ----
-  float l;
-  if (C::ONES_ROW) {
-    // output row HD (the ones row) = tile DT-1, row HD % 32, held by the lh = (HD % 32) / 4 % 2 lanes
-    constexpr int orow = HD % 32;
-    constexpr int oreg = 4 * (orow / 8) + orow % 4, olh = (orow / 4) % 2;
-    const float own = oacc[C::DT - 1][oreg];
-    const float other = xor32(own);
-    l = (lh == olh) ? own : other;
-  } else {
-    l = l_i + xor32(l_i);
-  }
-  const float inv = 1.0f / l;
+  const float inv = 1.0f / (l_i + xor32(l_i));
   unsigned short* op = a.out + b * a.o_sb + h * a.o_sh + (int64_t)(q0 + lr) * a.o_sn;
 #pragma unroll
   for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int d = 32 * dt + 8 * j + 4 * lh;
-      if (d < HD) {
-        const u32x2 o = {T::pack2(oacc[dt][4 * j] * inv, oacc[dt][4 * j + 1] * inv),
-                         T::pack2(oacc[dt][4 * j + 2] * inv, oacc[dt][4 * j + 3] * inv)};
-        *reinterpret_cast<u32x2*>(op + d) = o;
-      }
+      const u32x2 o = {T::pack2(oacc[dt][4 * j] * inv, oacc[dt][4 * j + 1] * inv),
+                       T::pack2(oacc[dt][4 * j + 2] * inv, oacc[dt][4 * j + 3] * inv)};
+      *reinterpret_cast<u32x2*>(op + 32 * dt + 8 * j + 4 * lh) = o;
     }
 }
 
@@ -941,15 +913,16 @@ __global__ __launch_bounds__(64 * Split16Cfg::WAVES, 3) void attn_global_split16
 
 // The unsplit form at hd 80 on 16 x 16 matrix instructions (see attn_global_split16_kernel for the lane's two queries and the order of its keys): 80 channels are two
 // k steps of 32 and one of 16, five channel tiles of V^T without padding, and a sixth tile whose channels are one for every key, from registers, the denominators: 24
-// instructions of 16 cycles a half row, where the 32 x 32 form (attn_global_bias_kernel, whose channels 80 to 95 were ones and zeros of V's rows) had 11 of 32.  What bounds it: the
-// power limit from about 256 workgroups of 256 queries on (it is 6 % behind alone at full clock, with the same waits), below that a wavefront's vector instructions, 64 a half row of which 16
-// are exponentials, and matrix instructions, issued one after another.  They stand one by one in turn: three side by side are 3 to 4 % slower.  A key row neither begins with a read
+// instructions of 16 cycles a half row, where the 32 x 32 form (attn_global_bias_kernel, whose channels 80 to 95 were ones and zeros of V's rows) had 11 of 32.  What bounds it: a
+// wavefront's vector instructions, 64 a half row of which 16 are exponentials, and matrix instructions, issued one after another, and from about 256 workgroups of 256 queries on the
+// power limit besides (15 to 17 %, the file's head).  They stand one by one in turn: three side by side are 3 to 4 % slower.  A key row neither begins with a read
 // of its rel_h (read a row ahead) nor ends with a wait for the V fragments that are on their way (the barrier alone, behind vmcnt): 4 to 6 %.  The
 // denominators as 16 additions 2 %, as v_dot2 7 % slower.
 // us, 32 x 32 / so (bf16; fp16): 1 x 8 heads 63.1 / 61.7; 63.5 / 60.5, 1 x 12 77.6 / 78.0; 82.1 / 80.7, 1 x 16 91.1 / 86.9; 97.8 / 91.7, 2 x 16 181.7 / 173.0; 194.8 / 182.3, 4 x 12 268
-// / 257; 288 / 271, 8 x 16 720 / 691; 768 / 738, 16 x 16 1431 / 1381; 1533 / 1457, 3 x 13 x 24 rows 40.3 / 38.4; 42.2 / 40.0; up to a wavefront a SIMD it is level to
-// 2.5 % behind (1 x 16 x 4 rows 9.2 / 9.35; 9.05 / 9.2, 1 x 12 x 8 12.2 / 12.4; 12.1 / 12.3, 1 x 8 x 16 19.0 / 19.2; 18.7 / 19.2): twice the matrix instructions to issue (K read a half row
-// ahead where it has landed: 12.6, 19.5).  The error against 64 bits is the same to three digits (2.33e-3, 2.92e-4 of the norm).
+// / 257; 288 / 271, 8 x 16 720 / 691; 768 / 738, 16 x 16 1431 / 1381; 1533 / 1457, 3 x 13 x 24 rows 40.3 / 38.4; 42.2 / 40.0; where
+// the power limit is far it is behind for its matrix cycles, 384 a half row for 352: a batch of one up to a wavefront a SIMD level to 2 % (24 grids, two types; 1 x 8 x 32 rows 30.8 / 31.4; 30.9 / 31.2, 1 x 12 x 8 12.1 / 12.1;
+// 12.0 / 12.1), on 144 of 256 CUs 3 to 4 % (1 x 12 x 48 rows 63.4 / 65.5; 65.2 / 68.1), where batches from four on are 1 to 7 % ahead at every number of wavefronts (8 x 16 x 4 rows 10.7 / 10.0; 10.9 / 10.0).  No
+// line between the two forms can look at the batch, on which a slice's bits are not to depend (K read a half row ahead where it has landed: 12.6, 19.5).  The error against 64 bits is the same to three digits (2.33e-3, 2.92e-4 of the norm).
 template <int WAVES>
 struct Bias16Cfg {
   static constexpr int HD = 80, PIECES = HD / 8;        // 16-byte pieces of a row = wave instructions of a tile
@@ -1267,8 +1240,8 @@ static void launch_bias(const AttnArgs& a, int form, hipStream_t stream) {
     else if (form == 4) hipLaunchKernelGGL((attn_global_bias16_kernel<T, 4>), grid(128), dim3(256), 0, stream, a);
     else hipLaunchKernelGGL((attn_global_split_kernel<T>), grid(64), dim3(256), 0, stream, a);
   } else {
-    if (form == 8) hipLaunchKernelGGL((attn_global_bias_kernel<T, HD, 8>), grid(256), dim3(512), 0, stream, a);
-    else if (form == 4) hipLaunchKernelGGL((attn_global_bias_kernel<T, HD, 4>), grid(128), dim3(256), 0, stream, a);
+    if (form == 8) hipLaunchKernelGGL((attn_global_bias_kernel<T, 8>), grid(256), dim3(512), 0, stream, a);
+    else if (form == 4) hipLaunchKernelGGL((attn_global_bias_kernel<T, 4>), grid(128), dim3(256), 0, stream, a);
     else if ((int64_t)a.B * a.nH * (a.N / 64) <= 256) hipLaunchKernelGGL((attn_global_split16_kernel<T, true>), grid(64), dim3(256), 0, stream, a);
     else hipLaunchKernelGGL((attn_global_split16_kernel<T, false>), grid(64), dim3(256), 0, stream, a);
   }
