@@ -122,7 +122,8 @@ int samfast_attn_relpos_windowed_fwd(
  * The same, told what the launches behind it will read: soon_n buffers on the same GPU (at most
  * SAMFAST_MAX_SOON; soon_bytes[i] bytes from soon[i]; the two arrays are read before the call returns).  Wavefronts that have no
  * queries read a word of each of their cache lines while the others multiply, so that they come out of the last-level cache when
- * they are wanted; results do not depend on it.  The buffers have to stay allocated as long as q does.
+ * they are wanted.  A hint: all or some of it is left out where no wavefront is idle or has room for the words, and results do not depend on it.  The buffers
+ * have to stay allocated as long as q does, in a recording too.
  */
 #define SAMFAST_MAX_SOON 8
 int samfast_attn_relpos_windowed_soon_fwd(

@@ -692,8 +692,8 @@ __global__ __launch_bounds__((WindowCfg<HD, TILES>::THREADS), 2) void attn_windo
   if (FUSED && !has_tile) {  // a wavefront without a query tile only helps with the staging and with the output
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();  // V complete (the barrier the others reach after their first score tile)
-    // The last wavefront of seven tiles' eight has none: it reads what comes next, while the others multiply, for 0.9 us of a launch of 20.  The
-    // words go behind the last key's row, where nobody looks: to registers, four at a time, an image's 38 MB took 7 us.  (The global kernel has no such
+    // The last wavefront of seven tiles' eight has none: it reads what comes next, while the others multiply.  This form of a launch of 20 us is 1.7
+    // longer (one image of ViT-L, twenty of them: bf16 3644 without, 3675 with 4 KB a launch, which gain nothing; int8 3247 / 3282).  The words go behind the last key's row, where nobody looks: to registers, four at a time, an image's 38 MB took 7 us.  (The global kernel has no such
     // wavefront: a chunk of each wavefront's every eight key rows, awaited with the next tile, lengthened it by 7 of 98 us.)
     if constexpr (SOON)
       if (wave_u == 7)

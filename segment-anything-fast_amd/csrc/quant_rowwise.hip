@@ -26,8 +26,8 @@ __host__ SF_DEVICE unsigned int quant_blocks(int64_t M, int rpb) { return ((unsi
 // Which RPB rows workgroup b takes, of quant_blocks(M, RPB): every XCD (workgroup modulo 8) a contiguous eighth, and that from its end.
 // The products on either side walk such eighths from their starts: what one of them has written last, and the last-level cache still holds, is read
 // first here, and what is written last here is read first by the next one.  us in the ViT-H encoder, 16 images, row by row / so: rows with LayerNorm 53.2 / 51.9, proj
-// and lin2 behind them 232.8 / 227.4 on average, rows with GELU, whose producer streams past the cache, 176 / 179; the
-// whole 58541 / 58305, 32 images with 2:4 MLPs 109600 / 108660, ViT-L 16 images 35121 / 34917, five 12081 / 11980; single images level.
+// and lin2 behind them 232.8 / 227.4 on average, rows with GELU, whose producer streams past the cache, 176 / 179; of
+// the present rows the whole 57620 / 57410 and 57760 / 57370, 32 images with 2:4 MLPs 108610 / 107490 and 108530 / 107390, ViT-L in bf16, whose rows are not these, level; single images level.
 // A Linear's own rows, without LayerNorm or GELU, are taken as they come by one wavefront (65536 x 1280 -> 3840 306.6 so, 309.4 from the ends) and by two through the cache (32768 x 2048
 // -> 2048 148 / 151); the other shared rows from the ends (65536 x 4096 -> 1024 378 / 338, 16384 x 5120 -> 1280 126.3 / 121.0, 65536 x 2560 -> 1280 268 / 260, 20480 x 3072 -> 768 72 / 69.8).
 SF_DEVICE unsigned int row_block(unsigned int b, int64_t M, int rpb) {
