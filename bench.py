@@ -734,7 +734,7 @@ def main():
     if not args.no_cpu_baseline:
         from oracle import image_encoder as oe
         cfg = {"vit_h": oe.VIT_H, "vit_l": oe.VIT_L, "vit_b": oe.VIT_B}[args.model]
-        # the host share of a one-GPU box is 16 cores whatever os.cpu_count() shows there
+        # a process beside one GPU has a share of 16 cores whatever os.cpu_count() shows there
         cores = min(os.cpu_count() or 1, int(os.environ.get("OMP_NUM_THREADS", "16")))
         torch.set_num_threads(cores)
         if default_workload and not args.main_only:

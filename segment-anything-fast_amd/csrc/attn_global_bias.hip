@@ -7,7 +7,7 @@
 // them.  No running maximum is taken in the common case, LDS reads meet no bank twice (GridRow), and the
 // workgroups of a head touch its K and V ahead, so that the rows come out of their XCD's L2.
 //   Bound: at 8 x 16 x 4096 x 80 (fp16 738 us, 931 TFLOP/s, bf16 691; attn_global_kernel 803 and 763) first the instructions of the two pipes, then the power
-//   limit: the same launch on zeros takes 600 us in bf16 and 620 in fp16, on values 707 and 749 (one box; of the 42 between the types half is fp16's test of the packed pairs, half its values' power).  On the
+//   limit: the same launch on zeros takes 600 us in bf16 and 620 in fp16, on values 707 and 749 (one machine; of the 42 between the types half is fp16's test of the packed pairs, half its values' power).  On the
 //   256 workgroups of 1 x 8 heads, where a SIMD has one wavefront, zeros are 2 to 5 % ahead (54.9 / 56.1, 54.9 / 57.9).  At one image of 12 heads of 64 channels
 //   (63.8 us against 82) the last, half-empty round and the prologue.
 //   (The encoder, which hands over tables, keeps attn_global_kernel: its int8 Linears turn any other order of these

@@ -51,7 +51,7 @@ def read_soon(depth: int, tokens: int, weights: Sequence[torch.Tensor]) -> Seque
     """Of `weights`, those of the products behind one of `depth` blocks' attention, what the window kernel's idle wavefront reads
     while the others multiply.  Weights that were not read lately come out of HBM, and an image's products wait for them a k tile at a
     time: proj first, then lin2, whose loop is the longest, then the next block's qkv, while they stay few enough to arrive under the attention; lin1's gains less than it
-    costs there.  us a recorded pass, none / so, the middle of four recordings of each by turns, the same to 0.3 % on two boxes: one image of ViT-L int8
+    costs there.  us a recorded pass, none / so, the middle of four recordings of each by turns, the same to 0.3 % on two machines: one image of ViT-L int8
     3262 / 3168, with 2:4 MLPs 3271 / 3116, ViT-H int8 5138 / 5065, 5011 / 4842, bf16 ViT-B 1591 / 1568, ViT-L 3661 / 3635, ViT-H 6255 / 6185 (proj alone; with
     lin2 6265 / 6309); two of ViT-B bf16 2670 / 2650, ViT-L int8 5396 / 5321, 4983 / 4921, ViT-H int8 level, bf16 11828 / 11669.
     The form that reads costs a launch of 20 us 1.7: two images of ViT-L bf16, 2 MB a block, are 6475 / 6514 (SOON_LEAST).  Encoders of other
